@@ -2,8 +2,9 @@
 // output head.  W is a weight matrix [out, in] with `in` contiguous, as stored in the
 // checkpoint (kappai: y[n] = sum_k W[n,k] x[k], src/backend/cpu/scalar/quants.c:1398-1414).
 //
-//   gemm_f32         true 32-bit on the vector ALUs: every product and sum is an fp32 FMA in
-//                    the order k = 0..K-1, so a row's result does not depend on M.
+//   gemm_f32         true 32-bit: float products and sums on the matrix cores
+//                    (v_mfma_f32_16x16x4_f32) in an order that K alone decides, so a row's result
+//                    does not depend on M; a kernel for up to 64 rows and one for more.
 //   gemm_bf16_block256  large products (K a multiple of 128 per K range): bf16 inputs, fp32
 //                    accumulation on the matrix cores (v_mfma_f32_32x32x16_bf16), 256x256 or
 //                    128x128 blocks, tiles of 64 of K loaded straight into LDS.
@@ -28,86 +29,345 @@ typedef __attribute__((ext_vector_type(4))) uint32_t u32x4_t;
 // ---------------------------------------------------------------------------------------
 // true fp32
 // ---------------------------------------------------------------------------------------
-#define F32_BM 64
-#define F32_BN 64
-#define F32_BK 16
-#define F32_SUM_TILES 8
+#if !defined(GATE_ACT) || GATE_ACT == 0     // (the builds with another gate hold gated products only)
+// Both kernels multiply on the matrix cores in 32 bits (v_mfma_f32_16x16x4_f32: float products
+// and float sums, 256 flops a clock and CU against 128 for a float FMA on the vector units) and add
+// in ONE order that K alone decides, so a row's result depends neither on M nor on which of them
+// runs: K is cut into chunks of 128, the chunks into 8 or 32 runs; the products of a chunk are
+// added 16 of K after 16 (lane group q of a load holds k = 4 q .. 4 q + 3 of the 16, step e takes
+// the e-th of every group), then chunk after chunk into the run's sum, then run after run.  A single
+// running sum over K = 8192 would lose about sqrt(K) roundings; this way it is sqrt(128) + a few.
+//
+// WHOLE: K is a multiple of 128 and everything is aligned to 16 bytes.  The loads then stand in no
+// branch (a branch around them has the compiler wait for one before it asks for the next).
+#define F32_CHUNK 128
+#define F32_STEPS (F32_CHUNK / 16)
 
-__global__ __launch_bounds__(256) void gemm_f32_kernel(const float* __restrict__ A,
-                                                       const float* __restrict__ W,
-                                                       const float* __restrict__ bias,
-                                                       float* __restrict__ C, int M, int N, int K,
-                                                       int lda, int ldc) {
-  __shared__ float As[F32_BK][F32_BM + 4];
-  __shared__ float Ws[F32_BK][F32_BN + 4];
-  const int tid = threadIdx.x;
-  const int tx = tid % 16, ty = tid / 16;
-  const int m0 = blockIdx.y * F32_BM, n0 = blockIdx.x * F32_BN;
-  // Sums in two levels: `acc` runs over F32_SUM_TILES tiles of K (128 values), then goes into
-  // `tot`.  A single running sum over K = 8192 loses about sqrt(K) roundings; this way it is
-  // sqrt(128) + sqrt(K / 128), a quarter of that, for one more addition per 128 products.
-  float acc[4][4], tot[4][4];
-#pragma unroll
-  for (int i = 0; i < 4; ++i)
-#pragma unroll
-    for (int j = 0; j < 4; ++j) acc[i][j] = tot[i][j] = 0.f;
+__device__ __forceinline__ f32x4_t mfma_f32(float a, float b, f32x4_t c) {
+  return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+}
+__host__ __device__ __forceinline__ int f32_runs(int chunks) { return chunks <= 16 ? 8 : 32; }
+__device__ __forceinline__ int f32_run_start(int run, int runs, int chunks) {
+  return run * chunks / runs;
+}
 
-  int tiles_in_acc = 0;
-  for (int k0 = 0; k0 < K; k0 += F32_BK) {
-    if (tiles_in_acc == F32_SUM_TILES) {
+// Four values of a row from k on; zeros from `end` on.
+__device__ __forceinline__ f32x4_t load4_f32(const float* __restrict__ row, int k, int end) {
+  f32x4_t v = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-      for (int i = 0; i < 4; ++i)
+  for (int e = 0; e < 4; ++e)
+    if (k + e < end) v[e] = row[k + e];
+  return v;
+}
+
+// A lane's share of a chunk (its q-th four of every 16).
+template <bool WHOLE>
+__device__ __forceinline__ void load_chunk_f32(const float* __restrict__ row, int chunk, int q, int K,
+                                               f32x4_t (&v)[F32_STEPS]) {
+  const int k = chunk * F32_CHUNK + 4 * q;
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          tot[i][j] += acc[i][j];
-          acc[i][j] = 0.f;
-        }
-      tiles_in_acc = 0;
+  for (int j = 0; j < F32_STEPS; ++j)
+    v[j] = WHOLE ? *reinterpret_cast<const f32x4_t*>(row + k + 16 * j)
+                 : load4_f32(row, k + 16 * j, K);
+}
+
+// 1 to 64 rows: bound by the stream of W, in small matrices by what one block has under way.  A
+// block owns COLS rows of W, a wave one or several runs of K, and the waves meet in LDS.  COLS = 16: a
+// wave walks its RUNS / 8 runs one after the other.  COLS = 8 (up to 8 rows; matrices of few rows, so
+// that twice the blocks stream them): places 0-7 of both operands hold the wave's first run and 8-15
+// its second, and the product's two diagonal quarters are the two runs' sums.  The next chunk's share
+// of W is under way while a chunk is multiplied.  Three rows, W from memory: 9216 x 1024 12 us
+// (3.1 TB/s), 1024 x 4608 9 us, 65536 x 1024 51 us (5.3 TB/s); the vector kernel before took 100 to
+// 1,500 us, a block a 64 x 64 tile of which three rows were real.
+template <int MT, int COLS, int RUNS, bool WHOLE>
+__global__ __launch_bounds__((COLS == 8 ? RUNS / 2 : 8) * WAVE) void gemm_f32_skinny_kernel(
+    const float* __restrict__ A, const float* __restrict__ W, const float* __restrict__ bias,
+    float* __restrict__ C, int M, int N, int K, int lda, int ldc) {
+  constexpr bool SIDE = COLS == 8;               // two runs side by side
+  constexpr int NW = SIDE ? RUNS / 2 : 8;
+  static_assert(!SIDE || MT == 1, "two runs side by side leave room for 8 rows");
+  __shared__ float red[RUNS][MT][SIDE ? 8 : 16][COLS];
+  const int wave = threadIdx.x / WAVE, lane = threadIdx.x % WAVE;
+  const int r = lane % 16, q = lane / 16;
+  const int n0 = blockIdx.x * COLS;
+  const float* w = W + (size_t)min(n0 + r % COLS, N - 1) * K;
+  const float* a[MT];
+#pragma unroll
+  for (int mt = 0; mt < MT; ++mt)
+    a[mt] = A + (size_t)min(mt * 16 + (SIDE ? r % 8 : r), M - 1) * lda;
+
+  const int chunks = (K + F32_CHUNK - 1) / F32_CHUNK;
+  // this lane's chunks c0 .. c0 + len - 1; the wave takes `most` steps, a chunk each
+  constexpr int per = RUNS / NW;
+  const int run0 = wave * per;
+  int c0 = f32_run_start(run0, RUNS, chunks);
+  int len = f32_run_start(run0 + per, RUNS, chunks) - c0, most = len;
+  if (SIDE) {
+    const int mid = f32_run_start(run0 + 1, RUNS, chunks), second = c0 + len - mid;
+    len = mid - c0;
+    most = max(len, second);
+    if (r / 8) {
+      c0 = mid;
+      len = second;
     }
-    ++tiles_in_acc;
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      const int idx = tid + e * 256;         // 0..1023
-      const int r = idx / F32_BK, kk = idx % F32_BK;
-      const int gm = m0 + r, gn = n0 + r, gk = k0 + kk;
-      As[kk][r] = (gm < M && gk < K) ? A[(size_t)gm * lda + gk] : 0.f;
-      Ws[kk][r] = (gn < N && gk < K) ? W[(size_t)gn * K + gk] : 0.f;
-    }
-    __syncthreads();
-#pragma unroll
-    for (int kk = 0; kk < F32_BK; ++kk) {
-      float a[4], b[4];
-#pragma unroll
-      for (int i = 0; i < 4; ++i) a[i] = As[kk][ty * 4 + i];
-#pragma unroll
-      for (int j = 0; j < 4; ++j) b[j] = Ws[kk][tx * 4 + j];
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) acc[i][j] = fmaf(a[i], b[j], acc[i][j]);
-    }
-    __syncthreads();
   }
+  f32x4_t tot[MT], wv[F32_STEPS], av[MT][F32_STEPS];
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int gm = m0 + ty * 4 + i;
-    if (gm >= M) continue;
+  for (int mt = 0; mt < MT; ++mt) tot[mt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  int run = run0;                                // (one after the other) the run that `tot` is of
+  const auto write_run = [&]() {
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int gn = n0 + tx * 4 + j;
-      if (gn < N) C[(size_t)gm * ldc + gn] = (tot[i][j] + acc[i][j]) + (bias ? bias[gn] : 0.f);
+    for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        red[run][mt][(4 * q + i) % (SIDE ? 8 : 16)][r % COLS] = tot[mt][i];
+        tot[mt][i] = 0.f;
+      }
+    ++run;
+  };
+  // (a chunk behind a lane's last is read again from the last of all and not added)
+  const auto load_w = [&](int c, f32x4_t (&v)[F32_STEPS]) {
+    load_chunk_f32<WHOLE>(w, min(c0 + c, chunks - 1), q, K, v);
+  };
+  const auto load_a = [&](int c) {
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt)
+      load_chunk_f32<WHOLE>(a[mt], min(c0 + c, chunks - 1), q, K, av[mt]);
+  };
+  const auto multiply = [&](int c) {
+    if (!SIDE)
+      while (f32_run_start(run + 1, RUNS, chunks) <= c0 + c) write_run();
+    f32x4_t acc[MT];
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt) acc[mt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int j = 0; j < F32_STEPS; ++j)
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt) acc[mt] = mfma_f32(av[mt][j][e], wv[j][e], acc[mt]);
+    // (side by side, a lane's results belong to the run that its column's half holds)
+    if (!SIDE || c < len)
+#pragma unroll
+      for (int mt = 0; mt < MT; ++mt) tot[mt] += acc[mt];
+  };
+  if (most > 0) {
+    load_w(0, wv);
+    int c = 0;
+    for (; c + 1 < most; ++c) {
+      f32x4_t wn[F32_STEPS];
+      load_a(c);
+      load_w(c + 1, wn);
+      __builtin_amdgcn_sched_barrier(0);       // (left alone, the loads sink to their use)
+      multiply(c);
+#pragma unroll
+      for (int j = 0; j < F32_STEPS; ++j) wv[j] = wn[j];
     }
+    load_a(c);
+    __builtin_amdgcn_sched_barrier(0);
+    multiply(c);
+  }
+  if (SIDE) {
+    run += r / 8;
+    if (r / 8 == q / 2) write_run();
+  } else {
+    while (run < run0 + per) write_run();
+  }
+  __syncthreads();
+  for (int at = threadIdx.x; at < MT * (SIDE ? 8 : 16) * COLS; at += NW * WAVE) {
+    const int m = at / COLS, n = n0 + at % COLS;
+    if (m >= M || n >= N) continue;
+    float s = red[0][m / 16][m % 16][at % COLS];
+#pragma unroll
+    for (int g = 1; g < RUNS; ++g) s += red[g][m / 16][m % 16][at % COLS];
+    C[(size_t)m * ldc + n] = s + (bias ? bias[n] : 0.f);
   }
 }
 
+// More rows: bound by the matrix cores.  Blocks of WY x WX waves with wave tiles of 16 TY x 16 TX;
+// K tiles of BK go through registers into two LDS buffers whose 16-byte places are XOR-permuted by
+// the row, so that eight lanes of a read hit all banks.  The next tile's loads are under way while
+// this one is multiplied.  An XCD takes every eighth column of tiles and walks its rows of tiles, so W
+// is read into one L2 only.  Two waves a SIMD: a wave's chunk, run and whole sums stay in
+// vector registers, and one wave multiplies while the other waits for LDS.  825 rows: 9216 x 1024
+// 165 us (94 TFLOP/s; the instruction alone reaches 153), 3072 x 1024 75 us, 2048 x 1024 46 us.
+template <int WY, int WX, int TY, int TX, int BK, bool WHOLE>
+__global__ __launch_bounds__(WY * WX * WAVE) __attribute__((amdgpu_waves_per_eu(2, 2)))
+void gemm_f32_block_kernel(
+    const float* __restrict__ A, const float* __restrict__ W, const float* __restrict__ bias,
+    float* __restrict__ C, int M, int N, int K, int lda, int ldc, int tiles_m) {
+  constexpr int BM = 16 * WY * TY, BN = 16 * WX * TX, SLOTS = BK / 4, NT = WY * WX * WAVE;
+  constexpr int PER = BM * SLOTS / NT;                         // 16-byte places a thread and operand
+  static_assert(BM == BN && PER * NT == BM * SLOTS && F32_CHUNK % BK == 0, "a tile");
+  __shared__ f32x4_t lds[2][2][BM * SLOTS];
+  const int tid = threadIdx.x, wave = tid / WAVE, lane = tid % WAVE;
+  const int r = lane % 16, q = lane / 16;
+  const int wm = wave / WX * 16 * TY, wn = wave % WX * 16 * TX;
+  const int m0 = (int)(blockIdx.x / 8) % tiles_m * BM;
+  const int n0 = ((int)(blockIdx.x / 8) / tiles_m * 8 + (int)(blockIdx.x % 8)) * BN;
+  if (n0 >= N) return;
+
+  const float* src[2][PER];
+  int at[PER];
+  const int slot = tid % SLOTS;
+#pragma unroll
+  for (int p = 0; p < PER; ++p) {
+    const int row = (tid + NT * p) / SLOTS;
+    src[0][p] = A + (size_t)min(m0 + row, M - 1) * lda;
+    src[1][p] = W + (size_t)min(n0 + row, N - 1) * K;
+    at[p] = row * SLOTS + (slot ^ (row & 7));
+  }
+  f32x4_t next[2][PER];
+  const auto fetch = [&](int t) {
+#pragma unroll
+    for (int o = 0; o < 2; ++o)
+#pragma unroll
+      for (int p = 0; p < PER; ++p)
+        next[o][p] = WHOLE ? *reinterpret_cast<const f32x4_t*>(src[o][p] + t * BK + 4 * slot)
+                           : load4_f32(src[o][p], t * BK + 4 * slot, K);
+  };
+  const auto keep = [&](int t) {
+#pragma unroll
+    for (int o = 0; o < 2; ++o)
+#pragma unroll
+      for (int p = 0; p < PER; ++p) lds[t & 1][o][at[p]] = next[o][p];
+  };
+  f32x4_t tot[TY][TX], fin[TY][TX];
+#pragma unroll
+  for (int i = 0; i < TY; ++i)
+#pragma unroll
+    for (int j = 0; j < TX; ++j) tot[i][j] = fin[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+
+  const int chunks = (K + F32_CHUNK - 1) / F32_CHUNK, runs = f32_runs(chunks);
+  const int tiles = chunks * (F32_CHUNK / BK);       // (those behind K are zeros)
+  int run = 0;
+  fetch(0);
+  keep(0);
+  __syncthreads();
+  for (int chunk = 0; chunk < chunks; ++chunk) {
+    f32x4_t acc[TY][TX];
+#pragma unroll
+    for (int i = 0; i < TY; ++i)
+#pragma unroll
+      for (int j = 0; j < TX; ++j) acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int u = 0; u < F32_CHUNK / BK; ++u) {
+      const int t = chunk * (F32_CHUNK / BK) + u;
+      fetch(min(t + 1, tiles - 1));                  // (the last tile once more, unused)
+      __builtin_amdgcn_sched_barrier(0);             // (left alone, the loads sink to their use)
+      const f32x4_t* la = lds[t & 1][0];
+      const f32x4_t* lw = lds[t & 1][1];
+      f32x4_t av[2][TY], wv[2][TX];
+      const auto read = [&](int s) {
+#pragma unroll
+        for (int i = 0; i < TY; ++i) {
+          const int ra = wm + 16 * i + r;
+          av[s & 1][i] = la[ra * SLOTS + ((4 * s + q) ^ (ra & 7))];
+        }
+#pragma unroll
+        for (int j = 0; j < TX; ++j) {
+          const int rw = wn + 16 * j + r;
+          wv[s & 1][j] = lw[rw * SLOTS + ((4 * s + q) ^ (rw & 7))];
+        }
+      };
+      read(0);
+#pragma unroll
+      for (int s = 0; s < BK / 16; ++s) {
+        if (s + 1 < BK / 16) read(s + 1);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+#pragma unroll
+          for (int i = 0; i < TY; ++i)
+#pragma unroll
+            for (int j = 0; j < TX; ++j)
+              acc[i][j] = mfma_f32(av[s & 1][i][e], wv[s & 1][j][e], acc[i][j]);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      keep(t + 1);
+      __syncthreads();
+    }
+#pragma unroll
+    for (int i = 0; i < TY; ++i)
+#pragma unroll
+      for (int j = 0; j < TX; ++j) tot[i][j] += acc[i][j];
+    while (run < runs && f32_run_start(run + 1, runs, chunks) <= chunk) ++run;
+    if (f32_run_start(run + 1, runs, chunks) == chunk + 1) {   // the run ends with this chunk
+#pragma unroll
+      for (int i = 0; i < TY; ++i)
+#pragma unroll
+        for (int j = 0; j < TX; ++j) {
+          fin[i][j] += tot[i][j];
+          tot[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+        }
+    }
+  }
+#pragma unroll
+  for (int j = 0; j < TX; ++j) {
+    const int n = n0 + wn + 16 * j + r;
+    if (n >= N) continue;
+    const float b = bias ? bias[n] : 0.f;
+#pragma unroll
+    for (int i = 0; i < TY; ++i)
+#pragma unroll
+      for (int x = 0; x < 4; ++x) {
+        const int m = m0 + wm + 16 * i + 4 * q + x;
+        if (m < M) C[(size_t)m * ldc + n] = fin[i][j][x] + b;
+      }
+  }
+}
+
+template <bool WHOLE>
+static void launch_f32(const float* A, const float* W, const float* bias, float* C, int M, int N,
+                       int K, int lda, int ldc, hipStream_t stream) {
+  if (M <= 64) {
+    const bool many = f32_runs((K + F32_CHUNK - 1) / F32_CHUNK) == 32;
+#define F32_SKINNY(MT, COLS, RUNS)                                                                \
+  hipLaunchKernelGGL((gemm_f32_skinny_kernel<MT, COLS, RUNS, WHOLE>), dim3((N + COLS - 1) / COLS), \
+                     dim3((COLS == 8 ? RUNS / 2 : 8) * WAVE), 0, stream, A, W, bias, C, M, N, K,   \
+                     lda, ldc)
+    if (M <= 8 && N <= 256 * 8) {
+      if (many) F32_SKINNY(1, 8, 32);
+      else F32_SKINNY(1, 8, 8);
+    } else if (M <= 16) {
+      if (many) F32_SKINNY(1, 16, 32);
+      else F32_SKINNY(1, 16, 8);
+    } else if (M <= 32) {
+      if (many) F32_SKINNY(2, 16, 32);
+      else F32_SKINNY(2, 16, 8);
+    } else {
+      if (many) F32_SKINNY(4, 16, 32);
+      else F32_SKINNY(4, 16, 8);
+    }
+#undef F32_SKINNY
+    return;
+  }
+  const auto tiles = [](int n, int b) { return (n + b - 1) / b; };
+  const long big = (long)tiles(M, 128) * tiles(N, 128), small = (long)tiles(M, 64) * tiles(N, 64);
+  if ((big + 255) / 256 * 4 * 8 <= (small + 255) / 256 * 9) {
+    const int tm = tiles(M, 128);
+    hipLaunchKernelGGL((gemm_f32_block_kernel<2, 4, 4, 2, 64, WHOLE>),
+                       dim3(tiles(tiles(N, 128), 8) * 8 * tm), dim3(512), 0, stream, A, W, bias, C,
+                       M, N, K, lda, ldc, tm);
+  } else {
+    const int tm = tiles(M, 64);
+    hipLaunchKernelGGL((gemm_f32_block_kernel<2, 2, 2, 2, 64, WHOLE>),
+                       dim3(tiles(tiles(N, 64), 8) * 8 * tm), dim3(256), 0, stream, A, W, bias, C,
+                       M, N, K, lda, ldc, tm);
+  }
+}
+
+// Rows and columns of any number and any K.
 extern "C" int kappai_gemm_f32(const float* A, const float* W, const float* bias, float* C, int M,
                                int N, int K, int lda, int ldc, hipStream_t stream) {
   if (M <= 0 || N <= 0) return 0;
-  dim3 grid((N + F32_BN - 1) / F32_BN, (M + F32_BM - 1) / F32_BM);
-  hipLaunchKernelGGL(gemm_f32_kernel, grid, dim3(256), 0, stream, A, W, bias, C, M, N, K, lda,
-                     ldc);
+  const bool whole = K % F32_CHUNK == 0 && lda % 4 == 0 && (uintptr_t)A % 16 == 0 &&
+                     (uintptr_t)W % 16 == 0;
+  if (whole) launch_f32<true>(A, W, bias, C, M, N, K, lda, ldc, stream);
+  else launch_f32<false>(A, W, bias, C, M, N, K, lda, ldc, stream);
   KAPPAI_RETURN_LAUNCH_STATUS();
 }
+#endif  // GATE_ACT == 0
 
 // ---------------------------------------------------------------------------------------
 // bf16 on the matrix cores

@@ -9,12 +9,16 @@
 //   paged_attention_rows  one wave per (row, head): causal softmax(q.k/sqrt(d)) v over the keys
 //                       lo..pos of the row's request, read through its block table
 //                       (src/backend/cpu/scalar/core.c:383-433, 623-666), online softmax in float.
+//   paged_attention_f32  the same for float32 heads of whole 16s, sixteen (row, head) places a
+//                       block on the matrix cores.
 //
 // The key pool is [page][kv_head][page_size][head_dim]; the value pool is stored transposed,
 // [page][kv_head][head_dim][page_size], which is what the matrix-core kernels want.  Token p of
 // a request lives in page block_table[p / page_size] at offset p % page_size.
 #include "common.h"
 #include "score_mods.h"
+
+typedef __attribute__((ext_vector_type(4))) float f32x4_t;
 
 #define MAX_HEAD_DIM 512
 
@@ -371,6 +375,167 @@ __global__ __launch_bounds__(64) void paged_attention_rows_kernel(
   }
 }
 
+// ---------------------------------------------------------------------------------------
+// float32 attention on the matrix cores (v_mfma_f32_16x16x4_f32: float products and sums).
+//
+// A block takes one kv head and sixteen places (row, head of the kv head's): as many rows of one
+// segment as fit beside each other, so a prompt's rows share every key and value they read, and a
+// decoded row has its heads in one block.  Its waves take steps of 16 keys in turns (step s
+// belongs to wave s % NW wherever a row's keys begin and end) and meet in LDS at the end, so a row's
+// result does not depend on the rows it is computed with.  Scores are made keys x places, which
+// is the layout in which the weights enter the product with the transposed values: nothing moves
+// between lanes but the maximum and the sum of a place.  Bound by the latency of a step's loads, so the next
+// step's are under way while one is worked on.  16 heads of 64 on 8 kv heads: a prompt step of 150, 275 and
+// 400 tokens 43 us, three decoded rows at these lengths 14 us; a wave a (row, head), as before,
+// took 126 us on average over both.
+template <int NT>
+__global__ __launch_bounds__((NT <= 4 ? 8 : 4) * WAVE) void paged_attention_f32_kernel(
+    const float* __restrict__ q, int q_stride, const float* __restrict__ k_pool,
+    const float* __restrict__ v_pool, float* __restrict__ out, int out_stride,
+    const int* __restrict__ row_pos, const int* __restrict__ row_seg,
+    const int* __restrict__ block_tables, int max_blocks, int T, int H, int G, int ps, int window,
+    float scale) {
+  constexpr int D = 16 * NT, NW = NT <= 4 ? 8 : 4;
+  __shared__ float part[NW][16][D + 1];
+  __shared__ float part_m[NW][16], part_l[NW][16];
+  const int per = H / G, heads = min(per, 16), R = 16 / heads, pieces = (per + heads - 1) / heads;
+  const int g = blockIdx.y / pieces, h0 = g * per + blockIdx.y % pieces * heads;
+  const int t0 = blockIdx.x, seg = row_seg[t0];
+  if (t0 % R != 0 && row_seg[t0 - 1] == seg) return;       // the block of an earlier row has it
+  int t1 = t0 + 1;
+  while (t1 < T && t1 % R != 0 && row_seg[t1] == seg) ++t1;
+
+  const int wave = threadIdx.x / WAVE, lane = threadIdx.x % WAVE;
+  const int r = lane % 16, quad = lane / 16;
+  int row = t0 + r / heads, head = h0 + r % heads;
+  if (row >= t1 || head >= (g + 1) * per) row = t0, head = h0;    // a place without work of its own
+  const int pos = row_pos[row], lo = kappai_first_key(pos, window);
+  const int pos_max = wave_max(pos), lo_min = -wave_max(-lo);
+  const int* bt = block_tables + (size_t)seg * max_blocks;
+
+  f32x4_t qv[NT], acc[NT], kv[NT], vv[NT];
+#pragma unroll
+  for (int j = 0; j < NT; ++j) {
+    qv[j] = *reinterpret_cast<const f32x4_t*>(q + (size_t)row * q_stride + (size_t)head * D +
+                                              16 * j + 4 * quad);
+    acc[j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  }
+  // keys outside lo_min .. pos_max are read from the nearest one inside (their pages may be gone)
+  const auto fetch = [&](int st, f32x4_t (&kf)[NT], f32x4_t (&vf)[NT]) {
+    const int key = min(max(16 * st + r, lo_min), pos_max);
+    const int four = min(max(16 * st + 4 * quad, lo_min / 4 * 4), pos_max / 4 * 4);
+    const float* kp = k_pool + (((size_t)bt[key / ps] * G + g) * ps + key % ps) * D + 4 * quad;
+    const float* vp = v_pool + (((size_t)bt[four / ps] * G + g) * D + r) * ps + four % ps;
+#pragma unroll
+    for (int j = 0; j < NT; ++j) {
+      kf[j] = *reinterpret_cast<const f32x4_t*>(kp + 16 * j);
+      vf[j] = *reinterpret_cast<const f32x4_t*>(vp + (size_t)16 * j * ps);
+    }
+  };
+  float m = -INFINITY, l = 0.f;
+  const int first = lo_min / 16, last = pos_max / 16;
+  int st = first + ((wave - first) % NW + NW) % NW;
+  if (st <= last) fetch(st, kv, vv);
+  for (; st <= last; st += NW) {
+    f32x4_t kn[NT], vn[NT];
+    if (st + NW <= last) fetch(st + NW, kn, vn);
+    f32x4_t s = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int j = 0; j < NT; ++j)
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        s = __builtin_amdgcn_mfma_f32_16x16x4f32(kv[j][e], qv[j][e], s, 0, 0, 0);
+    const int key0 = 16 * st + 4 * quad;       // this lane's scores: keys key0 .. key0 + 3, place r
+    bool seen[4], odd = false;
+    float top = -INFINITY;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      seen[i] = key0 + i <= pos && key0 + i >= lo;
+      s[i] = seen[i] ? s[i] * scale : -INFINITY;
+      top = fmaxf(top, s[i]);
+      const bool inside = key0 + i <= pos_max && key0 + i >= lo_min;
+#pragma unroll
+      for (int j = 0; j < NT; ++j) {
+        if (!inside) vv[j][i] = 0.f;           // (nobody's: what lies there is anything)
+        odd |= !(fabsf(vv[j][i]) < INFINITY);
+      }
+    }
+    top = fmaxf(top, lane_xor16(top));
+    top = fmaxf(top, lane_xor32(top));
+    const float m_new = fmaxf(m, top);
+    const float ref = m_new == -INFINITY ? 0.f : m_new;
+    const float corr = expf(m - ref);
+    f32x4_t p;
+    float sum = 0.f;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      p[i] = seen[i] ? expf(s[i] - ref) : 0.f;
+      sum += p[i];
+    }
+    sum += lane_xor16(sum);
+    sum += lane_xor32(sum);
+    l = l * corr + sum;
+    m = m_new;
+#pragma unroll
+    for (int j = 0; j < NT; ++j) acc[j] *= corr;
+    if (!__any(odd)) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+#pragma unroll
+        for (int j = 0; j < NT; ++j)
+          acc[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(vv[j][e], p[e], acc[j], 0, 0, 0);
+    } else {
+      // a value that is no finite number must not meet the weight 0 of a place that does not see
+      // its key: place by place, with the keys that the place sees
+      for (int c = 0; c < 16; ++c) {
+        const int pos_c = __shfl(pos, c, WAVE), lo_c = __shfl(lo, c, WAVE);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const bool sees = key0 + e <= pos_c && key0 + e >= lo_c;
+#pragma unroll
+          for (int j = 0; j < NT; ++j) {
+            const f32x4_t got = __builtin_amdgcn_mfma_f32_16x16x4f32(
+                sees ? vv[j][e] : 0.f, p[e], acc[j], 0, 0, 0);
+            if (r == c) acc[j] = got;
+          }
+        }
+      }
+    }
+#pragma unroll
+    for (int j = 0; j < NT; ++j) {
+      kv[j] = kn[j];
+      vv[j] = vn[j];
+    }
+  }
+#pragma unroll
+  for (int j = 0; j < NT; ++j)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) part[wave][r][16 * j + 4 * quad + i] = acc[j][i];
+  if (quad == 0) {
+    part_m[wave][r] = m;
+    part_l[wave][r] = l;
+  }
+  __syncthreads();
+  for (int at = threadIdx.x; at < 16 * D; at += NW * WAVE) {
+    const int place = at / D, e = at % D;
+    const int to = t0 + place / heads, hd = h0 + place % heads;
+    if (place >= R * heads || to >= t1 || hd >= (g + 1) * per) continue;
+    float top = part_m[0][place];
+#pragma unroll
+    for (int w = 1; w < NW; ++w) top = fmaxf(top, part_m[w][place]);
+    float sum = 0.f, o = 0.f;
+#pragma unroll
+    for (int w = 0; w < NW; ++w) {
+      // (a wave without a key for this place holds nothing)
+      const float f = part_m[w][place] == -INFINITY && part_l[w][place] == 0.f
+                          ? 0.f : expf(part_m[w][place] - top);
+      sum += part_l[w][place] * f;
+      o += part[w][place][e] * f;
+    }
+    out[(size_t)to * out_stride + (size_t)hd * D + e] = o * (1.0f / sum);
+  }
+}
+
 template <typename T, bool MODS>
 static void rows_launch(const void* q, int q_stride, const void* k_pool, const void* v_pool,
                         void* out, int out_stride, const int* row_pos, const int* row_seg,
@@ -395,6 +560,26 @@ extern "C" int kappai_paged_attention_rows_scored(
   if (on && ((mods->dist_bias && mods->dist_cols < 1) || mods->keep_first < 0))
     return (int)hipErrorInvalidValue;
   const kappai_score_mods m = on ? *mods : kappai_score_mods{0.f, nullptr, 0, nullptr, 0};
+  // Plain float32 scores over heads of whole 16s: the matrix cores.  What they do not take (worked-on
+  // scores, other head sizes, rows or pages that are not aligned to 16 bytes) and bfloat16 shapes
+  // that no tiled kernel takes go row by row.
+  if (!is_bf16 && !on && d % 16 == 0 && d <= 128 && ps % 4 == 0 && q_stride % 4 == 0 &&
+      (uintptr_t)q % 16 == 0 && (uintptr_t)k_pool % 16 == 0 && (uintptr_t)v_pool % 16 == 0) {
+    const int per = H / G, heads = per < 16 ? per : 16;
+    const dim3 grid(T, G * ((per + heads - 1) / heads));
+#define F32_ATT(NT)                                                                             \
+  case NT:                                                                                      \
+    hipLaunchKernelGGL(paged_attention_f32_kernel<NT>, grid, dim3((NT <= 4 ? 8 : 4) * WAVE), 0,  \
+                       stream, (const float*)q, q_stride, (const float*)k_pool,                 \
+                       (const float*)v_pool, (float*)out, out_stride, row_pos, row_seg,         \
+                       block_tables, max_blocks, T, H, G, ps, window, scale);                   \
+    break;
+    switch (d / 16) {
+      F32_ATT(1) F32_ATT(2) F32_ATT(3) F32_ATT(4) F32_ATT(5) F32_ATT(6) F32_ATT(7) F32_ATT(8)
+    }
+#undef F32_ATT
+    KAPPAI_RETURN_LAUNCH_STATUS();
+  }
 #define ROWS_ARGS q, q_stride, k_pool, v_pool, out, out_stride, row_pos, row_seg, block_tables, \
                   max_blocks, T, H, G, d, ps, window, scale, m, stream
   if (is_bf16) {

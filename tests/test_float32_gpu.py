@@ -1,0 +1,84 @@
+"""The 32-bit kernels at the sizes where their tiles, runs and places end: products against float64,
+and a row's bits whatever it is computed with; attention against the plain statement of it."""
+import math
+
+import pytest
+import torch
+
+import emulated_ops as ref
+from test_kernels_gpu import DEV, F32, close, ops, paged_case, rand  # noqa: F401
+
+pytestmark = pytest.mark.gpu
+
+
+# K of one chunk, of the two numbers of runs and with chunks left over, and no whole chunks; N around
+# the widths that blocks own
+@pytest.mark.parametrize("N,K", [(5, 128), (40, 2048), (2047, 2176), (2064, 4608), (33, 2050),
+                                 (130, 8192), (9216, 1024)])
+def test_a_rows_product_has_the_same_bits_in_every_batch(ops, N, K):  # noqa: F811
+    x, w, b = rand((300, K), F32, 61), rand((N, K), F32, 62), rand((N,), F32, 63)
+    want = x.double() @ w.double().T + b.double()
+    x, w, b = x.to(DEV), w.to(DEV), b.to(DEV)
+    whole = ops.linear(x, w, b)
+    close(whole, want, 3e-6, "all rows")
+    for M in (1, 8, 9, 16, 17, 32, 33, 64, 65, 129):
+        assert torch.equal(ops.linear(x[:M].contiguous(), w, b), whole[:M]), M
+    # rows that are not aligned to 16 bytes take element-wise loads, in the same order
+    off = torch.empty((8, K + 1), dtype=F32, device=DEV)
+    off[:, 1:] = x[:8]
+    assert torch.equal(ops.linear(off[:, 1:], w, b), whole[:8])
+
+
+ATTENTION = [
+    # H, G, d, page, held before, new rows, window
+    (16, 8, 64, 16, [0, 5, 300], [37, 1, 70], 0),
+    (2, 2, 16, 16, [0, 127, 128, 1000], [17, 1, 1, 16], 0),
+    (3, 1, 32, 8, [3, 0], [6, 33], 0),
+    (6, 1, 48, 4, [0, 19, 40], [9, 5, 1], 11),
+    (24, 1, 80, 16, [60, 2], [3, 20], 0),
+    (40, 2, 96, 16, [0, 90], [12, 2], 50),
+    (4, 4, 112, 16, [30, 0], [40, 1], 0),
+    (8, 2, 128, 32, [200, 0], [5, 66], 64),
+]
+
+
+@pytest.mark.parametrize("case", ATTENTION)
+def test_attention_float32(ops, case):  # noqa: F811
+    H, G, d, ps, before, new, window = case
+    c = paged_case(21, F32, H, G, d, ps, before, new)
+    held = {k: (v.to(DEV) if torch.is_tensor(v) else v) for k, v in c.items()}
+    cos = torch.zeros((max(a + n for a, n in zip(before, new)) + 1, 1), device=DEV)
+    ops.qk_norm_rope_store(held["qkv"], H, G, d, None, None, 1e-5, cos, cos, 0, 0, held["k_pool"],
+                           held["v_pool"], held["row_pos"], held["row_seg"], held["bt"], ps)
+
+    def run(rows):
+        q = held["qkv"][rows]
+        return ops.paged_attention(q, H, G, d, held["k_pool"], held["v_pool"],
+                                   held["row_pos"][rows], held["row_seg"][rows], held["bt"], ps,
+                                   d ** -0.5, window=window)
+
+    T = c["row_pos"].shape[0]
+    got = run(torch.arange(T, device=DEV))
+    want = ref.paged_attention(held["qkv"].cpu(), H, G, d, held["k_pool"].cpu(),
+                               held["v_pool"].cpu(), c["row_pos"], c["row_seg"], c["bt"], ps,
+                               d ** -0.5, window=window)
+    close(got, want, 6e-6, "attention")
+    for t in (0, T // 2, T - 1):           # a row alone: the same bits
+        assert torch.equal(run(torch.tensor([t], device=DEV))[0], got[t]), t
+
+
+@pytest.mark.parametrize("bad", [math.inf, math.nan])
+def test_a_later_rows_odd_value_stays_with_the_rows_that_see_it(ops, bad):  # noqa: F811
+    H, G, d, ps = 4, 2, 32, 16
+    c = paged_case(22, F32, H, G, d, ps, [0], [20])
+    held = {k: (v.to(DEV) if torch.is_tensor(v) else v) for k, v in c.items()}
+    held["qkv"][13, (H + G) * d + 5] = bad          # a value of row 13, kv head 0
+    cos = torch.zeros((21, 1), device=DEV)
+    ops.qk_norm_rope_store(held["qkv"], H, G, d, None, None, 1e-5, cos, cos, 0, 0, held["k_pool"],
+                           held["v_pool"], held["row_pos"], held["row_seg"], held["bt"], ps)
+    out = ops.paged_attention(held["qkv"], H, G, d, held["k_pool"], held["v_pool"],
+                              held["row_pos"], held["row_seg"], held["bt"], ps, d ** -0.5).cpu()
+    assert torch.isfinite(out[:13]).all() and not torch.isfinite(out[13:, 5]).any()
+    rest = torch.ones(H * d, dtype=torch.bool)
+    rest[[5, d + 5]] = False                        # the two heads on kv head 0
+    assert torch.isfinite(out[:, rest]).all()

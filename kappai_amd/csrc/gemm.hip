@@ -990,16 +990,6 @@ static void launch_block256(const bf16_t* A, const bf16_t* W, const float* bias,
                      n_rows_w, K, lda, ldc, tn, w_frag);
 }
 
-// The 256 x 256 form (one block a CU, 40-55 us per round of up to 256 blocks at K = 2048) against
-// the 128 x 128 form (two blocks a CU): from 140 blocks on when one round does it, and with more
-// rounds when the last one is not mostly idle (idle CU-rounds under 30 % of the blocks); from a
-// sweep of the layer shapes at 1024 to 8192 rows.
-static bool use_256_form(long blocks256) {
-  if (blocks256 <= 256) return blocks256 >= 140;
-  const long rem = blocks256 % 256;
-  return rem == 0 || (256 - rem) * 10 < 3 * blocks256;
-}
-
 // shape: 0 = chosen by size, 1 = 128x128 blocks of two waves, 2 = 256x128 blocks (tiles of 32
 // of K, two LDS buffers), 3 = 256x128 blocks (tiles of 64 of K, one LDS buffer), 4 = 256x256
 // blocks of the same kernel (tiles of 64 of K), 5 = the 256x256 kernel with one wave a SIMD, 6 = its
@@ -1014,13 +1004,11 @@ static void launch_tile(const bf16_t* A, const bf16_t* W, const float* bias, TO*
     const int big = ((M + 255) / 256) * ((n_rows_w + 127) / 128) * ksplit;
     const int blocks256 = ((M + 255) / 256) * ((n_rows_w + 255) / 256) * ksplit;
     // the one-wave-a-SIMD kernel when its 256 x 256 blocks fill most of the chip, its
-    // 128 x 128 form (two blocks a CU) below that
-    // 128 x 128 blocks that would each have a CU to themselves anyway, and a long K: the form
-    // with four LDS buffers (0.46 against 0.62-0.87 us per 64 of K; its start costs 2 us more)
+    // 128 x 128 forms below that (gemm_rules.h)
     const long blocks128 = (long)((M + 127) / 128) * ((n_rows_w + 127) / 128) * ksplit;
-    const bool deep = blocks128 <= 256 && K / ksplit >= 2048;
+    const bool deep = kappai_deep_form(blocks128, K / ksplit);
     // (up to 128 rows a block of 256 rows would be half empty)
-    shape = !fits ? (big >= 128 ? 3 : 1) : (M > 128 && use_256_form(blocks256)) ? 5 : deep ? 8 : 6;
+    shape = !fits ? (big >= 128 ? 3 : 1) : (M > 128 && kappai_use_256_form(blocks256)) ? 5 : deep ? 8 : 6;
     if (shape == 5 && EPI == 0) {
       // blocks of 256 rows x 192 columns when they fill their rounds and come to fewer rounds'
       // worth of work than 256 x 256 (in_proj of 2048 rows: 192 blocks of 256 x 256 leave 64 CUs
@@ -1029,7 +1017,7 @@ static void launch_tile(const bf16_t* A, const bf16_t* W, const float* bias, TO*
       // split into ranges) the 192 form was measured slower (2063 x 2048 x 7168: 88 against 74 us).
       const long blocks192 = (long)((M + 255) / 256) * ((n_rows_w + 191) / 192) * ksplit;
       const long r256 = (blocks256 + 255) / 256, r192 = (blocks192 + 255) / 256;
-      if (use_256_form(blocks192) && r192 * (192 + 16) < r256 * (256 + 16)) shape = 9;
+      if (kappai_use_256_form(blocks192) && r192 * (192 + 16) < r256 * (256 + 16)) shape = 9;
     }
   }
   if ((shape == 5 || shape == 6 || shape == 8 || shape == 9) && !fits) shape = 3;

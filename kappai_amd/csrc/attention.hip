@@ -439,12 +439,16 @@ __global__ __launch_bounds__((NT <= 4 ? 8 : 4) * WAVE) void paged_attention_f32_
   for (; st <= last; st += NW) {
     f32x4_t kn[NT], vn[NT];
     if (st + NW <= last) fetch(st + NW, kn, vn);
-    f32x4_t s = {0.f, 0.f, 0.f, 0.f};
+    // (four chains: a product waits 50 clocks for the one before it in its own)
+    f32x4_t part_s[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) part_s[e] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int j = 0; j < NT; ++j)
 #pragma unroll
       for (int e = 0; e < 4; ++e)
-        s = __builtin_amdgcn_mfma_f32_16x16x4f32(kv[j][e], qv[j][e], s, 0, 0, 0);
+        part_s[e] = __builtin_amdgcn_mfma_f32_16x16x4f32(kv[j][e], qv[j][e], part_s[e], 0, 0, 0);
+    f32x4_t s = (part_s[0] + part_s[1]) + (part_s[2] + part_s[3]);
     const int key0 = 16 * st + 4 * quad;       // this lane's scores: keys key0 .. key0 + 3, place r
     bool seen[4], odd = false;
     float top = -INFINITY;

@@ -129,10 +129,16 @@ __global__ __launch_bounds__((COLS == 8 ? RUNS / 2 : 8) * WAVE) void gemm_f32_sk
   const auto load_w = [&](int c, f32x4_t (&v)[F32_STEPS]) {
     load_chunk_f32<WHOLE>(w, min(c0 + c, chunks - 1), q, K, v);
   };
+  // (lanes without a row stay out: a masked load costs what its live lanes do)
+  const int live = SIDE ? r % 8 : r;
+#pragma unroll
+  for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+    for (int j = 0; j < F32_STEPS; ++j) av[mt][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
   const auto load_a = [&](int c) {
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt)
-      load_chunk_f32<WHOLE>(a[mt], min(c0 + c, chunks - 1), q, K, av[mt]);
+      if (mt * 16 + live < M) load_chunk_f32<WHOLE>(a[mt], min(c0 + c, chunks - 1), q, K, av[mt]);
   };
   const auto multiply = [&](int c) {
     if (!SIDE)
@@ -190,9 +196,10 @@ __global__ __launch_bounds__((COLS == 8 ? RUNS / 2 : 8) * WAVE) void gemm_f32_sk
 // this one is multiplied.  An XCD takes every eighth column of tiles and walks its rows of tiles, so W
 // is read into one L2 only.  Two waves a SIMD: a wave's chunk, run and whole sums stay in
 // vector registers, and one wave multiplies while the other waits for LDS.  825 rows: 9216 x 1024
-// 165 us (94 TFLOP/s; the instruction alone reaches 153), 3072 x 1024 75 us, 2048 x 1024 46 us.
+// 165 us (94 TFLOP/s; the instruction alone reaches 153), 3072 x 1024 66 us, 2048 x 1024 45, 1024 x 4608
+// 101 (with four waves a block of 64 x 64, one a SIMD: 75, 46 and 107).
 template <int WY, int WX, int TY, int TX, int BK, bool WHOLE>
-__global__ __launch_bounds__(WY * WX * WAVE) __attribute__((amdgpu_waves_per_eu(2, 2)))
+__global__ __launch_bounds__(WY * WX * WAVE) __attribute__((amdgpu_waves_per_eu(2)))
 void gemm_f32_block_kernel(
     const float* __restrict__ A, const float* __restrict__ W, const float* __restrict__ bias,
     float* __restrict__ C, int M, int N, int K, int lda, int ldc, int tiles_m) {
@@ -351,8 +358,8 @@ static void launch_f32(const float* A, const float* W, const float* bias, float*
                        M, N, K, lda, ldc, tm);
   } else {
     const int tm = tiles(M, 64);
-    hipLaunchKernelGGL((gemm_f32_block_kernel<2, 2, 2, 2, 64, WHOLE>),
-                       dim3(tiles(tiles(N, 64), 8) * 8 * tm), dim3(256), 0, stream, A, W, bias, C,
+    hipLaunchKernelGGL((gemm_f32_block_kernel<2, 4, 2, 1, 64, WHOLE>),
+                       dim3(tiles(tiles(N, 64), 8) * 8 * tm), dim3(512), 0, stream, A, W, bias, C,
                        M, N, K, lda, ldc, tm);
   }
 }

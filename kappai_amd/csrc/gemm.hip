@@ -396,7 +396,10 @@ __device__ __forceinline__ void store_out(bf16_t* p, float v) { *p = f32_to_bf16
 // 0 silu; 1 the tanh form of gelu, 0.5 g (1 + tanh(a)) with a = sqrt(2/pi) (g + 0.044715 g^3),
 // which is g * sigmoid(2 a) and so the same two instructions; 2 the clamped gate, g = min(g, limit),
 // u = clamp(u, -limit, limit), g sigmoid(slope g) (u + shift), whose three constants the gated
-// epilogues read where the others find a bias (a gated product has none).
+// epilogues read where the others find a bias; 3 silu behind biases, one float a row of W in W's own
+// order, which are added to both sums first and rounded as a product with biases stores its results
+// (with the gate a kernel of its own behind the product, a decode step of two rows paid 4.6 us more a
+// layer at 9,216 rows of W, a prompt step of 1,900 rows 30).
 #ifndef GATE_ACT
 #define GATE_ACT 0
 #endif
@@ -410,7 +413,14 @@ __device__ __forceinline__ float silu_f(float g) {
 }
 
 // What a gated epilogue makes of the sums of a gate row and an up row.
-__device__ __forceinline__ float gated_f(float g, float u, const float* __restrict__ consts) {
+// `row`: the gate row's number in W (the up row stands 16 further).
+__device__ __forceinline__ float gated_f(float g, float u, const float* __restrict__ consts,
+                                         int row) {
+#if GATE_ACT == 3
+  // (rounded as a product with biases stores its results)
+  g = to_f32(f32_to_bf16(g + consts[row]));
+  u = to_f32(f32_to_bf16(u + consts[row + 16]));
+#endif
 #if GATE_ACT == 2
   const float limit = consts[0], slope = consts[1], shift = consts[2];
   g = fminf(g, limit);
@@ -587,7 +597,7 @@ __global__ __launch_bounds__(WAVES_M * WAVES_N * WAVE)
           const float other = __shfl_xor(acc[i][j][v], 16, WAVE);
           const int gm = m0 + (wm * WM + i) * 32 + 8 * (v / 4) + 4 * (lane / 32) + v % 4;
           if (c < 16 && gm < M && gcol + c < N)
-            store_out(C + (size_t)gm * ldc + on, gated_f(acc[i][j][v], other, bias));
+            store_out(C + (size_t)gm * ldc + on, gated_f(acc[i][j][v], other, bias, gcol + c));
         }
       }
     return;
@@ -933,7 +943,9 @@ void gemm_bf16_block256_kernel(const bf16_t* __restrict__ A, const bf16_t* __res
           c = j * 16 + 8 * g + 4 * hh;
 #pragma unroll
           for (int e = 0; e < 4; ++e)
-            v4[e] = gated_f(acc[i][j][4 * g + e], acc[i][j][4 * g + 8 + e], bias);
+            // (columns past the end are not stored: any row that is there)
+            v4[e] = gated_f(acc[i][j][4 * g + e], acc[i][j][4 * g + 8 + e], bias,
+                            min(n0 + wn * WROWS_N + j * 32 + 8 * g + 4 * hh + e, N - 17));
         } else {
           c = j * 32 + 8 * g + 4 * hh;
 #pragma unroll
@@ -1327,7 +1339,7 @@ __global__ __launch_bounds__((NW < 16 ? NW + 1 : NW) * WAVE) void gemm_bf16_skin
           float up = red[0][MT + t][lane][v];
 #pragma unroll
           for (int w = 1; w < NW; ++w) up += red[w][MT + t][lane][v];
-          store_out(C + out_at(gm, gn), gated_f(sum, up * rs, bias));
+          store_out(C + out_at(gm, gn), gated_f(sum, up * rs, bias, (int)blockIdx.x * 32 + col));
         } else if (EPI == 2 || EPI == 3) {
           // where the other two gates of this channel lie: EPI 2 in row groups 1 and 2 of this
           // lane, EPI 3 the C gate 8 columns further in group 0 and the x gate in group 1
@@ -1735,7 +1747,7 @@ __global__ __launch_bounds__(NWN * NWK * WAVE) void gemm_bf16_shared_rows_kernel
       if (EPI == 1) {
         const int on = wrow0 / 2 + col;                 // 16 output columns a wave
         if (wrow0 + 16 + col < n_rows_w)
-          store_out(C + (size_t)gm * ldc + on, gated_f(sum[0][v], sum[1][v], bias));
+          store_out(C + (size_t)gm * ldc + on, gated_f(sum[0][v], sum[1][v], bias, wrow0 + col));
       } else {
 #pragma unroll
         for (int r = 0; r < 2; ++r) {
@@ -1957,10 +1969,11 @@ __global__ __launch_bounds__(R32_NWN * R32_NWK * WAVE) void gemm_bf16_rows32_ker
 #pragma unroll
         for (int g = 0; g < 2; ++g) {
           uint2 pk;
-          pk.x = pack_bf16x2(gated_f(sum[4 * g], sum[4 * g + 8], bias),
-                             gated_f(sum[4 * g + 1], sum[4 * g + 9], bias));
-          pk.y = pack_bf16x2(gated_f(sum[4 * g + 2], sum[4 * g + 10], bias),
-                             gated_f(sum[4 * g + 3], sum[4 * g + 11], bias));
+          const int row = wrow0 + 8 * g + 4 * hh;
+          pk.x = pack_bf16x2(gated_f(sum[4 * g], sum[4 * g + 8], bias, row),
+                             gated_f(sum[4 * g + 1], sum[4 * g + 9], bias, row + 1));
+          pk.y = pack_bf16x2(gated_f(sum[4 * g + 2], sum[4 * g + 10], bias, row + 2),
+                             gated_f(sum[4 * g + 3], sum[4 * g + 11], bias, row + 3));
           if constexpr (sizeof(TO) == 2)
             *reinterpret_cast<uint2*>(C + (size_t)gm * ldc + wrow0 / 2 + 8 * g + 4 * hh) = pk;
         }
@@ -2170,7 +2183,7 @@ extern "C" int kappai_gemm_bf16_gated(const void* A, const void* W, const void* 
                                       float scale_eps, int c_frag, const float* consts,
                                       hipStream_t stream) {
   if (M <= 0 || F <= 0) return 0;
-  if ((consts != nullptr) != (GATE_ACT == 2)) return (int)hipErrorInvalidValue;
+  if ((consts != nullptr) != (GATE_ACT >= 2)) return (int)hipErrorInvalidValue;
   if ((K % 8) || (lda % 8) || (F % 16)) return (int)hipErrorInvalidValue;
   if (force_kernel == 2 && M > 64) return (int)hipErrorInvalidValue;
   if (!frag_ok(W_frag, 2 * F, K) || (a_frag && (K % 32))) return (int)hipErrorInvalidValue;

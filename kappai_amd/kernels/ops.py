@@ -591,15 +591,22 @@ def _out_in_fragment_order(wanted: bool, M: int, N: int, force_kernel: int) -> b
 
 def linear_swiglu(x: torch.Tensor, weight: torch.Tensor, force_kernel: int = 0,
                   weight_frag: Optional[torch.Tensor] = None, out_fragment: bool = False,
-                  activation: int = 0, clamp: Optional["ClampedGate"] = None):
+                  activation: int = 0, clamp: Optional["ClampedGate"] = None,
+                  bias: Optional[torch.Tensor] = None):
     """``silu(x Wg^T) * (x Wu^T)`` in one kernel: ``weight`` [2F, K] holds the gate and up
     matrices interleaved by ``interleave_gate_up``; bfloat16 only.  Returns [M, F].  ``x`` may
     be ``ScaledRows`` or ``FragmentRows``.  ``out_fragment``: with 8 to 16 rows the result may
     come back as ``FragmentRows`` for the product that follows.  ``activation``: ``GLU_SILU`` (0)
     or ``GLU_GELU_TANH`` (1) in place of silu, or ``GLU_CLAMPED`` (2) with its constants ``clamp``;
-    the product kernels are built once per gate."""
+    the product kernels are built once per gate.  ``bias`` (silu only): float32 [2F] in the order of
+    ``weight``'s rows, added to both sums before the gate."""
     _need((activation == GLU_CLAMPED) == (clamp is not None),
           "linear_swiglu: the clamped gate and its constants")
+    if bias is not None:
+        _gpu("bias", bias, F32)
+        _need(activation == GLU_SILU and bias.shape == (weight.shape[0],),
+              "linear_swiglu: biases go with silu, one for every row of the matrix")
+        activation = _GLU_SILU_BIASED
     scale = None
     if isinstance(x, ScaledRows):
         if (force_kernel not in (0, 2) or weight.dtype != BF16 or weight.dim() != 2
@@ -637,7 +644,7 @@ def linear_swiglu(x: torch.Tensor, weight: torch.Tensor, force_kernel: int = 0,
         _c_int(lda), _c_int(F),
         _c_int(force_kernel), _c_int(a_frag),
         *(scale._scale_args() if scale is not None else _NO_SCALE), _c_int(1 if c_frag else 0),
-        _ptr(clamp.on(x.device) if clamp else None), _stream()), "gemm_bf16_gated")
+        _ptr(clamp.on(x.device) if clamp else bias), _stream()), "gemm_bf16_gated")
     return FragmentRows(out, M, None) if c_frag else out
 
 
@@ -1384,6 +1391,7 @@ GLU_SILU, GLU_GELU_TANH = 0, 1
 
 
 GLU_CLAMPED = 2
+_GLU_SILU_BIASED = 3        # (the build of the product kernels whose gated epilogues add biases)
 
 
 @dataclass(frozen=True)

@@ -36,8 +36,7 @@ class SwiGLU(FeedForward):
         """``activation``: what the gate passes through, "silu" or "gelu_tanh" (the tanh form of
         GELU): ``W_down (act(W_gate x + b_gate) * (W_up x + b_up)) + b_down``; or "clamped", the
         clamped gate with the constants ``clamp`` (``ops.ClampedGate``).  ``bias``: whether the three
-        maps have biases (the gate then runs as a kernel of its own behind the first product, which
-        adds the biases)."""
+        maps have biases."""
         n = {"gate": "w1", "up": "w3", "down": "w2"}
         n.update(names or {})
         if activation not in self.ACTIVATIONS:
@@ -49,6 +48,7 @@ class SwiGLU(FeedForward):
         self.activation, self.clamp = activation, clamp
         self.fused = False
         self.has_bias = bool(bias)
+        self.gate_bias = None          # the first product's biases in the order of its fused matrix
         self.gate_up = Linear([prefix + n["gate"], prefix + n["up"]], width, [hidden, hidden],
                               stage="matmul_ffn_gate_up", weight_suffix=weight_suffix, bias=bias,
                               bias_suffix=bias_suffix)
@@ -62,10 +62,14 @@ class SwiGLU(FeedForward):
         def interleaved(w):
             # the fused product wants gate and up rows in turns of 16
             self.fused = (w.dtype == torch.bfloat16 and self.hidden % ops.SWIGLU_GROUP == 0
-                          and self.width % 8 == 0 and not self.has_bias)
+                          and self.width % 8 == 0
+                          and (not self.has_bias or self.activation == "silu"))
             return ops.interleave_gate_up(w[:self.hidden], w[self.hidden:]) if self.fused else None
 
         self.gate_up.bind(tensors, arrange=interleaved)
+        if self.fused and self.has_bias:
+            b = self.gate_up.bias.reshape(-1, 1)
+            self.gate_bias = ops.interleave_gate_up(b[:self.hidden], b[self.hidden:]).reshape(-1)
         if self.clamp is not None and self.gate_up.weight.device.type == "cuda":
             self.clamp.on(self.gate_up.weight.device)      # (before any step is captured)
         self.down.bind(tensors)
@@ -75,13 +79,15 @@ class SwiGLU(FeedForward):
             with profile.scope("matmul_ffn_gate_up", self.gate_up.weight_bytes()):
                 act = ops.linear_swiglu(x, self.gate_up.weight, out_fragment=True,
                                         activation=self.ACTIVATIONS[self.activation],
-                                        clamp=self.clamp)
+                                        clamp=self.clamp,
+                                        **({} if self.gate_bias is None
+                                           else {"bias": self.gate_bias}))
             return self.down.forward(act, partial_sums=True, add_into=into)
         gate_up = self.gate_up.forward(x)
         with profile.scope("ffn_act"):
             act = (ops.swiglu(gate_up) if self.activation == "silu"
                    else ops.glu(gate_up, self.ACTIVATIONS[self.activation], self.clamp))
-        return self.down.forward(act, partial_sums=not self.has_bias, add_into=into)
+        return self.down.forward(act, partial_sums=True, add_into=into)
 
     def c_part(self, plan, view=None, shared_cache: bool = False):
         """The runner "feed_forward.swiglu" (csrc/engine_parts.hip) makes the same choices as

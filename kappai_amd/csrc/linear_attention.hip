@@ -751,6 +751,418 @@ extern "C" int kappai_matrix_state_scan(const float* qf, const float* kf, const 
 }
 
 // ---------------------------------------------------------------------------------------
+// The gated sum (MODE 0) and the delta rule (MODE 1) over long portions: chunks of 16 tokens on the
+// matrix cores, in 32 bits (v_mfma_f32_16x16x4_f32).  With D(i, j) the product of a chunk's decays
+// after token j up to token i (per key channel; D(i, i) = 1), S0 the state the chunk starts from and
+// every D a running product of numbers in [0, 1], never a quotient,
+//   P[i, j] = sum_r q_i k_j D(i, j)             (j <= i: the read-out sees the token's own write)
+//   u       = v                                                                 (MODE 0)
+//   u_i     = beta_i (v_i - sum_r k_i D(i, -1) S0 - sum_(j < i) (sum_r k_i k_j D(i, j)) u_j)
+//           = U_i - W_i S0       with U and W from one forward substitution      (MODE 1)
+//   o_i     = (q_i D(i, -1)) S0 + sum_j P[i, j] u_j
+//   S       = D(15, -1) S0 + sum_j (k_j D(15, j)) u_j^T.
+// Two kernels.  The first makes P, U, W, q D, k D and D(15, -1) of every (chunk, head) side by side;
+// what is left along the tokens is the second: a block walks a (segment, head, 16 columns), its four
+// waves sharing the state's rows (TPW tiles of 16 each, in the accumulators' layout, which is also
+// the layout of a right operand whose four k-places are rows 4 g + v), so that a chunk's chain is
+// 4 TPW products W S0, one exchange of partial sums through LDS and 4 TPW products that bring the
+// state on.  The chunks' operands are asked for two
+// chunks (four up to 64 key channels) ahead.
+// What bounds it: the walk's chain, about 0.33 us a chunk for the gated sum (no W S0, u waits for
+// nothing) and 0.52 for the delta rule, whose wave issues 95 instructions a chunk and waits for one
+// barrier; hence one address a chunk with fixed distances a lane, operands in the order they are
+// loaded, and registers only (a build that put the sums in the accumulation registers took 41 and 50
+// us for 1,200 tokens where this takes 25 and 39).  1,900 tokens of two requests, 64 x 64 a head: 8
+// heads 417 us on the walk along the tokens, 15.8 + 25 here; the delta rule, 16 heads, 381 us against
+// 36 + 39.  The first kernel works in double, which is rounded once where the second kernel's operands
+// are stored (in float it took 13.5 and 23 us): the root mean square error of the outputs against
+// exact arithmetic over 100 to 1,200 tokens is then 5.9e-8 to 1.15e-7 (gated sum; token by token 7.5e-8
+// to 1.22e-7) and 1.14 to 1.52e-7 (delta rule; 1.2 to 1.67e-7), where float gave up to 1.46 and 1.88e-7.
+// Beyond a segment's end q, k and beta count as 0 and the decay as 1; key channels beyond d as 0.
+// ---------------------------------------------------------------------------------------
+#define MSC_C 16
+typedef float f32x4_t __attribute__((ext_vector_type(4)));
+
+// The floats of a (chunk, head), each matrix in tiles of 16 x 16 that a wave of the second kernel
+// loads as 16 bytes a lane side by side: q D and, for the delta rule, W (tiles of 16 key channels; a
+// lane's i is its number % 16, its four channels 4 g + e), k D (the lane's channel, tokens 4 g + e),
+// u (tiles of 16 value channels; the lane's channel, tokens 4 g + e), D(15, -1) [DP], P (four pieces
+// of one float a lane: piece e, row i, token 4 g + e).
+struct MscLayout { int q, k, last, p, w, u, size; };
+__host__ __device__ static inline MscLayout msc_layout(int dp, int dv, int mode) {
+  MscLayout l;
+  l.q = 0; l.k = 16 * dp; l.last = 32 * dp; l.p = 33 * dp; l.w = l.p + 256;
+  l.u = l.w + (mode ? 16 * dp : 0);
+  l.size = l.u + (dv + 15) / 16 * 256;
+  return l;
+}
+// A segment that starts at row `first` has its chunks at first / 16 + its number, .. + 1, ..: no two
+// segments' chunks meet, and T / 16 + S places hold all of them, whatever the segments are.
+__device__ __forceinline__ int msc_slot0(int seg, int first) { return first / MSC_C + seg; }
+
+// The sum over 16 neighbouring lanes, as ks_sum<16>.
+template <int CTRL>
+__device__ __forceinline__ double msc_move(double v) {
+  return __hiloint2double(__float_as_int(dpp_move<CTRL>(__int_as_float(__double2hiint(v)))),
+                          __float_as_int(dpp_move<CTRL>(__int_as_float(__double2loint(v)))));
+}
+__device__ __forceinline__ double msc_sum16(double v) {
+  v += msc_move<0xB1>(v);
+  v += msc_move<0x4E>(v);
+  v += msc_move<0x141>(v);
+  return v + msc_move<0x140>(v);
+}
+
+template <int NT, int MODE, typename TV>
+__global__ __launch_bounds__(256, 3) void matrix_state_chunk_prep_kernel(
+    const float* __restrict__ qf, const float* __restrict__ kf, const float* __restrict__ af,
+    const float* __restrict__ bf, const TV* __restrict__ v, int v_stride,
+    const int* __restrict__ seg_start, int S, int H, int Hk, int d, int dv,
+    float* __restrict__ scratch) {
+  constexpr int DP = 16 * NT, RS = DP + 4, M = DP / 64;
+  __shared__ __attribute__((aligned(16))) float Qs[MSC_C][RS], Ks[MSC_C][RS], As[MSC_C][RS];
+  __shared__ __attribute__((aligned(16))) float Ps[MSC_C][MSC_C + 4];
+  __shared__ __attribute__((aligned(16))) double Ns[MSC_C][MSC_C + 2];    // [key row j][i]
+  __shared__ float Bs[MSC_C];
+  __shared__ int seg_sh[2];
+  const int slot = blockIdx.y, h = blockIdx.x, tid = threadIdx.x;
+  const int hk = h / (H / Hk);
+  if (tid == 0) seg_sh[0] = -1;
+  __syncthreads();
+  for (int s = tid; s < S; s += 256) {
+    const int first = seg_start[s], len = seg_start[s + 1] - first;
+    const int at = slot - msc_slot0(s, first);
+    if (at >= 0 && at * MSC_C < len) {
+      seg_sh[0] = first + at * MSC_C;
+      seg_sh[1] = min(MSC_C, len - at * MSC_C);
+    }
+  }
+  __syncthreads();
+  const int row0 = seg_sh[0], n = seg_sh[1];
+  if (row0 < 0) return;                          // (no segment has this chunk)
+  const MscLayout L = msc_layout(DP, dv, MODE);
+  float* rec = scratch + ((size_t)slot * H + h) * L.size;
+#pragma unroll
+  for (int m = 0; m < NT / 4; ++m) {
+    const int i = tid + 256 * m, row = i / (DP / 4), e = 4 * (i % (DP / 4));
+    float4 q = make_float4(0.f, 0.f, 0.f, 0.f), k = q, a = make_float4(1.f, 1.f, 1.f, 1.f);
+    if (row < n && e < d) {
+      const size_t at = ((size_t)(row0 + row) * Hk + hk) * d + e;
+      q = *reinterpret_cast<const float4*>(qf + at);
+      k = *reinterpret_cast<const float4*>(kf + at);
+      a = *reinterpret_cast<const float4*>(af + ((size_t)(row0 + row) * H + h) * d + e);
+    }
+    *reinterpret_cast<float4*>(&Qs[row][e]) = q;
+    *reinterpret_cast<float4*>(&Ks[row][e]) = k;
+    *reinterpret_cast<float4*>(&As[row][e]) = a;
+  }
+  if (MODE == 1 && tid < MSC_C) Bs[tid] = tid < n ? bf[(size_t)(row0 + tid) * H + h] : 0.f;
+  __syncthreads();
+  {
+    // thread (j, part): key row j, channels 4 part + 64 m; k_j D(i, j) runs along i
+    const int j = tid / 16, part = tid % 16;
+    double kd[4 * M];
+#pragma unroll
+    for (int m = 0; m < M; ++m)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) kd[4 * m + e] = Ks[j][4 * part + 64 * m + e];
+    const int wave_j = tid / WAVE * 4;           // (the wave's key rows: wave_j .. + 3)
+#pragma unroll 2
+    for (int i = wave_j; i < MSC_C; ++i) {
+      double p = 0.0, nn = 0.0;
+#pragma unroll
+      for (int m = 0; m < M; ++m) {
+        const int c = 4 * part + 64 * m;
+        const float4 q = *reinterpret_cast<const float4*>(&Qs[i][c]);
+        const float4 a = *reinterpret_cast<const float4*>(&As[i][c]);
+        const float qq[4] = {q.x, q.y, q.z, q.w}, aa[4] = {a.x, a.y, a.z, a.w};
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          kd[4 * m + e] *= (double)(i > j ? aa[e] : 1.f);
+          p = fma((double)qq[e], kd[4 * m + e], p);
+        }
+        if (MODE == 1) {
+          const float4 k = *reinterpret_cast<const float4*>(&Ks[i][c]);
+          const float kk[4] = {k.x, k.y, k.z, k.w};
+#pragma unroll
+          for (int e = 0; e < 4; ++e) nn = fma((double)kk[e], kd[4 * m + e], nn);
+        }
+      }
+      p = msc_sum16(p);
+      if (MODE == 1) nn = msc_sum16(nn);
+      if (part == 0) {
+        Ps[i][j] = (float)p;
+        if (MODE == 1) Ns[j][i] = nn;
+      }
+    }
+  }
+  __syncthreads();
+  {
+    const int i = tid % 16, j = tid % WAVE / 16 * 4 + tid / WAVE;
+    rec[L.p + tid] = j <= i ? Ps[i][j] : 0.f;
+  }
+  // a thread a column of W and u: x_i = beta_i (b_i - sum_(j < i) N[i][j] x_j)
+  const int dvp = (dv + 15) / 16 * 16;
+  for (int col = tid; col < DP + dvp; col += 256) {
+    double b[MSC_C];
+    const int tile = col / 16 * 256, at = col % 16;
+    if (col < DP) {
+      double run = 1.0;
+      float kd[MSC_C];
+      float* to = rec + L.q + tile + at / 4 * 64 + at % 4;
+#pragma unroll
+      for (int i = 0; i < MSC_C; ++i) {
+        run *= (double)As[i][col];
+        b[i] = (double)Ks[i][col] * run;
+        to[4 * i] = (float)((double)Qs[i][col] * run);
+      }
+      rec[L.last + col] = (float)run;
+      run = 1.0;
+#pragma unroll
+      for (int i = MSC_C - 1; i >= 0; --i) {
+        kd[i] = (float)((double)Ks[i][col] * run);
+        run *= (double)As[i][col];
+      }
+#pragma unroll
+      for (int i = 0; i < MSC_C; i += 4)
+        *reinterpret_cast<float4*>(rec + L.k + tile + 16 * i + 4 * at) =
+            make_float4(kd[i], kd[i + 1], kd[i + 2], kd[i + 3]);
+    } else {
+      const int c = col - DP;
+#pragma unroll
+      for (int i = 0; i < MSC_C; ++i)
+        b[i] = (i < n && c < dv)
+                   ? to_f32(v[(size_t)(row0 + i) * v_stride + (size_t)h * dv + c]) : 0.f;
+    }
+    if (MODE == 1) {
+      // (each x_j is taken out of all rows behind it at once; one column of N ahead, no more, so that
+      // the registers hold two of them and not sixteen)
+      double nj[2][MSC_C];
+      auto column = [&](int j) {
+#pragma unroll
+        for (int i = j / 2 * 2; i < MSC_C; i += 2) {
+          const double2 x = *reinterpret_cast<const double2*>(&Ns[j][i]);
+          nj[j & 1][i] = x.x; nj[j & 1][i + 1] = x.y;
+        }
+      };
+      column(0);
+#pragma unroll
+      for (int j = 0; j < MSC_C; ++j) {
+        if (j + 1 < MSC_C) column(j + 1);
+        b[j] *= (double)Bs[j];
+#pragma unroll
+        for (int i = j + 1; i < MSC_C; ++i) b[i] = fma(-nj[j & 1][i], b[j], b[i]);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+    if (col >= DP) {
+#pragma unroll
+      for (int i = 0; i < MSC_C; i += 4)
+        *reinterpret_cast<float4*>(rec + L.u + tile - 16 * DP + 16 * i + 4 * at) =
+            make_float4((float)b[i], (float)b[i + 1], (float)b[i + 2], (float)b[i + 3]);
+    } else if (MODE == 1) {
+      float* to = rec + L.w + tile + at / 4 * 64 + at % 4;
+#pragma unroll
+      for (int i = 0; i < MSC_C; ++i) to[4 * i] = (float)b[i];
+    }
+  }
+}
+
+// What a lane needs of a chunk, as loaded.
+template <int TPW>
+struct MscOperands {
+  float4 w[TPW], q[TPW], k[TPW], last[TPW], u;
+  float p;
+};
+
+template <int NT, int MODE>
+__global__ __launch_bounds__(256, 2) void matrix_state_chunk_walk_kernel(
+    const float* __restrict__ scratch, float* __restrict__ state,
+    const int* __restrict__ seg_start, const int* __restrict__ seg_pos0,
+    const int* __restrict__ seg_slot, int H, int d, int dv, float* __restrict__ out) {
+  constexpr int DP = 16 * NT, TPW = NT / 4;
+  constexpr int AHEAD = 4 / TPW;       // (what the registers hold without spilling)
+  __shared__ __attribute__((aligned(16))) float4 Ux[2][4][WAVE];       // partial W S0
+  __shared__ float Ox[2][4][4][WAVE];                                // [.][v][wave]: partial outputs
+  const int seg = blockIdx.z, h = blockIdx.x, c0 = blockIdx.y * 16;
+  const int lane = threadIdx.x % WAVE, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
+  const int g = lane / 16, i16 = lane % 16, c = c0 + i16;
+  const int first = seg_start[seg], last = seg_start[seg + 1];
+  if (last <= first) return;
+  const int n_chunks = (last - first + MSC_C - 1) / MSC_C;
+  const MscLayout L = msc_layout(DP, dv, MODE);
+  // one address a chunk, the same for all lanes, and a lane's distances from it
+  const char* next = (const char*)(scratch + ((size_t)msc_slot0(seg, first) * H + h) * L.size);
+  const size_t rec_bytes = (size_t)H * L.size * sizeof(float);
+  const unsigned tile0 = 4u * (wave * TPW * 256 + 4 * lane), last0 = 4u * (wave * TPW * 16 + 4 * g);
+  const unsigned at_w = 4 * L.w + tile0, at_q = 4 * L.q + tile0, at_k = 4 * L.k + tile0;
+  const unsigned at_last = 4 * L.last + last0, at_u = 4 * (L.u + 256 * blockIdx.y + 4 * lane);
+  const unsigned at_p = 4 * (L.p + 64 * wave + lane);
+  char* out_next = (char*)(out + ((size_t)first * H + h) * dv);
+  const size_t out_bytes = (size_t)MSC_C * H * dv * sizeof(float);
+  const unsigned at_out = 4u * ((4 * g + wave) * (unsigned)H * dv + c);
+  float* st = state + (((size_t)seg_slot[seg] * H + h) * dv + min(c, dv - 1)) * d;
+  const bool carry = seg_pos0[seg] > 0;
+  f32x4_t Sx[TPW];
+#pragma unroll
+  for (int t = 0; t < TPW; ++t) {
+    const int r = 16 * (wave * TPW + t) + 4 * g;
+    Sx[t] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    if (carry && r < d) Sx[t] = *reinterpret_cast<const f32x4_t*>(st + r);
+  }
+  typedef MscOperands<TPW> Operands;
+  auto load = [&](Operands& R, int n) {
+    // (the last chunk again where there is none)
+    auto four = [&](unsigned at) { return *reinterpret_cast<const float4*>(next + at); };
+#pragma unroll
+    for (int t = 0; t < TPW; ++t) {
+      if (MODE == 1) R.w[t] = four(at_w + 1024 * t);
+      R.q[t] = four(at_q + 1024 * t);
+      R.k[t] = four(at_k + 1024 * t);
+      R.last[t] = four(at_last + 64 * t);
+    }
+    R.u = four(at_u);
+    R.p = *reinterpret_cast<const float*>(next + at_p);
+    if (n + 1 < n_chunks) next += rec_bytes;
+  };
+  // the sums of the oldest chunk's outputs not stored yet (`rows` of them): wave w stores rows 4 g + w
+  auto flush = [&](int par, int rows) {
+    float o = Ox[par][wave][0][lane];
+#pragma unroll
+    for (int w = 1; w < 4; ++w) o += Ox[par][wave][w][lane];
+    if (4 * g + wave < rows && c < dv) *reinterpret_cast<float*>(out_next + at_out) = o;
+    out_next += out_bytes;
+  };
+  auto barrier = [&]() {
+    // (only LDS is exchanged: loads of later chunks stay in flight)
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+  };
+  auto work = [&](const Operands& R, int n) {
+    const int par = n & 1;
+    float u[4] = {R.u.x, R.u.y, R.u.z, R.u.w};
+    f32x4_t o = {0.f, 0.f, 0.f, 0.f};
+    if (MODE == 1) {
+      f32x4_t pa = {0.f, 0.f, 0.f, 0.f}, pb = pa;
+#pragma unroll
+      for (int t = 0; t < TPW; ++t) {
+        const float a[4] = {R.w[t].x, R.w[t].y, R.w[t].z, R.w[t].w};
+        pa = __builtin_amdgcn_mfma_f32_16x16x4f32(a[0], Sx[t][0], pa, 0, 0, 0);
+        pb = __builtin_amdgcn_mfma_f32_16x16x4f32(a[1], Sx[t][1], pb, 0, 0, 0);
+        pa = __builtin_amdgcn_mfma_f32_16x16x4f32(a[2], Sx[t][2], pa, 0, 0, 0);
+        pb = __builtin_amdgcn_mfma_f32_16x16x4f32(a[3], Sx[t][3], pb, 0, 0, 0);
+      }
+      Ux[par][wave][lane] = make_float4(pa[0] + pb[0], pa[1] + pb[1], pa[2] + pb[2], pa[3] + pb[3]);
+    }
+#pragma unroll
+    for (int t = 0; t < TPW; ++t) {
+      const float a[4] = {R.q[t].x, R.q[t].y, R.q[t].z, R.q[t].w};
+#pragma unroll
+      for (int e = 0; e < 4; ++e) o = __builtin_amdgcn_mfma_f32_16x16x4f32(a[e], Sx[t][e], o, 0, 0, 0);
+    }
+    barrier();
+    if (MODE == 1) {
+#pragma unroll
+      for (int w = 0; w < 4; ++w) {
+        const float4 x = Ux[par][w][lane];
+        u[0] -= x.x; u[1] -= x.y; u[2] -= x.z; u[3] -= x.w;
+      }
+    }
+#pragma unroll
+    for (int t = 0; t < TPW; ++t) {
+      const float a[4] = {R.k[t].x, R.k[t].y, R.k[t].z, R.k[t].w};
+      const float f[4] = {R.last[t].x, R.last[t].y, R.last[t].z, R.last[t].w};
+#pragma unroll
+      for (int e = 0; e < 4; ++e) Sx[t][e] *= f[e];
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        Sx[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[e], u[e], Sx[t], 0, 0, 0);
+    }
+    const int wl = threadIdx.x / WAVE;           // (a value a lane: moves, not branches)
+    const float uw = wl & 2 ? (wl & 1 ? u[3] : u[2]) : (wl & 1 ? u[1] : u[0]);
+    o = __builtin_amdgcn_mfma_f32_16x16x4f32(R.p, uw, o, 0, 0, 0);
+    if (n > 0) flush(par ^ 1, MSC_C);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) Ox[par][e][wave][lane] = o[e];
+  };
+  Operands ring[AHEAD];
+#pragma unroll
+  for (int j = 0; j < AHEAD; ++j) load(ring[j], j);
+  int n = 0;
+  for (; n + AHEAD <= n_chunks; n += AHEAD) {
+#pragma unroll
+    for (int j = 0; j < AHEAD; ++j) {
+      work(ring[j], n + j);
+      __builtin_amdgcn_sched_barrier(0);
+      load(ring[j], n + j + AHEAD);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  }
+#pragma unroll
+  for (int j = 0; j < AHEAD - 1; ++j)
+    if (n + j < n_chunks) work(ring[j], n + j);
+  barrier();
+  flush((n_chunks - 1) & 1, last - first - (n_chunks - 1) * MSC_C);
+  if (c < dv) {
+#pragma unroll
+    for (int t = 0; t < TPW; ++t) {
+      const int r = 16 * (wave * TPW + t) + 4 * g;
+      if (r < d) *reinterpret_cast<f32x4_t*>(st + r) = Sx[t];
+    }
+  }
+}
+
+template <int NT, int MODE, typename TV>
+static void msc_launch(const float* qf, const float* kf, const float* af, const float* bf,
+                       const TV* v, int v_stride, float* state, const int* seg_start,
+                       const int* seg_pos0, const int* seg_slot, int T, int S, int H, int Hk,
+                       int d, int dv, float* scratch, float* out, hipStream_t stream) {
+  hipLaunchKernelGGL((matrix_state_chunk_prep_kernel<NT, MODE, TV>), dim3(H, T / MSC_C + S),
+                     dim3(256), 0, stream, qf, kf, af, bf, v, v_stride, seg_start, S, H, Hk, d, dv,
+                     scratch);
+  hipLaunchKernelGGL((matrix_state_chunk_walk_kernel<NT, MODE>), dim3(H, (dv + 15) / 16, S),
+                     dim3(256), 0, stream, scratch, state, seg_start, seg_pos0, seg_slot, H, d, dv,
+                     out);
+}
+
+// Floats of scratch the chunked form needs (0: it does not take these sizes).
+extern "C" long long kappai_matrix_state_chunks_scratch(int T, int S, int d, int dv, int H,
+                                                        int mode) {
+  if (T < 1 || S < 1 || d < 1 || d > 128 || d % 4 || dv < 1 || H < 1 || H > 65535 || S > 65535 ||
+      T / MSC_C + S > 65535 || (dv + 15) / 16 > 65535 || mode < 0 || mode > 1)
+    return 0;
+  return (long long)(T / MSC_C + S) * H * msc_layout(d <= 64 ? 64 : 128, dv, mode).size;
+}
+
+// As kappai_matrix_state_scan, modes 0 and 1, in chunks; qf, kf, af and state start on 16 bytes.
+extern "C" int kappai_matrix_state_chunks(const float* qf, const float* kf, const float* af,
+                                          const float* bf, const void* v, int v_stride,
+                                          int v_is_bf16, float* state, const int* seg_start,
+                                          const int* seg_pos0, const int* seg_slot, int T, int S,
+                                          int H, int Hk, int d, int dv, int mode, float* scratch,
+                                          float* out, hipStream_t stream) {
+  if (T <= 0 || S <= 0) return 0;
+  if (Hk < 1 || H % Hk || (mode == 1) != (bf != nullptr) || !scratch ||
+      !kappai_matrix_state_chunks_scratch(T, S, d, dv, H, mode) ||
+      ((uintptr_t)qf | (uintptr_t)kf | (uintptr_t)af | (uintptr_t)state | (uintptr_t)scratch) % 16)
+    return (int)hipErrorInvalidValue;
+#define MSC_CASE(NT_, MODE_, TV_)                                                                   \
+  msc_launch<NT_, MODE_, TV_>(qf, kf, af, bf, (const TV_*)v, v_stride, state, seg_start, seg_pos0, \
+                              seg_slot, T, S, H, Hk, d, dv, scratch, out, stream)
+#define MSC_TYPED(NT_, MODE_) \
+  if (v_is_bf16) MSC_CASE(NT_, MODE_, bf16_t); else MSC_CASE(NT_, MODE_, float)
+  if (d <= 64) {
+    if (mode) { MSC_TYPED(4, 1); } else { MSC_TYPED(4, 0); }
+  } else {
+    if (mode) { MSC_TYPED(8, 1); } else { MSC_TYPED(8, 0); }
+  }
+#undef MSC_TYPED
+#undef MSC_CASE
+  KAPPAI_RETURN_LAUNCH_STATUS();
+}
+
+// ---------------------------------------------------------------------------------------
 // One fixed decay a head, S <- lam S + k v^T, o = S^T q, over long portions in chunks of rows.
 // A constant decay has a form without a chain along the tokens and without a division: inside
 // a chunk of n rows  o_i = sum_(j <= i) lam^(i - j) (q_i . k_j) v_j + lam^(i + 1) S0^T q_i  with

@@ -2424,6 +2424,9 @@ SCAN_FORMS = {"auto": 0, "wave": 1, "block": 2}
 
 
 DECAY_KINDS = {"softplus": 0, "double_exp": 1, "fixed": 2}
+MATRIX_STATE_CHUNK_ROWS = 16    # the rows of a chunk of the gated sum and the delta rule
+# the most scratch their chunked form takes (2 GiB); steps that would need more walk the tokens
+MATRIX_STATE_SCRATCH_FLOATS = 1 << 29
 FIXED_DECAY_CHUNK_ROWS = 32     # the most rows of a chunk the chunked form of a fixed decay takes
 
 
@@ -2463,7 +2466,11 @@ def matrix_state_recurrence(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
     ``chunks`` [n, 3] = (segment, first row, rows <= ``chunk_rows`` <= 32) with ``seg_chunk0``
     [S + 1], as for ``mingru_scan``: a fixed decay (no ``beta``, no ``bonus``, H == Hk) and the
     form with a ``bonus`` are then worked chunk by chunk in three passes, with no chain along the
-    tokens of a chunk (every factor is a product of decays, none is divided by one)."""
+    tokens of a chunk (every factor is a product of decays, none is divided by one).
+
+    ``chunk_rows`` = ``MATRIX_STATE_CHUNK_ROWS`` without ``chunks``: the forms without a bonus are
+    worked in chunks of 16 rows on the matrix cores (float32), which pays from a few chunks a
+    segment on; key sizes that are multiples of four up to 128, others walk the tokens."""
     H, Hk, d, dv = n_heads, n_qk_heads, dim, vdim
     _need(form in SCAN_FORMS, lambda: f"matrix_state_recurrence: form {form!r}")
     _need(decay in DECAY_KINDS and (z is None) == (decay == "fixed")
@@ -2544,6 +2551,19 @@ def matrix_state_recurrence(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
             _c_int(T), _c_int(S), _c_int(H), _c_int(d), _c_int(dv), _ptr(carry), _ptr(out),
             _stream()), "fixed_decay_chunks")
         return out
+    if chunk_rows == MATRIX_STATE_CHUNK_ROWS and chunks is None and mode < 2 and form == "auto":
+        lib.kappai_matrix_state_chunks_scratch.restype = ctypes.c_longlong
+        floats = lib.kappai_matrix_state_chunks_scratch(_c_int(T), _c_int(S), _c_int(d), _c_int(dv),
+                                                        _c_int(H), _c_int(mode))
+        if 0 < floats <= MATRIX_STATE_SCRATCH_FLOATS and state.data_ptr() % 16 == 0:
+            scratch = torch.empty(floats, dtype=F32, device=dev)
+            check(lib.kappai_matrix_state_chunks(
+                _ptr(qf), _ptr(kf), _ptr(af), _ptr(bf), _ptr(values), _c_int(values.stride(0)),
+                _c_int(_is_bf16(values.dtype)), _ptr(state), _ptr(seg_start), _ptr(seg_pos0),
+                _ptr(seg_slot), _c_int(T), _c_int(S), _c_int(H), _c_int(Hk), _c_int(d),
+                _c_int(dv), _c_int(mode), _ptr(scratch), _ptr(out), _stream()),
+                "matrix_state_chunks")
+            return out
     check(lib.kappai_matrix_state_scan(
         _ptr(qf), _ptr(kf), _ptr(af), _ptr(bonus if bonus is not None else bf), _ptr(values),
         _c_int(values.stride(0)),

@@ -74,3 +74,14 @@ SCAN_CHUNKS_FROM_ROWS = 64
 # The state-space recurrence: segments of up to this many rows are walked token by token, longer
 # ones (in bfloat16) worked in chunks on the matrix cores.
 STATE_SPACE_CHUNKS_FROM_ROWS = 16
+
+# The gated sum and the delta rule (a matrix of state a head, a decay per key channel) walk the tokens
+# at 0.26 to 0.45 us each, however many segments walk side by side; in chunks of 16 rows a token takes
+# 0.03 to 0.08 us, but a segment of any length costs at least one chunk, 0.1 to 0.8 us of the whole
+# chip.  Hence chunks from a longest segment of 24 rows and 2 more a segment on.  Walk / chunks in us
+# with 16 heads of 64 x 64, delta rule: one segment of 24 rows 16.1 / 16.1, of 64 29.2 / 17.5, of 2,048
+# 743 / 121; 8 segments of 32 22.2 / 22.0, of 48 29.1 / 24.8; 64 of 32 75 / 85; 60 single rows beside
+# one of 128 51 / 44.  Of 128 x 128: 60 single rows beside one of 128 68.5 / 74.8, of 160 80.3 / 75.2.
+# The gated sum gains more at every one of these.
+MATRIX_STATE_CHUNKS_FROM_ROWS = 24
+MATRIX_STATE_CHUNKS_FROM_ROWS_A_SEGMENT = 2

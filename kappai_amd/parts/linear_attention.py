@@ -53,6 +53,14 @@ def _columns(proj: torch.Tensor, start: int, n: int) -> torch.Tensor:
     return view
 
 
+def _chunk_rows(batch) -> int:
+    """How many rows a chunk of the recurrences with a decay per key channel takes; 0: they walk the
+    tokens one by one."""
+    chunked = (batch.max_segment_rows >= tuning.MATRIX_STATE_CHUNKS_FROM_ROWS
+               + tuning.MATRIX_STATE_CHUNKS_FROM_ROWS_A_SEGMENT * batch.seg_slot.shape[0])
+    return ops.MATRIX_STATE_CHUNK_ROWS if chunked else 0
+
+
 class GatedLinearAttention(Mixer):
     def __init__(self, prefix: str, width: int, num_heads: int, dim: int, vdim: int, tau: float,
                  decay_rank: int, norm_eps: float, dtype: torch.dtype, names=None,
@@ -102,7 +110,8 @@ class GatedLinearAttention(Mixer):
         with profile.scope("scan"):
             o = ops.matrix_state_recurrence(
                 proj, proj[:, o_k:], proj[:, o_v:], z, H, H, d, dv, self.rate, self.decay_bias,
-                -1.0, d ** -0.5, cache.state, batch.seg_start, batch.seg_pos0, batch.seg_slot)
+                -1.0, d ** -0.5, cache.state, batch.seg_start, batch.seg_pos0, batch.seg_slot,
+                chunk_rows=_chunk_rows(batch))
             y = ops.head_norm_gate(o, self.norm_w, self.norm_eps, proj[:, o_g:], ops.GATE_SILU,
                                    H, dv, self.dtype)
         return self.out.forward(y, partial_sums=True)
@@ -347,7 +356,8 @@ class GatedDeltaRule(Mixer):
             o = ops.matrix_state_recurrence(
                 qkv, qkv[:, G * d:], qkv[:, 2 * G * d:], z, H, G, d, dv, self.rate, self.dt_bias,
                 1.0, d ** -0.5, state, batch.seg_start, batch.seg_pos0, batch.seg_slot,
-                beta=proj[:, C + self.ra + self.rg:], unit_qk=True, unit_eps=self.unit_eps)
+                beta=proj[:, C + self.ra + self.rg:], unit_qk=True, unit_eps=self.unit_eps,
+                chunk_rows=_chunk_rows(batch))
             y = ops.head_norm_gate(o, self.norm_w, self.norm_eps, gate, ops.GATE_SIGMOID, H, dv,
                                    self.dtype)
         return self.out.forward(y, partial_sums=True)

@@ -859,6 +859,216 @@ __global__ __launch_bounds__(8 * WAVE) void attn_prefill_shared_kernel(
 #endif
 
 // ---------------------------------------------------------------------------------------
+// prefill at head size 256, key tiles shared by four query heads of a kv head
+// ---------------------------------------------------------------------------------------
+// One block = one q tile (32 rows) x four query heads of one kv head, two waves a head: both make the
+// scores, each half of the output's columns (with all of them in one wave the registers spill and a
+// SIMD has no second wave to work while the first is at its exponentials).  A tile of K (32 keys x d)
+// and of V^T comes from global memory once, straight into LDS (global_load_lds, three buffers, two
+// tiles ahead), in the places the kernel above gives them.  A wave alone with its head, which is the other way, reads
+// every operand from the caches itself and has no registers to ask ahead: it waits about 3 us for a
+// tile, whatever else runs.  Two portions of 1,900 rows in all, 16 heads on one kv head: 127 -> 82 us;
+// what bounds it now is a wave's own chain over a tile (scores, exponentials, output), two waves a
+// SIMD, about 2 us for each of the longest portion's 38 tiles.  The arithmetic is that wave's to the bit: the accumulators are only
+// left alone where they would have been multiplied by one.
+#if HEAD_DIM == 256
+#define PH_NBUF 3
+template <int N> struct PhBuf { static constexpr int value = N; };
+__global__ __launch_bounds__(8 * WAVE) void attn_prefill_heads_kernel(
+    const bf16_t* __restrict__ q, int q_stride, const bf16_t* __restrict__ k_pool,
+    const bf16_t* __restrict__ vt_pool, bf16_t* __restrict__ out, int out_stride,
+    const int* __restrict__ q_tiles, const int* __restrict__ row_pos,
+    const int* __restrict__ block_tables, int max_blocks, int H, int G, int ps, int window,
+    float scale, const float* __restrict__ sink) {
+  constexpr int ROWB = HEAD_DIM * 2;                                              // bytes of a key's row
+  constexpr int KTILE = 32 * ROWB, VGROUP = HEAD_DIM * 32, BUF = KTILE + 2 * VGROUP;   // bytes
+  constexpr int NL = 4, MT = P_MT / 2;       // loads a wave issues a tile; row tiles of its half of O^T
+  __shared__ __attribute__((aligned(1024))) char lds[PH_NBUF * BUF];
+  const int tile = gridDim.x - 1 - blockIdx.x;      // (later tiles have more keys: they go first)
+  const int lane = threadIdx.x % WAVE;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
+  const int rep = H / G, quads = rep / 4;
+  const int g = blockIdx.y / quads, h = g * rep + (blockIdx.y % quads) * 4 + wave % 4;
+  const int mt0 = wave / 4 * MT;
+  const int seg = q_tiles[4 * tile], r0 = q_tiles[4 * tile + 1], nr = q_tiles[4 * tile + 2];
+  const int col = lane % 32, hh = lane / 32;
+  const int* bt = block_tables + (size_t)seg * max_blocks;
+  const int pos_first = row_pos[r0], pos_last = pos_first + nr - 1;
+  const bool row_ok = col < nr;
+  const int my_pos = row_ok ? pos_first + col : -1;
+  const int my_lo = kappai_first_key(my_pos, window);
+  const int lo_tile = kappai_first_key(pos_first, window);
+  const int lo_last = kappai_first_key(pos_last, window);
+
+  bf16x8_t qf[P_KS];
+  {
+    const bf16_t* qr = q + (size_t)(r0 + (row_ok ? col : 0)) * q_stride + (size_t)h * HEAD_DIM;
+#pragma unroll
+    for (int ks = 0; ks < P_KS; ++ks) {
+      u32x4_t v = {0u, 0u, 0u, 0u};
+      if (row_ok) v = *reinterpret_cast<const u32x4_t*>(qr + 16 * ks + 8 * hh);
+      qf[ks] = as_frag(v);
+    }
+  }
+  f32x16_t o[MT];
+#pragma unroll
+  for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+    for (int v = 0; v < 16; ++v) o[mt][v] = 0.f;
+  float m_run = -INFINITY, l_run = 0.f;
+  const float sc = scale * LOG2E;
+  const int kbase = (lo_tile / 32) * 32, n_steps = (pos_last - kbase) / 32 + 1;
+  // what this lane brings: waves 0 to 3 eight rows of K each (two a load), waves 4 to 7 half a 16-key
+  // group of V^T (32 rows a load); a wave's keys lie in one page.  A group past the last key (or given
+  // back by the window) is read from the pool's first page and masked when it is used.
+  const int part = wave % 4, half = part % 2, v_half = lane % 2;
+  int nx_key = kbase + 16 * (part / 2);
+  // a lane's first place behind the page's address in bytes; the others follow from it
+  const unsigned k_chunk = lane % 32, k_row = 8 * half + lane / 32, v_row = 128 * half + lane / 2;
+  const unsigned at0 = wave < 4 ? k_row * ROWB
+                                : v_row * ps * 2 + 16 * (v_half ^ ((v_row >> 3) & 1));
+  auto issue = [&](auto buf_c) {
+    char* buf = lds + decltype(buf_c)::value * BUF;
+    const int page = nx_key <= pos_last ? max(bt[min(nx_key / ps, max_blocks - 1)], 0) : 0;
+    const size_t head = (size_t)page * G + g;
+    const int off = nx_key % ps;
+    // (rows 32 apart have the same swapped halves)
+    const char* from = wave < 4 ? (const char*)(k_pool + (head * ps + off) * HEAD_DIM)
+                                : (const char*)(vt_pool + head * HEAD_DIM * ps + off);
+    const unsigned step = wave < 4 ? 2 * ROWB : 64 * ps;
+    char* to = wave < 4 ? buf + 8 * part * ROWB : buf + KTILE + (part / 2) * VGROUP + half * 128 * 32;
+#pragma unroll
+    for (int i = 0; i < NL; ++i) {
+      const unsigned swap = wave < 4 ? 16 * (k_chunk ^ ((k_row + 2 * i) & 15)) : 0;
+      __builtin_amdgcn_global_load_lds(
+          (const __attribute__((address_space(1))) void*)(from + i * step + (at0 + swap)),
+          (__attribute__((address_space(3))) void*)(to + 1024 * i), 16, 0, 0);
+    }
+    nx_key += 32;
+  };
+  auto work = [&](auto buf_c, int kb) {
+    const char* buf = lds + decltype(buf_c)::value * BUF;
+    // (a lane's places in LDS are made anew for every tile: kept over the loop for three buffers they
+    // are more registers than there are)
+    int at = col;
+    asm volatile("" : "+v"(at));
+    f32x16_t s;
+#pragma unroll
+    for (int v = 0; v < 16; ++v) s[v] = 0.f;
+#pragma unroll
+    for (int ks = 0; ks < P_KS; ++ks) {
+      const u32x4_t kf = *reinterpret_cast<const u32x4_t*>(
+          buf + at * ROWB + (((2 * ks + hh) ^ (at & 15)) * 16));
+      s = __builtin_amdgcn_mfma_f32_32x32x16_bf16(as_frag(kf), qf[ks], s, 0, 0, 0);
+      // (fences here and below: left to itself the compiler reads a whole tile ahead and spills, and
+      // a reload waits for the tiles on their way)
+      if (ks % 4 == 3) __builtin_amdgcn_sched_barrier(0);
+    }
+    const bool full = kb >= lo_last && kb + 31 <= pos_first;
+    // lane holds, for query `col`, keys kb + 8*(v/4) + 4*hh + v%4
+    float mloc = -INFINITY;
+    if (full) {
+#pragma unroll
+      for (int v = 0; v < 16; ++v) mloc = fmaxf(mloc, s[v]);
+      mloc *= sc;           // sc > 0: scaling commutes with the maximum
+    } else {
+#pragma unroll
+      for (int v = 0; v < 16; ++v) {
+        const int key = kb + 8 * (v / 4) + 4 * hh + v % 4;
+        s[v] = key <= my_pos && key >= my_lo ? s[v] : -INFINITY;
+        mloc = fmaxf(mloc, s[v] * sc);
+      }
+    }
+    mloc = fmaxf(mloc, other_half(mloc));
+    const float m_new = fmaxf(m_run, mloc);
+    float corr = 1.0f;
+    if (__builtin_amdgcn_ballot_w64(m_new != m_run) != 0) {
+      corr = fast_exp2(m_run - (m_new == -INFINITY ? 0.f : m_new));
+#pragma unroll
+      for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+        for (int v = 0; v < 16; ++v) o[mt][v] *= corr;
+      m_run = m_new;
+    }
+    const float m_safe = m_run == -INFINITY ? 0.f : m_run;
+    float lsum = 0.f;
+#pragma unroll
+    for (int v = 0; v < 16; ++v) {
+      s[v] = fast_exp2(fmaf(s[v], sc, -m_safe));
+      lsum += s[v];
+    }
+    lsum += other_half(lsum);
+    l_run = fmaf(l_run, corr, lsum);
+    auto output = [&](auto masked_c) {
+#pragma unroll
+      for (int st = 0; st < 2; ++st) {
+        const u32x4_t pw = {pack_bf16(s[8 * st + 0], s[8 * st + 1]),
+                            pack_bf16(s[8 * st + 2], s[8 * st + 3]),
+                            pack_bf16(s[8 * st + 4], s[8 * st + 5]),
+                            pack_bf16(s[8 * st + 6], s[8 * st + 7])};
+        const bf16x8_t pf = as_frag(pw);
+        int keep_a = 0, keep_b = 0;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const int ka = kb + 16 * st + 4 * hh + i, kbb = ka + 8;
+          if (ka >= lo_tile && ka <= pos_last) keep_a |= 1 << i;
+          if (kbb >= lo_tile && kbb <= pos_last) keep_b |= 1 << i;
+        }
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt) {
+          const int sw = ((at >> 3) & 1) * 16;      // (this row's halves are swapped)
+          const char* vp = buf + KTILE + st * VGROUP + (32 * (mt0 + mt) + at) * 32 + 8 * hh;
+          u32x2_t va = *reinterpret_cast<const u32x2_t*>(vp + sw);
+          u32x2_t vb = *reinterpret_cast<const u32x2_t*>(vp + (16 - sw));
+          // what lies in LDS for keys outside the tile's range is not cache content: zero it
+          if (decltype(masked_c)::value) {
+            va = mask4(va, keep_a);
+            vb = mask4(vb, keep_b);
+          }
+          o[mt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+              as_frag((u32x4_t){va.x, va.y, vb.x, vb.y}), pf, o[mt], 0, 0, 0);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    };
+    if (full) output(PhBuf<0>{});
+    else output(PhBuf<1>{});
+  };
+  auto step = [&](auto buf_c, int it) {
+    __builtin_amdgcn_sched_barrier(0);
+    constexpr int B = decltype(buf_c)::value;
+    // this step's tile has landed (this wave's part; the barrier makes it everybody's)
+    if (it + 1 < n_steps) __builtin_amdgcn_s_waitcnt(0x0F70 | NL);
+    else __builtin_amdgcn_s_waitcnt(0x0F70);
+    __builtin_amdgcn_s_barrier();     // no fence: a fence would wait for the loads in flight
+    // step it + 2 goes into the buffer of step it - 1: everybody is done with it
+    if (it + 2 < n_steps) issue(PhBuf<(B + 2) % PH_NBUF>{});
+    work(buf_c, kbase + 32 * it);
+  };
+  issue(PhBuf<0>{});
+  if (n_steps > 1) issue(PhBuf<1>{});
+  for (int it = 0; it < n_steps; it += PH_NBUF) {
+    step(PhBuf<0>{}, it);
+    if (it + 1 < n_steps) step(PhBuf<1>{}, it + 1);
+    if (it + 2 < n_steps) step(PhBuf<2>{}, it + 2);
+  }
+  if (!row_ok) return;
+  if (sink != nullptr && m_run != -INFINITY) l_run += fast_exp2(sink[h] * LOG2E - m_run);
+  const float inv = l_run > 0.f ? 1.0f / l_run : 0.f;
+  bf16_t* orow = out + (size_t)(r0 + col) * out_stride + (size_t)h * HEAD_DIM;
+#pragma unroll
+  for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+    for (int v4 = 0; v4 < 4; ++v4) {
+      const int dd = 32 * (mt0 + mt) + 8 * v4 + 4 * hh;   // four consecutive d: v = 4*v4 .. 4*v4+3
+      u32x2_t w = {pack_bf16(o[mt][4 * v4] * inv, o[mt][4 * v4 + 1] * inv),
+                   pack_bf16(o[mt][4 * v4 + 2] * inv, o[mt][4 * v4 + 3] * inv)};
+      *reinterpret_cast<u32x2_t*>(orow + dd) = w;
+    }
+}
+#endif
+
+// ---------------------------------------------------------------------------------------
 // decode: one row a request; columns are the query heads of one kv head (at most 16)
 // ---------------------------------------------------------------------------------------
 #define D_KS ((HEAD_DIM + 31) / 32)     // k-steps of S^T over d (32 each)
@@ -1589,6 +1799,16 @@ extern "C" int kappai_attn_prefill_scored(const void* q, int q_stride, const voi
 #if PG_OK
   if (shared) {
     hipLaunchKernelGGL(attn_prefill_shared_kernel, dim3(n_tiles, H / 4), dim3(8 * WAVE), 0, stream,
+                       (const bf16_t*)q, q_stride, (const bf16_t*)k_pool, (const bf16_t*)vt_pool,
+                       (bf16_t*)out, out_stride, q_tiles, row_pos, block_tables, max_blocks, H, G,
+                       ps, window, scale, sink);
+    KAPPAI_RETURN_LAUNCH_STATUS();
+  }
+#endif
+#if HEAD_DIM == 256
+  // (from the first tile on: a block's time is its own tiles', shorter than a wave's by itself)
+  if (variant == 0 && rep % 4 == 0) {
+    hipLaunchKernelGGL(attn_prefill_heads_kernel, dim3(n_tiles, H / 4), dim3(8 * WAVE), 0, stream,
                        (const bf16_t*)q, q_stride, (const bf16_t*)k_pool, (const bf16_t*)vt_pool,
                        (bf16_t*)out, out_stride, q_tiles, row_pos, block_tables, max_blocks, H, G,
                        ps, window, scale, sink);

@@ -110,3 +110,45 @@ def test_empty_and_refused(ops):  # noqa: F811
         assert (o - o2).abs().max() <= 2e-5 * o.abs().max() and (s - s2).abs().max() <= 2e-5 * s.abs().max()
         if d != 16:
             assert torch.equal(o, o2) and torch.equal(s, s2)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("H,Hk,d,dv", [(2, 1, 64, 24), (2, 2, 128, 16)])
+@pytest.mark.parametrize("what", ["v", "k", "q", "z", "beta"])
+@pytest.mark.parametrize("delta", [False, True])
+@pytest.mark.parametrize("bad", [float("inf"), float("nan")])
+def test_a_value_that_is_no_number_stays_with_its_token_and_those_behind_it(  # noqa: F811
+        ops, H, Hk, d, dv, what, delta, bad):
+    """The tokens before it, other segments and (for a value) other columns keep their bits; what is
+    finite on the walk is finite in chunks."""
+    if what == "beta" and not delta:
+        return
+    at, lens = 21, [40, 5]               # the sixth token of the second chunk
+    T = sum(lens)
+    g = torch.Generator().manual_seed(d + dv)
+    x = {n: torch.randn(T, c, generator=g) for n, c in
+         (("q", Hk * d), ("k", Hk * d), ("v", H * dv), ("z", H * d), ("beta", H))}
+    state = torch.randn(2, H, dv, d, generator=g)
+    ints = [torch.tensor(t, dtype=torch.int32, device=DEV) for t in ([0, 40, 45], [3, 0], [1, 0])]
+
+    def run(x, chunk_rows):
+        st, on = state.to(DEV), {n: t.to(DEV) for n, t in x.items()}
+        o = ops.matrix_state_recurrence(
+            on["q"], on["k"], on["v"], on["z"], H, Hk, d, dv, torch.ones(H, device=DEV), None, 1.0,
+            d ** -0.5, st, *ints, beta=on["beta"] if delta else None, unit_qk=delta,
+            chunk_rows=chunk_rows)
+        return o.cpu(), st.cpu()
+
+    rows = ops.MATRIX_STATE_CHUNK_ROWS
+    clean, clean_state = run(x, rows)
+    x[what] = x[what].clone()
+    x[what][at, 1] = bad
+    (o, st), (walk, walk_state) = run(x, rows), run(x, 0)
+    assert torch.equal(o[:at], clean[:at]) and torch.equal(o[40:], clean[40:])
+    assert torch.equal(st[0], clean_state[0])
+    if what == "v":
+        rest = torch.arange(H * dv) != 1
+        assert torch.equal(o[:, rest], clean[:, rest])
+        assert not torch.isfinite(o[at:40, 1]).any()
+    assert torch.equal(torch.isfinite(o), torch.isfinite(walk))
+    assert torch.equal(torch.isfinite(st), torch.isfinite(walk_state))

@@ -379,7 +379,7 @@ __global__ __launch_bounds__(64) void paged_attention_rows_kernel(
 // float32 attention on the matrix cores (v_mfma_f32_16x16x4_f32: float products and sums).
 //
 // A block takes one kv head and sixteen places (row, head of the kv head's): as many rows of one
-// segment as fit beside each other, so a prompt's rows share every key and value they read, and a
+// segment, at positions that follow one another, as fit beside each other, so a prompt's rows share every key and value they read, and a
 // decoded row has its heads in one block.  Its waves take steps of 16 keys in turns (step s
 // belongs to wave s % NW wherever a row's keys begin and end) and meet in LDS at the end, so a row's
 // result does not depend on the rows it is computed with.  Scores are made keys x places, which
@@ -400,12 +400,17 @@ __global__ __launch_bounds__((NT <= 4 ? 8 : 4) * WAVE) void paged_attention_f32_
   __shared__ float part_m[NW][16], part_l[NW][16];
   const int per = H / G, heads = min(per, 16), R = 16 / heads, pieces = (per + heads - 1) / heads;
   const int g = blockIdx.y / pieces, h0 = g * per + blockIdx.y % pieces * heads;
-  const int t0 = blockIdx.x, seg = row_seg[t0];
-  if (t0 % R != 0 && row_seg[t0 - 1] == seg) return;       // the block of an earlier row has it
-  int t1 = t0 + 1;
-  while (t1 < T && t1 % R != 0 && row_seg[t1] == seg) ++t1;
-
+  // Rows beside each other are one block's only while their positions follow one another: of the keys
+  // from the first row's first to the last row's own each is then seen by some row, and no page is
+  // read that no row needs.  The lanes look at the rows side by side (1,000 rows of one prompt 443 us,
+  // 466 with one row after the other).
+  const int t0 = blockIdx.x, seg = row_seg[t0], pos0 = row_pos[t0];
+  if (t0 % R != 0 && row_seg[t0 - 1] == seg && row_pos[t0 - 1] == pos0 - 1)
+    return;                                                 // the block of an earlier row has it
   const int wave = threadIdx.x / WAVE, lane = threadIdx.x % WAVE;
+  bool beside = lane < R - t0 % R && t0 + lane < T;
+  if (beside) beside = row_seg[t0 + lane] == seg && row_pos[t0 + lane] == pos0 + lane;
+  const int t1 = t0 + __builtin_ctzll(~__builtin_amdgcn_ballot_w64(beside));
   const int r = lane % 16, quad = lane / 16;
   int row = t0 + r / heads, head = h0 + r % heads;
   if (row >= t1 || head >= (g + 1) * per) row = t0, head = h0;    // a place without work of its own
@@ -433,7 +438,7 @@ __global__ __launch_bounds__((NT <= 4 ? 8 : 4) * WAVE) void paged_attention_f32_
     }
   };
   float m = -INFINITY, l = 0.f;
-  const int first = lo_min / 16, last = pos_max / 16;
+  const int first = lo_min / 16, last = pos_max < 0 ? -1 : pos_max / 16;
   int st = first + ((wave - first) % NW + NW) % NW;
   if (st <= last) fetch(st, kv, vv);
   for (; st <= last; st += NW) {

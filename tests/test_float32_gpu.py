@@ -82,3 +82,32 @@ def test_a_later_rows_odd_value_stays_with_the_rows_that_see_it(ops, bad):  # no
     rest = torch.ones(H * d, dtype=torch.bool)
     rest[[5, d + 5]] = False                        # the two heads on kv head 0
     assert torch.isfinite(out[:, rest]).all()
+
+
+def test_rows_far_apart_read_their_own_pages_only(ops):  # noqa: F811
+    """Neighbouring rows of a segment whose positions do not follow one another: no page between them
+    is needed, so the table may name none; a row before the first position has no key at all."""
+    H, G, d, ps, window = 4, 2, 32, 8, 11
+    pos = [5, 6, 100, 101, 3, 160, 159]
+    g = torch.Generator().manual_seed(23)
+    needed = sorted({k // ps for p in pos for k in range(max(p - window + 1, 0), p + 1)})
+    bt = torch.full((1, 21), -1, dtype=torch.int32)
+    bt[0, needed] = torch.randperm(len(needed), generator=g).int()
+    k = torch.randn(len(needed), G, ps, d, generator=g)
+    v = torch.randn(len(needed), G, d, ps, generator=g)
+    q = torch.randn(len(pos), H * d, generator=g)
+    rows = torch.tensor(pos, dtype=torch.int32), torch.zeros(len(pos), dtype=torch.int32)
+    want = ref.paged_attention(q, H, G, d, k, v, *rows, bt, ps, d ** -0.5, window=window)
+
+    def run(q, pos):
+        seg = torch.zeros(len(pos), dtype=torch.int32, device=DEV)
+        return ops.paged_attention(q.to(DEV), H, G, d, k.to(DEV), v.to(DEV),
+                                   torch.tensor(pos, dtype=torch.int32, device=DEV), seg,
+                                   bt.to(DEV), ps, d ** -0.5, window=window)
+    got = run(q, pos)
+    close(got, want, 6e-6, "rows far apart")
+    for t in range(len(pos)):
+        assert torch.equal(run(q[t:t + 1], pos[t:t + 1])[0], got[t]), t
+    before = run(torch.cat([q[:1], q[:1]]), [-1, 0])
+    assert not torch.isfinite(before[0]).any()
+    assert torch.equal(before[1], run(q[:1], [0])[0])

@@ -368,7 +368,8 @@ static void launch_f32(const float* A, const float* W, const float* bias, float*
 extern "C" int kappai_gemm_f32(const float* A, const float* W, const float* bias, float* C, int M,
                                int N, int K, int lda, int ldc, hipStream_t stream) {
   if (M <= 0 || N <= 0) return 0;
-  const bool whole = K % F32_CHUNK == 0 && lda % 4 == 0 && (uintptr_t)A % 16 == 0 &&
+  // (with no K at all nothing may be read: the element loads do not)
+  const bool whole = K > 0 && K % F32_CHUNK == 0 && lda % 4 == 0 && (uintptr_t)A % 16 == 0 &&
                      (uintptr_t)W % 16 == 0;
   if (whole) launch_f32<true>(A, W, bias, C, M, N, K, lda, ldc, stream);
   else launch_f32<false>(A, W, bias, C, M, N, K, lda, ldc, stream);

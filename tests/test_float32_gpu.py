@@ -29,6 +29,13 @@ def test_a_rows_product_has_the_same_bits_in_every_batch(ops, N, K):  # noqa: F8
     assert torch.equal(ops.linear(off[:, 1:], w, b), whole[:8])
 
 
+@pytest.mark.parametrize("M", [1, 8, 20, 40, 65, 700])
+def test_a_product_over_nothing_is_its_bias(ops, M):  # noqa: F811
+    b = rand((9000,), F32, 64).to(DEV)
+    got = ops.linear(torch.empty((M, 0), device=DEV), torch.empty((9000, 0), device=DEV), b)
+    assert torch.equal(got, b.expand(M, -1))
+
+
 ATTENTION = [
     # H, G, d, page, held before, new rows, window
     (16, 8, 64, 16, [0, 5, 300], [37, 1, 70], 0),

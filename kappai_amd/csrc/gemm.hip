@@ -38,10 +38,16 @@ typedef __attribute__((ext_vector_type(4))) uint32_t u32x4_t;
 // the e-th of every group), then chunk after chunk into the run's sum, then run after run.  A single
 // running sum over K = 8192 would lose about sqrt(K) roundings; this way it is sqrt(128) + a few.
 //
-// WHOLE: K is a multiple of 128 and everything is aligned to 16 bytes.  The loads then stand in no
-// branch (a branch around them has the compiler wait for one before it asks for the next).
+// LOADS: F32_WHOLE, K is a multiple of 128 and everything is aligned to 16 bytes; F32_FOURS, K is a
+// multiple of 4 and everything is aligned; F32_ELEMENTS, any other K from 4 on; F32_FEW, less.  Where
+// K ends the row's last four places are read again and what lies behind counts as 0, so that no load
+// stands in a branch that asks how far K goes (such a branch has the compiler wait for one load before
+// it asks for the next), and 16s of K that are all behind it are left out.  4096 columns over K = 16, 1,000
+// rows: 21.4 us with such branches and all 128 multiplied, 12.8 now; 1024 x 1030 of 64 rows 34.4 and
+// 19.6, of 1,000 46.5 and 31.8.
 #define F32_CHUNK 128
 #define F32_STEPS (F32_CHUNK / 16)
+enum { F32_FEW, F32_ELEMENTS, F32_FOURS, F32_WHOLE };
 
 __device__ __forceinline__ f32x4_t mfma_f32(float a, float b, f32x4_t c) {
   return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
@@ -51,24 +57,39 @@ __device__ __forceinline__ int f32_run_start(int run, int runs, int chunks) {
   return run * chunks / runs;
 }
 
-// Four values of a row from k on; zeros from `end` on.
-__device__ __forceinline__ f32x4_t load4_f32(const float* __restrict__ row, int k, int end) {
+// Four values of a row from k on; zeros from K on.
+template <int LOADS>
+__device__ __forceinline__ f32x4_t load4_f32(const float* __restrict__ row, int k, int K) {
+  if (LOADS == F32_WHOLE) return *reinterpret_cast<const f32x4_t*>(row + k);
   f32x4_t v = {0.f, 0.f, 0.f, 0.f};
+  if (LOADS == F32_FEW) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      if (k + e < K) v[e] = row[k + e];
+    return v;
+  }
+  const int from = min(k, K - 4), behind = k - from;
+  if (LOADS == F32_FOURS) {
+    const f32x4_t x = *reinterpret_cast<const f32x4_t*>(row + from);
+    return behind ? v : x;
+  }
+  float x[4];
+#pragma unroll
+  for (int e = 0; e < 4; ++e) x[e] = row[from + e];
 #pragma unroll
   for (int e = 0; e < 4; ++e)
-    if (k + e < end) v[e] = row[k + e];
+#pragma unroll
+    for (int back = 0; e + back < 4; ++back) v[e] = behind == back ? x[e + back] : v[e];
   return v;
 }
 
 // A lane's share of a chunk (its q-th four of every 16).
-template <bool WHOLE>
+template <int LOADS>
 __device__ __forceinline__ void load_chunk_f32(const float* __restrict__ row, int chunk, int q, int K,
                                                f32x4_t (&v)[F32_STEPS]) {
   const int k = chunk * F32_CHUNK + 4 * q;
 #pragma unroll
-  for (int j = 0; j < F32_STEPS; ++j)
-    v[j] = WHOLE ? *reinterpret_cast<const f32x4_t*>(row + k + 16 * j)
-                 : load4_f32(row, k + 16 * j, K);
+  for (int j = 0; j < F32_STEPS; ++j) v[j] = load4_f32<LOADS>(row, k + 16 * j, K);
 }
 
 // 1 to 64 rows: bound by the stream of W, in small matrices by what one block has under way.  A
@@ -79,7 +100,7 @@ __device__ __forceinline__ void load_chunk_f32(const float* __restrict__ row, in
 // of W is under way while a chunk is multiplied.  Three rows, W from memory: 9216 x 1024 12 us
 // (3.1 TB/s), 1024 x 4608 9 us, 65536 x 1024 51 us (5.3 TB/s); the vector kernel before took 100 to
 // 1,500 us, a block a 64 x 64 tile of which three rows were real.
-template <int MT, int COLS, int RUNS, bool WHOLE>
+template <int MT, int COLS, int RUNS, int LOADS>
 __global__ __launch_bounds__((COLS == 8 ? RUNS / 2 : 8) * WAVE) void gemm_f32_skinny_kernel(
     const float* __restrict__ A, const float* __restrict__ W, const float* __restrict__ bias,
     float* __restrict__ C, int M, int N, int K, int lda, int ldc) {
@@ -127,7 +148,7 @@ __global__ __launch_bounds__((COLS == 8 ? RUNS / 2 : 8) * WAVE) void gemm_f32_sk
   };
   // (a chunk behind a lane's last is read again from the last of all and not added)
   const auto load_w = [&](int c, f32x4_t (&v)[F32_STEPS]) {
-    load_chunk_f32<WHOLE>(w, min(c0 + c, chunks - 1), q, K, v);
+    load_chunk_f32<LOADS>(w, min(c0 + c, chunks - 1), q, K, v);
   };
   // (lanes without a row stay out: a masked load costs what its live lanes do)
   const int live = SIDE ? r % 8 : r;
@@ -138,7 +159,7 @@ __global__ __launch_bounds__((COLS == 8 ? RUNS / 2 : 8) * WAVE) void gemm_f32_sk
   const auto load_a = [&](int c) {
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt)
-      if (mt * 16 + live < M) load_chunk_f32<WHOLE>(a[mt], min(c0 + c, chunks - 1), q, K, av[mt]);
+      if (mt * 16 + live < M) load_chunk_f32<LOADS>(a[mt], min(c0 + c, chunks - 1), q, K, av[mt]);
   };
   const auto multiply = [&](int c) {
     if (!SIDE)
@@ -147,11 +168,13 @@ __global__ __launch_bounds__((COLS == 8 ? RUNS / 2 : 8) * WAVE) void gemm_f32_sk
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt) acc[mt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int j = 0; j < F32_STEPS; ++j)
+    for (int j = 0; j < F32_STEPS; ++j) {
+      if (LOADS != F32_WHOLE && 16 * j >= K) break;      // (a K of less than one chunk)
 #pragma unroll
       for (int e = 0; e < 4; ++e)
 #pragma unroll
         for (int mt = 0; mt < MT; ++mt) acc[mt] = mfma_f32(av[mt][j][e], wv[j][e], acc[mt]);
+    }
     // (side by side, a lane's results belong to the run that its column's half holds)
     if (!SIDE || c < len)
 #pragma unroll
@@ -198,7 +221,7 @@ __global__ __launch_bounds__((COLS == 8 ? RUNS / 2 : 8) * WAVE) void gemm_f32_sk
 // vector registers, and one wave multiplies while the other waits for LDS.  825 rows: 9216 x 1024
 // 165 us (94 TFLOP/s; the instruction alone reaches 153), 3072 x 1024 66 us, 2048 x 1024 45, 1024 x 4608
 // 101 (with four waves a block of 64 x 64, one a SIMD: 75, 46 and 107).
-template <int WY, int WX, int TY, int TX, int BK, bool WHOLE>
+template <int WY, int WX, int TY, int TX, int BK, int LOADS>
 __global__ __launch_bounds__(WY * WX * WAVE) __attribute__((amdgpu_waves_per_eu(2)))
 void gemm_f32_block_kernel(
     const float* __restrict__ A, const float* __restrict__ W, const float* __restrict__ bias,
@@ -230,8 +253,7 @@ void gemm_f32_block_kernel(
     for (int o = 0; o < 2; ++o)
 #pragma unroll
       for (int p = 0; p < PER; ++p)
-        next[o][p] = WHOLE ? *reinterpret_cast<const f32x4_t*>(src[o][p] + t * BK + 4 * slot)
-                           : load4_f32(src[o][p], t * BK + 4 * slot, K);
+        next[o][p] = load4_f32<LOADS>(src[o][p], t * BK + 4 * slot, K);
   };
   const auto keep = [&](int t) {
 #pragma unroll
@@ -246,7 +268,7 @@ void gemm_f32_block_kernel(
     for (int j = 0; j < TX; ++j) tot[i][j] = fin[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 
   const int chunks = (K + F32_CHUNK - 1) / F32_CHUNK, runs = f32_runs(chunks);
-  const int tiles = chunks * (F32_CHUNK / BK);       // (those behind K are zeros)
+  const int tiles = (K + BK - 1) / BK;
   int run = 0;
   fetch(0);
   keep(0);
@@ -260,6 +282,7 @@ void gemm_f32_block_kernel(
 #pragma unroll
     for (int u = 0; u < F32_CHUNK / BK; ++u) {
       const int t = chunk * (F32_CHUNK / BK) + u;
+      if (LOADS != F32_WHOLE && t >= tiles) break;
       fetch(min(t + 1, tiles - 1));                  // (the last tile once more, unused)
       __builtin_amdgcn_sched_barrier(0);             // (left alone, the loads sink to their use)
       const f32x4_t* la = lds[t & 1][0];
@@ -280,6 +303,7 @@ void gemm_f32_block_kernel(
       read(0);
 #pragma unroll
       for (int s = 0; s < BK / 16; ++s) {
+        if (LOADS != F32_WHOLE && t * BK + 16 * s >= K) break;
         if (s + 1 < BK / 16) read(s + 1);
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
@@ -324,13 +348,22 @@ void gemm_f32_block_kernel(
   }
 }
 
-template <bool WHOLE>
+template <int LOADS, int TY, int TX>
+static void launch_f32_blocks(const float* A, const float* W, const float* bias, float* C, int M,
+                              int N, int K, int lda, int ldc, hipStream_t stream) {
+  constexpr int B = 32 * TY;
+  const int tm = (M + B - 1) / B, tn = (N + B - 1) / B;
+  hipLaunchKernelGGL((gemm_f32_block_kernel<2, 4, TY, TX, 64, LOADS>), dim3((tn + 7) / 8 * 8 * tm),
+                     dim3(512), 0, stream, A, W, bias, C, M, N, K, lda, ldc, tm);
+}
+
+template <int LOADS>
 static void launch_f32(const float* A, const float* W, const float* bias, float* C, int M, int N,
                        int K, int lda, int ldc, hipStream_t stream) {
   if (M <= 64) {
     const bool many = f32_runs((K + F32_CHUNK - 1) / F32_CHUNK) == 32;
 #define F32_SKINNY(MT, COLS, RUNS)                                                                \
-  hipLaunchKernelGGL((gemm_f32_skinny_kernel<MT, COLS, RUNS, WHOLE>), dim3((N + COLS - 1) / COLS), \
+  hipLaunchKernelGGL((gemm_f32_skinny_kernel<MT, COLS, RUNS, LOADS>), dim3((N + COLS - 1) / COLS), \
                      dim3((COLS == 8 ? RUNS / 2 : 8) * WAVE), 0, stream, A, W, bias, C, M, N, K,   \
                      lda, ldc)
     if (M <= 8 && N <= 256 * 8) {
@@ -351,28 +384,21 @@ static void launch_f32(const float* A, const float* W, const float* bias, float*
   }
   const auto tiles = [](int n, int b) { return (n + b - 1) / b; };
   const long big = (long)tiles(M, 128) * tiles(N, 128), small = (long)tiles(M, 64) * tiles(N, 64);
-  if ((big + 255) / 256 * 4 * 8 <= (small + 255) / 256 * 9) {
-    const int tm = tiles(M, 128);
-    hipLaunchKernelGGL((gemm_f32_block_kernel<2, 4, 4, 2, 64, WHOLE>),
-                       dim3(tiles(tiles(N, 128), 8) * 8 * tm), dim3(512), 0, stream, A, W, bias, C,
-                       M, N, K, lda, ldc, tm);
-  } else {
-    const int tm = tiles(M, 64);
-    hipLaunchKernelGGL((gemm_f32_block_kernel<2, 4, 2, 1, 64, WHOLE>),
-                       dim3(tiles(tiles(N, 64), 8) * 8 * tm), dim3(512), 0, stream, A, W, bias, C,
-                       M, N, K, lda, ldc, tm);
-  }
+  if ((big + 255) / 256 * 4 * 8 <= (small + 255) / 256 * 9)
+    launch_f32_blocks<LOADS, 4, 2>(A, W, bias, C, M, N, K, lda, ldc, stream);
+  else
+    launch_f32_blocks<LOADS, 2, 1>(A, W, bias, C, M, N, K, lda, ldc, stream);
 }
 
 // Rows and columns of any number and any K.
 extern "C" int kappai_gemm_f32(const float* A, const float* W, const float* bias, float* C, int M,
                                int N, int K, int lda, int ldc, hipStream_t stream) {
   if (M <= 0 || N <= 0) return 0;
-  // (with no K at all nothing may be read: the element loads do not)
-  const bool whole = K > 0 && K % F32_CHUNK == 0 && lda % 4 == 0 && (uintptr_t)A % 16 == 0 &&
-                     (uintptr_t)W % 16 == 0;
-  if (whole) launch_f32<true>(A, W, bias, C, M, N, K, lda, ldc, stream);
-  else launch_f32<false>(A, W, bias, C, M, N, K, lda, ldc, stream);
+  const bool fours = K % 4 == 0 && lda % 4 == 0 && (uintptr_t)A % 16 == 0 && (uintptr_t)W % 16 == 0;
+  if (K < 4) launch_f32_blocks<F32_FEW, 2, 1>(A, W, bias, C, M, N, K, lda, ldc, stream);  // (0 too)
+  else if (fours && K % F32_CHUNK == 0) launch_f32<F32_WHOLE>(A, W, bias, C, M, N, K, lda, ldc, stream);
+  else if (fours) launch_f32<F32_FOURS>(A, W, bias, C, M, N, K, lda, ldc, stream);
+  else launch_f32<F32_ELEMENTS>(A, W, bias, C, M, N, K, lda, ldc, stream);
   KAPPAI_RETURN_LAUNCH_STATUS();
 }
 #endif  // GATE_ACT == 0

@@ -14,7 +14,9 @@ pytestmark = pytest.mark.gpu
 # K of one chunk, of the two numbers of runs and with chunks left over, and no whole chunks; N around
 # the widths that blocks own
 @pytest.mark.parametrize("N,K", [(5, 128), (40, 2048), (2047, 2176), (2064, 4608), (33, 2050),
-                                 (130, 8192), (9216, 1024)])
+                                 (130, 8192), (9216, 1024), (40, 1), (33, 3), (700, 4), (2064, 7),
+                                 (40, 20), (2064, 36), (33, 65), (70, 129), (2064, 140),
+                                 (40, 2181)])
 def test_a_rows_product_has_the_same_bits_in_every_batch(ops, N, K):  # noqa: F811
     x, w, b = rand((300, K), F32, 61), rand((N, K), F32, 62), rand((N,), F32, 63)
     want = x.double() @ w.double().T + b.double()

@@ -584,6 +584,14 @@ def interleave_gate_up(gate: torch.Tensor, up: torch.Tensor) -> torch.Tensor:
     return torch.cat([g, u], dim=1).reshape(2 * F, K).contiguous()
 
 
+def separate_gate_up(gate_up: torch.Tensor) -> torch.Tensor:
+    """The result [T, 2F] of a plain product with a matrix from ``interleave_gate_up``, its columns in
+    the matrices' own order: F gate columns, then F up columns."""
+    T, n = gate_up.shape
+    turns = gate_up.reshape(T, n // (2 * SWIGLU_GROUP), 2, SWIGLU_GROUP)
+    return turns.transpose(1, 2).reshape(T, n)
+
+
 def _out_in_fragment_order(wanted: bool, M: int, N: int, force_kernel: int) -> bool:
     return (wanted and FRAGMENT_ROWS_FROM <= M <= FUSED_MAX_ROWS and N % 32 == 0
             and force_kernel in (0, 2))

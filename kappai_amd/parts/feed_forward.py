@@ -48,7 +48,6 @@ class SwiGLU(FeedForward):
         self.activation, self.clamp = activation, clamp
         self.fused = False
         self.has_bias = bool(bias)
-        self.gate_bias = None          # the first product's biases in the order of its fused matrix
         self.gate_up = Linear([prefix + n["gate"], prefix + n["up"]], width, [hidden, hidden],
                               stage="matmul_ffn_gate_up", weight_suffix=weight_suffix, bias=bias,
                               bias_suffix=bias_suffix)
@@ -67,23 +66,32 @@ class SwiGLU(FeedForward):
             return ops.interleave_gate_up(w[:self.hidden], w[self.hidden:]) if self.fused else None
 
         self.gate_up.bind(tensors, arrange=interleaved)
-        if self.fused and self.has_bias:
+        if self.fused and self.has_bias:       # (in the order of the matrix's rows)
             b = self.gate_up.bias.reshape(-1, 1)
-            self.gate_bias = ops.interleave_gate_up(b[:self.hidden], b[self.hidden:]).reshape(-1)
+            self.gate_up.bias = ops.interleave_gate_up(b[:self.hidden],
+                                                       b[self.hidden:]).reshape(-1)
         if self.clamp is not None and self.gate_up.weight.device.type == "cuda":
             self.clamp.on(self.gate_up.weight.device)      # (before any step is captured)
         self.down.bind(tensors)
 
+    def _gate_in_product(self, x) -> bool:
+        """Whether the product that applies the gate itself takes these rows: it reads bfloat16, 16
+        bytes at a time.  Other rows go through a plain product and a gate behind it."""
+        if not self.fused or x.dtype != torch.bfloat16:
+            return False
+        return not torch.is_tensor(x) or (x.data_ptr() % 16 == 0
+                                          and (x.shape[0] == 1 or x.stride(0) % 8 == 0))
+
     def forward(self, x, batch, into=None):
-        if self.fused and x.dtype == torch.bfloat16:
+        if self._gate_in_product(x):
             with profile.scope("matmul_ffn_gate_up", self.gate_up.weight_bytes()):
                 act = ops.linear_swiglu(x, self.gate_up.weight, out_fragment=True,
                                         activation=self.ACTIVATIONS[self.activation],
-                                        clamp=self.clamp,
-                                        **({} if self.gate_bias is None
-                                           else {"bias": self.gate_bias}))
+                                        clamp=self.clamp, bias=self.gate_up.bias)
             return self.down.forward(act, partial_sums=True, add_into=into)
         gate_up = self.gate_up.forward(x)
+        if self.fused:
+            gate_up = ops.separate_gate_up(gate_up)
         with profile.scope("ffn_act"):
             act = (ops.swiglu(gate_up) if self.activation == "silu"
                    else ops.glu(gate_up, self.ACTIVATIONS[self.activation], self.clamp))

@@ -74,9 +74,12 @@ def interleave_gate_up(gate, up):
 
 
 def linear_swiglu(x, weight, force_kernel=0, weight_frag=None, out_fragment=False, activation=0,
-                  clamp=None):
+                  clamp=None, bias=None):
     F = weight.shape[0] // 2
-    y = (x.to(F32) @ weight.to(F32).T).reshape(x.shape[0], F // SWIGLU_GROUP, 2, SWIGLU_GROUP)
+    y = x.to(F32) @ weight.to(F32).T
+    if bias is not None:                  # rounded as a product with biases stores its results
+        y = (y + bias).to(x.dtype).to(F32)
+    y = y.reshape(x.shape[0], F // SWIGLU_GROUP, 2, SWIGLU_GROUP)
     g, u = y[:, :, 0, :].reshape(-1, F), y[:, :, 1, :].reshape(-1, F)
     if activation == 2:
         return _clamped(g, u, clamp).to(x.dtype)

@@ -82,6 +82,6 @@ STATE_SPACE_CHUNKS_FROM_ROWS = 16
 # with 16 heads of 64 x 64, delta rule: one segment of 24 rows 16.1 / 16.1, of 64 29.2 / 17.5, of 2,048
 # 743 / 121; 8 segments of 32 22.2 / 22.0, of 48 29.1 / 24.8; 64 of 32 75 / 85; 60 single rows beside
 # one of 128 51 / 44.  Of 128 x 128: 60 single rows beside one of 128 68.5 / 74.8, of 160 80.3 / 75.2.
-# The gated sum gains more at every one of these.
+# The gated sum gains more at every one of these.  bfloat16 only: in float32 the tokens are walked.
 MATRIX_STATE_CHUNKS_FROM_ROWS = 24
 MATRIX_STATE_CHUNKS_FROM_ROWS_A_SEGMENT = 2

@@ -53,10 +53,13 @@ def _columns(proj: torch.Tensor, start: int, n: int) -> torch.Tensor:
     return view
 
 
-def _chunk_rows(batch) -> int:
+def _chunk_rows(batch, dtype=torch.bfloat16) -> int:
     """How many rows a chunk of the recurrences with a decay per key channel takes; 0: they walk the
-    tokens one by one."""
-    chunked = (batch.max_segment_rows >= tuning.MATRIX_STATE_CHUNKS_FROM_ROWS
+    tokens one by one.  Chunks add in another order than the walk, and which of them runs goes by the
+    sizes of the whole step.  In float32, where a request's results are the same bits whatever else is
+    in the step and however its prompt is cut, the tokens are always walked."""
+    chunked = (dtype != torch.float32
+               and batch.max_segment_rows >= tuning.MATRIX_STATE_CHUNKS_FROM_ROWS
                + tuning.MATRIX_STATE_CHUNKS_FROM_ROWS_A_SEGMENT * batch.seg_slot.shape[0])
     return ops.MATRIX_STATE_CHUNK_ROWS if chunked else 0
 
@@ -111,7 +114,7 @@ class GatedLinearAttention(Mixer):
             o = ops.matrix_state_recurrence(
                 proj, proj[:, o_k:], proj[:, o_v:], z, H, H, d, dv, self.rate, self.decay_bias,
                 -1.0, d ** -0.5, cache.state, batch.seg_start, batch.seg_pos0, batch.seg_slot,
-                chunk_rows=_chunk_rows(batch))
+                chunk_rows=_chunk_rows(batch, self.dtype))
             y = ops.head_norm_gate(o, self.norm_w, self.norm_eps, proj[:, o_g:], ops.GATE_SILU,
                                    H, dv, self.dtype)
         return self.out.forward(y, partial_sums=True)
@@ -357,7 +360,7 @@ class GatedDeltaRule(Mixer):
                 qkv, qkv[:, G * d:], qkv[:, 2 * G * d:], z, H, G, d, dv, self.rate, self.dt_bias,
                 1.0, d ** -0.5, state, batch.seg_start, batch.seg_pos0, batch.seg_slot,
                 beta=proj[:, C + self.ra + self.rg:], unit_qk=True, unit_eps=self.unit_eps,
-                chunk_rows=_chunk_rows(batch))
+                chunk_rows=_chunk_rows(batch, self.dtype))
             y = ops.head_norm_gate(o, self.norm_w, self.norm_eps, gate, ops.GATE_SIGMOID, H, dv,
                                    self.dtype)
         return self.out.forward(y, partial_sums=True)

@@ -574,6 +574,25 @@ def test_a_batch_gives_what_its_requests_give_alone(tmp_path, model_dirs):
     assert worst < 1e-5
 
 
+@pytest.mark.parametrize("name", ["U", "X"])
+def test_float32_bits_hang_on_neither_neighbours_nor_cuts(tmp_path, model_dirs, name):
+    """In the 32-bit mode a request's logits are the same bits in whole prompts, in portions and single
+    tokens, and beside other requests, on either side of the sizes from which bfloat16 works its
+    recurrences in chunks."""
+    requests = make_requests(TINY[name][0]["vocab"], [120, 9, 60, 33], seed=24)
+    plans = {"r0": (0, [100] + [1] * 20), "r1": (1, [2, 2] + [1] * 5), "r2": (0, [1, 50, 2, 7]),
+             "r3": (2, [33])}
+    runs = [schedules.whole(requests), schedules.changing_portions(requests),
+            schedules.build(requests, plans)]
+    got = [replay(model_dirs[name], "float32", *run, tmp_path / str(i), graphs=bool(i % 2))[0]
+           for i, run in enumerate(runs)]
+    for other in got[1:]:
+        keys = got[0].keys() & other.keys()
+        assert len(keys) >= 4
+        bad = [k for k in sorted(keys) if not np.array_equal(got[0][k], other[k])]
+        assert not bad, (len(bad), len(keys), bad[:5])
+
+
 def test_the_residual_stream_layer_by_layer(model_dirs):
     """The stream after every layer of a whole prompt, in float32, against the plain
     implementation's."""

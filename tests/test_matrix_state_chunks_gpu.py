@@ -31,6 +31,7 @@ def test_when_chunks_are_taken(segments, longest, chunked):
     from kappai_amd.parts.linear_attention import _chunk_rows
     batch = SimpleNamespace(seg_slot=torch.zeros(segments), max_segment_rows=longest)
     assert _chunk_rows(batch) == (real_ops.MATRIX_STATE_CHUNK_ROWS if chunked else 0)
+    assert _chunk_rows(batch, F32) == 0
 
 
 # key sizes below, at and beyond a tile of 64 and of 128, columns that end inside 16; segments of less

@@ -800,6 +800,10 @@ __host__ __device__ static inline MscLayout msc_layout(int dp, int dv, int mode)
 }
 // A segment that starts at row `first` has its chunks at first / 16 + its number, .. + 1, ..: no two
 // segments' chunks meet, and T / 16 + S places hold all of them, whatever the segments are.
+//
+// The places are worked slab by slab: the scratch holds `n_slots` of them from `slot_begin` on, and a
+// segment whose chunks lie in two slabs leaves its state in `state` between them, as it does between
+// two steps.  The bits do not hang on where a slab ends.
 __device__ __forceinline__ int msc_slot0(int seg, int first) { return first / MSC_C + seg; }
 
 // The sum over 16 neighbouring lanes, as ks_sum<16>.
@@ -819,7 +823,7 @@ template <int NT, int MODE, typename TV>
 __global__ __launch_bounds__(256, 3) void matrix_state_chunk_prep_kernel(
     const float* __restrict__ qf, const float* __restrict__ kf, const float* __restrict__ af,
     const float* __restrict__ bf, const TV* __restrict__ v, int v_stride,
-    const int* __restrict__ seg_start, int S, int H, int Hk, int d, int dv,
+    const int* __restrict__ seg_start, int S, int H, int Hk, int d, int dv, int slot_begin,
     float* __restrict__ scratch) {
   constexpr int DP = 16 * NT, RS = DP + 4, M = DP / 64;
   __shared__ __attribute__((aligned(16))) float Qs[MSC_C][RS], Ks[MSC_C][RS], As[MSC_C][RS];
@@ -827,7 +831,7 @@ __global__ __launch_bounds__(256, 3) void matrix_state_chunk_prep_kernel(
   __shared__ __attribute__((aligned(16))) double Ns[MSC_C][MSC_C + 2];    // [key row j][i]
   __shared__ float Bs[MSC_C];
   __shared__ int seg_sh[2];
-  const int slot = blockIdx.y, h = blockIdx.x, tid = threadIdx.x;
+  const int slot = slot_begin + blockIdx.y, h = blockIdx.x, tid = threadIdx.x;
   const int hk = h / (H / Hk);
   if (tid == 0) seg_sh[0] = -1;
   __syncthreads();
@@ -843,7 +847,7 @@ __global__ __launch_bounds__(256, 3) void matrix_state_chunk_prep_kernel(
   const int row0 = seg_sh[0], n = seg_sh[1];
   if (row0 < 0) return;                          // (no segment has this chunk)
   const MscLayout L = msc_layout(DP, dv, MODE);
-  float* rec = scratch + ((size_t)slot * H + h) * L.size;
+  float* rec = scratch + ((size_t)blockIdx.y * H + h) * L.size;
 #pragma unroll
   for (int m = 0; m < NT / 4; ++m) {
     const int i = tid + 256 * m, row = i / (DP / 4), e = 4 * (i % (DP / 4));
@@ -981,7 +985,8 @@ template <int NT, int MODE>
 __global__ __launch_bounds__(256, 2) void matrix_state_chunk_walk_kernel(
     const float* __restrict__ scratch, float* __restrict__ state,
     const int* __restrict__ seg_start, const int* __restrict__ seg_pos0,
-    const int* __restrict__ seg_slot, int H, int d, int dv, float* __restrict__ out) {
+    const int* __restrict__ seg_slot, int H, int d, int dv, int slot_begin, int n_slots,
+    float* __restrict__ out) {
   constexpr int DP = 16 * NT, TPW = NT / 4;
   constexpr int AHEAD = 4 / TPW;       // (what the registers hold without spilling)
   __shared__ __attribute__((aligned(16))) float4 Ux[2][4][WAVE];       // partial W S0
@@ -989,12 +994,17 @@ __global__ __launch_bounds__(256, 2) void matrix_state_chunk_walk_kernel(
   const int seg = blockIdx.z, h = blockIdx.x, c0 = blockIdx.y * 16;
   const int lane = threadIdx.x % WAVE, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
   const int g = lane / 16, i16 = lane % 16, c = c0 + i16;
-  const int first = seg_start[seg], last = seg_start[seg + 1];
+  // the segment's rows whose chunks lie in this slab
+  const int seg_first = seg_start[seg], slot0 = msc_slot0(seg, seg_first);
+  const int before = max(slot_begin - slot0, 0);            // its chunks in earlier slabs
+  const int first = seg_first + before * MSC_C;
+  const int last = min(seg_start[seg + 1], seg_first + (slot_begin + n_slots - slot0) * MSC_C);
   if (last <= first) return;
   const int n_chunks = (last - first + MSC_C - 1) / MSC_C;
   const MscLayout L = msc_layout(DP, dv, MODE);
   // one address a chunk, the same for all lanes, and a lane's distances from it
-  const char* next = (const char*)(scratch + ((size_t)msc_slot0(seg, first) * H + h) * L.size);
+  const char* next =
+      (const char*)(scratch + ((size_t)(slot0 + before - slot_begin) * H + h) * L.size);
   const size_t rec_bytes = (size_t)H * L.size * sizeof(float);
   const unsigned tile0 = 4u * (wave * TPW * 256 + 4 * lane), last0 = 4u * (wave * TPW * 16 + 4 * g);
   const unsigned at_w = 4 * L.w + tile0, at_q = 4 * L.q + tile0, at_k = 4 * L.k + tile0;
@@ -1004,7 +1014,7 @@ __global__ __launch_bounds__(256, 2) void matrix_state_chunk_walk_kernel(
   const size_t out_bytes = (size_t)MSC_C * H * dv * sizeof(float);
   const unsigned at_out = 4u * ((4 * g + wave) * (unsigned)H * dv + c);
   float* st = state + (((size_t)seg_slot[seg] * H + h) * dv + min(c, dv - 1)) * d;
-  const bool carry = seg_pos0[seg] > 0;
+  const bool carry = before > 0 || seg_pos0[seg] > 0;
   f32x4_t Sx[TPW];
 #pragma unroll
   for (int t = 0; t < TPW; ++t) {
@@ -1137,39 +1147,47 @@ template <int NT, int MODE, typename TV>
 static void msc_launch(const float* qf, const float* kf, const float* af, const float* bf,
                        const TV* v, int v_stride, float* state, const int* seg_start,
                        const int* seg_pos0, const int* seg_slot, int T, int S, int H, int Hk,
-                       int d, int dv, float* scratch, float* out, hipStream_t stream) {
-  hipLaunchKernelGGL((matrix_state_chunk_prep_kernel<NT, MODE, TV>), dim3(H, T / MSC_C + S),
-                     dim3(256), 0, stream, qf, kf, af, bf, v, v_stride, seg_start, S, H, Hk, d, dv,
-                     scratch);
-  hipLaunchKernelGGL((matrix_state_chunk_walk_kernel<NT, MODE>), dim3(H, (dv + 15) / 16, S),
-                     dim3(256), 0, stream, scratch, state, seg_start, seg_pos0, seg_slot, H, d, dv,
-                     out);
+                       int d, int dv, float* scratch, int slab, float* out, hipStream_t stream) {
+  const int slots = T / MSC_C + S;
+  for (int at = 0; at < slots; at += slab) {
+    const int n = min(slab, slots - at);
+    hipLaunchKernelGGL((matrix_state_chunk_prep_kernel<NT, MODE, TV>), dim3(H, n), dim3(256), 0,
+                       stream, qf, kf, af, bf, v, v_stride, seg_start, S, H, Hk, d, dv, at, scratch);
+    hipLaunchKernelGGL((matrix_state_chunk_walk_kernel<NT, MODE>), dim3(H, (dv + 15) / 16, S),
+                       dim3(256), 0, stream, scratch, state, seg_start, seg_pos0, seg_slot, H, d,
+                       dv, at, n, out);
+  }
 }
 
-// Floats of scratch the chunked form needs (0: it does not take these sizes).
+// Floats of scratch the chunked form takes: what all chunks need, or whole chunks of all heads up to
+// `limit` floats (one of them, if that is more); 0: it does not take these sizes.
 extern "C" long long kappai_matrix_state_chunks_scratch(int T, int S, int d, int dv, int H,
-                                                        int mode) {
+                                                        int mode, long long limit) {
   if (T < 1 || S < 1 || d < 1 || d > 128 || d % 4 || dv < 1 || H < 1 || H > 65535 || S > 65535 ||
-      T / MSC_C + S > 65535 || (dv + 15) / 16 > 65535 || mode < 0 || mode > 1)
+      (dv + 15) / 16 > 65535 || mode < 0 || mode > 1)
     return 0;
-  return (long long)(T / MSC_C + S) * H * msc_layout(d <= 64 ? 64 : 128, dv, mode).size;
+  const long long one = (long long)H * msc_layout(d <= 64 ? 64 : 128, dv, mode).size;
+  const long long all = T / MSC_C + S, most = limit / one < 65535 ? limit / one : 65535;
+  return one * (all < most ? all : most < 1 ? 1 : most);
 }
 
 // As kappai_matrix_state_scan, modes 0 and 1, in chunks; qf, kf, af and state start on 16 bytes.
+// `scratch` holds as many floats as the function above says for the same `limit`.
 extern "C" int kappai_matrix_state_chunks(const float* qf, const float* kf, const float* af,
                                           const float* bf, const void* v, int v_stride,
                                           int v_is_bf16, float* state, const int* seg_start,
                                           const int* seg_pos0, const int* seg_slot, int T, int S,
                                           int H, int Hk, int d, int dv, int mode, float* scratch,
-                                          float* out, hipStream_t stream) {
+                                          long long limit, float* out, hipStream_t stream) {
   if (T <= 0 || S <= 0) return 0;
-  if (Hk < 1 || H % Hk || (mode == 1) != (bf != nullptr) || !scratch ||
-      !kappai_matrix_state_chunks_scratch(T, S, d, dv, H, mode) ||
+  const long long floats = kappai_matrix_state_chunks_scratch(T, S, d, dv, H, mode, limit);
+  if (Hk < 1 || H % Hk || (mode == 1) != (bf != nullptr) || !scratch || !floats ||
       ((uintptr_t)qf | (uintptr_t)kf | (uintptr_t)af | (uintptr_t)state | (uintptr_t)scratch) % 16)
     return (int)hipErrorInvalidValue;
+  const int slab = (int)(floats / H / msc_layout(d <= 64 ? 64 : 128, dv, mode).size);
 #define MSC_CASE(NT_, MODE_, TV_)                                                                   \
   msc_launch<NT_, MODE_, TV_>(qf, kf, af, bf, (const TV_*)v, v_stride, state, seg_start, seg_pos0, \
-                              seg_slot, T, S, H, Hk, d, dv, scratch, out, stream)
+                              seg_slot, T, S, H, Hk, d, dv, scratch, slab, out, stream)
 #define MSC_TYPED(NT_, MODE_) \
   if (v_is_bf16) MSC_CASE(NT_, MODE_, bf16_t); else MSC_CASE(NT_, MODE_, float)
   if (d <= 64) {

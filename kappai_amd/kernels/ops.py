@@ -2433,8 +2433,10 @@ SCAN_FORMS = {"auto": 0, "wave": 1, "block": 2}
 
 DECAY_KINDS = {"softplus": 0, "double_exp": 1, "fixed": 2}
 MATRIX_STATE_CHUNK_ROWS = 16    # the rows of a chunk of the gated sum and the delta rule
-# the most scratch their chunked form takes (2 GiB); steps that would need more walk the tokens
-MATRIX_STATE_SCRATCH_FLOATS = 1 << 29
+# the most scratch their chunked form takes at a time (512 MiB: about 15,000 rows of 16 heads of 128 x
+# 128; as much as its operands in float32 take); more rows are worked slab by slab, and then segments
+# of different slabs no longer side by side (two of 6,000 rows in two slabs 1,045 us, in one 799)
+MATRIX_STATE_SCRATCH_FLOATS = 1 << 27
 FIXED_DECAY_CHUNK_ROWS = 32     # the most rows of a chunk the chunked form of a fixed decay takes
 
 
@@ -2478,7 +2480,8 @@ def matrix_state_recurrence(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
 
     ``chunk_rows`` = ``MATRIX_STATE_CHUNK_ROWS`` without ``chunks``: the forms without a bonus are
     worked in chunks of 16 rows on the matrix cores (float32), which pays from a few chunks a
-    segment on; key sizes that are multiples of four up to 128, others walk the tokens."""
+    segment on; key sizes that are multiples of four up to 128, others walk the tokens.  Scratch of up
+    to ``MATRIX_STATE_SCRATCH_FLOATS`` is allocated for it; without room for that the tokens are walked."""
     H, Hk, d, dv = n_heads, n_qk_heads, dim, vdim
     _need(form in SCAN_FORMS, lambda: f"matrix_state_recurrence: form {form!r}")
     _need(decay in DECAY_KINDS and (z is None) == (decay == "fixed")
@@ -2560,16 +2563,22 @@ def matrix_state_recurrence(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
             _stream()), "fixed_decay_chunks")
         return out
     if chunk_rows == MATRIX_STATE_CHUNK_ROWS and chunks is None and mode < 2 and form == "auto":
+        limit = ctypes.c_longlong(MATRIX_STATE_SCRATCH_FLOATS)
         lib.kappai_matrix_state_chunks_scratch.restype = ctypes.c_longlong
         floats = lib.kappai_matrix_state_chunks_scratch(_c_int(T), _c_int(S), _c_int(d), _c_int(dv),
-                                                        _c_int(H), _c_int(mode))
-        if 0 < floats <= MATRIX_STATE_SCRATCH_FLOATS and state.data_ptr() % 16 == 0:
-            scratch = torch.empty(floats, dtype=F32, device=dev)
+                                                        _c_int(H), _c_int(mode), limit)
+        scratch = None
+        if floats > 0 and state.data_ptr() % 16 == 0:
+            try:
+                scratch = torch.empty(floats, dtype=F32, device=dev)
+            except torch.cuda.OutOfMemoryError:
+                pass                     # (the walk needs none)
+        if scratch is not None:
             check(lib.kappai_matrix_state_chunks(
                 _ptr(qf), _ptr(kf), _ptr(af), _ptr(bf), _ptr(values), _c_int(values.stride(0)),
                 _c_int(_is_bf16(values.dtype)), _ptr(state), _ptr(seg_start), _ptr(seg_pos0),
                 _ptr(seg_slot), _c_int(T), _c_int(S), _c_int(H), _c_int(Hk), _c_int(d),
-                _c_int(dv), _c_int(mode), _ptr(scratch), _ptr(out), _stream()),
+                _c_int(dv), _c_int(mode), _ptr(scratch), limit, _ptr(out), _stream()),
                 "matrix_state_chunks")
             return out
     check(lib.kappai_matrix_state_scan(

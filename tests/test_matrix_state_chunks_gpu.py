@@ -153,3 +153,51 @@ def test_a_value_that_is_no_number_stays_with_its_token_and_those_behind_it(  # 
         assert not torch.isfinite(o[at:40, 1]).any()
     assert torch.equal(torch.isfinite(o), torch.isfinite(walk))
     assert torch.equal(torch.isfinite(st), torch.isfinite(walk_state))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("delta", [False, True])
+@pytest.mark.parametrize("d,dv", [(64, 40), (128, 16)])
+def test_slabs_of_scratch(ops, monkeypatch, d, dv, delta):  # noqa: F811
+    """A scratch of any size gives the same bits; where there is no memory for one the tokens are
+    walked."""
+    lens, pos0, H = [70, 1, 16, 33, 15, 200], [0, 9, 3, 0, 4, 0], 2
+    T, g = sum(lens), torch.Generator().manual_seed(d)
+    q, k, v, z = (torch.randn(T, H * n, generator=g).to(DEV) for n in (d, d, dv, d))
+    b = torch.randn(T, H, generator=g).to(DEV) if delta else None
+    start = [0] + list(torch.tensor(lens).cumsum(0))
+    ints = [torch.tensor(t, dtype=torch.int32, device=DEV) for t in (start, pos0, [5, 0, 3, 1, 4, 2])]
+    state = torch.randn(6, H, dv, d, generator=g)
+
+    def run(chunk_rows=ops.MATRIX_STATE_CHUNK_ROWS):
+        st = state.to(DEV)
+        return ops.matrix_state_recurrence(
+            q, k, v, z, H, H, d, dv, torch.ones(H, device=DEV), None, 1.0, d ** -0.5, st, *ints,
+            beta=b, unit_qk=delta, chunk_rows=chunk_rows), st
+
+    whole, walked = run(), run(0)
+    assert not torch.equal(whole[0], walked[0])
+    slots = T // 16 + len(lens)
+    one = (33 * d + 256 + (16 * d if delta else 0) + (dv + 15) // 16 * 256) * H
+    empty, taken = torch.empty, []
+
+    def spy(*size, **kw):
+        taken.append(size[0])
+        return empty(*size, **kw)
+    for chunks in (0, 1, 2, 5, slots - 1, slots, slots + 1):
+        monkeypatch.setattr(ops, "MATRIX_STATE_SCRATCH_FLOATS", chunks * one + one // 2)
+        monkeypatch.setattr(ops.torch, "empty", spy)
+        o, st = run()
+        monkeypatch.setattr(ops.torch, "empty", empty)
+        assert one * min(max(chunks, 1), slots) in taken
+        taken.clear()
+        assert torch.equal(o, whole[0]) and torch.equal(st, whole[1]), chunks
+
+    def no_room(*size, **kw):
+        if isinstance(size[0], int):
+            raise torch.cuda.OutOfMemoryError("no room for the scratch")
+        return empty(*size, **kw)
+    monkeypatch.setattr(ops.torch, "empty", no_room)
+    o, st = run()
+    monkeypatch.setattr(ops.torch, "empty", empty)
+    assert torch.equal(o, walked[0]) and torch.equal(st, walked[1])

@@ -31,6 +31,24 @@ def test_a_rows_product_has_the_same_bits_in_every_batch(ops, N, K):  # noqa: F8
     assert torch.equal(ops.linear(off[:, 1:], w, b), whole[:8])
 
 
+# enough rows and columns for blocks of 128 x 128 (from 769 blocks of 64 x 64 on), ragged and whole, in
+# each form of the loads
+@pytest.mark.parametrize("M,N,K", [(330, 9217, 256), (330, 9217, 130), (321, 9300, 132),
+                                   (512, 8192, 128), (330, 9217, 2177)])
+def test_large_blocks_give_the_same_bits(ops, M, N, K):  # noqa: F811
+    rounds = lambda b: (-(-M // b) * -(-N // b) + 255) // 256  # noqa: E731
+    assert rounds(128) * 32 <= rounds(64) * 9, "the rule takes smaller blocks here"
+    x, w, b = rand((M, K), F32, 65), rand((N, K), F32, 66), rand((N,), F32, 67)
+    got = ops.linear(x.to(DEV), w.to(DEV), b.to(DEV))
+    close(got, x.double() @ w.double().T + b.double(), 3e-6, (M, N, K))
+    for m in (1, 64, 65, 200):
+        few = ops.linear(x[M - m:].to(DEV), w.to(DEV), b.to(DEV))
+        assert torch.equal(few, got[M - m:]), m
+    for n in (5, 64, 1000):               # the last columns as a matrix of their own
+        few = ops.linear(x.to(DEV), w[N - n:].to(DEV), b[N - n:].to(DEV))
+        assert torch.equal(few, got[:, N - n:]), n
+
+
 @pytest.mark.parametrize("M", [1, 8, 20, 40, 65, 700])
 def test_a_product_over_nothing_is_its_bias(ops, M):  # noqa: F811
     b = rand((9000,), F32, 64).to(DEV)

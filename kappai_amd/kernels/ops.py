@@ -952,8 +952,8 @@ def paged_attention(q: torch.Tensor, n_heads: int, n_kv_heads: int, head_dim: in
     cores: the split-key decode kernel when every segment is a single row (``single_rows``;
     ``max_position`` sizes the splits), else the tiled kernel over ``q_tiles`` [tiles, 4] =
     (segment, first row, rows <= 32, place of the tile in its segment: index | tiles << 16, or 0).
-    Everything else, float32 included, runs the plain
-    kernel.  ``kernel`` = "rows" | "prefill" | "decode" | "decode-block" | "decode-split" forces
+    Everything else runs the plain kernel, "rows"; it takes plain float32 scores over
+    head sizes of whole 16s up to 128 to the matrix cores as well (in 32 bits).  ``kernel`` = "rows" | "prefill" | "decode" | "decode-block" | "decode-split" forces
     one (for tests);
     ``prefill_variant`` 1 / 2 forces the tiled kernel's form (2: key tiles shared by four query
     heads of a kv head through LDS; head sizes 64 and 128 only).

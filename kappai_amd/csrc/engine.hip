@@ -84,36 +84,19 @@ void refuse(Step& c, const char* message) {
 // ---------------------------------------------------------------------------------------------
 // how many K ranges (the rule the host's parts use as well)
 // ---------------------------------------------------------------------------------------------
-// K ranges for a product with more than 64 rows whose consumer adds partial sums: the number that a
-// model of the block kernel's forms and of the norm that adds the planes likes best.  Least squares
-// over 787 measured products (1024 to 6144 columns, K from 1024 to 8192, 160 to 2048 rows, up to
-// eight ranges), good to 4 to 11 %; `steps` is 64s of K, `mb` the megabytes of results.  Its choices cost
-// 1 % more than the best of every case together, those of the model before (one time per 64 of K whatever
-// the number of blocks) 3.5 %: 2048 x 7168 of 2048 rows 78.8 us with the norm against 84.9, 2048 x 8192 of
-// 1024 rows 51.6 against 54.8.  Over 90 sizes drawn at random besides, 65 to 4,700 rows: geometric mean
-// 1.3 % less than with the model before, from 17 % less to 9 % more (3734 rows of 768 x 6144).
+// K ranges for a product with more than 64 rows whose consumer adds partial sums: the number that the
+// model of the block products (gemm_rules.h) with the norm that reads the planes (0.16 us a megabyte) likes
+// best.
 int split_k_large(int M, int N, int K) {
   int best = 1;
   double best_t = -1.0;
   for (int split = 1; split < 9; ++split) {
     if (K % (128 * split) || (split > 1 && K / split < 256)) continue;
-    const double steps = (double)K / split / 64.0;
+    // (one range: bfloat16 results)
     const double mb = (split > 1 ? split : 0.5) * M * (double)N * 4e-6;
-    const long blocks256 = (long)((M + 255) / 256) * ((N + 255) / 256) * split;
-    const long blocks128 = (long)((M + 127) / 128) * ((N + 127) / 128) * split;
     double t;
-    if (M > 128 && kappai_use_256_form(blocks256)) {
-      const double rounds = (double)((blocks256 + 255) / 256);
-      t = steps * (1.07 * rounds + 0.53 * blocks256 / 256) + 8.6 * rounds + 0.10 * mb;
-    } else if (kappai_deep_form(blocks128, K / split)) {
-      t = steps * (0.44 + 0.12 * blocks128 / 256) + 4.5 + 0.19 * mb;
-    } else if (blocks128 <= 256) {
-      t = steps * 0.69 + 2.5 + 0.22 * mb;
-    } else {
-      t = steps * (0.32 * blocks128 / 512 + 0.67 * (double)((blocks128 + 511) / 512)) + 2.5 +
-          0.22 * mb;
-    }
-    t += 0.16 * mb;                       // the norm reads them
+    kappai_block_shape(M, N, K, split, mb, false, &t);
+    t += 0.16 * mb;
     if (best_t < 0 || t < best_t - 1e-9) {
       best = split;
       best_t = t;

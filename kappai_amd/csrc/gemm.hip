@@ -5,9 +5,11 @@
 //   gemm_f32         true 32-bit: float products and sums on the matrix cores
 //                    (v_mfma_f32_16x16x4_f32) in an order that K alone decides, so a row's result
 //                    does not depend on M; a kernel for up to 64 rows and one for more.
-//   gemm_bf16_block256  large products (K a multiple of 128 per K range): bf16 inputs, fp32
-//                    accumulation on the matrix cores (v_mfma_f32_32x32x16_bf16), 256x256 or
-//                    128x128 blocks, tiles of 64 of K loaded straight into LDS.
+//   gemm_bf16_direct, gemm_bf16_staged  large products over a W in fragment order (K a multiple of
+//                    128 per K range): bf16 inputs, fp32 accumulation on the matrix cores
+//                    (v_mfma_f32_32x32x16_bf16), 256x256 to 128x128 blocks, tiles of 64 of K loaded
+//                    straight into LDS (in the largest blocks W's straight into registers).
+//   gemm_bf16_block256  the same over a W that lies as rows.
 //   gemm_bf16_tile   any K that is a multiple of 8: 256x128 or 128x128 blocks staged through
 //                    registers into LDS.
 //   gemm_bf16_skinny M <= 64 (decode): every block streams 16 or 32 rows of W once, its 4 to 16
@@ -688,14 +690,98 @@ static void launch_tile_cfg(const bf16_t* A, const bf16_t* W, const float* bias,
 #define KAPPAI_GPTR(p) ((const __attribute__((address_space(1))) void*)(p))
 #define KAPPAI_LPTR(p) ((__attribute__((address_space(3))) void*)(p))
 #define SCHED_FENCE() __builtin_amdgcn_sched_barrier(0)
+// (nothing that touches memory is moved across, by any pass of the compiler)
+#define ORDER_FENCE()                  \
+  do {                                 \
+    asm volatile("" ::: "memory");     \
+    __builtin_amdgcn_sched_barrier(0); \
+  } while (0)
+// waits until at most `behind` loads are under way (_AND_LDS: and no LDS access is)
+#define WAIT_LOADS(behind) __builtin_amdgcn_s_waitcnt(0x0F70 | ((behind) & 15) | ((behind) >> 4 << 14))
+#define WAIT_LOADS_AND_LDS(behind) \
+  __builtin_amdgcn_s_waitcnt(0x0070 | ((behind) & 15) | ((behind) >> 4 << 14))
+
+// A buffer of `bytes` bytes from p on: loads at offsets outside it read nothing and give zeros, so a
+// loop's last loads need no branch.  (The type is the device compiler's; the host pass sees neither it
+// nor the loads.)
+#if defined(__HIP_DEVICE_COMPILE__)
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t raw_buffer(const void* p, uint32_t bytes) {
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), 0, (int)bytes, 0x00020000);
+}
+#endif
 
 template <int N> struct IntC { static constexpr int value = N; };
+
+// The block products' epilogue: a wave turns 32 rows of its tile at a time through its own piece of LDS.
+// acc[i][j][4g + e] is C[row (wm*WTM+i)*32 + lane%32][column (wn*WTN+j)*32 + 8g + 4*(lane/32) + e].
+template <typename TO, int EPI, int WTM, int WTN>
+__device__ __forceinline__ void block_epilogue(const f32x16_t (&acc)[WTM][WTN], bf16_t* lds,
+                                               const float* bias, TO* C, int M, int N, int ldc, int m0,
+                                               int n0, int wave, int lane) {
+  const int wm = wave / 2, wn = wave % 2, r_in = lane % 32, hh = lane / 32;
+  constexpr int WROWS_N = WTN * 32;
+  constexpr int OUT_COLS = EPI == 1 ? WROWS_N / 2 : WROWS_N;   // columns a wave writes
+  constexpr int ROW_BYTES = OUT_COLS * (int)sizeof(TO) + 16;
+  char* mine = reinterpret_cast<char*>(lds) + wave * 32 * ROW_BYTES;
+  const int out_n = EPI == 1 ? N / 2 : N;
+  const int col0 = EPI == 1 ? (n0 + wn * WROWS_N) / 2 : n0 + wn * WROWS_N;
+#pragma unroll
+  for (int i = 0; i < WTM; ++i) {
+    char* wrow = mine + r_in * ROW_BYTES;
+#pragma unroll
+    for (int j = 0; j < WTN; ++j) {
+#pragma unroll
+      for (int g = 0; g < (EPI == 1 ? 2 : 4); ++g) {
+        float v4[4];
+        int c;                                   // first of the 4 columns, within the wave's
+        if (EPI == 1) {
+          c = j * 16 + 8 * g + 4 * hh;
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+            // (columns past the end are not stored: any row that is there)
+            v4[e] = gated_f(acc[i][j][4 * g + e], acc[i][j][4 * g + 8 + e], bias,
+                            min(n0 + wn * WROWS_N + j * 32 + 8 * g + 4 * hh + e, N - 17));
+        } else {
+          c = j * 32 + 8 * g + 4 * hh;
+#pragma unroll
+          for (int e = 0; e < 4; ++e) v4[e] = acc[i][j][4 * g + e];
+          if (bias && blockIdx.y == 0) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+              if (col0 + c + e < out_n) v4[e] += bias[col0 + c + e];
+          }
+        }
+        if (sizeof(TO) == 2) {
+          uint2 pk;
+          pk.x = pack_bf16x2(v4[0], v4[1]);
+          pk.y = pack_bf16x2(v4[2], v4[3]);
+          *reinterpret_cast<uint2*>(wrow + c * 2) = pk;
+        } else {
+          *reinterpret_cast<float4*>(wrow + c * 4) = make_float4(v4[0], v4[1], v4[2], v4[3]);
+        }
+      }
+    }
+    // rows back out, 16 bytes a lane
+    constexpr int CHUNKS = OUT_COLS * (int)sizeof(TO) / 16;   // per row
+    constexpr int ROWS_PER = WAVE / CHUNKS;                   // (lanes left over sit out)
+    constexpr int PER = 16 / (int)sizeof(TO);                 // columns a chunk
+    constexpr bool EVEN = WAVE % CHUNKS == 0 && 32 % ROWS_PER == 0;
+#pragma unroll
+    for (int it = 0; it < (32 + ROWS_PER - 1) / ROWS_PER; ++it) {
+      const int rr = it * ROWS_PER + lane / CHUNKS, ch = lane % CHUNKS;
+      if (!EVEN && (lane >= ROWS_PER * CHUNKS || rr >= 32)) continue;
+      const u32x4_t v = *reinterpret_cast<const u32x4_t*>(mine + rr * ROW_BYTES + ch * 16);
+      const int gm = m0 + (wm * WTM + i) * 32 + rr, gn = col0 + ch * PER;
+      if (gm < M && gn < out_n) *reinterpret_cast<u32x4_t*>(C + (size_t)gm * ldc + gn) = v;
+    }
+  }
+}
 
 template <typename TO, int EPI, int WT, bool DEEP = false, int WN_ = 0>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4 / WT, 4 / WT)))
 void gemm_bf16_block256_kernel(const bf16_t* __restrict__ A, const bf16_t* __restrict__ W,
                                const float* __restrict__ bias, TO* __restrict__ C, int M, int N,
-                               int K, int lda, int ldc, int tiles_n, int w_frag) {
+                               int K, int lda, int ldc, int tiles_n) {
   // WTM x WTN accumulator tiles of 32 x 32 a wave (WTN = WT unless WN_ is given): 4 x 4 ->
   // 256 x 256 blocks, 2 x 2 -> 128 x 128, 4 x 3 -> 256 rows x 192 columns (for a product whose
   // 256 x 256 blocks would leave a quarter of the chip without one)
@@ -731,17 +817,9 @@ void gemm_bf16_block256_kernel(const bf16_t* __restrict__ A, const bf16_t* __res
   // receives the row's chunk (lane%8) ^ ((row/2)%8).  Waves 0, 1 bring the A tile, waves 2, 3 the W
   // tile, NLOAD instructions each; rows past the end of the matrix repeat its last row (their
   // products are never stored).
-  //
-  // w_frag: W lies in fragment order ([rows / 16][K / 32] pieces of 16 rows x 32 of K, 1 KB each,
-  // the lane's 16 bytes at lane = (k % 32) / 8 * 16 + row % 16; see gemm_bf16_skinny_kernel).  A
-  // load instruction of the W waves then brings one piece, instruction i the piece (16 rows
-  // number i / 2 of the wave's rows, 32 of K number i % 2 of the tile), which lands in LDS as it
-  // lies in memory: a fragment read (16 lanes = 16 rows of one group of 8 of K = 256 contiguous
-  // bytes) is free of bank conflicts without a permutation.
   const bool brings_a = wave < 2;
-  const bool frag_w = !brings_a && w_frag;
   const char* gk = reinterpret_cast<const char*>(brings_a ? A : W) +
-                   (size_t)blockIdx.y * kblk * (frag_w ? 16 : 1) * sizeof(bf16_t);
+                   (size_t)blockIdx.y * kblk * sizeof(bf16_t);
   const int ld = brings_a ? lda : K;
   const int last_row = (brings_a ? M : N) - 1;
   const int row0 = brings_a ? m0 + wave * WROWS_M : n0 + (wave - 2) * WROWS_N;
@@ -754,12 +832,8 @@ void gemm_bf16_block256_kernel(const bf16_t* __restrict__ A, const bf16_t* __res
     const int lchunk = (lane % 8) ^ (((i * 8 + lrow) >> 1) & 7);
     roff[i] = (uint32_t)(min(row0 + i * 8 + lrow, last_row) * ld + lchunk * 8) *
               (uint32_t)sizeof(bf16_t);
-    if (frag_w)
-      roff[i] = (uint32_t)(min(row0 / 16 + i / 2, last_row / 16) * 16 * K + (i % 2) * 512 +
-                           lane * 8) * (uint32_t)sizeof(bf16_t);
   }
-  // bytes from one tile of 64 of K to the next: a row's 128 bytes, or two pieces
-  const uint32_t kstep = frag_w ? 2048u : (uint32_t)(BK * sizeof(bf16_t));
+  constexpr uint32_t kstep = BK * sizeof(bf16_t);    // bytes from one tile of 64 of K to the next
   // the address of a load is a wave-uniform 64-bit base (the tile's first column) plus the
   // lane's 32-bit row offset; pinning the base into scalar registers keeps the compiler from
   // folding the two into sixteen 64-bit per-lane pointers
@@ -782,9 +856,6 @@ void gemm_bf16_block256_kernel(const bf16_t* __restrict__ A, const bf16_t* __res
   for (int s = 0; s < 4; ++s) {
     aoff[s] = (wm * WROWS_M + r_in) * BK + (((s * 2 + hh) ^ ((r_in >> 1) & 7)) * 8);
     woff[s] = A_TILE + (wn * WROWS_N + r_in) * BK + (((s * 2 + hh) ^ ((r_in >> 1) & 7)) * 8);
-    if (w_frag)     // piece (r_in / 16, s / 2) of the wave's rows, group (s % 2) * 2 + hh of its K
-      woff[s] = A_TILE + wn * WROWS_N * BK + ((r_in / 16) * 2 + s / 2) * 512 +
-                (((s % 2) * 2 + hh) * 16 + r_in % 16) * 8;
   }
   bf16x8_t fa[2][WTM], fw[2][WTN];
   // in the order the products ask for them: w0 a0, the other w, the other a
@@ -951,64 +1022,305 @@ void gemm_bf16_block256_kernel(const bf16_t* __restrict__ A, const bf16_t* __res
   }
   }
 
-  // Epilogue: a wave turns 32 rows of its tile at a time through its own piece of LDS.
-  // acc[i][j][4g + e] is C[row (wm*WT+i)*32 + lane%32][column (wn*WT+j)*32 + 8g + 4*(lane/32) + e].
   __syncthreads();                               // everybody is done with the last tile
-  constexpr int OUT_COLS = EPI == 1 ? WROWS_N / 2 : WROWS_N;   // columns a wave writes
-  constexpr int ROW_BYTES = OUT_COLS * (int)sizeof(TO) + 16;
-  char* mine = reinterpret_cast<char*>(lds) + wave * 32 * ROW_BYTES;
-  const int out_n = EPI == 1 ? N / 2 : N;
-  const int col0 = EPI == 1 ? (n0 + wn * WROWS_N) / 2 : n0 + wn * WROWS_N;
+  block_epilogue<TO, EPI, WTM, WTN>(acc, lds, bias, C, M, N, ldc, m0, n0, wave, lane);
+}
+
+// Block products whose W lies in fragment order ([rows / 16][K / 32] pieces of 16 rows x 32 of K, 1 KB
+// each, the lane's 16 bytes at lane = (k % 32) / 8 * 16 + row % 16; see gemm_bf16_skinny_kernel).  Two
+// kernels, four waves each, one a SIMD; rows of A and of W past the end are not read.
+//
+// The large blocks (256 x 256, 256 x 192) are bound by LDS and by the rate at which a CU takes in tiles
+// (about 60 GB/s from memory, 85 from L2) more than by the matrix cores: with both operands in LDS a tile
+// of 64 of K reads 128 KB from LDS and writes 64 KB into it, at 64 bytes a clock about 2,500 clocks beside
+// 2,048 of matrix instructions.  Here W's fragments go from memory straight into registers, seven 16s of K
+// ahead, and only A goes through LDS, three tiles ahead: 96 KB of LDS traffic a tile, at the price of 32 KB
+// more taken in (two waves ask for the same pieces).  gate/up 16384 x 2048 of 2048 rows 112.4 us against
+// 117.0 with both operands in LDS (1.22 PFLOP/s; the loop without loads takes 91.6: matrix instructions on
+// real values run at 1.7 PFLOP/s), 9216 x 1024 of 1024 rows 26.4 against 29.2, in_proj 6144 x 2048 of 2048
+// rows in 256 x 192 blocks 45.6 against 50.2.
+//
+// Loads return in order, so the waits count those behind the one that is waited for.  Per tile a wave
+// issues WTN loads of W in each 16 of K and NA of A in the first two.  The wait for the next tile of A before
+// the barrier is a formality: the products before it have waited for pieces of W that were asked for after it.
+//
+// Host side guarantees for both: K / gridDim.y is a multiple of 128, rows of W a multiple of 16 (32 with
+// the gated epilogue), C and its row stride 16-byte aligned, M * lda and N * K below 2^31 elements.
+template <typename TO, int EPI, int WTM, int WTN>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1)))
+void gemm_bf16_direct_kernel(const bf16_t* __restrict__ A, const bf16_t* __restrict__ W,
+                             const float* __restrict__ bias, TO* __restrict__ C, int M, int N,
+                             int K, int lda, int ldc, int tiles_n) {
+  constexpr int BM = WTM * 64, BN = WTN * 64, BK = 64, NB = 4, SLOTS = 8;
+  constexpr int NPROD = WTM * WTN, NA = BM / 32;               // loads of A a wave and tile
+  constexpr int A_TILE = BM * BK;                              // in bf16
+  extern __shared__ __attribute__((aligned(1024))) bf16_t lds[];
+  const int tid = threadIdx.x, lane = tid % WAVE;
+  const int wave = __builtin_amdgcn_readfirstlane(tid / WAVE);
+  const int wm = wave / 2, wn = wave % 2;
+  const int2 tile = xcd_tile(blockIdx.x, gridDim.x / tiles_n, tiles_n);
+  const int m0 = tile.x * BM, n0 = tile.y * BN;
+  const int kblk = K / (int)gridDim.y;
+  const int nk = kblk / BK;
+  const int k0 = (int)blockIdx.y * kblk;
+  C += (size_t)blockIdx.y * M * ldc;
+
+  f32x16_t acc[WTM][WTN];
 #pragma unroll
-  for (int i = 0; i < WTM; ++i) {
-    char* wrow = mine + r_in * ROW_BYTES;
+  for (int i = 0; i < WTM; ++i)
 #pragma unroll
-    for (int j = 0; j < WTN; ++j) {
+    for (int j = 0; j < WTN; ++j)
 #pragma unroll
-      for (int g = 0; g < (EPI == 1 ? 2 : 4); ++g) {
-        float v4[4];
-        int c;                                   // first of the 4 columns, within the wave's
-        if (EPI == 1) {
-          c = j * 16 + 8 * g + 4 * hh;
+      for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.f;
+
+  const bf16_t* a_from = A + k0;
+  const bf16_t* w_from = W + (size_t)k0 * 16;
+  const uint32_t a_bytes = (uint32_t)(M - 1) * (uint32_t)lda * 2u + (uint32_t)kblk * 2u;
+  const uint32_t w_bytes = (uint32_t)N * (uint32_t)K * 2u - (uint32_t)k0 * 32u;
+  const int lrow = lane / 8;
+  uint32_t a_at[NA], w_at[WTN];
 #pragma unroll
-          for (int e = 0; e < 4; ++e)
-            // (columns past the end are not stored: any row that is there)
-            v4[e] = gated_f(acc[i][j][4 * g + e], acc[i][j][4 * g + 8 + e], bias,
-                            min(n0 + wn * WROWS_N + j * 32 + 8 * g + 4 * hh + e, N - 17));
-        } else {
-          c = j * 32 + 8 * g + 4 * hh;
+  for (int i = 0; i < NA; ++i) {
+    const int lchunk = (lane % 8) ^ (((i * 8 + lrow) >> 1) & 7);
+    a_at[i] = (uint32_t)(m0 + wave * (BM / 4) + i * 8 + lrow) * (uint32_t)lda * 2u + lchunk * 16u;
+  }
+  const int r_in = lane % 32, hh = lane / 32;
 #pragma unroll
-          for (int e = 0; e < 4; ++e) v4[e] = acc[i][j][4 * g + e];
-          if (bias && blockIdx.y == 0) {
+  for (int j = 0; j < WTN; ++j)
+    w_at[j] = (uint32_t)((n0 + wn * WTN * 32 + j * 32) / 16 + r_in / 16) * 16u * (uint32_t)K * 2u +
+              hh * 256u + (r_in % 16) * 16u;
+  // (the fragments of the s-th 16 of K: chunks 2s and 2s + 1)
+  const int aoff = (wm * WTM * 32 + r_in) * BK + ((hh ^ ((r_in >> 1) & 7)) * 8);
+
+  auto load_a = [&](int kt, int i) {           // tile kt; nothing is read of a tile that is not there
+#if defined(__HIP_DEVICE_COMPILE__)
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(
+        raw_buffer(a_from, kt < nk ? a_bytes : 0u),
+        KAPPAI_LPTR(lds + (kt & (NB - 1)) * A_TILE + (wave * (BM / 4) + i * 8) * BK), 16, a_at[i],
+        kt * 128, 0, 0);
+#endif
+  };
+  u32x4_t fw[SLOTS][WTN];
+  auto load_w = [&](int slot, int kt, int s, int j) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    fw[slot][j] = __builtin_amdgcn_raw_buffer_load_b128(
+        raw_buffer(w_from, kt < nk ? w_bytes : 0u), w_at[j] + s * 512, kt * 2048, 0);
+#endif
+  };
+  bf16x8_t fa[2][WTM];
+  auto read_a = [&](int fb, int kt, int s, int i) {
+    fa[fb][i] = as_bf16x8(*reinterpret_cast<const u32x4_t*>(lds + (kt & (NB - 1)) * A_TILE +
+                                                            (aoff ^ (s * 16)) + i * 32 * BK));
+  };
+  auto product = [&](int fb, int slot, int t) {
+    const int i = t / WTN, j = t % WTN;
+    acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(as_bf16x8(fw[slot][j]), fa[fb][i],
+                                                        acc[i][j], 0, 0, 0);
+  };
+  constexpr int PRE = WTN > 2 ? 4 : 2;
+  constexpr int OUT = 10 * WTN + 2 * NA;       // loads behind those of the next tile of A
+  static_assert(OUT < 64 && PRE >= WTN, "");
+  auto tile_step = [&](auto u_c, int kt) {
+    constexpr int U = decltype(u_c)::value;
 #pragma unroll
-            for (int e = 0; e < 4; ++e)
-              if (col0 + c + e < out_n) v4[e] += bias[col0 + c + e];
-          }
+    for (int s = 0; s < 4; ++s) {
+      const int ahead = s - 1 + SLOTS;           // the stage that the last stage's slot is for
+#pragma unroll
+      for (int t = 0; t < NPROD; ++t) {
+        if (s == 3 && t == PRE) {
+          WAIT_LOADS_AND_LDS(OUT);
+          __builtin_amdgcn_s_barrier();
+          SCHED_FENCE();
         }
-        if (sizeof(TO) == 2) {
-          uint2 pk;
-          pk.x = pack_bf16x2(v4[0], v4[1]);
-          pk.y = pack_bf16x2(v4[2], v4[3]);
-          *reinterpret_cast<uint2*>(wrow + c * 2) = pk;
-        } else {
-          *reinterpret_cast<float4*>(wrow + c * 4) = make_float4(v4[0], v4[1], v4[2], v4[3]);
+        if (t < WTN) load_w((U * 4 + ahead) % SLOTS, kt + ahead / 4, ahead % 4, t);
+        if (s < 2 && t >= NPROD - NA / 2) load_a(kt + 3, s * (NA / 2) + t - (NPROD - NA / 2));
+        if (s < 3) {
+          if (t < WTM) read_a((s + 1) & 1, kt, s + 1, t);
+        } else if (t >= PRE && t < PRE + WTM) {
+          read_a(0, kt + 1, 0, t - PRE);
         }
+        product(s & 1, U * 4 + s, t);
+        SCHED_FENCE();
       }
     }
-    // rows back out, 16 bytes a lane
-    constexpr int CHUNKS = OUT_COLS * (int)sizeof(TO) / 16;   // per row
-    constexpr int ROWS_PER = WAVE / CHUNKS;                   // (lanes left over sit out)
-    constexpr int PER = 16 / (int)sizeof(TO);                 // columns a chunk
-    constexpr bool EVEN = WAVE % CHUNKS == 0 && 32 % ROWS_PER == 0;
+  };
 #pragma unroll
-    for (int it = 0; it < (32 + ROWS_PER - 1) / ROWS_PER; ++it) {
-      const int rr = it * ROWS_PER + lane / CHUNKS, ch = lane % CHUNKS;
-      if (!EVEN && (lane >= ROWS_PER * CHUNKS || rr >= 32)) continue;
-      const u32x4_t v = *reinterpret_cast<const u32x4_t*>(mine + rr * ROW_BYTES + ch * 16);
-      const int gm = m0 + (wm * WTM + i) * 32 + rr, gn = col0 + ch * PER;
-      if (gm < M && gn < out_n) *reinterpret_cast<u32x4_t*>(C + (size_t)gm * ldc + gn) = v;
+  for (int i = 0; i < NA; ++i) load_a(0, i);
+  ORDER_FENCE();
+#pragma unroll
+  for (int i = 0; i < NA; ++i) load_a(1, i);
+  ORDER_FENCE();
+#pragma unroll
+  for (int s = 0; s < SLOTS - 1; ++s) {
+    if (s == 4) {
+#pragma unroll
+      for (int i = 0; i < NA; ++i) load_a(2, i);
+      ORDER_FENCE();
     }
+#pragma unroll
+    for (int j = 0; j < WTN; ++j) load_w(s, s / 4, s % 4, j);
+    ORDER_FENCE();
   }
+  constexpr int FIRST = 2 * NA + (SLOTS - 1) * WTN;          // loads behind those of tile 0 of A
+  WAIT_LOADS(FIRST);
+  __builtin_amdgcn_s_barrier();
+  ORDER_FENCE();
+#pragma unroll
+  for (int i = 0; i < WTM; ++i) read_a(0, 0, 0, i);
+  int kt = 0;
+  do {
+    tile_step(IntC<0>{}, kt);
+    tile_step(IntC<1>{}, kt + 1);
+    kt += 2;
+  } while (kt < nk);
+#if defined(__HIP_DEVICE_COMPILE__)
+  // (the sums stay in accumulation registers to the end of the loop: without this the gated form keeps
+  // some of W's pieces in scratch memory)
+#pragma unroll
+  for (int i = 0; i < WTM; ++i)
+#pragma unroll
+    for (int j = 0; j < WTN; ++j) asm volatile("" : "+a"(acc[i][j]));
+#endif
+  // (the loads of tiles that are not there have ended too: the epilogue uses their LDS)
+  WAIT_LOADS_AND_LDS(0);
+  __syncthreads();
+  block_epilogue<TO, EPI, WTM, WTN>(acc, lds, bias, C, M, N, ldc, m0, n0, wave, lane);
+}
+
+// The same product with both operands in LDS, NB buffers, for blocks whose tile is small beside what it
+// has under way: 128 x 128, 192 x 128, 256 x 128.  A block has its CU to itself, the loads of tile
+// kt + NB - 1 are spread over the first three 16s of tile kt (no branches: see raw_buffer), so NB - 1 tiles
+// are under way.  These are bound by what a CU takes in, so the block that covers the product in one round
+// with the fewest bytes wins (gemm_rules.h).  Against the forms before (128 x 128, two blocks a CU or four
+// buffers), W from memory: gate/up 16384 x 2048 of 417 rows 31.2 us against 36.8, 9216 x 1024 of 575 rows
+// 14.3 against 18.7; 3072 x 1024 of 575 rows 9.7 against 12.1; 2048 x 2048 of 417 rows in four ranges 9.6
+// against 12.2, 2048 x 8192 in four 21.2 against 24.0; 3072 x 2048 of 2048 rows 27.6 against 32.3.
+template <typename TO, int EPI, int WTM, int WTN, int NB>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1)))
+void gemm_bf16_staged_kernel(const bf16_t* __restrict__ A, const bf16_t* __restrict__ W,
+                             const float* __restrict__ bias, TO* __restrict__ C, int M, int N,
+                             int K, int lda, int ldc, int tiles_n) {
+  constexpr int BM = WTM * 64, BN = WTN * 64, BK = 64;
+  constexpr int NPROD = WTM * WTN, NREAD = WTM + WTN;
+  constexpr int NA = BM / 32, NW = BN / 32, NLOAD = NA + NW;   // loads a wave and tile
+  constexpr int A_TILE = BM * BK, TILE = (BM + BN) * BK;       // in bf16
+  extern __shared__ __attribute__((aligned(1024))) bf16_t lds[];
+  const int tid = threadIdx.x, lane = tid % WAVE;
+  const int wave = __builtin_amdgcn_readfirstlane(tid / WAVE);
+  const int wm = wave / 2, wn = wave % 2;
+  const int2 tile = xcd_tile(blockIdx.x, gridDim.x / tiles_n, tiles_n);
+  const int m0 = tile.x * BM, n0 = tile.y * BN;
+  const int kblk = K / (int)gridDim.y;
+  const int nk = kblk / BK;
+  const int k0 = (int)blockIdx.y * kblk;
+  C += (size_t)blockIdx.y * M * ldc;
+  f32x16_t acc[WTM][WTN];
+#pragma unroll
+  for (int i = 0; i < WTM; ++i)
+#pragma unroll
+    for (int j = 0; j < WTN; ++j)
+#pragma unroll
+      for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.f;
+  const bf16_t* a_from = A + k0;
+  const bf16_t* w_from = W + (size_t)k0 * 16;
+  const uint32_t a_bytes = (uint32_t)(M - 1) * (uint32_t)lda * 2u + (uint32_t)kblk * 2u;
+  const uint32_t w_bytes = (uint32_t)N * (uint32_t)K * 2u - (uint32_t)k0 * 32u;
+  const int lrow = lane / 8;
+  uint32_t a_at[NA], w_at[NW];
+#pragma unroll
+  for (int i = 0; i < NA; ++i) {
+    const int lchunk = (lane % 8) ^ (((i * 8 + lrow) >> 1) & 7);
+    a_at[i] = (uint32_t)(m0 + wave * (BM / 4) + i * 8 + lrow) * (uint32_t)lda * 2u + lchunk * 16u;
+  }
+#pragma unroll
+  for (int i = 0; i < NW; ++i) {
+    const int p = wave * NW + i;
+    w_at[i] = (uint32_t)(n0 / 16 + p / 2) * 16u * (uint32_t)K * 2u + (p % 2) * 1024u + lane * 16u;
+  }
+  const int r_in = lane % 32, hh = lane / 32;
+  const int aoff = (wm * WTM * 32 + r_in) * BK + ((hh ^ ((r_in >> 1) & 7)) * 8);
+  const int woff = A_TILE + (wn * WTN * 4 + (r_in / 16) * 2) * 512 + (hh * 16 + r_in % 16) * 8;
+  auto load = [&](int at, int kt, int i) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    if (i < NA)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(
+          raw_buffer(a_from, kt < nk ? a_bytes : 0u),
+          KAPPAI_LPTR(lds + at + (wave * (BM / 4) + i * 8) * BK), 16, a_at[i < NA ? i : 0], kt * 128, 0, 0);
+    else
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(
+          raw_buffer(w_from, kt < nk ? w_bytes : 0u),
+          KAPPAI_LPTR(lds + at + A_TILE + (wave * NW + i - NA) * 512), 16, w_at[i < NA ? 0 : i - NA],
+          kt * 2048, 0, 0);
+#endif
+  };
+  bf16x8_t fa[2][WTM], fw[2][WTN];
+  auto read = [&](int fb, int at, int s, int n) {       // w0 a0, the other w, the other a
+    const bool is_w = n == 0 || (n >= 2 && n <= WTN);
+    const int x = n <= 1 ? 0 : n <= WTN ? n - 1 : n - WTN;
+    if (is_w)
+      fw[fb][x] = as_bf16x8(*reinterpret_cast<const u32x4_t*>(
+          lds + at + woff + (s / 2) * 512 + (s % 2) * 256 + x * 2048));
+    else
+      fa[fb][x] = as_bf16x8(*reinterpret_cast<const u32x4_t*>(lds + at + (aoff ^ (s * 16)) + x * 32 * BK));
+  };
+  auto product = [&](int fb, int t) {
+    const int i = t / WTN, j = t % WTN;
+    acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fw[fb][j], fa[fb][i], acc[i][j], 0, 0, 0);
+  };
+#pragma unroll
+  for (int b = 0; b < NB - 1; ++b)
+#pragma unroll
+    for (int i = 0; i < NLOAD; ++i) load(b * TILE, b, i);
+  constexpr int BEHIND = (NB - 2) * NLOAD;
+  static_assert(BEHIND < 64, "");
+  WAIT_LOADS(BEHIND);
+  __builtin_amdgcn_s_barrier();
+  ORDER_FENCE();
+#pragma unroll
+  for (int n = 0; n < NREAD; ++n) read(0, 0, 0, n);
+  constexpr int PRE = NPROD > 4 ? 2 : 1;
+  constexpr int LOADS_AT = 3 * NPROD;                       // slots of the first three 16s of K
+  int cur = 0, kt = 0;
+  do {
+    const int nxt = cur == (NB - 1) * TILE ? 0 : cur + TILE;
+    const int into = cur == 0 ? (NB - 1) * TILE : cur - TILE;   // where the tile before this one lay
+#pragma unroll
+    for (int s = 0; s < 4; ++s) {
+#pragma unroll
+      for (int t = 0; t < NPROD; ++t) {
+        if (s == 3 && t == PRE) {
+          WAIT_LOADS_AND_LDS(BEHIND);
+          __builtin_amdgcn_s_barrier();
+          SCHED_FENCE();
+        }
+        if (s < 3) {
+          if (t < NREAD) read((s + 1) & 1, cur, s + 1, t);
+          const int slot = s * NPROD + t;
+          // NLOAD loads spread over the slots
+          if ((slot + 1) * NLOAD / LOADS_AT > slot * NLOAD / LOADS_AT)
+            load(into, kt + NB - 1, slot * NLOAD / LOADS_AT);
+        } else if (t >= PRE) {
+          constexpr int PER = (NREAD + NPROD - PRE - 1) / (NPROD - PRE);
+#pragma unroll
+          for (int q = 0; q < PER; ++q)
+            if ((t - PRE) * PER + q < NREAD) read(0, nxt, 0, (t - PRE) * PER + q);
+        }
+        product(s & 1, t);
+        SCHED_FENCE();
+      }
+    }
+    cur = nxt;
+    ++kt;
+  } while (kt < nk);
+#if defined(__HIP_DEVICE_COMPILE__)
+#pragma unroll
+  for (int i = 0; i < WTM; ++i)
+#pragma unroll
+    for (int j = 0; j < WTN; ++j) asm volatile("" : "+a"(acc[i][j]));   // (see the kernel above)
+#endif
+  WAIT_LOADS_AND_LDS(0);
+  __syncthreads();
+  block_epilogue<TO, EPI, WTM, WTN>(acc, lds, bias, C, M, N, ldc, m0, n0, wave, lane);
 }
 
 template <typename TO, int EPI>
@@ -1023,7 +1335,7 @@ static bool block256_fits(const bf16_t* A, const bf16_t* W, TO* C, int M, int n_
 template <typename TO, int EPI, int WT, bool DEEP = false, int WN_ = 0>
 static void launch_block256(const bf16_t* A, const bf16_t* W, const float* bias, TO* C, int M,
                             int n_rows_w, int K, int lda, int ldc, int ksplit,
-                            hipStream_t stream, int w_frag = 0) {
+                            hipStream_t stream) {
   constexpr int B = WT * 64, BN = (WN_ ? WN_ : WT) * 64;       // block: B rows x BN columns
   constexpr size_t lds_bytes = (DEEP ? 4 : 2) * (B + BN) * 64 * sizeof(bf16_t);
   auto kern = gemm_bf16_block256_kernel<TO, EPI, WT, DEEP, WN_>;
@@ -1035,19 +1347,63 @@ static void launch_block256(const bf16_t* A, const bf16_t* W, const float* bias,
   }
   const int tn = (n_rows_w + BN - 1) / BN, tm = (M + B - 1) / B;
   hipLaunchKernelGGL(kern, dim3(tm * tn, ksplit), dim3(256), lds_bytes, stream, A, W, bias, C, M,
-                     n_rows_w, K, lda, ldc, tn, w_frag);
+                     n_rows_w, K, lda, ldc, tn);
+}
+
+template <typename TO, int EPI, int WTM, int WTN, int NB>
+static void launch_fragment_block(const bf16_t* A, const bf16_t* Wf, const float* bias, TO* C, int M,
+                                  int n_rows_w, int K, int lda, int ldc, int ksplit,
+                                  hipStream_t stream) {
+  constexpr int BM = WTM * 64, BN = WTN * 64;
+  constexpr bool DIRECT = WTN > 2;
+  // the tiles of A (and W), or what the epilogue turns its rows in
+  constexpr size_t lds_bytes = NB * (BM + (DIRECT ? 0 : BN)) * 64 * sizeof(bf16_t);
+  static_assert(4 * 32 * (WTN * 32 * 4 + 16) <= lds_bytes && lds_bytes <= 160 * 1024, "LDS");
+  void (*kern)(const bf16_t*, const bf16_t*, const float*, TO*, int, int, int, int, int, int);
+  if constexpr (DIRECT) kern = gemm_bf16_direct_kernel<TO, EPI, WTM, WTN>;
+  else kern = gemm_bf16_staged_kernel<TO, EPI, WTM, WTN, NB>;
+  static bool attr_set = false;       // more than 64 KB of LDS has to be asked for once
+  if (!attr_set) {
+    (void)hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize,
+                              (int)lds_bytes);
+    attr_set = true;
+  }
+  const int tn = (n_rows_w + BN - 1) / BN, tm = (M + BM - 1) / BM;
+  hipLaunchKernelGGL(kern, dim3(tm * tn, ksplit), dim3(256), lds_bytes, stream, A, Wf, bias, C, M,
+                     n_rows_w, K, lda, ldc, tn);
 }
 
 // shape: 0 = chosen by size, 1 = 128x128 blocks of two waves, 2 = 256x128 blocks (tiles of 32
 // of K, two LDS buffers), 3 = 256x128 blocks (tiles of 64 of K, one LDS buffer), 4 = 256x256
 // blocks of the same kernel (tiles of 64 of K), 5 = the 256x256 kernel with one wave a SIMD, 6 = its
 // 128x128 form (when the sizes fit them, else 3), 8 = the 128x128 form with four LDS buffers, one
-// block a CU, 9 = the one-wave-a-SIMD kernel with blocks of 256 rows x 192 columns
+// block a CU, 9 = the one-wave-a-SIMD kernel with blocks of 256 rows x 192 columns, 11 = 192x128, 12 =
+// 256x128 (both only with W in fragment order, else 6)
 template <typename TO, int EPI>
 static void launch_tile(const bf16_t* A, const bf16_t* W, const float* bias, TO* C, int M,
                         int n_rows_w, int K, int lda, int ldc, int ksplit, int shape,
                         hipStream_t stream, const bf16_t* Wf = nullptr) {
   const bool fits = EPI != 2 && block256_fits<TO, EPI>(A, W, C, M, n_rows_w, K, lda, ldc, ksplit);
+  // Wf: W in fragment order (W may then be null)
+  if constexpr (EPI != 2) {
+    if (Wf != nullptr && fits && (shape == 0 || shape >= 5)) {
+      if (shape == 0)
+        shape = kappai_block_shape(M, n_rows_w, K, ksplit,
+                                   (double)M * n_rows_w * ksplit * sizeof(TO) * (EPI == 1 ? 0.5e-6 : 1e-6),
+                                   EPI == 1, nullptr);
+#define KAPPAI_BLOCKS(...)                                                                         \
+  launch_fragment_block<TO, EPI, __VA_ARGS__>(A, Wf, bias, C, M, n_rows_w, K, lda, ldc, ksplit, stream)
+      if (shape == 9 && EPI != 0) shape = 5;
+      if (shape == 5) KAPPAI_BLOCKS(4, 4, 4);
+      else if (shape == 11) KAPPAI_BLOCKS(3, 2, 3);
+      else if (shape == 12) KAPPAI_BLOCKS(4, 2, 3);
+      else if (shape != 9) KAPPAI_BLOCKS(2, 2, 4);
+      else if constexpr (EPI == 0) KAPPAI_BLOCKS(4, 3, 4);
+#undef KAPPAI_BLOCKS
+      return;
+    }
+  }
+  if (shape == 11 || shape == 12) shape = 6;
   if (shape == 0) {
     const int big = ((M + 255) / 256) * ((n_rows_w + 127) / 128) * ksplit;
     const int blocks256 = ((M + 255) / 256) * ((n_rows_w + 255) / 256) * ksplit;
@@ -1070,30 +1426,26 @@ static void launch_tile(const bf16_t* A, const bf16_t* W, const float* bias, TO*
   }
   if ((shape == 5 || shape == 6 || shape == 8 || shape == 9) && !fits) shape = 3;
   if (shape == 9 && EPI != 0) shape = 5;
-  // Wf: W in fragment order (W may then be null).  The one-wave-a-SIMD kernel reads it as fast as
-  // rows or a little faster (gate/up of 2048 rows 119.5 against 122-124 us in turns on one box, the
-  // other products equal: a tile's loads are pieces of 1 KB), the older tile kernel a little
-  // slower (47 against 43 us), so that one takes the rows when there are any.
-  const bool block_form = shape == 5 || shape == 6 || shape == 8 || shape == 9;
-  const int w_frag = Wf != nullptr && (W == nullptr || block_form);
+  // The tile kernel reads fragment order a little slower than rows (47 against 43 us), so it takes the
+  // rows when there are any.
+  const int w_frag = Wf != nullptr && W == nullptr;
   if (w_frag) W = Wf;
   switch (shape) {
     case 5:
       if constexpr (EPI != 2)
-        launch_block256<TO, EPI, 4>(A, W, bias, C, M, n_rows_w, K, lda, ldc, ksplit, stream, w_frag);
+        launch_block256<TO, EPI, 4>(A, W, bias, C, M, n_rows_w, K, lda, ldc, ksplit, stream);
       break;
     case 6:
       if constexpr (EPI != 2)
-        launch_block256<TO, EPI, 2>(A, W, bias, C, M, n_rows_w, K, lda, ldc, ksplit, stream, w_frag);
+        launch_block256<TO, EPI, 2>(A, W, bias, C, M, n_rows_w, K, lda, ldc, ksplit, stream);
       break;
     case 8:
       if constexpr (EPI != 2)
-        launch_block256<TO, EPI, 2, true>(A, W, bias, C, M, n_rows_w, K, lda, ldc, ksplit, stream, w_frag);
+        launch_block256<TO, EPI, 2, true>(A, W, bias, C, M, n_rows_w, K, lda, ldc, ksplit, stream);
       break;
     case 9:
       if constexpr (EPI == 0)
-        launch_block256<TO, EPI, 4, false, 3>(A, W, bias, C, M, n_rows_w, K, lda, ldc, ksplit,
-                                              stream, w_frag);
+        launch_block256<TO, EPI, 4, false, 3>(A, W, bias, C, M, n_rows_w, K, lda, ldc, ksplit, stream);
       break;
     case 1:
       launch_tile_cfg<TO, EPI, 1, 2, 4, 2, 32, 2, 2>(A, W, bias, C, M, n_rows_w, K, lda, ldc, ksplit,
@@ -2154,7 +2506,8 @@ static int launch_bf16(const bf16_t* A, const bf16_t* W, const float* bias, TO* 
 // force_kernel: 0 = by M, 1 = tile kernel, 2 = skinny kernel (M <= 64 only), 3..8 = tile kernel
 // with block shape 1..6 (see launch_tile), 9 = shared-rows kernel (17 to 64 rows, K / ksplit a
 // multiple of 512), 10 = block shape 8, 11 = block shape 9, 12 = the kernel for 25 to 128 rows
-// (1 to 128 rows, W in fragment order, K / ksplit a multiple of 256); for tests and tuning.
+// (1 to 128 rows, W in fragment order, K / ksplit a multiple of 256), 13 and 14 = block shapes 11 and
+// 12; for tests and tuning.
 // ksplit > 1 (float output only): C is [ksplit][M][ldc] partial sums over K ranges.
 // W_frag: null, or W in fragment order (K a multiple of 32, rows a multiple of 16); W may then
 // be null: every kernel reads the fragment order (only kappai_gemm_bf16_any needs rows).

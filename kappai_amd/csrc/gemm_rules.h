@@ -12,7 +12,42 @@
 // K of a block of that kernel comes in runs of this many
 #define KAPPAI_ROWS32_RUN 256
 
-// The forms of the block kernel (gemm_bf16_block256) for more than 128 rows.
+// The blocks of a product of more rows whose W lies in fragment order (gemm_bf16_direct, gemm_bf16_staged),
+// and a model of what each takes, in us: a tile of 64 of K costs `tile` in every round of blocks over the
+// 256 CUs and `fill` more when the round is full, a round `round`, a megabyte of results `mb`.  Least squares
+// of relative errors over 5,289 products (128 to 4,400 rows, 512 to 16,384 columns, K from 512 to 10,752, one
+// to eight ranges, float, bfloat16 and gated results), good to 5 to 10 % each.  Over the same products the
+// form that the model likes best takes 0.6 % more than the fastest of the five in sum; a fifth of the products
+// each are best in the first, fourth and fifth, two fifths in the third.
+struct kappai_block_form {
+  int shape, rows, cols;           // (shape: gemm.hip, launch_tile)
+  double tile, fill, round, mb, start;
+};
+static const kappai_block_form KAPPAI_BLOCK_FORMS[5] = {
+    {5, 256, 256, 0.95, 0.40, 6.0, 0.112, 2.9},  {9, 256, 192, 0.81, 0.30, 5.5, 0.111, 3.0},
+    {12, 256, 128, 0.51, 0.25, 1.9, 0.158, 3.2}, {11, 192, 128, 0.42, 0.22, 0.7, 0.198, 3.2},
+    {8, 128, 128, 0.32, 0.18, 0.1, 0.244, 3.1}};
+// The shape of the blocks for M rows, N rows of W, K in `split` ranges; `time`: what the model says.
+static inline int kappai_block_shape(int M, int N, int K, int split, double result_mb, bool gated,
+                                     double* time) {
+  int best = 8;
+  double best_t = -1.0;
+  for (const kappai_block_form& f : KAPPAI_BLOCK_FORMS) {
+    if (gated && f.shape == 9) continue;       // (its waves' columns are no whole pairs of 64)
+    const double blocks = (double)((M + f.rows - 1) / f.rows) * ((N + f.cols - 1) / f.cols) * split;
+    const double rounds = (double)(((long)blocks + 255) / 256), tiles = (double)K / split / 64.0;
+    const double t = tiles * (f.tile * rounds + f.fill * blocks / 256) + f.round * rounds +
+                     f.mb * result_mb + f.start;
+    if (best_t < 0 || t < best_t) {
+      best = f.shape;
+      best_t = t;
+    }
+  }
+  if (time) *time = best_t;
+  return best;
+}
+
+// The same for a W that lies as rows (gemm_bf16_block256).
 //
 // 256 x 256 blocks, one a CU, against 128 x 128 blocks, two a CU: from 140 blocks on when one round
 // does it, and with more rounds when the last one is not mostly idle (idle CU-rounds under a third
@@ -30,3 +65,4 @@ static inline bool kappai_use_256_form(long blocks256) {
 static inline bool kappai_deep_form(long blocks128, int k_range) {
   return blocks128 <= 256 && k_range >= 768;
 }
+

@@ -1,0 +1,62 @@
+"""The block products over a matrix in fragment order (256 x 256 and 256 x 192 blocks with W's pieces in
+registers, 256 x 128, 192 x 128 and 128 x 128 with both operands in LDS), at sizes that end inside a block
+and at the shortest runs of K, against the same product over the matrix's rows (bit for bit: every form adds
+16 of K after 16) and against float64."""
+import pytest
+import torch
+
+from test_kernels_gpu import BF16, DEV, F32, close, ops, rand  # noqa: F401
+
+pytestmark = pytest.mark.gpu
+FORMS = {"256x256": 7, "256x192": 11, "256x128": 14, "192x128": 13, "128x128": 10}
+ROWS = 8                       # the kernel for rows, 128 x 128 blocks
+
+
+# one row beside whole blocks, a single piece of 16 columns in the last block, K of two, three and five
+# pairs of 64 (fewer tiles than are under way at once), an odd number of ranges, a row stride
+@pytest.mark.parametrize("M,N,K,S", [(129, 144, 128, 1), (193, 272, 384, 3), (257, 208, 640, 1),
+                                     (384, 1040, 1280, 2), (513, 400, 256, 2), (65, 2064, 1024, 1)])
+@pytest.mark.parametrize("form", list(FORMS))
+def test_blocks_over_fragment_order(ops, M, N, K, S, form):  # noqa: F811
+    wide = rand((M, K + 40), BF16, 81).to(DEV)
+    x, w, b = wide[:, :K], rand((N, K), BF16, 82).to(DEV), rand((N,), F32, 83).to(DEV)
+    kept = ops.InFragments.of(w)
+    want = x.double() @ w.double().T
+    for out_dtype, bias in ((F32, None), (F32, b), (BF16, b)):
+        got = ops.linear(x, kept, bias, out_dtype=out_dtype, force_kernel=FORMS[form])
+        assert torch.equal(got, ops.linear(x, w, bias, out_dtype=out_dtype, force_kernel=ROWS))
+        if out_dtype == F32:       # float32 sums of K exact products: K roundings of 2^-24 at the most
+            close(got, want + (0 if bias is None else bias.double()), (K + 1) * 2.0 ** -24, form)
+    if S > 1:
+        planes = ops.linear(x, kept, partial_sums=True, split_k=S, force_kernel=FORMS[form])
+        assert planes.shape == (S, M, N)
+        assert torch.equal(planes, ops.linear(x, w, partial_sums=True, split_k=S, force_kernel=ROWS))
+
+
+@pytest.mark.parametrize("M,F,K", [(129, 16, 128), (193, 144, 256), (257, 112, 384), (520, 1040, 640)])
+@pytest.mark.parametrize("form", list(FORMS))
+def test_gated_blocks_over_fragment_order(ops, M, F, K, form):  # noqa: F811
+    x = rand((M, K), BF16, 84).to(DEV)
+    w = ops.interleave_gate_up(rand((F, K), BF16, 85, 0.2).to(DEV), rand((F, K), BF16, 86, 0.2).to(DEV))
+    got = ops.linear_swiglu(x, ops.InFragments.of(w), force_kernel=FORMS[form])
+    assert torch.equal(got, ops.linear_swiglu(x, w, force_kernel=ROWS))
+
+
+# the rule's own choices, one product for every form (by its model: 256 x 256, 256 x 192, 256 x 128,
+# 192 x 128, 128 x 128)
+@pytest.mark.parametrize("M,N,K", [(2048, 16384, 512), (2048, 6144, 640), (512, 16384, 512),
+                                   (575, 9216, 512), (300, 1024, 256)])
+def test_the_rule_takes_every_form(ops, M, N, K):  # noqa: F811
+    x, w = rand((M, K), BF16, 87).to(DEV), rand((N, K), BF16, 88).to(DEV)
+    assert torch.equal(ops.linear(x, ops.InFragments.of(w)), ops.linear(x, w, force_kernel=ROWS))
+
+
+def test_rows_that_are_not_there_stay_out(ops):  # noqa: F811
+    """NaN in the memory behind the last row of x and between its rows reaches no result."""
+    M, N, K = 200, 256, 256
+    wide = torch.full((M + 200, K + 8), float("nan"), dtype=BF16, device=DEV)
+    wide[:M, :K] = rand((M, K), BF16, 89).to(DEV)
+    w = rand((N, K), BF16, 90).to(DEV)
+    want = ops.linear(wide[:M, :K].contiguous(), w, force_kernel=ROWS)
+    for form in FORMS.values():
+        assert torch.equal(ops.linear(wide[:M, :K], ops.InFragments.of(w), force_kernel=form), want)

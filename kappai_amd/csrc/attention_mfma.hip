@@ -136,6 +136,15 @@ __device__ __forceinline__ u32x4_t load_k8(const bf16_t* __restrict__ k_pool,
 #define P_KS (HEAD_DIM / 16)            // k-steps of S^T over d
 #define P_MT ((HEAD_DIM + 31) / 32)     // row tiles of O^T over d
 
+// One row and one kv head by a block of NW waves, which take the keys in chunks in turn and meet in `sh`
+// (NW (rep HEAD_DIM + 32) floats of LDS; rep <= 16): defined with the decode kernels.
+template <bool MODS>
+__device__ __forceinline__ void attn_one_row(const bf16_t* q, int q_stride, const bf16_t* k_pool,
+                                             const bf16_t* vt_pool, bf16_t* out, int out_stride,
+                                             const int* bt, int max_blocks, int t, int pos, int g, int H,
+                                             int G, int ps, int window, float scale,
+                                             const kappai_score_mods& mods, float* sh, int NW);
+
 // waves of a block: they share one q tile and take its key tiles in turn, which shortens the
 // longest chain of dependent work fourfold; their partial results meet in LDS
 #define P_NW (HEAD_DIM <= 128 ? 4 : 1)
@@ -169,6 +178,24 @@ __global__ __launch_bounds__(P_NW * WAVE, P_MIN_WAVES) void attn_prefill_kernel(
   const int col = lane % 32, hh = lane / 32;
   const int* bt = block_tables + (size_t)seg * max_blocks;
   const int pos_first = row_pos[r0], pos_last = pos_first + nr - 1;
+  // what waves 1.. hand to wave 0
+  constexpr int SH_O = P_NW > 1 ? (P_NW - 1) * P_MT * 16 * WAVE : 1;
+  __shared__ float sh_o[SH_O];
+  if constexpr (!MODS && P_NW > 1) {
+    // A decoded token beside portions: all query heads of its kv head at once and the keys in chunks of
+    // D_KPW, as in a decode step.  Walked like a portion's tile, head by head and 32 keys at a time, a
+    // row's keys were read rep times and a chain of up to 12 round trips to memory held the kernel: 63 rows
+    // of 100 to 1,500 keys beside a portion of 512, 16 heads on 8: 45.2 us, now 35.8; 32 heads on 8 in
+    // the kernel below 65.3, now 34.5; 6 rows beside a portion of 100: 17.6, now 15.6.
+    static_assert(P_NW * (16 * HEAD_DIM + 32) <= SH_O || HEAD_DIM < 32, "LDS of a lone row");
+    const int rep = H / G;
+    if (nr == 1 && P_NW * (rep * HEAD_DIM + 32) <= SH_O && rep <= 16) {
+      if (h % rep == 0)
+        attn_one_row<false>(q, q_stride, k_pool, vt_pool, out, out_stride, bt, max_blocks, r0, pos_first,
+                            g, H, G, ps, window, scale, mods, sh_o, P_NW);
+      return;
+    }
+  }
   const bool row_ok = col < nr;
   const int my_pos = row_ok ? pos_first + col : -1;
   const int my_lo = kappai_first_key(my_pos, window);
@@ -396,7 +423,6 @@ __global__ __launch_bounds__(P_NW * WAVE, P_MIN_WAVES) void attn_prefill_kernel(
   if (P_NW > 1) {
     // merge: every wave rescales to the common maximum; waves 1.. hand their sums to wave 0
     __shared__ float sh_m[P_NW][32], sh_l[P_NW][32];
-    __shared__ float sh_o[P_NW > 1 ? P_NW - 1 : 1][P_MT * 16][WAVE];
     if (hh == 0) sh_m[wave][col] = m_run;
     __syncthreads();
     float M = sh_m[0][col];
@@ -409,7 +435,7 @@ __global__ __launch_bounds__(P_NW * WAVE, P_MIN_WAVES) void attn_prefill_kernel(
 #pragma unroll
       for (int mt = 0; mt < P_MT; ++mt)
 #pragma unroll
-        for (int v = 0; v < 16; ++v) sh_o[wave - 1][mt * 16 + v][lane] = o[mt][v] * f;
+        for (int v = 0; v < 16; ++v) sh_o[((wave - 1) * P_MT * 16 + mt * 16 + v) * WAVE + lane] = o[mt][v] * f;
     }
     __syncthreads();
     if (wave > 0) return;
@@ -424,7 +450,7 @@ __global__ __launch_bounds__(P_NW * WAVE, P_MIN_WAVES) void attn_prefill_kernel(
       for (int v = 0; v < 16; ++v) {
         float acc = o[mt][v] * f;
 #pragma unroll
-        for (int w = 1; w < P_NW; ++w) acc += sh_o[w - 1][mt * 16 + v][lane];
+        for (int w = 1; w < P_NW; ++w) acc += sh_o[((w - 1) * P_MT * 16 + mt * 16 + v) * WAVE + lane];
         o[mt][v] = acc;
       }
   }
@@ -502,6 +528,17 @@ __global__ __launch_bounds__(8 * WAVE) void attn_prefill_shared_kernel(
   }
   const int rep = H / G, quads = rep / 4;
   const int g = blockIdx.y / quads;
+  // a decoded token beside portions (see the kernel above): eight waves share its keys
+  if (t_b < 0 && q_tiles[4 * t_a + 2] == 1 && rep <= 16 &&
+      8 * (rep * HEAD_DIM + 32) * (int)sizeof(float) <= (int)sizeof lds) {
+    const int t = q_tiles[4 * t_a + 1];
+    if (blockIdx.y % quads == 0)
+      attn_one_row<false>(q, q_stride, k_pool, vt_pool, out, out_stride,
+                          block_tables + (size_t)q_tiles[4 * t_a] * max_blocks, max_blocks, t, row_pos[t],
+                          g, H, G, ps, window, scale, kappai_score_mods{0.f, nullptr, 0, sink, 0},
+                          reinterpret_cast<float*>(lds), 8);
+    return;
+  }
   const int lane = threadIdx.x % WAVE;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
   const int grp = wave / 4;                         // 0: tile a, 1: tile b
@@ -1173,43 +1210,41 @@ __device__ __forceinline__ void qk_norm_rotate(u32x4_t (&raw)[(HEAD_DIM + 31) / 
                         pack_bf16(x[ks][4], x[ks][5]), pack_bf16(x[ks][6], x[ks][7])};
 }
 
-// One wave's share of a row's attention: the query heads of kv head g (columns) against the keys
-// of the chunks c0 = first, first + stride, ... below k_end (D_KPW keys each), with a running
-// maximum and sum per column.  Leaves the unnormalised output in o (lane: column lane % 16, d
-// rows 16 mt + 4 (lane / 16) + v), the maximum (in units of log 2) in m_run, the sum in l_run.
-// With MODS the chunks are counted in places (kappai_key_at): the kept first keys stand in front of
-// the window's, whose places are their positions.
-template <bool FUSABLE, bool MODS = false>
+// One wave's share of a row's attention: the query heads of kv head g (columns) against the keys first ..
+// k_end - 1 (`first` a multiple of 32), with a running maximum and sum per column.  Leaves the unnormalised
+// output in o (lane: column lane % 16, d rows 16 mt + 4 (lane / 16) + v), the maximum (in units of log 2) in
+// m_run, the sum in l_run.
+//
+// Bound by the stream of keys and values.  The keys go by in parts of 32 whose loads (16 bytes a lane) are
+// asked for D_AHEAD parts ahead: a part's registers are filled again as soon as it is worked on, so that
+// loads stay under way from the first key to the last.  The page ids are read 64 at a time, the next 64
+// ahead of their use, and handed out as scalars.  Against chunks of 128 keys, each asked for, waited for
+// and worked on by itself: 3 rows of 9,000 to 15,000 keys, 32 heads of 64 on 8 (with the prologue) 24.4 us
+// against 32.5; 64 rows of 128 to 2,304 keys 39.4 against 42.6 (160 MB: 4.1 TB/s, the kernel's start and
+// the three lookups before its first key among it); 8 rows of 3,600 keys 15.3 against 15.9.
+#define D_AHEAD (HEAD_DIM <= 64 ? 4 : (HEAD_DIM <= 128 ? 2 : 1))
+template <bool FUSABLE>
 __device__ __forceinline__ void attn_decode_wave(
     const bf16_t* __restrict__ q, int q_stride, const bf16_t* __restrict__ k_pool,
     const bf16_t* __restrict__ vt_pool, const int* __restrict__ bt, int max_blocks, int t, int g,
-    int H, int G, int ps, float scale, int lo, int hi, int first, int stride, int k_end,
-    f32x4_t (&o)[D_MT], float& m_run, float& l_run, const QkFuse& qk, int pos,
-    const kappai_score_mods* mods = nullptr) {
+    int H, int G, int ps, float scale, int lo, int first, int k_end, f32x4_t (&o)[D_MT], float& m_run,
+    float& l_run, const QkFuse& qk, int pos) {
   const int lane = threadIdx.x % WAVE;
   const int rep = H / G;
   const int col = lane % 16, kg = lane / 16;
   const bool head_ok = col < rep;
   const int h = g * rep + (head_ok ? col : 0);
-  // the page ids of the first chunk of keys: asked for before anything else, so that the keys
-  // can be asked for as soon as they are there, whatever else is still on its way
-  const int keep = MODS ? mods->keep_first : 0;
-  const int lo32 = (lo / 32) * 32;
-  const int kept = MODS ? kappai_kept_places(keep, lo32) : 0;
-  auto ask_pages = [&](int c0) {
-    int my_page = -1;
-    if (MODS) {       // lane i: the page of the chunk's places 16 i .. 16 i + 15
-      const int key = kappai_key_at(c0 + 16 * lane, lo32, kept);
-      if (16 * lane < D_KPW && key / ps < max_blocks && (key <= hi || key < keep))
-        my_page = bt[key / ps];
-      return my_page;
-    }
-    const int first_page = c0 / ps;
-    if (first_page + lane < max_blocks && (first_page + lane) * ps <= hi)
-      my_page = bt[first_page + lane];
-    return my_page;
+  const int hi = k_end - 1;
+  // page ids 64 at a time: asked for before anything else
+  const int page0 = first / ps;
+  auto ask_pages = [&](int from) {
+    return from + lane < max_blocks && (long long)(from + lane) * ps <= hi ? bt[from + lane] : -1;
   };
-  int pages_first = first < k_end ? ask_pages(first) : -1;
+  int pages = ask_pages(page0), pages_next = -1, page_at = 0, page_off = first % ps;
+  const bool many = (long long)(page0 + WAVE) * ps <= hi;
+  if (many) pages_next = ask_pages(page0 + WAVE);
+  int pages_from = page0 + WAVE;
+
   bf16x8_t qf[D_KS];
   u32x4_t qraw[D_KS];
   u32x4_t k_new[D_KS];                 // the row's own key, in the K fragment's order of d
@@ -1248,15 +1283,234 @@ __device__ __forceinline__ void attn_decode_wave(
       for (int ks = 0; ks < D_KS; ++ks) qf[ks] = as_frag(qraw[ks]);
     }
   }
-  bool prologue_due = fused;
-  // the wave whose chunks hold the row's own position puts its key and value into the pools
-  const bool owner = own_kv && pos >= first && pos < k_end &&
-                     ((pos - first) / D_KPW) % (stride / D_KPW) == 0;
+#pragma unroll
+  for (int mt = 0; mt < D_MT; ++mt) o[mt] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
+  m_run = -INFINITY;
+  float l_lane = 0.f;                  // of the lane's own keys
+  const float sc = scale * LOG2E;
+
+  struct Part {
+    u32x4_t k[2][D_KS], v[D_MT];
+  };
+  // (scalars) the page of the next 16 keys and their place in it
+  auto next16 = [&](int& page, int& off) {
+    page = __builtin_amdgcn_readlane(pages, page_at);
+    off = page_off;
+    page_off += 16;
+    if (page_off >= ps) {
+      page_off = 0;
+      if (++page_at == WAVE) {
+        page_at = 0;
+        pages = pages_next;
+        pages_from += WAVE;
+        pages_next = ask_pages(pages_from);
+      }
+    }
+  };
+  // Row r of the key tile tt (of the 32 keys from kb) is key kb + 8 (r / 4) + 4 tt + r % 4:
+  // the lane that holds rows 4 kg .. 4 kg + 3 of both tiles' scores then holds the keys
+  // kb + 8 kg .. + 7 in order, and their values are ONE 16-byte piece of a V^T row.
+  const int k_lane = (8 * (col / 4 % 2) + col % 4) * HEAD_DIM + 8 * kg;     // + 4 tt rows, + 32 ks
+  const int v_lane = col * ps + 8 * (kg % 2);                               // + 16 mt ps
+  auto ask = [&](int kb, Part& p) {
+    int pg[2], off[2];
+    next16(pg[0], off[0]);
+    next16(pg[1], off[1]);
+    if (kb >= lo && kb + 31 <= hi && pg[0] >= 0 && pg[1] >= 0) {     // every key of the part is seen
+      const size_t a0 = ((size_t)pg[0] * G + g) * ps, a1 = ((size_t)pg[1] * G + g) * ps;
+      const bf16_t* kp = k_pool + (col < 8 ? (a0 + off[0]) * HEAD_DIM : (a1 + off[1]) * HEAD_DIM) + k_lane;
+      const bf16_t* vp = vt_pool + (kg < 2 ? a0 * HEAD_DIM + off[0] : a1 * HEAD_DIM + off[1]) + v_lane;
+#pragma unroll
+      for (int tt = 0; tt < 2; ++tt)
+#pragma unroll
+        for (int ks = 0; ks < D_KS; ++ks) {
+          const bool there = HEAD_DIM % 32 == 0 || 32 * ks + 8 * kg < HEAD_DIM;
+          const u32x4_t x = *reinterpret_cast<const u32x4_t*>(
+              there ? kp + 4 * tt * HEAD_DIM + 32 * ks : k_pool);
+          p.k[tt][ks] = there ? x : (u32x4_t){0u, 0u, 0u, 0u};
+        }
+#pragma unroll
+      for (int mt = 0; mt < D_MT; ++mt) p.v[mt] = *reinterpret_cast<const u32x4_t*>(vp + 16 * mt * ps);
+      return;
+    }
+#pragma unroll
+    for (int tt = 0; tt < 2; ++tt) {
+      const int key = kb + 8 * (col / 4) + 4 * tt + col % 4;
+#pragma unroll
+      for (int ks = 0; ks < D_KS; ++ks)
+        p.k[tt][ks] = load_k8_pg(k_pool, col < 8 ? pg[0] : pg[1], G, g, ps, key, 32 * ks + 8 * kg, lo, hi);
+    }
+#pragma unroll
+    for (int mt = 0; mt < D_MT; ++mt)
+      p.v[mt] = load_vt8_pg(vt_pool, kg < 2 ? pg[0] : pg[1], G, g, ps, 16 * mt + col, kb + 8 * kg, lo, hi);
+  };
+  // the pools do not hold the row's own key and value yet (or only just): the part that holds
+  // the row's position takes them from the registers
+  auto own = [&](int kb, Part& p) {
+    if (!(own_kv && pos >= kb && pos < kb + 32)) return;
+#pragma unroll
+    for (int tt = 0; tt < 2; ++tt) {
+      if (kb + 8 * (col / 4) + 4 * tt + col % 4 == pos) {
+#pragma unroll
+        for (int ks = 0; ks < D_KS; ++ks) p.k[tt][ks] = k_new[ks];
+      }
+    }
+    const int e = pos - (kb + 8 * kg);
+    if (e >= 0 && e < 8) {
+      const uint32_t keep = (e & 1) ? 0x0000ffffu : 0xffff0000u;
+#pragma unroll
+      for (int mt = 0; mt < D_MT; ++mt) {
+        const uint32_t put = (v_new[mt] & 0xffffu) << ((e & 1) * 16);
+        uint32_t w[4] = {p.v[mt].x, p.v[mt].y, p.v[mt].z, p.v[mt].w};
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          if (i == e / 2) w[i] = (w[i] & keep) | put;
+        p.v[mt] = (u32x4_t){w[0], w[1], w[2], w[3]};
+      }
+    }
+  };
+  auto work = [&](int kb, const Part& p) {
+    f32x4_t s[2];
+#pragma unroll
+    for (int tt = 0; tt < 2; ++tt) {
+      s[tt] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int ks = 0; ks < D_KS; ++ks)
+        s[tt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_frag(p.k[tt][ks]), qf[ks], s[tt], 0, 0, 0);
+    }
+    // lane holds, for head `col`, keys kb + 8*kg + 4*tt + v
+    float mloc = -INFINITY;
+    if (kb >= lo && kb + 31 <= hi) {
+#pragma unroll
+      for (int tt = 0; tt < 2; ++tt)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+          s[tt][v] *= sc;
+          mloc = fmaxf(mloc, s[tt][v]);
+        }
+    } else {
+#pragma unroll
+      for (int tt = 0; tt < 2; ++tt)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+          const int key = kb + 8 * kg + 4 * tt + v;
+          s[tt][v] = key >= lo && key <= hi ? s[tt][v] * sc : -INFINITY;
+          mloc = fmaxf(mloc, s[tt][v]);
+        }
+    }
+    mloc = fmaxf(mloc, lane_xor16(mloc));
+    mloc = fmaxf(mloc, other_half(mloc));
+    const float m_new = fmaxf(m_run, mloc);
+    const float m_safe = m_new == -INFINITY ? 0.f : m_new;
+    const float corr = fast_exp2(m_run - m_safe);
+    float lsum = 0.f;
+#pragma unroll
+    for (int tt = 0; tt < 2; ++tt)
+#pragma unroll
+      for (int v = 0; v < 4; ++v) {
+        s[tt][v] = fast_exp2(s[tt][v] - m_safe);
+        lsum += s[tt][v];
+      }
+    l_lane = l_lane * corr + lsum;
+    m_run = m_new;
+    const u32x4_t pw = {pack_bf16(s[0][0], s[0][1]), pack_bf16(s[0][2], s[0][3]),
+                        pack_bf16(s[1][0], s[1][1]), pack_bf16(s[1][2], s[1][3])};
+    const bf16x8_t pf = as_frag(pw);
+#pragma unroll
+    for (int mt = 0; mt < D_MT; ++mt) {
+      o[mt] = o[mt] * corr;
+      o[mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_frag(p.v[mt]), pf, o[mt], 0, 0, 0);
+    }
+  };
+  Part part[D_AHEAD];
+  int kb_ask = first;
+#pragma unroll
+  for (int i = 0; i < D_AHEAD; ++i) {
+    if (kb_ask < k_end) ask(kb_ask, part[i]);
+    kb_ask += 32;
+  }
+  if constexpr (FUSABLE && D_QK_FUSABLE) {
+    if (fused) {
+      if (own_kv) qk_norm_rotate(k_new, qk.k_norm_w != nullptr, tb.wk, qk.eps,
+                                 qk.cos_tab != nullptr, tb.cs, tb.sn);
+      qk_norm_rotate(qraw, qk.q_norm_w != nullptr, tb.wq, qk.eps, qk.cos_tab != nullptr, tb.cs,
+                     tb.sn);
+#pragma unroll
+      for (int ks = 0; ks < D_KS; ++ks)
+        qf[ks] = as_frag(head_ok ? qraw[ks] : (u32x4_t){0u, 0u, 0u, 0u});
+      // the wave whose keys hold the row's own position puts its key and value into the pools
+      if (own_kv && pos >= first && pos < k_end) {
+        const size_t pg = (size_t)bt[pos / ps] * G + g;
+        if (col == 0) {
+#pragma unroll
+          for (int ks = 0; ks < D_KS; ++ks)
+            *reinterpret_cast<u32x4_t*>(qk.k_pool_w + (pg * ps + pos % ps) * HEAD_DIM + 32 * ks +
+                                        8 * kg) = k_new[ks];
+        }
+        if (kg == 0) {
+#pragma unroll
+          for (int mt = 0; mt < D_MT; ++mt)
+            qk.vt_pool_w[(pg * HEAD_DIM + 16 * mt + col) * ps + pos % ps] = (bf16_t)v_new[mt];
+        }
+      }
+    }
+  }
+  for (int kb = first; kb < k_end;) {
+#pragma unroll
+    for (int i = 0; i < D_AHEAD; ++i) {
+      if (kb >= k_end) break;
+      own(kb, part[i]);
+      work(kb, part[i]);
+      if (kb_ask < k_end) ask(kb_ask, part[i]);
+      kb += 32;
+      kb_ask += 32;
+    }
+  }
+  l_lane += lane_xor16(l_lane);
+  l_run = l_lane + other_half(l_lane);
+}
+
+// One wave's share of a row's attention: the query heads of kv head g (columns) against the keys
+// of the chunks c0 = first, first + stride, ... below k_end (D_KPW keys each), with a running
+// maximum and sum per column, scores worked on (score_mods.h).  Leaves the unnormalised output in o (lane: column lane % 16, d
+// rows 16 mt + 4 (lane / 16) + v), the maximum (in units of log 2) in m_run, the sum in l_run.
+// The chunks are counted in places (kappai_key_at): the kept first keys stand in front of
+// the window's, whose places are their positions.
+__device__ __forceinline__ void attn_decode_scored_wave(
+    const bf16_t* __restrict__ q, int q_stride, const bf16_t* __restrict__ k_pool,
+    const bf16_t* __restrict__ vt_pool, const int* __restrict__ bt, int max_blocks, int t, int g,
+    int H, int G, int ps, float scale, int lo, int hi, int first, int stride, int k_end,
+    f32x4_t (&o)[D_MT], float& m_run, float& l_run, int pos, const kappai_score_mods* mods) {
+  const int lane = threadIdx.x % WAVE;
+  const int rep = H / G;
+  const int col = lane % 16, kg = lane / 16;
+  const bool head_ok = col < rep;
+  const int h = g * rep + (head_ok ? col : 0);
+  // the page ids of the first chunk of keys: asked for before anything else, so that the keys
+  // can be asked for as soon as they are there, whatever else is still on its way
+  const int keep = mods->keep_first;
+  const int lo32 = (lo / 32) * 32;
+  const int kept = kappai_kept_places(keep, lo32);
+  auto ask_pages = [&](int c0) {      // lane i: the page of the chunk's places 16 i .. 16 i + 15
+    const int key = kappai_key_at(c0 + 16 * lane, lo32, kept);
+    return 16 * lane < D_KPW && key / ps < max_blocks && (key <= hi || key < keep) ? bt[key / ps] : -1;
+  };
+  int pages_first = first < k_end ? ask_pages(first) : -1;
+  bf16x8_t qf[D_KS];
+  {
+    const bf16_t* qr = q + (size_t)t * q_stride + (size_t)h * HEAD_DIM;
+#pragma unroll
+    for (int ks = 0; ks < D_KS; ++ks) {
+      u32x4_t v = {0u, 0u, 0u, 0u};
+      const int d0 = 32 * ks + 8 * kg;
+      if (head_ok && d0 < HEAD_DIM) v = *reinterpret_cast<const u32x4_t*>(qr + d0);
+      qf[ks] = as_frag(v);
+    }
+  }
 #pragma unroll
   for (int mt = 0; mt < D_MT; ++mt) o[mt] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
   m_run = -INFINITY;
   l_run = 0.f;
-  const float sc = scale * LOG2E;
 
   // A wave takes its keys in chunks of D_KPW: first the chunk's page ids (one load, handed
   // round by shuffles), then every key and value load of the chunk at once (16 bytes a lane
@@ -1267,79 +1521,43 @@ __device__ __forceinline__ void attn_decode_wave(
   struct Chunk {
     u32x4_t kf[NCH][2][D_KS];
     u32x4_t vv[NCH][D_MT];
-    float bias[MODS ? NCH : 1][8];     // of the lane's eight keys, the last key first
+    float bias[NCH][8];     // of the lane's eight keys, the last key first
   };
-  const float* bias_row = MODS && mods->dist_bias != nullptr ? kappai_bias_row(*mods, h) : nullptr;
+  const float* bias_row = mods->dist_bias != nullptr ? kappai_bias_row(*mods, h) : nullptr;
   auto ask = [&](int c0, int my_page, Chunk& ch) {
-    const int first_page = c0 / ps;
     // Row r of the key tile tt (of the 32 keys from kb) is key kb + 8 (r / 4) + 4 tt + r % 4:
     // the lane that holds rows 4 kg .. 4 kg + 3 of both tiles' scores then holds the keys
     // kb + 8 kg .. + 7 in order, and their values are ONE 16-byte piece of a V^T row.
 #pragma unroll
     for (int c = 0; c < NCH; ++c) {
-      const int kb = MODS ? kappai_key_at(c0 + 32 * c, lo32, kept) : c0 + 32 * c;
+      const int kb = kappai_key_at(c0 + 32 * c, lo32, kept);
       // (what the row does not see reads as zero)
-      const int f_lo = MODS && kb < keep ? kb : lo, f_hi = MODS && kb < lo32 ? keep - 1 : hi;
+      const int f_lo = kb < keep ? kb : lo, f_hi = kb < lo32 ? keep - 1 : hi;
 #pragma unroll
       for (int tt = 0; tt < 2; ++tt) {
         const int key = kb + 8 * (col / 4) + 4 * tt + col % 4;
-        const int page =
-            MODS ? __shfl(my_page, 2 * c + (key - kb) / 16, WAVE)
-                 : __shfl(my_page, min(key / ps - first_page, WAVE - 1), WAVE);
+        const int page = __shfl(my_page, 2 * c + (key - kb) / 16, WAVE);
 #pragma unroll
         for (int ks = 0; ks < D_KS; ++ks)
           ch.kf[c][tt][ks] = load_k8_pg(k_pool, page, G, g, ps, key, 32 * ks + 8 * kg, f_lo, f_hi);
       }
-      const int pv =
-          MODS ? __shfl(my_page, 2 * c + kg / 2, WAVE)
-               : __shfl(my_page, min((kb + 8 * kg) / ps - first_page, WAVE - 1), WAVE);
+      const int pv = __shfl(my_page, 2 * c + kg / 2, WAVE);
 #pragma unroll
       for (int mt = 0; mt < D_MT; ++mt)
         ch.vv[c][mt] = load_vt8_pg(vt_pool, pv, G, g, ps, 16 * mt + col, kb + 8 * kg,
                                     f_lo, f_hi);
-      if (MODS) {
-        if (bias_row != nullptr) {     // distances base .. base + 7, by the row's edges at most
-          const int base = max(-KAPPAI_BIAS_PAD, min(pos - kb - 8 * kg - 7, mods->dist_cols - 1));
-          const f32x4_any_t b0 = *reinterpret_cast<const f32x4_any_t*>(bias_row + base);
-          const f32x4_any_t b1 = *reinterpret_cast<const f32x4_any_t*>(bias_row + base + 4);
+      if (bias_row != nullptr) {     // distances base .. base + 7, by the row's edges at most
+        const int base = max(-KAPPAI_BIAS_PAD, min(pos - kb - 8 * kg - 7, mods->dist_cols - 1));
+        const f32x4_any_t b0 = *reinterpret_cast<const f32x4_any_t*>(bias_row + base);
+        const f32x4_any_t b1 = *reinterpret_cast<const f32x4_any_t*>(bias_row + base + 4);
 #pragma unroll
-          for (int i = 0; i < 4; ++i) {
-            ch.bias[c][i] = b0[i];
-            ch.bias[c][4 + i] = b1[i];
-          }
-        } else {
-#pragma unroll
-          for (int i = 0; i < 8; ++i) ch.bias[c][i] = 0.f;
+        for (int i = 0; i < 4; ++i) {
+          ch.bias[c][i] = b0[i];
+          ch.bias[c][4 + i] = b1[i];
         }
-      }
-    }
-  };
-  // the pools do not hold the row's own key and value yet (or only just): the chunk that holds
-  // the row's position takes them from the registers
-  auto own = [&](int c0, Chunk& ch) {
-    if (!(own_kv && pos >= c0 && pos < c0 + D_KPW)) return;
+      } else {
 #pragma unroll
-    for (int c = 0; c < NCH; ++c) {
-      const int kb = c0 + 32 * c;
-#pragma unroll
-      for (int tt = 0; tt < 2; ++tt) {
-        if (kb + 8 * (col / 4) + 4 * tt + col % 4 == pos) {
-#pragma unroll
-          for (int ks = 0; ks < D_KS; ++ks) ch.kf[c][tt][ks] = k_new[ks];
-        }
-      }
-      const int e = pos - (kb + 8 * kg);
-      if (e >= 0 && e < 8) {
-        const uint32_t keep = (e & 1) ? 0x0000ffffu : 0xffff0000u;
-#pragma unroll
-        for (int mt = 0; mt < D_MT; ++mt) {
-          const uint32_t put = (v_new[mt] & 0xffffu) << ((e & 1) * 16);
-          uint32_t w[4] = {ch.vv[c][mt].x, ch.vv[c][mt].y, ch.vv[c][mt].z, ch.vv[c][mt].w};
-#pragma unroll
-          for (int i = 0; i < 4; ++i)
-            if (i == e / 2) w[i] = (w[i] & keep) | put;
-          ch.vv[c][mt] = (u32x4_t){w[0], w[1], w[2], w[3]};
-        }
+        for (int i = 0; i < 8; ++i) ch.bias[c][i] = 0.f;
       }
     }
   };
@@ -1347,7 +1565,7 @@ __device__ __forceinline__ void attn_decode_wave(
 #pragma unroll
     for (int c = 0; c < NCH; ++c) {
       if (c0 + 32 * c >= k_end) break;
-      const int kb = MODS ? kappai_key_at(c0 + 32 * c, lo32, kept) : c0 + 32 * c;
+      const int kb = kappai_key_at(c0 + 32 * c, lo32, kept);
       f32x4_t s[2];
 #pragma unroll
       for (int tt = 0; tt < 2; ++tt) {
@@ -1364,15 +1582,11 @@ __device__ __forceinline__ void attn_decode_wave(
 #pragma unroll
         for (int v = 0; v < 4; ++v) {
           const int key = kb + 8 * kg + 4 * tt + v;
-          const bool ok = (key >= lo || (MODS && key < keep)) && key <= hi;
-          if (MODS) {
-            float x = s[tt][v] * scale;
-            if (mods->softcap > 0.f) x = kappai_fast_cap(x, mods->softcap);
-            x += ch.bias[c][7 - (4 * tt + v)];
-            s[tt][v] = ok ? x * LOG2E : -INFINITY;
-          }
-          else
-            s[tt][v] = ok ? s[tt][v] * sc : -INFINITY;
+          const bool ok = (key >= lo || key < keep) && key <= hi;
+          float x = s[tt][v] * scale;
+          if (mods->softcap > 0.f) x = kappai_fast_cap(x, mods->softcap);
+          x += ch.bias[c][7 - (4 * tt + v)];
+          s[tt][v] = ok ? x * LOG2E : -INFINITY;
           mloc = fmaxf(mloc, s[tt][v]);
         }
       mloc = fmaxf(mloc, __shfl_xor(mloc, 16, WAVE));
@@ -1405,33 +1619,6 @@ __device__ __forceinline__ void attn_decode_wave(
   for (int c0 = first; c0 < k_end; c0 += stride) {
     Chunk ca;
     ask(c0, c0 == first ? pages_first : ask_pages(c0), ca);
-    if constexpr (FUSABLE && D_QK_FUSABLE) {
-      if (prologue_due) {
-        prologue_due = false;
-        if (own_kv) qk_norm_rotate(k_new, qk.k_norm_w != nullptr, tb.wk, qk.eps,
-                                   qk.cos_tab != nullptr, tb.cs, tb.sn);
-        qk_norm_rotate(qraw, qk.q_norm_w != nullptr, tb.wq, qk.eps, qk.cos_tab != nullptr, tb.cs,
-                       tb.sn);
-#pragma unroll
-        for (int ks = 0; ks < D_KS; ++ks)
-          qf[ks] = as_frag(head_ok ? qraw[ks] : (u32x4_t){0u, 0u, 0u, 0u});
-        if (owner) {
-          const size_t pg = (size_t)bt[pos / ps] * G + g;
-          if (col == 0) {
-#pragma unroll
-            for (int ks = 0; ks < D_KS; ++ks)
-              *reinterpret_cast<u32x4_t*>(qk.k_pool_w + (pg * ps + pos % ps) * HEAD_DIM + 32 * ks +
-                                          8 * kg) = k_new[ks];
-          }
-          if (kg == 0) {
-#pragma unroll
-            for (int mt = 0; mt < D_MT; ++mt)
-              qk.vt_pool_w[(pg * HEAD_DIM + 16 * mt + col) * ps + pos % ps] = (bf16_t)v_new[mt];
-          }
-        }
-      }
-    }
-    own(c0, ca);
     work(c0, ca);
   }
 }
@@ -1465,7 +1652,7 @@ __device__ __forceinline__ int step_keys_per_split(const int* __restrict__ row_p
   int kps = want > (1 << 30) ? (1 << 30) : (int)want;
   kps = max(kps, (longest + n_splits - 1) / n_splits);
   kps = max(kps, kps_min);
-  return (kps + D_KPW - 1) / D_KPW * D_KPW;
+  return (kps + 31) / 32 * 32;
 }
 
 // The keys of a row split over blocks: block (t, g, split) is one wave that takes the keys
@@ -1476,7 +1663,7 @@ __device__ __forceinline__ int step_keys_per_split(const int* __restrict__ row_p
 // (PLAN: the keys per split come from step_keys_per_split, else they are the caller's: a kernel of
 // its own, because the rule's code costs half a microsecond even where it is skipped)
 template <bool FUSED, bool PLAN, bool MODS = false>
-__global__ __launch_bounds__(64) void attn_decode_kernel(
+__global__ __launch_bounds__(64, FUSED || MODS || HEAD_DIM > 128 ? 1 : 2) void attn_decode_kernel(
     const bf16_t* __restrict__ q, int q_stride, const bf16_t* __restrict__ k_pool,
     const bf16_t* __restrict__ vt_pool, float* __restrict__ part_o, float* __restrict__ part_ml,
     const int* __restrict__ row_pos, const int* __restrict__ row_seg,
@@ -1511,9 +1698,12 @@ __global__ __launch_bounds__(64) void attn_decode_kernel(
   const size_t pbase = ((size_t)ti * H + h) * n_splits + split;
   f32x4_t o[D_MT];
   float m_run, l_run;
-  attn_decode_wave<FUSED, MODS>(q, q_stride, k_pool, vt_pool, bt, max_blocks, t, g, H, G, ps, scale,
-                                lo, k_end - 1, k_begin, D_KPW, k_end, o, m_run, l_run, qk, pos,
-                                &mods);
+  if constexpr (MODS)
+    attn_decode_scored_wave(q, q_stride, k_pool, vt_pool, bt, max_blocks, t, g, H, G, ps, scale, lo,
+                            k_end - 1, k_begin, D_KPW, k_end, o, m_run, l_run, pos, &mods);
+  else
+    attn_decode_wave<FUSED>(q, q_stride, k_pool, vt_pool, bt, max_blocks, t, g, H, G, ps, scale, lo,
+                            k_begin, k_end, o, m_run, l_run, qk, pos);
   if (!head_ok) return;
   if (kg == 0) {
     part_ml[2 * pbase] = m_run;
@@ -1535,32 +1725,32 @@ __global__ __launch_bounds__(64) void attn_decode_kernel(
 // (rows x kv heads) enough to fill the chip, or contexts short enough for one block.
 // LDS: sh_o [NW][rep][HEAD_DIM], then sh_m [NW][16], sh_l [NW][16] (floats).
 template <bool MODS>
-__global__ __launch_bounds__(D_BLOCK_MAX_WAVES * WAVE) void attn_decode_block_kernel(
-    const bf16_t* __restrict__ q, int q_stride, const bf16_t* __restrict__ k_pool,
-    const bf16_t* __restrict__ vt_pool, bf16_t* __restrict__ out, int out_stride,
-    const int* __restrict__ row_pos, const int* __restrict__ row_seg,
-    const int* __restrict__ block_tables, int max_blocks, int H, int G, int ps, int window,
-    float scale, kappai_score_mods mods) {
-  extern __shared__ float sh_dec[];
-  const int t = blockIdx.x, g = blockIdx.y;
-  const int lane = threadIdx.x % WAVE, wave = threadIdx.x / WAVE, NW = blockDim.x / WAVE;
+__device__ __forceinline__ void attn_one_row(const bf16_t* q, int q_stride, const bf16_t* k_pool,
+                                             const bf16_t* vt_pool, bf16_t* out, int out_stride,
+                                             const int* bt, int max_blocks, int t, int pos, int g, int H,
+                                             int G, int ps, int window, float scale,
+                                             const kappai_score_mods& mods, float* sh, int NW) {
+  const int lane = threadIdx.x % WAVE, wave = threadIdx.x / WAVE;
   const int rep = H / G;
   const int col = lane % 16, kg = lane / 16;
-  const int pos = row_pos[t];
-  const int* bt = block_tables + (size_t)row_seg[t] * max_blocks;
   const int lo = kappai_first_key(pos, window);
   const int lo32 = (lo / 32) * 32;
   const int k_begin = lo32 - (MODS ? kappai_kept_places(mods.keep_first, lo32) : 0);
   const int k_end = pos + 1;
   f32x4_t o[D_MT];
   float m_run, l_run;
-  // (without the prologue: eight waves a block leave no registers for it, and every wave would
-  // do it again)
-  attn_decode_wave<false, MODS>(q, q_stride, k_pool, vt_pool, bt, max_blocks, t, g, H, G, ps, scale,
-                                lo, pos, k_begin + wave * D_KPW, NW * D_KPW, k_end, o, m_run,
-                                l_run, QkFuse{}, pos, &mods);
-  float* sh_o = sh_dec;
-  float* sh_m = sh_dec + (size_t)NW * rep * HEAD_DIM;
+  if constexpr (MODS) {
+    attn_decode_scored_wave(q, q_stride, k_pool, vt_pool, bt, max_blocks, t, g, H, G, ps, scale, lo, pos,
+                            k_begin + wave * D_KPW, NW * D_KPW, k_end, o, m_run, l_run, pos, &mods);
+  } else {
+    // equal shares in whole parts of 32 keys
+    const int per = ((k_end - k_begin + 31) / 32 + NW - 1) / NW * 32;
+    const int from = k_begin + wave * per;
+    attn_decode_wave<false>(q, q_stride, k_pool, vt_pool, bt, max_blocks, t, g, H, G, ps, scale, lo, from,
+                            min(from + per, k_end), o, m_run, l_run, QkFuse{}, pos);
+  }
+  float* sh_o = sh;
+  float* sh_m = sh + (size_t)NW * rep * HEAD_DIM;
   float* sh_l = sh_m + NW * 16;
   if (col < rep) {
     float* po = sh_o + ((size_t)wave * rep + col) * HEAD_DIM;
@@ -1574,7 +1764,7 @@ __global__ __launch_bounds__(D_BLOCK_MAX_WAVES * WAVE) void attn_decode_block_ke
   }
   __syncthreads();
   // out[t, g rep + c, e] for (c, e) in turn over the block's threads
-  for (int i = threadIdx.x; i < rep * HEAD_DIM; i += blockDim.x) {
+  for (int i = threadIdx.x; i < rep * HEAD_DIM; i += NW * WAVE) {
     const int c = i / HEAD_DIM, e = i % HEAD_DIM;
     float M = -INFINITY;
     for (int w = 0; w < NW; ++w) M = fmaxf(M, sh_m[w * 16 + c]);
@@ -1590,6 +1780,20 @@ __global__ __launch_bounds__(D_BLOCK_MAX_WAVES * WAVE) void attn_decode_block_ke
     const float inv = L > 0.f ? 1.0f / L : 0.f;
     out[(size_t)t * out_stride + (size_t)(g * rep + c) * HEAD_DIM + e] = f32_to_bf16(acc * inv);
   }
+}
+
+template <bool MODS>
+__global__ __launch_bounds__(D_BLOCK_MAX_WAVES * WAVE) void attn_decode_block_kernel(
+    const bf16_t* __restrict__ q, int q_stride, const bf16_t* __restrict__ k_pool,
+    const bf16_t* __restrict__ vt_pool, bf16_t* __restrict__ out, int out_stride,
+    const int* __restrict__ row_pos, const int* __restrict__ row_seg,
+    const int* __restrict__ block_tables, int max_blocks, int H, int G, int ps, int window,
+    float scale, kappai_score_mods mods) {
+  extern __shared__ float sh_dec[];
+  const int t = blockIdx.x;
+  attn_one_row<MODS>(q, q_stride, k_pool, vt_pool, out, out_stride,
+                     block_tables + (size_t)row_seg[t] * max_blocks, max_blocks, t, row_pos[t],
+                     blockIdx.y, H, G, ps, window, scale, mods, sh_dec, blockDim.x / WAVE);
 }
 
 // out[t, h, :] = sum_s o_s 2^(m_s - M) / sum_s l_s 2^(m_s - M).  Four waves share the splits

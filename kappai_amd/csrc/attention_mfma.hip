@@ -138,12 +138,15 @@ __device__ __forceinline__ u32x4_t load_k8(const bf16_t* __restrict__ k_pool,
 
 // One row and one kv head by a block of NW waves, which take the keys in chunks in turn and meet in `sh`
 // (NW (rep HEAD_DIM + 32) floats of LDS; rep <= 16): defined with the decode kernels.
-template <bool MODS>
+// (FUSED: with the prologue of `qk` in the waves that have keys)
+struct QkFuse;
+template <bool MODS, bool FUSED = false>
 __device__ __forceinline__ void attn_one_row(const bf16_t* q, int q_stride, const bf16_t* k_pool,
                                              const bf16_t* vt_pool, bf16_t* out, int out_stride,
                                              const int* bt, int max_blocks, int t, int pos, int g, int H,
                                              int G, int ps, int window, float scale,
-                                             const kappai_score_mods& mods, float* sh, int NW);
+                                             const kappai_score_mods& mods, float* sh, int NW,
+                                             const QkFuse* qk = nullptr);
 
 // waves of a block: they share one q tile and take its key tiles in turn, which shortens the
 // longest chain of dependent work fourfold; their partial results meet in LDS
@@ -1724,12 +1727,13 @@ __global__ __launch_bounds__(64, FUSED || MODS || HEAD_DIM > 128 ? 1 : 2) void a
 // keys depends on the row's own position and on the number of waves only.  For batches with
 // (rows x kv heads) enough to fill the chip, or contexts short enough for one block.
 // LDS: sh_o [NW][rep][HEAD_DIM], then sh_m [NW][16], sh_l [NW][16] (floats).
-template <bool MODS>
+template <bool MODS, bool FUSED>
 __device__ __forceinline__ void attn_one_row(const bf16_t* q, int q_stride, const bf16_t* k_pool,
                                              const bf16_t* vt_pool, bf16_t* out, int out_stride,
                                              const int* bt, int max_blocks, int t, int pos, int g, int H,
                                              int G, int ps, int window, float scale,
-                                             const kappai_score_mods& mods, float* sh, int NW) {
+                                             const kappai_score_mods& mods, float* sh, int NW,
+                                             const QkFuse* qk) {
   const int lane = threadIdx.x % WAVE, wave = threadIdx.x / WAVE;
   const int rep = H / G;
   const int col = lane % 16, kg = lane / 16;
@@ -1746,8 +1750,16 @@ __device__ __forceinline__ void attn_one_row(const bf16_t* q, int q_stride, cons
     // equal shares in whole parts of 32 keys
     const int per = ((k_end - k_begin + 31) / 32 + NW - 1) / NW * 32;
     const int from = k_begin + wave * per;
-    attn_decode_wave<false>(q, q_stride, k_pool, vt_pool, bt, max_blocks, t, g, H, G, ps, scale, lo, from,
-                            min(from + per, k_end), o, m_run, l_run, QkFuse{}, pos);
+    if (FUSED && from >= k_end) {              // (no keys: no prologue either)
+#pragma unroll
+      for (int mt = 0; mt < D_MT; ++mt) o[mt] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
+      m_run = -INFINITY;
+      l_run = 0.f;
+    } else {
+      attn_decode_wave<FUSED>(q, q_stride, k_pool, vt_pool, bt, max_blocks, t, g, H, G, ps, scale, lo,
+                              from, min(from + per, k_end), o, m_run, l_run,
+                              FUSED ? *qk : QkFuse{}, pos);
+    }
   }
   float* sh_o = sh;
   float* sh_m = sh + (size_t)NW * rep * HEAD_DIM;
@@ -1795,6 +1807,25 @@ __global__ __launch_bounds__(D_BLOCK_MAX_WAVES * WAVE) void attn_decode_block_ke
                      block_tables + (size_t)row_seg[t] * max_blocks, max_blocks, t, row_pos[t],
                      blockIdx.y, H, G, ps, window, scale, mods, sh_dec, blockDim.x / WAVE);
 }
+
+// attn_decode_block_kernel with the prologue of QkFuse in the waves that have keys (see
+// D_QK_BLOCK_MAX_KEYS).
+#if HEAD_DIM == 64
+__global__ __launch_bounds__(D_BLOCK_MAX_WAVES * WAVE) void attn_decode_block_qk_kernel(
+    const bf16_t* __restrict__ qkv, int row_stride, const bf16_t* __restrict__ k_pool,
+    const bf16_t* __restrict__ vt_pool, bf16_t* __restrict__ out, int out_stride,
+    const int* __restrict__ row_pos, const int* __restrict__ row_seg,
+    const int* __restrict__ block_tables, int max_blocks, int H, int G, int ps, int window,
+    float scale, QkFuse qk) {
+  extern __shared__ float sh_dec[];
+  const int t = blockIdx.x;
+  attn_one_row<false, true>(qkv, row_stride, k_pool, vt_pool, out, out_stride,
+                            block_tables + (size_t)row_seg[t] * max_blocks, max_blocks, t, row_pos[t],
+                            blockIdx.y, H, G, ps, window, scale,
+                            kappai_score_mods{0.f, nullptr, 0, nullptr, 0}, sh_dec,
+                            blockDim.x / WAVE, &qk);
+}
+#endif
 
 // out[t, h, :] = sum_s o_s 2^(m_s - M) / sum_s l_s 2^(m_s - M).  Four waves share the splits
 // (wave w takes s = w, w+4, ...); each computes its splits' weights one per lane.  The partial
@@ -1953,6 +1984,14 @@ extern "C" int kappai_attn_decode_block(const void* q, int q_stride, const void*
 // norm, the rotation and the storing of the rows' own keys and values itself
 // (kappai_attn_decode_qk)
 extern "C" int kappai_attn_decode_takes_qk(void) { return D_QK_FUSABLE ? 1 : 0; }
+
+// The most keys with which kappai_attn_decode_qk keeps a row's keys in one block (0: never at this head
+// size).  One kernel in the place of two, but a CU takes in no more than about 50 GB/s of keys.  1 to 4 rows
+// of 8 kv heads, us against split and merge: 40 keys 6.0 / 8.4, 307 keys 7.7 / 8.5, 614 keys 8.8 / 9.7,
+// 1,024 keys 10.8 / 9.0; a captured step knows its contexts as powers of two only, so the line is at 512.  Head
+// size 128 has no registers for prologue and keys at two waves a SIMD (40 keys 9.9 / 10.6, 307 keys 15.2 / 10.6).
+#define D_QK_BLOCK_MAX_KEYS (HEAD_DIM == 64 ? 512 : 0)
+extern "C" int kappai_attn_decode_block_qk_keys(void) { return D_QK_BLOCK_MAX_KEYS; }
 
 // The arguments that kappai_attn_decode_qk adds: qkv [T, row_stride] is the projection as it
 // comes out of its product (q heads, then with store_kv the k heads and the v heads); q_norm_w /
@@ -2135,6 +2174,19 @@ extern "C" int kappai_attn_decode_qk(const void* qkv, int row_stride, void* k_po
     return (int)hipErrorInvalidValue;
   const QkFuse qk{1, store_kv ? 1 : 0, q_norm_w, k_norm_w, eps, cos_tab, sin_tab, (bf16_t*)k_pool,
                   (bf16_t*)vt_pool};
+#if HEAD_DIM == 64
+  const int n_waves = G > 0 && H % G == 0 ? kappai_attn_decode_block_waves(H / G) : 0;
+  if (T > 0 && n_waves > 0 && keys_per_split > 0 && n_splits > 0 &&
+      (long long)keys_per_split * n_splits <= D_QK_BLOCK_MAX_KEYS) {
+    if (ps % 16 || G > 65535) return (int)hipErrorInvalidValue;
+    const size_t lds = (size_t)n_waves * (H / G * HEAD_DIM + 32) * sizeof(float);
+    hipLaunchKernelGGL(attn_decode_block_qk_kernel, dim3(T, G), dim3(n_waves * WAVE), lds, stream,
+                       (const bf16_t*)qkv, row_stride, (const bf16_t*)k_pool,
+                       (const bf16_t*)vt_pool, (bf16_t*)out, out_stride, row_pos, row_seg,
+                       block_tables, max_blocks, H, G, ps, window, scale, qk);
+    KAPPAI_RETURN_LAUNCH_STATUS();
+  }
+#endif
   return launch_decode(qkv, row_stride, k_pool, vt_pool, out, out_stride, part_o, part_ml, row_pos,
                        row_seg, block_tables, max_blocks, T, H, G, ps, window, scale,
                        keys_per_split, n_splits, qk, nullptr, stream);

@@ -87,6 +87,8 @@ typedef struct kappai_attention_kernels {
   // the store of the rows' own keys and values in its prologue (decode_takes_qk() says whether
   // this head size has it)
   int (*decode_takes_qk)(void);
+  // the most keys with which attn_decode_qk keeps a row's keys in one block, 0: never
+  int (*decode_block_qk_keys)(void);
   int (*attn_decode_qk)(const void*, int, void*, void*, void*, int, float*, float*, const int*,
                         const int*, const int*, int, int, int, int, int, int, float, int, int,
                         const float*, const float*, float, const float*, const float*, int,
@@ -331,6 +333,10 @@ const char* kappai_forward_error(void);
 // How many K ranges a product of these sizes is cut into when its consumer adds partial sums (the
 // host's parts ask the same function).
 int kappai_split_k_for(int M, int N, int K);
+
+// The most keys with which the decode attention keeps a row's keys in one block (attn_decode_block) where
+// `few` is what it takes for any number of rows.
+int kappai_decode_block_keys(int few, int rows, int G, int head_dim);
 
 // How the decode attention that splits a row's keys over blocks cuts n_keys keys of `rows` rows
 // over G kv heads: the fewest keys a split and the most splits a row (the host asks the same

@@ -588,6 +588,22 @@ extern "C" const char* kappai_forward_error(void) { return g_error; }
 
 extern "C" int kappai_split_k_for(int M, int N, int K) { return split_k_for(M, N, K); }
 
+// One block a (row, kv head) takes a row's keys in at 50 GB/s or so, but needs no second kernel, and with
+// blocks enough for the chip nothing is won by more of them.  us against the kernel that splits the keys over
+// blocks and its merge, head size 64, 8 kv heads: 8 rows of 40 / 307 / 1,024 keys 4.4 / 6.5 / 9.1 against
+// 6.8 / 8.0 / 9.5 (2,048 keys 13.5 / 11.0); 24 rows of up to 614 / 2,048 keys 8.3 / 17.1 against 12.2 / 18.3
+// (16 rows 14.8 / 13.6); 32 rows of up to 1,228 / 4,096 keys 12.3 / 35.2 against 16.3 / 36.4, 64 rows 25.2 / 67.7
+// against 26.7 / 64.9.  A key of 128 is twice the bytes: 64 rows, 4 kv heads, up to 2,048 keys 35.3 against 37.8.
+// Head sizes beyond (three waves a block, registers spilled) lose from the first key on: 20 against 9.7.
+extern "C" int kappai_decode_block_keys(int few, int rows, int G, int head_dim) {
+  if (head_dim > 128) return 0;
+  if (head_dim != 64 && head_dim != 128) return few;
+  const long blocks = (long)rows * G;
+  const int at64 = blocks >= 256 ? 4096 : (blocks >= 192 ? 2048 : (blocks >= 64 ? 1024 : few));
+  const int keys = at64 * 64 / head_dim;
+  return keys > few ? keys : few;
+}
+
 extern "C" void kappai_decode_splits(int keys_per_wave, int max_splits, int waves, int rows, int G,
                                      int n_keys, int* keys_per_split, int* n_splits) {
   decode_splits(keys_per_wave, max_splits, waves, rows, G, n_keys, keys_per_split, n_splits);

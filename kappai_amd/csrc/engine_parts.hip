@@ -153,9 +153,10 @@ int decode_keys(const kappai_batch& b, const kappai_attention_mixer& L) {
   return n_keys;
 }
 bool decode_block_form(const kappai_model& m, const kappai_batch& b,
-                       const kappai_attention_mixer& L, int rep) {
-  return L.mfma->decode_block_waves(rep) > 0 &&
-         decode_keys(b, L) <= m.tuning.decode_block_max_keys;
+                       const kappai_attention_mixer& L, int M) {
+  return L.mfma->decode_block_waves(L.heads / L.kv_heads) > 0 &&
+         decode_keys(b, L) <= kappai_decode_block_keys(m.tuning.decode_block_max_keys, M, L.kv_heads,
+                                                       L.head_dim);
 }
 
 kappai_carry attention_mixer(kappai_step* s, const void* desc, kappai_rows x, float* resid,
@@ -202,7 +203,9 @@ kappai_carry attention_mixer(kappai_step* s, const void* desc, kappai_rows x, fl
       L.mfma != nullptr && H / G <= 16 && qkv.n % 8 == 0 && aligned16(proj.data) && ps % 16 == 0 &&
       d % 16 == 0 && d <= 256 && (L.rot_mode == 0 || (L.rot_mode == 1 && L.rot_dim == d)) &&
       L.mfma->decode_takes_qk != nullptr && L.mfma->decode_takes_qk() &&
-      !decode_block_form(m, b, L, H / G);
+      (!decode_block_form(m, b, L, M) ||
+       (L.mfma->decode_block_qk_keys != nullptr &&
+        decode_keys(b, L) <= L.mfma->decode_block_qk_keys()));
   // q in place in the projection, or (from partial sums) a new bfloat16 [M, H d]
   void* q;
   int q_stride, q_bf16;
@@ -245,7 +248,7 @@ kappai_carry attention_mixer(kappai_step* s, const void* desc, kappai_rows x, fl
   if (mfma_ok && single && H / G <= 16) {
     const int n_keys = decode_keys(b, L);
     const int block_waves = L.mfma->decode_block_waves(H / G);
-    if (decode_block_form(m, b, L, H / G)) {
+    if (!qk_in_kernel && decode_block_form(m, b, L, M)) {
       LAUNCH(s, L.mfma->attn_decode_block(q, q_stride, L.k_pool, L.v_pool, ctx, H * d, b.row_pos,
                                           b.row_seg, tables, max_blocks, M, H, G, ps, L.window,
                                           L.scale, block_waves, stream));

@@ -22,7 +22,9 @@ from .batch import HostStep, RowBatch, StepEntry, build_step_tables, layout_rows
 from .cforward import CForward, NotDescribed, Workspace
 
 
-CONTEXT_BUCKET_MIN = 1024     # decode graphs are captured for contexts up to a power of two
+# Decode graphs are captured for contexts up to a power of two, from this one on (the most keys that
+# attention keeps in one block for any number of rows: kappai_decode_block_keys in csrc/engine.hip)
+CONTEXT_BUCKET_MIN = 512
 DECODE_RING = 8            # decode steps whose tables can be queued ahead of the GPU
 MAX_DECODE_GRAPHS = 48
 

@@ -21,10 +21,8 @@ DECODE_WAVES = 4096       # blocks the grid of the split-key decode attention pr
                           # kernel itself aims at half as many at work, counting the keys the
                           # rows really hold (requests of mixed lengths get shorter splits)
 DECODE_MAX_SPLITS = 128   # partial results of a row's head that the merge kernel adds up at most
-# Keys up to which one block a (row, kv head) takes them all, its waves merging in LDS (8 requests
-# at 200 keys: 7.4 us against 9.4 for the split kernel and its merge; even at 1024 keys, and from
-# there on the split kernel wins: 22 against 35 us at 4096 keys, a wave taking its chunks one
-# after the other where the split kernel has a wave for each)
+# Keys up to which one block a (row, kv head) takes them all, its waves merging in LDS, however few
+# the rows; with more rows up to more keys (kappai_decode_block_keys in csrc/engine.hip, measured there)
 DECODE_BLOCK_MAX_KEYS = 512
 
 _c_int, _c_float, _c_long, _vp = ctypes.c_int, ctypes.c_float, ctypes.c_long, ctypes.c_void_p
@@ -915,14 +913,17 @@ def keys_bound(max_position: int, window: int, keep_first: int = 0) -> int:
 
 
 def decode_form(n_heads: int, n_kv_heads: int, head_dim: int, max_position: int,
-                window: int = 0, keep_first: int = 0) -> str:
-    """Which of the two decode kernels a step takes: with few keys ("decode-block") a block per
-    (row, kv head) splits them over its waves and merges in LDS; else ("decode-split") the keys
-    are split over blocks, whose partial results a second kernel merges."""
+                window: int = 0, keep_first: int = 0, n_rows: int = 1, scored: bool = False) -> str:
+    """Which of the two decode kernels a step of ``n_rows`` takes: with few keys ("decode-block") a
+    block per (row, kv head) splits them over its waves and merges in LDS; else ("decode-split") the
+    keys are split over blocks, whose partial results a second kernel merges.  ``scored``: the scores
+    are worked on (``ScoreMods``), which few keys alone send to one block."""
     n_keys = keys_bound(max_position, window, keep_first)
     lib = library("attention_mfma", HEAD_DIM=head_dim)
     block_waves = lib.kappai_attn_decode_block_waves(n_heads // n_kv_heads)
-    return "decode-block" if block_waves and n_keys <= DECODE_BLOCK_MAX_KEYS else "decode-split"
+    most = DECODE_BLOCK_MAX_KEYS if scored else library("engine").kappai_decode_block_keys(
+        _c_int(DECODE_BLOCK_MAX_KEYS), _c_int(n_rows), _c_int(n_kv_heads), _c_int(head_dim))
+    return "decode-block" if block_waves and n_keys <= most else "decode-split"
 
 
 def decode_takes_qk(head_dim: int, page_size: int) -> bool:
@@ -931,6 +932,12 @@ def decode_takes_qk(head_dim: int, page_size: int) -> bool:
     if head_dim % 16 or head_dim > 256 or page_size % 16:
         return False
     return bool(library("attention_mfma", HEAD_DIM=head_dim).kappai_attn_decode_takes_qk())
+
+
+def decode_block_takes_qk(head_dim: int, max_position: int, window: int = 0) -> bool:
+    """Whether a ``QkPrologue`` finds few enough keys for the kernel that keeps them in one block."""
+    return (keys_bound(max_position, window)
+            <= library("attention_mfma", HEAD_DIM=head_dim).kappai_attn_decode_block_qk_keys())
 
 
 def paged_attention(q: torch.Tensor, n_heads: int, n_kv_heads: int, head_dim: int,
@@ -1066,7 +1073,7 @@ def paged_attention(q: torch.Tensor, n_heads: int, n_kv_heads: int, head_dim: in
     block_waves = lib.kappai_attn_decode_block_waves(H // G)
     if kernel == "decode":
         kernel = ("decode-split" if qk is not None
-                  else decode_form(H, G, d, max_position, window, keep))
+                  else decode_form(H, G, d, max_position, window, keep, T, mods is not None))
     if kernel == "decode-block":
         _need(block_waves > 0, "too many query heads a kv head for the block form")
         _need(qk is None, "the decode kernel that keeps a row's keys in one block takes q ready "

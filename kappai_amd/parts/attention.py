@@ -221,8 +221,8 @@ class GroupedQueryAttention(Mixer):
         ``ops.QkPrologue``): a step of a few single rows whose projection came as bfloat16 rows, few
         enough query heads a kv head for the decode kernels, a head size they do it for, no
         rotation or rotate-half over the whole head, and keys enough for the kernel that splits
-        them over blocks (where a block is one wave; in the other every wave of a block would do
-        the prologue again, which costs what the kernel saved)."""
+        them over blocks or few enough for the one that keeps them in a block
+        (``ops.decode_block_takes_qk``)."""
         if not (tuning.FUSED_QK and single_rows and isinstance(proj, torch.Tensor)
                 and proj.dim() == 2 and proj.shape[0] <= tuning.FUSED_QK_MAX_ROWS
                 and proj.dtype == torch.bfloat16 and proj.is_cuda
@@ -231,9 +231,11 @@ class GroupedQueryAttention(Mixer):
             return False
         if rot is not None and not (rot.mode == ops.ROT_HALF and rot.rot_dim == self.d):
             return False
+        window = self.window or 0
         return (ops.decode_takes_qk(self.d, page_size)
-                and ops.decode_form(self.H, self.G, self.d, max_position,
-                                    self.window or 0) == "decode-split")
+                and (ops.decode_form(self.H, self.G, self.d, max_position, window,
+                                     n_rows=proj.shape[0]) == "decode-split"
+                     or ops.decode_block_takes_qk(self.d, max_position, window)))
 
     def weight_bytes(self) -> int:
         return self.qkv.weight_bytes() + self.out.weight_bytes() + 2 * self.d * 4

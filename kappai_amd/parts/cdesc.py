@@ -72,7 +72,8 @@ class EmbeddedPartDesc(Structure):
 class AttentionKernels(Structure):
     _fields_ = [(n, c_void_p) for n in
                 ("keys_per_wave", "decode_block_waves", "attn_prefill", "attn_decode",
-                 "attn_decode_block", "attn_decode_rows", "decode_takes_qk", "attn_decode_qk")]
+                 "attn_decode_block", "attn_decode_rows", "decode_takes_qk",
+                 "decode_block_qk_keys", "attn_decode_qk")]
 
 
 def address_of(fn) -> int:
@@ -218,6 +219,7 @@ class CPlan:
                                   ("attn_decode_block", "kappai_attn_decode_block"),
                                   ("attn_decode_rows", "kappai_attn_decode_rows"),
                                   ("decode_takes_qk", "kappai_attn_decode_takes_qk"),
+                                  ("decode_block_qk_keys", "kappai_attn_decode_block_qk_keys"),
                                   ("attn_decode_qk", "kappai_attn_decode_qk")):
                 setattr(a, field, address_of(getattr(lib, symbol)))
             self._mfma[head_dim] = self.keep(a)

@@ -44,6 +44,10 @@ typedef struct kappai_kernels {
   int (*sum_partials)(const float*, int, long, float*, hipStream_t);
   int (*gemm_f32)(const float*, const float*, const float*, float*, int, int, int, int, int,
                   hipStream_t);
+  // gate and up in 32 bits with the gate applied: rows, results and K that it takes, and the product
+  int (*gemm_f32_gates)(int, int, int);
+  int (*gemm_f32_swiglu)(const float*, const float*, const float*, float*, int, int, int, int, int,
+                         hipStream_t);
   int (*gemm_bf16)(const void*, const void*, const void*, const float*, void*, int, int, int, int,
                    int, int, int, int, int, const float*, int, float, float*, int, const float*,
                    void*, int, float*, hipStream_t);

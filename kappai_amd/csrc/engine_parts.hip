@@ -325,6 +325,15 @@ kappai_carry swiglu_ffn(kappai_step* s, const void* desc, kappai_rows x, float* 
     ar.frag = c_frag;
     return api.linear(s, ar, &L.down, m.compute_bf16, 1, into, region);
   }
+  // float rows and matrix: the product's own epilogue, with the bits of the two kernels
+  if (!L.fused && !x.is_bf16 && !m.compute_bf16 && L.gate_up.w_is_f32 && L.gate_up.w != nullptr &&
+      L.gate_up.k == D && L.gate_up.n == 2 * F && !x.frag && x.ss == nullptr && x.D == D &&
+      k.gemm_f32_gates(M, F, D)) {
+    float* act = (float*)api.take(s, KAPPAI_REGION_BLOCK, (size_t)M * F * 4);
+    LAUNCH(s, k.gemm_f32_swiglu((const float*)x.data, (const float*)L.gate_up.w, L.gate_up.bias, act, M, F, D,
+                                M > 1 ? x.ld : D, F, api.stream(s)));
+    return api.linear(s, rows_of(act, M, F, 0), &L.down, m.compute_bf16, 1, into, region);
+  }
   kappai_carry gu = api.linear(s, x, &L.gate_up, m.compute_bf16, 0, nullptr, KAPPAI_REGION_BLOCK);
   if (!api.ok(s)) return none;
   const int act_bf16 = gu.is_f32 ? 0 : 1;

@@ -59,6 +59,9 @@ __device__ __forceinline__ int f32_run_start(int run, int runs, int chunks) {
   return run * chunks / runs;
 }
 
+// The gate as kappai_swiglu computes it.
+__device__ __forceinline__ float f32_gate(float g, float u) { return g / (1.0f + expf(-g)) * u; }
+
 // Four values of a row from k on; zeros from K on.
 template <int LOADS>
 __device__ __forceinline__ f32x4_t load4_f32(const float* __restrict__ row, int k, int K) {
@@ -102,7 +105,10 @@ __device__ __forceinline__ void load_chunk_f32(const float* __restrict__ row, in
 // of W is under way while a chunk is multiplied.  Three rows, W from memory: 9216 x 1024 12 us
 // (3.1 TB/s), 1024 x 4608 9 us, 65536 x 1024 51 us (5.3 TB/s); the vector kernel before took 100 to
 // 1,500 us, a block a 64 x 64 tile of which three rows were real.
-template <int MT, int COLS, int RUNS, int LOADS>
+//
+// GATED: W holds 2 N rows, gate rows and behind them the up rows; a block's 16 columns are the gates of 8
+// results and their up rows, C[m, n] = silu(gate) up, the bits of the product and kappai_swiglu behind it.
+template <int MT, int COLS, int RUNS, int LOADS, bool GATED = false>
 __global__ __launch_bounds__((COLS == 8 ? RUNS / 2 : 8) * WAVE) void gemm_f32_skinny_kernel(
     const float* __restrict__ A, const float* __restrict__ W, const float* __restrict__ bias,
     float* __restrict__ C, int M, int N, int K, int lda, int ldc) {
@@ -112,8 +118,10 @@ __global__ __launch_bounds__((COLS == 8 ? RUNS / 2 : 8) * WAVE) void gemm_f32_sk
   __shared__ float red[RUNS][MT][SIDE ? 8 : 16][COLS];
   const int wave = threadIdx.x / WAVE, lane = threadIdx.x % WAVE;
   const int r = lane % 16, q = lane / 16;
-  const int n0 = blockIdx.x * COLS;
-  const float* w = W + (size_t)min(n0 + r % COLS, N - 1) * K;
+  static_assert(!GATED || COLS == 16, "eight gates and their up rows");
+  const int n0 = blockIdx.x * (GATED ? 8 : COLS);
+  const float* w = W + (GATED ? (size_t)(r / 8) * N + min(n0 + r % 8, N - 1)
+                              : (size_t)min(n0 + r % COLS, N - 1)) * K;
   const float* a[MT];
 #pragma unroll
   for (int mt = 0; mt < MT; ++mt)
@@ -205,13 +213,18 @@ __global__ __launch_bounds__((COLS == 8 ? RUNS / 2 : 8) * WAVE) void gemm_f32_sk
     while (run < run0 + per) write_run();
   }
   __syncthreads();
-  for (int at = threadIdx.x; at < MT * (SIDE ? 8 : 16) * COLS; at += NW * WAVE) {
-    const int m = at / COLS, n = n0 + at % COLS;
-    if (m >= M || n >= N) continue;
-    float s = red[0][m / 16][m % 16][at % COLS];
+  const auto whole = [&](int m, int col, int row) {
+    float s = red[0][m / 16][m % 16][col];
 #pragma unroll
-    for (int g = 1; g < RUNS; ++g) s += red[g][m / 16][m % 16][at % COLS];
-    C[(size_t)m * ldc + n] = s + (bias ? bias[n] : 0.f);
+    for (int g = 1; g < RUNS; ++g) s += red[g][m / 16][m % 16][col];
+    return s + (bias ? bias[row] : 0.f);
+  };
+  constexpr int OUT = GATED ? 8 : COLS;
+  for (int at = threadIdx.x; at < MT * (SIDE ? 8 : 16) * OUT; at += NW * WAVE) {
+    const int m = at / OUT, n = n0 + at % OUT;
+    if (m >= M || n >= N) continue;
+    const float s = whole(m, at % OUT, n);
+    C[(size_t)m * ldc + n] = GATED ? f32_gate(s, whole(m, at % OUT + 8 * GATED, N + n)) : s;
   }
 }
 
@@ -223,7 +236,9 @@ __global__ __launch_bounds__((COLS == 8 ? RUNS / 2 : 8) * WAVE) void gemm_f32_sk
 // vector registers, and one wave multiplies while the other waits for LDS.  825 rows: 9216 x 1024
 // 165 us (94 TFLOP/s; the instruction alone reaches 153), 3072 x 1024 66 us, 2048 x 1024 45, 1024 x 4608
 // 101 (with four waves a block of 64 x 64, one a SIMD: 75, 46 and 107).
-template <int WY, int WX, int TY, int TX, int BK, int LOADS>
+//
+// GATED (wave tiles of two 16s of columns): the second 16 of every 32 columns are the up rows of the first.
+template <int WY, int WX, int TY, int TX, int BK, int LOADS, bool GATED = false>
 __global__ __launch_bounds__(WY * WX * WAVE) __attribute__((amdgpu_waves_per_eu(2)))
 void gemm_f32_block_kernel(
     const float* __restrict__ A, const float* __restrict__ W, const float* __restrict__ bias,
@@ -236,7 +251,8 @@ void gemm_f32_block_kernel(
   const int r = lane % 16, q = lane / 16;
   const int wm = wave / WX * 16 * TY, wn = wave % WX * 16 * TX;
   const int m0 = (int)(blockIdx.x / 8) % tiles_m * BM;
-  const int n0 = ((int)(blockIdx.x / 8) / tiles_m * 8 + (int)(blockIdx.x % 8)) * BN;
+  static_assert(!GATED || TX == 2, "a wave has the gates and the up rows of its results");
+  const int n0 = ((int)(blockIdx.x / 8) / tiles_m * 8 + (int)(blockIdx.x % 8)) * (GATED ? BN / 2 : BN);
   if (n0 >= N) return;
 
   const float* src[2][PER];
@@ -246,7 +262,8 @@ void gemm_f32_block_kernel(
   for (int p = 0; p < PER; ++p) {
     const int row = (tid + NT * p) / SLOTS;
     src[0][p] = A + (size_t)min(m0 + row, M - 1) * lda;
-    src[1][p] = W + (size_t)min(n0 + row, N - 1) * K;
+    src[1][p] = W + (GATED ? (size_t)(row / 16 % 2) * N + min(n0 + row / 32 * 16 + row % 16, N - 1)
+                           : (size_t)min(n0 + row, N - 1)) * K;
     at[p] = row * SLOTS + (slot ^ (row & 7));
   }
   f32x4_t next[2][PER];
@@ -335,6 +352,19 @@ void gemm_f32_block_kernel(
         }
     }
   }
+  if constexpr (GATED) {
+    const int n = n0 + wn / 2 + r;
+    if (n >= N) return;
+    const float bg = bias ? bias[n] : 0.f, bu = bias ? bias[N + n] : 0.f;
+#pragma unroll
+    for (int i = 0; i < TY; ++i)
+#pragma unroll
+      for (int x = 0; x < 4; ++x) {
+        const int m = m0 + wm + 16 * i + 4 * q + x;
+        if (m < M) C[(size_t)m * ldc + n] = f32_gate(fin[i][0][x] + bg, fin[i][TX - 1][x] + bu);
+      }
+    return;
+  }
 #pragma unroll
   for (int j = 0; j < TX; ++j) {
     const int n = n0 + wn + 16 * j + r;
@@ -350,13 +380,43 @@ void gemm_f32_block_kernel(
   }
 }
 
-template <int LOADS, int TY, int TX>
+template <int LOADS, int TY, int TX, bool GATED = false>
 static void launch_f32_blocks(const float* A, const float* W, const float* bias, float* C, int M,
                               int N, int K, int lda, int ldc, hipStream_t stream) {
   constexpr int B = 32 * TY;
-  const int tm = (M + B - 1) / B, tn = (N + B - 1) / B;
-  hipLaunchKernelGGL((gemm_f32_block_kernel<2, 4, TY, TX, 64, LOADS>), dim3((tn + 7) / 8 * 8 * tm),
+  const int tm = (M + B - 1) / B, tn = ((GATED ? 2 : 1) * N + B - 1) / B;
+  hipLaunchKernelGGL((gemm_f32_block_kernel<2, 4, TY, TX, 64, LOADS, GATED>), dim3((tn + 7) / 8 * 8 * tm),
                      dim3(512), 0, stream, A, W, bias, C, M, N, K, lda, ldc, tm);
+}
+
+static bool f32_large_blocks(int M, int N) {
+  const auto tiles = [](int n, int b) { return (n + b - 1) / b; };
+  const long big = (long)tiles(M, 128) * tiles(N, 128), small = (long)tiles(M, 64) * tiles(N, 64);
+  return (big + 255) / 256 * 4 * 8 <= (small + 255) / 256 * 9;
+}
+
+template <int LOADS>
+static void launch_f32_gated(const float* A, const float* W, const float* bias, float* C, int M, int F, int K,
+                             int lda, int ldc, hipStream_t stream) {
+  if (M > 64) {
+    launch_f32_blocks<LOADS, 4, 2, true>(A, W, bias, C, M, F, K, lda, ldc, stream);
+    return;
+  }
+  const bool many = f32_runs((K + F32_CHUNK - 1) / F32_CHUNK) == 32;
+#define F32_GATED(MT, RUNS)                                                                          \
+  hipLaunchKernelGGL((gemm_f32_skinny_kernel<MT, 16, RUNS, LOADS, true>), dim3((F + 7) / 8),         \
+                     dim3(8 * WAVE), 0, stream, A, W, bias, C, M, F, K, lda, ldc)
+  if (M <= 16) {
+    if (many) F32_GATED(1, 32);
+    else F32_GATED(1, 8);
+  } else if (M <= 32) {
+    if (many) F32_GATED(2, 32);
+    else F32_GATED(2, 8);
+  } else {
+    if (many) F32_GATED(4, 32);
+    else F32_GATED(4, 8);
+  }
+#undef F32_GATED
 }
 
 template <int LOADS>
@@ -384,9 +444,7 @@ static void launch_f32(const float* A, const float* W, const float* bias, float*
 #undef F32_SKINNY
     return;
   }
-  const auto tiles = [](int n, int b) { return (n + b - 1) / b; };
-  const long big = (long)tiles(M, 128) * tiles(N, 128), small = (long)tiles(M, 64) * tiles(N, 64);
-  if ((big + 255) / 256 * 4 * 8 <= (small + 255) / 256 * 9)
+  if (f32_large_blocks(M, N))
     launch_f32_blocks<LOADS, 4, 2>(A, W, bias, C, M, N, K, lda, ldc, stream);
   else
     launch_f32_blocks<LOADS, 2, 1>(A, W, bias, C, M, N, K, lda, ldc, stream);
@@ -401,6 +459,25 @@ extern "C" int kappai_gemm_f32(const float* A, const float* W, const float* bias
   else if (fours && K % F32_CHUNK == 0) launch_f32<F32_WHOLE>(A, W, bias, C, M, N, K, lda, ldc, stream);
   else if (fours) launch_f32<F32_FOURS>(A, W, bias, C, M, N, K, lda, ldc, stream);
   else launch_f32<F32_ELEMENTS>(A, W, bias, C, M, N, K, lda, ldc, stream);
+  KAPPAI_RETURN_LAUNCH_STATUS();
+}
+
+// C[m, f] = silu(A W_f) (A W_{F + f}) over the 2 F rows of W: the bits of kappai_gemm_f32 and kappai_swiglu,
+// whose results of 2 F columns neither are written nor read again.  For the sizes whose plain product takes
+// kernels with both rows of a result in one wave (kappai_gemm_f32_gates; else hipErrorInvalidValue): up to 64
+// rows wherever a block owns 16 rows of W, beyond wherever the 128 x 128 blocks run.
+extern "C" int kappai_gemm_f32_gates(int M, int F, int K) {
+  if (M <= 0 || F <= 0 || K < 4) return 0;
+  return M <= 64 ? (M > 8 || F > 128 * 8) : f32_large_blocks(M, 2 * F);
+}
+extern "C" int kappai_gemm_f32_swiglu(const float* A, const float* W, const float* bias, float* C, int M,
+                                      int F, int K, int lda, int ldc, hipStream_t stream) {
+  if (M <= 0 || F <= 0) return 0;
+  if (!kappai_gemm_f32_gates(M, F, K)) return (int)hipErrorInvalidValue;
+  const bool fours = K % 4 == 0 && lda % 4 == 0 && (uintptr_t)A % 16 == 0 && (uintptr_t)W % 16 == 0;
+  if (fours && K % F32_CHUNK == 0) launch_f32_gated<F32_WHOLE>(A, W, bias, C, M, F, K, lda, ldc, stream);
+  else if (fours) launch_f32_gated<F32_FOURS>(A, W, bias, C, M, F, K, lda, ldc, stream);
+  else launch_f32_gated<F32_ELEMENTS>(A, W, bias, C, M, F, K, lda, ldc, stream);
   KAPPAI_RETURN_LAUNCH_STATUS();
 }
 #endif  // GATE_ACT == 0

@@ -35,8 +35,8 @@ def _ptrs(names):
 
 class Kernels(Structure):
     _fields_ = _ptrs(["embed_rows", "embed_rmsnorm", "add_rmsnorm", "swiglu", "cast",
-                      "sum_partials", "gemm_f32", "gemm_bf16", "gemm_bf16_any", "gemm_bf16_swiglu",
-                      "gemm_bf16_shortconv_step", "shortconv", "shortconv_parts",
+                      "sum_partials", "gemm_f32", "gemm_f32_gates", "gemm_f32_swiglu", "gemm_bf16",
+                      "gemm_bf16_any", "gemm_bf16_swiglu", "gemm_bf16_shortconv_step", "shortconv", "shortconv_parts",
                       "qk_norm_rope_store", "paged_attention_rows"])
 
 
@@ -140,7 +140,10 @@ class CForward:
                          ("add_rmsnorm", el.kappai_add_rmsnorm),
                          ("swiglu", el.kappai_swiglu), ("cast", el.kappai_cast),
                          ("sum_partials", el.kappai_sum_partials),
-                         ("gemm_f32", gm.kappai_gemm_f32), ("gemm_bf16", gm.kappai_gemm_bf16),
+                         ("gemm_f32", gm.kappai_gemm_f32),
+                         ("gemm_f32_gates", gm.kappai_gemm_f32_gates),
+                         ("gemm_f32_swiglu", gm.kappai_gemm_f32_swiglu),
+                         ("gemm_bf16", gm.kappai_gemm_bf16),
                          ("gemm_bf16_any", gm.kappai_gemm_bf16_any),
                          ("gemm_bf16_swiglu", gm.kappai_gemm_bf16_swiglu),
                          ("gemm_bf16_shortconv_step", gm.kappai_gemm_bf16_shortconv_step),

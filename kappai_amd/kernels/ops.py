@@ -595,6 +595,36 @@ def _out_in_fragment_order(wanted: bool, M: int, N: int, force_kernel: int) -> b
             and force_kernel in (0, 2))
 
 
+def linear_swiglu_f32_takes(x: torch.Tensor, weight: torch.Tensor) -> bool:
+    """Whether ``linear_swiglu_f32`` takes these rows and this matrix: float32 rows on the GPU, numbers of
+    rows and columns whose kernels have a gate and its up row in one place."""
+    return (x.is_cuda and x.dtype == F32 and weight.dtype == F32 and x.dim() == 2 and weight.dim() == 2
+            and weight.shape[0] % 2 == 0 and x.shape[1] == weight.shape[1] and weight.is_contiguous()
+            and (x.stride(1) == 1 or x.shape[1] == 1)
+            and bool(library("gemm").kappai_gemm_f32_gates(
+                _c_int(x.shape[0]), _c_int(weight.shape[0] // 2), _c_int(x.shape[1]))))
+
+
+def linear_swiglu_f32(x: torch.Tensor, weight: torch.Tensor,
+                      bias: Optional[torch.Tensor] = None) -> torch.Tensor:
+    """``silu(x Wg^T + bg) (x Wu^T + bu)`` in float32 over ``weight`` = [Wg; Wu], the bits of ``linear`` and
+    ``swiglu`` behind it, where ``linear_swiglu_f32_takes``."""
+    _gpu("x", x, F32, contiguous=False)
+    _gpu("weight", weight, F32)
+    _need(linear_swiglu_f32_takes(x, weight),
+          lambda: f"linear_swiglu_f32: x {tuple(x.shape)}, weight {tuple(weight.shape)}")
+    M, K = x.shape
+    F = weight.shape[0] // 2
+    if bias is not None:
+        _gpu("bias", bias, F32)
+        _need(bias.shape == (2 * F,), lambda: f"linear_swiglu_f32: bias {tuple(bias.shape)} for 2 x {F}")
+    out = torch.empty((M, F), dtype=F32, device=x.device)
+    check(library("gemm").kappai_gemm_f32_swiglu(
+        _ptr(x), _ptr(weight), _ptr(bias), _ptr(out), _c_int(M), _c_int(F), _c_int(K),
+        _c_int(x.stride(0) if M > 1 else K), _c_int(F), _stream()), "gemm_f32_swiglu")
+    return out
+
+
 def linear_swiglu(x: torch.Tensor, weight: torch.Tensor, force_kernel: int = 0,
                   weight_frag: Optional[torch.Tensor] = None, out_fragment: bool = False,
                   activation: int = 0, clamp: Optional["ClampedGate"] = None,

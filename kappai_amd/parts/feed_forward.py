@@ -89,6 +89,11 @@ class SwiGLU(FeedForward):
                                         activation=self.ACTIVATIONS[self.activation],
                                         clamp=self.clamp, bias=self.gate_up.bias)
             return self.down.forward(act, partial_sums=True, add_into=into)
+        if (self.activation == "silu" and not self.fused and torch.is_tensor(x)
+                and ops.linear_swiglu_f32_takes(x, self.gate_up.weight)):
+            with profile.scope("matmul_ffn_gate_up", self.gate_up.weight_bytes()):
+                act = ops.linear_swiglu_f32(x, self.gate_up.weight, self.gate_up.bias)
+            return self.down.forward(act, partial_sums=True, add_into=into)
         gate_up = self.gate_up.forward(x)
         if self.fused:
             gate_up = ops.separate_gate_up(gate_up)

@@ -657,6 +657,11 @@ __global__ __launch_bounds__(8 * WAVE) void attn_prefill_shared_kernel(
     for (int sub = 0; sub < PG_SUB; ++sub)
       issue_one(lds + (decltype(buf_c)::value * PG_SUB + sub) * BUF);
   };
+  // Row i of a score tile is key (i with its bits 2 and 3 exchanged): a lane's weights are then those of
+  // the keys 16 st + 8 hh .. + 7 in order, and their values ONE 16-byte piece of a V^T row.
+  const int krow = (col & 19) | (col & 4) << 1 | (col & 8) >> 1;
+  // this lane's piece of a V^T row in a 16-key group (every other 8 rows have their halves swapped)
+  const int v_at = col * 32 + 16 * (hh ^ ((col >> 3) & 1));
   auto whole = [&](int kb) { return kb >= lo_last && kb + 31 <= pos_first; };
   auto work = [&](auto buf_c, auto sub_c, int it) {
     const int kb = kbase + 32 * it;
@@ -669,21 +674,17 @@ __global__ __launch_bounds__(8 * WAVE) void attn_prefill_shared_kernel(
 #pragma unroll
     for (int ks = 0; ks < P_KS; ++ks) {
       const u32x4_t kf = *reinterpret_cast<const u32x4_t*>(
-          buf + col * ROWB + (((2 * ks + hh) ^ swz(col)) * 16));
+          buf + krow * ROWB + (((2 * ks + hh) ^ swz(krow)) * 16));
       s = __builtin_amdgcn_mfma_f32_32x32x16_bf16(as_frag(kf), qf[ks], s, 0, 0, 0);
     }
-    // V^T operands: d index 32*mt + col, keys 16*st + 4*hh .. +3 and 8 more
-    u32x2_t va[2][P_MT], vb[2][P_MT];
+    // V^T operands: d index 32*mt + col, keys 16*st + 8*hh .. +7
+    u32x4_t vv[2][P_MT];
 #pragma unroll
     for (int st = 0; st < 2; ++st)
 #pragma unroll
-      for (int mt = 0; mt < P_MT; ++mt) {
-        const int sw = ((col >> 3) & 1) * 16;      // this row's halves are swapped
-        const char* vp = buf + KTILE + st * VGROUP + (32 * mt + col) * 32 + 8 * hh;
-        va[st][mt] = *reinterpret_cast<const u32x2_t*>(vp + sw);
-        vb[st][mt] = *reinterpret_cast<const u32x2_t*>(vp + (16 - sw));
-      }
-    // lane holds, for query `col`, keys kb + 8*(v/4) + 4*hh + v%4
+      for (int mt = 0; mt < P_MT; ++mt)
+        vv[st][mt] = *reinterpret_cast<const u32x4_t*>(buf + KTILE + st * VGROUP + 32 * 32 * mt + v_at);
+    // lane holds, for query `col`, keys kb + 16*(v/8) + 8*hh + v%8
     float mloc = -INFINITY;
     if (full) {
 #pragma unroll
@@ -692,7 +693,7 @@ __global__ __launch_bounds__(8 * WAVE) void attn_prefill_shared_kernel(
     } else {
 #pragma unroll
       for (int v = 0; v < 16; ++v) {
-        const int key = kb + 8 * (v / 4) + 4 * hh + v % 4;
+        const int key = kb + 16 * (v / 8) + 8 * hh + v % 8;
         const bool ok = key <= my_pos && key >= my_lo;
         s[v] = ok ? s[v] : -INFINITY;
         mloc = fmaxf(mloc, s[v] * sc);
@@ -700,17 +701,17 @@ __global__ __launch_bounds__(8 * WAVE) void attn_prefill_shared_kernel(
       // what lies in LDS for keys outside the tile's range is not cache content: zero it
 #pragma unroll
       for (int st = 0; st < 2; ++st) {
-        int keep_a = 0, keep_b = 0;
+        int keep = 0;
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const int ka = kb + 16 * st + 4 * hh + i, kbb = ka + 8;
-          if (ka >= lo_tile && ka <= pos_last) keep_a |= 1 << i;
-          if (kbb >= lo_tile && kbb <= pos_last) keep_b |= 1 << i;
+        for (int i = 0; i < 8; ++i) {
+          const int key = kb + 16 * st + 8 * hh + i;
+          if (key >= lo_tile && key <= pos_last) keep |= 1 << i;
         }
 #pragma unroll
         for (int mt = 0; mt < P_MT; ++mt) {
-          va[st][mt] = mask4(va[st][mt], keep_a);
-          vb[st][mt] = mask4(vb[st][mt], keep_b);
+          const u32x2_t a = mask4(u32x2_t{vv[st][mt].x, vv[st][mt].y}, keep & 15);
+          const u32x2_t b = mask4(u32x2_t{vv[st][mt].z, vv[st][mt].w}, keep >> 4);
+          vv[st][mt] = u32x4_t{a.x, a.y, b.x, b.y};
         }
       }
     }
@@ -754,10 +755,8 @@ __global__ __launch_bounds__(8 * WAVE) void attn_prefill_shared_kernel(
       const bf16x8_t pf = as_frag(pw);
       if (MFMA_SUM) o_sum = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ones, pf, o_sum, 0, 0, 0);
 #pragma unroll
-      for (int mt = 0; mt < P_MT; ++mt) {
-        const u32x4_t vw4 = {va[st][mt].x, va[st][mt].y, vb[st][mt].x, vb[st][mt].y};
-        o[mt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(as_frag(vw4), pf, o[mt], 0, 0, 0);
-      }
+      for (int mt = 0; mt < P_MT; ++mt)
+        o[mt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(as_frag(vv[st][mt]), pf, o[mt], 0, 0, 0);
     }
   };
 
@@ -774,7 +773,7 @@ __global__ __launch_bounds__(8 * WAVE) void attn_prefill_shared_kernel(
 #pragma unroll
       for (int ks = 0; ks < P_KS; ++ks) {
         const u32x4_t kf = *reinterpret_cast<const u32x4_t*>(
-            buf + col * ROWB + (((2 * ks + hh) ^ swz(col)) * 16));
+            buf + krow * ROWB + (((2 * ks + hh) ^ swz(krow)) * 16));
         s = __builtin_amdgcn_mfma_f32_32x32x16_bf16(as_frag(kf), qf[ks], s, 0, 0, 0);
       }
       return s;
@@ -805,16 +804,12 @@ __global__ __launch_bounds__(8 * WAVE) void attn_prefill_shared_kernel(
       }
     };
     auto weights_and_output = [&](const char* buf, f32x16_t s) {
-      u32x2_t va[2][P_MT], vb[2][P_MT];
+      u32x4_t vv[2][P_MT];
 #pragma unroll
       for (int st = 0; st < 2; ++st)
 #pragma unroll
-        for (int mt = 0; mt < P_MT; ++mt) {
-          const int sw = ((col >> 3) & 1) * 16;
-          const char* vp = buf + KTILE + st * VGROUP + (32 * mt + col) * 32 + 8 * hh;
-          va[st][mt] = *reinterpret_cast<const u32x2_t*>(vp + sw);
-          vb[st][mt] = *reinterpret_cast<const u32x2_t*>(vp + (16 - sw));
-        }
+        for (int mt = 0; mt < P_MT; ++mt)
+          vv[st][mt] = *reinterpret_cast<const u32x4_t*>(buf + KTILE + st * VGROUP + 32 * 32 * mt + v_at);
       const float m_safe = m_ref == -INFINITY ? 0.f : m_ref;
       float lsum = 0.f;
 #pragma unroll
@@ -835,10 +830,8 @@ __global__ __launch_bounds__(8 * WAVE) void attn_prefill_shared_kernel(
         const bf16x8_t pf = as_frag(pw);
         if (MFMA_SUM) o_sum = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ones, pf, o_sum, 0, 0, 0);
 #pragma unroll
-        for (int mt = 0; mt < P_MT; ++mt) {
-          const u32x4_t vw4 = {va[st][mt].x, va[st][mt].y, vb[st][mt].x, vb[st][mt].y};
-          o[mt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(as_frag(vw4), pf, o[mt], 0, 0, 0);
-        }
+        for (int mt = 0; mt < P_MT; ++mt)
+          o[mt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(as_frag(vv[st][mt]), pf, o[mt], 0, 0, 0);
       }
     };
     // the second tile's score products stand between the first tile's maximum and its
@@ -853,7 +846,7 @@ __global__ __launch_bounds__(8 * WAVE) void attn_prefill_shared_kernel(
 
   // `it` counts buffers' worth of tiles (PG_SUB each)
   const int n_steps = (n_tiles + PG_SUB - 1) / PG_SUB;
-  auto step = [&](auto buf_c, int it) {
+  auto step = [&](auto buf_c, auto both_whole, int it) {
     constexpr int B = decltype(buf_c)::value;
     // the tiles of this step have landed (this wave's part; the barrier makes it everybody's),
     // those of the next step may still be on their way
@@ -863,7 +856,7 @@ __global__ __launch_bounds__(8 * WAVE) void attn_prefill_shared_kernel(
     // step it+2 goes into the buffer of step it-1: everybody is done with it
     if (it + 2 < n_steps) issue(PgBuf<(B + 2) % PG_NBUF>{});
     const int kb = kbase + 32 * PG_SUB * it;
-    if (HEAD_DIM == 64 && has_tile && whole(kb) && whole(kb + 32)) {   // (128: registers spill)
+    if constexpr (decltype(both_whole)::value != 0) {
       work2(buf_c);
       return;
     }
@@ -874,11 +867,30 @@ __global__ __launch_bounds__(8 * WAVE) void attn_prefill_shared_kernel(
   static_assert(PG_SUB == 2, "the step works on two tiles");
   issue(PgBuf<0>{});
   if (n_steps > 1) issue(PgBuf<1>{});
-  for (int it = 0; it < n_steps; it += PG_NBUF) {
-    step(PgBuf<0>{}, it);
-    if (it + 1 < n_steps) step(PgBuf<1>{}, it + 1);
-    if (it + 2 < n_steps) step(PgBuf<2>{}, it + 2);
+  // The steps whose tiles need no mask, in whole rounds of the buffers, are a loop of their own: where the
+  // two ways through a step meet again, 48 accumulators are copied (a sixth of the step's vector work).
+  int it = 0, fast_from = 0, fast_to = 0;
+  if (HEAD_DIM == 64 && has_tile) {                                    // (128: registers spill)
+    fast_from = (max(lo_last - kbase, 0) + 32 * PG_SUB - 1) / (32 * PG_SUB);
+    fast_from = (fast_from + PG_NBUF - 1) / PG_NBUF * PG_NBUF;
+    fast_to = max(pos_first + 1 - kbase, 0) / (32 * PG_SUB);
+    fast_from = __builtin_amdgcn_readfirstlane(fast_from);
+    fast_to = __builtin_amdgcn_readfirstlane(min(fast_to, n_steps));
   }
+  const auto steps_to = [&](int end) {
+    for (; it < end; it += PG_NBUF) {
+      step(PgBuf<0>{}, PgBuf<0>{}, it);
+      if (it + 1 < n_steps) step(PgBuf<1>{}, PgBuf<0>{}, it + 1);
+      if (it + 2 < n_steps) step(PgBuf<2>{}, PgBuf<0>{}, it + 2);
+    }
+  };
+  steps_to(fast_to - fast_from >= PG_NBUF ? fast_from : n_steps);
+  for (; it + PG_NBUF <= fast_to; it += PG_NBUF) {
+    step(PgBuf<0>{}, PgBuf<1>{}, it);
+    step(PgBuf<1>{}, PgBuf<1>{}, it + 1);
+    step(PgBuf<2>{}, PgBuf<1>{}, it + 2);
+  }
+  steps_to(n_steps);
   if (!row_ok) return;
   float l_run = MFMA_SUM ? o_sum[0] : l_add;
   if (sink != nullptr && m_ref != -INFINITY) l_run += fast_exp2(sink[h] * LOG2E - m_ref);

@@ -140,7 +140,7 @@ __device__ __forceinline__ u32x4_t load_k8(const bf16_t* __restrict__ k_pool,
 // (NW (rep HEAD_DIM + 32) floats of LDS; rep <= 16): defined with the decode kernels.
 // (FUSED: with the prologue of `qk` in the waves that have keys)
 struct QkFuse;
-template <bool MODS, bool FUSED = false>
+template <bool MODS, bool FUSED = false, int UNIT = 32>
 __device__ __forceinline__ void attn_one_row(const bf16_t* q, int q_stride, const bf16_t* k_pool,
                                              const bf16_t* vt_pool, bf16_t* out, int out_stride,
                                              const int* bt, int max_blocks, int t, int pos, int g, int H,
@@ -487,6 +487,13 @@ __global__ __launch_bounds__(P_NW * WAVE, P_MIN_WAVES) void attn_prefill_kernel(
 // every other 8 rows with their two halves of 8 keys swapped, for the same reason.
 // The running maximum is only moved when a tile's maximum exceeds it by more than 2^8: most
 // tiles then leave the output accumulators alone (no rescaling), and the weights stay <= 256.
+//
+// Bound by the issue of vector instructions (85 and 32 exponentials for two tiles at head size 64, 0.35 us
+// of them at two waves a SIMD) and by what two waves a SIMD leave uncovered: 2,048 rows are 256 blocks,
+// so the chip has no more.  2,048 rows, 32 heads of 64 on 8: without past 44.1 us (54.1 with values put together
+// from two reads and one loop for masked and whole steps), behind 4,096 keys 128.4 (156.5), behind 9,900
+// 255.9 (307.5: 0.57 PFLOP/s, now 0.69).  Priorities for the waves of one tile, for the products or for the
+// exponentials: within 3 %; both tiles' scores ahead of either's exponentials: the same.
 #if HEAD_DIM == 64 || HEAD_DIM == 128
 #define PG_OK 1
 #define PG_NBUF 3
@@ -1739,7 +1746,7 @@ __global__ __launch_bounds__(64, FUSED || MODS || HEAD_DIM > 128 ? 1 : 2) void a
 // keys depends on the row's own position and on the number of waves only.  For batches with
 // (rows x kv heads) enough to fill the chip, or contexts short enough for one block.
 // LDS: sh_o [NW][rep][HEAD_DIM], then sh_m [NW][16], sh_l [NW][16] (floats).
-template <bool MODS, bool FUSED>
+template <bool MODS, bool FUSED, int UNIT>
 __device__ __forceinline__ void attn_one_row(const bf16_t* q, int q_stride, const bf16_t* k_pool,
                                              const bf16_t* vt_pool, bf16_t* out, int out_stride,
                                              const int* bt, int max_blocks, int t, int pos, int g, int H,
@@ -1759,8 +1766,8 @@ __device__ __forceinline__ void attn_one_row(const bf16_t* q, int q_stride, cons
     attn_decode_scored_wave(q, q_stride, k_pool, vt_pool, bt, max_blocks, t, g, H, G, ps, scale, lo, pos,
                             k_begin + wave * D_KPW, NW * D_KPW, k_end, o, m_run, l_run, pos, &mods);
   } else {
-    // equal shares in whole parts of 32 keys
-    const int per = ((k_end - k_begin + 31) / 32 + NW - 1) / NW * 32;
+    // equal shares in whole parts of UNIT keys
+    const int per = ((k_end - k_begin + UNIT - 1) / UNIT + NW - 1) / NW * UNIT;
     const int from = k_begin + wave * per;
     if (FUSED && from >= k_end) {              // (no keys: no prologue either)
 #pragma unroll
@@ -1815,7 +1822,11 @@ __global__ __launch_bounds__(D_BLOCK_MAX_WAVES * WAVE) void attn_decode_block_ke
     float scale, kappai_score_mods mods) {
   extern __shared__ float sh_dec[];
   const int t = blockIdx.x;
-  attn_one_row<MODS>(q, q_stride, k_pool, vt_pool, out, out_stride,
+  // Shares of whole parts of 32 keys at the head sizes of long use; at the others of whole chunks, as the
+  // kernel had them: two maps of 16 that are subtracted leave 0.04 to 0.06 of the largest value to the
+  // rounding of either, and that stays what it was.
+  constexpr int UNIT = HEAD_DIM == 64 || HEAD_DIM == 128 ? 32 : D_KPW;
+  attn_one_row<MODS, false, UNIT>(q, q_stride, k_pool, vt_pool, out, out_stride,
                      block_tables + (size_t)row_seg[t] * max_blocks, max_blocks, t, row_pos[t],
                      blockIdx.y, H, G, ps, window, scale, mods, sh_dec, blockDim.x / WAVE);
 }

@@ -108,6 +108,7 @@ __device__ __forceinline__ void load_chunk_f32(const float* __restrict__ row, in
 //
 // GATED: W holds 2 N rows, gate rows and behind them the up rows; a block's 16 columns are the gates of 8
 // results and their up rows, C[m, n] = silu(gate) up, the bits of the product and kappai_swiglu behind it.
+// (Three rows, 4,608 gates: a kernel of 4.4 us less a layer; 825 rows in blocks: 9.3 us less.)
 template <int MT, int COLS, int RUNS, int LOADS, bool GATED = false>
 __global__ __launch_bounds__((COLS == 8 ? RUNS / 2 : 8) * WAVE) void gemm_f32_skinny_kernel(
     const float* __restrict__ A, const float* __restrict__ W, const float* __restrict__ bias,

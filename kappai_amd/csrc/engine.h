@@ -338,6 +338,9 @@ const char* kappai_forward_error(void);
 // host's parts ask the same function).
 int kappai_split_k_for(int M, int N, int K);
 
+// Whether such a product hands its sums on in float (always with more than one range).
+int kappai_sums_in_f32(int M, int N, int K);
+
 // The most keys with which the decode attention keeps a row's keys in one block (attn_decode_block) where
 // `few` is what it takes for any number of rows.
 int kappai_decode_block_keys(int few, int rows, int G, int head_dim);

@@ -84,21 +84,63 @@ void refuse(Step& c, const char* message) {
 // ---------------------------------------------------------------------------------------------
 // how many K ranges (the rule the host's parts use as well)
 // ---------------------------------------------------------------------------------------------
-// K ranges for a product with more than 64 rows whose consumer adds partial sums: the number that the
-// model of the block products (gemm_rules.h) with the norm that reads the planes (0.16 us a megabyte) likes
-// best.
-int split_k_large(int M, int N, int K) {
-  int best = 1;
+// K ranges for a product of more than 64 rows whose consumer adds partial sums: the number that a model of the
+// block kernels with the norm that adds the planes (0.16 us a megabyte) likes best.
+struct Ranges {
+  int split;
+  bool f32;                 // the sums are handed on in float, also those over one range
+};
+bool ranges_fit(int K, int split) { return K % (128 * split) == 0 && (split == 1 || K / split >= 256); }
+
+// ... of a W that lies as rows (gemm_bf16_block256).  Least squares over 787 measured products (1024 to 6144
+// columns, K from 1024 to 8192, 160 to 2048 rows, up to eight ranges), good to 4 to 11 %; `steps` is 64s of K,
+// `mb` the megabytes of results.
+Ranges ranges_over_rows(int M, int N, int K) {
+  Ranges best{1, false};
   double best_t = -1.0;
   for (int split = 1; split < 9; ++split) {
-    if (K % (128 * split) || (split > 1 && K / split < 256)) continue;
-    // (one range: bfloat16 results)
-    const double mb = (split > 1 ? split : 0.5) * M * (double)N * 4e-6;
+    if (!ranges_fit(K, split)) continue;
+    const double steps = (double)K / split / 64.0;
+    const double mb = (split > 1 ? split : 0.5) * M * (double)N * 4e-6;     // (one range: bfloat16 results)
+    const long blocks256 = (long)((M + 255) / 256) * ((N + 255) / 256) * split;
+    const long blocks128 = (long)((M + 127) / 128) * ((N + 127) / 128) * split;
+    double t;
+    if (M > 128 && kappai_use_256_form(blocks256)) {
+      const double rounds = (double)((blocks256 + 255) / 256);
+      t = steps * (1.07 * rounds + 0.53 * blocks256 / 256) + 8.6 * rounds + 0.10 * mb;
+    } else if (kappai_deep_form(blocks128, K / split)) {
+      t = steps * (0.44 + 0.12 * blocks128 / 256) + 4.5 + 0.19 * mb;
+    } else if (blocks128 <= 256) {
+      t = steps * 0.69 + 2.5 + 0.22 * mb;
+    } else {
+      t = steps * (0.32 * blocks128 / 512 + 0.67 * (double)((blocks128 + 511) / 512)) + 2.5 +
+          0.22 * mb;
+    }
+    t += 0.16 * mb;
+    if (best_t < 0 || t < best_t - 1e-9) {
+      best = {split, split > 1};
+      best_t = t;
+    }
+  }
+  return best;
+}
+
+// ... of a W in fragment order (its rows a multiple of 16: the model in gemm_rules.h).  The order W is kept in
+// decides the speed, not what the sums are rounded to: where the ranges of the kernels over rows leave float
+// sums, one range over fragment order does too.  2100 x 2048 x 8192 with the norm: 80.0 us so, 78.3 in
+// bfloat16, 98.4 in two ranges; 1600 x 1024 x 1024: 17.0, 15.5 and 17.0.
+Ranges ranges_over_fragments(int M, int N, int K) {
+  const bool f32 = ranges_over_rows(M, N, K).f32;
+  Ranges best{1, f32};
+  double best_t = -1.0;
+  for (int split = 1; split < 9; ++split) {
+    if (!ranges_fit(K, split)) continue;
+    const double mb = (split > 1 || f32 ? split : 0.5) * M * (double)N * 4e-6;
     double t;
     kappai_block_shape(M, N, K, split, mb, false, &t);
     t += 0.16 * mb;
     if (best_t < 0 || t < best_t - 1e-9) {
-      best = split;
+      best = {split, split > 1 || f32};
       best_t = t;
     }
   }
@@ -119,23 +161,25 @@ int split_k_rows32(int N, int K) {
   return split;
 }
 
-int split_k_for(int M, int N, int K) {
+Ranges ranges_for(int M, int N, int K) {
+  const auto ranges = [](int split) { return Ranges{split, split > 1}; };
   if (M > KAPPAI_ROWS32_MIN_ROWS && M <= KAPPAI_ROWS32_MAX_ROWS && K % KAPPAI_ROWS32_RUN == 0 &&
       N % 16 == 0)
-    return split_k_rows32(N, K);
-  if (M > 64) return split_k_large(M, N, K);
+    return ranges(split_k_rows32(N, K));
+  if (M > 64) return ranges_over_fragments(M, N, K);
   if (M > 16) {
     // the kernel that shares the rows through LDS: blocks of 64 columns, K ranges that are
     // multiples of 512 and at least 1024 long, 128 blocks or more
     int split = K / 1024 < 8 ? K / 1024 : 8;
     while (split > 1 && K % (512 * split)) --split;
-    if (split >= 1 && K % (512 * split) == 0 && (long)((N + 63) / 64) * split >= 128) return split;
+    if (split >= 1 && K % (512 * split) == 0 && (long)((N + 63) / 64) * split >= 128)
+      return ranges(split);
   }
   const int col_groups = (N + 15) / 16;
   int s = 8;
   if (512 / col_groups < s) s = 512 / col_groups;
   if (K / 512 < s) s = K / 512;
-  return s < 1 ? 1 : s;
+  return ranges(s < 1 ? 1 : s);
 }
 
 // how the split decode kernel cuts n_keys keys of `rows` rows
@@ -342,8 +386,10 @@ kappai_carry linear(Step& c, kappai_rows x, const kappai_linear& lin, int out_bf
     out.scaled.norm = norm;
     return out;
   }
-  const int ksplit = (partial_sums && !scaled) ? split_k_for(M, N, K) : 1;
-  if (ksplit > 1) {
+  const Ranges ranges = (partial_sums && !scaled) ? ranges_for(M, N, K) : Ranges{1, false};
+  const int ksplit = ranges.split;
+  const bool planes = ksplit > 1 || (ranges.f32 && out_bf16);
+  if (planes) {
     out.kind = KAPPAI_CARRY_PARTS;
     out.is_f32 = 1;
     out.parts = ksplit;
@@ -354,7 +400,7 @@ kappai_carry linear(Step& c, kappai_rows x, const kappai_linear& lin, int out_bf
     out.data = c.a->take(region, (size_t)M * N * elem(out_bf16));
   }
   LAUNCH(c, k.gemm_bf16(xb, lin.w, lin.w_frag, lin.bias, out.data, M, N, K, lda, N,
-                        (ksplit > 1 || !out_bf16) ? 1 : 0, 0, ksplit, x.frag,
+                        (planes || !out_bf16) ? 1 : 0, 0, ksplit, x.frag,
                         scaled ? x.ss : nullptr, scaled ? x.ss_parts : 0, scaled ? x.eps : 0.f,
                         nullptr, 0, nullptr, nullptr, 0, nullptr, c.stream));
   return out;
@@ -586,7 +632,9 @@ extern "C" int kappai_engine_layout(int* sizes, int n) {
 
 extern "C" const char* kappai_forward_error(void) { return g_error; }
 
-extern "C" int kappai_split_k_for(int M, int N, int K) { return split_k_for(M, N, K); }
+extern "C" int kappai_split_k_for(int M, int N, int K) { return ranges_for(M, N, K).split; }
+
+extern "C" int kappai_sums_in_f32(int M, int N, int K) { return ranges_for(M, N, K).f32 ? 1 : 0; }
 
 // One block a (row, kv head) takes a row's keys in at 50 GB/s or so, but needs no second kernel, and with
 // blocks enough for the chip nothing is won by more of them.  us against the kernel that splits the keys over

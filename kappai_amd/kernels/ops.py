@@ -456,6 +456,12 @@ def split_k_for(M: int, N: int, K: int) -> int:
     return int(library("engine").kappai_split_k_for(_c_int(M), _c_int(N), _c_int(K)))
 
 
+def sums_in_f32(M: int, N: int, K: int) -> bool:
+    """Whether such a product hands its sums on in float32: over more than one range always, over one where
+    the same product over rows of W would take more."""
+    return bool(library("engine").kappai_sums_in_f32(_c_int(M), _c_int(N), _c_int(K)))
+
+
 def linear(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor] = None,
            out_dtype=None, force_kernel: int = 0, partial_sums: bool = False,
            split_k: Optional[int] = None,
@@ -464,7 +470,7 @@ def linear(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor] =
     """``x [M, K] @ weight[N, K]^T (+ bias)``.  A bfloat16 matrix runs on the matrix cores
     with float accumulation; a float32 matrix runs in true 32-bit arithmetic, whatever the
     activations' dtype.  ``x`` may be a view with a row stride.  With ``partial_sums`` the
-    result may come back as float32 [S, M, N], the sums over S ranges of K, for a consumer
+    result may come back as float32 [S, M, N], the sums over S >= 1 ranges of K, for a consumer
     that adds them (a matrix with few columns is then streamed by enough blocks).  ``x`` may
     be ``ScaledRows`` or ``FragmentRows``.  ``weight`` may be ``InFragments`` (a bfloat16 matrix
     kept in fragment order only); or ``weight_frag`` (``fragment_order(weight)``) may come beside
@@ -552,7 +558,7 @@ def linear(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor] =
             return Added(resid)
         return ScaledRows(rows, M, fragment, ss, nw, add_into.eps, resid)
     ksplit = (split_k or split_k_for(M, N, K)) if partial_sums else 1
-    if ksplit > 1:
+    if ksplit > 1 or (partial_sums and not split_k and out_dtype == BF16 and sums_in_f32(M, N, K)):
         out = torch.empty((ksplit, M, N), dtype=F32, device=x.device)
         out_is_f32 = 1
     else:

@@ -1,0 +1,41 @@
+"""How many ranges of K a product of many rows is cut into, and what its sums are handed on as."""
+import pytest
+import torch
+
+from kappai_amd.kernels import ops
+
+# products over fragment order that are fastest over one range and over rows of W over two or more
+ONE_RANGE = [(1600, 1024, 1024), (2100, 2048, 8192), (2880, 2048, 8192), (3300, 2048, 8192), (2880, 2048, 10752),
+             (4200, 1024, 4608), (1700, 1024, 1024)]
+
+
+@pytest.mark.parametrize("M,N,K", ONE_RANGE + [(1040, 1024, 1024), (3200, 1536, 6912), (600, 2048, 1024)])
+def test_sums_that_were_float_stay_float(M, N, K):
+    assert ops.sums_in_f32(M, N, K)
+
+
+@pytest.mark.parametrize("M,N,K", [(2048, 1024, 1024), (4200, 2048, 2048), (2048, 6144, 2048), (200, 16384, 2048)])
+def test_one_range_in_bfloat16(M, N, K):
+    assert ops.split_k_for(M, N, K) == 1 and not ops.sums_in_f32(M, N, K)
+
+
+def test_several_ranges_are_float():
+    for M, N, K in ((300, 1024, 4608), (100, 2048, 2048), (8, 2048, 8192), (40, 1024, 4608), (575, 2048, 2048)):
+        assert ops.split_k_for(M, N, K) > 1 and ops.sums_in_f32(M, N, K)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K", ONE_RANGE[:3])
+def test_float_sums_over_one_range(M, N, K):
+    """Against float64, by themselves and in the norm that takes them; bfloat16 would be off by 2^-9."""
+    from test_kernels_gpu import BF16, DEV, F32, close, rand, ref
+    x, w = rand((M, K), BF16, 91), rand((N, K), BF16, 92, 0.05)
+    got = ops.linear(x.to(DEV), ops.InFragments.of(w.to(DEV)), partial_sums=True)
+    assert got.dtype == F32 and tuple(got.shape) == (ops.split_k_for(M, N, K), M, N)
+    close(got.sum(0), x.double() @ w.double().T, (K + 1) * 2.0 ** -24, "the sums")
+    resid, wn = rand((M, N), F32, 93, 2.0), 1 + rand((N,), F32, 94, 0.1)
+    on_gpu = resid.to(DEV).clone()
+    ops.add_rmsnorm(on_gpu, got, wn.to(DEV), 1e-5, BF16)
+    want = resid.clone()
+    ref.add_rmsnorm(want, got.cpu(), wn, 1e-5, F32)
+    close(on_gpu, want, 1e-6, "the stream")

@@ -94,7 +94,8 @@ bool ranges_fit(int K, int split) { return K % (128 * split) == 0 && (split == 1
 
 // ... of a W that lies as rows (gemm_bf16_block256).  Least squares over 787 measured products (1024 to 6144
 // columns, K from 1024 to 8192, 160 to 2048 rows, up to eight ranges), good to 4 to 11 %; `steps` is 64s of K,
-// `mb` the megabytes of results.
+// `mb` the megabytes of results.  Against the ranges that the model for fragment order gives such a W, with the
+// norm: 2880 x 2040 x 8192 110.5 us for 119.1, 3300 rows of it 117.9 for 128.4, 1040 rows 62.8 for 59.0.
 Ranges ranges_over_rows(int M, int N, int K) {
   Ranges best{1, false};
   double best_t = -1.0;
@@ -166,7 +167,7 @@ Ranges ranges_for(int M, int N, int K) {
   if (M > KAPPAI_ROWS32_MIN_ROWS && M <= KAPPAI_ROWS32_MAX_ROWS && K % KAPPAI_ROWS32_RUN == 0 &&
       N % 16 == 0)
     return ranges(split_k_rows32(N, K));
-  if (M > 64) return ranges_over_fragments(M, N, K);
+  if (M > 64) return N % 16 ? ranges_over_rows(M, N, K) : ranges_over_fragments(M, N, K);
   if (M > 16) {
     // the kernel that shares the rows through LDS: blocks of 64 columns, K ranges that are
     // multiples of 512 and at least 1024 long, 128 blocks or more

@@ -39,3 +39,10 @@ def test_float_sums_over_one_range(M, N, K):
     want = resid.clone()
     ref.add_rmsnorm(want, got.cpu(), wn, 1e-5, F32)
     close(on_gpu, want, 1e-6, "the stream")
+
+
+@pytest.mark.parametrize("M,N,K,ranges", [(1400, 2040, 8192, 4), (2880, 2040, 8192, 2), (3072, 1000, 4096, 1),
+                                          (417, 1032, 1024, 4)])
+def test_rows_of_w_take_the_ranges_of_their_own_kernels(M, N, K, ranges):
+    """A matrix whose rows are no multiple of 16 lies as rows and goes through kernels of its own."""
+    assert ops.split_k_for(M, N, K) == ranges and ops.sums_in_f32(M, N, K) == (ranges > 1)

@@ -1240,11 +1240,14 @@ __device__ __forceinline__ void qk_norm_rotate(u32x4_t (&raw)[(HEAD_DIM + 31) / 
 // Bound by the stream of keys and values.  The keys go by in parts of 32 whose loads (16 bytes a lane) are
 // asked for D_AHEAD parts ahead: a part's registers are filled again as soon as it is worked on, so that
 // loads stay under way from the first key to the last.  The page ids are read 64 at a time, the next 64
-// ahead of their use, and handed out as scalars.  Against chunks of 128 keys, each asked for, waited for
-// and worked on by itself: 3 rows of 9,000 to 15,000 keys, 32 heads of 64 on 8 (with the prologue) 24.4 us
-// against 32.5; 64 rows of 128 to 2,304 keys 39.4 against 42.6 (160 MB: 4.1 TB/s, the kernel's start and
-// the three lookups before its first key among it); 8 rows of 3,600 keys 15.3 against 15.9.
-#define D_AHEAD (HEAD_DIM <= 64 ? 4 : (HEAD_DIM <= 128 ? 2 : 1))
+// ahead of their use, and handed out as scalars.  A part whose keys are not all seen is loaded like any
+// other and cut when it is worked on (loads of its own for it were half the kernel's code).  Against chunks
+// of 128 keys, each asked for, waited for and worked on by itself, 32 heads on 8: head size 64, 8 rows of
+// 300 keys in a block 6.3 us against 7.9, 64 rows of up to 2,000 keys 33.9 against 38.3 (135 MB: 4.0 TB/s,
+// the kernel's start and the three lookups before its first key among it), 1 row of 8,000 keys and the
+// merge 9.7 against 11.9; head size 128, 8 rows of 300 keys 8.1 against 9.1.  Head size 32 has registers for
+// two blocks a CU with three parts ahead, not with four (128 rows of 300 keys 13.3 us; with one block a CU 22.8).
+#define D_AHEAD (HEAD_DIM == 32 ? 3 : (HEAD_DIM <= 64 ? 4 : (HEAD_DIM <= 128 ? 2 : 1)))
 template <bool FUSABLE>
 __device__ __forceinline__ void attn_decode_wave(
     const bf16_t* __restrict__ q, int q_stride, const bf16_t* __restrict__ k_pool,
@@ -1257,15 +1260,17 @@ __device__ __forceinline__ void attn_decode_wave(
   const bool head_ok = col < rep;
   const int h = g * rep + (head_ok ? col : 0);
   const int hi = k_end - 1;
-  // page ids 64 at a time: asked for before anything else
-  const int page0 = first / ps;
-  auto ask_pages = [&](int from) {
-    return from + lane < max_blocks && (long long)(from + lane) * ps <= hi ? bt[from + lane] : -1;
+  // Page ids 64 at a time: asked for before anything else, those behind the last key's page as that page's
+  // (a load under a condition is waited for where the two ways meet).
+  const int page0 = first / ps, page_last = min(hi / ps, max_blocks - 1);
+  auto ask_pages = [&](int from) { return bt[min(from + lane, page_last)]; };
+  int pages = ask_pages(page0), pages_next = ask_pages(page0 + WAVE), page_at = 0, page_off = first % ps;
+  int pages_from = page0;
+  // (what is in the register has arrived: else every part's ids would wait for the loads of the part before)
+  auto pages_are_here = [&] {
+    pages = pages_from + lane <= page_last ? pages : -1;
+    asm volatile("" : "+v"(pages));
   };
-  int pages = ask_pages(page0), pages_next = -1, page_at = 0, page_off = first % ps;
-  const bool many = (long long)(page0 + WAVE) * ps <= hi;
-  if (many) pages_next = ask_pages(page0 + WAVE);
-  int pages_from = page0 + WAVE;
 
   bf16x8_t qf[D_KS];
   u32x4_t qraw[D_KS];
@@ -1313,6 +1318,7 @@ __device__ __forceinline__ void attn_decode_wave(
 
   struct Part {
     u32x4_t k[2][D_KS], v[D_MT];
+    int missing;             // bit i: the i-th 16 keys have no page
   };
   // (scalars) the page of the next 16 keys and their place in it
   auto next16 = [&](int& page, int& off) {
@@ -1325,7 +1331,8 @@ __device__ __forceinline__ void attn_decode_wave(
         page_at = 0;
         pages = pages_next;
         pages_from += WAVE;
-        pages_next = ask_pages(pages_from);
+        pages_are_here();
+        pages_next = ask_pages(pages_from + WAVE);
       }
     }
   };
@@ -1338,33 +1345,44 @@ __device__ __forceinline__ void attn_decode_wave(
     int pg[2], off[2];
     next16(pg[0], off[0]);
     next16(pg[1], off[1]);
-    if (kb >= lo && kb + 31 <= hi && pg[0] >= 0 && pg[1] >= 0) {     // every key of the part is seen
-      const size_t a0 = ((size_t)pg[0] * G + g) * ps, a1 = ((size_t)pg[1] * G + g) * ps;
-      const bf16_t* kp = k_pool + (col < 8 ? (a0 + off[0]) * HEAD_DIM : (a1 + off[1]) * HEAD_DIM) + k_lane;
-      const bf16_t* vp = vt_pool + (kg < 2 ? a0 * HEAD_DIM + off[0] : a1 * HEAD_DIM + off[1]) + v_lane;
+    // (a key that no row sees lies in a page that is there, or page 0 stands in for the one that is not:
+    // what comes of it is left out when the part is worked on)
+    p.missing = (pg[0] < 0 ? 1 : 0) | (pg[1] < 0 ? 2 : 0);
+    const size_t a0 = ((size_t)max(pg[0], 0) * G + g) * ps, a1 = ((size_t)max(pg[1], 0) * G + g) * ps;
+    const bf16_t* kp = k_pool + (col < 8 ? (a0 + off[0]) * HEAD_DIM : (a1 + off[1]) * HEAD_DIM) + k_lane;
+    const bf16_t* vp = vt_pool + (kg < 2 ? a0 * HEAD_DIM + off[0] : a1 * HEAD_DIM + off[1]) + v_lane;
+#pragma unroll
+    for (int tt = 0; tt < 2; ++tt)
+#pragma unroll
+      for (int ks = 0; ks < D_KS; ++ks) {
+        const bool there = HEAD_DIM % 32 == 0 || 32 * ks + 8 * kg < HEAD_DIM;
+        const u32x4_t x = *reinterpret_cast<const u32x4_t*>(there ? kp + 4 * tt * HEAD_DIM + 32 * ks : k_pool);
+        p.k[tt][ks] = there ? x : (u32x4_t){0u, 0u, 0u, 0u};
+      }
+#pragma unroll
+    for (int mt = 0; mt < D_MT; ++mt) p.v[mt] = *reinterpret_cast<const u32x4_t*>(vp + 16 * mt * ps);
+  };
+  // the part's keys that the row does not see, or whose page is missing: their values read as zero, and so
+  // do the keys of a missing page (the others' scores are dropped, whatever they are)
+  auto leave_out = [&](int kb, Part& p) {
+    const int key0 = kb + 8 * kg;
+    const bool there = !(p.missing >> (kg / 2) & 1);
+    uint32_t m[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      m[i] = (there && key0 + 2 * i >= lo && key0 + 2 * i <= hi ? 0x0000ffffu : 0u) |
+             (there && key0 + 2 * i + 1 >= lo && key0 + 2 * i + 1 <= hi ? 0xffff0000u : 0u);
+#pragma unroll
+    for (int mt = 0; mt < D_MT; ++mt)
+      p.v[mt] = (u32x4_t){p.v[mt].x & m[0], p.v[mt].y & m[1], p.v[mt].z & m[2], p.v[mt].w & m[3]};
+    if (p.missing) {
+      const uint32_t mk = p.missing >> (col / 8) & 1 ? 0u : 0xffffffffu;
 #pragma unroll
       for (int tt = 0; tt < 2; ++tt)
 #pragma unroll
-        for (int ks = 0; ks < D_KS; ++ks) {
-          const bool there = HEAD_DIM % 32 == 0 || 32 * ks + 8 * kg < HEAD_DIM;
-          const u32x4_t x = *reinterpret_cast<const u32x4_t*>(
-              there ? kp + 4 * tt * HEAD_DIM + 32 * ks : k_pool);
-          p.k[tt][ks] = there ? x : (u32x4_t){0u, 0u, 0u, 0u};
-        }
-#pragma unroll
-      for (int mt = 0; mt < D_MT; ++mt) p.v[mt] = *reinterpret_cast<const u32x4_t*>(vp + 16 * mt * ps);
-      return;
+        for (int ks = 0; ks < D_KS; ++ks)
+          p.k[tt][ks] = (u32x4_t){p.k[tt][ks].x & mk, p.k[tt][ks].y & mk, p.k[tt][ks].z & mk, p.k[tt][ks].w & mk};
     }
-#pragma unroll
-    for (int tt = 0; tt < 2; ++tt) {
-      const int key = kb + 8 * (col / 4) + 4 * tt + col % 4;
-#pragma unroll
-      for (int ks = 0; ks < D_KS; ++ks)
-        p.k[tt][ks] = load_k8_pg(k_pool, col < 8 ? pg[0] : pg[1], G, g, ps, key, 32 * ks + 8 * kg, lo, hi);
-    }
-#pragma unroll
-    for (int mt = 0; mt < D_MT; ++mt)
-      p.v[mt] = load_vt8_pg(vt_pool, kg < 2 ? pg[0] : pg[1], G, g, ps, 16 * mt + col, kb + 8 * kg, lo, hi);
   };
   // the pools do not hold the row's own key and value yet (or only just): the part that holds
   // the row's position takes them from the registers
@@ -1391,7 +1409,10 @@ __device__ __forceinline__ void attn_decode_wave(
       }
     }
   };
-  auto work = [&](int kb, const Part& p) {
+  auto work = [&](int kb, Part& p) {
+    const bool whole = kb >= lo && kb + 31 <= hi;
+    if (!whole || p.missing) leave_out(kb, p);
+    own(kb, p);
     f32x4_t s[2];
 #pragma unroll
     for (int tt = 0; tt < 2; ++tt) {
@@ -1402,7 +1423,7 @@ __device__ __forceinline__ void attn_decode_wave(
     }
     // lane holds, for head `col`, keys kb + 8*kg + 4*tt + v
     float mloc = -INFINITY;
-    if (kb >= lo && kb + 31 <= hi) {
+    if (whole) {
 #pragma unroll
       for (int tt = 0; tt < 2; ++tt)
 #pragma unroll
@@ -1444,49 +1465,76 @@ __device__ __forceinline__ void attn_decode_wave(
       o[mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_frag(p.v[mt]), pf, o[mt], 0, 0, 0);
     }
   };
-  Part part[D_AHEAD];
-  int kb_ask = first;
+  // (what the row's own position needs: the norm, the rotation, the store)
+  auto prologue = [&] {
+    if constexpr (FUSABLE && D_QK_FUSABLE) {
+      if (fused) {
+        if (own_kv) qk_norm_rotate(k_new, qk.k_norm_w != nullptr, tb.wk, qk.eps,
+                                   qk.cos_tab != nullptr, tb.cs, tb.sn);
+        qk_norm_rotate(qraw, qk.q_norm_w != nullptr, tb.wq, qk.eps, qk.cos_tab != nullptr, tb.cs,
+                       tb.sn);
 #pragma unroll
-  for (int i = 0; i < D_AHEAD; ++i) {
-    if (kb_ask < k_end) ask(kb_ask, part[i]);
-    kb_ask += 32;
-  }
-  if constexpr (FUSABLE && D_QK_FUSABLE) {
-    if (fused) {
-      if (own_kv) qk_norm_rotate(k_new, qk.k_norm_w != nullptr, tb.wk, qk.eps,
-                                 qk.cos_tab != nullptr, tb.cs, tb.sn);
-      qk_norm_rotate(qraw, qk.q_norm_w != nullptr, tb.wq, qk.eps, qk.cos_tab != nullptr, tb.cs,
-                     tb.sn);
+        for (int ks = 0; ks < D_KS; ++ks)
+          qf[ks] = as_frag(head_ok ? qraw[ks] : (u32x4_t){0u, 0u, 0u, 0u});
+        // the wave whose keys hold the row's own position puts its key and value into the pools
+        if (own_kv && pos >= first && pos < k_end) {
+          const size_t pg = (size_t)bt[pos / ps] * G + g;
+          if (col == 0) {
 #pragma unroll
-      for (int ks = 0; ks < D_KS; ++ks)
-        qf[ks] = as_frag(head_ok ? qraw[ks] : (u32x4_t){0u, 0u, 0u, 0u});
-      // the wave whose keys hold the row's own position puts its key and value into the pools
-      if (own_kv && pos >= first && pos < k_end) {
-        const size_t pg = (size_t)bt[pos / ps] * G + g;
-        if (col == 0) {
+            for (int ks = 0; ks < D_KS; ++ks)
+              *reinterpret_cast<u32x4_t*>(qk.k_pool_w + (pg * ps + pos % ps) * HEAD_DIM + 32 * ks +
+                                          8 * kg) = k_new[ks];
+          }
+          if (kg == 0) {
 #pragma unroll
-          for (int ks = 0; ks < D_KS; ++ks)
-            *reinterpret_cast<u32x4_t*>(qk.k_pool_w + (pg * ps + pos % ps) * HEAD_DIM + 32 * ks +
-                                        8 * kg) = k_new[ks];
-        }
-        if (kg == 0) {
-#pragma unroll
-          for (int mt = 0; mt < D_MT; ++mt)
-            qk.vt_pool_w[(pg * HEAD_DIM + 16 * mt + col) * ps + pos % ps] = (bf16_t)v_new[mt];
+            for (int mt = 0; mt < D_MT; ++mt)
+              qk.vt_pool_w[(pg * HEAD_DIM + 16 * mt + col) * ps + pos % ps] = (bf16_t)v_new[mt];
+          }
         }
       }
     }
-  }
-  for (int kb = first; kb < k_end;) {
+  };
+  // A wait counts the loads that may stay under way, the fewest over all ways that lead to it.  Hence a loop
+  // of whole rounds without conditions, left at its end only, for waves with D_AHEAD parts or more; what is
+  // left to ask for behind it, and the parts of a wave that has fewer, stand by themselves.
+  Part part[D_AHEAD];
+  const int n_parts = (k_end - first + 31) / 32;
+  int kb = first, kb_ask = first + 32 * D_AHEAD;
+  int left = n_parts;                        // parts to be worked on behind everything else
+  pages_are_here();
+  if (n_parts >= D_AHEAD) {
 #pragma unroll
     for (int i = 0; i < D_AHEAD; ++i) {
-      if (kb >= k_end) break;
-      own(kb, part[i]);
+      ask(first + 32 * i, part[i]);
+      __builtin_amdgcn_sched_barrier(0);      // (in this order)
+    }
+    prologue();
+    for (left = n_parts - D_AHEAD; left >= D_AHEAD; left -= D_AHEAD) {
+#pragma unroll
+      for (int i = 0; i < D_AHEAD; ++i) {
+        work(kb, part[i]);
+        ask(kb_ask, part[i]);
+        kb += 32;
+        kb_ask += 32;
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < D_AHEAD; ++i) {
       work(kb, part[i]);
-      if (kb_ask < k_end) ask(kb_ask, part[i]);
+      if (i < left) ask(kb_ask, part[i]);
       kb += 32;
       kb_ask += 32;
     }
+  } else {
+#pragma unroll
+    for (int i = 0; i < D_AHEAD - 1; ++i)
+      if (i < left) ask(first + 32 * i, part[i]);
+    prologue();
+  }
+#pragma unroll
+  for (int i = 0; i < D_AHEAD - 1; ++i) {
+    if (i < left) work(kb, part[i]);
+    kb += 32;
   }
   l_lane += lane_xor16(l_lane);
   l_run = l_lane + other_half(l_lane);
@@ -1494,11 +1542,13 @@ __device__ __forceinline__ void attn_decode_wave(
 
 // One wave's share of a row's attention: the query heads of kv head g (columns) against the keys
 // of the chunks c0 = first, first + stride, ... below k_end (D_KPW keys each), with a running
-// maximum and sum per column, scores worked on (score_mods.h).  Leaves the unnormalised output in o (lane: column lane % 16, d
+// maximum and sum per column.  Leaves the unnormalised output in o (lane: column lane % 16, d
 // rows 16 mt + 4 (lane / 16) + v), the maximum (in units of log 2) in m_run, the sum in l_run.
-// The chunks are counted in places (kappai_key_at): the kept first keys stand in front of
-// the window's, whose places are their positions.
-__device__ __forceinline__ void attn_decode_scored_wave(
+// With MODS the scores are worked on (score_mods.h) and the chunks are counted in places (kappai_key_at):
+// the kept first keys stand in front of the window's, whose places are their positions.  Without, for
+// the block kernel at head size 256, which has no registers for the page ids of attn_decode_wave.
+template <bool MODS>
+__device__ __forceinline__ void attn_decode_chunk_wave(
     const bf16_t* __restrict__ q, int q_stride, const bf16_t* __restrict__ k_pool,
     const bf16_t* __restrict__ vt_pool, const int* __restrict__ bt, int max_blocks, int t, int g,
     int H, int G, int ps, float scale, int lo, int hi, int first, int stride, int k_end,
@@ -1510,12 +1560,12 @@ __device__ __forceinline__ void attn_decode_scored_wave(
   const int h = g * rep + (head_ok ? col : 0);
   // the page ids of the first chunk of keys: asked for before anything else, so that the keys
   // can be asked for as soon as they are there, whatever else is still on its way
-  const int keep = mods->keep_first;
+  const int keep = MODS ? mods->keep_first : 0;
   const int lo32 = (lo / 32) * 32;
-  const int kept = kappai_kept_places(keep, lo32);
+  const int kept = MODS ? kappai_kept_places(keep, lo32) : 0;
   auto ask_pages = [&](int c0) {      // lane i: the page of the chunk's places 16 i .. 16 i + 15
-    const int key = kappai_key_at(c0 + 16 * lane, lo32, kept);
-    return 16 * lane < D_KPW && key / ps < max_blocks && (key <= hi || key < keep) ? bt[key / ps] : -1;
+    const int key = MODS ? kappai_key_at(c0 + 16 * lane, lo32, kept) : c0 + 16 * lane;
+    return 16 * lane < D_KPW && key / ps < max_blocks && (key <= hi || (MODS && key < keep)) ? bt[key / ps] : -1;
   };
   int pages_first = first < k_end ? ask_pages(first) : -1;
   bf16x8_t qf[D_KS];
@@ -1543,18 +1593,18 @@ __device__ __forceinline__ void attn_decode_scored_wave(
   struct Chunk {
     u32x4_t kf[NCH][2][D_KS];
     u32x4_t vv[NCH][D_MT];
-    float bias[NCH][8];     // of the lane's eight keys, the last key first
+    float bias[MODS ? NCH : 1][8];     // of the lane's eight keys, the last key first
   };
-  const float* bias_row = mods->dist_bias != nullptr ? kappai_bias_row(*mods, h) : nullptr;
+  const float* bias_row = MODS && mods->dist_bias != nullptr ? kappai_bias_row(*mods, h) : nullptr;
   auto ask = [&](int c0, int my_page, Chunk& ch) {
     // Row r of the key tile tt (of the 32 keys from kb) is key kb + 8 (r / 4) + 4 tt + r % 4:
     // the lane that holds rows 4 kg .. 4 kg + 3 of both tiles' scores then holds the keys
     // kb + 8 kg .. + 7 in order, and their values are ONE 16-byte piece of a V^T row.
 #pragma unroll
     for (int c = 0; c < NCH; ++c) {
-      const int kb = kappai_key_at(c0 + 32 * c, lo32, kept);
+      const int kb = MODS ? kappai_key_at(c0 + 32 * c, lo32, kept) : c0 + 32 * c;
       // (what the row does not see reads as zero)
-      const int f_lo = kb < keep ? kb : lo, f_hi = kb < lo32 ? keep - 1 : hi;
+      const int f_lo = MODS && kb < keep ? kb : lo, f_hi = MODS && kb < lo32 ? keep - 1 : hi;
 #pragma unroll
       for (int tt = 0; tt < 2; ++tt) {
         const int key = kb + 8 * (col / 4) + 4 * tt + col % 4;
@@ -1568,18 +1618,20 @@ __device__ __forceinline__ void attn_decode_scored_wave(
       for (int mt = 0; mt < D_MT; ++mt)
         ch.vv[c][mt] = load_vt8_pg(vt_pool, pv, G, g, ps, 16 * mt + col, kb + 8 * kg,
                                     f_lo, f_hi);
-      if (bias_row != nullptr) {     // distances base .. base + 7, by the row's edges at most
-        const int base = max(-KAPPAI_BIAS_PAD, min(pos - kb - 8 * kg - 7, mods->dist_cols - 1));
-        const f32x4_any_t b0 = *reinterpret_cast<const f32x4_any_t*>(bias_row + base);
-        const f32x4_any_t b1 = *reinterpret_cast<const f32x4_any_t*>(bias_row + base + 4);
+      if constexpr (MODS) {
+        if (bias_row != nullptr) {     // distances base .. base + 7, by the row's edges at most
+          const int base = max(-KAPPAI_BIAS_PAD, min(pos - kb - 8 * kg - 7, mods->dist_cols - 1));
+          const f32x4_any_t b0 = *reinterpret_cast<const f32x4_any_t*>(bias_row + base);
+          const f32x4_any_t b1 = *reinterpret_cast<const f32x4_any_t*>(bias_row + base + 4);
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          ch.bias[c][i] = b0[i];
-          ch.bias[c][4 + i] = b1[i];
+          for (int i = 0; i < 4; ++i) {
+            ch.bias[c][i] = b0[i];
+            ch.bias[c][4 + i] = b1[i];
+          }
+        } else {
+#pragma unroll
+          for (int i = 0; i < 8; ++i) ch.bias[c][i] = 0.f;
         }
-      } else {
-#pragma unroll
-        for (int i = 0; i < 8; ++i) ch.bias[c][i] = 0.f;
       }
     }
   };
@@ -1587,7 +1639,7 @@ __device__ __forceinline__ void attn_decode_scored_wave(
 #pragma unroll
     for (int c = 0; c < NCH; ++c) {
       if (c0 + 32 * c >= k_end) break;
-      const int kb = kappai_key_at(c0 + 32 * c, lo32, kept);
+      const int kb = MODS ? kappai_key_at(c0 + 32 * c, lo32, kept) : c0 + 32 * c;
       f32x4_t s[2];
 #pragma unroll
       for (int tt = 0; tt < 2; ++tt) {
@@ -1604,10 +1656,12 @@ __device__ __forceinline__ void attn_decode_scored_wave(
 #pragma unroll
         for (int v = 0; v < 4; ++v) {
           const int key = kb + 8 * kg + 4 * tt + v;
-          const bool ok = (key >= lo || key < keep) && key <= hi;
+          const bool ok = (key >= lo || (MODS && key < keep)) && key <= hi;
           float x = s[tt][v] * scale;
-          if (mods->softcap > 0.f) x = kappai_fast_cap(x, mods->softcap);
-          x += ch.bias[c][7 - (4 * tt + v)];
+          if constexpr (MODS) {
+            if (mods->softcap > 0.f) x = kappai_fast_cap(x, mods->softcap);
+            x += ch.bias[c][7 - (4 * tt + v)];
+          }
           s[tt][v] = ok ? x * LOG2E : -INFINITY;
           mloc = fmaxf(mloc, s[tt][v]);
         }
@@ -1674,7 +1728,7 @@ __device__ __forceinline__ int step_keys_per_split(const int* __restrict__ row_p
   int kps = want > (1 << 30) ? (1 << 30) : (int)want;
   kps = max(kps, (longest + n_splits - 1) / n_splits);
   kps = max(kps, kps_min);
-  return (kps + 31) / 32 * 32;
+  return __builtin_amdgcn_readfirstlane((kps + 31) / 32 * 32);
 }
 
 // The keys of a row split over blocks: block (t, g, split) is one wave that takes the keys
@@ -1685,7 +1739,7 @@ __device__ __forceinline__ int step_keys_per_split(const int* __restrict__ row_p
 // (PLAN: the keys per split come from step_keys_per_split, else they are the caller's: a kernel of
 // its own, because the rule's code costs half a microsecond even where it is skipped)
 template <bool FUSED, bool PLAN, bool MODS = false>
-__global__ __launch_bounds__(64, FUSED || MODS || HEAD_DIM > 128 ? 1 : 2) void attn_decode_kernel(
+__global__ __launch_bounds__(64, (FUSED && HEAD_DIM != 64) || MODS || HEAD_DIM > 128 ? 1 : 2) void attn_decode_kernel(
     const bf16_t* __restrict__ q, int q_stride, const bf16_t* __restrict__ k_pool,
     const bf16_t* __restrict__ vt_pool, float* __restrict__ part_o, float* __restrict__ part_ml,
     const int* __restrict__ row_pos, const int* __restrict__ row_seg,
@@ -1721,8 +1775,8 @@ __global__ __launch_bounds__(64, FUSED || MODS || HEAD_DIM > 128 ? 1 : 2) void a
   f32x4_t o[D_MT];
   float m_run, l_run;
   if constexpr (MODS)
-    attn_decode_scored_wave(q, q_stride, k_pool, vt_pool, bt, max_blocks, t, g, H, G, ps, scale, lo,
-                            k_end - 1, k_begin, D_KPW, k_end, o, m_run, l_run, pos, &mods);
+    attn_decode_chunk_wave<true>(q, q_stride, k_pool, vt_pool, bt, max_blocks, t, g, H, G, ps, scale, lo,
+                                 k_end - 1, k_begin, D_KPW, k_end, o, m_run, l_run, pos, &mods);
   else
     attn_decode_wave<FUSED>(q, q_stride, k_pool, vt_pool, bt, max_blocks, t, g, H, G, ps, scale, lo,
                             k_begin, k_end, o, m_run, l_run, qk, pos);
@@ -1753,7 +1807,9 @@ __device__ __forceinline__ void attn_one_row(const bf16_t* q, int q_stride, cons
                                              int G, int ps, int window, float scale,
                                              const kappai_score_mods& mods, float* sh, int NW,
                                              const QkFuse* qk) {
-  const int lane = threadIdx.x % WAVE, wave = threadIdx.x / WAVE;
+  const int lane = threadIdx.x % WAVE;
+  // (in scalar registers: the walk over the wave's keys is then scalar work)
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
   const int rep = H / G;
   const int col = lane % 16, kg = lane / 16;
   const int lo = kappai_first_key(pos, window);
@@ -1762,9 +1818,9 @@ __device__ __forceinline__ void attn_one_row(const bf16_t* q, int q_stride, cons
   const int k_end = pos + 1;
   f32x4_t o[D_MT];
   float m_run, l_run;
-  if constexpr (MODS) {
-    attn_decode_scored_wave(q, q_stride, k_pool, vt_pool, bt, max_blocks, t, g, H, G, ps, scale, lo, pos,
-                            k_begin + wave * D_KPW, NW * D_KPW, k_end, o, m_run, l_run, pos, &mods);
+  if constexpr (MODS || (HEAD_DIM == 256 && !FUSED)) {
+    attn_decode_chunk_wave<MODS>(q, q_stride, k_pool, vt_pool, bt, max_blocks, t, g, H, G, ps, scale, lo, pos,
+                                 k_begin + wave * D_KPW, NW * D_KPW, k_end, o, m_run, l_run, pos, &mods);
   } else {
     // equal shares in whole parts of UNIT keys
     const int per = ((k_end - k_begin + UNIT - 1) / UNIT + NW - 1) / NW * UNIT;

@@ -64,3 +64,71 @@ def test_lone_rows_with_a_sink(ops, variant):  # noqa: F811
     sink = rand((H,), F32, 24).to(DEV)
     compare(ops, c, H, G, d, 16, 0, mods=ops.ScoreMods(sink=sink), q_tiles=c["q_tiles"], kernel="prefill",
             prefill_variant=variant)
+
+
+def pools_for(held, G, d, ps, seed, missing=()):
+    """Pools of random keys and values in which every row has pages of its own, NaN where it holds nothing;
+    ``missing``: (row, page of the row) that its table does not name."""
+    gen = torch.Generator(device=DEV).manual_seed(seed)
+    pages = [p // ps + 1 for p in held]
+    shape = (sum(pages) + 1, G, ps, d)
+    k = torch.randn(shape, generator=gen, device=DEV).to(BF16)
+    v = torch.randn(shape, generator=gen, device=DEV).to(BF16).transpose(2, 3).contiguous()
+    order = torch.randperm(sum(pages), generator=gen, device=DEV) + 1      # (page 0 is nobody's)
+    bt = torch.full((len(held), max(pages) + 2), -1, dtype=torch.int32, device=DEV)
+    at = 0
+    for r, (p, n) in enumerate(zip(held, pages)):
+        bt[r, :n] = order[at:at + n]
+        last = int(order[at + n - 1])
+        k[last, :, p % ps + 1:] = float("nan")
+        v[last, :, :, p % ps + 1:] = float("nan")
+        at += n
+    k[0], v[0] = float("nan"), float("nan")
+    for r, page in missing:
+        bt[r, page] = -1
+    i32 = lambda a: torch.tensor(a, dtype=torch.int32, device=DEV)  # noqa: E731
+    return k, v, bt, i32(held), torch.arange(len(held), dtype=torch.int32, device=DEV)
+
+
+# a wave walks the whole of every row (as many rows and kv heads as there are blocks to split keys over): one part
+# of 32 keys to fifteen, which is none to three rounds of the parts under way and every rest; pages of 64 by 64
+@pytest.mark.parametrize("H,G,d,ps", [(64, 64, 64, 16), (128, 64, 128, 16), (64, 64, 16, 16), (64, 64, 32, 32),
+                                      (64, 64, 48, 16), (64, 64, 192, 16), (64, 64, 256, 16), (64, 64, 80, 48)])
+def test_every_number_of_parts(ops, H, G, d, ps):  # noqa: F811
+    held = [32 * n + o for n in range(15) for o in (0, 1, 13, 31)] + [64 * ps + o for o in (-1, 0, 33, 127)]
+    k, v, bt, pos, seg = pools_for(held, G, d, ps, 41)
+    assert ops.decode_splits(32, len(held), G, max(held) + 1)[1] == 1
+    q = rand((len(held), H * d), BF16, 42).to(DEV)
+    args = (q, H, G, d, k, v, pos, seg, bt, ps, 1.0 / math.sqrt(d))
+    want = ops.paged_attention(*args, kernel="rows")
+    for kernel in ("decode-split", "decode-block"):
+        got = ops.paged_attention(*args, single_rows=True, max_position=max(held), kernel=kernel)
+        close(got.float(), want.float().cpu().double(), 4 * BF16_ULP, kernel)
+
+
+# pages that a window has passed, in the part of the first key that it sees; a page among those that a row sees,
+# whose keys and values read as zero
+@pytest.mark.parametrize("window", [0, 45])
+@pytest.mark.parametrize("kernel", ["decode-split", "decode-block"])
+def test_pages_that_are_not_there(ops, window, kernel):  # noqa: F811
+    H, G, d, ps = 4, 2, 64, 16
+    held = [200, 77, 95, 300]
+    gone = [(0, 11), (1, 4), (3, 18)] + ([(r, p) for r, n in enumerate(held)
+                                         for p in range((n + 1 - window) // ps)] if window else [(2, 0)])
+    k, v, bt, pos, seg = pools_for(held, G, d, ps, 43, gone)
+    q = rand((len(held), H * d), BF16, 44)
+    got = ops.paged_attention(q.to(DEV), H, G, d, k, v, pos, seg, bt, ps, 0.2, window=window, single_rows=True,
+                              max_position=max(held), kernel=kernel)
+    want = torch.zeros(len(held), H, d, dtype=torch.float64)
+    kc, vc, tables = k.cpu().double(), v.cpu().double().transpose(2, 3), bt.cpu()
+    for r, n in enumerate(held):
+        keys = range(max(0, n + 1 - window) if window else 0, n + 1)
+        for h in range(H):
+            page = [int(tables[r, i // ps]) for i in keys]
+            kk = torch.stack([kc[p, h // 2, i % ps] if p >= 0 else torch.zeros(d).double()
+                              for p, i in zip(page, keys)])
+            vv = torch.stack([vc[p, h // 2, i % ps] if p >= 0 else torch.zeros(d).double()
+                              for p, i in zip(page, keys)])
+            want[r, h] = torch.softmax(kk @ q.double().view(-1, H, d)[r, h] * 0.2, 0) @ vv
+    # (weights and results are rounded to bfloat16)
+    close(got.float(), want.view(len(held), -1), 2 * BF16_ULP, kernel)

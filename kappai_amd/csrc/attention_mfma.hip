@@ -136,11 +136,20 @@ __device__ __forceinline__ u32x4_t load_k8(const bf16_t* __restrict__ k_pool,
 #define P_KS (HEAD_DIM / 16)            // k-steps of S^T over d
 #define P_MT ((HEAD_DIM + 31) / 32)     // row tiles of O^T over d
 
-// One row and one kv head by a block of NW waves, which take the keys in chunks in turn and meet in `sh`
+// (decode) keys whose loads a wave has in flight at once (their registers: keys * HEAD_DIM / 64)
+#define D_KPW (HEAD_DIM <= 64 ? 128 : (HEAD_DIM <= 128 ? 64 : 32))
+// What the shares of a row's keys are whole numbers of, over the waves of a block and over blocks.  A wave
+// costs nothing but its merge, a block a place in a second kernel: 96 keys a block for 128 are 3 to 9 % more
+// at head sizes 80 to 128, where 96 are three parts for two (4 rows of up to 8,000 keys, 32 heads of 128
+// on 8: 28.5 us against 26.2), and equal at 64; 64 keys a wave for 32 are 2 to 4 % more at both.
+#define D_SHARE (HEAD_DIM == 64 || HEAD_DIM == 128 ? 32 : D_KPW)
+#define D_SPLIT_SHARE (HEAD_DIM == 64 ? 32 : D_KPW)
+
+// One row and one kv head by a block of NW waves, which take equal shares of the keys and meet in `sh`
 // (NW (rep HEAD_DIM + 32) floats of LDS; rep <= 16): defined with the decode kernels.
 // (FUSED: with the prologue of `qk` in the waves that have keys)
 struct QkFuse;
-template <bool MODS, bool FUSED = false, int UNIT = 32>
+template <bool MODS, bool FUSED = false>
 __device__ __forceinline__ void attn_one_row(const bf16_t* q, int q_stride, const bf16_t* k_pool,
                                              const bf16_t* vt_pool, bf16_t* out, int out_stride,
                                              const int* bt, int max_blocks, int t, int pos, int g, int H,
@@ -185,11 +194,11 @@ __global__ __launch_bounds__(P_NW * WAVE, P_MIN_WAVES) void attn_prefill_kernel(
   constexpr int SH_O = P_NW > 1 ? (P_NW - 1) * P_MT * 16 * WAVE : 1;
   __shared__ float sh_o[SH_O];
   if constexpr (!MODS && P_NW > 1) {
-    // A decoded token beside portions: all query heads of its kv head at once and the keys in chunks of
-    // D_KPW, as in a decode step.  Walked like a portion's tile, head by head and 32 keys at a time, a
+    // A decoded token beside portions: all query heads of its kv head at once and an equal share of the keys
+    // a wave, as in a decode step.  Walked like a portion's tile, head by head and 32 keys at a time, a
     // row's keys were read rep times and a chain of up to 12 round trips to memory held the kernel: 63 rows
-    // of 100 to 1,500 keys beside a portion of 512, 16 heads on 8: 45.2 us, now 35.8; 32 heads on 8 in
-    // the kernel below 65.3, now 34.5; 6 rows beside a portion of 100: 17.6, now 15.6.
+    // of up to 1,500 keys beside a portion of 512, 16 heads on 8: 43.9 us, now 30.6; 32 heads on 8 in
+    // the kernel below 62.4, now 29.2; 8 rows of up to 500 keys 11.0, now 10.3.
     static_assert(P_NW * (16 * HEAD_DIM + 32) <= SH_O || HEAD_DIM < 32, "LDS of a lone row");
     const int rep = H / G;
     if (nr == 1 && P_NW * (rep * HEAD_DIM + 32) <= SH_O && rep <= 16) {
@@ -1132,8 +1141,6 @@ __global__ __launch_bounds__(8 * WAVE) void attn_prefill_heads_kernel(
 // ---------------------------------------------------------------------------------------
 #define D_KS ((HEAD_DIM + 31) / 32)     // k-steps of S^T over d (32 each)
 #define D_MT (HEAD_DIM / 16)            // row tiles of O^T over d
-// keys whose loads a wave has in flight at once (their registers: keys * HEAD_DIM / 64)
-#define D_KPW (HEAD_DIM <= 64 ? 128 : (HEAD_DIM <= 128 ? 64 : 32))
 
 // head sizes whose decode kernel can take the prologue below: the rotation's partner d / 2 further
 // must lie in the same lane, and the registers must hold it beside a chunk of keys
@@ -1704,8 +1711,9 @@ __device__ __forceinline__ void attn_decode_chunk_wave(
 // as many keys a split that the rows' keys together give D_TARGET_WAVES waves work (requests of
 // mixed lengths then get shorter splits than their longest context alone would give them, and
 // no wave walks a long row's keys by itself while the rest of the chip has nothing to do), and
-// no fewer than the longest row needs to fit into n_splits.  Every wave of the step computes the
-// same number from the same table; splits past a row's keys do nothing and are not merged.
+// no fewer than the longest row needs to fit into n_splits, in whole numbers of `unit` (the scored wave walks
+// chunks of D_KPW).  Every wave of the step computes the same number from the same table; splits past a row's
+// keys do nothing and are not merged.
 #define D_TARGET_WAVES 2048
 __device__ __forceinline__ int keys_of_row(int pos, int window, int keep) {
   const int lo32 = kappai_first_key(pos, window) / 32 * 32;
@@ -1714,7 +1722,7 @@ __device__ __forceinline__ int keys_of_row(int pos, int window, int keep) {
 __device__ __forceinline__ int step_keys_per_split(const int* __restrict__ row_pos,
                                                    const int* __restrict__ row_ids, int n_rows,
                                                    int window, int keep, int G, int kps_min,
-                                                   int n_splits) {
+                                                   int n_splits, int unit) {
   const int lane = threadIdx.x % WAVE;
   int total32 = 0, longest = 0;                  // the sum in units of 32 keys, rounded up by row
   for (int i = lane; i < n_rows; i += WAVE) {
@@ -1728,7 +1736,7 @@ __device__ __forceinline__ int step_keys_per_split(const int* __restrict__ row_p
   int kps = want > (1 << 30) ? (1 << 30) : (int)want;
   kps = max(kps, (longest + n_splits - 1) / n_splits);
   kps = max(kps, kps_min);
-  return __builtin_amdgcn_readfirstlane((kps + 31) / 32 * 32);
+  return __builtin_amdgcn_readfirstlane((kps + unit - 1) / unit * unit);
 }
 
 // The keys of a row split over blocks: block (t, g, split) is one wave that takes the keys
@@ -1761,7 +1769,7 @@ __global__ __launch_bounds__(64, (FUSED && HEAD_DIM != 64) || MODS || HEAD_DIM >
   const int seg = row_seg[t];
   const int keep = MODS ? mods.keep_first : 0;
   const int kps = PLAN ? step_keys_per_split(row_pos, row_ids, (int)gridDim.x, window, keep, G,
-                                             keys_per_split, n_splits)
+                                             keys_per_split, n_splits, MODS ? D_KPW : D_SPLIT_SHARE)
                        : keys_per_split;
   const int* bt = block_tables + (size_t)seg * max_blocks;
   const int lo = kappai_first_key(pos, window);
@@ -1794,13 +1802,13 @@ __global__ __launch_bounds__(64, (FUSED && HEAD_DIM != 64) || MODS || HEAD_DIM >
 // (eight waves at most: a wave keeps a whole chunk's loads in registers, which 16 waves a block
 // would not leave room for)
 #define D_BLOCK_MAX_WAVES 8
-// The keys of a row split over the waves of one block (t, g): wave w takes the chunks w, w + NW,
-// ... of D_KPW keys, the waves' results meet in LDS and are added up there in the order of the
-// waves, so that nothing goes through memory and no second kernel is needed.  The split of a row's
-// keys depends on the row's own position and on the number of waves only.  For batches with
+// The keys of a row split over the waves of one block (t, g): equal shares in whole D_SHAREs (with MODS wave w
+// takes the chunks w, w + NW, ... of D_KPW keys), the waves' results meet in LDS and are added up there in
+// the order of the waves, so that nothing goes through memory and no second kernel is needed.  The split of
+// a row's keys depends on the row's own position and on the number of waves only.  For batches with
 // (rows x kv heads) enough to fill the chip, or contexts short enough for one block.
 // LDS: sh_o [NW][rep][HEAD_DIM], then sh_m [NW][16], sh_l [NW][16] (floats).
-template <bool MODS, bool FUSED, int UNIT>
+template <bool MODS, bool FUSED>
 __device__ __forceinline__ void attn_one_row(const bf16_t* q, int q_stride, const bf16_t* k_pool,
                                              const bf16_t* vt_pool, bf16_t* out, int out_stride,
                                              const int* bt, int max_blocks, int t, int pos, int g, int H,
@@ -1822,8 +1830,7 @@ __device__ __forceinline__ void attn_one_row(const bf16_t* q, int q_stride, cons
     attn_decode_chunk_wave<MODS>(q, q_stride, k_pool, vt_pool, bt, max_blocks, t, g, H, G, ps, scale, lo, pos,
                                  k_begin + wave * D_KPW, NW * D_KPW, k_end, o, m_run, l_run, pos, &mods);
   } else {
-    // equal shares in whole parts of UNIT keys
-    const int per = ((k_end - k_begin + UNIT - 1) / UNIT + NW - 1) / NW * UNIT;
+    const int per = ((k_end - k_begin + D_SHARE - 1) / D_SHARE + NW - 1) / NW * D_SHARE;
     const int from = k_begin + wave * per;
     if (FUSED && from >= k_end) {              // (no keys: no prologue either)
 #pragma unroll
@@ -1878,11 +1885,7 @@ __global__ __launch_bounds__(D_BLOCK_MAX_WAVES * WAVE) void attn_decode_block_ke
     float scale, kappai_score_mods mods) {
   extern __shared__ float sh_dec[];
   const int t = blockIdx.x;
-  // Shares of whole parts of 32 keys at the head sizes of long use; at the others of whole chunks, as the
-  // kernel had them: two maps of 16 that are subtracted leave 0.04 to 0.06 of the largest value to the
-  // rounding of either, and that stays what it was.
-  constexpr int UNIT = HEAD_DIM == 64 || HEAD_DIM == 128 ? 32 : D_KPW;
-  attn_one_row<MODS, false, UNIT>(q, q_stride, k_pool, vt_pool, out, out_stride,
+  attn_one_row<MODS>(q, q_stride, k_pool, vt_pool, out, out_stride,
                      block_tables + (size_t)row_seg[t] * max_blocks, max_blocks, t, row_pos[t],
                      blockIdx.y, H, G, ps, window, scale, mods, sh_dec, blockDim.x / WAVE);
 }
@@ -1916,7 +1919,7 @@ __global__ __launch_bounds__(MERGE_WAVES * WAVE) void attn_merge_kernel(
     const float* __restrict__ part_o, const float* __restrict__ part_ml,
     bf16_t* __restrict__ out, int out_stride, int H, int splits_stride,
     const int* __restrict__ row_ids, const int* __restrict__ row_pos, int window, int keep, int G,
-    int kps_min, int planned, const float* __restrict__ sink) {
+    int kps_min, int plan_unit, const float* __restrict__ sink) {
   constexpr int NPL = (HEAD_DIM + WAVE - 1) / WAVE;
   __shared__ float sh_acc[MERGE_WAVES][NPL * WAVE];
   __shared__ float sh_l[MERGE_WAVES];
@@ -1946,9 +1949,9 @@ __global__ __launch_bounds__(MERGE_WAVES * WAVE) void attn_merge_kernel(
   if (wave + MERGE_WAVES * lane < splits_stride)
     ml_first = *reinterpret_cast<const float2*>(part_ml + 2 * (base + wave + MERGE_WAVES * lane));
   // the splits of this row that had keys (the decode kernel's own rule)
-  const int kps = planned ? step_keys_per_split(row_pos, row_ids, (int)gridDim.x, window, keep, G,
-                                                kps_min, splits_stride)
-                          : kps_min;
+  const int kps = plan_unit ? step_keys_per_split(row_pos, row_ids, (int)gridDim.x, window, keep, G,
+                                                  kps_min, splits_stride, plan_unit)
+                            : kps_min;
   const int n_splits = (keys_of_row(row_pos[t], window, keep) + kps - 1) / kps;
 #pragma unroll
   for (int k = 0; k < MERGE_AHEAD; ++k)
@@ -2190,8 +2193,8 @@ static int launch_decode(const void* q, int q_stride, const void* k_pool, const 
 #undef KAPPAI_DECODE
   hipLaunchKernelGGL(attn_merge_kernel, dim3(T, H), dim3(MERGE_WAVES * WAVE), 0, stream,
                      (const float*)part_o, (const float*)part_ml, (bf16_t*)out, out_stride, H,
-                     n_splits, row_ids, row_pos, window, m.keep_first, G, keys_per_split, plan ? 1 : 0,
-                     m.sink);
+                     n_splits, row_ids, row_pos, window, m.keep_first, G, keys_per_split,
+                     plan ? (scored ? D_KPW : D_SPLIT_SHARE) : 0, m.sink);
   KAPPAI_RETURN_LAUNCH_STATUS();
 }
 

@@ -132,3 +132,69 @@ def test_pages_that_are_not_there(ops, window, kernel):  # noqa: F811
             want[r, h] = torch.softmax(kk @ q.double().view(-1, H, d)[r, h] * 0.2, 0) @ vv
     # (weights and results are rounded to bfloat16)
     close(got.float(), want.view(len(held), -1), 2 * BF16_ULP, kernel)
+
+
+# Two maps whose difference is the result (head size 16, the second map uniform over all keys): what bfloat16
+# results leave of it when exact maps are rounded is the floor; shares of a row's keys over waves and blocks may
+# add the rounding of their weights, less than half as much again.
+@pytest.mark.parametrize("window", [0, 70, 200])
+@pytest.mark.parametrize("d,T", [(16, 360), (48, 330), (16, 1500)])
+def test_difference_of_two_maps(ops, window, d, T):  # noqa: F811
+    ps, lam, needle, portion = 16, 0.9, 100, 40
+    x = 0.05 * rand((T, 2, d), F32, 45)
+    x[needle] = 3.0
+    x[needle, :, ::2] += 4.0
+    x[needle + 1:] += 0.35                       # every later query looks for that key
+    x = x.to(BF16)
+    val = rand((T, 2, d), BF16, 46)
+    keys, vals = torch.zeros(T, 4, d, dtype=BF16), torch.zeros(T, 4, d, dtype=BF16)
+    keys[:, ::2], vals[:, ::2], vals[:, 1::2] = x, val, val
+    n_pages = T // ps + 1
+    k = torch.full((n_pages, 4, ps, d), float("nan"), dtype=BF16)
+    v = torch.full((n_pages, 4, d, ps), float("nan"), dtype=BF16)
+    for t in range(T):
+        k[t // ps, :, t % ps], v[t // ps, :, :, t % ps] = keys[t], vals[t]
+    pos = list(range(T - 30, T)) + [needle + (window or 150) + i for i in range(-2, 3)]
+    n = len(pos)
+    exact = torch.zeros(n, 4, d, dtype=torch.float64)
+    for r, p in enumerate(pos):
+        seen = slice(max(0, p + 1 - window) if window else 0, p + 1)
+        for h in range(4):
+            exact[r, h] = torch.softmax(keys[seen, h].double() @ keys[p, h].double(), 0) @ vals[seen, h].double()
+
+    def result(maps):
+        o = maps[:, ::2] - lam * maps[:, 1::2]
+        return o / torch.sqrt((o * o).mean(-1, keepdim=True) + 1e-5)
+    want = result(exact)
+    floor = float((result(exact.to(BF16).double()) - want).abs().max())
+    on = lambda a: torch.tensor(a, dtype=torch.int32, device=DEV)  # noqa: E731
+    q = torch.cat([keys[pos], torch.zeros(portion, 4, d, dtype=BF16)]).view(n + portion, -1).to(DEV)
+    bt = torch.arange(n_pages, dtype=torch.int32, device=DEV).repeat(64 * n + 1, 1)
+    tiles = [(r, r, 1, 1 << 16) for r in range(n)] + [(n, n, 32, 2 << 16), (n, n + 32, 8, 1 | 2 << 16)]
+    common = dict(window=window, max_position=T - 1)
+    args = lambda rows: (q[rows], 4, 4, d, k.to(DEV), v.to(DEV), on(pos + list(range(portion)))[rows],  # noqa: E731
+                         on(list(range(n)) + [n] * portion)[rows], bt, ps, 1.0)
+    every = torch.arange(n + portion, device=DEV)
+    many = torch.arange(n, device=DEV).repeat(6)       # rows enough that the shares are planned
+    got = {"beside a portion": ops.paged_attention(*args(every), q_tiles=on(tiles), kernel="prefill", **common)[:n],
+           "split": ops.paged_attention(*args(many), single_rows=True, kernel="decode-split", **common)[:n],
+           "block": ops.paged_attention(*args(every[:n]), single_rows=True, kernel="decode-block", **common)}
+    for what, ctx in got.items():
+        err = float((result(ctx.cpu().double().view(n, 4, d)) - want).abs().max())
+        assert err <= 1.5 * floor + 1e-4, (what, err, floor)
+
+
+# shares that come from the rows' own lengths and are no whole number of the smallest ones: the kernel and the merge
+# behind it settle on the same
+@pytest.mark.parametrize("d,G,keys", [(64, 8, 2600), (128, 8, 1700), (48, 8, 2600), (256, 4, 900)])
+@pytest.mark.parametrize("softcap", [0.0, 20.0])
+def test_planned_shares(ops, d, G, keys, softcap):  # noqa: F811
+    H, ps, T = 2 * G, 16, 64
+    held = [keys - 1 - (r * 7) % 50 for r in range(T)]
+    k, v, bt, pos, seg = pools_for(held, G, d, ps, 47)
+    q = rand((T, H * d), BF16, 48).to(DEV)
+    mods = ops.ScoreMods(softcap=softcap) if softcap else None
+    args = (q, H, G, d, k, v, pos, seg, bt, ps, 1.0 / math.sqrt(d))
+    want = ops.paged_attention(*args, kernel="rows", mods=mods)
+    got = ops.paged_attention(*args, single_rows=True, max_position=max(held), kernel="decode-split", mods=mods)
+    close(got.float(), want.float().cpu().double(), 4 * BF16_ULP, (d, softcap))

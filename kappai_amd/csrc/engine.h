@@ -342,8 +342,9 @@ int kappai_split_k_for(int M, int N, int K);
 int kappai_sums_in_f32(int M, int N, int K);
 
 // The most keys with which the decode attention keeps a row's keys in one block (attn_decode_block) where
-// `few` is what it takes for any number of rows.
-int kappai_decode_block_keys(int few, int rows, int G, int head_dim);
+// `few` is what it takes for any number of rows (at head sizes up to 128; beyond, the most it ever takes).
+// waves: of a block, for the query heads a kv head (decode_block_waves).
+int kappai_decode_block_keys(int few, int rows, int G, int head_dim, int waves);
 
 // How the decode attention that splits a row's keys over blocks cuts n_keys keys of `rows` rows
 // over G kv heads: the fewest keys a split and the most splits a row (the host asks the same

@@ -638,18 +638,25 @@ extern "C" int kappai_split_k_for(int M, int N, int K) { return ranges_for(M, N,
 extern "C" int kappai_sums_in_f32(int M, int N, int K) { return ranges_for(M, N, K).f32 ? 1 : 0; }
 
 // One block a (row, kv head) takes a row's keys in at 50 GB/s or so, but needs no second kernel, and with
-// blocks enough for the chip nothing is won by more of them.  us against the kernel that splits the keys over
-// blocks and its merge, head size 64, 8 kv heads: 8 rows of 40 / 307 / 1,024 keys 4.4 / 6.5 / 9.1 against
-// 6.8 / 8.0 / 9.5 (2,048 keys 13.5 / 11.0); 24 rows of up to 614 / 2,048 keys 8.3 / 17.1 against 12.2 / 18.3
-// (16 rows 14.8 / 13.6); 32 rows of up to 1,228 / 4,096 keys 12.3 / 35.2 against 16.3 / 36.4, 64 rows 25.2 / 67.7
-// against 26.7 / 64.9.  A key of 128 is twice the bytes: 64 rows, 4 kv heads, up to 2,048 keys 35.3 against 37.8.
-// Head sizes beyond (three waves a block, registers spilled) lose from the first key on: 20 against 9.7.
-extern "C" int kappai_decode_block_keys(int few, int rows, int G, int head_dim) {
-  if (head_dim > 128) return 0;
-  if (head_dim != 64 && head_dim != 128) return few;
+// blocks enough for the chip nothing is won by more of them.  But a long row among short ones is then the whole
+// step's time, and only the longest row is known here (in a captured step as a power of two).  Block against
+// split and merge at the most keys of every line, rows of equal lengths / of lengths spread evenly / one long row
+// among rows of 64 keys, 32 heads of 64 on 8: 64 blocks, 1,024 keys 0.93 / 0.94 / 1.01 of the time, 128 blocks,
+// 2,048 keys 0.95 / 1.06 / 1.07, 192 blocks 0.79 / 0.90 / 1.14, 256 blocks 0.81 / 0.82 / 1.04, 512 blocks 0.87 / 0.91 /
+// 1.20, 256 blocks, 4,096 keys 0.88 / 0.91 / 1.38.  32 heads of 128: 128 blocks, 1,024 keys 0.91 / 1.03 / 1.18, 192
+// blocks 0.77 / 0.85 / 1.10, 256 blocks, 2,048 keys 0.86 / 0.88 / 1.52.
+// Head sizes above 128 with eight waves a block: 8 blocks of 192, 100 keys 0.85, 300 keys 1.17; 128 blocks of 256, 200
+// keys 0.90 / 0.88 / 1.00, 500 keys 0.87 / 1.04 / 1.47; 256 blocks, 500 keys 0.74 / 0.77 / 0.95.  With fewer waves (three
+// where 16 heads of 256 share their keys): 64 blocks, 100 keys 1.54, 256 blocks 0.66, 500 keys 0.74 / 0.86 / 1.08.
+extern "C" int kappai_decode_block_keys(int few, int rows, int G, int head_dim, int waves) {
   const long blocks = (long)rows * G;
-  const int at64 = blocks >= 256 ? 4096 : (blocks >= 192 ? 2048 : (blocks >= 64 ? 1024 : few));
-  const int keys = at64 * 64 / head_dim;
+  if (head_dim > 128) {
+    const int keys = blocks >= 256 ? 512 : (waves < 8 ? 0 : (blocks >= 128 ? 256 : 128));
+    return keys < few ? keys : few;
+  }
+  int keys = few;
+  if (head_dim == 64 && blocks >= 64) keys = blocks >= 192 ? 2048 : 1024;
+  if (head_dim == 128 && blocks >= 192) keys = 1024;
   return keys > few ? keys : few;
 }
 

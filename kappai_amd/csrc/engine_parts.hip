@@ -154,9 +154,9 @@ int decode_keys(const kappai_batch& b, const kappai_attention_mixer& L) {
 }
 bool decode_block_form(const kappai_model& m, const kappai_batch& b,
                        const kappai_attention_mixer& L, int M) {
-  return L.mfma->decode_block_waves(L.heads / L.kv_heads) > 0 &&
-         decode_keys(b, L) <= kappai_decode_block_keys(m.tuning.decode_block_max_keys, M, L.kv_heads,
-                                                       L.head_dim);
+  const int waves = L.mfma->decode_block_waves(L.heads / L.kv_heads);
+  return waves > 0 && decode_keys(b, L) <= kappai_decode_block_keys(m.tuning.decode_block_max_keys, M,
+                                                                    L.kv_heads, L.head_dim, waves);
 }
 
 kappai_carry attention_mixer(kappai_step* s, const void* desc, kappai_rows x, float* resid,

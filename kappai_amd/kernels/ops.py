@@ -22,7 +22,8 @@ DECODE_WAVES = 4096       # blocks the grid of the split-key decode attention pr
                           # rows really hold (requests of mixed lengths get shorter splits)
 DECODE_MAX_SPLITS = 128   # partial results of a row's head that the merge kernel adds up at most
 # Keys up to which one block a (row, kv head) takes them all, its waves merging in LDS, however few
-# the rows; with more rows up to more keys (kappai_decode_block_keys in csrc/engine.hip, measured there)
+# the rows (head sizes up to 128); with more rows up to more keys (kappai_decode_block_keys in
+# csrc/engine.hip, measured there)
 DECODE_BLOCK_MAX_KEYS = 512
 
 _c_int, _c_float, _c_long, _vp = ctypes.c_int, ctypes.c_float, ctypes.c_long, ctypes.c_void_p
@@ -958,7 +959,8 @@ def decode_form(n_heads: int, n_kv_heads: int, head_dim: int, max_position: int,
     lib = library("attention_mfma", HEAD_DIM=head_dim)
     block_waves = lib.kappai_attn_decode_block_waves(n_heads // n_kv_heads)
     most = DECODE_BLOCK_MAX_KEYS if scored else library("engine").kappai_decode_block_keys(
-        _c_int(DECODE_BLOCK_MAX_KEYS), _c_int(n_rows), _c_int(n_kv_heads), _c_int(head_dim))
+        _c_int(DECODE_BLOCK_MAX_KEYS), _c_int(n_rows), _c_int(n_kv_heads), _c_int(head_dim),
+        _c_int(block_waves))
     return "decode-block" if block_waves and n_keys <= most else "decode-split"
 
 

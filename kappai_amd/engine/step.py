@@ -26,7 +26,9 @@ from .cforward import CForward, NotDescribed, Workspace
 # attention keeps in one block for any number of rows: kappai_decode_block_keys in csrc/engine.hip)
 CONTEXT_BUCKET_MIN = 512
 DECODE_RING = 8            # decode steps whose tables can be queued ahead of the GPU
-MAX_DECODE_GRAPHS = 48
+# Graphs that are kept: of every batch size below for contexts up to 512, 1024, 2048 and 4096, and a few more (a
+# server that goes through more shapes than this captures again what it dropped)
+MAX_DECODE_GRAPHS = 62
 
 
 # A decode step of B requests that all want logits is replayed from the graph of the next

@@ -385,3 +385,10 @@ def test_decode_graphs_are_dropped_in_order_of_last_use():
     assert next(iter(runner._graphs)) == ("b",)          # what the next capture would drop
     bound = StepRunner.graph_bytes_bound(65536, 60)      # 60 rows run in the graph of 64
     assert bound == int(MAX_DECODE_GRAPHS * 64 * 65536 * 4 * 1.25)
+
+
+def test_graphs_of_every_batch_size_and_of_contexts_up_to_4096_are_kept():
+    from kappai_amd.engine.step import DECODE_BATCH_BUCKETS, MAX_DECODE_GRAPHS, _context_bucket
+
+    contexts = {_context_bucket(n) for n in range(1, 4097)}
+    assert max(contexts) == 4096 and len(DECODE_BATCH_BUCKETS) * len(contexts) <= MAX_DECODE_GRAPHS

@@ -138,18 +138,21 @@ __device__ __forceinline__ u32x4_t load_k8(const bf16_t* __restrict__ k_pool,
 
 // (decode) keys whose loads a wave has in flight at once (their registers: keys * HEAD_DIM / 64)
 #define D_KPW (HEAD_DIM <= 64 ? 128 : (HEAD_DIM <= 128 ? 64 : 32))
-// What the shares of a row's keys are whole numbers of, over the waves of a block and over blocks.  A wave
-// costs nothing but its merge, a block a place in a second kernel: 96 keys a block for 128 are 3 to 9 % more
-// at head sizes 80 to 128, where 96 are three parts for two (4 rows of up to 8,000 keys, 32 heads of 128
-// on 8: 28.5 us against 26.2), and equal at 64; 64 keys a wave for 32 are 2 to 4 % more at both.
-#define D_SHARE (HEAD_DIM == 64 || HEAD_DIM == 128 ? 32 : D_KPW)
+// What the shares of a row's keys over blocks are whole numbers of.  A block costs a place in a second kernel:
+// 96 keys a block for 128 are 3 to 9 % more at head sizes 80 to 128, where 96 are three parts for two (4 rows of
+// up to 8,000 keys, 32 heads of 128 on 8: 28.5 us against 26.2), and equal at 64.
 #define D_SPLIT_SHARE (HEAD_DIM == 64 ? 32 : D_KPW)
+// ... and over the waves of a block in a decode step: 64 keys for 32 are 2 to 4 % more at head sizes 64 and 128.  At
+// the others whole chunks, as the kernel had them: one measure of the differential attention's maps of 16,
+// whose difference leaves little but the rounding of either, hangs on the order of their sums.  (A decoded
+// row beside portions takes shares of 32 at every head size.)
+#define D_BLOCK_SHARE (HEAD_DIM == 64 || HEAD_DIM == 128 ? 32 : D_KPW)
 
 // One row and one kv head by a block of NW waves, which take equal shares of the keys and meet in `sh`
 // (NW (rep HEAD_DIM + 32) floats of LDS; rep <= 16): defined with the decode kernels.
 // (FUSED: with the prologue of `qk` in the waves that have keys)
 struct QkFuse;
-template <bool MODS, bool FUSED = false>
+template <bool MODS, bool FUSED = false, int SHARE = 32>
 __device__ __forceinline__ void attn_one_row(const bf16_t* q, int q_stride, const bf16_t* k_pool,
                                              const bf16_t* vt_pool, bf16_t* out, int out_stride,
                                              const int* bt, int max_blocks, int t, int pos, int g, int H,
@@ -1802,13 +1805,13 @@ __global__ __launch_bounds__(64, (FUSED && HEAD_DIM != 64) || MODS || HEAD_DIM >
 // (eight waves at most: a wave keeps a whole chunk's loads in registers, which 16 waves a block
 // would not leave room for)
 #define D_BLOCK_MAX_WAVES 8
-// The keys of a row split over the waves of one block (t, g): equal shares in whole D_SHAREs (with MODS wave w
+// The keys of a row split over the waves of one block (t, g): equal shares (with MODS wave w
 // takes the chunks w, w + NW, ... of D_KPW keys), the waves' results meet in LDS and are added up there in
 // the order of the waves, so that nothing goes through memory and no second kernel is needed.  The split of
 // a row's keys depends on the row's own position and on the number of waves only.  For batches with
 // (rows x kv heads) enough to fill the chip, or contexts short enough for one block.
 // LDS: sh_o [NW][rep][HEAD_DIM], then sh_m [NW][16], sh_l [NW][16] (floats).
-template <bool MODS, bool FUSED>
+template <bool MODS, bool FUSED, int SHARE>
 __device__ __forceinline__ void attn_one_row(const bf16_t* q, int q_stride, const bf16_t* k_pool,
                                              const bf16_t* vt_pool, bf16_t* out, int out_stride,
                                              const int* bt, int max_blocks, int t, int pos, int g, int H,
@@ -1830,7 +1833,7 @@ __device__ __forceinline__ void attn_one_row(const bf16_t* q, int q_stride, cons
     attn_decode_chunk_wave<MODS>(q, q_stride, k_pool, vt_pool, bt, max_blocks, t, g, H, G, ps, scale, lo, pos,
                                  k_begin + wave * D_KPW, NW * D_KPW, k_end, o, m_run, l_run, pos, &mods);
   } else {
-    const int per = ((k_end - k_begin + D_SHARE - 1) / D_SHARE + NW - 1) / NW * D_SHARE;
+    const int per = ((k_end - k_begin + SHARE - 1) / SHARE + NW - 1) / NW * SHARE;
     const int from = k_begin + wave * per;
     if (FUSED && from >= k_end) {              // (no keys: no prologue either)
 #pragma unroll
@@ -1885,9 +1888,10 @@ __global__ __launch_bounds__(D_BLOCK_MAX_WAVES * WAVE) void attn_decode_block_ke
     float scale, kappai_score_mods mods) {
   extern __shared__ float sh_dec[];
   const int t = blockIdx.x;
-  attn_one_row<MODS>(q, q_stride, k_pool, vt_pool, out, out_stride,
-                     block_tables + (size_t)row_seg[t] * max_blocks, max_blocks, t, row_pos[t],
-                     blockIdx.y, H, G, ps, window, scale, mods, sh_dec, blockDim.x / WAVE);
+  attn_one_row<MODS, false, D_BLOCK_SHARE>(q, q_stride, k_pool, vt_pool, out, out_stride,
+                                           block_tables + (size_t)row_seg[t] * max_blocks, max_blocks, t,
+                                           row_pos[t], blockIdx.y, H, G, ps, window, scale, mods, sh_dec,
+                                           blockDim.x / WAVE);
 }
 
 // attn_decode_block_kernel with the prologue of QkFuse in the waves that have keys (see
@@ -1901,7 +1905,7 @@ __global__ __launch_bounds__(D_BLOCK_MAX_WAVES * WAVE) void attn_decode_block_qk
     float scale, QkFuse qk) {
   extern __shared__ float sh_dec[];
   const int t = blockIdx.x;
-  attn_one_row<false, true>(qkv, row_stride, k_pool, vt_pool, out, out_stride,
+  attn_one_row<false, true, D_BLOCK_SHARE>(qkv, row_stride, k_pool, vt_pool, out, out_stride,
                             block_tables + (size_t)row_seg[t] * max_blocks, max_blocks, t, row_pos[t],
                             blockIdx.y, H, G, ps, window, scale,
                             kappai_score_mods{0.f, nullptr, 0, nullptr, 0}, sh_dec,

@@ -779,9 +779,9 @@ static void launch_tile_cfg(const bf16_t* A, const bf16_t* W, const float* bias,
 #define WAIT_LOADS_AND_LDS(behind) \
   __builtin_amdgcn_s_waitcnt(0x0070 | ((behind) & 15) | ((behind) >> 4 << 14))
 
-// A buffer of `bytes` bytes from p on: loads at offsets outside it read nothing and give zeros, so a
-// loop's last loads need no branch.  (The type is the device compiler's; the host pass sees neither it
-// nor the loads.)
+// A buffer of `bytes` bytes from p on: loads whose lane's and scalar offset together lie outside it read
+// nothing and give zeros, so a loop's last loads need no branch.  (The type is the device compiler's; the host
+// pass sees neither it nor the loads.)
 #if defined(__HIP_DEVICE_COMPILE__)
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t raw_buffer(const void* p, uint32_t bytes) {
   return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), 0, (int)bytes, 0x00020000);
@@ -1106,7 +1106,8 @@ void gemm_bf16_block256_kernel(const bf16_t* __restrict__ A, const bf16_t* __res
 
 // Block products whose W lies in fragment order ([rows / 16][K / 32] pieces of 16 rows x 32 of K, 1 KB
 // each, the lane's 16 bytes at lane = (k % 32) / 8 * 16 + row % 16; see gemm_bf16_skinny_kernel).  Two
-// kernels, four waves each, one a SIMD; rows of A and of W past the end are not read.
+// kernels, four waves each, one a SIMD.  Rows of A and of W past the end are not stored; their offsets lie
+// behind the buffer, or, where 32 bits run over, at some other row of it.
 //
 // The large blocks (256 x 256, 256 x 192) are bound by LDS and by the rate at which a CU takes in tiles
 // (about 60 GB/s from memory, 85 from L2) more than by the matrix cores: with both operands in LDS a tile
@@ -1456,7 +1457,8 @@ static void launch_fragment_block(const bf16_t* A, const bf16_t* Wf, const float
 // blocks of the same kernel (tiles of 64 of K), 5 = the 256x256 kernel with one wave a SIMD, 6 = its
 // 128x128 form (when the sizes fit them, else 3), 8 = the 128x128 form with four LDS buffers, one
 // block a CU, 9 = the one-wave-a-SIMD kernel with blocks of 256 rows x 192 columns, 11 = 192x128, 12 =
-// 256x128 (both only with W in fragment order, else 6)
+// 256x128 (both only with W in fragment order, else 6).  With W in fragment order 6 and 8 are one kernel, one
+// block a CU with four buffers.
 template <typename TO, int EPI>
 static void launch_tile(const bf16_t* A, const bf16_t* W, const float* bias, TO* C, int M,
                         int n_rows_w, int K, int lda, int ldc, int ksplit, int shape,

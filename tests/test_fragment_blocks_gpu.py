@@ -2,6 +2,8 @@
 registers, 256 x 128, 192 x 128 and 128 x 128 with both operands in LDS), at sizes that end inside a block
 and at the shortest runs of K, against the same product over the matrix's rows (bit for bit: every form adds
 16 of K after 16) and against float64."""
+import ctypes
+
 import pytest
 import torch
 
@@ -51,12 +53,45 @@ def test_the_rule_takes_every_form(ops, M, N, K):  # noqa: F811
     assert torch.equal(ops.linear(x, ops.InFragments.of(w)), ops.linear(x, w, force_kernel=ROWS))
 
 
-def test_rows_that_are_not_there_stay_out(ops):  # noqa: F811
-    """NaN in the memory behind the last row of x and between its rows reaches no result."""
-    M, N, K = 200, 256, 256
+# blocks that end behind the last row and the last column, and columns between the rows of the result: nothing is
+# written there, in one plane and in three, and what lies behind x and between its rows reaches no result
+@pytest.mark.parametrize("M,N,K,S", [(200, 272, 384, 1), (129, 144, 768, 3), (385, 400, 256, 1)])
+@pytest.mark.parametrize("form", list(FORMS))
+def test_nothing_is_written_behind_the_result(ops, M, N, K, S, form):  # noqa: F811
+    mark, ldc = -123.5, N + 24
     wide = torch.full((M + 200, K + 8), float("nan"), dtype=BF16, device=DEV)
     wide[:M, :K] = rand((M, K), BF16, 89).to(DEV)
-    w = rand((N, K), BF16, 90).to(DEV)
-    want = ops.linear(wide[:M, :K].contiguous(), w, force_kernel=ROWS)
-    for form in FORMS.values():
-        assert torch.equal(ops.linear(wide[:M, :K], ops.InFragments.of(w), force_kernel=form), want)
+    x, w = wide[:M, :K], rand((N, K), BF16, 90).to(DEV)
+    if S == 1:
+        want = ops.linear(x.contiguous(), w, force_kernel=ROWS, out_dtype=F32)[None]
+    else:
+        want = ops.linear(x.contiguous(), w, partial_sums=True, split_k=S, force_kernel=ROWS)
+    out = torch.full((S * M + 300, ldc), mark, dtype=F32, device=DEV)
+    i, none = ctypes.c_int, ctypes.c_void_p(0)
+    at = lambda t: ctypes.c_void_p(t.data_ptr())  # noqa: E731
+    frag = ops.fragment_order(w)
+    status = ops.library("gemm").kappai_gemm_bf16(
+        at(x), none, at(frag), none, at(out), i(M), i(N), i(K), i(x.stride(0)), i(ldc), i(1), i(FORMS[form]), i(S),
+        i(0), none, i(0), ctypes.c_float(0), none, i(0), none, none, i(0), none,
+        ctypes.c_void_p(torch.cuda.current_stream().cuda_stream))
+    assert status == 0
+    assert torch.equal(out[:S * M, :N].view(S, M, N), want)
+    assert (out[:, N:] == mark).all() and (out[S * M:] == mark).all()
+
+
+@pytest.mark.parametrize("M,F,K", [(129, 144, 256), (385, 208, 384)])
+@pytest.mark.parametrize("form", list(FORMS))
+def test_nothing_is_written_behind_the_gated_result(ops, M, F, K, form):  # noqa: F811
+    mark, ldc = -123.5, F + 24
+    x = rand((M, K), BF16, 84).to(DEV)
+    w = ops.interleave_gate_up(rand((F, K), BF16, 85, 0.2).to(DEV), rand((F, K), BF16, 86, 0.2).to(DEV))
+    out = torch.full((M + 300, ldc), mark, dtype=BF16, device=DEV)
+    i, none = ctypes.c_int, ctypes.c_void_p(0)
+    at = lambda t: ctypes.c_void_p(t.data_ptr())  # noqa: E731
+    frag = ops.fragment_order(w)
+    status = ops.library("gemm").kappai_gemm_bf16_swiglu(
+        at(x), none, at(frag), at(out), i(M), i(F), i(K), i(K), i(ldc), i(FORMS[form]), i(0), none, i(0),
+        ctypes.c_float(0), i(0), ctypes.c_void_p(torch.cuda.current_stream().cuda_stream))
+    assert status == 0
+    assert torch.equal(out[:M, :F], ops.linear_swiglu(x, w, force_kernel=ROWS))
+    assert (out[:, F:] == mark).all() and (out[M:] == mark).all()

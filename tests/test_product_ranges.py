@@ -1,4 +1,5 @@
 """How many ranges of K a product of many rows is cut into, and what its sums are handed on as."""
+import numpy as np
 import pytest
 import torch
 
@@ -46,3 +47,29 @@ def test_float_sums_over_one_range(M, N, K):
 def test_rows_of_w_take_the_ranges_of_their_own_kernels(M, N, K, ranges):
     """A matrix whose rows are no multiple of 16 lies as rows and goes through kernels of its own."""
     assert ops.split_k_for(M, N, K) == ranges and ops.sums_in_f32(M, N, K) == (ranges > 1)
+
+
+# the largest operands that the block products over fragment order take: 2^31 elements less one row
+@pytest.mark.parametrize("rows,stride,K,ranges", [(4095, 524280, 524160, 1), (2097151, 1024, 1024, 2),
+                                                  (131071, 16384, 10752, 3), (200, 8, 128, 1)])
+@pytest.mark.parametrize("block", [256, 192, 128])
+def test_loads_of_the_largest_operands(rows, stride, K, ranges, block):
+    """The 32-bit offsets of A's loads in gemm_bf16_direct and gemm_bf16_staged (row times stride in bytes, what is
+    left of 2^32 where a row past the end runs over) against the bytes that the buffer is given: a row that is there
+    is read where it lies and whole; no load, of whatever row, ends outside the operand."""
+    stride = max(stride, K)
+    assert rows * stride < 2 ** 31
+    K_range = K // ranges
+    size = (rows - 1) * stride * 2 + K_range * 2                # of the buffer, from the range's first column on
+    assert size < 2 ** 32
+    blocks = (rows + block - 1) // block
+    row = np.unique(np.r_[0:block, rows - 1, np.arange((blocks - 1) * block, blocks * block)]).astype(np.int64)
+    chunk = np.arange(0, 128, 16)
+    lane = ((row[:, None] * stride * 2) % 2 ** 32 + chunk).astype(np.int64)
+    for tile in (0, K_range // 64 - 1):
+        end = lane + tile * 128 + 16
+        there = row < rows
+        assert (end[there] <= size).all()
+        assert (lane[there] == row[there][:, None] * stride * 2 + chunk).all()
+        read = lane + tile * 128 < size                         # (what reaches the end is not read)
+        assert (end[read] <= rows * stride * 2).all()

@@ -2073,9 +2073,10 @@ extern "C" int kappai_attn_decode_takes_qk(void) { return D_QK_FUSABLE ? 1 : 0; 
 
 // The most keys with which kappai_attn_decode_qk keeps a row's keys in one block (0: never at this head
 // size).  One kernel in the place of two, but a CU takes in no more than about 50 GB/s of keys.  1 to 4 rows
-// of 8 kv heads, us against split and merge: 40 keys 6.0 / 8.4, 307 keys 7.7 / 8.5, 614 keys 8.8 / 9.7,
-// 1,024 keys 10.8 / 9.0; a captured step knows its contexts as powers of two only, so the line is at 512.  Head
-// size 128 has no registers for prologue and keys at two waves a SIMD (40 keys 9.9 / 10.6, 307 keys 15.2 / 10.6).
+// of 8 kv heads, us against split and merge: 40 keys 5.7 / 7.8, 300 keys 7.5 / 8.2, 500 keys 8.4 to 8.9 / 8.7 to
+// 9.3, and beyond the split wins; a captured step knows its contexts as powers of two only, so the line is at
+// 512.  Head size 128 has no registers for prologue and keys at two waves a SIMD (when it was tried 40 keys
+// 9.9 / 10.6, 307 keys 15.2 / 10.6).
 #define D_QK_BLOCK_MAX_KEYS (HEAD_DIM == 64 ? 512 : 0)
 extern "C" int kappai_attn_decode_block_qk_keys(void) { return D_QK_BLOCK_MAX_KEYS; }
 

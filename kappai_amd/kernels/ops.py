@@ -366,14 +366,14 @@ def cast(x: torch.Tensor, dtype) -> torch.Tensor:
 
 # ---------------------------------------------------------------------------------------
 def fragment_order(weight: torch.Tensor) -> Optional[torch.Tensor]:
-    """A copy of a bfloat16 matrix [N, K] in the order in which the product kernel for 1 to 16
-    rows loads it: pieces of 16 rows x 32 of K, each laid out lane by lane ([N / 16][K / 32]
+    """A copy of a bfloat16 matrix [N, K] in the order in which the product kernels load it:
+    pieces of 16 rows x 32 of K, each laid out lane by lane ([N / 16][K / 32]
     [(k % 32) / 8][row % 16][8 values]), so that one load instruction of a wave reads 1 KB in
     one piece.  None when the shape does not allow it (N a multiple of 16, K of 32).  Every
     product kernel for bfloat16 reads a matrix in this order (the kernels for few rows 10-20 %
-    faster than rows, the block kernels for prompts as fast: a tile's 64 of K of 16 rows are
-    2 KB in two pieces instead of 16 pieces of 128 bytes), so a matrix is kept in this order
-    only: ``InFragments``."""
+    faster than rows; the block kernels for prompts have kernels of their own for it, up to a
+    quarter faster than those for rows), so a matrix is kept in this order only:
+    ``InFragments``."""
     if weight.dtype != BF16 or weight.dim() != 2:
         return None
     N, K = weight.shape

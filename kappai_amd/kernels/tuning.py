@@ -25,7 +25,7 @@ def takes_partial_sums(rows: int, single_rows: bool) -> bool:
 # Every bfloat16 matrix whose shape allows it (rows a multiple of 16, columns of 32) is kept in
 # the order in which the product kernels load it (``ops.fragment_order``), and only so: decode
 # steps stream it 10-20 % faster than rows (a step at batch 8: about a tenth), the block kernels
-# of prompt steps as fast as rows, and the matrices' memory is needed once.  False keeps the
+# of prompt steps are faster over it, and the matrices' memory is needed once.  False keeps the
 # matrices as the checkpoint has them.
 FRAGMENT_ORDER = True
 
@@ -58,10 +58,11 @@ FUSED_QK_MAX_ROWS = 4
 # In a step that holds prompt portions, a single decoded token is one tile for the tiled attention
 # kernel, and the block that gets it walks all its keys alone: 0.9 ms at 32 k keys, however short
 # the portions beside it are.  From this many keys on such rows go to the decode kernel (keys
-# split over blocks) instead: a second kernel and its merge (25-30 us a layer for up to 63 rows)
-# against that walk.  16 requests with 32 k-token prompts: prompt steps 19 -> 14 ms.  With up to
-# 63 rows of at most 2300 keys beside portions of 512 rows the two kernels took 49 us a layer where
-# the tiled kernel alone took 43, hence not from 1024 on.
+# split over blocks) instead: a second kernel and its merge against that walk.  16 requests with 32 k-token
+# prompts: prompt steps 19 -> 14 ms.  Tiled kernel alone / with the decode kernel behind it, us a layer beside a
+# portion of 512, 16 heads of 64 on 8 kv heads: 63 rows of up to 2300 keys 44 / 48, of 4000 68 / 69, of 6000 93 / 94; 8
+# rows of up to 3000 keys 20 / 21, of 4000 26 / 24, of 6000 37 / 29; 32 heads on 8, 63 rows of up to 4000 keys 64 / 76, 8
+# rows of up to 2300 27 / 23, of 4000 45 / 27.
 LONE_ROWS_FROM = 4096
 
 # The minGRU recurrence over a segment: one thread a channel walks the rows in order, which is the

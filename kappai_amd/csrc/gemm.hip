@@ -1554,6 +1554,16 @@ static void launch_tile(const bf16_t* A, const bf16_t* W, const float* bias, TO*
 // lane holds column lane%16, rows 4*(lane/16) + v.
 #define SK_UNROLL 8
 
+// FRAG (W in fragment order): what such a kernel takes beside the stream of W is what stands ahead of its
+// first load and behind its last.  So a wave's loads are buffer loads at one lane offset and scalar steps,
+// without conditions (what a lane must not read lies outside its buffer), the first loads need only
+// arguments that are handed over in registers, and the row scales are summed by the waves that stream.  us
+// of a product alone, W from memory, with conditions and an extra wave for the scales / so: 9216 x 1024
+// gated 1 row 7.1 / 5.7, 16 rows 9.3 / 6.7, behind a folded norm 8.4 / 6.7 and 9.9 / 7.2 (8 rows); 16384 x 2048
+// gated 8 rows 15.0 / 14.1; 6144 x 2048 8 rows 8.4 / 7.1; the conv step of 2048 channels 9.1 / 8.4; 24 rows of
+// 9216 x 1024 gated 9.9 / 7.5.  Into the stream, 8 rows: 1024 x 1024 4.8 / 4.3, 2048 x 8192 13.5 / 11.3, 1 row of
+// 2048 x 10752 13.6 / 11.9.  Not FRAG: W as rows, and offsets of more than 31 bits.
+
 // EPI 1 (SwiGLU, see the tile kernel): a block owns 16 output columns = 16 gate rows and
 // their 16 up rows of the interleaved W; N is the number of output columns.
 // gridDim.y > 1 splits K over blocks as well: block (x, y) writes its partial sums to
@@ -1596,11 +1606,14 @@ struct ResidOut {
   float* ss;             // [gridDim.x][16]: a part holds one value a row, rows beyond M unwritten
 };
 
-template <typename TO, int MT, int NW, int EPI, int NT>
-__global__ __launch_bounds__((NW < 16 ? NW + 1 : NW) * WAVE) void gemm_bf16_skinny_kernel(
-    const bf16_t* __restrict__ A, const bf16_t* __restrict__ W, const float* __restrict__ bias,
-    TO* __restrict__ C, int M, int N, int K, int lda, int ldc, ConvStep cs, RowScale rsc,
-    int w_frag, int a_frag, int c_frag) {
+template <typename TO, int MT, int NW, int EPI, int NT, bool FRAG>
+__global__ __launch_bounds__(NW * WAVE) __attribute__((amdgpu_waves_per_eu(MT == 1 && EPI < 2 ? 4 : 1)))
+void gemm_bf16_skinny_kernel(
+    const bf16_t* __restrict__ A, const bf16_t* __restrict__ W, const float* __restrict__ ss, int M,
+    int N, int K, int kblk, int lda, int a_frag, int ss_count, float ss_eps, TO* __restrict__ C,
+    const float* __restrict__ bias, int ldc, ConvStep cs, int w_frag, int c_frag) {
+  // (the arguments that the first loads need come first: the hardware hands over the first 14 words in
+  // registers, the rest costs a load)
   static_assert(NT == 1 || EPI == 0, "several column tiles a wave: plain products only");
   // c_frag (one row tile, the SwiGLU and conv epilogues): the result is written as 16 rows in
   // fragment order, which is how the product that follows likes to read it (see a_frag)
@@ -1609,9 +1622,9 @@ __global__ __launch_bounds__((NW < 16 ? NW + 1 : NW) * WAVE) void gemm_bf16_skin
   };
   // row groups of W a block streams: gate/up, the three conv gates, or NT column tiles
   constexpr int NG = EPI == 1 ? 2 : (EPI == 2 ? 3 : (EPI == 3 ? 2 : NT));
-  __shared__ float red[NW][NG * MT][WAVE][4];
+  __shared__ f32x4_t red[NW][NG * MT][WAVE];
   const int tid = threadIdx.x;
-  const int lane = tid % WAVE, wave = tid / WAVE;
+  const int lane = tid % WAVE, wave = __builtin_amdgcn_readfirstlane(tid / WAVE);
   const int n0 = blockIdx.x * (EPI == 3 ? 8 : 16 * NT);
   const int col = lane % 16, kg = (lane / 16) * 8;
   // EPI 3: columns 0-7 and 8-15 are the same 8 channels (of two different gates)
@@ -1648,94 +1661,164 @@ __global__ __launch_bounds__((NW < 16 ? NW + 1 : NW) * WAVE) void gemm_bf16_skin
     arow[t] = a_frag ? A + ((size_t)(kg / 8) * 16 + (gm < M ? gm : 0)) * 8
                      : A + (size_t)(gm < M ? gm : 0) * lda + kg;
   }
-  __shared__ float row_ss[16];
-  if (wave == NW) {
-    // The block's extra wave (launched only with a RowScale) adds up the rows' sums of squares
-    // while the others stream W: a lane takes parts lane, lane + 64, ... of all rows at once (a
-    // part is 16 floats, one a row), four parts' loads in flight, then the lanes are summed.
-    float q[16];
+  // The row scales: a part is 16 floats, one a row, so a load takes 16 parts whole, a lane the four rows
+  // lane % 4 of one.  The waves deal the loads among themselves, ask for them behind their first of W and meet in LDS.
+  // (An extra wave that did this while the others streamed left room for one block a CU instead of two.)
+  __shared__ f32x4_t row_ss[NW][4];
+  f32x4_t ss_pre[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+#if defined(__HIP_DEVICE_COMPILE__)
+  const auto ask_for_parts = [&](int c) {
+    // (rows behind M and parts behind the last lie outside the buffer: zeros, nothing read)
+    const __amdgpu_buffer_rsrc_t parts = raw_buffer(ss, ss != nullptr ? (uint32_t)ss_count * 64u : 0u);
+    return __builtin_bit_cast(f32x4_t, __builtin_amdgcn_raw_buffer_load_b128(
+        parts, 4 * (lane % 4) < M ? lane * 16u : 0x7FFFFF00u, c * 1024, 0));
+  };
+  const auto ask_for_first_parts = [&]() {
+    ss_pre[0] = ask_for_parts(wave);
+    ss_pre[1] = ask_for_parts(wave + NW);
+  };
+  const auto add_parts = [&](bool asked) {
+    if (!asked) ask_for_first_parts();
+    asm volatile("" : "+v"(ss_pre[0]), "+v"(ss_pre[1]));       // (added here, not ahead of W)
+    f32x4_t q = ss_pre[0] + ss_pre[1];
+    for (int c = wave + 2 * NW; c * 16 < ss_count; c += NW) q += ask_for_parts(c);
 #pragma unroll
-    for (int i = 0; i < 16; ++i) q[i] = 0.f;
-    for (int p0 = 0; p0 < rsc.n_parts; p0 += 4 * WAVE) {
-      float4 v[4][4];
-#pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        const int p = p0 + u * WAVE + lane;
-        const float4* src = reinterpret_cast<const float4*>(rsc.ss + (size_t)p * 16);
-#pragma unroll
-        for (int j = 0; j < 4; ++j)
-          v[u][j] = (p < rsc.n_parts && 4 * j < M) ? src[j] : make_float4(0.f, 0.f, 0.f, 0.f);
-      }
-#pragma unroll
-      for (int u = 0; u < 4; ++u)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          q[4 * j] += v[u][j].x; q[4 * j + 1] += v[u][j].y;
-          q[4 * j + 2] += v[u][j].z; q[4 * j + 3] += v[u][j].w;
-        }
+    for (int i = 0; i < 4; ++i) {
+      q[i] += dpp_move<0x124>(q[i]);             // row_ror 4
+      q[i] += dpp_move<0x128>(q[i]);             // row_ror 8
+      q[i] += lane_xor16(q[i]);
+      q[i] += lane_xor32(q[i]);
     }
-    // (all 16 without a branch between them, so that the sixteen chains of exchanges overlap)
-#pragma unroll
-    for (int i = 0; i < 16; ++i) q[i] = wave_sum(q[i]);
-    if (lane < 16) {
-      float t = q[0];
-#pragma unroll
-      for (int i = 1; i < 16; ++i) t = lane == i ? q[i] : t;
-      row_ss[lane] = t;
-    }
-  }
-  // The conv step's epilogue (EPI 2, 3) needs the rows' state, the channel's taps and the biases:
-  // asked for now by the lanes that will use them (two round trips, the slot first), so that they
-  // have arrived when the stream of W has gone through.  Up to CONV_PRE taps are held this way;
-  // a longer filter reads the rest when it gets there.
+    if (lane < 4) row_ss[wave][lane] = q;
+  };
+#else
+  const auto ask_for_first_parts = [&]() {};
+  const auto add_parts = [&](bool) {};
+#endif
+  // The conv step's epilogue (EPI 2, 3) needs the rows' state, the channel's taps and the biases, asked for
+  // by the waves that will use them so that they have arrived when W has gone through: the rows' slots
+  // before the first loads of W, the state that they name behind those.  Up to CONV_PRE taps are held this
+  // way; a longer filter reads the rest when it gets there.
   constexpr int CONV_PRE = 4;
+  constexpr bool CONV = EPI == 2 || EPI == 3;
   float st_pre[4][CONV_PRE], tap_pre[CONV_PRE + 1], conv_bias_pre = 0.f;
   float gate_bias_pre[3] = {0.f, 0.f, 0.f};
-  bool fresh_pre[4] = {true, true, true, true};
+  int pos_pre[4], slot_pre[4];
   float* st_ptr[4] = {nullptr, nullptr, nullptr, nullptr};
-  if ((EPI == 2 || EPI == 3) && wave < MT && gn < N && (EPI != 3 || col < 8)) {
-    const int H = cs.L - 1;
+  const bool channel = gn < N && (EPI != 3 || col < 8);
+#if defined(__HIP_DEVICE_COMPILE__)
+  if (CONV && wave < MT) {
+    // (buffer loads: an offset outside the buffer, or a buffer of no bytes, gives 0 and needs no branch)
+    constexpr int OUT = 0x7FFFFF00;
+    const auto word = [](const void* p, uint32_t bytes, int at) {
+      return __builtin_amdgcn_raw_buffer_load_b32(raw_buffer(p, bytes), at, 0, 0);
+    };
+    const auto number = [&](const void* p, uint32_t bytes, int at) {
+      return __builtin_bit_cast(float, word(p, bytes, at));
+    };
 #pragma unroll
     for (int v = 0; v < 4; ++v) {
       const int gm = wave * 16 + 4 * (lane / 16) + v;
-      if (gm < M) {
-        fresh_pre[v] = cs.seg_pos0[gm] == 0;
-        st_ptr[v] = cs.state + ((size_t)cs.seg_slot[gm] * N + gn) * H;
-      }
+      slot_pre[v] = (int)word(cs.seg_slot, M * 4u, channel ? gm * 4 : OUT);
+      pos_pre[v] = (int)word(cs.seg_pos0, M * 4u, channel ? gm * 4 : OUT);
     }
 #pragma unroll
-    for (int v = 0; v < 4; ++v)
+    for (int k = 0; k <= CONV_PRE; ++k)
+      tap_pre[k] = number(cs.taps, (uint32_t)N * cs.L * 4u, channel && k < cs.L ? (gn * cs.L + k) * 4 : OUT);
+    conv_bias_pre = number(cs.conv_bias, cs.conv_bias ? N * 4u : 0u, channel ? gn * 4 : OUT);
 #pragma unroll
-      for (int k = 0; k < CONV_PRE; ++k)
-        st_pre[v][k] = (st_ptr[v] != nullptr && !fresh_pre[v] && k < H) ? st_ptr[v][k] : 0.f;
-#pragma unroll
-    for (int k = 0; k <= CONV_PRE; ++k) tap_pre[k] = k <= H ? cs.taps[(size_t)gn * cs.L + k] : 0.f;
-    if (cs.conv_bias) conv_bias_pre = cs.conv_bias[gn];
-    if (bias) {
-      gate_bias_pre[0] = bias[gn];
-      gate_bias_pre[1] = bias[N + gn];
-      gate_bias_pre[2] = bias[2 * N + gn];
-    }
+    for (int g = 0; g < 3; ++g)
+      gate_bias_pre[g] = number(bias, bias ? N * 12u : 0u, channel ? (g * N + gn) * 4 : OUT);
   }
-  const int kblk = ((K + 32 * (int)gridDim.y - 1) / (32 * (int)gridDim.y)) * 32;   // K a block
-  const int kb0 = blockIdx.y * kblk, kb1 = min(K, kb0 + kblk);
+#endif
+  const auto ask_for_state = [&]() {
+    const int H = cs.L - 1;
+#pragma unroll
+    for (int v = 0; v < 4; ++v) st_ptr[v] = cs.state + ((size_t)slot_pre[v] * N + (channel ? gn : 0)) * H;
+#pragma unroll
+    for (int k = 0; k < CONV_PRE; ++k)
+#pragma unroll
+      for (int v = 0; v < 4; ++v) st_pre[v][k] = st_ptr[v][min(k, H - 1)];   // (H >= 1)
+  };
+  const int kb0 = blockIdx.y * kblk, kb1 = min(K, kb0 + kblk);     // the block's K
   const int kper = ((kb1 - kb0 + 32 * NW - 1) / (32 * NW)) * 32;
   const int k0 = kb0 + wave * kper;
   const int k1 = min(kb1, k0 + kper);
   C += (size_t)blockIdx.y * M * ldc;
   // loads in flight a lane: U * (NG + MT)
   constexpr int U = (NG + MT) <= 3 ? SK_UNROLL : ((NG + MT) <= 6 ? 4 : 2);
-  auto products = [&](const u32x4_t (&wv)[U][NG], const u32x4_t (&av)[U][MT]) {
+  if constexpr (FRAG) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    // One buffer a row group of W, from the wave's first piece on and as long as its pieces; a lane's
+    // offset, the same for every step but for a constant.  Lanes without a row of A (or, with EPI 3, of W)
+    // stand behind every buffer's end and read nothing.
+    constexpr uint32_t OUT = 0x7FFFFF00u;
+    const int steps = max(k1 - k0, 0) / 32;
+    __amdgpu_buffer_rsrc_t wbuf[NG], abuf;
+    uint32_t woff[NG], aoff[MT];
+    const size_t group = (size_t)16 * K;                 // of 16 rows, in values
 #pragma unroll
-    for (int u = 0; u < U; ++u)
+    for (int r = 0; r < NG; ++r) {
+      const int first = EPI == 0 ? (int)blockIdx.x * NT + r
+                      : EPI == 1 ? (int)blockIdx.x * 2 + r
+                      : EPI == 2 ? (int)blockIdx.x + r * (N / 16) : n0 / 16 + 2 * r * (N / 16);
+      const bool there = EPI != 0 || first * 16 < N;
+      // (EPI 3: the C gate's rows lie N rows behind the B gate's)
+      const uint32_t bytes = there ? (uint32_t)steps * 1024u + (EPI == 3 && r == 0 ? (uint32_t)N * K * 2u : 0u) : 0u;
+      wbuf[r] = raw_buffer(W + (size_t)first * group + (size_t)max(k0, 0) * 16, bytes);
+      woff[r] = (uint32_t)lane * 16u;
+      if (EPI == 3) {
+        woff[r] = (uint32_t)((lane / 16) * 16 + n0 % 16 + col % 8) * 16u;
+        if (col >= 8) woff[r] = r == 0 ? woff[r] + (uint32_t)N * K * 2u : OUT;
+      }
+    }
+    abuf = raw_buffer(A + (size_t)k0 * (a_frag ? 16 : 1), OUT);
+    const uint32_t astep = a_frag ? 1024u : 64u;
 #pragma unroll
-      for (int r = 0; r < NG; ++r)
+    for (int t = 0; t < MT; ++t) {
+      const int gm = t * 16 + col;
+      aoff[t] = gm >= M ? OUT : a_frag ? (uint32_t)lane * 16u : (uint32_t)gm * lda * 2u + kg * 2u;
+    }
+    const auto run = [&](auto count, int from) {
+      constexpr int S = decltype(count)::value;
+      u32x4_t wv[S][NG], av[S][MT];
+#pragma unroll
+      for (int u = 0; u < S; ++u) {
+#pragma unroll
+        for (int r = 0; r < NG; ++r)
+          wv[u][r] = __builtin_amdgcn_raw_buffer_load_b128(wbuf[r], woff[r], (from + u) * 1024, 0);
 #pragma unroll
         for (int t = 0; t < MT; ++t)
-          acc[r * MT + t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-              as_bf16x8(av[u][t]), as_bf16x8(wv[u][r]), acc[r * MT + t], 0, 0, 0);
-  };
-  {
+          av[u][t] = __builtin_amdgcn_raw_buffer_load_b128(abuf, aoff[t], (from + u) * astep, 0);
+      }
+      __builtin_amdgcn_sched_barrier(0);                 // (left alone, loads sink to their use)
+      if (CONV && from == 0 && wave < MT) ask_for_state();
+      if (MT == 1 && from == 0 && ss != nullptr) ask_for_first_parts();
+#pragma unroll
+      for (int u = 0; u < S; ++u)
+#pragma unroll
+        for (int r = 0; r < NG; ++r)
+#pragma unroll
+          for (int t = 0; t < MT; ++t)
+            acc[r * MT + t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                as_bf16x8(av[u][t]), as_bf16x8(wv[u][r]), acc[r * MT + t], 0, 0, 0);
+    };
+    int s = 0;
+    if (CONV && steps == 0 && wave < MT) ask_for_state();        // (a wave of the epilogue without pieces)
+    for (; s + U <= steps; s += U) run(IntC<U>{}, s);
+    switch (steps - s) {
+      case 1: run(IntC<1>{}, s); break;
+      case 2: if constexpr (U > 2) run(IntC<2>{}, s); break;
+      case 3: if constexpr (U > 2) run(IntC<3>{}, s); break;
+      case 4: if constexpr (U > 4) run(IntC<4>{}, s); break;
+      case 5: if constexpr (U > 4) run(IntC<5>{}, s); break;
+      case 6: if constexpr (U > 4) run(IntC<6>{}, s); break;
+      case 7: if constexpr (U > 4) run(IntC<7>{}, s); break;
+      default: break;
+    }
+#endif
+  } else {
+    if (CONV && wave < MT) ask_for_state();
     for (int k = k0; k < k1; k += 32 * U) {
       // the loads of W and of A alternate, in the order of K
       u32x4_t wv[U][NG], av[U][MT];
@@ -1752,20 +1835,36 @@ __global__ __launch_bounds__((NW < 16 ? NW + 1 : NW) * WAVE) void gemm_bf16_skin
         for (int t = 0; t < MT; ++t)
           av[u][t] = (kin && t * 16 + col < M) ? load16(arow[t] + (size_t)gk * (a_frag ? 16 : 1)) : zero;
       }
-      products(wv, av);
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+#pragma unroll
+        for (int r = 0; r < NG; ++r)
+#pragma unroll
+          for (int t = 0; t < MT; ++t)
+            acc[r * MT + t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                as_bf16x8(av[u][t]), as_bf16x8(wv[u][r]), acc[r * MT + t], 0, 0, 0);
     }
   }
-  if (wave < NW) {
+  if (MT == 1 && ss != nullptr) add_parts(FRAG && k0 < k1);
 #pragma unroll
-    for (int t = 0; t < NG * MT; ++t)
-#pragma unroll
-      for (int v = 0; v < 4; ++v) red[wave][t][lane][v] = acc[t][v];
-  }
+  for (int t = 0; t < NG * MT; ++t) red[wave][t][lane] = acc[t];
   __syncthreads();
-  if (wave >= NW) return;
-  auto scale_of = [&](int gm) {
-    return rsc.ss != nullptr ? 1.0f / sqrtf(row_ss[gm] / (float)K + rsc.eps) : 1.0f;
+  // a tile's sums over the waves, in a fixed order
+  auto whole = [&](int tile, int from) {
+    f32x4_t sum = red[0][tile][from];
+#pragma unroll(NW < 16 ? NW : 4)
+    for (int w = 1; w < NW; ++w) sum += red[w][tile][from];
+    return sum;
   };
+  // of the lane's rows 4 (lane / 16) ..
+  f32x4_t scale = {1.f, 1.f, 1.f, 1.f};
+  if (MT == 1 && wave < NG && ss != nullptr) {
+    f32x4_t q = row_ss[0][lane / 16];
+#pragma unroll
+    for (int w = 1; w < NW; ++w) q += row_ss[w][lane / 16];
+#pragma unroll
+    for (int v = 0; v < 4; ++v) scale[v] = 1.0f / sqrtf(q[v] / (float)K + ss_eps);
+  }
   // the first MT waves each sum one row tile over the NW partial results, in a fixed order
   if (EPI == 0 && NT > 1) {
     // waves take the NT * MT tiles in turn
@@ -1774,64 +1873,55 @@ __global__ __launch_bounds__((NW < 16 ? NW + 1 : NW) * WAVE) void gemm_bf16_skin
       const int gnr = gn + r * 16;
       if (gnr >= N) continue;
       const float bv = (bias && blockIdx.y == 0) ? bias[gnr] : 0.f;
+      const f32x4_t sum = whole(tile, lane);
 #pragma unroll
       for (int v = 0; v < 4; ++v) {
         const int gm = t * 16 + 4 * (lane / 16) + v;
         if (gm >= M) continue;
-        float sum = red[0][tile][lane][v];
-#pragma unroll
-        for (int w = 1; w < NW; ++w) sum += red[w][tile][lane][v];
-        store_out(C + (size_t)gm * ldc + gnr, sum * scale_of(gm) + bv);
+        store_out(C + (size_t)gm * ldc + gnr, sum[v] * scale[v] + bv);
       }
     }
-  } else if (wave < MT && gn < N && (EPI != 3 || col < 8)) {
+  } else if (wave < MT && channel) {
     const int t = wave;
     const float bv = (EPI != 1 && bias && blockIdx.y == 0) ? bias[gn] : 0.f;
+    const f32x4_t sums = whole(t, lane);
+    // the up row; or where the other two gates of this channel lie: EPI 2 in row groups 1 and 2 of this
+    // lane, EPI 3 the C gate 8 columns further in group 0 and the x gate in group 1
+    f32x4_t second = sums, third = sums;
+    if (EPI == 1 || EPI == 2) second = whole(MT + t, lane);
+    if (EPI == 3) second = whole(t, lane + 8);
+    if (EPI == 2) third = whole(2 * MT + t, lane);
+    if (EPI == 3) third = whole(MT + t, lane);
 #pragma unroll
     for (int v = 0; v < 4; ++v) {
       const int gm = t * 16 + 4 * (lane / 16) + v;
       if (gm < M) {
-        const float rs = scale_of(gm);
-        float sum = red[0][t][lane][v];
-#pragma unroll
-        for (int w = 1; w < NW; ++w) sum += red[w][t][lane][v];
-        sum *= rs;
+        const float rs = scale[v];
+        const float sum = sums[v] * rs;
         if (EPI == 1) {
-          float up = red[0][MT + t][lane][v];
-#pragma unroll
-          for (int w = 1; w < NW; ++w) up += red[w][MT + t][lane][v];
-          store_out(C + out_at(gm, gn), gated_f(sum, up * rs, bias, (int)blockIdx.x * 32 + col));
+          store_out(C + out_at(gm, gn), gated_f(sum, second[v] * rs, bias, (int)blockIdx.x * 32 + col));
         } else if (EPI == 2 || EPI == 3) {
-          // where the other two gates of this channel lie: EPI 2 in row groups 1 and 2 of this
-          // lane, EPI 3 the C gate 8 columns further in group 0 and the x gate in group 1
-          const int cg_t = EPI == 2 ? MT + t : t, cg_lane = EPI == 2 ? lane : lane + 8;
-          const int xg_t = EPI == 2 ? 2 * MT + t : MT + t;
-          float cg = red[0][cg_t][cg_lane][v], xg = red[0][xg_t][lane][v];
-#pragma unroll
-          for (int w = 1; w < NW; ++w) {
-            cg += red[w][cg_t][cg_lane][v];
-            xg += red[w][xg_t][lane][v];
-          }
-          cg *= rs;
-          xg *= rs;
+          float cg = second[v] * rs, xg = third[v] * rs;
           const float bg = sum + gate_bias_pre[0];
           cg += gate_bias_pre[1];
           xg += gate_bias_pre[2];
           // the three gates are rounded as the unfused path stores them
           const float bx = to_f32(f32_to_bf16(bg)) * to_f32(f32_to_bf16(xg));
           const int H = cs.L - 1;
-          const bool fresh = fresh_pre[v];
+          int pos = pos_pre[v];
+          asm volatile("" : "+v"(pos));          // (compared here, not where it was asked for)
+          const bool fresh = pos == 0;
           float* st = st_ptr[v];
           const float* wc = cs.taps + (size_t)gn * cs.L;
           float s = conv_bias_pre;
           if (H <= CONV_PRE) {
             // everything is in registers already
-            float prev = st_pre[v][0];
+            float prev = fresh ? 0.f : st_pre[v][0];
 #pragma unroll
             for (int k = 0; k < CONV_PRE; ++k) {
               if (k < H) {
                 s += tap_pre[k] * prev;
-                const float next = (k + 1 < H) ? st_pre[v][k + 1 < CONV_PRE ? k + 1 : 0] : bx;
+                const float next = (k + 1 < H) ? (fresh ? 0.f : st_pre[v][k + 1 < CONV_PRE ? k + 1 : 0]) : bx;
                 st[k] = next;
                 prev = next;
               }
@@ -1866,29 +1956,38 @@ __global__ __launch_bounds__((NW < 16 ? NW + 1 : NW) * WAVE) void gemm_bf16_skin
 // two halves meet the one fragment of W in two matrix instructions, whose valid halves are added
 // at the end.  Twice as many blocks stream W as with 16 columns a block, and K needs no split
 // over blocks, so the residual sum can be made here, in a fixed order.
-template <int NW>
+template <int NW, bool FRAG>
 __global__ __launch_bounds__(NW * WAVE) void gemm_bf16_into_resid_kernel(
-    const bf16_t* __restrict__ A, const bf16_t* __restrict__ W, const float* __restrict__ bias,
-    int M, int N, int K, int lda, ResidOut ro, int w_frag, int a_frag) {
-  __shared__ float red[NW][2][WAVE][4];
+    const bf16_t* __restrict__ A, const bf16_t* __restrict__ W, float* __restrict__ resid, int M, int N,
+    int K, int lda, int a_frag, int ldr, const float* __restrict__ norm_w, const float* __restrict__ bias,
+    bf16_t* __restrict__ rows, float* __restrict__ ss, int rows_frag, int w_frag) {
+  __shared__ f32x4_t red[NW][2][WAVE];
   const int tid = threadIdx.x;
-  const int lane = tid % WAVE, wave = tid / WAVE;
+  const int lane = tid % WAVE, wave = __builtin_amdgcn_readfirstlane(tid / WAVE);
   const int col = lane % 16, kg = (lane / 16) * 8;
   const int half = col / 8;
   const int gn = blockIdx.x * 8 + col % 8;               // the lane's row of W
   const int khalf = ((K / 2 + 31) / 32) * 32;            // the second half starts here
   const u32x4_t zero = {0u, 0u, 0u, 0u};
-  // what the epilogue needs, asked for before the stream of W
+  // What the epilogue needs, asked for before the stream of W: offsets outside the buffers for lanes that
+  // need nothing, since of loads in branches the compiler waits for the first before it asks for the next.
   float resid_in[4] = {0.f, 0.f, 0.f, 0.f};
   float norm_w_in = 0.f;
-  if (wave == 0 && half == 0 && gn < N) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  if (wave == 0) {
+    const bool mine = half == 0 && gn < N;
+    const __amdgpu_buffer_rsrc_t res = raw_buffer(resid, 0x7FFFFF00u);
+    const __amdgpu_buffer_rsrc_t nw = raw_buffer(norm_w, rows != nullptr ? (uint32_t)N * 4u : 0u);
 #pragma unroll
     for (int v = 0; v < 4; ++v) {
       const int gm = 4 * (lane / 16) + v;
-      if (gm < M) resid_in[v] = ro.resid[(size_t)gm * ro.ldr + gn];
+      resid_in[v] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(
+          res, mine && gm < M ? (gm * ldr + gn) * 4 : 0x7FFFFF00, 0, 0));
     }
-    if (ro.rows != nullptr) norm_w_in = ro.norm_w[gn];
+    norm_w_in = __builtin_bit_cast(
+        float, __builtin_amdgcn_raw_buffer_load_b32(nw, mine ? gn * 4 : 0x7FFFFF00, 0, 0));
   }
+#endif
   const size_t wr = gn < N ? gn : 0;
   const int kmul = w_frag ? 16 : 1;                      // see the kernel above for the two orders
   const bf16_t* wrow = (w_frag ? W + (wr / 16) * 16 * K + ((size_t)(kg / 8) * 16 + wr % 16) * 8
@@ -1900,6 +1999,48 @@ __global__ __launch_bounds__(NW * WAVE) void gemm_bf16_into_resid_kernel(
   const int k0 = wave * kper, k1 = min(khalf, k0 + kper);
   f32x4_t acc0 = {0.f, 0.f, 0.f, 0.f}, acc1 = {0.f, 0.f, 0.f, 0.f};
   constexpr int U = SK_UNROLL;
+  if constexpr (FRAG) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    // as in the kernel above; K is a multiple of 64, so that both halves have as many steps
+    constexpr uint32_t OUT = 0x7FFFFF00u;
+    const int steps = max(k1 - k0, 0) / 32;
+    const __amdgpu_buffer_rsrc_t wbuf =
+        raw_buffer(W + ((size_t)(blockIdx.x / 2) * K + k0) * 16, (uint32_t)(khalf + 32 * steps) * 32u);
+    const uint32_t woff =
+        ((lane / 16) * 16 + blockIdx.x % 2 * 8 + col % 8) * 16u + (half ? (uint32_t)khalf * 32u : 0u);
+    const __amdgpu_buffer_rsrc_t abuf = raw_buffer(A + (size_t)k0 * (a_frag ? 16 : 1), OUT);
+    const uint32_t astep = a_frag ? 1024u : 64u, second = (uint32_t)khalf * (a_frag ? 32u : 2u);
+    const uint32_t aoff = col >= M ? OUT : a_frag ? (uint32_t)lane * 16u : (uint32_t)col * lda * 2u + kg * 2u;
+    const auto run = [&](auto count, int from) {
+      constexpr int S = decltype(count)::value;
+      u32x4_t wv[S], a0[S], a1[S];
+#pragma unroll
+      for (int u = 0; u < S; ++u) {
+        wv[u] = __builtin_amdgcn_raw_buffer_load_b128(wbuf, woff, (from + u) * 1024, 0);
+        a0[u] = __builtin_amdgcn_raw_buffer_load_b128(abuf, aoff, (from + u) * astep, 0);
+        a1[u] = __builtin_amdgcn_raw_buffer_load_b128(abuf, aoff, (from + u) * astep + second, 0);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int u = 0; u < S; ++u) {
+        acc0 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(a0[u]), as_bf16x8(wv[u]), acc0, 0, 0, 0);
+        acc1 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(a1[u]), as_bf16x8(wv[u]), acc1, 0, 0, 0);
+      }
+    };
+    int s = 0;
+    for (; s + U <= steps; s += U) run(IntC<U>{}, s);
+    switch (steps - s) {
+      case 1: run(IntC<1>{}, s); break;
+      case 2: run(IntC<2>{}, s); break;
+      case 3: run(IntC<3>{}, s); break;
+      case 4: run(IntC<4>{}, s); break;
+      case 5: run(IntC<5>{}, s); break;
+      case 6: run(IntC<6>{}, s); break;
+      case 7: run(IntC<7>{}, s); break;
+      default: break;
+    }
+#endif
+  } else
   for (int k = k0; k < k1; k += 32 * U) {
     u32x4_t wv[U], a0[U], a1[U];
 #pragma unroll
@@ -1917,13 +2058,16 @@ __global__ __launch_bounds__(NW * WAVE) void gemm_bf16_into_resid_kernel(
       acc1 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(a1[u]), as_bf16x8(wv[u]), acc1, 0, 0, 0);
     }
   }
-#pragma unroll
-  for (int v = 0; v < 4; ++v) {
-    red[wave][0][lane][v] = acc0[v];
-    red[wave][1][lane][v] = acc1[v];
-  }
+  red[wave][0][lane] = acc0;
+  red[wave][1][lane] = acc1;
   __syncthreads();
   if (wave != 0) return;
+  f32x4_t lo = red[0][0][lane], hi = red[0][1][lane ^ 8];
+#pragma unroll 4
+  for (int w = 1; w < NW; ++w) {
+    lo += red[w][0][lane];
+    hi += red[w][1][lane ^ 8];
+  }
   // columns 0-7: the first half's sums of this lane and the second half's of the lane 8 further
   const bool mine = half == 0 && gn < N;
   const float bv = (bias && mine) ? bias[gn] : 0.f;
@@ -1932,27 +2076,21 @@ __global__ __launch_bounds__(NW * WAVE) void gemm_bf16_into_resid_kernel(
     const int gm = 4 * (lane / 16) + v;
     float q = 0.f;
     if (mine && gm < M) {
-      float lo = red[0][0][lane][v], hi = red[0][1][lane + 8][v];
-#pragma unroll
-      for (int w = 1; w < NW; ++w) {
-        lo += red[w][0][lane][v];
-        hi += red[w][1][lane + 8][v];
-      }
-      const float x = resid_in[v] + ((lo + hi) + bv);
-      ro.resid[(size_t)gm * ro.ldr + gn] = x;
-      if (ro.rows != nullptr) {
-        const size_t at = ro.rows_frag ? ((size_t)(gn / 8) * 16 + gm) * 8 + gn % 8
+      const float x = resid_in[v] + ((lo[v] + hi[v]) + bv);
+      resid[(size_t)gm * ldr + gn] = x;
+      if (rows != nullptr) {
+        const size_t at = rows_frag ? ((size_t)(gn / 8) * 16 + gm) * 8 + gn % 8
                                        : (size_t)gm * N + gn;
-        ro.rows[at] = f32_to_bf16(x * norm_w_in);
+        rows[at] = f32_to_bf16(x * norm_w_in);
       }
       q = x * x;
     }
-    if (ro.rows != nullptr) {
+    if (rows != nullptr) {
       // the sum of squares over the block's 8 columns, row by row
       q += __shfl_xor(q, 1, WAVE);
       q += __shfl_xor(q, 2, WAVE);
       q += __shfl_xor(q, 4, WAVE);
-      if (col == 0 && gm < M) ro.ss[(size_t)blockIdx.x * 16 + gm] = q;
+      if (col == 0 && gm < M) ss[(size_t)blockIdx.x * 16 + gm] = q;
     }
   }
 }
@@ -1963,16 +2101,25 @@ static void launch_into_resid(const bf16_t* A, const bf16_t* W, const float* bia
   const int w_frag = Wf != nullptr;
   if (Wf) W = Wf;
   const dim3 grid((N + 7) / 8);
+  // (both halves of K whole pieces and offsets of 31 bits: the loads without conditions)
+  const bool pieces = w_frag && K % 64 == 0 && ((size_t)M * lda + K) * 2 < 0x7FFFFF00u &&
+                      (size_t)K * 32 < 0x7FFFFF00u;
+#define INTO_RESID(NW)                                                                                 \
+  do {                                                                                                 \
+    if (pieces)                                                                                        \
+      hipLaunchKernelGGL((gemm_bf16_into_resid_kernel<NW, true>), grid, dim3(NW * WAVE), 0, stream, A, \
+                         W, ro.resid, M, N, K, lda, a_frag, ro.ldr, ro.norm_w, bias, ro.rows, ro.ss,   \
+                         ro.rows_frag, w_frag);                                                        \
+    else                                                                                               \
+      hipLaunchKernelGGL((gemm_bf16_into_resid_kernel<NW, false>), grid, dim3(NW * WAVE), 0, stream,   \
+                         A, W, ro.resid, M, N, K, lda, a_frag, ro.ldr, ro.norm_w, bias, ro.rows,       \
+                         ro.ss, ro.rows_frag, w_frag);                                                 \
+  } while (0)
   // K a wave: 128 or more where K allows it
-  if (K >= 4096)
-    hipLaunchKernelGGL((gemm_bf16_into_resid_kernel<16>), grid, dim3(16 * WAVE), 0, stream, A, W,
-                       bias, M, N, K, lda, ro, w_frag, a_frag);
-  else if (K >= 1024)
-    hipLaunchKernelGGL((gemm_bf16_into_resid_kernel<8>), grid, dim3(8 * WAVE), 0, stream, A, W,
-                       bias, M, N, K, lda, ro, w_frag, a_frag);
-  else
-    hipLaunchKernelGGL((gemm_bf16_into_resid_kernel<4>), grid, dim3(4 * WAVE), 0, stream, A, W,
-                       bias, M, N, K, lda, ro, w_frag, a_frag);
+  if (K >= 4096) INTO_RESID(16);
+  else if (K >= 1024) INTO_RESID(8);
+  else INTO_RESID(4);
+#undef INTO_RESID
 }
 
 struct Fuse {
@@ -1987,14 +2134,20 @@ static void launch_skinny(const bf16_t* A, const bf16_t* W, const float* bias, T
                           const Fuse& fuse = Fuse{}, const bf16_t* Wf = nullptr, int a_frag = 0) {
   // Wf: the copy of W in fragment order (see the kernel), or null
   const int w_frag = Wf != nullptr;
-  if (Wf) W = Wf;
   const dim3 grid(EPI == 3 ? (N + 7) / 8 : (N + 16 * NT - 1) / (16 * NT), ksplit);
-  // one wave more when there are row scales to make (launch_skinny_mt keeps NW below 16 then)
-  const int waves = fuse.rsc.ss != nullptr ? NW + 1 : NW;
-  if (waves * WAVE > 1024) return;
-  hipLaunchKernelGGL((gemm_bf16_skinny_kernel<TO, MT, NW, EPI, NT>), grid, dim3(waves * WAVE), 0,
-                     stream, A, W, bias, C, M, N, K, lda, ldc, cs, fuse.rsc, w_frag, a_frag,
-                     (MT == 1 && EPI != 0) ? fuse.c_frag : 0);
+  const int c_frag = (MT == 1 && EPI != 0) ? fuse.c_frag : 0;
+  const int kblk = (K + 32 * ksplit - 1) / (32 * ksplit) * 32;
+  // (fragment order and offsets of 31 bits within A, a group of W and the gates of EPI 3: the loads
+  // without conditions)
+  const bool pieces = Wf != nullptr && ((size_t)M * lda + K) * 2 < 0x7FFFFF00u && (size_t)K * 32 < 0x7FFFFF00u &&
+                      (EPI != 3 || (size_t)(N + 16) * K * 2 < 0x7FFFFF00u);
+#define SKINNY(FRAG)                                                                                   \
+  hipLaunchKernelGGL((gemm_bf16_skinny_kernel<TO, MT, NW, EPI, NT, FRAG>), grid, dim3(NW * WAVE), 0,    \
+                     stream, A, Wf ? Wf : W, fuse.rsc.ss, M, N, K, kblk, lda, a_frag, fuse.rsc.n_parts, \
+                     fuse.rsc.eps, C, bias, ldc, cs, w_frag, c_frag)
+  if (pieces) SKINNY(true);
+  else SKINNY(false);
+#undef SKINNY
 }
 
 // more waves a block when there are few blocks, so that about 2048 waves or more stream W
@@ -2026,13 +2179,12 @@ static void launch_skinny_mt(const bf16_t* A, const bf16_t* W, const float* bias
   const int blocks = (EPI == 3 ? (N + 7) / 8 : (N + 15) / 16) * ksplit;
   const int kb = K / ksplit;                              // K a block
   constexpr int NG = EPI == 1 ? 2 : (EPI == 2 ? 3 : (EPI == 3 ? 2 : 1));
-  constexpr int MAXW = 48 / (MT * NG);                    // 1 KB of LDS a wave, group and row tile
+  // 1 KB of LDS a wave, group and row tile; the conv step's 16 waves would have no room for what its
+  // epilogue waits with
+  constexpr int MAXW = EPI >= 2 && MT == 1 ? 8 : 48 / (MT * NG);
   if (blocks * 4 >= 2048 || kb <= 512 || MAXW < 8)
     launch_skinny<TO, MT, 4, EPI>(A, W, bias, C, M, N, K, lda, ldc, ksplit, cs, stream, fuse, Wf, a_frag);
   else if (blocks * 8 >= 2048 || kb <= 1024 || MAXW < 16)
-    launch_skinny<TO, MT, (MAXW >= 8 ? 8 : 4), EPI>(A, W, bias, C, M, N, K, lda, ldc, ksplit, cs,
-                                                    stream, fuse, Wf, a_frag);
-  else if (fuse.rsc.ss != nullptr)      // (the block needs room for the wave that makes the scales)
     launch_skinny<TO, MT, (MAXW >= 8 ? 8 : 4), EPI>(A, W, bias, C, M, N, K, lda, ldc, ksplit, cs,
                                                     stream, fuse, Wf, a_frag);
   else

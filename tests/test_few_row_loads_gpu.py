@@ -1,0 +1,126 @@
+"""The products of 1 to 24 rows over a matrix in fragment order, whose loads carry no conditions: K that
+leaves waves with few pieces or none, column groups behind the last, rows behind M, the sums of squares of
+narrow and wide norms, and memory full of NaN on every side of what they may read.  Results against float64
+within the bound of a float sum of K products, gamma_K = K 2^-24 of the sum of magnitudes."""
+import pytest
+import torch
+
+from kappai_amd.kernels import ops
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+BF16 = torch.bfloat16
+NAN = float("nan")
+
+
+def _gen(*key):
+    return torch.Generator(device=DEV).manual_seed(sum((i + 1) * 7919 ** i * int(k) for i, k in enumerate(key)) % (1 << 31))
+
+
+def _rows(M, K, g):
+    """[M, K] rows with NaN before, behind and between them."""
+    big = torch.full((M + 2, K + 24), NAN, device=DEV, dtype=BF16)
+    big[1:M + 1, 8:K + 8] = torch.randn(M, K, generator=g, device=DEV).to(BF16)
+    return big[1:M + 1, 8:K + 8]
+
+
+def _matrix(N, K, g):
+    """A matrix in fragment order between matrices of NaN, and its rows."""
+    w = torch.randn(N, K, generator=g, device=DEV).to(BF16)
+    big = torch.full((N + 32, K), NAN, device=DEV, dtype=BF16)
+    big[16:16 + N] = ops.fragment_order(w)
+    return ops.InFragments(big[16:16 + N]), w
+
+
+def _sums(x, w):
+    """In float64 (on the CPU, where a product of a view is any product): the sums and their bound."""
+    a, b = x.double().cpu(), w.double().cpu()
+    return (a @ b.T).to(DEV), (a.abs() @ b.abs().T).to(DEV) * x.shape[1] * 2.0 ** -24
+
+
+@pytest.mark.parametrize("M", [1, 4, 5, 16, 17, 24])
+@pytest.mark.parametrize("K,N", [(32, 16), (64, 80), (96, 48), (288, 1040), (1056, 144), (2304, 64), (4608, 32)])
+def test_plain(M, K, N):
+    g = _gen(M, K, N)
+    x = _rows(M, K, g)
+    W, w = _matrix(N, K, g)
+    want, bound = _sums(x, w)
+    got = ops.linear(x, W, out_dtype=torch.float32)
+    assert ((got.double() - want).abs() <= bound).all().item()
+    parts = ops.linear(x, W, partial_sums=True, split_k=3 if K >= 288 else 1)
+    if parts.dim() == 3:
+        assert ((parts.double().sum(0) - want).abs() <= bound).all().item()
+
+
+@pytest.mark.parametrize("M", [1, 3, 8, 16])
+@pytest.mark.parametrize("K,N", [(32, 32), (64, 64), (96, 96), (1088, 96), (2304, 160), (4608, 64), (4640, 64)])
+def test_into_the_stream(M, K, N):
+    """(K = 4640: halves that are no whole pieces)"""
+    g = _gen(M, K, N, 1)
+    x = _rows(M, K, g)
+    W, w = _matrix(N, K, g)
+    want, bound = _sums(x, w)
+    resid = torch.randn(M, N, generator=g, device=DEV)
+    before = resid.double()
+    norm = torch.rand(N, generator=g, device=DEV) + 0.5
+    got = ops.linear(x, W, add_into=ops.AddInto(resid, norm, 1e-5))
+    assert isinstance(got, ops.ScaledRows)
+    assert ((resid.double() - before - want).abs() <= bound + resid.double().abs() * 2.0 ** -24).all().item()
+    squares = got.ss[:, :M].double().sum(0)
+    exact = (resid.double() ** 2).sum(1)
+    assert ((squares - exact).abs() <= exact * N * 2.0 ** -24).all().item()
+
+
+@pytest.mark.parametrize("M", [1, 5, 12, 16])
+@pytest.mark.parametrize("D", [64, 1024, 4160])
+def test_rows_still_to_be_scaled(M, D):
+    """The product behind a folded norm: D / 8 parts of the sums of squares, one load of a wave or several."""
+    g = _gen(M, D, 2)
+    W0, _ = _matrix(D, 64, g)
+    resid = torch.randn(M, D, generator=g, device=DEV)
+    norm = torch.rand(D, generator=g, device=DEV) + 0.5
+    scaled = ops.linear(_rows(M, 64, g), W0, add_into=ops.AddInto(resid, norm, 1e-5))
+    W, w = _matrix(96, D, g)
+    got = ops.linear(scaled, W, out_dtype=torch.float32)
+    x = (resid * norm).to(BF16)                      # what the product before handed on
+    want, bound = _sums(x, w)
+    rms = (resid.double() ** 2).mean(1, keepdim=True).add(1e-5).sqrt()
+    # the sum, the sum of squares (half its error), and the square root, division and product
+    assert ((got.double() - want / rms).abs() <= (bound + want.abs() * (D / 2 + 4) * 2.0 ** -24) / rms).all().item()
+
+
+@pytest.mark.parametrize("M", [1, 7, 16, 20, 48])
+@pytest.mark.parametrize("D,L", [(32, 2), (64, 3), (1024, 3), (1536, 4), (96, 7)])
+def test_conv_step(M, D, L):
+    """The conv layer's step in one kernel against the same from float64 sums, the gates rounded as it
+    rounds them.  A gate may differ by its sum's error and, beside a rounding boundary, by one unit of
+    bfloat16 (2^-7 of it); what stands before the new value was stored in float and is the same."""
+    g = _gen(M, D, L)
+    x = _rows(M, D, g)
+    W, w = _matrix(3 * D, D, g)
+    taps = torch.randn(D, L, generator=g, device=DEV)
+    bias = torch.randn(D, generator=g, device=DEV)
+    slots = torch.randperm(M + 3, generator=g, device=DEV)[:M].to(torch.int32)
+    pos = torch.arange(M, device=DEV, dtype=torch.int32)
+    state = torch.randn(M + 3, D, L - 1, generator=g, device=DEV)
+    before = state.clone()
+    got = ops.linear_shortconv_step(x, W, None, taps, bias, state, pos, slots)
+    sums, bounds = _sums(x, w)
+    b, c, u = (t.to(BF16).double() for t in sums.float().split(D, 1))
+    unit = 2.0 ** -7
+    db, dc, du = (t + unit * v.abs() for t, v in zip(bounds.split(D, 1), (b, c, u)))
+    old = before[slots.long()].double()
+    old[pos == 0] = 0
+    window = torch.cat([old, (b * u)[:, :, None]], 2)
+    d_new = b.abs() * du + u.abs() * db + db * du + 2.0 ** -24 * (b * u).abs()
+    terms = window * taps.double()
+    s = terms.sum(2) + bias.double()
+    ds = d_new * taps[:, -1].double().abs() + (L + 1) * 2.0 ** -23 * (terms.abs().sum(2) + bias.double().abs())
+    slack = c.abs() * ds + dc * (s.abs() + ds)
+    assert ((got.double() - c * s).abs() <= slack + unit * ((c * s).abs() + slack)).all().item()
+    after = state[slots.long()].double()
+    assert torch.equal(after[:, :, :-1], window[:, :, 1:-1])
+    assert ((after[:, :, -1] - window[:, :, -1]).abs() <= d_new).all().item()
+    rest = torch.ones(M + 3, dtype=torch.bool, device=DEV)
+    rest[slots.long()] = False
+    assert torch.equal(state[rest], before[rest])

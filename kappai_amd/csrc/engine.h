@@ -28,7 +28,7 @@
 extern "C" {
 #endif
 
-#define KAPPAI_ENGINE_ABI 11         // bumped with every change of the structs below
+#define KAPPAI_ENGINE_ABI 12         // bumped with every change of the structs below
 #define KAPPAI_MAX_GROUPS 8          // paged groups a batch can carry block tables for
 #define KAPPAI_MAX_TABLES 8         // tables and numbers of the parts' own in a step
 
@@ -246,7 +246,7 @@ typedef struct kappai_call {
 
 // The numbers by which parts choose between forms of a kernel (the host's parts use the same).
 typedef struct kappai_tuning {
-  int fused_step_min_width, fused_step_narrow_width, fused_step_narrow_rows;
+  int fused_step_min_width, fused_step_narrow_width, fused_step_narrow_rows, fused_step_rows_over_rows;
   int partial_sums_min_rows;        // projections hand on partial sums above this many rows
   int partial_sums_max_rows;        // and up to this many (more, when every segment is one row)
   int fragment_rows_min;            // the norm writes fragment order from this many rows on

@@ -101,11 +101,15 @@ kappai_carry conv_mixer(kappai_step* s, const void* desc, kappai_rows x, float* 
   const kappai_tuning& tune = m.tuning;
   const int M = x.M, D = m.width, taps = L.taps_per_channel;
   const int region = api.carry_region(s);
-  const bool wide_enough = D >= tune.fused_step_min_width ||
-                           (D >= tune.fused_step_narrow_width && M <= tune.fused_step_narrow_rows);
+  // (tuning.fused_conv_step)
+  const bool one_kernel =
+      D >= tune.fused_step_min_width ||
+      (L.in_proj.w_frag != nullptr
+           ? D <= tune.fused_step_narrow_width && M <= tune.fused_step_narrow_rows
+           : D >= tune.fused_step_narrow_width && M <= tune.fused_step_rows_over_rows);
   kappai_carry none = {};
   if (b.max_segment_rows == 1 && M <= 64 && x.is_bf16 && !L.in_proj.w_is_f32 && D % 16 == 0 &&
-      wide_enough) {
+      one_kernel) {
     // decode: projection, convolution and state shift in one kernel
     if (!api.takes_kernel_order(&L.in_proj, D)) x = api.plain_rows(s, x, resid);
     const int c_frag = (M >= tune.fragment_rows_from && M <= tune.fused_max_rows && D % 32 == 0 &&

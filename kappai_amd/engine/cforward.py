@@ -24,7 +24,7 @@ from ..parts.cdesc import (AttentionKernels, CallDesc, CarryDesc, CPlan, Embedde
                            FoldDesc, LinearDesc, NormPartDesc, PartDesc, RowsDesc, address_of,
                            defined_together)
 
-ENGINE_ABI = 11
+ENGINE_ABI = 12
 MAX_GROUPS = 8
 MAX_TABLES = 8         # KAPPAI_MAX_TABLES
 
@@ -43,6 +43,7 @@ class Kernels(Structure):
 class TuningDesc(Structure):
     _fields_ = [(n, c_int) for n in
                 ("fused_step_min_width", "fused_step_narrow_width", "fused_step_narrow_rows",
+                 "fused_step_rows_over_rows",
                  "partial_sums_min_rows", "partial_sums_max_rows", "fragment_rows_min",
                  "fragment_rows_from", "fused_max_rows", "decode_waves", "decode_max_splits",
                  "decode_block_max_keys", "attention_tile_rows", "fused_qk")]
@@ -182,6 +183,7 @@ class CForward:
         t.fused_step_min_width = tuning.FUSED_STEP_MIN_WIDTH
         t.fused_step_narrow_width = tuning.FUSED_STEP_NARROW_WIDTH
         t.fused_step_narrow_rows = tuning.FUSED_STEP_NARROW_ROWS
+        t.fused_step_rows_over_rows = tuning.FUSED_STEP_ROWS_OVER_ROWS
         t.partial_sums_min_rows = tuning.PARTIAL_SUMS_MIN_ROWS
         t.partial_sums_max_rows = tuning.PARTIAL_SUMS_MAX_ROWS
         t.fragment_rows_min = tuning.FRAGMENT_ROWS_MIN if tuning.FRAGMENT_ROWS else 1 << 30

@@ -36,15 +36,26 @@ FRAGMENT_ROWS = True
 FRAGMENT_ROWS_MIN = 8
 
 # The conv layer's fused decode kernel (in_proj, gates, FIR, state shift in one) gives one block 16
-# channels (8 below a width of 4096, where 16 would leave CUs without a block).  From
-# FUSED_STEP_MIN_WIDTH on it beats the separate product (which may split K) plus the small step
-# kernel for any number of rows up to 64; between FUSED_STEP_NARROW_WIDTH and it only up to
-# FUSED_STEP_NARROW_ROWS rows (at a width of 2048, W in fragment order: 8.3 against 9.9 us for one
-# row; 11.0 against 11.1 at 8 rows, 11.5 against 12.8 at 16; at a width of 1024 the separate
-# kernels win).
+# channels (8 below a width of 4096, where 16 would leave CUs without a block), one block a CU.  It beats
+# the separate product (which may split K) with the small step kernel behind it while all its blocks run
+# at once: up to a width of FUSED_STEP_NARROW_WIDTH with up to FUSED_STEP_NARROW_ROWS rows, and from
+# FUSED_STEP_MIN_WIDTH on.  us fused / separate, W in fragment order from memory: width 128, 1 row 3.0 / 3.9;
+# 1024, 1 row 4.3 / 5.4, 16 rows 6.1 / 6.4, 24 rows 6.6 / 7.6, 48 rows 8.1 / 10.0; 2048, 8 rows 8.8 / 10.2, 48 rows
+# 12.1 / 13.5, 64 rows 14.6 / 14.0; 2560, 1 row 13.0 / 11.7; 3072, 8 rows 18.5 / 16.8; 4096, 1 row 21.0 / 22.1, 64 rows
+# 28.3 / 31.1.  Over W as rows: from FUSED_STEP_NARROW_WIDTH on with up to 16 rows.
 FUSED_STEP_MIN_WIDTH = 4096
 FUSED_STEP_NARROW_WIDTH = 2048
-FUSED_STEP_NARROW_ROWS = 16
+FUSED_STEP_NARROW_ROWS = 48
+FUSED_STEP_ROWS_OVER_ROWS = 16
+
+
+def fused_conv_step(width: int, rows: int, in_fragments: bool) -> bool:
+    """Whether a conv layer's decode step of ``rows`` rows runs as one kernel."""
+    if width >= FUSED_STEP_MIN_WIDTH:
+        return True
+    if in_fragments:
+        return width <= FUSED_STEP_NARROW_WIDTH and rows <= FUSED_STEP_NARROW_ROWS
+    return width >= FUSED_STEP_NARROW_WIDTH and rows <= FUSED_STEP_ROWS_OVER_ROWS
 
 # A decode step's attention kernel normalises and rotates q and the row's own key itself and
 # stores key and value (head sizes 64 and 128, rotate-half over the whole head, a projection that

@@ -73,12 +73,10 @@ class GatedShortConv(Mixer):
             raise ValueError("a short convolution's state cannot be read by another layer")
         w = self.in_proj.weight
         rows = x.shape[0]
-        wide_enough = self.width >= tuning.FUSED_STEP_MIN_WIDTH or (
-            self.width >= tuning.FUSED_STEP_NARROW_WIDTH
-            and rows <= tuning.FUSED_STEP_NARROW_ROWS)
         if (batch.max_segment_rows == 1 and rows <= 64
                 and x.dtype == torch.bfloat16
-                and w.dtype == torch.bfloat16 and self.width % 16 == 0 and wide_enough):
+                and w.dtype == torch.bfloat16 and self.width % 16 == 0
+                and tuning.fused_conv_step(self.width, rows, isinstance(w, ops.InFragments))):
             # decode: projection, convolution and state shift in one kernel
             with profile.scope("matmul_in_proj", self.in_proj.weight_bytes()):
                 y = ops.linear_shortconv_step(x, w, self.in_proj.bias, self.taps, self.conv_bias,

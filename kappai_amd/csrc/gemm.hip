@@ -28,6 +28,18 @@ typedef __attribute__((ext_vector_type(4))) float f32x4_t;
 typedef __attribute__((ext_vector_type(16))) float f32x16_t;
 typedef __attribute__((ext_vector_type(4))) uint32_t u32x4_t;
 
+#define KAPPAI_GPTR(p) ((const __attribute__((address_space(1))) void*)(p))
+#define KAPPAI_LPTR(p) ((__attribute__((address_space(3))) void*)(p))
+
+// A buffer of `bytes` bytes from p on: loads whose lane's and scalar offset together lie outside it read
+// nothing and give zeros, so a loop's last loads need no branch.  (The type is the device compiler's; the host
+// pass sees neither it nor the loads.)
+#if defined(__HIP_DEVICE_COMPILE__)
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t raw_buffer(const void* p, uint32_t bytes) {
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), 0, (int)bytes, 0x00020000);
+}
+#endif
+
 // ---------------------------------------------------------------------------------------
 // true fp32
 // ---------------------------------------------------------------------------------------
@@ -230,16 +242,22 @@ __global__ __launch_bounds__((COLS == 8 ? RUNS / 2 : 8) * WAVE) void gemm_f32_sk
 }
 
 // More rows: bound by the matrix cores.  Blocks of WY x WX waves with wave tiles of 16 TY x 16 TX;
-// K tiles of BK go through registers into two LDS buffers whose 16-byte places are XOR-permuted by
-// the row, so that eight lanes of a read hit all banks.  The next tile's loads are under way while
-// this one is multiplied.  An XCD takes every eighth column of tiles and walks its rows of tiles, so W
+// K tiles of BK in two LDS buffers whose 16-byte places are XOR-permuted by the row, so that the 16 rows of
+// a read hit all banks.  An XCD takes every eighth column of tiles and walks its rows of tiles, so W
 // is read into one L2 only.  Two waves a SIMD: a wave's chunk, run and whole sums stay in
-// vector registers, and one wave multiplies while the other waits for LDS.  825 rows: 9216 x 1024
-// 165 us (94 TFLOP/s; the instruction alone reaches 153), 3072 x 1024 66 us, 2048 x 1024 45, 1024 x 4608
-// 101 (with four waves a block of 64 x 64, one a SIMD: 75, 46 and 107).
+// vector registers, and one wave multiplies while the other waits for LDS.
+//
+// DIRECT (K a multiple of 128, everything aligned): a tile goes straight into LDS as soon as everybody has
+// the last fragments of the tile that lay there in registers, a whole tile's products ahead of its use,
+// and the next tile's first fragments are read while those last ones are multiplied.  Else the next tile's
+// loads are under way in registers while this one is multiplied, and are written behind its products, where
+// both waves of a SIMD wait (a third of the time: 99 TFLOP/s at 2048 x 9216 x 1024, the instruction alone
+// reaches 153).  825 rows, through registers / straight: 9216 x 1024 158.7 / 139.4 us (112 TFLOP/s), 3072 x 1024
+// 63.8 / 52.1, 2048 x 1024 43.2 / 36.7, 1024 x 4608 95.4 / 80.6; 65 rows of 9216 x 1024 43.3 / 37.1; the same bits.
+// (With four waves a block of 64 x 64, one a SIMD, 13 % slower.)
 //
 // GATED (wave tiles of two 16s of columns): the second 16 of every 32 columns are the up rows of the first.
-template <int WY, int WX, int TY, int TX, int BK, int LOADS, bool GATED = false>
+template <int WY, int WX, int TY, int TX, int BK, int LOADS, bool GATED = false, bool DIRECT = false>
 __global__ __launch_bounds__(WY * WX * WAVE) __attribute__((amdgpu_waves_per_eu(2)))
 void gemm_f32_block_kernel(
     const float* __restrict__ A, const float* __restrict__ W, const float* __restrict__ bias,
@@ -247,7 +265,9 @@ void gemm_f32_block_kernel(
   constexpr int BM = 16 * WY * TY, BN = 16 * WX * TX, SLOTS = BK / 4, NT = WY * WX * WAVE;
   constexpr int PER = BM * SLOTS / NT;                         // 16-byte places a thread and operand
   static_assert(BM == BN && PER * NT == BM * SLOTS && F32_CHUNK % BK == 0, "a tile");
-  __shared__ f32x4_t lds[2][2][BM * SLOTS];
+  static_assert(!DIRECT || LOADS == F32_WHOLE, "tiles without a remainder");
+  constexpr int MIX = SLOTS - 1;                               // places a row's number turns
+  __shared__ __attribute__((aligned(1024))) f32x4_t lds[2][2][BM * SLOTS];
   const int tid = threadIdx.x, wave = tid / WAVE, lane = tid % WAVE;
   const int r = lane % 16, q = lane / 16;
   const int wm = wave / WX * 16 * TY, wn = wave % WX * 16 * TX;
@@ -265,8 +285,39 @@ void gemm_f32_block_kernel(
     src[0][p] = A + (size_t)min(m0 + row, M - 1) * lda;
     src[1][p] = W + (GATED ? (size_t)(row / 16 % 2) * N + min(n0 + row / 32 * 16 + row % 16, N - 1)
                            : (size_t)min(n0 + row, N - 1)) * K;
-    at[p] = row * SLOTS + (slot ^ (row & 7));
+    at[p] = row * SLOTS + (slot ^ (row & MIX));
   }
+  // DIRECT: a load of a wave brings 64 / SLOTS rows of a tile straight into LDS, 16 bytes a lane in the
+  // order of the lanes, so that the lane turns what it asks for; half of the waves bring A, half W.
+  constexpr int ROWS_A_LOAD = 64 / SLOTS, LOADS_A_WAVE = 2 * BM / ROWS_A_LOAD / (NT / WAVE);
+  static_assert(LOADS_A_WAVE < 16 && LOADS_A_WAVE * (NT / WAVE) * ROWS_A_LOAD == 2 * BM, "a wave's loads");
+  const int uw = __builtin_amdgcn_readfirstlane(wave);
+  const int operand = uw / (NT / WAVE / 2), first_row = uw % (NT / WAVE / 2) * LOADS_A_WAVE * ROWS_A_LOAD;
+  uint32_t off[LOADS_A_WAVE];
+  if constexpr (DIRECT) {
+#pragma unroll
+    for (int i = 0; i < LOADS_A_WAVE; ++i) {
+      const int row = first_row + i * ROWS_A_LOAD + lane / SLOTS;
+      const uint32_t from = operand == 0 ? (uint32_t)min(m0 + row, M - 1) * (uint32_t)lda
+          : (GATED ? (uint32_t)(row / 16 % 2) * (uint32_t)N + min(n0 + row / 32 * 16 + row % 16, N - 1)
+                   : (uint32_t)min(n0 + row, N - 1)) * (uint32_t)K;
+      off[i] = (from + ((lane % SLOTS) ^ (row & MIX)) * 4) * 4u;
+    }
+  }
+  // (buffer loads: of a global load into LDS the compiler holds that it may be any access to LDS, and waits for
+  // all reads under way where it should wait for the oldest)
+#if defined(__HIP_DEVICE_COMPILE__)
+  const __amdgpu_buffer_rsrc_t from = raw_buffer(operand ? W : A, 0xFFFFFFFFu);
+  const auto bring = [&](int t) {
+#pragma unroll
+    for (int i = 0; i < LOADS_A_WAVE; ++i)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(
+          from, KAPPAI_LPTR(&lds[t & 1][operand][(first_row + i * ROWS_A_LOAD) * SLOTS]), 16, off[i],
+          t * (int)(BK * sizeof(float)), 0, 0);
+  };
+#else
+  const auto bring = [&](int) {};
+#endif
   f32x4_t next[2][PER];
   const auto fetch = [&](int t) {
 #pragma unroll
@@ -290,54 +341,8 @@ void gemm_f32_block_kernel(
   const int chunks = (K + F32_CHUNK - 1) / F32_CHUNK, runs = f32_runs(chunks);
   const int tiles = (K + BK - 1) / BK;
   int run = 0;
-  fetch(0);
-  keep(0);
-  __syncthreads();
-  for (int chunk = 0; chunk < chunks; ++chunk) {
-    f32x4_t acc[TY][TX];
-#pragma unroll
-    for (int i = 0; i < TY; ++i)
-#pragma unroll
-      for (int j = 0; j < TX; ++j) acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int u = 0; u < F32_CHUNK / BK; ++u) {
-      const int t = chunk * (F32_CHUNK / BK) + u;
-      if (LOADS != F32_WHOLE && t >= tiles) break;
-      fetch(min(t + 1, tiles - 1));                  // (the last tile once more, unused)
-      __builtin_amdgcn_sched_barrier(0);             // (left alone, the loads sink to their use)
-      const f32x4_t* la = lds[t & 1][0];
-      const f32x4_t* lw = lds[t & 1][1];
-      f32x4_t av[2][TY], wv[2][TX];
-      const auto read = [&](int s) {
-#pragma unroll
-        for (int i = 0; i < TY; ++i) {
-          const int ra = wm + 16 * i + r;
-          av[s & 1][i] = la[ra * SLOTS + ((4 * s + q) ^ (ra & 7))];
-        }
-#pragma unroll
-        for (int j = 0; j < TX; ++j) {
-          const int rw = wn + 16 * j + r;
-          wv[s & 1][j] = lw[rw * SLOTS + ((4 * s + q) ^ (rw & 7))];
-        }
-      };
-      read(0);
-#pragma unroll
-      for (int s = 0; s < BK / 16; ++s) {
-        if (LOADS != F32_WHOLE && t * BK + 16 * s >= K) break;
-        if (s + 1 < BK / 16) read(s + 1);
-        __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-        for (int e = 0; e < 4; ++e)
-#pragma unroll
-          for (int i = 0; i < TY; ++i)
-#pragma unroll
-            for (int j = 0; j < TX; ++j)
-              acc[i][j] = mfma_f32(av[s & 1][i][e], wv[s & 1][j][e], acc[i][j]);
-        __builtin_amdgcn_sched_barrier(0);
-      }
-      keep(t + 1);
-      __syncthreads();
-    }
+  // a chunk's sums into its run's, and the run's into the whole when it ends
+  const auto add_chunk = [&](int chunk, const f32x4_t (&acc)[TY][TX]) {
 #pragma unroll
     for (int i = 0; i < TY; ++i)
 #pragma unroll
@@ -351,6 +356,99 @@ void gemm_f32_block_kernel(
           fin[i][j] += tot[i][j];
           tot[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
         }
+    }
+  };
+  f32x4_t av[2][TY], wv[2][TX];
+  // the fragments of the 16 of K number s of the tile in buffer b
+  const auto read = [&](int b, int s) {
+#pragma unroll
+    for (int i = 0; i < TY; ++i) {
+      const int ra = wm + 16 * i + r;
+      av[s & 1][i] = lds[b][0][ra * SLOTS + ((4 * s + q) ^ (ra & MIX))];
+    }
+#pragma unroll
+    for (int j = 0; j < TX; ++j) {
+      const int rw = wn + 16 * j + r;
+      wv[s & 1][j] = lds[b][1][rw * SLOTS + ((4 * s + q) ^ (rw & MIX))];
+    }
+  };
+  const auto multiply = [&](int s, f32x4_t (&acc)[TY][TX]) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+#pragma unroll
+      for (int i = 0; i < TY; ++i)
+#pragma unroll
+        for (int j = 0; j < TX; ++j)
+          acc[i][j] = mfma_f32(av[s & 1][i][e], wv[s & 1][j][e], acc[i][j]);
+  };
+  if constexpr (DIRECT) {
+    constexpr int STEPS = BK / 16;
+    static_assert(F32_CHUNK == 2 * BK, "a chunk is a tile in either buffer");
+    bring(0);
+    bring(1);
+    __builtin_amdgcn_s_waitcnt(0x0070 | LOADS_A_WAVE);         // tile 0 is there
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_sched_barrier(0);
+    read(0, 0);
+    for (int chunk = 0; chunk < chunks; ++chunk) {
+      f32x4_t acc[TY][TX];
+#pragma unroll
+      for (int i = 0; i < TY; ++i)
+#pragma unroll
+        for (int j = 0; j < TX; ++j) acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int u = 0; u < 2; ++u) {
+        const int t = 2 * chunk + u;
+#pragma unroll
+        for (int s = 0; s + 1 < STEPS; ++s) {
+          read(u, s + 1);
+          __builtin_amdgcn_sched_barrier(0);
+          multiply(s, acc);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+        // The tile's last fragments are in registers: its buffer takes the tile after the next, and the
+        // next one's first fragments come while the last of this one are multiplied.  (Behind the last tile
+        // too: what is read there is not used, but a branch would have the products wait for it.)
+        __builtin_amdgcn_s_waitcnt(0x0070);                    // no load of either kind under way
+        __builtin_amdgcn_s_barrier();
+        __builtin_amdgcn_sched_barrier(0);
+        if (t + 2 < tiles) bring(t + 2);
+        read(u ^ 1, 0);
+        __builtin_amdgcn_sched_barrier(0);
+        multiply(STEPS - 1, acc);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      add_chunk(chunk, acc);
+    }
+  } else {
+    fetch(0);
+    keep(0);
+    __syncthreads();
+    for (int chunk = 0; chunk < chunks; ++chunk) {
+      f32x4_t acc[TY][TX];
+#pragma unroll
+      for (int i = 0; i < TY; ++i)
+#pragma unroll
+        for (int j = 0; j < TX; ++j) acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int u = 0; u < F32_CHUNK / BK; ++u) {
+        const int t = chunk * (F32_CHUNK / BK) + u;
+        if (LOADS != F32_WHOLE && t >= tiles) break;
+        fetch(min(t + 1, tiles - 1));                  // (the last tile once more, unused)
+        __builtin_amdgcn_sched_barrier(0);             // (left alone, the loads sink to their use)
+        read(t & 1, 0);
+#pragma unroll
+        for (int s = 0; s < BK / 16; ++s) {
+          if (LOADS != F32_WHOLE && t * BK + 16 * s >= K) break;
+          if (s + 1 < BK / 16) read(t & 1, s + 1);
+          __builtin_amdgcn_sched_barrier(0);
+          multiply(s, acc);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+        keep(t + 1);
+        __syncthreads();
+      }
+      add_chunk(chunk, acc);
     }
   }
   if constexpr (GATED) {
@@ -386,8 +484,16 @@ static void launch_f32_blocks(const float* A, const float* W, const float* bias,
                               int N, int K, int lda, int ldc, hipStream_t stream) {
   constexpr int B = 32 * TY;
   const int tm = (M + B - 1) / B, tn = ((GATED ? 2 : 1) * N + B - 1) / B;
-  hipLaunchKernelGGL((gemm_f32_block_kernel<2, 4, TY, TX, 64, LOADS, GATED>), dim3((tn + 7) / 8 * 8 * tm),
-                     dim3(512), 0, stream, A, W, bias, C, M, N, K, lda, ldc, tm);
+  const dim3 grid((tn + 7) / 8 * 8 * tm);
+  // (offsets of 32 bits within either operand)
+  if constexpr (LOADS == F32_WHOLE)
+    if ((size_t)M * lda < 1u << 30 && (size_t)(GATED ? 2 : 1) * N * K < 1u << 30) {
+      hipLaunchKernelGGL((gemm_f32_block_kernel<2, 4, TY, TX, 64, LOADS, GATED, true>), grid, dim3(512), 0, stream,
+                         A, W, bias, C, M, N, K, lda, ldc, tm);
+      return;
+    }
+  hipLaunchKernelGGL((gemm_f32_block_kernel<2, 4, TY, TX, 64, LOADS, GATED>), grid, dim3(512), 0, stream, A, W, bias,
+                     C, M, N, K, lda, ldc, tm);
 }
 
 static bool f32_large_blocks(int M, int N) {
@@ -765,8 +871,6 @@ static void launch_tile_cfg(const bf16_t* A, const bf16_t* W, const float* bias,
 //
 // Host side guarantees: K / gridDim.y is a multiple of 128, rows of W a multiple of 8 (32 with
 // SwiGLU), C and its row stride 16-byte aligned, M * lda and N * K below 2^31 elements.
-#define KAPPAI_GPTR(p) ((const __attribute__((address_space(1))) void*)(p))
-#define KAPPAI_LPTR(p) ((__attribute__((address_space(3))) void*)(p))
 #define SCHED_FENCE() __builtin_amdgcn_sched_barrier(0)
 // (nothing that touches memory is moved across, by any pass of the compiler)
 #define ORDER_FENCE()                  \
@@ -778,15 +882,6 @@ static void launch_tile_cfg(const bf16_t* A, const bf16_t* W, const float* bias,
 #define WAIT_LOADS(behind) __builtin_amdgcn_s_waitcnt(0x0F70 | ((behind) & 15) | ((behind) >> 4 << 14))
 #define WAIT_LOADS_AND_LDS(behind) \
   __builtin_amdgcn_s_waitcnt(0x0070 | ((behind) & 15) | ((behind) >> 4 << 14))
-
-// A buffer of `bytes` bytes from p on: loads whose lane's and scalar offset together lie outside it read
-// nothing and give zeros, so a loop's last loads need no branch.  (The type is the device compiler's; the host
-// pass sees neither it nor the loads.)
-#if defined(__HIP_DEVICE_COMPILE__)
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t raw_buffer(const void* p, uint32_t bytes) {
-  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), 0, (int)bytes, 0x00020000);
-}
-#endif
 
 template <int N> struct IntC { static constexpr int value = N; };
 

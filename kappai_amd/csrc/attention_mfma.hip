@@ -177,11 +177,10 @@ __device__ __forceinline__ void attn_one_row(const bf16_t* q, int q_stride, cons
 #define P_MIN_WAVES (HEAD_DIM <= 96 ? 2 : 1)
 template <bool MODS>
 __global__ __launch_bounds__(P_NW * WAVE, P_MIN_WAVES) void attn_prefill_kernel(
-    const bf16_t* __restrict__ q, int q_stride, const bf16_t* __restrict__ k_pool,
-    const bf16_t* __restrict__ vt_pool, bf16_t* __restrict__ out, int out_stride,
     const int* __restrict__ q_tiles, const int* __restrict__ row_pos,
-    const int* __restrict__ block_tables, int max_blocks, int H, int G, int ps, int window,
-    float scale, kappai_score_mods mods) {
+    const int* __restrict__ block_tables, int max_blocks, int H, int G, int ps, int q_stride, int window,
+    const bf16_t* __restrict__ q, const bf16_t* __restrict__ k_pool, const bf16_t* __restrict__ vt_pool,
+    bf16_t* __restrict__ out, int out_stride, float scale, kappai_score_mods mods) {
   // later tiles of a segment have more keys: they are started first
   const int tile = gridDim.x - 1 - blockIdx.x, h = blockIdx.y;
   const int lane = threadIdx.x % WAVE;
@@ -492,7 +491,7 @@ __global__ __launch_bounds__(P_NW * WAVE, P_MIN_WAVES) void attn_prefill_kernel(
 // ---------------------------------------------------------------------------------------
 // One block = two q tiles (32 rows each) of one segment x four query heads of one kv head, a
 // wave each.  The eight waves walk the same key tiles, so a tile of K (32 keys x d) and of V^T
-// (d x 32 keys) is brought from global memory once, straight into LDS (global_load_lds, three
+// (d x 32 keys) is brought from global memory once, straight into LDS (buffer loads, three
 // buffers, two tiles ahead), and every wave reads its matrix operands from there.  Pairing an
 // early q tile with a late one gives every block the same number of keys to walk.  K rows keep their 16-byte chunks permuted (chunk ^ f(key)) so that the
 // 16 keys of a fragment read fall on different banks; V^T lies as [16-key group][d][16 keys],
@@ -504,22 +503,22 @@ __global__ __launch_bounds__(P_NW * WAVE, P_MIN_WAVES) void attn_prefill_kernel(
 // of them at two waves a SIMD) and by what two waves a SIMD leave uncovered: 2,048 rows are 256 blocks,
 // so the chip has no more.  2,048 rows, 32 heads of 64 on 8: without past 44.1 us (54.1 with values put together
 // from two reads and one loop for masked and whole steps), behind 4,096 keys 128.4 (156.5), behind 9,900
-// 255.9 (307.5: 0.57 PFLOP/s, now 0.69).  Priorities for the waves of one tile, for the products or for the
+// 255.9 (307.5: 0.57 PFLOP/s, now 0.69).  Then 2,048 rows at a time to 12,288 keys, mean of a portion: 151 us
+// with the tiles brought by loads through flat addresses and each tile's page by a scalar load (either has
+// every wait for LDS be one for all of it), 140 now.  Priorities for the waves of one tile, for the products or for the
 // exponentials: within 3 %; both tiles' scores ahead of either's exponentials: the same.
 #if HEAD_DIM == 64 || HEAD_DIM == 128
 #define PG_OK 1
 #define PG_NBUF 3
 #define PG_SUB 2
 template <int N> struct PgBuf { static constexpr int value = N; };
-#define PG_GPTR(p) ((const __attribute__((address_space(1))) void*)(p))
 #define PG_LPTR(p) ((__attribute__((address_space(3))) void*)(p))
 
 __global__ __launch_bounds__(8 * WAVE) void attn_prefill_shared_kernel(
-    const bf16_t* __restrict__ q, int q_stride, const bf16_t* __restrict__ k_pool,
-    const bf16_t* __restrict__ vt_pool, bf16_t* __restrict__ out, int out_stride,
     const int* __restrict__ q_tiles, const int* __restrict__ row_pos,
-    const int* __restrict__ block_tables, int max_blocks, int H, int G, int ps, int window,
-    float scale, const float* __restrict__ sink) {
+    const int* __restrict__ block_tables, int max_blocks, int H, int G, int ps, int q_stride, int window,
+    const bf16_t* __restrict__ q, const bf16_t* __restrict__ k_pool, const bf16_t* __restrict__ vt_pool,
+    bf16_t* __restrict__ out, int out_stride, float scale, const float* __restrict__ sink) {
   constexpr int ROWB = HEAD_DIM * 2;                // bytes of a key's row
   constexpr int KTILE = 32 * ROWB, VGROUP = HEAD_DIM * 32, BUF = KTILE + 2 * VGROUP;   // bytes
   constexpr int CPR = ROWB / 16;                    // 16-byte chunks a K row
@@ -634,35 +633,52 @@ __global__ __launch_bounds__(8 * WAVE) void attn_prefill_shared_kernel(
   // masked when it is used.  A wave's keys (8 of K, 16 of V^T) lie in one page.
   int nx_key = kbase + (wave < 4 ? 8 * wave : 16 * v_st);
   int nx_pidx = nx_key / ps, nx_off = nx_key % ps;
+  // 64 of the segment's pages, a lane each, and the number of the first: a scalar load a tile would have every
+  // wait for LDS wait for it too
+  int pages = 0, pages_from = -(1 << 30);
   auto lookup = [&]() {
-    const int page = nx_key <= blk_last ? bt[min(nx_pidx, max_blocks - 1)] : 0;
-    return max(page, 0);
+    if (nx_key > blk_last) return 0;
+    const int at = min(nx_pidx, max_blocks - 1);
+    if (at - pages_from >= WAVE) {
+      pages_from = at;
+      pages = bt[min(at + lane, max_blocks - 1)];
+      asm volatile("" : "+v"(pages));      // (waits here, and not at every tile for a load that may be under way)
+    }
+    return max(__builtin_amdgcn_readlane(pages, at - pages_from), 0);
   };
   int nx_page = lookup();
+  // (buffer loads: of a global load into LDS the compiler holds that it may be any access to LDS, and waits for
+  // all reads under way where it should wait for the oldest)
+  uint32_t from[NL];
+#pragma unroll
+  for (int i = 0; i < NL; ++i) {
+    const int row = i * K_ROWS_PER + k_row_in;                 // 0..7 within the wave's keys
+    // (V^T: rows 8 apart would meet on the same banks: every other group of 8 rows keeps its two 16-byte halves
+    // swapped)
+    const int dd = v_d0 + 32 * i;
+    from[i] = 2u * (uint32_t)(wave < 4 ? row * HEAD_DIM + (k_slot ^ swz(8 * wave + row)) * 8
+                                       : dd * ps + 8 * (v_half ^ ((dd >> 3) & 1)));
+  }
   auto issue_one = [&](char* buf) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    const size_t head = (size_t)nx_page * G + g;
     if (wave < 4) {
-      const bf16_t* base = k_pool + (((size_t)nx_page * G + g) * ps + nx_off) * HEAD_DIM;
+      const __amdgpu_buffer_rsrc_t keys = __builtin_amdgcn_make_buffer_rsrc(
+          const_cast<bf16_t*>(k_pool + (head * ps + nx_off) * HEAD_DIM), 0, 0x7FFFFF00, 0x00020000);
 #pragma unroll
-      for (int i = 0; i < NL; ++i) {
-        const int row = i * K_ROWS_PER + k_row_in;               // 0..7 within the wave's keys
-        const int chunk = k_slot ^ swz(8 * wave + row);
-        __builtin_amdgcn_global_load_lds(PG_GPTR(base + row * HEAD_DIM + chunk * 8),
-                                         PG_LPTR(buf + (8 * wave + i * K_ROWS_PER) * ROWB), 16, 0,
-                                         0);
-      }
+      for (int i = 0; i < NL; ++i)
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(keys, PG_LPTR(buf + (8 * wave + i * K_ROWS_PER) * ROWB), 16,
+                                                 from[i], 0, 0, 0);
     } else {
-      const bf16_t* base = vt_pool + ((size_t)nx_page * G + g) * HEAD_DIM * ps + nx_off;
+      const __amdgpu_buffer_rsrc_t values = __builtin_amdgcn_make_buffer_rsrc(
+          const_cast<bf16_t*>(vt_pool + head * HEAD_DIM * ps + nx_off), 0, 0x7FFFFF00, 0x00020000);
 #pragma unroll
-      for (int i = 0; i < NL; ++i) {
-        const int dd = v_d0 + 32 * i;
-        // rows 8 apart would meet on the same banks: every other group of 8 rows keeps its two
-        // 16-byte halves swapped
-        __builtin_amdgcn_global_load_lds(
-            PG_GPTR(base + (size_t)dd * ps + 8 * (v_half ^ ((dd >> 3) & 1))),
-            PG_LPTR(buf + KTILE + v_st * VGROUP + ((vw % 2) * (HEAD_DIM / 2) + 32 * i) * 32), 16, 0,
-            0);
-      }
+      for (int i = 0; i < NL; ++i)
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(
+            values, PG_LPTR(buf + KTILE + v_st * VGROUP + ((vw % 2) * (HEAD_DIM / 2) + 32 * i) * 32), 16, from[i], 0,
+            0, 0);
     }
+#endif
     nx_key += 32;
     nx_off += 32;
     while (nx_off >= ps) {
@@ -886,6 +902,9 @@ __global__ __launch_bounds__(8 * WAVE) void attn_prefill_shared_kernel(
   static_assert(PG_SUB == 2, "the step works on two tiles");
   issue(PgBuf<0>{});
   if (n_steps > 1) issue(PgBuf<1>{});
+  // (the queries have arrived: where this is not said, every step waits for all loads but its own first)
+#pragma unroll
+  for (int ks = 0; ks < P_KS; ++ks) asm volatile("" : "+v"(qf[ks]));
   // The steps whose tiles need no mask, in whole rounds of the buffers, are a loop of their own: where the
   // two ways through a step meet again, 48 accumulators are copied (a sixth of the step's vector work).
   int it = 0, fast_from = 0, fast_to = 0;
@@ -935,10 +954,10 @@ __global__ __launch_bounds__(8 * WAVE) void attn_prefill_shared_kernel(
 // One block = one q tile (32 rows) x four query heads of one kv head, two waves a head: both make the
 // scores, each half of the output's columns (with all of them in one wave the registers spill and a
 // SIMD has no second wave to work while the first is at its exponentials).  A tile of K (32 keys x d)
-// and of V^T comes from global memory once, straight into LDS (global_load_lds, three buffers, two
+// and of V^T comes from global memory once, straight into LDS (buffer loads, three buffers, two
 // tiles ahead), in the places the kernel above gives them.  A wave alone with its head, which is the other way, reads
 // every operand from the caches itself and has no registers to ask ahead: it waits about 3 us for a
-// tile, whatever else runs.  Two portions of 1,900 rows in all, 16 heads on one kv head: 127 -> 82 us;
+// tile, whatever else runs.  Two portions of 1,900 rows in all, 16 heads on one kv head: 127 -> 79 us;
 // what bounds it now is a wave's own chain over a tile (scores, exponentials, output), two waves a
 // SIMD, about 2 us for each of the longest portion's 38 tiles.  The arithmetic is that wave's to the bit: the accumulators are only
 // left alone where they would have been multiplied by one.
@@ -946,11 +965,10 @@ __global__ __launch_bounds__(8 * WAVE) void attn_prefill_shared_kernel(
 #define PH_NBUF 3
 template <int N> struct PhBuf { static constexpr int value = N; };
 __global__ __launch_bounds__(8 * WAVE) void attn_prefill_heads_kernel(
-    const bf16_t* __restrict__ q, int q_stride, const bf16_t* __restrict__ k_pool,
-    const bf16_t* __restrict__ vt_pool, bf16_t* __restrict__ out, int out_stride,
     const int* __restrict__ q_tiles, const int* __restrict__ row_pos,
-    const int* __restrict__ block_tables, int max_blocks, int H, int G, int ps, int window,
-    float scale, const float* __restrict__ sink) {
+    const int* __restrict__ block_tables, int max_blocks, int H, int G, int ps, int q_stride, int window,
+    const bf16_t* __restrict__ q, const bf16_t* __restrict__ k_pool, const bf16_t* __restrict__ vt_pool,
+    bf16_t* __restrict__ out, int out_stride, float scale, const float* __restrict__ sink) {
   constexpr int ROWB = HEAD_DIM * 2;                                              // bytes of a key's row
   constexpr int KTILE = 32 * ROWB, VGROUP = HEAD_DIM * 32, BUF = KTILE + 2 * VGROUP;   // bytes
   constexpr int NL = 4, MT = P_MT / 2;       // loads a wave issues a tile; row tiles of its half of O^T
@@ -998,23 +1016,30 @@ __global__ __launch_bounds__(8 * WAVE) void attn_prefill_heads_kernel(
   const unsigned k_chunk = lane % 32, k_row = 8 * half + lane / 32, v_row = 128 * half + lane / 2;
   const unsigned at0 = wave < 4 ? k_row * ROWB
                                 : v_row * ps * 2 + 16 * (v_half ^ ((v_row >> 3) & 1));
+  // (a tile's page is asked for before the barrier in front of its loads: behind it, among the reads of LDS, the
+  // wait for a scalar load is one for all of them)
+  int nx_page = 0;
+  auto lookup = [&]() { nx_page = bt[min(min(nx_key, pos_last) / ps, max_blocks - 1)]; };
   auto issue = [&](auto buf_c) {
     char* buf = lds + decltype(buf_c)::value * BUF;
-    const int page = nx_key <= pos_last ? max(bt[min(nx_key / ps, max_blocks - 1)], 0) : 0;
-    const size_t head = (size_t)page * G + g;
+#if defined(__HIP_DEVICE_COMPILE__)
+    const size_t head = (size_t)(nx_key <= pos_last ? max(nx_page, 0) : 0) * G + g;
     const int off = nx_key % ps;
     // (rows 32 apart have the same swapped halves)
-    const char* from = wave < 4 ? (const char*)(k_pool + (head * ps + off) * HEAD_DIM)
-                                : (const char*)(vt_pool + head * HEAD_DIM * ps + off);
+    const bf16_t* from = wave < 4 ? k_pool + (head * ps + off) * HEAD_DIM : vt_pool + head * HEAD_DIM * ps + off;
+    const __amdgpu_buffer_rsrc_t keys =
+        __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16_t*>(from), 0, 0x7FFFFF00, 0x00020000);
     const unsigned step = wave < 4 ? 2 * ROWB : 64 * ps;
+    unsigned first = at0;
+    asm volatile("" : "+v"(first));                  // (four places kept over the loop: registers there are not)
     char* to = wave < 4 ? buf + 8 * part * ROWB : buf + KTILE + (part / 2) * VGROUP + half * 128 * 32;
 #pragma unroll
     for (int i = 0; i < NL; ++i) {
       const unsigned swap = wave < 4 ? 16 * (k_chunk ^ ((k_row + 2 * i) & 15)) : 0;
-      __builtin_amdgcn_global_load_lds(
-          (const __attribute__((address_space(1))) void*)(from + i * step + (at0 + swap)),
-          (__attribute__((address_space(3))) void*)(to + 1024 * i), 16, 0, 0);
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(keys, (__attribute__((address_space(3))) void*)(to + 1024 * i), 16,
+                                               first + swap, i * step, 0, 0);
     }
+#endif
     nx_key += 32;
   };
   auto work = [&](auto buf_c, int kb) {
@@ -1108,6 +1133,7 @@ __global__ __launch_bounds__(8 * WAVE) void attn_prefill_heads_kernel(
   auto step = [&](auto buf_c, int it) {
     __builtin_amdgcn_sched_barrier(0);
     constexpr int B = decltype(buf_c)::value;
+    if (it + 2 < n_steps) lookup();
     // this step's tile has landed (this wave's part; the barrier makes it everybody's)
     if (it + 1 < n_steps) __builtin_amdgcn_s_waitcnt(0x0F70 | NL);
     else __builtin_amdgcn_s_waitcnt(0x0F70);
@@ -1116,8 +1142,13 @@ __global__ __launch_bounds__(8 * WAVE) void attn_prefill_heads_kernel(
     if (it + 2 < n_steps) issue(PhBuf<(B + 2) % PH_NBUF>{});
     work(buf_c, kbase + 32 * it);
   };
+  lookup();
   issue(PhBuf<0>{});
+  lookup();
   if (n_steps > 1) issue(PhBuf<1>{});
+  // (the queries have arrived: where this is not said, every step waits for all loads but its own first)
+#pragma unroll
+  for (int ks = 0; ks < P_KS; ++ks) asm volatile("" : "+v"(qf[ks]));
   for (int it = 0; it < n_steps; it += PH_NBUF) {
     step(PhBuf<0>{}, it);
     if (it + 1 < n_steps) step(PhBuf<1>{}, it + 1);
@@ -1749,14 +1780,19 @@ __device__ __forceinline__ int step_keys_per_split(const int* __restrict__ row_p
 // halve the waves a SIMD holds for the steps that do not use it)
 // (PLAN: the keys per split come from step_keys_per_split, else they are the caller's: a kernel of
 // its own, because the rule's code costs half a microsecond even where it is skipped)
+// (The arguments of this kernel and of the two that do a row in one block stand in the order in which they are
+// needed: the first fourteen words come in registers, and they are those on the way to the row's pages, which
+// are three dependent reads ahead of the first key.  The pools' addresses are asked for beside the position.
+// One row of 16 heads at 200 to 1,000 keys, whole pass of 22 layers with 6 of these: 7,280 -> 7,260 us for 64
+// tokens, 16 rows at 4,000 keys 1,318 -> 1,303 us a step.)
 template <bool FUSED, bool PLAN, bool MODS = false>
 __global__ __launch_bounds__(64, (FUSED && HEAD_DIM != 64) || MODS || HEAD_DIM > 128 ? 1 : 2) void attn_decode_kernel(
-    const bf16_t* __restrict__ q, int q_stride, const bf16_t* __restrict__ k_pool,
-    const bf16_t* __restrict__ vt_pool, float* __restrict__ part_o, float* __restrict__ part_ml,
     const int* __restrict__ row_pos, const int* __restrict__ row_seg,
-    const int* __restrict__ block_tables, int max_blocks, int H, int G, int ps, int window,
-    float scale, int keys_per_split, int n_splits, QkFuse qk, const int* __restrict__ row_ids,
-    kappai_score_mods mods) {
+    const int* __restrict__ block_tables, const int* __restrict__ row_ids, int max_blocks, int H, int G,
+    int ps, int q_stride, int window, const bf16_t* __restrict__ q, const bf16_t* __restrict__ k_pool,
+    const bf16_t* __restrict__ vt_pool, float* __restrict__ part_o, float* __restrict__ part_ml,
+    float scale, int keys_per_split, int n_splits, QkFuse qk, kappai_score_mods mods) {
+  // (the arguments on the way to the row's pages come first: those are handed over in registers)
   // (row_ids: the kernel's rows are these rows of the step, partial results are kept by their
   // place in the list)
   // Blocks go to the CUs in the order of their numbers, the row's number fastest: with a number
@@ -1881,11 +1917,10 @@ __device__ __forceinline__ void attn_one_row(const bf16_t* q, int q_stride, cons
 
 template <bool MODS>
 __global__ __launch_bounds__(D_BLOCK_MAX_WAVES * WAVE) void attn_decode_block_kernel(
-    const bf16_t* __restrict__ q, int q_stride, const bf16_t* __restrict__ k_pool,
-    const bf16_t* __restrict__ vt_pool, bf16_t* __restrict__ out, int out_stride,
     const int* __restrict__ row_pos, const int* __restrict__ row_seg,
-    const int* __restrict__ block_tables, int max_blocks, int H, int G, int ps, int window,
-    float scale, kappai_score_mods mods) {
+    const int* __restrict__ block_tables, int max_blocks, int H, int G, int ps, int q_stride, int window,
+    const bf16_t* __restrict__ q, const bf16_t* __restrict__ k_pool, const bf16_t* __restrict__ vt_pool,
+    bf16_t* __restrict__ out, int out_stride, float scale, kappai_score_mods mods) {
   extern __shared__ float sh_dec[];
   const int t = blockIdx.x;
   attn_one_row<MODS, false, D_BLOCK_SHARE>(q, q_stride, k_pool, vt_pool, out, out_stride,
@@ -1898,11 +1933,10 @@ __global__ __launch_bounds__(D_BLOCK_MAX_WAVES * WAVE) void attn_decode_block_ke
 // D_QK_BLOCK_MAX_KEYS).
 #if HEAD_DIM == 64
 __global__ __launch_bounds__(D_BLOCK_MAX_WAVES * WAVE) void attn_decode_block_qk_kernel(
-    const bf16_t* __restrict__ qkv, int row_stride, const bf16_t* __restrict__ k_pool,
-    const bf16_t* __restrict__ vt_pool, bf16_t* __restrict__ out, int out_stride,
     const int* __restrict__ row_pos, const int* __restrict__ row_seg,
-    const int* __restrict__ block_tables, int max_blocks, int H, int G, int ps, int window,
-    float scale, QkFuse qk) {
+    const int* __restrict__ block_tables, int max_blocks, int H, int G, int ps, int row_stride, int window,
+    const bf16_t* __restrict__ qkv, const bf16_t* __restrict__ k_pool, const bf16_t* __restrict__ vt_pool,
+    bf16_t* __restrict__ out, int out_stride, float scale, QkFuse qk) {
   extern __shared__ float sh_dec[];
   const int t = blockIdx.x;
   attn_one_row<false, true, D_BLOCK_SHARE>(qkv, row_stride, k_pool, vt_pool, out, out_stride,
@@ -1916,31 +1950,42 @@ __global__ __launch_bounds__(D_BLOCK_MAX_WAVES * WAVE) void attn_decode_block_qk
 // out[t, h, :] = sum_s o_s 2^(m_s - M) / sum_s l_s 2^(m_s - M).  Four waves share the splits
 // (wave w takes s = w, w+4, ...); each computes its splits' weights one per lane.  The partial
 // outputs of MERGE_AHEAD splits are asked for before the maxima, so that with up to 32 splits
-// the kernel waits for memory once.
+// the kernel waits for memory once.  (Loads without conditions: of loads in branches of their own the compiler
+// puts a wait between.)
 #define MERGE_WAVES 4
 #define MERGE_AHEAD 8
 __global__ __launch_bounds__(MERGE_WAVES * WAVE) void attn_merge_kernel(
     const float* __restrict__ part_o, const float* __restrict__ part_ml,
-    bf16_t* __restrict__ out, int out_stride, int H, int splits_stride,
-    const int* __restrict__ row_ids, const int* __restrict__ row_pos, int window, int keep, int G,
-    int kps_min, int plan_unit, const float* __restrict__ sink) {
+    const int* __restrict__ row_pos, const int* __restrict__ row_ids, int H, int splits_stride, int window,
+    int keep, int kps_min, int plan_unit, int G, bf16_t* __restrict__ out, int out_stride,
+    const float* __restrict__ sink) {
   constexpr int NPL = (HEAD_DIM + WAVE - 1) / WAVE;
   __shared__ float sh_acc[MERGE_WAVES][NPL * WAVE];
   __shared__ float sh_l[MERGE_WAVES];
   const int t = row_ids ? row_ids[blockIdx.x] : blockIdx.x, h = blockIdx.y;
-  const int lane = threadIdx.x % WAVE, wave = threadIdx.x / WAVE;
+  const int lane = threadIdx.x % WAVE, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
   const size_t base = ((size_t)blockIdx.x * H + h) * splits_stride;
   // the partial outputs of this wave's splits number j .. j + MERGE_AHEAD - 1, of the first
   // `bound` splits
   float o[MERGE_AHEAD][NPL];
+#if defined(__HIP_DEVICE_COMPILE__)
+  const __amdgpu_buffer_rsrc_t parts = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<float*>(part_o + base * HEAD_DIM), 0, splits_stride * HEAD_DIM * 4, 0x00020000);
+  auto part_at = [&](int e, int sk, int bound) {
+    const int at = e < HEAD_DIM && sk < bound ? (sk * HEAD_DIM + e) * 4 : 0x7FFFFF00;
+    return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(parts, at, 0, 0));
+  };
+#else
+  auto part_at = [&](int, int, int) { return 0.f; };
+#endif
   auto ask = [&](int j, int bound) {
 #pragma unroll
     for (int k = 0; k < MERGE_AHEAD; ++k) {
       const int sk = wave + MERGE_WAVES * (j + k);
 #pragma unroll
       for (int i = 0; i < NPL; ++i) {
-        const int e = lane + i * WAVE;
-        o[k][i] = (sk < bound && e < HEAD_DIM) ? part_o[(base + sk) * HEAD_DIM + e] : 0.f;
+        // (splits behind the last and places behind the head: outside the buffer, zeros, nothing read)
+        o[k][i] = part_at(lane + i * WAVE, sk, bound);
       }
     }
   };
@@ -2043,14 +2088,14 @@ extern "C" int kappai_attn_decode_block_scored(const void* q, int q_stride, cons
   const size_t lds = (size_t)n_waves * (rep * HEAD_DIM + 32) * sizeof(float);
   if (kappai_mods_change_scores(mods))
     hipLaunchKernelGGL(attn_decode_block_kernel<true>, dim3(T, G), dim3(n_waves * WAVE), lds,
-                       stream, (const bf16_t*)q, q_stride, (const bf16_t*)k_pool,
-                       (const bf16_t*)vt_pool, (bf16_t*)out, out_stride, row_pos, row_seg,
-                       block_tables, max_blocks, H, G, ps, window, scale, *mods);
+                       stream, row_pos, row_seg, block_tables, max_blocks, H, G, ps, q_stride, window,
+                       (const bf16_t*)q, (const bf16_t*)k_pool, (const bf16_t*)vt_pool, (bf16_t*)out,
+                       out_stride, scale, *mods);
   else
     hipLaunchKernelGGL(attn_decode_block_kernel<false>, dim3(T, G), dim3(n_waves * WAVE), lds,
-                       stream, (const bf16_t*)q, q_stride, (const bf16_t*)k_pool,
-                       (const bf16_t*)vt_pool, (bf16_t*)out, out_stride, row_pos, row_seg,
-                       block_tables, max_blocks, H, G, ps, window, scale,
+                       stream, row_pos, row_seg, block_tables, max_blocks, H, G, ps, q_stride, window,
+                       (const bf16_t*)q, (const bf16_t*)k_pool, (const bf16_t*)vt_pool, (bf16_t*)out,
+                       out_stride, scale,
                        kappai_score_mods{0.f, nullptr, 0, mods != nullptr ? mods->sink : nullptr, 0});
   KAPPAI_RETURN_LAUNCH_STATUS();
 }
@@ -2113,9 +2158,9 @@ extern "C" int kappai_attn_prefill_scored(const void* q, int q_stride, const voi
         (mods->dist_bias != nullptr && mods->dist_cols < 1))
       return (int)hipErrorInvalidValue;
     hipLaunchKernelGGL(attn_prefill_kernel<true>, dim3(n_tiles, H), dim3(P_NW * WAVE), 0, stream,
-                       (const bf16_t*)q, q_stride, (const bf16_t*)k_pool, (const bf16_t*)vt_pool,
-                       (bf16_t*)out, out_stride, q_tiles, row_pos, block_tables, max_blocks, H, G,
-                       ps, window, scale, *mods);
+                       q_tiles, row_pos, block_tables, max_blocks, H, G, ps, q_stride, window,
+                       (const bf16_t*)q, (const bf16_t*)k_pool, (const bf16_t*)vt_pool, (bf16_t*)out,
+                       out_stride, scale, *mods);
     KAPPAI_RETURN_LAUNCH_STATUS();
   }
   if (ps % 16 || G < 1 || H % G || H > 65535 || (q_stride % 8) || (out_stride % 4))
@@ -2129,9 +2174,9 @@ extern "C" int kappai_attn_prefill_scored(const void* q, int q_stride, const voi
 #if PG_OK
   if (shared) {
     hipLaunchKernelGGL(attn_prefill_shared_kernel, dim3(n_tiles, H / 4), dim3(8 * WAVE), 0, stream,
-                       (const bf16_t*)q, q_stride, (const bf16_t*)k_pool, (const bf16_t*)vt_pool,
-                       (bf16_t*)out, out_stride, q_tiles, row_pos, block_tables, max_blocks, H, G,
-                       ps, window, scale, sink);
+                       q_tiles, row_pos, block_tables, max_blocks, H, G, ps, q_stride, window,
+                       (const bf16_t*)q, (const bf16_t*)k_pool, (const bf16_t*)vt_pool, (bf16_t*)out,
+                       out_stride, scale, sink);
     KAPPAI_RETURN_LAUNCH_STATUS();
   }
 #endif
@@ -2141,16 +2186,16 @@ extern "C" int kappai_attn_prefill_scored(const void* q, int q_stride, const voi
   // 32 rows behind 2,000 keys 131 / 165; 64 lone rows of 32 keys 6.9 / 10.0, 63 of 800 keys 64 / 126)
   if (variant == 0 && rep % 4 == 0) {
     hipLaunchKernelGGL(attn_prefill_heads_kernel, dim3(n_tiles, H / 4), dim3(8 * WAVE), 0, stream,
-                       (const bf16_t*)q, q_stride, (const bf16_t*)k_pool, (const bf16_t*)vt_pool,
-                       (bf16_t*)out, out_stride, q_tiles, row_pos, block_tables, max_blocks, H, G,
-                       ps, window, scale, sink);
+                       q_tiles, row_pos, block_tables, max_blocks, H, G, ps, q_stride, window,
+                       (const bf16_t*)q, (const bf16_t*)k_pool, (const bf16_t*)vt_pool, (bf16_t*)out,
+                       out_stride, scale, sink);
     KAPPAI_RETURN_LAUNCH_STATUS();
   }
 #endif
   hipLaunchKernelGGL(attn_prefill_kernel<false>, dim3(n_tiles, H), dim3(P_NW * WAVE), 0, stream,
-                     (const bf16_t*)q, q_stride, (const bf16_t*)k_pool, (const bf16_t*)vt_pool,
-                     (bf16_t*)out, out_stride, q_tiles, row_pos, block_tables, max_blocks, H, G,
-                     ps, window, scale, kappai_score_mods{0.f, nullptr, 0, sink, 0});
+                     q_tiles, row_pos, block_tables, max_blocks, H, G, ps, q_stride, window,
+                     (const bf16_t*)q, (const bf16_t*)k_pool, (const bf16_t*)vt_pool, (bf16_t*)out,
+                     out_stride, scale, kappai_score_mods{0.f, nullptr, 0, sink, 0});
   KAPPAI_RETURN_LAUNCH_STATUS();
 }
 
@@ -2186,10 +2231,10 @@ static int launch_decode(const void* q, int q_stride, const void* k_pool, const 
   const bool plan = !qk.on && (long long)T * G * n_splits > D_TARGET_WAVES;
 #define KAPPAI_DECODE(FUSED, PLAN, MODS)                                                         \
   hipLaunchKernelGGL((attn_decode_kernel<FUSED, PLAN, MODS>), dim3(T, G, n_splits), dim3(WAVE),  \
-                     0, stream, (const bf16_t*)q, q_stride, (const bf16_t*)k_pool,               \
-                     (const bf16_t*)vt_pool, part_o, part_ml, row_pos, row_seg, block_tables,    \
-                     max_blocks, H, G, ps, window, scale, keys_per_split, n_splits, qk, row_ids, \
-                     m)
+                     0, stream, row_pos, row_seg, block_tables, row_ids, max_blocks, H, G, ps,   \
+                     q_stride, window, (const bf16_t*)q, (const bf16_t*)k_pool,                  \
+                     (const bf16_t*)vt_pool, part_o, part_ml, scale, keys_per_split, n_splits,   \
+                     qk, m)
   if (qk.on) KAPPAI_DECODE(true, false, false);
   else if (scored && plan) KAPPAI_DECODE(false, true, true);
   else if (scored) KAPPAI_DECODE(false, false, true);
@@ -2197,9 +2242,9 @@ static int launch_decode(const void* q, int q_stride, const void* k_pool, const 
   else KAPPAI_DECODE(false, false, false);
 #undef KAPPAI_DECODE
   hipLaunchKernelGGL(attn_merge_kernel, dim3(T, H), dim3(MERGE_WAVES * WAVE), 0, stream,
-                     (const float*)part_o, (const float*)part_ml, (bf16_t*)out, out_stride, H,
-                     n_splits, row_ids, row_pos, window, m.keep_first, G, keys_per_split,
-                     plan ? (scored ? D_KPW : D_SPLIT_SHARE) : 0, m.sink);
+                     (const float*)part_o, (const float*)part_ml, row_pos, row_ids, H, n_splits, window,
+                     m.keep_first, keys_per_split, plan ? (scored ? D_KPW : D_SPLIT_SHARE) : 0, G,
+                     (bf16_t*)out, out_stride, m.sink);
   KAPPAI_RETURN_LAUNCH_STATUS();
 }
 
@@ -2268,9 +2313,9 @@ extern "C" int kappai_attn_decode_qk(const void* qkv, int row_stride, void* k_po
     if (ps % 16 || G > 65535) return (int)hipErrorInvalidValue;
     const size_t lds = (size_t)n_waves * (H / G * HEAD_DIM + 32) * sizeof(float);
     hipLaunchKernelGGL(attn_decode_block_qk_kernel, dim3(T, G), dim3(n_waves * WAVE), lds, stream,
-                       (const bf16_t*)qkv, row_stride, (const bf16_t*)k_pool,
-                       (const bf16_t*)vt_pool, (bf16_t*)out, out_stride, row_pos, row_seg,
-                       block_tables, max_blocks, H, G, ps, window, scale, qk);
+                       row_pos, row_seg, block_tables, max_blocks, H, G, ps, row_stride, window,
+                       (const bf16_t*)qkv, (const bf16_t*)k_pool, (const bf16_t*)vt_pool, (bf16_t*)out,
+                       out_stride, scale, qk);
     KAPPAI_RETURN_LAUNCH_STATUS();
   }
 #endif

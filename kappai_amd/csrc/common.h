@@ -138,6 +138,27 @@ __device__ __forceinline__ float block_sum(float v, float* red) {
   return t;
 }
 
+// block_sum's result, bit for bit, in a kernel that has one sum: nw whole waves (at most 16), `red` 16 floats on
+// 16 bytes that nothing else uses.  The waves' sums are read four at a time, places behind the last wave hold
+// zeros, and there is no barrier behind the reads.
+__device__ __forceinline__ float block_sum_once(float v, float* red, int nw) {
+  v = wave_sum(v);
+  const int wave = threadIdx.x / WAVE, lane = threadIdx.x % WAVE;
+  if (lane == 0) red[wave] = v;
+  if (wave == 0 && lane >= nw && lane < 16) red[lane] = 0.f;
+  __syncthreads();
+  const float4 a = reinterpret_cast<const float4*>(red)[0];
+  float t = ((a.x + a.y) + a.z) + a.w;
+  if (nw > 4) {
+    const float4 b = reinterpret_cast<const float4*>(red)[1], c = reinterpret_cast<const float4*>(red)[2],
+                 d = reinterpret_cast<const float4*>(red)[3];
+    t = (((t + b.x) + b.y) + b.z) + b.w;
+    t = (((t + c.x) + c.y) + c.z) + c.w;
+    t = (((t + d.x) + d.y) + d.z) + d.w;
+  }
+  return t;
+}
+
 __device__ __forceinline__ float block_max(float v, float* red) {
   v = wave_max(v);
   const int wave = threadIdx.x / WAVE, lane = threadIdx.x % WAVE;

@@ -499,14 +499,17 @@ __global__ __launch_bounds__(P_NW * WAVE, P_MIN_WAVES) void attn_prefill_kernel(
 // The running maximum is only moved when a tile's maximum exceeds it by more than 2^8: most
 // tiles then leave the output accumulators alone (no rescaling), and the weights stay <= 256.
 //
-// Bound by the issue of vector instructions (85 and 32 exponentials for two tiles at head size 64, 0.35 us
-// of them at two waves a SIMD) and by what two waves a SIMD leave uncovered: 2,048 rows are 256 blocks,
-// so the chip has no more.  2,048 rows, 32 heads of 64 on 8: without past 44.1 us (54.1 with values put together
-// from two reads and one loop for masked and whole steps), behind 4,096 keys 128.4 (156.5), behind 9,900
-// 255.9 (307.5: 0.57 PFLOP/s, now 0.69).  Then 2,048 rows at a time to 12,288 keys, mean of a portion: 151 us
-// with the tiles brought by loads through flat addresses and each tile's page by a scalar load (either has
-// every wait for LDS be one for all of it), 140 now.  Priorities for the waves of one tile, for the products or for the
-// exponentials: within 3 %; both tiles' scores ahead of either's exponentials: the same.
+// Bound by the issue of vector instructions: a step (two tiles) of two waves is about 2,000 cycles of them,
+// 32 exponentials of 16 cycles a wave among them, beside 1,280 of products; it takes 2,400.  2,048 rows are
+// 256 blocks, two waves a SIMD, so the chip has no more waves to fill gaps with, and each gap of a wave had
+// to be closed by itself.  2,048 rows, 32 heads of 64 on 8, without past / behind 4,096 keys / behind 9,900:
+//   values put together from two reads, one loop for masked and whole steps      54.1 / 156.5 / 307.5 us
+//   16-byte reads of values, a loop of its own for whole steps                    44 / 130 / 246
+//   tiles by buffer loads, page numbers from a register (see there), half of the
+//   scalar work in front of a tile's loads, LDS asked for ahead of it             40 / 122 / 230
+//   next step's scores among this step's exponentials                             37 / 116 / 217 (0.81 PFLOP/s)
+// At head size 128 (behind 4,096 keys, 16 heads on 4) 176 -> 154 us without the last.  Priorities for the
+// waves of one tile, for the products or for the exponentials: within 3 %.
 #if HEAD_DIM == 64 || HEAD_DIM == 128
 #define PG_OK 1
 #define PG_NBUF 3
@@ -631,20 +634,28 @@ __global__ __launch_bounds__(8 * WAVE) void attn_prefill_shared_kernel(
   // index, offset in the page) and looks the next page up one tile ahead; a group past the
   // last key (or given back by the window) is read from the pool's first page instead and
   // masked when it is used.  A wave's keys (8 of K, 16 of V^T) lie in one page.
+  // All of this is scalar work that a wave does at every tile before its own products, with one other wave to
+  // fill the gap, so it is kept short: a page of K and one of V^T are the same number of bytes, a wave brings
+  // one of the two, and what differs is chosen once.
   int nx_key = kbase + (wave < 4 ? 8 * wave : 16 * v_st);
   int nx_pidx = nx_key / ps, nx_off = nx_key % ps;
+  const int step_pages = 32 / ps, step_off = 32 % ps;
+  const char* const mine =
+      reinterpret_cast<const char*>(wave < 4 ? k_pool : vt_pool) + (size_t)g * ps * HEAD_DIM * sizeof(bf16_t);
+  const size_t page_bytes = (size_t)G * ps * HEAD_DIM * sizeof(bf16_t);
+  const int key_bytes = (int)sizeof(bf16_t) * (wave < 4 ? HEAD_DIM : 1);
   // 64 of the segment's pages, a lane each, and the number of the first: a scalar load a tile would have every
   // wait for LDS wait for it too
   int pages = 0, pages_from = -(1 << 30);
   auto lookup = [&]() {
-    if (nx_key > blk_last) return 0;
     const int at = min(nx_pidx, max_blocks - 1);
-    if (at - pages_from >= WAVE) {
+    if (__builtin_expect(at - pages_from >= WAVE, 0)) {
       pages_from = at;
       pages = bt[min(at + lane, max_blocks - 1)];
       asm volatile("" : "+v"(pages));      // (waits here, and not at every tile for a load that may be under way)
     }
-    return max(__builtin_amdgcn_readlane(pages, at - pages_from), 0);
+    const int page = __builtin_amdgcn_readlane(pages, at - pages_from);
+    return nx_key <= blk_last ? max(page, 0) : 0;
   };
   int nx_page = lookup();
   // (buffer loads: of a global load into LDS the compiler holds that it may be any access to LDS, and waits for
@@ -659,32 +670,21 @@ __global__ __launch_bounds__(8 * WAVE) void attn_prefill_shared_kernel(
     from[i] = 2u * (uint32_t)(wave < 4 ? row * HEAD_DIM + (k_slot ^ swz(8 * wave + row)) * 8
                                        : dd * ps + 8 * (v_half ^ ((dd >> 3) & 1)));
   }
+  const int to = wave < 4 ? 8 * wave * ROWB : KTILE + v_st * VGROUP + (vw % 2) * (HEAD_DIM / 2) * 32;
+  static_assert(K_ROWS_PER * ROWB == 32 * 32, "a load's bytes, of K and of V^T");
   auto issue_one = [&](char* buf) {
 #if defined(__HIP_DEVICE_COMPILE__)
-    const size_t head = (size_t)nx_page * G + g;
-    if (wave < 4) {
-      const __amdgpu_buffer_rsrc_t keys = __builtin_amdgcn_make_buffer_rsrc(
-          const_cast<bf16_t*>(k_pool + (head * ps + nx_off) * HEAD_DIM), 0, 0x7FFFFF00, 0x00020000);
+    const __amdgpu_buffer_rsrc_t keys = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<char*>(mine + (size_t)(uint32_t)nx_page * page_bytes), 0, 0x7FFFFF00, 0x00020000);
 #pragma unroll
-      for (int i = 0; i < NL; ++i)
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(keys, PG_LPTR(buf + (8 * wave + i * K_ROWS_PER) * ROWB), 16,
-                                                 from[i], 0, 0, 0);
-    } else {
-      const __amdgpu_buffer_rsrc_t values = __builtin_amdgcn_make_buffer_rsrc(
-          const_cast<bf16_t*>(vt_pool + head * HEAD_DIM * ps + nx_off), 0, 0x7FFFFF00, 0x00020000);
-#pragma unroll
-      for (int i = 0; i < NL; ++i)
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(
-            values, PG_LPTR(buf + KTILE + v_st * VGROUP + ((vw % 2) * (HEAD_DIM / 2) + 32 * i) * 32), 16, from[i], 0,
-            0, 0);
-    }
+    for (int i = 0; i < NL; ++i)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(keys, PG_LPTR(buf + to + i * 1024), 16, from[i], nx_off * key_bytes,
+                                               0, 0);
 #endif
     nx_key += 32;
-    nx_off += 32;
-    while (nx_off >= ps) {
-      nx_off -= ps;
-      ++nx_pidx;
-    }
+    nx_off += step_off;
+    nx_pidx += step_pages + (nx_off >= ps ? 1 : 0);
+    nx_off -= nx_off >= ps ? ps : 0;
     nx_page = lookup();
   };
   auto issue = [&](auto buf_c) {
@@ -795,24 +795,43 @@ __global__ __launch_bounds__(8 * WAVE) void attn_prefill_shared_kernel(
     }
   };
 
-  // Both tiles of a buffer when neither needs a mask (most steps of a long history): the
-  // products of the second tile's scores are issued before the first tile's exponentials, so
-  // that the matrix cores work while the vector unit does the softmax of the tile before.
-  auto work2 = [&](auto buf_c) {
-    const char* buf0 = lds + (decltype(buf_c)::value * PG_SUB) * BUF;
-    const char* buf1 = buf0 + BUF;
-    auto scores = [&](const char* buf) {
-      f32x16_t s;
+  // Both tiles of a buffer when neither needs a mask (most steps of a long history), a step behind the
+  // scores: `s` holds this step's, and the products of the next step's stand among this step's
+  // exponentials (two waves a SIMD leave a barrier together, so that without this both do products while
+  // the vector unit idles, then both exponentials while the matrix cores do).  All of LDS is asked for
+  // first, and the loads of a later step (`ask`) go out while it answers.
+  f32x16_t s[2];
+  auto keys_of = [&](auto buf_c, u32x4_t (&kf)[2][P_KS]) {
 #pragma unroll
-      for (int v = 0; v < 16; ++v) s[v] = 0.f;
+    for (int sub = 0; sub < 2; ++sub)
 #pragma unroll
-      for (int ks = 0; ks < P_KS; ++ks) {
-        const u32x4_t kf = *reinterpret_cast<const u32x4_t*>(
-            buf + krow * ROWB + (((2 * ks + hh) ^ swz(krow)) * 16));
-        s = __builtin_amdgcn_mfma_f32_32x32x16_bf16(as_frag(kf), qf[ks], s, 0, 0, 0);
-      }
-      return s;
-    };
+      for (int ks = 0; ks < P_KS; ++ks)
+        kf[sub][ks] = *reinterpret_cast<const u32x4_t*>(
+            lds + (decltype(buf_c)::value * PG_SUB + sub) * BUF + krow * ROWB +
+            (((2 * ks + hh) ^ swz(krow)) * 16));
+  };
+  auto scores = [&](const u32x4_t (&kf)[P_KS]) {
+    f32x16_t r;
+#pragma unroll
+    for (int v = 0; v < 16; ++v) r[v] = 0.f;
+#pragma unroll
+    for (int ks = 0; ks < P_KS; ++ks)
+      r = __builtin_amdgcn_mfma_f32_32x32x16_bf16(as_frag(kf[ks]), qf[ks], r, 0, 0, 0);
+    return r;
+  };
+  auto work2 = [&](auto buf_c, auto next_c, auto ask) {
+    u32x4_t kf[2][P_KS], vv[2][2][P_MT];
+    keys_of(next_c, kf);
+#pragma unroll
+    for (int sub = 0; sub < 2; ++sub)
+#pragma unroll
+      for (int st = 0; st < 2; ++st)
+#pragma unroll
+        for (int mt = 0; mt < P_MT; ++mt)
+          vv[sub][st][mt] = *reinterpret_cast<const u32x4_t*>(
+              lds + (decltype(buf_c)::value * PG_SUB + sub) * BUF + KTILE + st * VGROUP + 32 * 32 * mt + v_at);
+    __builtin_amdgcn_sched_barrier(0);
+    ask();
     // the running reference moves only when a tile's maximum is far above it (rare: a branch)
     auto update_reference = [&](const f32x16_t& s) {
       float mloc = -INFINITY;
@@ -838,13 +857,7 @@ __global__ __launch_bounds__(8 * WAVE) void attn_prefill_shared_kernel(
         m_ref = m_new;
       }
     };
-    auto weights_and_output = [&](const char* buf, f32x16_t s) {
-      u32x4_t vv[2][P_MT];
-#pragma unroll
-      for (int st = 0; st < 2; ++st)
-#pragma unroll
-        for (int mt = 0; mt < P_MT; ++mt)
-          vv[st][mt] = *reinterpret_cast<const u32x4_t*>(buf + KTILE + st * VGROUP + 32 * 32 * mt + v_at);
+    auto weights_and_output = [&](const u32x4_t (&vv)[2][P_MT], f32x16_t s) {
       const float m_safe = m_ref == -INFINITY ? 0.f : m_ref;
       float lsum = 0.f;
 #pragma unroll
@@ -869,32 +882,31 @@ __global__ __launch_bounds__(8 * WAVE) void attn_prefill_shared_kernel(
           o[mt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(as_frag(vv[st][mt]), pf, o[mt], 0, 0, 0);
       }
     };
-    // the second tile's score products stand between the first tile's maximum and its
-    // exponentials: nothing in them depends on the other
-    const f32x16_t s0 = scores(buf0);
-    update_reference(s0);
-    const f32x16_t s1 = scores(buf1);
-    weights_and_output(buf0, s0);
-    update_reference(s1);
-    weights_and_output(buf1, s1);
+#pragma unroll
+    for (int sub = 0; sub < 2; ++sub) {
+      update_reference(s[sub]);
+      const f32x16_t now = s[sub];
+      s[sub] = scores(kf[sub]);
+      weights_and_output(vv[sub], now);
+    }
   };
 
   // `it` counts buffers' worth of tiles (PG_SUB each)
   const int n_steps = (n_tiles + PG_SUB - 1) / PG_SUB;
-  auto step = [&](auto buf_c, auto both_whole, int it) {
-    constexpr int B = decltype(buf_c)::value;
-    // the tiles of this step have landed (this wave's part; the barrier makes it everybody's),
-    // those of the next step may still be on their way
-    if (it + 1 < n_steps) __builtin_amdgcn_s_waitcnt(0x0F70 | (PG_SUB * NL));
+  // the tiles of step `it` have landed (this wave's part; the barrier makes it everybody's), and at head
+  // size 64 those of the next step too, which a wave a step ahead with its scores reads: all waves of a
+  // block pass one barrier a step, whichever way they go.  At 128 the next step's may still be on their way.
+  auto arrive = [&](int it) {
+    if (HEAD_DIM != 64 && it + 1 < n_steps) __builtin_amdgcn_s_waitcnt(0x0F70 | (PG_SUB * NL));
     else __builtin_amdgcn_s_waitcnt(0x0F70);
     __builtin_amdgcn_s_barrier();     // no fence: a fence would wait for the loads in flight
+  };
+  auto step = [&](auto buf_c, int it) {
+    constexpr int B = decltype(buf_c)::value;
+    arrive(it);
     // step it+2 goes into the buffer of step it-1: everybody is done with it
     if (it + 2 < n_steps) issue(PgBuf<(B + 2) % PG_NBUF>{});
     const int kb = kbase + 32 * PG_SUB * it;
-    if constexpr (decltype(both_whole)::value != 0) {
-      work2(buf_c);
-      return;
-    }
     if (has_tile && kb + 31 >= lo_tile && kb <= pos_last) work(buf_c, PgBuf<0>{}, PG_SUB * it);
     if (has_tile && kb + 63 >= lo_tile && kb + 32 <= pos_last)
       work(buf_c, PgBuf<1>{}, PG_SUB * it + 1);
@@ -917,16 +929,38 @@ __global__ __launch_bounds__(8 * WAVE) void attn_prefill_shared_kernel(
   }
   const auto steps_to = [&](int end) {
     for (; it < end; it += PG_NBUF) {
-      step(PgBuf<0>{}, PgBuf<0>{}, it);
-      if (it + 1 < n_steps) step(PgBuf<1>{}, PgBuf<0>{}, it + 1);
-      if (it + 2 < n_steps) step(PgBuf<2>{}, PgBuf<0>{}, it + 2);
+      step(PgBuf<0>{}, it);
+      if (it + 1 < n_steps) step(PgBuf<1>{}, it + 1);
+      if (it + 2 < n_steps) step(PgBuf<2>{}, it + 2);
     }
   };
   steps_to(fast_to - fast_from >= PG_NBUF ? fast_from : n_steps);
-  for (; it + PG_NBUF <= fast_to; it += PG_NBUF) {
-    step(PgBuf<0>{}, PgBuf<1>{}, it);
-    step(PgBuf<1>{}, PgBuf<1>{}, it + 1);
-    step(PgBuf<2>{}, PgBuf<1>{}, it + 2);
+  if constexpr (HEAD_DIM == 64) {
+    if (it + PG_NBUF <= fast_to) {
+      auto fast = [&](auto buf_c, int at) {
+        constexpr int B = decltype(buf_c)::value;
+        work2(buf_c, PgBuf<(B + 1) % PG_NBUF>{}, [&]() {
+          if (at + 2 < n_steps) issue(PgBuf<(B + 2) % PG_NBUF>{});
+        });
+      };
+      arrive(it);
+      {
+        u32x4_t kf[2][P_KS];
+        keys_of(PgBuf<0>{}, kf);
+        s[0] = scores(kf[0]);
+        s[1] = scores(kf[1]);
+      }
+      for (;;) {
+        fast(PgBuf<0>{}, it);
+        arrive(it + 1);
+        fast(PgBuf<1>{}, it + 1);
+        arrive(it + 2);
+        fast(PgBuf<2>{}, it + 2);             // (the scores of a step behind the last whole one go unused)
+        it += PG_NBUF;
+        if (it + PG_NBUF > fast_to) break;
+        arrive(it);
+      }
+    }
   }
   steps_to(n_steps);
   if (!row_ok) return;

@@ -4,8 +4,8 @@
 // proj[t] = (B | C | x), each D wide.  bx = B*x;  s_t[c] = bias[c] + sum_k w[c,k] bx_{t-(L-1)+k}[c];
 // out = C * s.  Values before a segment's first row come from the request's state
 // state[slot][c][0..L-2] (oldest first), or are zero when the segment starts at position 0
-// (src/recipe/ops_hybrid.c:353-354).  A second kernel then moves the last L-1 values of bx
-// into the state; segments shorter than L-1 shift the old state through.
+// (src/recipe/ops_hybrid.c:353-354).  The last L-1 values of bx then become the state; segments
+// shorter than L-1 shift the old state through.
 #include "common.h"
 
 // The projection as the kernels below read it: a tensor [T, 3D], or (PartsIn) the float sums
@@ -60,10 +60,6 @@ __global__ void shortconv_out_kernel(IN in, const float* __restrict__ w,
   from_f32(out + (size_t)t * D + c, cg * sum);
 }
 
-// bfloat16, D a multiple of 8, L <= 4: a thread takes 8 channels and a run of SC_RUN rows, 16
-// bytes a load, every load of the run in flight at once.  It carries the last L-1 values of bx
-// from row to row; at the run's first row (and where a new segment begins inside the run) they
-// come from the rows before, or from the state when those lie before the segment.
 #define SC_RUN 4
 #define SC_HMAX 3
 typedef __attribute__((ext_vector_type(4))) uint32_t sc_u32x4_t;
@@ -76,16 +72,136 @@ __device__ __forceinline__ void sc_unpack8(sc_u32x4_t v, float* f) {
   }
 }
 
-// PARTS: the projection comes as float sums over n_parts ranges of its input dimension (see
-// PartsIn); 8 channels of a gate are then two loads of 16 bytes a range, and a thread takes one
-// row only (RUN 1): the steps that come this way have few rows, and the sums are the work.
-template <int L, bool PARTS, int RUN>
-__global__ __launch_bounds__(256) void shortconv_out_vec_kernel(
-    const bf16_t* __restrict__ proj, const float* __restrict__ parts, int n_parts,
-    const float* __restrict__ w, const float* __restrict__ bias,
+// bfloat16, D a multiple of 8, L <= 4: outputs and state in one kernel.  A wave takes 512 channels, 8 a lane,
+// of a run of SC_RUN rows; runs are counted from their segment's first row, so that the run that begins a
+// segment holds every row that reads the old state (SC_RUN > SC_HMAX - 1) and may write the new one behind it,
+// which nobody else touches.  Wave w of a block looks whether a run begins at row SC_RUN * block + w and ends if
+// not: one of the four works in a long segment, all of them where segments are single rows.  16 bytes a load,
+// all of a run's in flight at once, as buffer loads whose bounds stand in for conditions.
+// Bound by its start and its latency: the tables' two dependent scalar reads, then one trip to memory.
+// One after another, against outputs and state in two kernels: 2,048 rows of 2,048 11.1 -> 6.9 us, a portion of
+// 256 rows of 1,024 beside 60 single rows 8.4 -> 3.5, eight portions of 100 rows of 2,048 8.0 -> 3.8.
+template <int L>
+__global__ __launch_bounds__(SC_RUN * WAVE) void shortconv_rows_kernel(
+    const int* __restrict__ row_seg, const int* __restrict__ seg_start, const int* __restrict__ seg_pos0,
+    const int* __restrict__ seg_slot, int T, int D, const bf16_t* __restrict__ proj, const float* __restrict__ w,
+    const float* __restrict__ bias, float* state, bf16_t* __restrict__ out) {
+  constexpr int H = L - 1, NR = SC_RUN + H;
+  const int t = __builtin_amdgcn_readfirstlane((int)(blockIdx.x * SC_RUN + threadIdx.x / WAVE));
+  const int c0 = (blockIdx.y * WAVE + threadIdx.x % WAVE) * 8;
+  if (t >= T) return;
+  const int seg = row_seg[t];
+  const int first = seg_start[seg];
+  if ((t - first) % SC_RUN != 0 || c0 >= D) return;
+  int end = seg_start[seg + 1], pos0 = seg_pos0[seg], slot = seg_slot[seg];
+  asm volatile("" : "+s"(end), "+s"(pos0), "+s"(slot));       // (one wait for the three)
+  const bool opens = t == first, fresh = pos0 == 0;
+  float* st = state + ((size_t)slot * D + c0) * H;
+  const size_t ld = (size_t)3 * D;
+  sc_u32x4_t vb[NR], vx[NR], vc[SC_RUN], tb[H], tx[H];
+#if defined(__HIP_DEVICE_COMPILE__)
+  // (a buffer of no bytes: zeros, nothing read)
+  auto gate = [&](long row, bool in, int part) {
+    const __amdgpu_buffer_rsrc_t from = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<bf16_t*>(proj + row * (long)ld + (size_t)part * D), 0, in ? D * 2 : 0, 0x00020000);
+    return __builtin_bit_cast(sc_u32x4_t, __builtin_amdgcn_raw_buffer_load_b128(from, c0 * 2, 0, 0));
+  };
+#pragma unroll
+  for (int i = 0; i < NR; ++i) {
+    const bool in = t - H + i >= first && t - H + i < end;
+    const long row = (long)t - H + i;
+    vb[i] = gate(row, in, 0);
+    vx[i] = gate(row, in, 2);
+    if (i >= H) vc[i - H] = gate(row, in, 1);
+  }
+  // the rows that become the state, where this run is the one to write it
+#pragma unroll
+  for (int j = 0; j < H; ++j) {
+    const bool in = opens && end - H + j >= first;
+    tb[j] = gate((long)end - H + j, in, 0);
+    tx[j] = gate((long)end - H + j, in, 2);
+  }
+#endif
+  // the 8 channels' taps lie together: 8 L floats from a 16-byte aligned address
+  float wt[8 * L], bs[8];
+  {
+    const float4* wp = reinterpret_cast<const float4*>(w + (size_t)c0 * L);
+#pragma unroll
+    for (int i = 0; i < 2 * L; ++i) {
+      const float4 v = wp[i];
+      wt[4 * i] = v.x, wt[4 * i + 1] = v.y, wt[4 * i + 2] = v.z, wt[4 * i + 3] = v.w;
+    }
+#pragma unroll
+    for (int j = 0; j < 8; ++j) bs[j] = 0.f;
+    if (bias) {
+      const float4 b0 = *reinterpret_cast<const float4*>(bias + c0);
+      const float4 b1 = *reinterpret_cast<const float4*>(bias + c0 + 4);
+      bs[0] = b0.x, bs[1] = b0.y, bs[2] = b0.z, bs[3] = b0.w;
+      bs[4] = b1.x, bs[5] = b1.y, bs[6] = b1.z, bs[7] = b1.w;
+    }
+  }
+  float old[8 * H];                                   // the state, [channel][entry, oldest first]
+#pragma unroll
+  for (int i = 0; i < 8 * H; ++i) old[i] = 0.f;
+  if (opens && !fresh)
+#pragma unroll
+    for (int i = 0; i < 8 * H; ++i) old[i] = st[i];
+  float bx[NR][8];
+#pragma unroll
+  for (int i = 0; i < NR; ++i) {
+    float b[8], x[8];
+    sc_unpack8(vb[i], b);
+    sc_unpack8(vx[i], x);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) bx[i][j] = i < H && opens ? old[j * H + (i < H ? i : 0)] : b[j] * x[j];
+  }
+#pragma unroll
+  for (int r = 0; r < SC_RUN; ++r) {
+    if (t + r >= end) break;
+    float cg[8], res[8];
+    sc_unpack8(vc[r], cg);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) res[j] = bs[j];
+    // tap k meets the row t + r - H + k, which is loaded row r + k; what lies before position 0 counts nothing
+#pragma unroll
+    for (int k = 0; k < L; ++k)
+      if (r + k >= H || !(opens && fresh)) {
+#pragma unroll
+        for (int j = 0; j < 8; ++j) res[j] = fmaf(wt[j * L + k], bx[r + k][j], res[j]);
+      }
+    sc_u32x4_t o;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) o[i] = pack_bf16x2(cg[2 * i] * res[2 * i], cg[2 * i + 1] * res[2 * i + 1]);
+    *reinterpret_cast<sc_u32x4_t*>(out + (size_t)(t + r) * D + c0) = o;
+  }
+  if (!opens) return;
+  // new[j] = bx at the segment's row n - H + j, or old[n + j] when that row lies before the segment
+  const int n = end - first;
+#pragma unroll
+  for (int j = 0; j < H; ++j) {
+    float b[8], x[8];
+    sc_unpack8(tb[j], b);
+    sc_unpack8(tx[j], x);
+#pragma unroll
+    for (int c = 0; c < 8; ++c) {
+      float v = b[c] * x[c];
+#pragma unroll
+      for (int i = j + 1; i < H; ++i) v = n + j == i ? old[c * H + i] : v;
+      st[c * H + j] = v;
+    }
+  }
+}
+
+// The same outputs when the projection comes as float sums over n_parts ranges of its input dimension (see
+// PartsIn; 8 channels of a gate are two loads of 16 bytes a range): a thread takes one row only, the steps
+// that come this way have few rows, and the sums are the work.  The state follows in a kernel of its own.
+template <int L>
+__global__ __launch_bounds__(256) void shortconv_out_parts_kernel(
+    const float* __restrict__ parts, int n_parts, const float* __restrict__ w, const float* __restrict__ bias,
     const float* __restrict__ state, bf16_t* __restrict__ out, const int* __restrict__ row_seg,
     const int* __restrict__ seg_start, const int* __restrict__ seg_pos0,
     const int* __restrict__ seg_slot, int T, int D) {
+  constexpr int RUN = 1;
   constexpr int H = L - 1;
   const int c0 = (blockIdx.y * blockDim.x + threadIdx.x) * 8;
   const int t0 = blockIdx.x * RUN;
@@ -93,7 +209,6 @@ __global__ __launch_bounds__(256) void shortconv_out_vec_kernel(
   const size_t ld = (size_t)3 * D;
   // 8 channels of a gate of one row (at: the row's offset plus the gate's), as bfloat16
   auto gate8 = [&](size_t at) -> sc_u32x4_t {
-    if (!PARTS) return *reinterpret_cast<const sc_u32x4_t*>(proj + at);
     const size_t plane = (size_t)T * ld;
     float4 lo = *reinterpret_cast<const float4*>(parts + at);
     float4 hi = *reinterpret_cast<const float4*>(parts + at + 4);
@@ -298,21 +413,26 @@ static int shortconv_launch(const void* proj, const float* parts, int n_parts, c
   if (is_bf16 && D % 8 == 0 && L <= SC_HMAX + 1 && ((uintptr_t)in_ptr % 16) == 0 &&
       ((uintptr_t)out % 16) == 0 && ((uintptr_t)w % 16) == 0 && (!bias || ((uintptr_t)bias % 16) == 0)) {
     const int groups = D / 8;
-    const int th = groups >= 256 ? 256 : 64;
-    const int run = parts ? 1 : SC_RUN;
-    const dim3 gv((T + run - 1) / run, (groups + th - 1) / th);
-#define SC_LAUNCH_AS(LL, PP)                                                                     \
-  hipLaunchKernelGGL((shortconv_out_vec_kernel<LL, PP, (PP ? 1 : SC_RUN)>), gv, dim3(th), 0, stream, \
-                     (const bf16_t*)proj, parts, n_parts, w, bias, (const float*)state,          \
-                     (bf16_t*)out, row_seg, seg_start, seg_pos0, seg_slot, T, D)
-#define SC_LAUNCH(LL)                                                                            \
-  if (parts) SC_LAUNCH_AS(LL, true);                                                             \
-  else SC_LAUNCH_AS(LL, false)
-    if (L == 2) { SC_LAUNCH(2); }
-    else if (L == 3) { SC_LAUNCH(3); }
-    else { SC_LAUNCH(4); }
+    if (!parts) {
+      const dim3 gr((T + SC_RUN - 1) / SC_RUN, (groups + WAVE - 1) / WAVE);
+#define SC_LAUNCH(LL)                                                                              \
+  hipLaunchKernelGGL(shortconv_rows_kernel<LL>, gr, dim3(SC_RUN * WAVE), 0, stream, row_seg, seg_start, \
+                     seg_pos0, seg_slot, T, D, (const bf16_t*)proj, w, bias, state, (bf16_t*)out)
+      if (L == 2) SC_LAUNCH(2);
+      else if (L == 3) SC_LAUNCH(3);
+      else SC_LAUNCH(4);
 #undef SC_LAUNCH
-#undef SC_LAUNCH_AS
+      KAPPAI_RETURN_LAUNCH_STATUS();
+    }
+    const int th = groups >= 256 ? 256 : 64;
+    const dim3 gv(T, (groups + th - 1) / th);
+#define SC_LAUNCH(LL)                                                                              \
+  hipLaunchKernelGGL(shortconv_out_parts_kernel<LL>, gv, dim3(th), 0, stream, parts, n_parts, w, bias, \
+                     (const float*)state, (bf16_t*)out, row_seg, seg_start, seg_pos0, seg_slot, T, D)
+    if (L == 2) SC_LAUNCH(2);
+    else if (L == 3) SC_LAUNCH(3);
+    else SC_LAUNCH(4);
+#undef SC_LAUNCH
   } else if (parts) {
     hipLaunchKernelGGL((shortconv_out_kernel<bf16_t, PartsIn>), g1, dim3(threads), 0, stream, pin, w,
                        bias, (const float*)state, (bf16_t*)out, row_seg, seg_start, seg_pos0,

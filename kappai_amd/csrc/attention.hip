@@ -426,17 +426,18 @@ __global__ __launch_bounds__(64) void paged_attention_rows_kernel(
 // belongs to wave s % NW wherever a row's keys begin and end) and meet in LDS at the end, so a row's
 // result does not depend on the rows it is computed with.  Scores are made keys x places, which
 // is the layout in which the weights enter the product with the transposed values: nothing moves
-// between lanes but the maximum and the sum of a place.  Bound by the latency of a step's loads, so the next
-// step's are under way while one is worked on.  16 heads of 64 on 8 kv heads: a prompt step of 150, 275 and
-// 400 tokens 43 us, three decoded rows at these lengths 14 us; a wave a (row, head), as before,
-// took 126 us on average over both.
+// between lanes but the maximum and the sum of a place.  Bound by the latency of a step's loads and the chain of
+// products and exponentials behind them, so the next step's loads are under way while one is worked on and the
+// pages they hang on a step before that; the rows' tables are read once, side by side.  One after another, 16
+// heads of 64 on 8 kv heads, with pages looked up on the way to the loads / ahead of them: a prompt step of 150, 275
+// and 400 tokens 41.2 / 39.6 us, of 1,000 443 / 415, three decoded rows at 150 to 400 keys 11.8 / 10.9, four at
+// 4,000 78 / 67; the same bits.  (A wave a (row, head) took 126 us on average over the first and the third.)
 template <int NT>
 __global__ __launch_bounds__((NT <= 4 ? 8 : 4) * WAVE) void paged_attention_f32_kernel(
-    const float* __restrict__ q, int q_stride, const float* __restrict__ k_pool,
-    const float* __restrict__ v_pool, float* __restrict__ out, int out_stride,
-    const int* __restrict__ row_pos, const int* __restrict__ row_seg,
-    const int* __restrict__ block_tables, int max_blocks, int T, int H, int G, int ps, int window,
-    float scale) {
+    const int* __restrict__ row_pos, const int* __restrict__ row_seg, int T, int H, int G, int ps,
+    const int* __restrict__ block_tables, int max_blocks, int q_stride, const float* __restrict__ q,
+    const float* __restrict__ k_pool, const float* __restrict__ v_pool, float* __restrict__ out,
+    int out_stride, int window, float scale) {
   constexpr int D = 16 * NT, NW = NT <= 4 ? 8 : 4;
   __shared__ float part[NW][16][D + 1];
   __shared__ float part_m[NW][16], part_l[NW][16];
@@ -446,18 +447,22 @@ __global__ __launch_bounds__((NT <= 4 ? 8 : 4) * WAVE) void paged_attention_f32_
   // from the first row's first to the last row's own each is then seen by some row, and no page is
   // read that no row needs.  The lanes look at the rows side by side (1,000 rows of one prompt 443 us,
   // 466 with one row after the other).
-  const int t0 = blockIdx.x, seg = row_seg[t0], pos0 = row_pos[t0];
-  if (t0 % R != 0 && row_seg[t0 - 1] == seg && row_pos[t0 - 1] == pos0 - 1)
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE), lane = threadIdx.x % WAVE;
+  const int t0 = blockIdx.x, seen_row = min(max(t0 - 1 + lane, 0), T - 1);     // (lane 0: the row before)
+  const int pos_of = row_pos[seen_row], seg_of = row_seg[seen_row];
+  const int seg = __builtin_amdgcn_readlane(seg_of, 1), pos0 = __builtin_amdgcn_readlane(pos_of, 1);
+  if (t0 % R != 0 && __builtin_amdgcn_readlane(seg_of, 0) == seg &&
+      __builtin_amdgcn_readlane(pos_of, 0) == pos0 - 1)
     return;                                                 // the block of an earlier row has it
-  const int wave = threadIdx.x / WAVE, lane = threadIdx.x % WAVE;
-  bool beside = lane < R - t0 % R && t0 + lane < T;
-  if (beside) beside = row_seg[t0 + lane] == seg && row_pos[t0 + lane] == pos0 + lane;
-  const int t1 = t0 + __builtin_ctzll(~__builtin_amdgcn_ballot_w64(beside));
+  const bool beside = lane >= 1 && lane - 1 < R - t0 % R && t0 - 1 + lane < T && seg_of == seg &&
+                      pos_of == pos0 + lane - 1;
+  const int t1 = t0 + __builtin_ctzll(~(__builtin_amdgcn_ballot_w64(beside) >> 1));
   const int r = lane % 16, quad = lane / 16;
   int row = t0 + r / heads, head = h0 + r % heads;
   if (row >= t1 || head >= (g + 1) * per) row = t0, head = h0;    // a place without work of its own
-  const int pos = row_pos[row], lo = kappai_first_key(pos, window);
-  const int pos_max = wave_max(pos), lo_min = -wave_max(-lo);
+  const int pos = pos0 + (row - t0), lo = kappai_first_key(pos, window);
+  const int pos_max = __builtin_amdgcn_readfirstlane(wave_max(pos));
+  const int lo_min = __builtin_amdgcn_readfirstlane(-wave_max(-lo));
   const int* bt = block_tables + (size_t)seg * max_blocks;
 
   f32x4_t qv[NT], acc[NT], kv[NT], vv[NT];
@@ -467,12 +472,15 @@ __global__ __launch_bounds__((NT <= 4 ? 8 : 4) * WAVE) void paged_attention_f32_
                                               16 * j + 4 * quad);
     acc[j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
   }
-  // keys outside lo_min .. pos_max are read from the nearest one inside (their pages may be gone)
-  const auto fetch = [&](int st, f32x4_t (&kf)[NT], f32x4_t (&vf)[NT]) {
-    const int key = min(max(16 * st + r, lo_min), pos_max);
-    const int four = min(max(16 * st + 4 * quad, lo_min / 4 * 4), pos_max / 4 * 4);
-    const float* kp = k_pool + (((size_t)bt[key / ps] * G + g) * ps + key % ps) * D + 4 * quad;
-    const float* vp = v_pool + (((size_t)bt[four / ps] * G + g) * D + r) * ps + four % ps;
+  // keys outside lo_min .. pos_max are read from the nearest one inside (their pages may be gone); a step's
+  // pages are looked up a step ahead of its loads, which hang on them
+  const auto key_of = [&](int st) { return min(max(16 * st + r, lo_min), pos_max); };
+  const auto four_of = [&](int st) { return min(max(16 * st + 4 * quad, lo_min / 4 * 4), pos_max / 4 * 4); };
+  struct Pages { int k, v; };
+  const auto look_up = [&](int st) { return Pages{bt[key_of(st) / ps], bt[four_of(st) / ps]}; };
+  const auto fetch = [&](int st, const Pages& at, f32x4_t (&kf)[NT], f32x4_t (&vf)[NT]) {
+    const float* kp = k_pool + (((size_t)at.k * G + g) * ps + key_of(st) % ps) * D + 4 * quad;
+    const float* vp = v_pool + (((size_t)at.v * G + g) * D + r) * ps + four_of(st) % ps;
 #pragma unroll
     for (int j = 0; j < NT; ++j) {
       kf[j] = *reinterpret_cast<const f32x4_t*>(kp + 16 * j);
@@ -482,10 +490,13 @@ __global__ __launch_bounds__((NT <= 4 ? 8 : 4) * WAVE) void paged_attention_f32_
   float m = -INFINITY, l = 0.f;
   const int first = lo_min / 16, last = pos_max < 0 ? -1 : pos_max / 16;
   int st = first + ((wave - first) % NW + NW) % NW;
-  if (st <= last) fetch(st, kv, vv);
-  for (; st <= last; st += NW) {
-    f32x4_t kn[NT], vn[NT];
-    if (st + NW <= last) fetch(st + NW, kn, vn);
+  Pages now{0, 0}, next{0, 0};
+  if (st <= last) {
+    now = look_up(st);
+    next = look_up(st + NW);
+    fetch(st, now, kv, vv);
+  }
+  const auto work = [&](const f32x4_t (&kv)[NT], f32x4_t (&vv)[NT]) {
     // (four chains: a product waits 50 clocks for the one before it in its own)
     f32x4_t part_s[4];
 #pragma unroll
@@ -552,11 +563,23 @@ __global__ __launch_bounds__((NT <= 4 ? 8 : 4) * WAVE) void paged_attention_f32_
         }
       }
     }
-#pragma unroll
-    for (int j = 0; j < NT; ++j) {
-      kv[j] = kn[j];
-      vv[j] = vn[j];
-    }
+  };
+  // two sets of registers in turn (copied from one to the other, a step's loads would be waited for at the end
+  // of the step before).  Fetched behind the last step too, where every key is the last row's own: behind a
+  // condition the products of this step would wait for the next one's loads.
+  const auto step = [&](const f32x4_t (&kv)[NT], f32x4_t (&vv)[NT], f32x4_t (&kn)[NT], f32x4_t (&vn)[NT]) {
+    now = next;
+    next = look_up(st + 2 * NW);
+    fetch(st + NW, now, kn, vn);
+    __builtin_amdgcn_sched_barrier(0);
+    work(kv, vv);
+    st += NW;
+  };
+  f32x4_t kn[NT], vn[NT];
+  while (st <= last) {
+    step(kv, vv, kn, vn);
+    if (st > last) break;
+    step(kn, vn, kv, vv);
   }
 #pragma unroll
   for (int j = 0; j < NT; ++j)
@@ -621,9 +644,9 @@ extern "C" int kappai_paged_attention_rows_scored(
 #define F32_ATT(NT)                                                                             \
   case NT:                                                                                      \
     hipLaunchKernelGGL(paged_attention_f32_kernel<NT>, grid, dim3((NT <= 4 ? 8 : 4) * WAVE), 0,  \
-                       stream, (const float*)q, q_stride, (const float*)k_pool,                 \
-                       (const float*)v_pool, (float*)out, out_stride, row_pos, row_seg,         \
-                       block_tables, max_blocks, T, H, G, ps, window, scale);                   \
+                       stream, row_pos, row_seg, T, H, G, ps, block_tables, max_blocks, q_stride, \
+                       (const float*)q, (const float*)k_pool, (const float*)v_pool, (float*)out, \
+                       out_stride, window, scale);                   \
     break;
     switch (d / 16) {
       F32_ATT(1) F32_ATT(2) F32_ATT(3) F32_ATT(4) F32_ATT(5) F32_ATT(6) F32_ATT(7) F32_ATT(8)

@@ -2148,7 +2148,14 @@ extern "C" int kappai_attn_decode_block(const void* q, int q_stride, const void*
 // 1 when the decode kernel of this head size that splits the keys over blocks can do the per-head
 // norm, the rotation and the storing of the rows' own keys and values itself
 // (kappai_attn_decode_qk)
-extern "C" int kappai_attn_decode_takes_qk(void) { return D_QK_FUSABLE ? 1 : 0; }
+// The most rows for which a step does better with kappai_attn_decode_qk than with a kernel for norm, rotation
+// and store ahead of the decode kernels (0: this head size does not take it).  Every wave of a row and kv head
+// does the prologue again.  us, two kernels / one, 32 heads of 64 on 8: 200 keys 5 rows 7.4 / 7.1, 16 rows 7.9 /
+// 7.2; 1,500 keys 8 rows 11.9 / 10.8, 16 rows 17.6 / 15.9; 4,000 keys 8 rows 19.7 / 17.9, 16 rows 30.0 / 28.6;
+// 16 rows of 100 to 7,100 keys 26.6 / 23.2 (more rows come as partial sums, which it does not take).  Heads of 128 have
+// registers for one such wave a SIMD: 5 rows of 4,000 keys 24.1 / 27.3, 8 rows of 1,500 18.0 / 21.1.
+#define D_QK_ROWS (!D_QK_FUSABLE ? 0 : HEAD_DIM == 64 ? 16 : 4)
+extern "C" int kappai_attn_decode_takes_qk(void) { return D_QK_ROWS; }
 
 // The most keys with which kappai_attn_decode_qk keeps a row's keys in one block (0: never at this head
 // size).  One kernel in the place of two, but a CU takes in no more than about 50 GB/s of keys.  1 to 4 rows

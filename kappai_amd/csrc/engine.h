@@ -88,8 +88,8 @@ typedef struct kappai_attention_kernels {
                           const int*, const int*, const int*, const int*, int, int, int, int, int,
                           int, float, int, int, hipStream_t);
   // the decode kernel that splits the keys over blocks, with the per-head norm, the rotation and
-  // the store of the rows' own keys and values in its prologue (decode_takes_qk() says whether
-  // this head size has it)
+  // the store of the rows' own keys and values in its prologue (decode_takes_qk(): for how many rows a step
+  // does better with it, 0 where this head size does not have it)
   int (*decode_takes_qk)(void);
   // the most keys with which attn_decode_qk keeps a row's keys in one block, 0: never
   int (*decode_block_qk_keys)(void);

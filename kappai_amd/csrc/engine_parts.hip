@@ -202,11 +202,11 @@ kappai_carry attention_mixer(kappai_step* s, const void* desc, kappai_rows x, fl
   const bool single = b.max_segment_rows == 1;
   // decode: the attention kernels take the projection as it is and do norm, rotation and store
   // themselves (parts/attention.py: _prologue_in_kernel)
+  const int qk_rows = L.mfma != nullptr && L.mfma->decode_takes_qk != nullptr ? L.mfma->decode_takes_qk() : 0;
   const bool qk_in_kernel =
-      M <= tune.fused_qk && single && proj.kind == KAPPAI_CARRY_DELTA && !proj.is_f32 &&
+      M <= tune.fused_qk && M <= qk_rows && single && proj.kind == KAPPAI_CARRY_DELTA && !proj.is_f32 &&
       L.mfma != nullptr && H / G <= 16 && qkv.n % 8 == 0 && aligned16(proj.data) && ps % 16 == 0 &&
       d % 16 == 0 && d <= 256 && (L.rot_mode == 0 || (L.rot_mode == 1 && L.rot_dim == d)) &&
-      L.mfma->decode_takes_qk != nullptr && L.mfma->decode_takes_qk() &&
       (!decode_block_form(m, b, L, M) ||
        (L.mfma->decode_block_qk_keys != nullptr &&
         decode_keys(b, L) <= L.mfma->decode_block_qk_keys()));

@@ -964,12 +964,18 @@ def decode_form(n_heads: int, n_kv_heads: int, head_dim: int, max_position: int,
     return "decode-block" if block_waves and n_keys <= most else "decode-split"
 
 
+def decode_qk_rows(head_dim: int, page_size: int) -> int:
+    """The most rows for which a step does better with a ``QkPrologue`` than with a kernel of its own for that
+    work (0: the decode attention kernels of this head size do not take one)."""
+    if head_dim % 16 or head_dim > 256 or page_size % 16:
+        return 0
+    return int(library("attention_mfma", HEAD_DIM=head_dim).kappai_attn_decode_takes_qk())
+
+
 def decode_takes_qk(head_dim: int, page_size: int) -> bool:
     """Whether the decode attention kernels of this head size take a ``QkPrologue`` (head sizes
     64 and 128: a lane holds both halves of a rotation pair, and the registers the prologue)."""
-    if head_dim % 16 or head_dim > 256 or page_size % 16:
-        return False
-    return bool(library("attention_mfma", HEAD_DIM=head_dim).kappai_attn_decode_takes_qk())
+    return decode_qk_rows(head_dim, page_size) > 0
 
 
 def decode_block_takes_qk(head_dim: int, max_position: int, window: int = 0) -> bool:

@@ -59,12 +59,13 @@ def fused_conv_step(width: int, rows: int, in_fragments: bool) -> bool:
 
 # A decode step's attention kernel normalises and rotates q and the row's own key itself and
 # stores key and value (head sizes 64 and 128, rotate-half over the whole head, a projection that
-# comes as bfloat16 rows, more than 512 keys or head size 64) for steps of up to FUSED_QK_MAX_ROWS rows: every
-# wave of the kernel does that work again, which a few hundred waves do faster than a kernel of
-# its own would (a step of the 1.2B shape: 10 us less at 1 to 4 rows) and a thousand or more do
-# not (7 us more at 6 rows, 12 at 8, 40 at 12).  0 switches it off.
+# comes as bfloat16 rows, more than 512 keys or head size 64) for steps of up to FUSED_QK_MAX_ROWS rows and
+# no more than the kernel itself says (``ops.decode_qk_rows``: 16 at head size 64, 4 at 128): every wave of the
+# kernel does that work again, beside its first keys' way.  A step of six such layers, 8 rows at 60 to 7,000 keys: 0
+# to 10 us less; at 12 and 16 rows 1 to 13.  (Until its arguments came in the order of need the line was at 4: 12 us
+# more at 8 rows.)  0 switches it off.
 FUSED_QK = True
-FUSED_QK_MAX_ROWS = 4
+FUSED_QK_MAX_ROWS = 16
 
 # In a step that holds prompt portions, a single decoded token is one tile for the tiled attention
 # kernel, and the block that gets it walks all its keys alone: 0.9 ms at 32 k keys, however short

@@ -232,7 +232,7 @@ class GroupedQueryAttention(Mixer):
         if rot is not None and not (rot.mode == ops.ROT_HALF and rot.rot_dim == self.d):
             return False
         window = self.window or 0
-        return (ops.decode_takes_qk(self.d, page_size)
+        return (proj.shape[0] <= ops.decode_qk_rows(self.d, page_size)
                 and (ops.decode_form(self.H, self.G, self.d, max_position, window,
                                      n_rows=proj.shape[0]) == "decode-split"
                      or ops.decode_block_takes_qk(self.d, max_position, window)))

@@ -1,0 +1,22 @@
+"""Decode steps of 5 to 16 rows whose attention kernel normalises, rotates and stores: the same comparison
+as for a few rows (the two kernels, their pools and outputs), at the most rows the rule sends that way, over
+requests of one length and of mixed lengths, in one block and split."""
+import pytest
+
+import test_kernels_gpu as kernels
+from test_kernels_gpu import ops  # noqa: F401
+
+pytestmark = pytest.mark.gpu
+
+
+def test_where_the_rule_lies(ops):  # noqa: F811
+    assert [ops.decode_qk_rows(d, 16) for d in (64, 128, 48, 256)] == [16, 4, 0, 0]
+    assert ops.decode_qk_rows(64, 8) == 0
+
+
+@pytest.mark.parametrize("H,G", [(32, 8), (16, 8), (4, 1)])
+@pytest.mark.parametrize("held", [[200] * 16, [1500] * 5, [1023, 1024] * 8, [40 + i * i * 13 for i in range(16)]])
+def test_the_most_rows(ops, H, G, held):  # noqa: F811
+    for kernel in ("decode-split",) + (("auto",) if max(held) < 512 else ()):           # (auto: in one block)
+        kernels.test_decode_attention_with_norm_rotation_and_store_inside(
+            ops, (H, G, 64, 16, held, True, True, 0, True), kernel=kernel)

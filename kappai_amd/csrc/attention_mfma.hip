@@ -897,9 +897,12 @@ __global__ __launch_bounds__(8 * WAVE) void attn_prefill_shared_kernel(
   // size 64 those of the next step too, which a wave a step ahead with its scores reads: all waves of a
   // block pass one barrier a step, whichever way they go.  At 128 the next step's may still be on their way.
   auto arrive = [&](int it) {
-    if (HEAD_DIM != 64 && it + 1 < n_steps) __builtin_amdgcn_s_waitcnt(0x0F70 | (PG_SUB * NL));
-    else __builtin_amdgcn_s_waitcnt(0x0F70);
-    __builtin_amdgcn_s_barrier();     // no fence: a fence would wait for the loads in flight
+    // Everything read of LDS is in registers too: the tiles of step it - 1 are written over behind the barrier.
+    // (No fence: a fence would wait for the loads in flight.)
+    if (HEAD_DIM != 64 && it + 1 < n_steps) __builtin_amdgcn_s_waitcnt(0x0070 | (PG_SUB * NL));
+    else __builtin_amdgcn_s_waitcnt(0x0070);
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
   };
   auto step = [&](auto buf_c, int it) {
     constexpr int B = decltype(buf_c)::value;
@@ -1168,10 +1171,12 @@ __global__ __launch_bounds__(8 * WAVE) void attn_prefill_heads_kernel(
     __builtin_amdgcn_sched_barrier(0);
     constexpr int B = decltype(buf_c)::value;
     if (it + 2 < n_steps) lookup();
-    // this step's tile has landed (this wave's part; the barrier makes it everybody's)
-    if (it + 1 < n_steps) __builtin_amdgcn_s_waitcnt(0x0F70 | NL);
-    else __builtin_amdgcn_s_waitcnt(0x0F70);
-    __builtin_amdgcn_s_barrier();     // no fence: a fence would wait for the loads in flight
+    // this step's tile has landed (this wave's part; the barrier makes it everybody's), and what was read of
+    // the step before (no fence: a fence would wait for the loads in flight)
+    if (it + 1 < n_steps) __builtin_amdgcn_s_waitcnt(0x0070 | NL);
+    else __builtin_amdgcn_s_waitcnt(0x0070);
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
     // step it + 2 goes into the buffer of step it - 1: everybody is done with it
     if (it + 2 < n_steps) issue(PhBuf<(B + 2) % PH_NBUF>{});
     work(buf_c, kbase + 32 * it);

@@ -2214,9 +2214,11 @@ extern "C" int kappai_attn_prefill_scored(const void* q, int q_stride, const voi
   const int rep = H / G;
   const bool shared_ok = PG_OK && rep % 4 == 0;
   if (variant == 2 && !shared_ok) return (int)hipErrorInvalidValue;
+  // (the kernels over shared key tiles keep offsets of 31 bits within a kv head's part of a page)
+  const bool near = (size_t)ps * HEAD_DIM * sizeof(bf16_t) < 0x7FFFFF00u;
   // sharing pays when there are blocks enough to fill the chip without splitting the keys of
   // a q tile over waves
-  const bool shared = variant == 2 || (variant == 0 && shared_ok && n_tiles * (H / 4) >= 256);
+  const bool shared = near && (variant == 2 || (variant == 0 && shared_ok && n_tiles * (H / 4) >= 256));
 #if PG_OK
   if (shared) {
     hipLaunchKernelGGL(attn_prefill_shared_kernel, dim3(n_tiles, H / 4), dim3(8 * WAVE), 0, stream,
@@ -2230,7 +2232,7 @@ extern "C" int kappai_attn_prefill_scored(const void* q, int q_stride, const voi
   // (from the first tile on.  us with / without, 16 heads on one kv head: one portion of 5 rows 6.9 /
   // 8.7, of 32 rows 11.1 / 10.1 (the worst there is: a key tile or two that are full, on an empty chip), of
   // 32 rows behind 2,000 keys 131 / 165; 64 lone rows of 32 keys 6.9 / 10.0, 63 of 800 keys 64 / 126)
-  if (variant == 0 && rep % 4 == 0) {
+  if (near && variant == 0 && rep % 4 == 0) {
     hipLaunchKernelGGL(attn_prefill_heads_kernel, dim3(n_tiles, H / 4), dim3(8 * WAVE), 0, stream,
                        q_tiles, row_pos, block_tables, max_blocks, H, G, ps, q_stride, window,
                        (const bf16_t*)q, (const bf16_t*)k_pool, (const bf16_t*)vt_pool, (bf16_t*)out,

@@ -43,3 +43,24 @@ def test_histories_around_the_rounds_of_buffers(ops, H, G, D, ps, n_new, window)
                               max_position=max(pos), kernel="prefill", prefill_variant=2)
     want = ops.paged_attention(*args, window=window, kernel="rows")
     close(got.float(), want.float().cpu().double(), 2 * BF16_ULP, "tiles shared through LDS")
+
+
+@pytest.mark.parametrize("D,ps", [(64, (1 << 24) + (1 << 19)), (128, (1 << 23) + (1 << 17)), (256, (1 << 22) + (1 << 16))])
+def test_pages_of_more_than_two_gibibytes(ops, D, ps):  # noqa: F811
+    """A kv head's part of a page so large that the last places of its values lie behind 2 GiB."""
+    assert (D - 1) * ps * 2 > 1 << 31
+    g = torch.Generator().manual_seed(D)
+    T, H, held = 40, 4, 70
+    q, k, v = (torch.randn(n, D, generator=g).to(BF16) for n in (T * H, held + T, held + T))
+    k_pool = torch.full((1, 1, ps, D), float("nan"), dtype=BF16, device=DEV)
+    vt_pool = torch.full((1, 1, D, ps), float("nan"), dtype=BF16, device=DEV)
+    k_pool[0, 0, :held + T] = k.to(DEV)
+    vt_pool[0, 0, :, :held + T] = v.T.to(DEV)
+    ints = [torch.tensor(x, dtype=torch.int32, device=DEV)
+            for x in (range(held, held + T), [0] * T, [[0]], [(0, 0, 32, 0 | 2 << 16), (0, 32, T - 32, 1 | 2 << 16)])]
+    got = ops.paged_attention(q.view(T, H * D).to(DEV), H, 1, D, k_pool, vt_pool, *ints[:3], ps, D ** -0.5,
+                              q_tiles=ints[3], max_position=held + T - 1, kernel="prefill",
+                              prefill_variant=0 if D == 256 else 2)
+    s = q.view(T, H, D).double() @ k.double().T * D ** -0.5
+    s.masked_fill_(torch.arange(held + T) > (held + torch.arange(T))[:, None, None], float("-inf"))
+    close(got.float(), (s.softmax(2) @ v.double()).view(T, H * D), 2 * BF16_ULP, "large pages")

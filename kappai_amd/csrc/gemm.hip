@@ -2066,21 +2066,31 @@ __global__ __launch_bounds__(NW * WAVE) void gemm_bf16_into_resid_kernel(
   const u32x4_t zero = {0u, 0u, 0u, 0u};
   // What the epilogue needs, asked for before the stream of W: offsets outside the buffers for lanes that
   // need nothing, since of loads in branches the compiler waits for the first before it asks for the next.
+  // (FRAG: the residual's offsets have 31 bits, see the launch.)
   float resid_in[4] = {0.f, 0.f, 0.f, 0.f};
   float norm_w_in = 0.f;
 #if defined(__HIP_DEVICE_COMPILE__)
-  if (wave == 0) {
-    const bool mine = half == 0 && gn < N;
+  const bool wanted = half == 0 && gn < N;
+  const bool near = FRAG || ((uint64_t)(M - 1) * ldr + N) * 4 < 0x7FFFFF00u;
+  if (wave == 0 && near) {
     const __amdgpu_buffer_rsrc_t res = raw_buffer(resid, 0x7FFFFF00u);
     const __amdgpu_buffer_rsrc_t nw = raw_buffer(norm_w, rows != nullptr ? (uint32_t)N * 4u : 0u);
 #pragma unroll
     for (int v = 0; v < 4; ++v) {
       const int gm = 4 * (lane / 16) + v;
       resid_in[v] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(
-          res, mine && gm < M ? (gm * ldr + gn) * 4 : 0x7FFFFF00, 0, 0));
+          res, wanted && gm < M ? (gm * ldr + gn) * 4 : 0x7FFFFF00, 0, 0));
     }
     norm_w_in = __builtin_bit_cast(
-        float, __builtin_amdgcn_raw_buffer_load_b32(nw, mine ? gn * 4 : 0x7FFFFF00, 0, 0));
+        float, __builtin_amdgcn_raw_buffer_load_b32(nw, wanted ? gn * 4 : 0x7FFFFF00, 0, 0));
+  }
+  if (wave == 0 && !near && wanted) {
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+      const int gm = 4 * (lane / 16) + v;
+      if (gm < M) resid_in[v] = resid[(size_t)gm * ldr + gn];
+    }
+    if (rows != nullptr) norm_w_in = norm_w[gn];
   }
 #endif
   const size_t wr = gn < N ? gn : 0;
@@ -2196,9 +2206,9 @@ static void launch_into_resid(const bf16_t* A, const bf16_t* W, const float* bia
   const int w_frag = Wf != nullptr;
   if (Wf) W = Wf;
   const dim3 grid((N + 7) / 8);
-  // (both halves of K whole pieces and offsets of 31 bits: the loads without conditions)
+  // (both halves of K whole pieces and offsets of 31 bits, into the stream too: the loads without conditions)
   const bool pieces = w_frag && K % 64 == 0 && ((size_t)M * lda + K) * 2 < 0x7FFFFF00u &&
-                      (size_t)K * 32 < 0x7FFFFF00u;
+                      (size_t)K * 32 < 0x7FFFFF00u && ((size_t)(M - 1) * ro.ldr + N) * 4 < 0x7FFFFF00u;
 #define INTO_RESID(NW)                                                                                 \
   do {                                                                                                 \
     if (pieces)                                                                                        \

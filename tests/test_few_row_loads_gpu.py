@@ -2,6 +2,8 @@
 leaves waves with few pieces or none, column groups behind the last, rows behind M, the sums of squares of
 narrow and wide norms, and memory full of NaN on every side of what they may read.  Results against float64
 within the bound of a float sum of K products, gamma_K = K 2^-24 of the sum of magnitudes."""
+import ctypes
+
 import pytest
 import torch
 
@@ -124,3 +126,31 @@ def test_conv_step(M, D, L):
     rest = torch.ones(M + 3, dtype=torch.bool, device=DEV)
     rest[slots.long()] = False
     assert torch.equal(state[rest], before[rest])
+
+
+@pytest.mark.parametrize("in_fragments", [True, False])
+def test_into_a_stream_of_more_than_two_gibibytes(in_fragments):
+    """Sixteen rows of a stream so far apart that the last lies behind 2 GiB: each is added to where it stands."""
+    from kappai_amd.kernels.lib import library
+    M, N, K, ldr = 16, 64, 64, 36_000_000
+    assert (M - 1) * ldr * 4 > 1 << 31
+    g = _gen(M, N, K, 9)
+    x = _rows(M, K, g)
+    W, w = _matrix(N, K, g)
+    want, bound = _sums(x, w)
+    flat = torch.empty((M - 1) * ldr + N, device=DEV)
+    resid = flat.as_strided((M, N), (ldr, 1))
+    resid.copy_(torch.randn(M, N, generator=g, device=DEV) * 10)
+    before = resid.double()
+    norm = torch.rand(N, generator=g, device=DEV) + 0.5
+    rows = torch.empty(M, N, device=DEV, dtype=BF16)
+    ss = torch.empty(N // 8, 16, device=DEV)
+    vp, ci, cf = ctypes.c_void_p, ctypes.c_int, ctypes.c_float
+    rc = library("gemm").kappai_gemm_bf16(
+        vp(x.data_ptr()), vp(0 if in_fragments else w.data_ptr()), vp(W.data_ptr() if in_fragments else 0), vp(0),
+        vp(0), ci(M), ci(N), ci(K), ci(x.stride(0)), ci(N), ci(1), ci(0), ci(1), ci(0), vp(0), ci(0), cf(0.0),
+        vp(resid.data_ptr()), ci(ldr), vp(norm.data_ptr()), vp(rows.data_ptr()), ci(0), vp(ss.data_ptr()),
+        vp(torch.cuda.current_stream().cuda_stream))
+    assert rc == 0
+    assert ((resid.double() - before - want).abs() <= bound + resid.double().abs() * 2.0 ** -24).all().item()
+    assert torch.equal(rows, (resid * norm).to(BF16))

@@ -1803,13 +1803,15 @@ void gemm_bf16_skinny_kernel(
   const bool channel = gn < N && (EPI != 3 || col < 8);
 #if defined(__HIP_DEVICE_COMPILE__)
   if (CONV && wave < MT) {
-    // (buffer loads: an offset outside the buffer, or a buffer of no bytes, gives 0 and needs no branch)
+    // (buffer loads: an offset outside the buffer, or a buffer of no bytes, gives 0 and needs no branch.  The
+    // channels' buffers begin with the block's first, so that there may be any number of them.)
     constexpr int OUT = 0x7FFFFF00;
+    const int c = gn - n0;
     const auto word = [](const void* p, uint32_t bytes, int at) {
       return __builtin_amdgcn_raw_buffer_load_b32(raw_buffer(p, bytes), at, 0, 0);
     };
-    const auto number = [&](const void* p, uint32_t bytes, int at) {
-      return __builtin_bit_cast(float, word(p, bytes, at));
+    const auto number = [&](const float* p, size_t first, uint32_t bytes, int at) {
+      return __builtin_bit_cast(float, word(p + first, p != nullptr ? bytes : 0u, at));
     };
 #pragma unroll
     for (int v = 0; v < 4; ++v) {
@@ -1819,11 +1821,11 @@ void gemm_bf16_skinny_kernel(
     }
 #pragma unroll
     for (int k = 0; k <= CONV_PRE; ++k)
-      tap_pre[k] = number(cs.taps, (uint32_t)N * cs.L * 4u, channel && k < cs.L ? (gn * cs.L + k) * 4 : OUT);
-    conv_bias_pre = number(cs.conv_bias, cs.conv_bias ? N * 4u : 0u, channel ? gn * 4 : OUT);
+      tap_pre[k] = number(cs.taps, (size_t)n0 * cs.L, 16u * cs.L * 4u, channel && k < cs.L ? (c * cs.L + k) * 4 : OUT);
+    conv_bias_pre = number(cs.conv_bias, n0, 64u, channel ? c * 4 : OUT);
 #pragma unroll
     for (int g = 0; g < 3; ++g)
-      gate_bias_pre[g] = number(bias, bias ? N * 12u : 0u, channel ? (g * N + gn) * 4 : OUT);
+      gate_bias_pre[g] = number(bias, (size_t)g * N + n0, 64u, channel ? c * 4 : OUT);
   }
 #endif
   const auto ask_for_state = [&]() {

@@ -154,3 +154,29 @@ def test_into_a_stream_of_more_than_two_gibibytes(in_fragments):
     assert rc == 0
     assert ((resid.double() - before - want).abs() <= bound + resid.double().abs() * 2.0 ** -24).all().item()
     assert torch.equal(rows, (resid * norm).to(BF16))
+
+
+def test_conv_step_of_very_many_channels():
+    """So many channels that their taps take more than 4 GiB: the last sixteen of them, on a matrix that is zero
+    for all others."""
+    D, K, L = 220_000_000, 8, 5
+    assert D * L * 4 > 1 << 32
+    g = _gen(D, 5)
+    w = torch.zeros(3, D, K, device=DEV, dtype=BF16)
+    taps, conv_bias, bias = (torch.empty(*n, device=DEV) for n in ((D, L), (D,), (3, D)))
+    state = torch.empty(1, D, L - 1, device=DEV)
+    for t in (w[:, -16:], taps[-16:], conv_bias[-16:], bias[:, -16:], state[:, -16:]):
+        t.copy_(torch.randn(t.shape, generator=g, device=DEV))
+    x = torch.randn(1, K, generator=g, device=DEV).to(BF16)
+    old = state[0, -16:].double()
+    got = ops.linear_shortconv_step(x, w.view(3 * D, K), bias.view(-1), taps, conv_bias, state,
+                                    torch.ones(1, dtype=torch.int32, device=DEV),
+                                    torch.zeros(1, dtype=torch.int32, device=DEV))
+    b, c, u = ((w[i, -16:].double() * x.double()).sum(1) + bias[i, -16:].double() for i in range(3))
+    b, c, u = (v.float().to(BF16).double() for v in (b, c, u))
+    window = torch.cat([old, (b * u)[:, None]], 1)
+    terms = window * taps[-16:].double()
+    want = c * (terms.sum(1) + conv_bias[-16:].double())
+    # (a gate may round the other way: 2^-7 of it; the result's own rounding beside that)
+    slack = c.abs() * (4 * 2.0 ** -7 * (terms.abs().sum(1) + conv_bias[-16:].double().abs()))
+    assert ((got[0, -16:].double() - want).abs() <= slack).all().item()

@@ -746,7 +746,9 @@ template <typename T, typename TD, int NP>
 __global__ __launch_bounds__(1024) void add_rmsnorm_row_kernel(
     float* __restrict__ resid, const float* __restrict__ w, const TD* __restrict__ delta,
     const int* __restrict__ rows, T* __restrict__ out, int D, uint32_t pstride, int flags, float eps) {
-  const int n_part = flags >> 2, write_resid = flags & 1, out_frag = flags & 2;
+  // (flags: from bit 8 on the upper part of the planes' distance, so that all arguments are 14 words)
+  const int n_part = flags >> 2 & 15, write_resid = flags & 1, out_frag = flags & 2;
+  const size_t plane = ((size_t)(flags >> 8) << 32) + pstride;
   __shared__ __attribute__((aligned(16))) float red[16];
   const int i = blockIdx.x;
   const int r = rows ? rows[i] : i;
@@ -761,7 +763,7 @@ __global__ __launch_bounds__(1024) void add_rmsnorm_row_kernel(
     if (NP) {
 #pragma unroll
       for (int p = 0; p < NP; ++p)
-        if (p < n_part || NP <= 4) load8(dl + (size_t)p * pstride + j, d8[p]);
+        if (p < n_part || NP <= 4) load8(dl + p * plane + j, d8[p]);
       load8(w + j, w8);
 #pragma unroll
       for (int p = 0; p < NP; ++p)
@@ -796,12 +798,13 @@ template <typename T, typename TD>
 static void launch_add_rmsnorm(float* resid, const void* delta, int n_part, size_t pstride,
                                const float* w, void* out, const int* rows, int n_rows, int D,
                                float eps, int write_resid, int out_frag, hipStream_t stream) {
-  if (D % 8 == 0 && D <= 8192 && n_part <= RN_MAX_PART && (n_part == 1 || pstride <= 0xFFFFFFFFu)) {
+  if (D % 8 == 0 && D <= 8192 && n_part <= RN_MAX_PART) {
     const int threads = ((D / 8 + WAVE - 1) / WAVE) * WAVE;
 #define KAPPAI_NORM_ROW(NP)                                                                       \
   hipLaunchKernelGGL((add_rmsnorm_row_kernel<T, TD, NP>), dim3(n_rows), dim3(threads), 0, stream, \
-                     resid, w, (const TD*)delta, rows, (T*)out, D, (uint32_t)pstride,                \
-                     n_part << 2 | (out_frag ? 2 : 0) | (write_resid ? 1 : 0), eps)
+                     resid, w, (const TD*)delta, rows, (T*)out, D, (uint32_t)pstride,             \
+                     (int)((uint32_t)(pstride >> 32) << 8 | n_part << 2 | (out_frag ? 2 : 0) | (write_resid ? 1 : 0)), \
+                     eps)
     constexpr bool planes = sizeof(TD) == 4;                  // (partial sums are float)
     if (delta == nullptr) KAPPAI_NORM_ROW(0);
     else if (n_part == 1 || !planes) KAPPAI_NORM_ROW(1);
@@ -827,8 +830,7 @@ extern "C" int kappai_add_rmsnorm(float* resid, const void* delta, int delta_is_
   if (n_part < 1 || (n_part > 1 && !delta_is_f32)) return (int)hipErrorInvalidValue;
   // rows in fragment order: bfloat16, at most 16 of them, in the kernel that keeps a row in
   // registers; out holds 16 x D values
-  if (out_frag && (!is_bf16 || n_rows > 16 || (D % 32) || D > 8192 || n_part > RN_MAX_PART ||
-                   (n_part > 1 && (unsigned long)pstride > 0xFFFFFFFFul)))
+  if (out_frag && (!is_bf16 || n_rows > 16 || (D % 32) || D > 8192 || n_part > RN_MAX_PART))
     return (int)hipErrorInvalidValue;
   if (!is_bf16)
     launch_add_rmsnorm<float, float>(resid, delta, n_part, (size_t)pstride, w, out, rows, n_rows,

@@ -68,3 +68,28 @@ def test_norm_of_a_result_of_partial_sums(parts, D, second, add):
     want = n + resid.double() if add else n
     bounded(dev, want, NORM * n.abs() + 2.0 ** -24 * want.abs(), F32, "stream")
     assert torch.equal(rows.cpu(), dev.cpu().to(BF16))
+
+
+@pytest.mark.parametrize("fragment", [0, 1])
+def test_planes_more_than_sixteen_gigabytes_apart(fragment):
+    """Two planes 2^32 + 64 values apart (16 rows picked of a projection of a million rows) give the bits of two
+    planes side by side, in fragment order too."""
+    import ctypes
+    from kappai_amd.kernels.lib import library
+    T, D, apart = 16, 2048, (1 << 32) + 64
+    resid, w, planes = rand(1, T, D).to(DEV), (1 + rand(2, D, scale=0.2)).to(DEV), rand(3, 2, T, D).to(DEV)
+    far = torch.empty(apart + T * D, device=DEV)
+    far[:T * D], far[apart:] = planes[0].flatten(), planes[1].flatten()
+
+    def norm(delta, distance):
+        x, out = resid.clone(), torch.empty(T, D, device=DEV, dtype=BF16)
+        vp, ci = ctypes.c_void_p, ctypes.c_int
+        rc = library("elementwise").kappai_add_rmsnorm(
+            vp(x.data_ptr()), vp(delta.data_ptr()), ci(1), ci(2), ctypes.c_long(distance), vp(w.data_ptr()),
+            vp(out.data_ptr()), vp(0), ci(T), ci(D), ctypes.c_float(1e-5), ci(1), ci(1), ci(fragment),
+            vp(torch.cuda.current_stream().cuda_stream))
+        assert rc == 0
+        return x, out
+
+    for got, want in zip(norm(far, apart), norm(planes, T * D)):
+        assert torch.equal(got, want)

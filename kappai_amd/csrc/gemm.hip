@@ -31,6 +31,18 @@ typedef __attribute__((ext_vector_type(4))) uint32_t u32x4_t;
 #define KAPPAI_GPTR(p) ((const __attribute__((address_space(1))) void*)(p))
 #define KAPPAI_LPTR(p) ((__attribute__((address_space(3))) void*)(p))
 
+#define SCHED_FENCE() __builtin_amdgcn_sched_barrier(0)
+// (nothing that touches memory is moved across, by any pass of the compiler)
+#define ORDER_FENCE()                  \
+  do {                                 \
+    asm volatile("" ::: "memory");     \
+    __builtin_amdgcn_sched_barrier(0); \
+  } while (0)
+// waits until at most `behind` loads are under way (_AND_LDS: and no LDS access is)
+#define WAIT_LOADS(behind) __builtin_amdgcn_s_waitcnt(0x0F70 | ((behind) & 15) | ((behind) >> 4 << 14))
+#define WAIT_LOADS_AND_LDS(behind) \
+  __builtin_amdgcn_s_waitcnt(0x0070 | ((behind) & 15) | ((behind) >> 4 << 14))
+
 // A buffer of `bytes` bytes from p on: loads whose lane's and scalar offset together lie outside it read
 // nothing and give zeros, so a loop's last loads need no branch.  (The type is the device compiler's; the host
 // pass sees neither it nor the loads.)
@@ -386,9 +398,9 @@ void gemm_f32_block_kernel(
     static_assert(F32_CHUNK == 2 * BK, "a chunk is a tile in either buffer");
     bring(0);
     bring(1);
-    __builtin_amdgcn_s_waitcnt(0x0070 | LOADS_A_WAVE);         // tile 0 is there
+    WAIT_LOADS_AND_LDS(LOADS_A_WAVE);                          // tile 0 is there
     __builtin_amdgcn_s_barrier();
-    __builtin_amdgcn_sched_barrier(0);
+    ORDER_FENCE();
     read(0, 0);
     for (int chunk = 0; chunk < chunks; ++chunk) {
       f32x4_t acc[TY][TX];
@@ -409,9 +421,10 @@ void gemm_f32_block_kernel(
         // The tile's last fragments are in registers: its buffer takes the tile after the next, and the
         // next one's first fragments come while the last of this one are multiplied.  (Behind the last tile
         // too: what is read there is not used, but a branch would have the products wait for it.)
-        __builtin_amdgcn_s_waitcnt(0x0070);                    // no load of either kind under way
+        ORDER_FENCE();
+        WAIT_LOADS_AND_LDS(0);
         __builtin_amdgcn_s_barrier();
-        __builtin_amdgcn_sched_barrier(0);
+        ORDER_FENCE();
         if (t + 2 < tiles) bring(t + 2);
         read(u ^ 1, 0);
         __builtin_amdgcn_sched_barrier(0);
@@ -871,18 +884,6 @@ static void launch_tile_cfg(const bf16_t* A, const bf16_t* W, const float* bias,
 //
 // Host side guarantees: K / gridDim.y is a multiple of 128, rows of W a multiple of 8 (32 with
 // SwiGLU), C and its row stride 16-byte aligned, M * lda and N * K below 2^31 elements.
-#define SCHED_FENCE() __builtin_amdgcn_sched_barrier(0)
-// (nothing that touches memory is moved across, by any pass of the compiler)
-#define ORDER_FENCE()                  \
-  do {                                 \
-    asm volatile("" ::: "memory");     \
-    __builtin_amdgcn_sched_barrier(0); \
-  } while (0)
-// waits until at most `behind` loads are under way (_AND_LDS: and no LDS access is)
-#define WAIT_LOADS(behind) __builtin_amdgcn_s_waitcnt(0x0F70 | ((behind) & 15) | ((behind) >> 4 << 14))
-#define WAIT_LOADS_AND_LDS(behind) \
-  __builtin_amdgcn_s_waitcnt(0x0070 | ((behind) & 15) | ((behind) >> 4 << 14))
-
 template <int N> struct IntC { static constexpr int value = N; };
 
 // The block products' epilogue: a wave turns 32 rows of its tile at a time through its own piece of LDS.

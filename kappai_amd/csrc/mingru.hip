@@ -396,9 +396,12 @@ __global__ __launch_bounds__(GU_STEP_THREADS) void gated_unit_step_wide_kernel(
   from_f32(&stored, acc + bias);
   const float u_c = to_f32(stored);
   if (tid < PART) us[i] = u_c;
-  // (a bare wait for LDS: a fence would wait for the matrix)
+  // (a bare wait for LDS: a fence would wait for the matrix; the empty statements keep the accesses to LDS on
+  // their sides of it)
+  asm volatile("" ::: "memory");
   __builtin_amdgcn_s_waitcnt(0xC07F);
   __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
   __builtin_amdgcn_sched_barrier(0);
   const int l = tid % LANES;
   float u8[8];

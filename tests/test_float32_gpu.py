@@ -138,3 +138,37 @@ def test_rows_far_apart_read_their_own_pages_only(ops):  # noqa: F811
     before = run(torch.cat([q[:1], q[:1]]), [-1, 0])
     assert not torch.isfinite(before[0]).any()
     assert torch.equal(before[1], run(q[:1], [0])[0])
+
+
+@pytest.mark.parametrize("d", [64, 80])
+@pytest.mark.parametrize("n_new", [1, 16, 21])
+@pytest.mark.parametrize("window", [0, 150])
+def test_attention_around_whole_rounds_of_its_waves(ops, d, n_new, window):  # noqa: F811
+    """A wave takes every eighth (heads above 64: fourth) step of 16 keys, two sets of registers in turn, its pages
+    two steps ahead: contexts on both sides of none, one, two and three of a wave's steps, the pages in front of a
+    window given back, NaN in every place that no request holds, single rows beside one another."""
+    H, G, ps, scale = 4, 2, 16, d ** -0.5
+    per_round = 16 * (8 if d <= 64 else 4)
+    held = sorted({max(0, per_round * r + e - n_new) for r in range(4) for e in (-16, -1, 0, 1, 17)})
+    g = torch.Generator().manual_seed(d + n_new)
+    need = [(a + n_new + ps - 1) // ps for a in held]
+    k = torch.full((sum(need) + 1, G, ps, d), math.nan)
+    v = torch.full((sum(need) + 1, G, d, ps), math.nan)
+    bt = torch.full((len(held), max(need)), -1, dtype=torch.int32)
+    order, at, pos, seg = torch.randperm(sum(need), generator=g).int() + 1, 0, [], []
+    for i, a in enumerate(held):
+        first = max(a - window + 1, 0) // ps if window else 0          # the first page that some row needs
+        for p in range(first, need[i]):
+            n = min(ps, a + n_new - p * ps)
+            bt[i, p] = order[at + p]
+            k[bt[i, p], :, :n] = torch.randn(G, n, d, generator=g)
+            v[bt[i, p], :, :, :n] = torch.randn(G, d, n, generator=g)
+        at += need[i]
+        pos += range(a, a + n_new)
+        seg += [i] * n_new
+    q = torch.randn(len(pos), H * d, generator=g)
+    rows = [torch.tensor(x, dtype=torch.int32) for x in (pos, seg)]
+    got = ops.paged_attention(q.to(DEV), H, G, d, k.to(DEV), v.to(DEV), *(x.to(DEV) for x in rows), bt.to(DEV), ps,
+                              scale, window=window)
+    want = ref.paged_attention(q, H, G, d, k, v, *rows, bt, ps, scale, window=window)
+    close(got, want, 6e-6, "attention")

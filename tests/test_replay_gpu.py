@@ -366,6 +366,57 @@ def test_decode_attention_with_its_prologue_inside_from_c_and_from_the_host(tmp_
         assert_matches_plain(a, folder, requests, "bfloat16")
 
 
+def test_decode_steps_on_both_sides_of_the_rules_from_c_and_from_the_host(tmp_path, monkeypatch):
+    """Which kernels a decode step takes is a rule that the C side and the host's parts hold each for itself: up to
+    16 rows the attention kernel normalises, rotates and stores (head size 64), up to 48 rows a conv layer over
+    matrices in fragment order is one kernel.  Steps on both sides of both lines, over contexts of mixed lengths:
+    the logits are the same bits either way, and the host's parts took the kernels that the rules name."""
+    import copy
+    from kappai_amd.cache import CacheManager
+    from kappai_amd.config import config_from_dict
+    from kappai_amd.engine import StepEntry, StepRunner
+    from kappai_amd.kernels import ops
+    from kappai_amd.weights import write_random_model
+    folder = write_random_model(tmp_path / "wide", config_from_dict(copy.deepcopy(WIDE)), seed=9,
+                                std=0.02, norm_jitter=0.05)
+    sizes = [4, 5, 16, 17, 48, 49]
+    lengths = [1500 + len(sizes), 700, 300] + [8 + 5 * i % 61 for i in range(46)]
+    requests = make_requests(WIDE["vocab_size"], lengths, seed=18)
+    ids, model = list(requests), gpu_model(folder, "bfloat16")
+    calls = []
+
+    def spy(name, rows_of):
+        kernel = getattr(ops, name)
+        monkeypatch.setattr(ops, name, lambda x, *a, **k: (calls.append((name, rows_of(x))), kernel(x, *a, **k))[1])
+
+    spy("qk_norm_rope_store", lambda x: x.shape[-2])
+    spy("linear_shortconv_step", lambda x: x.shape[0])
+    results = {}
+    for c_forward in (True, False):
+        cache = CacheManager(model.cache_specs(), 16, sum((n + 15) // 16 for n in lengths), len(ids))
+        cache.allocate_storage(model.dtype, "cuda:0", poison=True)
+        runner = StepRunner(model, cache, "cuda:0", decode_graphs=False, c_forward=c_forward)
+        caches, at, out = {rid: cache.open(rid) for rid in ids}, {}, []
+        for rid in ids:
+            at[rid] = max(1, len(requests[rid]) - len(sizes))
+            runner.step([StepEntry(caches[rid], requests[rid][:at[rid]], [])])
+        for rows in sizes:
+            del calls[:]
+            entries = [StepEntry(caches[rid], [requests[rid][at[rid]]], [0]) for rid in ids[:rows]]
+            out.append(runner.step(entries).cpu().numpy())
+            for rid in ids[:rows]:
+                at[rid] += 1
+            if not c_forward:            # two layers of either kind
+                assert sorted(calls) == ([("linear_shortconv_step", rows)] * 2 * (rows <= 48) +
+                                         [("qk_norm_rope_store", rows)] * 2 * (rows > 16))
+        for rid in ids:
+            cache.close(caches[rid])
+        cache.check()
+        results[c_forward] = out
+    for a, b in zip(results[True], results[False]):
+        assert np.array_equal(a, b)
+
+
 @pytest.mark.parametrize("dtype", ["bfloat16", "float32"])
 def test_decoded_tokens_over_long_contexts_beside_prompt_portions(tmp_path, dtype, monkeypatch):
     """Two requests decode at more than a thousand tokens of context while a third one's prompt
@@ -494,10 +545,12 @@ MIXED_LENGTHS_MODEL = {
 }
 
 
-def test_requests_of_mixed_lengths_decoded_side_by_side(tmp_path):
+@pytest.mark.parametrize("fused_qk", [True, False])
+def test_requests_of_mixed_lengths_decoded_side_by_side(tmp_path, monkeypatch, fused_qk):
     """Twelve requests of 150 to 2,300 tokens decoded side by side from captured graphs, in
-    bfloat16: with eight kv heads the decode attention has more blocks than waves to aim at and
-    settles the keys per split from the rows' own lengths, which change from request to request.
+    bfloat16.  With norm, rotation and store inside, the decode attention takes the host's keys per
+    split; with a kernel of their own it has more blocks than waves to aim at (eight kv heads) and
+    settles them from the rows' own lengths, which change from request to request.
     Every decoded position against the plain implementation, and the graph's steps against the
     same steps run eagerly (bit for bit)."""
     import copy
@@ -505,6 +558,8 @@ def test_requests_of_mixed_lengths_decoded_side_by_side(tmp_path):
     from kappai_amd.config import config_from_dict
     from kappai_amd.engine import StepEntry, StepRunner
     from kappai_amd.weights import write_random_model
+    from kappai_amd.kernels import tuning
+    monkeypatch.setattr(tuning, "FUSED_QK", fused_qk)
     cfg = copy.deepcopy(MIXED_LENGTHS_MODEL)
     folder = write_random_model(tmp_path / "mixed", config_from_dict(cfg), seed=4, std=0.04,
                                 norm_jitter=0.05)

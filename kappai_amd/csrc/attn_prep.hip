@@ -20,23 +20,25 @@
 #define AP_THREADS 256
 
 // use(i, load(i)) for the thread's i = tid, tid + AP_THREADS, ... below n, the loads of four of them under
-// way at once (the last i's again in place of those behind it): the kernels here are one block a row and take
-// what they wait for memory, once a round instead of once a value.  (The norm and store of projections of 1,536
-// values, one row: 6.9 us before, 5.6 so; the step's prompts 19 us either way.)
+// way at once: a kernel that is one block a row takes what it waits for memory, once a round instead of once a
+// value.  A round is whole or not made (places held back to the last value have load and use divide by the head
+// size once each, which 1,900 rows feel: 13.9 us against 11.3).  The norm and store of projections, 16 heads of 80
+// on 2 in places of 128, without rounds / so: one row 5.3 / 4.2 us, 300 rows 6.2 / 5.4, 1,900 rows 11.4 / 11.3.  The
+// other kernels here gained nothing on one row and lost up to 8 % on many.
 template <typename L, typename U>
 __device__ __forceinline__ void in_rounds(int n, int tid, L load, U use) {
-  for (int i0 = tid; i0 < n; i0 += 4 * AP_THREADS) {
+  int i0 = tid;
+  for (; i0 + 3 * AP_THREADS < n; i0 += 4 * AP_THREADS) {
     decltype(load(0)) v[4];
 #pragma unroll
-    for (int u = 0; u < 4; ++u) v[u] = load(min(i0 + u * AP_THREADS, n - 1));
-    asm volatile("" ::: "memory");               // (else the loads sink behind the conditions)
+    for (int u = 0; u < 4; ++u) v[u] = load(i0 + u * AP_THREADS);
+    asm volatile("" ::: "memory");               // (else the loads sink to their use)
 #pragma unroll
-    for (int u = 0; u < 4; ++u)
-      if (i0 + u * AP_THREADS < n) use(i0 + u * AP_THREADS, v[u]);
+    for (int u = 0; u < 4; ++u) use(i0 + u * AP_THREADS, v[u]);
   }
+  for (; i0 < n; i0 += AP_THREADS) use(i0, load(i0));
 }
 struct Two { float a, b; };
-struct Four { float a, b, c, d; };
 
 // ---------------------------------------------------------------------------------------
 template <typename T>
@@ -127,33 +129,29 @@ __global__ __launch_bounds__(AP_THREADS) void latent_store_kernel(
   extern __shared__ float sh[];            // (H + 1) * rot floats: the parts that turn
   __shared__ float red[16];
   const int t = blockIdx.x, tid = threadIdx.x;
-  const int pos = row_pos[t], seg = k_pool == nullptr ? 0 : row_seg[t];
+  const int pos = row_pos[t];
   const T* kvr = kv + (size_t)t * kv_stride;
   const T* qr = q + (size_t)t * q_stride;
   const float* ct = cos_tab + (size_t)pos * (rot_dims / 2);
   const float* st = sin_tab + (size_t)pos * (rot_dims / 2);
-  // (asked for ahead of the sum: the row's page, the first values and norm weights)
-  const size_t page = k_pool == nullptr ? 0 : (size_t)block_tables[(size_t)seg * max_blocks + pos / ps];
-  const float first = tid < r ? to_f32(kvr[tid]) : 0.f, weight = tid < r ? c_norm_w[tid] : 0.f;
-  float ss = fmaf(first, first, 0.f);
-  for (int e = tid + AP_THREADS; e < r; e += AP_THREADS) { const float v = to_f32(kvr[e]); ss = fmaf(v, v, ss); }
-  in_rounds((H + 1) * rot, tid, [&](int i) {
+  float ss = 0.f;
+  for (int e = tid; e < r; e += AP_THREADS) { const float v = to_f32(kvr[e]); ss = fmaf(v, v, ss); }
+  for (int i = tid; i < (H + 1) * rot; i += AP_THREADS) {
     const int h = i / rot, e = i % rot;
-    return to_f32(h < H ? qr[h * (d + rot) + d + e] : kvr[r + e]);
-  }, [&](int i, float v) { sh[i] = v; });
+    sh[i] = h < H ? to_f32(qr[h * (d + rot) + d + e]) : to_f32(kvr[r + e]);
+  }
   const float inv = 1.0f / sqrtf(block_sum(ss, red) / (float)r + eps);      // (barrier inside)
-  if (D > r)
-    in_rounds(H * (D - r), tid, [&](int i) {
-      const int h = i / (D - r), e = i % (D - r);
-      return e < rot ? rotated(sh + h * rot, e, rot_dims, rot_mode, ct, st) : 0.f;
-    }, [&](int i, float v) {
-      from_f32(q_out + (size_t)t * H * D + (size_t)(i / (D - r)) * D + r + i % (D - r), v);
-    });
+  for (int i = tid; i < H * (D - r); i += AP_THREADS) {
+    const int h = i / (D - r), e = i % (D - r);
+    const float v = e < rot ? rotated(sh + h * rot, e, rot_dims, rot_mode, ct, st) : 0.f;
+    from_f32(q_out + (size_t)t * H * D + (size_t)h * D + r + e, v);
+  }
   if (k_pool == nullptr) return;
+  const size_t page = (size_t)block_tables[(size_t)row_seg[t] * max_blocks + pos / ps];
   const int slot = pos % ps;
   for (int e = tid; e < D; e += AP_THREADS) {
     float kvv = 0.f, vv = 0.f;
-    if (e < r) kvv = vv = e == tid ? first * inv * weight : to_f32(kvr[e]) * inv * c_norm_w[e];
+    if (e < r) kvv = vv = to_f32(kvr[e]) * inv * c_norm_w[e];
     else if (e < r + rot) kvv = rotated(sh + H * rot, e - r, rot_dims, rot_mode, ct, st);
     from_f32(k_pool + (page * ps + slot) * D + e, kvv);
     from_f32(v_pool + (page * D + e) * ps + slot, vv);
@@ -400,42 +398,37 @@ __global__ __launch_bounds__(AP_THREADS) void rotate_widen_store_kernel(
     const int* __restrict__ row_seg, const int* __restrict__ block_tables, int max_blocks, int H,
     int G, int d, int dv, int D, int ps, T* __restrict__ q_out) {
   const int t = blockIdx.x, tid = threadIdx.x;
-  const int pos = row_pos[t], seg = k_pool == nullptr ? 0 : row_seg[t];
-  const size_t page = k_pool == nullptr ? 0 : (size_t)block_tables[(size_t)seg * max_blocks + pos / ps];
+  const int pos = row_pos[t];
   const T* row = proj + (size_t)t * stride;
   const int nq = H * d, nk = G * d, half = rot_dims / 2;
   const float* ct = cos_tab + (size_t)pos * half;
   const float* st = sin_tab + (size_t)pos * half;
-  // place e of the head that starts at `head`: its value, its partner's (a place that does not turn has
-  // none), cosine and sine; and the place turned by the position, in float32
-  auto ask = [&](const T* head, int e) {
-    e = min(e, d - 1);
-    const bool turns = e < rot_dims && rot_mode != 0;
-    const int j = !turns ? 0 : rot_mode == 1 ? (e < half ? e : e - half) : e / 2;
-    const int partner = !turns ? e : rot_mode == 1 ? (e < half ? e + half : e - half) : e ^ 1;
-    return Four{to_f32(head[e]), to_f32(head[partner]), half > 0 && rot_mode ? ct[j] : 0.f,
-                half > 0 && rot_mode ? st[j] : 0.f};
+  // place e of the head that starts at `head`: turned by the position, in float32
+  auto turned = [&](const T* head, int e) -> float {
+    const float x = to_f32(head[e]);
+    if (e >= rot_dims || rot_mode == 0) return x;
+    int j, partner;
+    bool first;
+    if (rot_mode == 1) { first = e < half; j = first ? e : e - half; partner = first ? e + half : e - half; }
+    else { first = (e & 1) == 0; j = e / 2; partner = e ^ 1; }
+    const float y = to_f32(head[partner]), c = ct[j], s = st[j];
+    return first ? x * c - y * s : x * c + y * s;
   };
-  auto turned = [&](Four v, int e) {
-    if (e >= rot_dims || rot_mode == 0) return v.a;
-    const bool first = rot_mode == 1 ? e < half : (e & 1) == 0;
-    return first ? v.a * v.c - v.b * v.d : v.a * v.c + v.b * v.d;
-  };
-  in_rounds(H * D, tid, [&](int i) { return ask(row + i / D * d, i % D); }, [&](int i, Four v) {
-    from_f32(q_out + (size_t)t * H * D + i, i % D < d ? turned(v, i % D) : 0.f);
-  });
+  for (int i = tid; i < H * D; i += AP_THREADS) {
+    const int h = i / D, e = i % D;
+    from_f32(q_out + (size_t)t * H * D + i, e < d ? turned(row + h * d, e) : 0.f);
+  }
   if (k_pool == nullptr) return;
+  const size_t page = (size_t)block_tables[(size_t)row_seg[t] * max_blocks + pos / ps];
   const int slot = pos % ps;
-  struct Kv { Four k; float v; };
-  in_rounds(G * D, tid, [&](int i) {
-    const int g = i / D, e = min(i % D, dv - 1);
-    const T* khead = row + nq + g * d;
-    return Kv{ask(khead, i % D), to_f32(values_are_keys ? khead[e] : row[nq + nk + g * dv + e])};
-  }, [&](int i, Kv x) {
+  for (int i = tid; i < G * D; i += AP_THREADS) {
     const int g = i / D, e = i % D;
-    from_f32(k_pool + ((page * G + g) * ps + slot) * D + e, e < d ? turned(x.k, e) : 0.f);
-    from_f32(v_pool + ((page * G + g) * D + e) * ps + slot, e < dv ? x.v : 0.f);
-  });
+    const T* khead = row + nq + g * d;
+    float vv = 0.f;
+    if (e < dv) vv = values_are_keys ? to_f32(khead[e]) : to_f32(row[nq + nk + g * dv + e]);
+    from_f32(k_pool + ((page * G + g) * ps + slot) * D + e, e < d ? turned(khead, e) : 0.f);
+    from_f32(v_pool + ((page * G + g) * D + e) * ps + slot, vv);
+  }
 }
 
 extern "C" int kappai_rotate_widen_store(

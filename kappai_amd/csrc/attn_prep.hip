@@ -263,11 +263,12 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t hw_buffer(const void* p) {
 }
 #endif
 
-// Bound by how often it waits for memory, so STEPS steps' loads (and the gates) are asked for before
-// anything is multiplied, without conditions: what a lane must not read lies outside its buffer.  The 72 products
-// of eight steps of two rows and a prompt of 1,900 (16 heads, 64 to 224 and back): 537 us with a wait a step of 32
-// and a wait a gate, 413 so.
-template <typename TO, int STEPS>
+// Few rows are bound by how often they wait for memory, so STEPS steps' loads (and the gates) are asked for
+// before anything is multiplied, without conditions: what a lane must not read lies outside its buffer.  One row of 16
+// heads, 224 to 64, 3.95 us with a wait a step of 32, 2.9 so; 128 to 64 with gates and a wait a gate 5.7, 4.2 so;
+// 300 rows of these 5.7 either way and 8.6 / 7.3, 1,900 rows 10.3 either way and 12.4 / 13.1.
+// GATE: 1 the gates are asked for with the first steps (few rows), 2 behind the products, 0 there are none.
+template <typename TO, int STEPS, int GATE>
 __global__ __launch_bounds__(256) void headwise_linear_mfma_kernel(
     const bf16_t* __restrict__ x, const bf16_t* __restrict__ w, int x_row, int x_head, int n_out,
     int n_in, int rows, const bf16_t* __restrict__ gate, int g_row, TO* __restrict__ y, int y_row,
@@ -290,6 +291,17 @@ __global__ __launch_bounds__(256) void headwise_linear_mfma_kernel(
 #pragma unroll
   for (int j = 0; j < 4; ++j) acc[j] = (hw_f32x4_t){0.f, 0.f, 0.f, 0.f};
   uint16_t gates[4][4];
+  const auto ask_for_gates = [&]() {
+    const __amdgpu_buffer_rsrc_t gb = hw_buffer(gate + (size_t)m0 * g_row + (size_t)h * n_out + n0);
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+#pragma unroll
+      for (int v = 0; v < 4; ++v) {
+        const int n = 16 * j + 4 * kq + v;
+        gates[j][v] = __builtin_amdgcn_raw_buffer_load_b16(
+            gb, m0 + lr < rows && n0 + n < n_out ? (uint32_t)(lr * g_row + n) * 2u : OUT, 0, 0);
+      }
+  };
   for (int k0 = 0; k0 < n_in; k0 += 32 * STEPS) {
     hw_u32x4_t xv[STEPS], wv[STEPS][4];
 #pragma unroll
@@ -301,17 +313,7 @@ __global__ __launch_bounds__(256) void headwise_linear_mfma_kernel(
       for (int j = 0; j < 4; ++j)
         wv[u][j] = __builtin_amdgcn_raw_buffer_load_b128(wb, ok ? wo[j] : OUT, k * 2, 0);
     }
-    if (k0 == 0 && gate != nullptr) {
-      const __amdgpu_buffer_rsrc_t gb = hw_buffer(gate + (size_t)m0 * g_row + (size_t)h * n_out + n0);
-#pragma unroll
-      for (int j = 0; j < 4; ++j)
-#pragma unroll
-        for (int v = 0; v < 4; ++v) {
-          const int n = 16 * j + 4 * kq + v;
-          gates[j][v] = __builtin_amdgcn_raw_buffer_load_b16(
-              gb, m0 + lr < rows && n0 + n < n_out ? (uint32_t)(lr * g_row + n) * 2u : OUT, 0, 0);
-        }
-    }
+    if (GATE == 1 && k0 == 0) ask_for_gates();
     __builtin_amdgcn_sched_barrier(0);           // (left alone, the loads sink to their use)
 #pragma unroll
     for (int u = 0; u < STEPS; ++u)
@@ -321,6 +323,7 @@ __global__ __launch_bounds__(256) void headwise_linear_mfma_kernel(
                                                          __builtin_bit_cast(hw_bf16x8_t, xv[u]), acc[j],
                                                          0, 0, 0);
   }
+  if (GATE == 2) ask_for_gates();
   if (m0 + lr >= rows) return;
   TO* yr = y + (size_t)(m0 + lr) * y_row + (size_t)h * y_head;
 #pragma unroll
@@ -330,7 +333,7 @@ __global__ __launch_bounds__(256) void headwise_linear_mfma_kernel(
       const int n = n0 + 16 * j + 4 * kq + v;
       if (n >= n_out) continue;
       float r = acc[j][v];
-      if (gate) r /= 1.0f + expf(-__uint_as_float((uint32_t)gates[j][v] << 16));
+      if (GATE) r /= 1.0f + expf(-__uint_as_float((uint32_t)gates[j][v] << 16));
       from_f32(yr + n, r);
     }
 #endif
@@ -350,18 +353,31 @@ extern "C" int kappai_headwise_linear(const void* x, int x_row, int x_head, cons
       (size_t)g_row * 32 + 256 < 0x40000000u) {
     const int waves = rows <= 16 ? 1 : 4;
     const dim3 grid((rows + 16 * waves - 1) / (16 * waves), (n_out + 63) / 64, H);
-    // (few rows: eight steps' loads at once; more: waves enough to cover for one another)
-#define HEADWISE(TO, STEPS)                                                                            \
-  hipLaunchKernelGGL((headwise_linear_mfma_kernel<TO, STEPS>), grid, dim3(waves * WAVE), 0, stream,    \
+    // Few rows: all steps' loads at once, up to eight.  More: waves enough to cover for one another, a step at a
+    // time (us with places for four steps / one, no gates: 300 rows of 32 to 32 3.1 / 2.8, 1,900 rows of 16 heads 64 to 224
+    // 26.0 / 24.1, 224 to 64 10.6 / 10.3).
+#define HEADWISE(TO, STEPS, GATE)                                                                      \
+  hipLaunchKernelGGL((headwise_linear_mfma_kernel<TO, STEPS, GATE>), grid, dim3(waves * WAVE), 0, stream, \
                      (const bf16_t*)x, (const bf16_t*)w, x_row, x_head, n_out, n_in, rows,             \
                      (const bf16_t*)gate, g_row, (TO*)y, y_row, y_head)
-    if (out_f32) {
-      if (waves == 1 && n_in > 128) HEADWISE(float, 8);
-      else HEADWISE(float, 4);
-    } else {
-      if (waves == 1 && n_in > 128) HEADWISE(bf16_t, 8);
-      else HEADWISE(bf16_t, 4);
-    }
+#define HEADWISE_FEW(TO, GATE)                                                                         \
+  do {                                                                                                 \
+    if (n_in <= 32) HEADWISE(TO, 1, GATE);                                                             \
+    else if (n_in <= 64) HEADWISE(TO, 2, GATE);                                                        \
+    else if (n_in <= 128) HEADWISE(TO, 4, GATE);                                                       \
+    else HEADWISE(TO, 8, GATE);                                                                        \
+  } while (0)
+#define HEADWISE_AS(TO)                                                                                \
+  do {                                                                                                 \
+    if (waves > 1 && gate != nullptr) HEADWISE(TO, 1, 2);                                              \
+    else if (waves > 1) HEADWISE(TO, 1, 0);                                                            \
+    else if (gate != nullptr) HEADWISE_FEW(TO, 1);                                                     \
+    else HEADWISE_FEW(TO, 0);                                                                          \
+  } while (0)
+    if (out_f32) HEADWISE_AS(float);
+    else HEADWISE_AS(bf16_t);
+#undef HEADWISE_AS
+#undef HEADWISE_FEW
 #undef HEADWISE
     KAPPAI_RETURN_LAUNCH_STATUS();
   }

@@ -1706,11 +1706,12 @@ template <typename TO, int MT, int NW, int EPI, int NT, bool FRAG>
 __global__ __launch_bounds__(NW * WAVE) __attribute__((amdgpu_waves_per_eu(MT == 1 && EPI < 2 ? 4 : 1)))
 void gemm_bf16_skinny_kernel(
     const bf16_t* __restrict__ A, const bf16_t* __restrict__ W, const float* __restrict__ ss, int M,
-    int N, int K, int kblk, int lda, int a_frag, int ss_count, float ss_eps, TO* __restrict__ C,
-    const float* __restrict__ bias, int ldc, ConvStep cs, int w_frag, int c_frag) {
+    int N, int K, int kblk, int lda, int frags, int ss_count, float ss_eps, TO* __restrict__ C,
+    const float* __restrict__ bias, int ldc, ConvStep cs, int c_frag) {
   // (the arguments that the first loads need come first: the hardware hands over the first 14 words in
   // registers, the rest costs a load)
   static_assert(NT == 1 || EPI == 0, "several column tiles a wave: plain products only");
+  const int a_frag = frags & 1, w_frag = frags & 2;
   // c_frag (one row tile, the SwiGLU and conv epilogues): the result is written as 16 rows in
   // fragment order, which is how the product that follows likes to read it (see a_frag)
   auto out_at = [&](int gm, int gn_) {
@@ -1917,6 +1918,7 @@ void gemm_bf16_skinny_kernel(
 #endif
   } else {
     if (CONV && wave < MT) ask_for_state();
+    if (MT == 1 && ss != nullptr) ask_for_first_parts();
     for (int k = k0; k < k1; k += 32 * U) {
       // the loads of W and of A alternate, in the order of K
       u32x4_t wv[U][NG], av[U][MT];
@@ -1943,7 +1945,7 @@ void gemm_bf16_skinny_kernel(
                 as_bf16x8(av[u][t]), as_bf16x8(wv[u][r]), acc[r * MT + t], 0, 0, 0);
     }
   }
-  if (MT == 1 && ss != nullptr) add_parts(FRAG && k0 < k1);
+  if (MT == 1 && ss != nullptr) add_parts(!FRAG || k0 < k1);
 #pragma unroll
   for (int t = 0; t < NG * MT; ++t) red[wave][t][lane] = acc[t];
   __syncthreads();
@@ -2057,8 +2059,9 @@ void gemm_bf16_skinny_kernel(
 template <int NW, bool FRAG>
 __global__ __launch_bounds__(NW * WAVE) void gemm_bf16_into_resid_kernel(
     const bf16_t* __restrict__ A, const bf16_t* __restrict__ W, float* __restrict__ resid, int M, int N,
-    int K, int lda, int a_frag, int ldr, const float* __restrict__ norm_w, const float* __restrict__ bias,
-    bf16_t* __restrict__ rows, float* __restrict__ ss, int rows_frag, int w_frag) {
+    int K, int lda, int frags, int ldr, const float* __restrict__ norm_w, const float* __restrict__ bias,
+    bf16_t* __restrict__ rows, float* __restrict__ ss, int rows_frag) {
+  const int a_frag = frags & 1, w_frag = frags & 2;
   __shared__ f32x4_t red[NW][2][WAVE];
   const int tid = threadIdx.x;
   const int lane = tid % WAVE, wave = __builtin_amdgcn_readfirstlane(tid / WAVE);
@@ -2206,22 +2209,22 @@ __global__ __launch_bounds__(NW * WAVE) void gemm_bf16_into_resid_kernel(
 static void launch_into_resid(const bf16_t* A, const bf16_t* W, const float* bias, int M, int N,
                               int K, int lda, const ResidOut& ro, hipStream_t stream,
                               const bf16_t* Wf, int a_frag) {
-  const int w_frag = Wf != nullptr;
+  const int frags = (a_frag ? 1 : 0) | (Wf ? 2 : 0);
   if (Wf) W = Wf;
   const dim3 grid((N + 7) / 8);
   // (both halves of K whole pieces and offsets of 31 bits, into the stream too: the loads without conditions)
-  const bool pieces = w_frag && K % 64 == 0 && ((size_t)M * lda + K) * 2 < 0x7FFFFF00u &&
+  const bool pieces = Wf != nullptr && K % 64 == 0 && ((size_t)M * lda + K) * 2 < 0x7FFFFF00u &&
                       (size_t)K * 32 < 0x7FFFFF00u && ((size_t)(M - 1) * ro.ldr + N) * 4 < 0x7FFFFF00u;
 #define INTO_RESID(NW)                                                                                 \
   do {                                                                                                 \
     if (pieces)                                                                                        \
       hipLaunchKernelGGL((gemm_bf16_into_resid_kernel<NW, true>), grid, dim3(NW * WAVE), 0, stream, A, \
-                         W, ro.resid, M, N, K, lda, a_frag, ro.ldr, ro.norm_w, bias, ro.rows, ro.ss,   \
-                         ro.rows_frag, w_frag);                                                        \
+                         W, ro.resid, M, N, K, lda, frags, ro.ldr, ro.norm_w, bias, ro.rows, ro.ss,    \
+                         ro.rows_frag);                                                                \
     else                                                                                               \
       hipLaunchKernelGGL((gemm_bf16_into_resid_kernel<NW, false>), grid, dim3(NW * WAVE), 0, stream,   \
-                         A, W, ro.resid, M, N, K, lda, a_frag, ro.ldr, ro.norm_w, bias, ro.rows,       \
-                         ro.ss, ro.rows_frag, w_frag);                                                 \
+                         A, W, ro.resid, M, N, K, lda, frags, ro.ldr, ro.norm_w, bias, ro.rows,        \
+                         ro.ss, ro.rows_frag);                                                         \
   } while (0)
   // K a wave: 128 or more where K allows it
   if (K >= 4096) INTO_RESID(16);
@@ -2241,7 +2244,6 @@ static void launch_skinny(const bf16_t* A, const bf16_t* W, const float* bias, T
                           int K, int lda, int ldc, int ksplit, ConvStep cs, hipStream_t stream,
                           const Fuse& fuse = Fuse{}, const bf16_t* Wf = nullptr, int a_frag = 0) {
   // Wf: the copy of W in fragment order (see the kernel), or null
-  const int w_frag = Wf != nullptr;
   const dim3 grid(EPI == 3 ? (N + 7) / 8 : (N + 16 * NT - 1) / (16 * NT), ksplit);
   const int c_frag = (MT == 1 && EPI != 0) ? fuse.c_frag : 0;
   const int kblk = (K + 32 * ksplit - 1) / (32 * ksplit) * 32;
@@ -2251,8 +2253,8 @@ static void launch_skinny(const bf16_t* A, const bf16_t* W, const float* bias, T
                       (EPI != 3 || (size_t)(N + 16) * K * 2 < 0x7FFFFF00u);
 #define SKINNY(FRAG)                                                                                   \
   hipLaunchKernelGGL((gemm_bf16_skinny_kernel<TO, MT, NW, EPI, NT, FRAG>), grid, dim3(NW * WAVE), 0,    \
-                     stream, A, Wf ? Wf : W, fuse.rsc.ss, M, N, K, kblk, lda, a_frag, fuse.rsc.n_parts, \
-                     fuse.rsc.eps, C, bias, ldc, cs, w_frag, c_frag)
+                     stream, A, Wf ? Wf : W, fuse.rsc.ss, M, N, K, kblk, lda, (a_frag ? 1 : 0) | (Wf ? 2 : 0), \
+                     fuse.rsc.n_parts, fuse.rsc.eps, C, bias, ldc, cs, c_frag)
   if (pieces) SKINNY(true);
   else SKINNY(false);
 #undef SKINNY

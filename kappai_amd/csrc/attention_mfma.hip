@@ -646,7 +646,7 @@ __global__ __launch_bounds__(8 * WAVE) void attn_prefill_shared_kernel(
   const int key_bytes = (int)sizeof(bf16_t) * (wave < 4 ? HEAD_DIM : 1);
   // 64 of the segment's pages, a lane each, and the number of the first: a scalar load a tile would have every
   // wait for LDS wait for it too
-  int pages = 0, pages_from = -(1 << 30);
+  int pages_from = min(nx_pidx, max_blocks - 1), pages = bt[min(pages_from + lane, max_blocks - 1)];
   auto lookup = [&]() {
     const int at = min(nx_pidx, max_blocks - 1);
     if (__builtin_expect(at - pages_from >= WAVE, 0)) {
@@ -657,7 +657,8 @@ __global__ __launch_bounds__(8 * WAVE) void attn_prefill_shared_kernel(
     const int page = __builtin_amdgcn_readlane(pages, at - pages_from);
     return nx_key <= blk_last ? max(page, 0) : 0;
   };
-  int nx_page = lookup();
+  // (the first by a scalar load beside those 64, which it does not wait for: two portions of 16 tiles gain 0.3 us)
+  int nx_page = nx_key <= blk_last ? max(bt[pages_from], 0) : 0;
   // (buffer loads: of a global load into LDS the compiler holds that it may be any access to LDS, and waits for
   // all reads under way where it should wait for the oldest)
   uint32_t from[NL];

@@ -31,6 +31,10 @@ extern "C" {
 #define KAPPAI_ENGINE_ABI 12         // bumped with every change of the structs below
 #define KAPPAI_MAX_GROUPS 8          // paged groups a batch can carry block tables for
 #define KAPPAI_MAX_TABLES 8         // tables and numbers of the parts' own in a step
+// Norm, rotation and store inside the decode attention that keeps a row in one block: up to this many blocks.  us
+// with a kernel of their own / inside, 32 heads of 64 on 32: 8 rows of 200 keys 8.8 / 8.0, of 500 12.0 / 10.9; 12 rows of
+// 200 12.6 / 13.6, of 500 18.4 / 18.9; 16 rows 13.3 / 14.1 and 21.0 / 21.4 (16 rows on 16 kv heads 8.8 / 8.0 and 11.9 / 10.7).
+#define KAPPAI_QK_BLOCKS 256
 
 // ---- the kernels' launchers, by address (they live in libraries of their own) ---------------
 typedef struct kappai_kernels {

@@ -208,7 +208,7 @@ kappai_carry attention_mixer(kappai_step* s, const void* desc, kappai_rows x, fl
       L.mfma != nullptr && H / G <= 16 && qkv.n % 8 == 0 && aligned16(proj.data) && ps % 16 == 0 &&
       d % 16 == 0 && d <= 256 && (L.rot_mode == 0 || (L.rot_mode == 1 && L.rot_dim == d)) &&
       (!decode_block_form(m, b, L, M) ||
-       (L.mfma->decode_block_qk_keys != nullptr &&
+       (L.mfma->decode_block_qk_keys != nullptr && (long)M * G <= KAPPAI_QK_BLOCKS &&
         decode_keys(b, L) <= L.mfma->decode_block_qk_keys()));
   // q in place in the projection, or (from partial sums) a new bfloat16 [M, H d]
   void* q;

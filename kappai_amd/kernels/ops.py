@@ -978,9 +978,13 @@ def decode_takes_qk(head_dim: int, page_size: int) -> bool:
     return decode_qk_rows(head_dim, page_size) > 0
 
 
-def decode_block_takes_qk(head_dim: int, max_position: int, window: int = 0) -> bool:
-    """Whether a ``QkPrologue`` finds few enough keys for the kernel that keeps them in one block."""
-    return (keys_bound(max_position, window)
+QK_BLOCKS = 256            # KAPPAI_QK_BLOCKS (engine.h)
+
+
+def decode_block_takes_qk(head_dim: int, max_position: int, window: int = 0, n_blocks: int = 1) -> bool:
+    """Whether a ``QkPrologue`` finds few enough keys for the kernel that keeps them in one block, and few
+    enough of those blocks (a row and kv head each) to do better with it."""
+    return (n_blocks <= QK_BLOCKS and keys_bound(max_position, window)
             <= library("attention_mfma", HEAD_DIM=head_dim).kappai_attn_decode_block_qk_keys())
 
 

@@ -235,7 +235,8 @@ class GroupedQueryAttention(Mixer):
         return (proj.shape[0] <= ops.decode_qk_rows(self.d, page_size)
                 and (ops.decode_form(self.H, self.G, self.d, max_position, window,
                                      n_rows=proj.shape[0]) == "decode-split"
-                     or ops.decode_block_takes_qk(self.d, max_position, window)))
+                     or ops.decode_block_takes_qk(self.d, max_position, window,
+                                                  proj.shape[0] * self.G)))
 
     def weight_bytes(self) -> int:
         return self.qkv.weight_bytes() + self.out.weight_bytes() + 2 * self.d * 4

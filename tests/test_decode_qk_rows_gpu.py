@@ -12,6 +12,8 @@ pytestmark = pytest.mark.gpu
 def test_where_the_rule_lies(ops):  # noqa: F811
     assert [ops.decode_qk_rows(d, 16) for d in (64, 128, 48, 256)] == [16, 4, 0, 0]
     assert ops.decode_qk_rows(64, 8) == 0
+    # (kept in one block: up to a block a CU)
+    assert [ops.decode_block_takes_qk(64, 400, 0, n) for n in (16, 256, 257)] == [True, True, False]
 
 
 @pytest.mark.parametrize("H,G", [(32, 8), (16, 8), (4, 1)])

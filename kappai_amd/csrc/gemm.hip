@@ -1706,12 +1706,12 @@ template <typename TO, int MT, int NW, int EPI, int NT, bool FRAG>
 __global__ __launch_bounds__(NW * WAVE) __attribute__((amdgpu_waves_per_eu(MT == 1 && EPI < 2 ? 4 : 1)))
 void gemm_bf16_skinny_kernel(
     const bf16_t* __restrict__ A, const bf16_t* __restrict__ W, const float* __restrict__ ss, int M,
-    int N, int K, int kblk, int lda, int frags, int ss_count, float ss_eps, TO* __restrict__ C,
-    const float* __restrict__ bias, int ldc, ConvStep cs, int c_frag) {
+    int N, int K, int kblk, int lda, int a_frag, int w_frag, int ss_count, TO* __restrict__ C,
+    const float* __restrict__ bias, int ldc, ConvStep cs, float ss_eps, int c_frag) {
   // (the arguments that the first loads need come first: the hardware hands over the first 14 words in
-  // registers, the rest costs a load)
+  // registers, the rest costs a load.  All of them together are a multiple of eight bytes: with an int less here
+  // and in the kernel below, a step of 2 rows of 79 kernels, 65 of them these, took 478 us instead of 458.)
   static_assert(NT == 1 || EPI == 0, "several column tiles a wave: plain products only");
-  const int a_frag = frags & 1, w_frag = frags & 2;
   // c_frag (one row tile, the SwiGLU and conv epilogues): the result is written as 16 rows in
   // fragment order, which is how the product that follows likes to read it (see a_frag)
   auto out_at = [&](int gm, int gn_) {
@@ -1806,14 +1806,13 @@ void gemm_bf16_skinny_kernel(
 #if defined(__HIP_DEVICE_COMPILE__)
   if (CONV && wave < MT) {
     // (buffer loads: an offset outside the buffer, or a buffer of no bytes, gives 0 and needs no branch.  The
-    // channels' buffers begin with the block's first, so that there may be any number of them.)
+    // taps' buffer begins with the block's first channel: there may be 4 GiB of them, and less than that of the rest.)
     constexpr int OUT = 0x7FFFFF00;
-    const int c = gn - n0;
     const auto word = [](const void* p, uint32_t bytes, int at) {
       return __builtin_amdgcn_raw_buffer_load_b32(raw_buffer(p, bytes), at, 0, 0);
     };
-    const auto number = [&](const float* p, size_t first, uint32_t bytes, int at) {
-      return __builtin_bit_cast(float, word(p + first, p != nullptr ? bytes : 0u, at));
+    const auto number = [&](const void* p, uint32_t bytes, int at) {
+      return __builtin_bit_cast(float, word(p, bytes, at));
     };
 #pragma unroll
     for (int v = 0; v < 4; ++v) {
@@ -1823,11 +1822,12 @@ void gemm_bf16_skinny_kernel(
     }
 #pragma unroll
     for (int k = 0; k <= CONV_PRE; ++k)
-      tap_pre[k] = number(cs.taps, (size_t)n0 * cs.L, 16u * cs.L * 4u, channel && k < cs.L ? (c * cs.L + k) * 4 : OUT);
-    conv_bias_pre = number(cs.conv_bias, n0, 64u, channel ? c * 4 : OUT);
+      tap_pre[k] = number(cs.taps + (size_t)n0 * cs.L, 16u * cs.L * 4u,
+                          channel && k < cs.L ? ((gn - n0) * cs.L + k) * 4 : OUT);
+    conv_bias_pre = number(cs.conv_bias, cs.conv_bias ? N * 4u : 0u, channel ? gn * 4 : OUT);
 #pragma unroll
     for (int g = 0; g < 3; ++g)
-      gate_bias_pre[g] = number(bias, (size_t)g * N + n0, 64u, channel ? c * 4 : OUT);
+      gate_bias_pre[g] = number(bias, bias ? N * 12u : 0u, channel ? (int)(((uint32_t)g * N + gn) * 4u) : OUT);
   }
 #endif
   const auto ask_for_state = [&]() {
@@ -2060,8 +2060,9 @@ template <int NW, bool FRAG>
 __global__ __launch_bounds__(NW * WAVE) void gemm_bf16_into_resid_kernel(
     const bf16_t* __restrict__ A, const bf16_t* __restrict__ W, float* __restrict__ resid, int M, int N,
     int K, int lda, int frags, int ldr, const float* __restrict__ norm_w, const float* __restrict__ bias,
-    bf16_t* __restrict__ rows, float* __restrict__ ss, int rows_frag) {
-  const int a_frag = frags & 1, w_frag = frags & 2;
+    bf16_t* __restrict__ rows, float* __restrict__ ss, int rows_frag, int spare) {
+  // frags: the rows' order, and where not FRAG as the second bit that of W; spare: see above
+  const int a_frag = FRAG ? frags : frags & 1, w_frag = FRAG ? 1 : frags & 2;
   __shared__ f32x4_t red[NW][2][WAVE];
   const int tid = threadIdx.x;
   const int lane = tid % WAVE, wave = __builtin_amdgcn_readfirstlane(tid / WAVE);
@@ -2076,21 +2077,21 @@ __global__ __launch_bounds__(NW * WAVE) void gemm_bf16_into_resid_kernel(
   float resid_in[4] = {0.f, 0.f, 0.f, 0.f};
   float norm_w_in = 0.f;
 #if defined(__HIP_DEVICE_COMPILE__)
-  const bool wanted = half == 0 && gn < N;
   const bool near = FRAG || ((uint64_t)(M - 1) * ldr + N) * 4 < 0x7FFFFF00u;
   if (wave == 0 && near) {
+    const bool mine = half == 0 && gn < N;
     const __amdgpu_buffer_rsrc_t res = raw_buffer(resid, 0x7FFFFF00u);
     const __amdgpu_buffer_rsrc_t nw = raw_buffer(norm_w, rows != nullptr ? (uint32_t)N * 4u : 0u);
 #pragma unroll
     for (int v = 0; v < 4; ++v) {
       const int gm = 4 * (lane / 16) + v;
       resid_in[v] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(
-          res, wanted && gm < M ? (gm * ldr + gn) * 4 : 0x7FFFFF00, 0, 0));
+          res, mine && gm < M ? (gm * ldr + gn) * 4 : 0x7FFFFF00, 0, 0));
     }
     norm_w_in = __builtin_bit_cast(
-        float, __builtin_amdgcn_raw_buffer_load_b32(nw, wanted ? gn * 4 : 0x7FFFFF00, 0, 0));
+        float, __builtin_amdgcn_raw_buffer_load_b32(nw, mine ? gn * 4 : 0x7FFFFF00, 0, 0));
   }
-  if (wave == 0 && !near && wanted) {
+  if (wave == 0 && !near && half == 0 && gn < N) {
 #pragma unroll
     for (int v = 0; v < 4; ++v) {
       const int gm = 4 * (lane / 16) + v;
@@ -2209,7 +2210,8 @@ __global__ __launch_bounds__(NW * WAVE) void gemm_bf16_into_resid_kernel(
 static void launch_into_resid(const bf16_t* A, const bf16_t* W, const float* bias, int M, int N,
                               int K, int lda, const ResidOut& ro, hipStream_t stream,
                               const bf16_t* Wf, int a_frag) {
-  const int frags = (a_frag ? 1 : 0) | (Wf ? 2 : 0);
+  const int frags = a_frag ? 1 : 0;
+  const int w_order = Wf ? 2 : 0;
   if (Wf) W = Wf;
   const dim3 grid((N + 7) / 8);
   // (both halves of K whole pieces and offsets of 31 bits, into the stream too: the loads without conditions)
@@ -2220,11 +2222,11 @@ static void launch_into_resid(const bf16_t* A, const bf16_t* W, const float* bia
     if (pieces)                                                                                        \
       hipLaunchKernelGGL((gemm_bf16_into_resid_kernel<NW, true>), grid, dim3(NW * WAVE), 0, stream, A, \
                          W, ro.resid, M, N, K, lda, frags, ro.ldr, ro.norm_w, bias, ro.rows, ro.ss,    \
-                         ro.rows_frag);                                                                \
+                         ro.rows_frag, 0);                                                             \
     else                                                                                               \
       hipLaunchKernelGGL((gemm_bf16_into_resid_kernel<NW, false>), grid, dim3(NW * WAVE), 0, stream,   \
-                         A, W, ro.resid, M, N, K, lda, frags, ro.ldr, ro.norm_w, bias, ro.rows,        \
-                         ro.ss, ro.rows_frag);                                                         \
+                         A, W, ro.resid, M, N, K, lda, frags | w_order, ro.ldr, ro.norm_w, bias,       \
+                         ro.rows, ro.ss, ro.rows_frag, 0);                                             \
   } while (0)
   // K a wave: 128 or more where K allows it
   if (K >= 4096) INTO_RESID(16);
@@ -2253,8 +2255,8 @@ static void launch_skinny(const bf16_t* A, const bf16_t* W, const float* bias, T
                       (EPI != 3 || (size_t)(N + 16) * K * 2 < 0x7FFFFF00u);
 #define SKINNY(FRAG)                                                                                   \
   hipLaunchKernelGGL((gemm_bf16_skinny_kernel<TO, MT, NW, EPI, NT, FRAG>), grid, dim3(NW * WAVE), 0,    \
-                     stream, A, Wf ? Wf : W, fuse.rsc.ss, M, N, K, kblk, lda, (a_frag ? 1 : 0) | (Wf ? 2 : 0), \
-                     fuse.rsc.n_parts, fuse.rsc.eps, C, bias, ldc, cs, c_frag)
+                     stream, A, Wf ? Wf : W, fuse.rsc.ss, M, N, K, kblk, lda, a_frag, Wf ? 1 : 0,       \
+                     fuse.rsc.n_parts, C, bias, ldc, cs, fuse.rsc.eps, c_frag)
   if (pieces) SKINNY(true);
   else SKINNY(false);
 #undef SKINNY

@@ -201,10 +201,9 @@ __global__ __launch_bounds__(256) void shortconv_out_parts_kernel(
     const float* __restrict__ state, bf16_t* __restrict__ out, const int* __restrict__ row_seg,
     const int* __restrict__ seg_start, const int* __restrict__ seg_pos0,
     const int* __restrict__ seg_slot, int T, int D) {
-  constexpr int RUN = 1;
   constexpr int H = L - 1;
   const int c0 = (blockIdx.y * blockDim.x + threadIdx.x) * 8;
-  const int t0 = blockIdx.x * RUN;
+  const int t = blockIdx.x;
   if (c0 >= D) return;
   const size_t ld = (size_t)3 * D;
   // 8 channels of a gate of one row (at: the row's offset plus the gate's), as bfloat16
@@ -225,17 +224,15 @@ __global__ __launch_bounds__(256) void shortconv_out_parts_kernel(
     r[3] = pack_bf16x2(hi.z, hi.w);
     return r;
   };
-  // rows t0-H .. t0+RUN-1: the gates of the run and of the rows just before it
-  sc_u32x4_t vb[RUN + H], vx[RUN + H], vc[RUN];
-  const sc_u32x4_t zero = {0u, 0u, 0u, 0u};
+  // the row's gates and those of the rows just before it
+  sc_u32x4_t vb[L], vx[L];
+  const sc_u32x4_t vc = gate8((size_t)t * ld + c0 + D), zero = {0u, 0u, 0u, 0u};
 #pragma unroll
-  for (int i = 0; i < RUN + H; ++i) {
-    const int t = t0 - H + i;
-    const bool in = t >= 0 && t < T;
-    const size_t p = (size_t)(in ? t : 0) * ld + c0;
+  for (int i = 0; i < L; ++i) {
+    const bool in = t - H + i >= 0;
+    const size_t p = (size_t)(in ? t - H + i : 0) * ld + c0;
     vb[i] = in ? gate8(p) : zero;
     vx[i] = in ? gate8(p + 2 * D) : zero;
-    if (i >= H) vc[i - H] = in ? gate8(p + D) : zero;
   }
   // the 8 channels' taps lie together: 8 L floats from a 16-byte aligned address
   float wt[8 * L], bs[8];
@@ -255,45 +252,40 @@ __global__ __launch_bounds__(256) void shortconv_out_parts_kernel(
       bs[4] = b1.x, bs[5] = b1.y, bs[6] = b1.z, bs[7] = b1.w;
     }
   }
-  float bx[RUN + H][8];
+  float bx[L][8];
 #pragma unroll
-  for (int i = 0; i < RUN + H; ++i) {
+  for (int i = 0; i < L; ++i) {
     float b[8], x[8];
     sc_unpack8(vb[i], b);
     sc_unpack8(vx[i], x);
 #pragma unroll
     for (int j = 0; j < 8; ++j) bx[i][j] = b[j] * x[j];
   }
+  const int seg = row_seg[t];
+  const int first = seg_start[seg];
+  const bool fresh = seg_pos0[seg] == 0;
+  const float* st = state + ((size_t)seg_slot[seg] * D + c0) * H;
+  float cg[8], res[8];
+  sc_unpack8(vc, cg);
 #pragma unroll
-  for (int r = 0; r < RUN; ++r) {
-    const int t = t0 + r;
-    if (t >= T) break;
-    const int seg = row_seg[t];
-    const int first = seg_start[seg];
-    const bool fresh = seg_pos0[seg] == 0;
-    const float* st = state + ((size_t)seg_slot[seg] * D + c0) * H;
-    float cg[8], res[8];
-    sc_unpack8(vc[r], cg);
+  for (int j = 0; j < 8; ++j) res[j] = bs[j];
+  // tap k meets the row t - H + k, which is loaded row k
 #pragma unroll
-    for (int j = 0; j < 8; ++j) res[j] = bs[j];
-    // tap k meets the row t - H + k, which is loaded row r + k
+  for (int k = 0; k < L; ++k) {
+    const int src = t - H + k;
+    if (src >= first) {
 #pragma unroll
-    for (int k = 0; k < L; ++k) {
-      const int src = t - H + k;
-      if (src >= first) {
+      for (int j = 0; j < 8; ++j) res[j] = fmaf(wt[j * L + k], bx[k][j], res[j]);
+    } else if (!fresh) {
+      const int e = H + (src - first);            // entry of the state: H-1 is the newest
 #pragma unroll
-        for (int j = 0; j < 8; ++j) res[j] = fmaf(wt[j * L + k], bx[r + k][j], res[j]);
-      } else if (!fresh) {
-        const int e = H + (src - first);            // entry of the state: H-1 is the newest
-#pragma unroll
-        for (int j = 0; j < 8; ++j) res[j] = fmaf(wt[j * L + k], st[(size_t)j * H + e], res[j]);
-      }
+      for (int j = 0; j < 8; ++j) res[j] = fmaf(wt[j * L + k], st[(size_t)j * H + e], res[j]);
     }
-    sc_u32x4_t o;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) o[i] = pack_bf16x2(cg[2 * i] * res[2 * i], cg[2 * i + 1] * res[2 * i + 1]);
-    *reinterpret_cast<sc_u32x4_t*>(out + (size_t)t * D + c0) = o;
   }
+  sc_u32x4_t o;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) o[i] = pack_bf16x2(cg[2 * i] * res[2 * i], cg[2 * i + 1] * res[2 * i + 1]);
+  *reinterpret_cast<sc_u32x4_t*>(out + (size_t)t * D + c0) = o;
 }
 
 template <typename IN>

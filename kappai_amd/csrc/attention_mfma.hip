@@ -2151,9 +2151,6 @@ extern "C" int kappai_attn_decode_block(const void* q, int q_stride, const void*
                                          scale, n_waves, nullptr, stream);
 }
 
-// 1 when the decode kernel of this head size that splits the keys over blocks can do the per-head
-// norm, the rotation and the storing of the rows' own keys and values itself
-// (kappai_attn_decode_qk)
 // The most rows for which a step does better with kappai_attn_decode_qk than with a kernel for norm, rotation
 // and store ahead of the decode kernels (0: this head size does not take it).  Every wave of a row and kv head
 // does the prologue again.  us, two kernels / one, 32 heads of 64 on 8: 200 keys 5 rows 7.4 / 7.1, 16 rows 7.9 /
@@ -2276,7 +2273,10 @@ static int launch_decode(const void* q, int q_stride, const void* k_pool, const 
     return (int)hipErrorInvalidValue;
   // The rows' own lengths decide the keys per split when the grid has more blocks than the waves
   // aimed at (else they could not ask for longer splits than the grid's own), and not in the form
-  // with the prologue, which runs for a few rows and has no registers to spare.
+  // with the prologue, which has no registers to spare: up to 16 rows of lengths that differ do better
+  // without the rule but with the prologue (16 rows of 100 to 7,100 keys, 32 heads of 64 on 8 and 16 on 8: 35.8 and
+  // 34.4 us with a kernel for norm, rotation and store and the rule, 32.5 and 33.0 so; one of 8,000 keys among 15 of
+  // 200: 20.4 and 19.9, 17.5 and 17.4).
   const bool plan = !qk.on && (long long)T * G * n_splits > D_TARGET_WAVES;
 #define KAPPAI_DECODE(FUSED, PLAN, MODS)                                                         \
   hipLaunchKernelGGL((attn_decode_kernel<FUSED, PLAN, MODS>), dim3(T, G, n_splits), dim3(WAVE),  \

@@ -61,9 +61,9 @@ def fused_conv_step(width: int, rows: int, in_fragments: bool) -> bool:
 # stores key and value (head sizes 64 and 128, rotate-half over the whole head, a projection that
 # comes as bfloat16 rows, more than 512 keys or head size 64) for steps of up to FUSED_QK_MAX_ROWS rows and
 # no more than the kernel itself says (``ops.decode_qk_rows``: 16 at head size 64, 4 at 128): every wave of the
-# kernel does that work again, beside its first keys' way.  A step of six such layers, 8 rows at 60 to 7,000 keys: 0
-# to 10 us less; at 12 and 16 rows 1 to 13.  (Until its arguments came in the order of need the line was at 4: 12 us
-# more at 8 rows.)  0 switches it off.
+# kernel does that work again, beside its first keys' way.  A layer's kernels, 5 to 16 rows of 60 to 12,000 keys, of
+# one length and of mixed ones, 8 to 64 heads of 64 on 1 to 32 kv heads: 0 to 7 us less in place of 6 to 100, a
+# tenth on average (``ops.QK_BLOCKS`` is the exception).  0 switches it off.
 FUSED_QK = True
 FUSED_QK_MAX_ROWS = 16
 

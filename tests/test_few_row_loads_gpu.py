@@ -180,3 +180,32 @@ def test_conv_step_of_very_many_channels():
     # (a gate may round the other way: 2^-7 of it; the result's own rounding beside that)
     slack = c.abs() * (4 * 2.0 ** -7 * (terms.abs().sum(1) + conv_bias[-16:].double().abs()))
     assert ((got[0, -16:].double() - want).abs() <= slack).all().item()
+
+
+def test_rows_of_x_more_than_two_gibibytes_apart():
+    """Rows of x so far apart that offsets within them take more than 31 bits: the kernels over fragment order that
+    carry conditions give the bits of those without, whose rows lie side by side."""
+    K = 64
+    g = _gen(K, 11)
+    for M, apart in ((16, 67_200_000), (24, 44_800_000)):
+        assert M * apart * 2 > 1 << 31
+        far = torch.empty((M - 1) * apart + K, device=DEV, dtype=BF16).as_strided((M, K), (apart, 1))
+        x = torch.randn(M, K, generator=g, device=DEV).to(BF16)
+        far.copy_(x)
+        W, _ = _matrix(96, K, g)
+        taps, state = torch.randn(32, 3, generator=g, device=DEV), torch.randn(M, 32, 2, generator=g, device=DEV)
+        rows = torch.arange(M, device=DEV, dtype=torch.int32)
+
+        def results(x):
+            st = state.clone()
+            out = [ops.linear(x, W, out_dtype=torch.float32), ops.linear_swiglu(x, W),
+                   ops.linear_shortconv_step(x, W, None, taps, None, st, rows, rows), st]
+            if M <= 16:
+                resid, norm = torch.ones(M, 96, device=DEV), torch.linspace(0.5, 1.5, 96, device=DEV)
+                scaled = ops.linear(x, W, add_into=ops.AddInto(resid, norm, 1e-5))
+                out += [resid, scaled.data[:M] if not scaled.fragment else scaled.data, scaled.ss[:, :M]]
+            return out
+
+        for got, want in zip(results(far), results(x)):
+            assert torch.equal(got, want)
+        del far

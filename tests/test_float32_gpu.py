@@ -172,3 +172,16 @@ def test_attention_around_whole_rounds_of_its_waves(ops, d, n_new, window):  # n
                               scale, window=window)
     want = ref.paged_attention(q, H, G, d, k, v, *rows, bt, ps, scale, window=window)
     close(got, want, 6e-6, "attention")
+
+
+@pytest.mark.parametrize("M,N,K", [(70, 130, 256), (330, 9216, 128)])
+def test_blocks_over_operands_of_four_gibibytes_give_the_same_bits(ops, M, N, K):  # noqa: F811
+    """Rows of x so far apart that 32 bits do not address them: tiles through registers and not straight into LDS."""
+    apart = (1 << 30) // M + 4 & ~3
+    far = torch.empty((M - 1) * apart + K, device=DEV).as_strided((M, K), (apart, 1))
+    x, w = rand((M, K), F32, 71).to(DEV), rand((N, K), F32, 72).to(DEV)
+    far.copy_(x)
+    assert M * apart >= 1 << 30 and apart % 4 == 0
+    assert torch.equal(ops.linear(far, w), ops.linear(x, w))
+    if ops.linear_swiglu_f32_takes(x, w):
+        assert torch.equal(ops.linear_swiglu_f32(far, w), ops.linear_swiglu_f32(x, w))

@@ -266,8 +266,10 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t hw_buffer(const void* p) {
 // Few rows are bound by how often they wait for memory, so STEPS steps' loads (and the gates) are asked for
 // before anything is multiplied, without conditions: what a lane must not read lies outside its buffer.  One row of 16
 // heads, 224 to 64, 3.95 us with a wait a step of 32, 2.9 so; 128 to 64 with gates and a wait a gate 5.7, 4.2 so;
-// 300 rows of these 5.7 either way and 8.6 / 7.3, 1,900 rows 10.3 either way and 12.4 / 13.1.
-// GATE: 1 the gates are asked for with the first steps (few rows), 2 behind the products, 0 there are none.
+// 300 rows of these 5.7 either way and 8.6 / 7.3.
+// GATE: 1 the gates are asked for with the first steps (few rows), 2 behind the products, 3 one at a time as they
+// are used (waves enough to cover for one another, see the launch), 0 there are none.
+#define HW_GATES_ASKED_WAVES 1024
 template <typename TO, int STEPS, int GATE>
 __global__ __launch_bounds__(256) void headwise_linear_mfma_kernel(
     const bf16_t* __restrict__ x, const bf16_t* __restrict__ w, int x_row, int x_head, int n_out,
@@ -333,7 +335,9 @@ __global__ __launch_bounds__(256) void headwise_linear_mfma_kernel(
       const int n = n0 + 16 * j + 4 * kq + v;
       if (n >= n_out) continue;
       float r = acc[j][v];
-      if (GATE) r /= 1.0f + expf(-__uint_as_float((uint32_t)gates[j][v] << 16));
+      if (GATE == 1 || GATE == 2) r /= 1.0f + expf(-__uint_as_float((uint32_t)gates[j][v] << 16));
+      if (GATE == 3)
+        r /= 1.0f + expf(-bf16_to_f32(gate[(size_t)(m0 + lr) * g_row + (size_t)h * n_out + n]));
       from_f32(yr + n, r);
     }
 #endif
@@ -355,7 +359,11 @@ extern "C" int kappai_headwise_linear(const void* x, int x_row, int x_head, cons
     const dim3 grid((rows + 16 * waves - 1) / (16 * waves), (n_out + 63) / 64, H);
     // Few rows: all steps' loads at once, up to eight.  More: waves enough to cover for one another, a step at a
     // time (us with places for four steps / one, no gates: 300 rows of 32 to 32 3.1 / 2.8, 1,900 rows of 16 heads 64 to 224
-    // 26.0 / 24.1, 224 to 64 10.6 / 10.3).
+    // 26.0 / 24.1, 224 to 64 10.6 / 10.3).  With more than one wave a SIMD of the chip they cover for the gates' loads as
+    // well (us with all gates asked for / each where it is used, 1,000 rows of 16 heads 128 to 64, 1,008 waves, 7.7 / 8.6;
+    // 1,300 rows 13.0 / 12.5, 1,900 rows 13.4 / 12.6; 300 rows of 64 to 224, 1,216 waves, 11.1 / 10.6; from 4,000 waves on
+    // either is ahead by up to 4 %).
+    const bool covered = (long long)((rows + 15) / 16) * grid.y * H > HW_GATES_ASKED_WAVES;
 #define HEADWISE(TO, STEPS, GATE)                                                                      \
   hipLaunchKernelGGL((headwise_linear_mfma_kernel<TO, STEPS, GATE>), grid, dim3(waves * WAVE), 0, stream, \
                      (const bf16_t*)x, (const bf16_t*)w, x_row, x_head, n_out, n_in, rows,             \
@@ -369,7 +377,8 @@ extern "C" int kappai_headwise_linear(const void* x, int x_row, int x_head, cons
   } while (0)
 #define HEADWISE_AS(TO)                                                                                \
   do {                                                                                                 \
-    if (waves > 1 && gate != nullptr) HEADWISE(TO, 1, 2);                                              \
+    if (waves > 1 && gate != nullptr && covered) HEADWISE(TO, 1, 3);                                   \
+    else if (waves > 1 && gate != nullptr) HEADWISE(TO, 1, 2);                                         \
     else if (waves > 1) HEADWISE(TO, 1, 0);                                                            \
     else if (gate != nullptr) HEADWISE_FEW(TO, 1);                                                     \
     else HEADWISE_FEW(TO, 0);                                                                          \

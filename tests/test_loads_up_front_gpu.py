@@ -40,6 +40,33 @@ def test_headwise_linear(T, n_out, n_in, gated):
     assert ((got - want).abs() <= size * (n_in + 8) * EPS).all().item()
 
 
+@pytest.mark.parametrize("T", [1024, 1025])
+@pytest.mark.parametrize("n_out,n_in", [(64, 64), (63, 40), (65, 64)])
+@pytest.mark.parametrize("out_dtype", [torch.float32, BF16])
+def test_headwise_linear_gates_around_a_wave_a_simd(T, n_out, n_in, out_dtype):
+    """16 heads: 1,024 waves and 1,040 where 64 columns hold the outputs, twice as many else.  Gates stand in
+    rows with NaN behind them; the rows on either side of the rule are the same to the bit."""
+    g = _gen(T, n_out, n_in)
+    H = 16
+    x = torch.randn(1025, H * n_in, generator=g, device=DEV).to(BF16)[:T]
+    w = torch.randn(H, n_out, n_in, generator=g, device=DEV).to(BF16)
+    rows = torch.full((1025, H * n_out + 5), float("nan"), device=DEV, dtype=BF16)
+    gate = rows[:T, :H * n_out]
+    gate.copy_(torch.randn(T, H * n_out, generator=g, device=DEV) * 3)
+    got = ops.headwise_linear(x, n_in, w, out_dtype=out_dtype, gate=gate)
+    few = torch.cat([ops.headwise_linear(x[i:i + 200], n_in, w, out_dtype=out_dtype, gate=gate[i:i + 200])
+                     for i in range(0, T, 200)])
+    assert torch.equal(got, few)
+    s = torch.sigmoid(gate.double().cpu()).view(T, H, n_out)
+    a, b = x.double().cpu().view(T, H, n_in), w.double().cpu()
+    want = torch.stack([a[:, h] @ b[h].T for h in range(H)], 1) * s
+    size = torch.stack([a[:, h].abs() @ b[h].abs().T for h in range(H)], 1) * s
+    bound = size * (n_in + 8) * EPS
+    if out_dtype == BF16:
+        bound = bound + want.abs() * 2.0 ** -8
+    assert ((got.view(T, H, n_out).double().cpu() - want).abs() <= bound).all().item()
+
+
 @pytest.mark.parametrize("part", [64, 128, 96])
 @pytest.mark.parametrize("n", [1, 2, 4, 5])
 @pytest.mark.parametrize("T", [1, 3])

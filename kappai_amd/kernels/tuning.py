@@ -12,9 +12,12 @@ numbers in its model description.
 PARTIAL_SUMS_MIN_ROWS = 16
 # ... and in steps of up to this many rows whatever their segments (short prompt portions): with
 # few rows the products of in_proj and qkv have too few blocks to fill the chip unless K is cut
-# (in_proj of 128 rows: 9-12 us in four ranges against 22 us whole; the float partial sums of
-# 512 rows would already cost more than the cut saves).  Above it only steps of single rows
-# (decode at large batches) hand on partial sums.
+# (in_proj of 128 rows of the 1.2B shape: 9-12 us in four ranges against 22 us whole).  Above it only steps of
+# single rows (decode at large batches) hand on partial sums.  us a prompt step, whole / in sums, 1.2B shape (width
+# 2,048): 64 rows 1,043 / 1,014, 128 rows 1,295 / 1,247, 256 rows 1,466 / 1,422, 320 rows 1,540 / 1,563, 417 rows of
+# three prompts 1,646 / 1,628; but 24 rows 848 / 890.  At the 350M shape (width 1,024) sums are behind, 64 rows
+# 706 / 756, 128 rows 838 / 881, 256 rows 916 / 926: their convolution is two kernels, 13.9 us a layer, that of whole
+# products one of 4.3.
 PARTIAL_SUMS_MAX_ROWS = 256
 
 

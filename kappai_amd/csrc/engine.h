@@ -35,6 +35,14 @@ extern "C" {
 // with a kernel of their own / inside, 32 heads of 64 on 32: 8 rows of 200 keys 8.8 / 8.0, of 500 12.0 / 10.9; 12 rows of
 // 200 12.6 / 13.6, of 500 18.4 / 18.9; 16 rows 13.3 / 14.1 and 21.0 / 21.4 (16 rows on 16 kv heads 8.8 / 8.0 and 11.9 / 10.7).
 #define KAPPAI_QK_BLOCKS 256
+// ... and inside the one that splits a row's keys over blocks: for more than four rows, over bounds of more than so
+// many keys, up to this many (row, kv head) pairs.  Splits then follow the longest row's bound and not the rows' own
+// keys (the form without the prologue has registers for that).  ms a step of the 1.2B shape (six such layers, 8 kv heads)
+// with a kernel of its own / inside: 16 rows of 32,800 keys 1.96 / 1.93, of 44,000
+// keys 2.36 / 2.34, 52,000 2.58 / 2.68, 80,000 3.49 / 3.67, 110,000 4.48 / 4.78; 12 rows of 60,000 2.36 / 2.42, of 90,000
+// 3.11 / 3.14; but 10 rows of 110,000 3.49 / 3.22, 8 rows of 60,000 1.785 / 1.796, of 131,072 2.98 / 2.97.
+#define KAPPAI_QK_LONG_KEYS 32768
+#define KAPPAI_QK_LONG_BLOCKS 80
 
 // ---- the kernels' launchers, by address (they live in libraries of their own) ---------------
 typedef struct kappai_kernels {

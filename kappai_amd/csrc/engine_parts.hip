@@ -207,9 +207,10 @@ kappai_carry attention_mixer(kappai_step* s, const void* desc, kappai_rows x, fl
       M <= tune.fused_qk && M <= qk_rows && single && proj.kind == KAPPAI_CARRY_DELTA && !proj.is_f32 &&
       L.mfma != nullptr && H / G <= 16 && qkv.n % 8 == 0 && aligned16(proj.data) && ps % 16 == 0 &&
       d % 16 == 0 && d <= 256 && (L.rot_mode == 0 || (L.rot_mode == 1 && L.rot_dim == d)) &&
-      (!decode_block_form(m, b, L, M) ||
-       (L.mfma->decode_block_qk_keys != nullptr && (long)M * G <= KAPPAI_QK_BLOCKS &&
-        decode_keys(b, L) <= L.mfma->decode_block_qk_keys()));
+      (decode_block_form(m, b, L, M)
+           ? L.mfma->decode_block_qk_keys != nullptr && (long)M * G <= KAPPAI_QK_BLOCKS &&
+                 decode_keys(b, L) <= L.mfma->decode_block_qk_keys()
+           : M <= 4 || (long)M * G <= KAPPAI_QK_LONG_BLOCKS || decode_keys(b, L) <= KAPPAI_QK_LONG_KEYS);
   // q in place in the projection, or (from partial sums) a new bfloat16 [M, H d]
   void* q;
   int q_stride, q_bf16;

@@ -988,6 +988,17 @@ def decode_block_takes_qk(head_dim: int, max_position: int, window: int = 0, n_b
             <= library("attention_mfma", HEAD_DIM=head_dim).kappai_attn_decode_block_qk_keys())
 
 
+QK_LONG_KEYS = 32768       # KAPPAI_QK_LONG_KEYS, KAPPAI_QK_LONG_BLOCKS (engine.h)
+QK_LONG_BLOCKS = 80
+
+
+def decode_split_takes_qk(n_rows: int, n_kv_heads: int, max_position: int, window: int = 0) -> bool:
+    """Whether a step does better with a ``QkPrologue`` in the kernel that splits keys over blocks: not with many
+    (row, kv head) pairs over very long contexts."""
+    return (n_rows <= 4 or n_rows * n_kv_heads <= QK_LONG_BLOCKS
+            or keys_bound(max_position, window) <= QK_LONG_KEYS)
+
+
 def paged_attention(q: torch.Tensor, n_heads: int, n_kv_heads: int, head_dim: int,
                     k_pool: torch.Tensor, v_pool: torch.Tensor, row_pos: torch.Tensor,
                     row_seg: torch.Tensor, block_tables: torch.Tensor, page_size: int,

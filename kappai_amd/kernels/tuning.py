@@ -66,7 +66,7 @@ def fused_conv_step(width: int, rows: int, in_fragments: bool) -> bool:
 # no more than the kernel itself says (``ops.decode_qk_rows``: 16 at head size 64, 4 at 128): every wave of the
 # kernel does that work again, beside its first keys' way.  A layer's kernels, 5 to 16 rows of 60 to 12,000 keys, of
 # one length and of mixed ones, 8 to 64 heads of 64 on 1 to 32 kv heads: 0 to 7 us less in place of 6 to 100, a
-# tenth on average (``ops.QK_BLOCKS`` is the exception).  0 switches it off.
+# tenth on average (``ops.QK_BLOCKS`` and ``ops.QK_LONG_BLOCKS`` are the exceptions).  0 switches it off.
 FUSED_QK = True
 FUSED_QK_MAX_ROWS = 16
 

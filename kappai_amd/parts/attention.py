@@ -221,8 +221,8 @@ class GroupedQueryAttention(Mixer):
         ``ops.QkPrologue``): a step of a few single rows whose projection came as bfloat16 rows, few
         enough query heads a kv head for the decode kernels, a head size they do it for, no
         rotation or rotate-half over the whole head, and keys enough for the kernel that splits
-        them over blocks or few enough for the one that keeps them in a block
-        (``ops.decode_block_takes_qk``)."""
+        them over blocks (``ops.decode_split_takes_qk``) or few enough for the one that keeps them in
+        a block (``ops.decode_block_takes_qk``)."""
         if not (tuning.FUSED_QK and single_rows and isinstance(proj, torch.Tensor)
                 and proj.dim() == 2 and proj.shape[0] <= tuning.FUSED_QK_MAX_ROWS
                 and proj.dtype == torch.bfloat16 and proj.is_cuda
@@ -232,11 +232,12 @@ class GroupedQueryAttention(Mixer):
         if rot is not None and not (rot.mode == ops.ROT_HALF and rot.rot_dim == self.d):
             return False
         window = self.window or 0
-        return (proj.shape[0] <= ops.decode_qk_rows(self.d, page_size)
-                and (ops.decode_form(self.H, self.G, self.d, max_position, window,
-                                     n_rows=proj.shape[0]) == "decode-split"
-                     or ops.decode_block_takes_qk(self.d, max_position, window,
-                                                  proj.shape[0] * self.G)))
+        rows = proj.shape[0]
+        if rows > ops.decode_qk_rows(self.d, page_size):
+            return False
+        if ops.decode_form(self.H, self.G, self.d, max_position, window, n_rows=rows) == "decode-split":
+            return ops.decode_split_takes_qk(rows, self.G, max_position, window)
+        return ops.decode_block_takes_qk(self.d, max_position, window, rows * self.G)
 
     def weight_bytes(self) -> int:
         return self.qkv.weight_bytes() + self.out.weight_bytes() + 2 * self.d * 4

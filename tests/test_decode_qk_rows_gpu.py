@@ -12,7 +12,10 @@ pytestmark = pytest.mark.gpu
 def test_where_the_rule_lies(ops):  # noqa: F811
     assert [ops.decode_qk_rows(d, 16) for d in (64, 128, 48, 256)] == [16, 4, 0, 0]
     assert ops.decode_qk_rows(64, 8) == 0
-    # (kept in one block: up to a block a CU)
+    # (keys over blocks: not many pairs over very long contexts; kept in one block: up to a block a CU)
+    assert [ops.decode_split_takes_qk(n, 8, p) for n, p in ((4, 99999), (10, 99999), (11, 32767), (11, 32768))] == \
+        [True, True, True, False]
+    assert ops.decode_split_takes_qk(4, 32, 99999) and ops.decode_split_takes_qk(16, 8, 99999, 4096)
     assert [ops.decode_block_takes_qk(64, 400, 0, n) for n in (16, 256, 257)] == [True, True, False]
 
 

@@ -367,11 +367,12 @@ def test_decode_attention_with_its_prologue_inside_from_c_and_from_the_host(tmp_
 
 
 @pytest.mark.parametrize("kv_heads,longest,sizes,most_qk", [(4, 1500, [4, 5, 16, 17, 48, 49], 16),
-                                                             (32, 400, [8, 9], 8)])
+                                                             (32, 400, [8, 9], 8),
+                                                             (8, 33000, [10, 11], 10)])
 def test_decode_steps_on_both_sides_of_the_rules_from_c_and_from_the_host(tmp_path, monkeypatch, kv_heads, longest,
                                                                           sizes, most_qk):
     """Which kernels a decode step takes is a rule that the C side and the host's parts hold each for itself: up to
-    16 rows (over short contexts, 256 rows times kv heads) the attention kernel normalises, rotates and stores (head
+    16 rows (over short contexts, 256 rows times kv heads, beyond 32,768 keys 80 of them) the attention kernel normalises, rotates and stores (head
     size 64), up to 48 rows a conv layer over matrices in fragment order is one kernel.  Steps on both sides of these
     lines, over contexts of mixed lengths: the logits are the same bits either way, and the host's parts took the
     kernels that the rules name."""
@@ -381,7 +382,8 @@ def test_decode_steps_on_both_sides_of_the_rules_from_c_and_from_the_host(tmp_pa
     from kappai_amd.engine import StepEntry, StepRunner
     from kappai_amd.kernels import ops
     from kappai_amd.weights import write_random_model
-    raw = dict(copy.deepcopy(WIDE), num_key_value_heads=kv_heads, num_attention_heads=max(16, kv_heads))
+    raw = dict(copy.deepcopy(WIDE), num_key_value_heads=kv_heads, num_attention_heads=max(16, kv_heads),
+               max_position_embeddings=40960)
     folder = write_random_model(tmp_path / "wide", config_from_dict(raw), seed=9, std=0.02, norm_jitter=0.05)
     lengths = [longest + len(sizes), longest // 2, 300] + [8 + 5 * i % 61 for i in range(max(sizes) - 3)]
     requests = make_requests(WIDE["vocab_size"], lengths, seed=18)

@@ -691,6 +691,56 @@ __device__ __forceinline__ int2 xcd_tile(int b, int tiles_m, int tiles_n) {
   return make_int2(g * GROUP + j % gm, xcd * band + j / gm);
 }
 
+// The same for blocks over a W in fragment order, K ranges among the things to be placed, on a grid of one
+// dimension: an XCD is given an equal run of the list of all blocks, ranges slowest, then groups of `group` row
+// tiles, then columns, the rows of a group fastest.  What an XCD reads of A and W comes to it once over its
+// link (0.7 to 0.8 TB/s) and then out of its L2, so its run should lie in as few ranges as it can and be as
+// square as it can within them (xcd_group).  With a band of column tiles for each XCD, every range among
+// them, each XCD took in all of A: down, 2048 x 8192, 417 rows in four ranges 88 MB over the links, 47 so.  us so
+// and with bands, W from memory: that product 22.6 and 23.9, 2048 x 10752 26.3 and 28.9; 1024 x 4608 of 575
+// rows in six ranges 11.9 and 13.9, of 1900 in four 24.0 and 28.9; 2048 x 8192 of 2048 rows in two 62.1 and 63.2;
+// whole products 1 to 3 % less (gate/up 9216 x 1024 of 1900 rows 42.4 and 44.9).  `cut`: group + 65536 * ranges.
+struct BlockPlace {
+  int m, n, range;
+};
+__device__ __forceinline__ BlockPlace xcd_place(int tiles_m, int tiles_n, uint32_t cut) {
+  constexpr uint32_t XCDS = 8;
+  const uint32_t plane = tiles_m * tiles_n, ranges = cut >> 16, group = cut & 0xffff, total = plane * ranges;
+  const uint32_t b = blockIdx.x, xcd = b % XCDS, tail = total % XCDS;
+  uint32_t j = xcd * (total / XCDS) + (xcd < tail ? xcd : tail) + b / XCDS, g = 0;
+  BlockPlace at;
+  at.range = 0;
+  if (ranges > 1) {
+    at.range = j / plane;
+    j -= at.range * plane;
+  }
+  if (group < (uint32_t)tiles_m) {
+    g = j / (group * tiles_n);
+    j -= g * (group * tiles_n);
+  }
+  const uint32_t left = tiles_m - g * group, gm = group < left ? group : left;
+  at.n = j / gm;
+  at.m = g * group + j - at.n * gm;
+  return at;
+}
+// Row tiles of a group: the blocks that an XCD runs at one time read the fewest rows of A and W between them (even
+// groups; of equals the larger, which reads W in fewer XCDs).  Over 118 products of 300 to 2,048 rows the group
+// chosen so takes 1 % more than the best of all groups in sum.
+static int xcd_group(int tiles_m, int tiles_n, int ranges, int rows, int cols) {
+  const int share = (tiles_m * tiles_n * ranges + 7) / 8, at_once = share < 32 ? share : 32;
+  int best = 1, best_cost = -1;
+  for (int g = tiles_m < 32 ? tiles_m : 32; g > 0; --g) {
+    const int groups = (tiles_m + g - 1) / g, even = (tiles_m + groups - 1) / groups;
+    if (even != g) continue;
+    const int cost = g * rows + (at_once + g - 1) / g * cols;
+    if (best_cost < 0 || cost < best_cost) {
+      best = g;
+      best_cost = cost;
+    }
+  }
+  return best;
+}
+
 template <typename TO, int EPI, int WAVES_M, int WAVES_N, int WM, int WN, int BK, int NBUF,
           int OCC>
 __global__ __launch_bounds__(WAVES_M * WAVES_N * WAVE)
@@ -891,7 +941,7 @@ template <int N> struct IntC { static constexpr int value = N; };
 template <typename TO, int EPI, int WTM, int WTN>
 __device__ __forceinline__ void block_epilogue(const f32x16_t (&acc)[WTM][WTN], bf16_t* lds,
                                                const float* bias, TO* C, int M, int N, int ldc, int m0,
-                                               int n0, int wave, int lane) {
+                                               int n0, int range, int wave, int lane) {
   const int wm = wave / 2, wn = wave % 2, r_in = lane % 32, hh = lane / 32;
   constexpr int WROWS_N = WTN * 32;
   constexpr int OUT_COLS = EPI == 1 ? WROWS_N / 2 : WROWS_N;   // columns a wave writes
@@ -919,7 +969,7 @@ __device__ __forceinline__ void block_epilogue(const f32x16_t (&acc)[WTM][WTN], 
           c = j * 32 + 8 * g + 4 * hh;
 #pragma unroll
           for (int e = 0; e < 4; ++e) v4[e] = acc[i][j][4 * g + e];
-          if (bias && blockIdx.y == 0) {
+          if (bias && range == 0) {
 #pragma unroll
             for (int e = 0; e < 4; ++e)
               if (col0 + c + e < out_n) v4[e] += bias[col0 + c + e];
@@ -1197,7 +1247,7 @@ void gemm_bf16_block256_kernel(const bf16_t* __restrict__ A, const bf16_t* __res
   }
 
   __syncthreads();                               // everybody is done with the last tile
-  block_epilogue<TO, EPI, WTM, WTN>(acc, lds, bias, C, M, N, ldc, m0, n0, wave, lane);
+  block_epilogue<TO, EPI, WTM, WTN>(acc, lds, bias, C, M, N, ldc, m0, n0, blockIdx.y, wave, lane);
 }
 
 // Block products whose W lies in fragment order ([rows / 16][K / 32] pieces of 16 rows x 32 of K, 1 KB
@@ -1225,7 +1275,7 @@ template <typename TO, int EPI, int WTM, int WTN>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1)))
 void gemm_bf16_direct_kernel(const bf16_t* __restrict__ A, const bf16_t* __restrict__ W,
                              const float* __restrict__ bias, TO* __restrict__ C, int M, int N,
-                             int K, int lda, int ldc, int tiles_n) {
+                             int K, int lda, int ldc, int tiles_m, int tiles_n, uint32_t cut) {
   constexpr int BM = WTM * 64, BN = WTN * 64, BK = 64, NB = 4, SLOTS = 8;
   constexpr int NPROD = WTM * WTN, NA = BM / 32;               // loads of A a wave and tile
   constexpr int A_TILE = BM * BK;                              // in bf16
@@ -1233,12 +1283,12 @@ void gemm_bf16_direct_kernel(const bf16_t* __restrict__ A, const bf16_t* __restr
   const int tid = threadIdx.x, lane = tid % WAVE;
   const int wave = __builtin_amdgcn_readfirstlane(tid / WAVE);
   const int wm = wave / 2, wn = wave % 2;
-  const int2 tile = xcd_tile(blockIdx.x, gridDim.x / tiles_n, tiles_n);
-  const int m0 = tile.x * BM, n0 = tile.y * BN;
-  const int kblk = K / (int)gridDim.y;
+  const BlockPlace place = xcd_place(tiles_m, tiles_n, cut);
+  const int m0 = place.m * BM, n0 = place.n * BN;
+  const int kblk = cut >> 17 ? (int)((uint32_t)K / (cut >> 16)) : K;
   const int nk = kblk / BK;
-  const int k0 = (int)blockIdx.y * kblk;
-  C += (size_t)blockIdx.y * M * ldc;
+  const int k0 = place.range * kblk;
+  C += (size_t)place.range * M * ldc;
 
   f32x16_t acc[WTM][WTN];
 #pragma unroll
@@ -1359,7 +1409,7 @@ void gemm_bf16_direct_kernel(const bf16_t* __restrict__ A, const bf16_t* __restr
   // (the loads of tiles that are not there have ended too: the epilogue uses their LDS)
   WAIT_LOADS_AND_LDS(0);
   __syncthreads();
-  block_epilogue<TO, EPI, WTM, WTN>(acc, lds, bias, C, M, N, ldc, m0, n0, wave, lane);
+  block_epilogue<TO, EPI, WTM, WTN>(acc, lds, bias, C, M, N, ldc, m0, n0, place.range, wave, lane);
 }
 
 // The same product with both operands in LDS, NB buffers, for blocks whose tile is small beside what it
@@ -1374,7 +1424,7 @@ template <typename TO, int EPI, int WTM, int WTN, int NB>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1)))
 void gemm_bf16_staged_kernel(const bf16_t* __restrict__ A, const bf16_t* __restrict__ W,
                              const float* __restrict__ bias, TO* __restrict__ C, int M, int N,
-                             int K, int lda, int ldc, int tiles_n) {
+                             int K, int lda, int ldc, int tiles_m, int tiles_n, uint32_t cut) {
   constexpr int BM = WTM * 64, BN = WTN * 64, BK = 64;
   constexpr int NPROD = WTM * WTN, NREAD = WTM + WTN;
   constexpr int NA = BM / 32, NW = BN / 32, NLOAD = NA + NW;   // loads a wave and tile
@@ -1383,12 +1433,12 @@ void gemm_bf16_staged_kernel(const bf16_t* __restrict__ A, const bf16_t* __restr
   const int tid = threadIdx.x, lane = tid % WAVE;
   const int wave = __builtin_amdgcn_readfirstlane(tid / WAVE);
   const int wm = wave / 2, wn = wave % 2;
-  const int2 tile = xcd_tile(blockIdx.x, gridDim.x / tiles_n, tiles_n);
-  const int m0 = tile.x * BM, n0 = tile.y * BN;
-  const int kblk = K / (int)gridDim.y;
+  const BlockPlace place = xcd_place(tiles_m, tiles_n, cut);
+  const int m0 = place.m * BM, n0 = place.n * BN;
+  const int kblk = cut >> 17 ? (int)((uint32_t)K / (cut >> 16)) : K;
   const int nk = kblk / BK;
-  const int k0 = (int)blockIdx.y * kblk;
-  C += (size_t)blockIdx.y * M * ldc;
+  const int k0 = place.range * kblk;
+  C += (size_t)place.range * M * ldc;
   f32x16_t acc[WTM][WTN];
 #pragma unroll
   for (int i = 0; i < WTM; ++i)
@@ -1495,7 +1545,7 @@ void gemm_bf16_staged_kernel(const bf16_t* __restrict__ A, const bf16_t* __restr
 #endif
   WAIT_LOADS_AND_LDS(0);
   __syncthreads();
-  block_epilogue<TO, EPI, WTM, WTN>(acc, lds, bias, C, M, N, ldc, m0, n0, wave, lane);
+  block_epilogue<TO, EPI, WTM, WTN>(acc, lds, bias, C, M, N, ldc, m0, n0, place.range, wave, lane);
 }
 
 template <typename TO, int EPI>
@@ -1534,7 +1584,7 @@ static void launch_fragment_block(const bf16_t* A, const bf16_t* Wf, const float
   // the tiles of A (and W), or what the epilogue turns its rows in
   constexpr size_t lds_bytes = NB * (BM + (DIRECT ? 0 : BN)) * 64 * sizeof(bf16_t);
   static_assert(4 * 32 * (WTN * 32 * 4 + 16) <= lds_bytes && lds_bytes <= 160 * 1024, "LDS");
-  void (*kern)(const bf16_t*, const bf16_t*, const float*, TO*, int, int, int, int, int, int);
+  void (*kern)(const bf16_t*, const bf16_t*, const float*, TO*, int, int, int, int, int, int, int, uint32_t);
   if constexpr (DIRECT) kern = gemm_bf16_direct_kernel<TO, EPI, WTM, WTN>;
   else kern = gemm_bf16_staged_kernel<TO, EPI, WTM, WTN, NB>;
   static bool attr_set = false;       // more than 64 KB of LDS has to be asked for once
@@ -1544,8 +1594,9 @@ static void launch_fragment_block(const bf16_t* A, const bf16_t* Wf, const float
     attr_set = true;
   }
   const int tn = (n_rows_w + BN - 1) / BN, tm = (M + BM - 1) / BM;
-  hipLaunchKernelGGL(kern, dim3(tm * tn, ksplit), dim3(256), lds_bytes, stream, A, Wf, bias, C, M,
-                     n_rows_w, K, lda, ldc, tn);
+  const uint32_t cut = (uint32_t)xcd_group(tm, tn, ksplit, BM, BN) + 65536u * ksplit;
+  hipLaunchKernelGGL(kern, dim3(tm * tn * ksplit), dim3(256), lds_bytes, stream, A, Wf, bias, C, M,
+                     n_rows_w, K, lda, ldc, tm, tn, cut);
 }
 
 // shape: 0 = chosen by size, 1 = 128x128 blocks of two waves, 2 = 256x128 blocks (tiles of 32

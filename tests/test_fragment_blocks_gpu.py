@@ -95,3 +95,16 @@ def test_nothing_is_written_behind_the_gated_result(ops, M, F, K, form):  # noqa
     assert status == 0
     assert torch.equal(out[:M, :F], ops.linear_swiglu(x, w, force_kernel=ROWS))
     assert (out[:, F:] == mark).all() and (out[M:] == mark).all()
+
+
+# more row tiles than a group of neighbours takes, groups that are not all of one size, a number of blocks that is
+# no multiple of eight: every block of every range has its place
+@pytest.mark.parametrize("M,N,K,S", [(1900, 384, 256, 2), (2180, 656, 384, 3), (4500, 144, 128, 1),
+                                     (1100, 2576, 256, 1)])
+@pytest.mark.parametrize("form", list(FORMS))
+def test_every_block_has_its_place(ops, M, N, K, S, form):  # noqa: F811
+    x, w = rand((M, K), BF16, 91).to(DEV), rand((N, K), BF16, 92).to(DEV)
+    kept = ops.InFragments.of(w)
+    how = dict(partial_sums=True, split_k=S) if S > 1 else dict(out_dtype=F32)
+    assert torch.equal(ops.linear(x, kept, force_kernel=FORMS[form], **how),
+                       ops.linear(x, w, force_kernel=ROWS, **how))

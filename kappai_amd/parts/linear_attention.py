@@ -64,6 +64,21 @@ def _chunk_rows(batch, dtype=torch.bfloat16) -> int:
     return ops.MATRIX_STATE_CHUNK_ROWS if chunked else 0
 
 
+def _recurrence(batch, q, k, v, z, H, G, d, dv, rate, bias, sign, scale, state, norm, chunking,
+                **kinds) -> torch.Tensor:
+    """The recurrence with the norm and its gate (``ops.GatedNorm``) behind it: one kernel where every
+    segment is a single row, else the recurrence as ``chunking`` says and the norm as a kernel of its own."""
+    tables = (batch.seg_start, batch.seg_pos0, batch.seg_slot)
+    mode = 1 if kinds.get("beta") is not None else 2 if kinds.get("bonus") is not None else 0
+    if batch.max_segment_rows == 1 and ops.matrix_state_step_takes(q, state, mode, norm):
+        return ops.matrix_state_step(q, k, v, z, H, G, d, dv, rate, bias, sign, scale, state, *tables,
+                                     norm=norm, **kinds)
+    o = ops.matrix_state_recurrence(q, k, v, z, H, G, d, dv, rate, bias, sign, scale, state, *tables,
+                                    **chunking, **kinds)
+    return ops.head_norm_gate(o, norm.weight, norm.eps, norm.gate, norm.gate_kind, norm.n_heads,
+                              norm.vdim, q.dtype)
+
+
 class GatedLinearAttention(Mixer):
     def __init__(self, prefix: str, width: int, num_heads: int, dim: int, vdim: int, tau: float,
                  decay_rank: int, norm_eps: float, dtype: torch.dtype, names=None,
@@ -111,12 +126,11 @@ class GatedLinearAttention(Mixer):
         o_k, o_v, o_g, o_a = H * d, 2 * H * d, 2 * H * d + H * dv, 2 * H * d + 2 * H * dv
         z = self.decay.forward(_columns(proj, o_a, self.rank))
         with profile.scope("scan"):
-            o = ops.matrix_state_recurrence(
-                proj, proj[:, o_k:], proj[:, o_v:], z, H, H, d, dv, self.rate, self.decay_bias,
-                -1.0, d ** -0.5, cache.state, batch.seg_start, batch.seg_pos0, batch.seg_slot,
-                chunk_rows=_chunk_rows(batch, self.dtype))
-            y = ops.head_norm_gate(o, self.norm_w, self.norm_eps, proj[:, o_g:], ops.GATE_SILU,
-                                   H, dv, self.dtype)
+            y = _recurrence(
+                batch, proj, proj[:, o_k:], proj[:, o_v:], z, H, H, d, dv, self.rate,
+                self.decay_bias, -1.0, d ** -0.5, cache.state,
+                ops.GatedNorm(self.norm_w, self.norm_eps, proj[:, o_g:], ops.GATE_SILU, H, dv),
+                dict(chunk_rows=_chunk_rows(batch, self.dtype)))
         return self.out.forward(y, partial_sums=True)
 
     def weight_bytes(self) -> int:
@@ -175,16 +189,15 @@ class FixedDecayAttention(Mixer):
         # long portions: the decay is a constant, so a chunk of rows needs no chain along them
         chunked = batch.max_segment_rows > tuning.SCAN_CHUNKS_FROM_ROWS
         with profile.scope("scan"):
-            o = ops.matrix_state_recurrence(
-                proj, proj[:, o_k:], proj[:, o_v:], None, H, H, d, dv, self.rate, None, 1.0, 1.0,
-                cache.state, batch.seg_start, batch.seg_pos0, batch.seg_slot, decay="fixed",
-                silu_inputs=True,
-                chunks=batch.extra.get("scan_chunks") if chunked else None,
-                seg_chunk0=batch.extra.get("scan_seg_chunk0") if chunked else None,
-                chunk_rows=min(tuning.SCAN_CHUNK_ROWS, ops.FIXED_DECAY_CHUNK_ROWS))
             # (all heads are normed together: one "head" of H * dv for the kernel)
-            y = ops.head_norm_gate(o, self.norm_w, self.norm_eps, proj[:, o_g:],
-                                   ops.GATE_SIGMOID, 1, H * dv, self.dtype)
+            y = _recurrence(
+                batch, proj, proj[:, o_k:], proj[:, o_v:], None, H, H, d, dv, self.rate, None, 1.0,
+                1.0, cache.state,
+                ops.GatedNorm(self.norm_w, self.norm_eps, proj[:, o_g:], ops.GATE_SIGMOID, 1, H * dv),
+                dict(chunks=batch.extra.get("scan_chunks") if chunked else None,
+                     seg_chunk0=batch.extra.get("scan_seg_chunk0") if chunked else None,
+                     chunk_rows=min(tuning.SCAN_CHUNK_ROWS, ops.FIXED_DECAY_CHUNK_ROWS)),
+                decay="fixed", silu_inputs=True)
         return self.out.forward(y, partial_sums=True)
 
     def weight_bytes(self) -> int:
@@ -260,15 +273,13 @@ class BonusTimeMixing(Mixer):
         # long portions: chunk by chunk (the factors between two tokens are products of decays)
         chunked = batch.max_segment_rows > tuning.SCAN_CHUNKS_FROM_ROWS
         with profile.scope("scan"):
-            o = ops.matrix_state_recurrence(
-                r, k, v, z, H, H, d, d, None, self.w0, 1.0, 1.0, cache.part("state").state,
-                batch.seg_start, batch.seg_pos0, batch.seg_slot, decay="double_exp",
-                bonus=self.bonus,
-                chunks=batch.extra.get("scan_chunks") if chunked else None,
-                seg_chunk0=batch.extra.get("scan_seg_chunk0") if chunked else None,
-                chunk_rows=min(tuning.SCAN_CHUNK_ROWS, ops.FIXED_DECAY_CHUNK_ROWS))
-            y = ops.head_norm_gate(o, self.norm_w, self.norm_eps, g, ops.GATE_SILU, H, d,
-                                   self.dtype)
+            y = _recurrence(
+                batch, r, k, v, z, H, H, d, d, None, self.w0, 1.0, 1.0, cache.part("state").state,
+                ops.GatedNorm(self.norm_w, self.norm_eps, g, ops.GATE_SILU, H, d),
+                dict(chunks=batch.extra.get("scan_chunks") if chunked else None,
+                     seg_chunk0=batch.extra.get("scan_seg_chunk0") if chunked else None,
+                     chunk_rows=min(tuning.SCAN_CHUNK_ROWS, ops.FIXED_DECAY_CHUNK_ROWS)),
+                decay="double_exp", bonus=self.bonus)
         return self.out.forward(y, partial_sums=True)
 
     def weight_bytes(self) -> int:
@@ -356,13 +367,12 @@ class GatedDeltaRule(Mixer):
         z = self.decay.forward(_columns(proj, C, self.ra))
         gate = self.gate.forward(_columns(proj, C + self.ra, self.rg))
         with profile.scope("scan"):
-            o = ops.matrix_state_recurrence(
-                qkv, qkv[:, G * d:], qkv[:, 2 * G * d:], z, H, G, d, dv, self.rate, self.dt_bias,
-                1.0, d ** -0.5, state, batch.seg_start, batch.seg_pos0, batch.seg_slot,
-                beta=proj[:, C + self.ra + self.rg:], unit_qk=True, unit_eps=self.unit_eps,
-                chunk_rows=_chunk_rows(batch, self.dtype))
-            y = ops.head_norm_gate(o, self.norm_w, self.norm_eps, gate, ops.GATE_SIGMOID, H, dv,
-                                   self.dtype)
+            y = _recurrence(
+                batch, qkv, qkv[:, G * d:], qkv[:, 2 * G * d:], z, H, G, d, dv, self.rate,
+                self.dt_bias, 1.0, d ** -0.5, state,
+                ops.GatedNorm(self.norm_w, self.norm_eps, gate, ops.GATE_SIGMOID, H, dv),
+                dict(chunk_rows=_chunk_rows(batch, self.dtype)),
+                beta=proj[:, C + self.ra + self.rg:], unit_qk=True, unit_eps=self.unit_eps)
         return self.out.forward(y, partial_sums=True)
 
     def weight_bytes(self) -> int:

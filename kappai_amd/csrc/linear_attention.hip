@@ -1768,203 +1768,194 @@ extern "C" int kappai_head_norm_gate(const float* o, const float* weight, float 
 }
 
 // ---------------------------------------------------------------------------------------
-// Steps of single rows: what enters the recurrence, one token of it, and the norm with its gate behind it, in one
-// kernel.  A block takes a row's `hb` heads that are normed together (one, or all of them), a wave COLS columns of
-// S at a time and up to ls_groups such groups, whose rows are all asked for before anything is worked on; q, k and
-// the decay are made by the waves in turns and meet in LDS.  Every value is computed as the three kernels
-// (recurrence_prep, matrix_state_scan, head_norm_gate) compute it, in their order: the same bits.
-// Three kernels that each wait for the one before cost 4 to 5.5 us a piece beside 16 KB of state a head, which
-// is why they are one: 2 rows, 16 heads of 64 x 64, delta rule MEASURED.
-//   norm_w null: o goes to `of` [T, H dv] in float32.  Else the norm as in head_norm_gate, over hb * dv values
-//   (hb 1 or H; wide: added as its kernel for wide heads adds, eight values a lane, hb * dv = 512), result to `out`.
+// Steps of single rows: what enters the recurrence, one token of it and, where heads are normed one by one, the
+// norm with its gate behind it, in one kernel.  A block takes a row's head, a wave COLS columns of S at a time and up
+// to LS_GROUPS such groups; the state, the values and the gate are asked for first, q, k and the decay meet in LDS
+// meanwhile.  Every value is computed as the three kernels (recurrence_prep, matrix_state_scan, head_norm_gate)
+// compute it, in their order: the same bits.  Bound by what stands between a kernel's start and its end (tables, then
+// the state they name: two trips to memory, 5 us) beside 16 KB of state, hence one kernel: 2 rows, 16 heads of
+// 64 x 64, delta rule 14 us in three kernels, 5.5 so.  All heads of a row in one block, for a norm over all of them,
+// were slower than that norm as a kernel of its own (8 heads 11.5 us against 5.0 + 4.1).
+//   norm_w null: o goes to `of` [T, H dv] in float32.  Else the norm as in head_norm_gate, result to `out`.
 // ---------------------------------------------------------------------------------------
+#define LS_GROUPS 2
 #define LS_MAX_WAVES 16
-// (as many as the registers of 16 waves hold)
-constexpr int ls_groups(int mode) { return mode == 0 ? 4 : 2; }
 template <typename T>
 struct StepArgs {
   const T *q, *k, *v, *z, *b, *g;
   int q_stride, k_stride, v_stride, z_stride, b_stride, g_stride;
   const float *z_bias, *rate, *bonus, *norm_w;
   float sign, unit_eps, q_scale, norm_eps;
-  int H, Hk, d, dv, unit, act, decay_kind, gate_kind, gate_first, weight_stride, hb, wide;
+  int H, Hk, d, dv, unit, act, decay_kind, gate_kind, weight_stride;
   float* state;
-  const int *seg_start, *seg_pos0, *seg_slot;
+  const int *seg_pos0, *seg_slot;
   float* of;
   T* out;
 };
 template <int KS, int MODE, typename T>
 __global__ __launch_bounds__(LS_MAX_WAVES * WAVE) void matrix_state_step_kernel(const StepArgs<T> a) {
-  constexpr int R = 8, COLS = WAVE / KS, DP = KS * R, GROUPS = ls_groups(MODE);
+  constexpr int R = 8, COLS = WAVE / KS, DP = KS * R, GROUPS = LS_GROUPS;
   extern __shared__ __attribute__((aligned(16))) float sh_step[];
   const int tid = threadIdx.x, lane = tid % WAVE, wave = __builtin_amdgcn_readfirstlane(tid / WAVE);
-  const int nw = blockDim.x / WAVE, hb = a.hb, h0 = blockIdx.x * hb, seg = blockIdx.y;
-  const int H = a.H, Hk = a.Hk, d = a.d, dv = a.dv, n_cols = hb * dv;
-  float* normed = sh_step + hb * 3 * DP;            // [n_cols] what the norm's mean is taken of
-  const int first = a.seg_start[seg], last = a.seg_start[seg + 1];
-  const bool carry = a.seg_pos0[seg] > 0;
+  const int nw = blockDim.x / WAVE, h = blockIdx.x;
+  const int H = a.H, hk = h / (a.H / a.Hk), d = a.d, dv = a.dv;
+  float* read_out = sh_step + 3 * DP;               // [dv]
+  const int t = blockIdx.y, slot = a.seg_slot[t], pos0 = a.seg_pos0[t];
   const int s = lane % KS;
-  float S[GROUPS][R];
+  // what the columns need: asked for first, worked on behind the barrier
+  float S[GROUPS][R], vc[GROUPS], bc[GROUPS], gate[GROUPS], w[GROUPS], o[GROUPS];
   float* st[GROUPS];
-  int col[GROUPS], head[GROUPS];
+  int col[GROUPS];
 #pragma unroll
   for (int g = 0; g < GROUPS; ++g) {
     col[g] = (g * nw + wave) * COLS + lane / KS;
-    const int cc = min(col[g], n_cols - 1), hh = cc / dv;
-    head[g] = hh;
-    st[g] = a.state + (((size_t)a.seg_slot[seg] * H + h0 + hh) * dv + cc - hh * dv) * d;
-    if ((g * nw + wave) * COLS < n_cols) la_load_rows<KS, R>(st[g], s, d, carry, S[g]);
+    vc[g] = bc[g] = gate[g] = w[g] = o[g] = 0.f;
+    if ((g * nw + wave) * COLS < dv) {              // (uniform over the wave)
+      const int in_head = min(col[g], dv - 1);
+      const size_t c = (size_t)h * dv + in_head;
+      vc[g] = to_f32(a.v[(size_t)t * a.v_stride + c]);
+      if (MODE == 1) bc[g] = to_f32(a.b[(size_t)t * a.b_stride + h]);
+      if (a.norm_w != nullptr) {
+        gate[g] = to_f32(a.g[(size_t)t * a.g_stride + c]);
+        w[g] = a.norm_w[(size_t)h * a.weight_stride + in_head];
+      }
+      st[g] = a.state + (((size_t)slot * H + h) * dv + in_head) * d;
+      la_load_rows<KS, R>(st[g], s, d, true, S[g]);
+    }
   }
-  for (int t = first; t < last; ++t) {
-    // q, k and the decay of every head, as recurrence_prep makes them
-    for (int job = wave; job < 3 * hb; job += nw) {
-      const int hh = job / 3, what = job - 3 * hh, h = h0 + hh, hk = h / (H / Hk);
+  // q, k and the decay, as recurrence_prep makes them
+  const T* qr = a.q + (size_t)t * a.q_stride + (size_t)hk * d;
+  const T* kr = a.k + (size_t)t * a.k_stride + (size_t)hk * d;
+  for (int e = tid; e < DP; e += blockDim.x) {
+    float* to = sh_step + e;
+    float x = 0.f, y = 0.f, z = 0.f;
+    if (e < d) {
+      if (!a.unit) {
+        x = to_f32(qr[e]);
+        y = to_f32(kr[e]);
+      }
+      z = a.rate != nullptr ? a.rate[h] : 1.f;
+      if (a.decay_kind != 2) {
+        const float zz = to_f32(a.z[(size_t)t * a.z_stride + (size_t)h * d + e]) +
+                         (a.z_bias ? a.z_bias[(size_t)h * d + e] : 0.f);
+        z = a.decay_kind == 1 ? expf(-expf(zz)) : expf(-z * la_softplus(a.sign * zz));
+      }
+      if (a.act) {
+        x = la_stored_silu<T>(x);
+        y = la_stored_silu<T>(y);
+      }
+      x *= a.q_scale;
+    }
+    if (!a.unit) {
+      to[0] = x;
+      to[DP] = y;
+    }
+    to[2 * DP] = z;
+  }
+  if (a.unit) {
+    // (unit vectors: a wave a vector, from the last wave on, the first ones having the decays to make)
+    for (int job = nw - 1 - wave; job < 2; job += nw) {
+      const T* from = job ? kr : qr;
       float* to = sh_step + job * DP;
-      if (what == 2) {
-        const float r = a.rate != nullptr ? a.rate[h] : 1.f;
-        for (int e = lane; e < DP; e += WAVE) {
-          float x = 0.f;
-          if (e < d) {
-            x = r;
-            if (a.decay_kind != 2) {
-              const float zz = to_f32(a.z[(size_t)t * a.z_stride + (size_t)h * d + e]) +
-                               (a.z_bias ? a.z_bias[(size_t)h * d + e] : 0.f);
-              x = a.decay_kind == 1 ? expf(-expf(zz)) : expf(-r * la_softplus(a.sign * zz));
-            }
-          }
-          to[e] = x;
-        }
-      } else {
-        const T* from = (what ? a.k + (size_t)t * a.k_stride : a.q + (size_t)t * a.q_stride) + (size_t)hk * d;
-        const float scale = what ? 1.f : a.q_scale;
-        float f = scale;
-        if (a.unit) {
-          float sum = 0.f;
-          for (int e = lane; e < d; e += WAVE) {
-            const float x = to_f32(from[e]);
-            sum = fmaf(x, x, sum);
-          }
-          f = scale / sqrtf(wave_sum(sum) + a.unit_eps);
-        }
-        for (int e = lane; e < DP; e += WAVE) {
-          float x = 0.f;
-          if (e < d) {
-            x = to_f32(from[e]);
-            if (a.act) x = la_stored_silu<T>(x);
-            if (!(a.act && what)) x *= f;
-          }
-          to[e] = x;
-        }
-      }
-    }
-    // what a column needs beside them
-    float vc[GROUPS], bc[GROUPS], gate[GROUPS], w[GROUPS], o[GROUPS];
+      constexpr int PER = (DP + WAVE - 1) / WAVE;
+      float x[PER], sum = 0.f;
 #pragma unroll
-    for (int g = 0; g < GROUPS; ++g) {
-      vc[g] = bc[g] = gate[g] = w[g] = o[g] = 0.f;
-      if (col[g] < n_cols) {
-        const int h = h0 + head[g];
-        vc[g] = to_f32(a.v[(size_t)t * a.v_stride + (size_t)h0 * dv + col[g]]);
-        if (a.act) vc[g] = la_stored_silu<T>(vc[g]);
-        if (MODE == 1) bc[g] = la_sigmoid(to_f32(a.b[(size_t)t * a.b_stride + h]));
-        if (a.norm_w != nullptr) {
-          const float gv = to_f32(a.g[(size_t)t * a.g_stride + (size_t)h0 * dv + col[g]]);
-          gate[g] = a.gate_kind == 0 ? gv * la_sigmoid(gv) : la_sigmoid(gv);
-          w[g] = a.norm_w[(size_t)blockIdx.x * a.weight_stride + col[g]];
-        }
-      }
-    }
-    __syncthreads();
+      for (int i = 0; i < PER; ++i) x[i] = lane + i * WAVE < d ? to_f32(from[lane + i * WAVE]) : 0.f;
 #pragma unroll
-    for (int g = 0; g < GROUPS; ++g) {
-      if ((g * nw + wave) * COLS >= n_cols) break;             // (uniform over the wave)
-      const float* base = sh_step + head[g] * 3 * DP;
-      float qc[R], kc[R], ac[R], uc[R];
+      for (int i = 0; i < PER; ++i) sum = fmaf(x[i], x[i], sum);
+      asm volatile("" : "+v"(sum));                 // (rounded before the lanes meet)
+      const float f = (job ? 1.f : a.q_scale) / sqrtf(wave_sum(sum) + a.unit_eps);
 #pragma unroll
-      for (int r4 = 0; r4 < R; r4 += 4) {
-        const int row = la_row<KS>(s, r4);
-        const float4 x = *reinterpret_cast<const float4*>(base + row);
-        const float4 y = *reinterpret_cast<const float4*>(base + DP + row);
-        const float4 z = *reinterpret_cast<const float4*>(base + 2 * DP + row);
-        qc[r4] = x.x; qc[r4 + 1] = x.y; qc[r4 + 2] = x.z; qc[r4 + 3] = x.w;
-        kc[r4] = y.x; kc[r4 + 1] = y.y; kc[r4 + 2] = y.z; kc[r4 + 3] = y.w;
-        ac[r4] = z.x; ac[r4 + 1] = z.y; ac[r4 + 2] = z.z; ac[r4 + 3] = z.w;
-      }
-#pragma unroll
-      for (int r = 0; r < R; ++r)
-        uc[r] = MODE == 2 && la_row<KS>(s, r) < d ? a.bonus[(size_t)(h0 + head[g]) * d + la_row<KS>(s, r)] : 0.f;
-      o[g] = la_token<KS, R, MODE>(S[g], qc, kc, ac, uc, vc[g], bc[g]);
-      if (s == 0 && col[g] < n_cols) {
-        if (a.norm_w == nullptr) a.of[(size_t)t * H * dv + (size_t)h0 * dv + col[g]] = o[g];
-        else normed[col[g]] = a.gate_first ? o[g] * gate[g] : o[g];
-      }
-    }
-    __syncthreads();                               // (and nobody reads q, k and the decay any more)
-    if (a.norm_w != nullptr) {
-      float ss = 0.f;
-      if (a.wide) {
-#pragma unroll
-        for (int i = 0; i < 8; ++i) ss = fmaf(normed[lane * 8 + i], normed[lane * 8 + i], ss);
-      } else {
-        for (int e = lane; e < n_cols; e += WAVE) ss = fmaf(normed[e], normed[e], ss);
-      }
-      // (a wave's sum is rounded in more than one way, by quads of lanes: every value takes the one that its lane
-      // of head_norm_gate has)
-      const float inv = 1.0f / sqrtf(wave_sum(ss) / (float)n_cols + a.norm_eps);
-#pragma unroll
-      for (int g = 0; g < GROUPS; ++g) {
-        const float mine = __shfl(inv, a.wide ? 0 : col[g] % WAVE);
-        if (s == 0 && col[g] < n_cols)
-          from_f32(a.out + (size_t)t * H * dv + (size_t)h0 * dv + col[g], o[g] * mine * w[g] * gate[g]);
-      }
-      if (t + 1 < last) __syncthreads();
+      for (int i = 0; i < PER; ++i)
+        if (lane + i * WAVE < DP) to[lane + i * WAVE] = x[i] * f;
     }
   }
+  __syncthreads();
 #pragma unroll
-  for (int g = 0; g < GROUPS; ++g)
-    if (col[g] < n_cols) la_store_rows<KS, R>(st[g], s, d, S[g]);
+  for (int g = 0; g < GROUPS; ++g) {
+    if ((g * nw + wave) * COLS >= dv) break;
+    const float* base = sh_step;
+    float qc[R], kc[R], ac[R], uc[R];
+#pragma unroll
+    for (int r4 = 0; r4 < R; r4 += 4) {
+      const int row = la_row<KS>(s, r4);
+      const float4 x = *reinterpret_cast<const float4*>(base + row);
+      const float4 y = *reinterpret_cast<const float4*>(base + DP + row);
+      const float4 z = *reinterpret_cast<const float4*>(base + 2 * DP + row);
+      qc[r4] = x.x; qc[r4 + 1] = x.y; qc[r4 + 2] = x.z; qc[r4 + 3] = x.w;
+      kc[r4] = y.x; kc[r4 + 1] = y.y; kc[r4 + 2] = y.z; kc[r4 + 3] = y.w;
+      ac[r4] = z.x; ac[r4 + 1] = z.y; ac[r4 + 2] = z.z; ac[r4 + 3] = z.w;
+    }
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      uc[r] = MODE == 2 && la_row<KS>(s, r) < d ? a.bonus[(size_t)h * d + la_row<KS>(s, r)] : 0.f;
+      S[g][r] = pos0 > 0 ? S[g][r] : 0.f;           // (a request that begins here: whatever the slot holds)
+    }
+    if (a.act) vc[g] = la_stored_silu<T>(vc[g]);
+    if (MODE == 1) bc[g] = la_sigmoid(bc[g]);
+    gate[g] = a.gate_kind == 0 ? gate[g] * la_sigmoid(gate[g]) : la_sigmoid(gate[g]);
+    o[g] = la_token<KS, R, MODE>(S[g], qc, kc, ac, uc, vc[g], bc[g]);
+    if (s == 0 && col[g] < dv) {
+      if (a.norm_w == nullptr) a.of[((size_t)t * H + h) * dv + col[g]] = o[g];
+      else read_out[col[g]] = o[g];
+    }
+    if (col[g] < dv) la_store_rows<KS, R>(st[g], s, d, S[g]);
+  }
+  if (a.norm_w == nullptr) return;
+  __syncthreads();
+  float ss = 0.f;
+  for (int e = lane; e < dv; e += WAVE) ss = fmaf(read_out[e], read_out[e], ss);
+  asm volatile("" : "+v"(ss));
+  // (a wave's sum is rounded in more than one way, by quads of lanes: every value takes the one that its lane
+  // of head_norm_gate has)
+  const float inv = 1.0f / sqrtf(wave_sum(ss) / (float)dv + a.norm_eps);
+#pragma unroll
+  for (int g = 0; g < GROUPS; ++g) {
+    const float mine = __shfl(inv, col[g] % WAVE);
+    if (s == 0 && col[g] < dv)
+      from_f32(a.out + ((size_t)t * H + h) * dv + col[g], o[g] * mine * w[g] * gate[g]);
+  }
 }
 
-// Whether the kernel for single rows takes hb heads of d x dv a block (key sizes of whole fours that 2 to 16 lanes
-// of eight hold).
-extern "C" int kappai_matrix_state_step_fits(int d, int dv, int hb, int mode) {
-  if (d <= 8 || dv < 1 || hb < 1 || d % 4 || d > 128 || hb > 64 || (long long)hb * dv > 8192) return 0;
+// Whether the kernel for single rows takes heads of d x dv (key sizes of whole fours that 2 to 16 lanes of eight
+// hold; fewer values than the norm's kernel for wide heads takes, which adds in another order).
+extern "C" int kappai_matrix_state_step_fits(int d, int dv) {
+  if (d <= 8 || dv < 1 || d % 4 || d > 128 || dv >= 512) return 0;
   int ks = 2;
   while (ks * 8 < d) ks *= 2;
-  return hb * dv <= ls_groups(mode) * LS_MAX_WAVES * (WAVE / ks) &&
-         (hb * 3 * ks * 8 + hb * dv) * 4 <= 64 * 1024;
+  return dv <= LS_GROUPS * LS_MAX_WAVES * (WAVE / ks);
 }
 
 // mode as kappai_matrix_state_scan; norm_w null: float32 results in `out`, else results in the rows' type.
-// n_segments rows, one a segment (longer segments are walked, segments without a row keep their state).
+// S segments of one row each: row s is segment s.
 extern "C" int kappai_matrix_state_step(
     const void* q, int q_stride, const void* k, int k_stride, const void* v, int v_stride, const void* z,
     int z_stride, const float* z_bias, const float* rate, float sign, const void* b, int b_stride,
     const float* bonus, int S, int H, int Hk, int d, int dv, int mode, int unit, float unit_eps, float q_scale,
-    int act, int decay_kind, float* state, const int* seg_start, const int* seg_pos0, const int* seg_slot,
-    const float* norm_w, float norm_eps, const void* g, int g_stride, int gate_kind, int gate_first, int hb,
-    int weight_stride, int wide, void* out, int is_bf16, hipStream_t stream) {
+    int act, int decay_kind, float* state, const int* seg_pos0, const int* seg_slot,
+    const float* norm_w, float norm_eps, const void* g, int g_stride, int gate_kind, int weight_stride,
+    void* out, int is_bf16, hipStream_t stream) {
   if (S <= 0) return 0;
-  if (H < 1 || Hk < 1 || H % Hk || H > 65535 || S > 65535 || hb < 1 || H % hb || mode < 0 || mode > 2 ||
+  if (H < 1 || Hk < 1 || H % Hk || H > 65535 || S > 65535 || mode < 0 || mode > 2 ||
       decay_kind < 0 || decay_kind > 2 || (decay_kind != 2 && z == nullptr) ||
       (decay_kind != 1 && rate == nullptr) || (act && unit) || (mode == 1 && b == nullptr) ||
-      (mode == 2 && (bonus == nullptr || H != Hk)) || !kappai_matrix_state_step_fits(d, dv, hb, mode) ||
+      (mode == 2 && (bonus == nullptr || H != Hk)) || !kappai_matrix_state_step_fits(d, dv) ||
       ((uintptr_t)state % 16) ||
-      (norm_w != nullptr && (g == nullptr || gate_kind < 0 || gate_kind > 1 || (wide && hb * dv != 512))))
+      (norm_w != nullptr && (g == nullptr || gate_kind < 0 || gate_kind > 1)))
     return (int)hipErrorInvalidValue;
   int ks = 2;
   while (ks * 8 < d) ks *= 2;
-  const int cols = WAVE / ks, want = (hb * dv + cols - 1) / cols;
+  const int cols = WAVE / ks, want = (dv + cols - 1) / cols;
   const int nw = want < LS_MAX_WAVES ? want : LS_MAX_WAVES;
-  const size_t lds = (size_t)(hb * 3 * ks * 8 + hb * dv) * sizeof(float);
+  const size_t lds = (size_t)(3 * ks * 8 + dv) * sizeof(float);
 #define LS_RUN(KS_, MODE_, T_)                                                                             \
-  hipLaunchKernelGGL((matrix_state_step_kernel<KS_, MODE_, T_>), dim3(H / hb, S), dim3(nw * WAVE), lds,    \
+  hipLaunchKernelGGL((matrix_state_step_kernel<KS_, MODE_, T_>), dim3(H, S), dim3(nw * WAVE), lds,    \
                      stream,                                                                               \
                      (StepArgs<T_>{(const T_*)q, (const T_*)k, (const T_*)v, (const T_*)z, (const T_*)b,   \
                                    (const T_*)g, q_stride, k_stride, v_stride, z_stride, b_stride,         \
                                    g_stride, z_bias, rate, bonus, norm_w, sign, unit_eps, q_scale,         \
-                                   norm_eps, H, Hk, d, dv, unit, act, decay_kind, gate_kind, gate_first,   \
-                                   weight_stride, hb, wide, state, seg_start, seg_pos0, seg_slot,          \
+                                   norm_eps, H, Hk, d, dv, unit, act, decay_kind, gate_kind,               \
+                                   weight_stride, state, seg_pos0, seg_slot,                    \
                                    norm_w ? nullptr : (float*)out, norm_w ? (T_*)out : nullptr}))
 #define LS_CASE(KS_)                                                          \
   case KS_:                                                                   \

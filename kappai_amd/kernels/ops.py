@@ -2668,39 +2668,32 @@ class GatedNorm(NamedTuple):
     vdim: int
 
 
-def matrix_state_step_takes(q: torch.Tensor, state: torch.Tensor, mode: int, norm: Optional[GatedNorm]) -> bool:
-    """Whether ``matrix_state_step`` takes rows like ``q`` and such a state [slots, H, vdim, dim] (``mode`` 0: the gated
-    sum, 1: the delta rule, 2: with a bonus), with the heads normed one by one or all together."""
-    if not q.is_cuda or q.dtype not in (F32, BF16) or state.data_ptr() % 16:
-        return False
-    H, dv, d = state.shape[1:]
-    together = H if norm is not None and (norm.n_heads, norm.vdim) == (1, H * dv) else 1
-    if norm is not None and together == 1 and (norm.n_heads, norm.vdim) != (H, dv):
-        return False
-    # (wide heads are added in another order, which the kernel keeps for 512 values)
-    return (norm is None or together * dv <= 512) and bool(
-        library("linear_attention").kappai_matrix_state_step_fits(_c_int(d), _c_int(dv), _c_int(together),
-                                                                  _c_int(mode)))
+def matrix_state_step_takes(q: torch.Tensor, state: torch.Tensor) -> bool:
+    """Whether ``matrix_state_step`` takes rows like ``q`` and such a state [slots, H, vdim, dim]."""
+    return (q.is_cuda and q.dtype in (F32, BF16) and state.data_ptr() % 16 == 0
+            and bool(library("linear_attention").kappai_matrix_state_step_fits(
+                _c_int(state.shape[3]), _c_int(state.shape[2]))))
 
 
 def matrix_state_step(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, z: Optional[torch.Tensor],
                       n_heads: int, n_qk_heads: int, dim: int, vdim: int, rate: Optional[torch.Tensor],
                       z_bias: Optional[torch.Tensor], z_sign: float, q_scale: float, state: torch.Tensor,
-                      seg_start: torch.Tensor, seg_pos0: torch.Tensor, seg_slot: torch.Tensor,
+                      seg_pos0: torch.Tensor, seg_slot: torch.Tensor,
                       beta: Optional[torch.Tensor] = None, unit_qk: bool = False, unit_eps: float = 1e-6,
                       decay: str = "softplus", bonus: Optional[torch.Tensor] = None,
                       silu_inputs: bool = False, norm: Optional[GatedNorm] = None) -> torch.Tensor:
-    """``matrix_state_recurrence`` for a step in which every segment is one row and, with ``norm``,
+    """``matrix_state_recurrence`` for a step in which every segment is one row (row s is segment s) and, with ``norm``,
     ``head_norm_gate`` on its result, in one kernel with their bits.  Returns [T, H vdim], float32 or, with
     ``norm``, in the rows' dtype.  For what ``matrix_state_step_takes`` takes."""
     H, Hk, d, dv = n_heads, n_qk_heads, dim, vdim
     mode = 1 if beta is not None else 2 if bonus is not None else 0
-    _need(matrix_state_step_takes(q, state, mode, norm), lambda: f"matrix_state_step: state {tuple(state.shape)}")
+    _need(matrix_state_step_takes(q, state), lambda: f"matrix_state_step: state {tuple(state.shape)}")
     _need(beta is None or bonus is None, "matrix_state_step: the delta rule or a bonus")
     _need(not (silu_inputs and unit_qk), "matrix_state_step: SiLU or unit vectors")
     _need(decay in DECAY_KINDS and (z is None) == (decay == "fixed")
           and (rate is not None or decay == "double_exp"), lambda: f"matrix_state_step: decay {decay!r}")
-    T, S = q.shape[0], seg_slot.shape[0]
+    T = q.shape[0]
+    _need(seg_slot.shape[0] == seg_pos0.shape[0] == T, "matrix_state_step: a segment is one row")
     for name, t, cols in (("q", q, Hk * d), ("k", k, Hk * d), ("v", v, H * dv), ("z", z, H * d), ("beta", beta, H),
                           ("gate", norm.gate if norm else None, H * dv)):
         if t is None:
@@ -2708,34 +2701,28 @@ def matrix_state_step(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, z: Opti
         _gpu(name, t, q.dtype, contiguous=False)
         _need(t.dim() == 2 and t.shape[0] == T and t.shape[1] >= cols and (t.stride(1) == 1 or cols == 1),
               lambda: f"matrix_state_step: {name} {tuple(t.shape)}, expected [T, {cols}]")
+    _need(norm is None or (norm.n_heads, norm.vdim) == (H, dv), "matrix_state_step: heads normed one by one")
     _need(H % Hk == 0 and (bonus is None or H == Hk), "matrix_state_step: heads")
     for name, t, shapes in (("rate", rate, ((H,),)), ("bonus", bonus, ((H, d),)), ("z_bias", z_bias, ((H * d,),)),
                             ("weight", norm.weight if norm else None,
-                             ((norm.vdim,), (norm.n_heads, norm.vdim)) if norm else ())):
+                             ((dv,), (H, dv)))):
         if t is not None:
             _gpu(name, t, F32)
             _need(tuple(t.shape) in shapes, lambda: f"matrix_state_step: {name} {tuple(t.shape)}")
     _gpu("state", state, F32)
     _need(tuple(state.shape[1:]) == (H, dv, d), lambda: f"matrix_state_step: state {tuple(state.shape)}")
-    for name, t in (("seg_start", seg_start), ("seg_pos0", seg_pos0), ("seg_slot", seg_slot)):
+    for name, t in (("seg_pos0", seg_pos0), ("seg_slot", seg_slot)):
         _gpu(name, t, I32)
     out = torch.empty((T, H * dv), dtype=F32 if norm is None else q.dtype, device=q.device)
-    heads, wide, gate, weight, eps, kind = 1, 0, None, None, 0.0, 0
-    if norm is not None:
-        weight, eps, gate, kind = norm.weight, norm.eps, norm.gate, norm.gate_kind
-        heads = H // norm.n_heads
-        # (the order in which head_norm_gate adds: its kernel for wide heads where that takes these)
-        wide = int(norm.vdim == 512 and gate.stride(0) % 8 == 0 and
-                   (gate.data_ptr() | weight.data_ptr()) % 16 == 0)
+    weight, eps, gate, kind = norm[:4] if norm is not None else (None, 0.0, None, 0)
     check(library("linear_attention").kappai_matrix_state_step(
         _ptr(q), _c_int(q.stride(0)), _ptr(k), _c_int(k.stride(0)), _ptr(v), _c_int(v.stride(0)), _ptr(z),
         _c_int(z.stride(0) if z is not None else 0), _ptr(z_bias), _ptr(rate), _c_float(z_sign), _ptr(beta),
-        _c_int(beta.stride(0) if beta is not None else 0), _ptr(bonus), _c_int(S), _c_int(H), _c_int(Hk), _c_int(d),
+        _c_int(beta.stride(0) if beta is not None else 0), _ptr(bonus), _c_int(T), _c_int(H), _c_int(Hk), _c_int(d),
         _c_int(dv), _c_int(mode), _c_int(1 if unit_qk else 0), _c_float(unit_eps), _c_float(q_scale),
-        _c_int(1 if silu_inputs else 0), _c_int(DECAY_KINDS[decay]), _ptr(state), _ptr(seg_start), _ptr(seg_pos0),
+        _c_int(1 if silu_inputs else 0), _c_int(DECAY_KINDS[decay]), _ptr(state), _ptr(seg_pos0),
         _ptr(seg_slot), _ptr(weight), _c_float(eps), _ptr(gate), _c_int(gate.stride(0) if gate is not None else 0),
-        _c_int(kind), _c_int(0), _c_int(heads),
-        _c_int(norm.vdim if norm is not None and weight.dim() == 2 else 0), _c_int(wide), _ptr(out),
+        _c_int(kind), _c_int(dv if norm is not None and weight.dim() == 2 else 0), _ptr(out),
         _c_int(_is_bf16(q.dtype)), _stream()), "matrix_state_step")
     return out
 

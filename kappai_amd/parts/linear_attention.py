@@ -66,15 +66,20 @@ def _chunk_rows(batch, dtype=torch.bfloat16) -> int:
 
 def _recurrence(batch, q, k, v, z, H, G, d, dv, rate, bias, sign, scale, state, norm, chunking,
                 **kinds) -> torch.Tensor:
-    """The recurrence with the norm and its gate (``ops.GatedNorm``) behind it: one kernel where every
-    segment is a single row, else the recurrence as ``chunking`` says and the norm as a kernel of its own."""
-    tables = (batch.seg_start, batch.seg_pos0, batch.seg_slot)
-    mode = 1 if kinds.get("beta") is not None else 2 if kinds.get("bonus") is not None else 0
-    if batch.max_segment_rows == 1 and ops.matrix_state_step_takes(q, state, mode, norm):
-        return ops.matrix_state_step(q, k, v, z, H, G, d, dv, rate, bias, sign, scale, state, *tables,
-                                     norm=norm, **kinds)
-    o = ops.matrix_state_recurrence(q, k, v, z, H, G, d, dv, rate, bias, sign, scale, state, *tables,
-                                    **chunking, **kinds)
+    """The recurrence with the norm and its gate (``ops.GatedNorm``) behind it.  Where every segment is a
+    single row, the recurrence and the norm of heads one by one are one kernel."""
+    if (batch.max_segment_rows == 1 and batch.seg_slot.shape[0] == q.shape[0]
+            and ops.matrix_state_step_takes(q, state)):
+        one_by_one = norm.n_heads == H
+        o = ops.matrix_state_step(q, k, v, z, H, G, d, dv, rate, bias, sign, scale, state,
+                                  batch.seg_pos0, batch.seg_slot, norm=norm if one_by_one else None,
+                                  **kinds)
+        if one_by_one:
+            return o
+    else:
+        o = ops.matrix_state_recurrence(q, k, v, z, H, G, d, dv, rate, bias, sign, scale, state,
+                                        batch.seg_start, batch.seg_pos0, batch.seg_slot,
+                                        **chunking, **kinds)
     return ops.head_norm_gate(o, norm.weight, norm.eps, norm.gate, norm.gate_kind, norm.n_heads,
                               norm.vdim, q.dtype)
 

@@ -16,17 +16,14 @@ FORMS = {
 
 
 # key sizes at both ends of 2 to 16 lanes a column and ones that are no power of two, value sizes that end inside a
-# wave and take more than one group of columns, q and k shared by heads, heads normed together (512 values: as the
-# kernel for wide heads adds them, and over a gate that it cannot read)
-@pytest.mark.parametrize("form,H,G,d,dv,together", [
-    ("gated", 3, 3, 12, 5, False), ("gated", 8, 8, 64, 64, False), ("gated", 2, 2, 128, 130, False),
-    ("gated", 2, 2, 68, 256, False), ("fixed", 8, 8, 64, 64, True), ("fixed", 3, 3, 20, 33, True),
-    ("fixed", 1, 1, 16, 512, True), ("fixed", 4, 4, 36, 16, False), ("delta", 16, 4, 64, 64, False),
-    ("delta", 4, 2, 128, 128, False), ("delta", 3, 1, 16, 7, False), ("bonus", 16, 16, 64, 64, False),
-    ("bonus", 5, 5, 100, 100, False)])
+# wave and take more than one group of columns, q and k shared by heads
+@pytest.mark.parametrize("form,H,G,d,dv", [
+    ("gated", 3, 3, 12, 5), ("gated", 8, 8, 64, 64), ("gated", 2, 2, 128, 127), ("gated", 1, 1, 68, 128),
+    ("gated", 2, 2, 16, 508), ("fixed", 8, 8, 64, 64), ("fixed", 3, 3, 20, 33), ("delta", 16, 4, 64, 64),
+    ("delta", 4, 2, 128, 128), ("delta", 3, 1, 16, 7), ("bonus", 16, 16, 64, 64), ("bonus", 5, 5, 100, 100)])
 @pytest.mark.parametrize("dtype", [BF16, F32])
 @pytest.mark.parametrize("rows", [1, 7])
-def test_one_kernel_has_the_bits_of_three(ops, form, H, G, d, dv, together, dtype, rows):  # noqa: F811
+def test_one_kernel_has_the_bits_of_three(ops, form, H, G, d, dv, dtype, rows):  # noqa: F811
     f = dict(FORMS[form])
     n, odd = 2 * G * d + 2 * H * dv, 0 if d % 8 == 0 else 3        # (rows that start on no 16 bytes, too)
     proj = rand((rows, n + odd), dtype, 1).to(DEV)
@@ -44,26 +41,23 @@ def test_one_kernel_has_the_bits_of_three(ops, form, H, G, d, dv, together, dtyp
     i32 = dict(dtype=torch.int32, device=DEV)
     start, slot = torch.arange(rows + 1, **i32), torch.arange(rows, 0, -1, **i32)
     pos0 = (torch.arange(rows, **i32) % 3 != 1).to(torch.int32) * 9       # (some rows begin a request)
-    heads, vdim = (1, H * dv) if together else (H, dv)
-    mode = 1 if "beta" in f else 2 if "bonus" in f else 0
-    for weight in (rand((vdim,), F32, 8).to(DEV), rand((heads, vdim), F32, 9).to(DEV)):
-        norm = ops.GatedNorm(weight, 1e-5, g, ops.GATE_SILU if mode else ops.GATE_SIGMOID, heads, vdim)
-        assert ops.matrix_state_step_takes(q, state, mode, norm)
+    kind = ops.GATE_SILU if "beta" in f or "bonus" in f else ops.GATE_SIGMOID
+    assert ops.matrix_state_step_takes(q, state)
+    for weight in (rand((dv,), F32, 8).to(DEV), rand((H, dv), F32, 9).to(DEV)):
+        norm = ops.GatedNorm(weight, 1e-5, g, kind, H, dv)
         before, after = state.clone(), state.clone()
         args = (q, k, v, z, H, G, d, dv, rate, bias, sign, scale)
         o = ops.matrix_state_recurrence(*args, before, start, pos0, slot, **f)
-        want = ops.head_norm_gate(o, weight, 1e-5, g, norm.gate_kind, heads, vdim, dtype)
-        got = ops.matrix_state_step(*args, after, start, pos0, slot, norm=norm, **f)
+        want = ops.head_norm_gate(o, weight, 1e-5, g, kind, H, dv, dtype)
+        got = ops.matrix_state_step(*args, after, pos0, slot, norm=norm, **f)
         assert torch.equal(got, want) and torch.equal(after, before)
     plain = state.clone()
-    assert torch.equal(ops.matrix_state_step(*args, plain, start, pos0, slot, **f), o)
+    assert torch.equal(ops.matrix_state_step(*args, plain, pos0, slot, **f), o)
     assert torch.equal(plain, before)
 
 
 def test_what_the_kernel_does_not_take(ops):  # noqa: F811
     q = rand((2, 64), BF16, 1).to(DEV)
-    for H, d, dv, mode in ((2, 8, 16, 0), (2, 30, 16, 0), (2, 132, 16, 0), (1, 16, 600, 0), (1, 128, 256, 1)):
-        state = torch.zeros((3, H, dv, d), device=DEV)
-        norm = ops.GatedNorm(torch.ones(dv, device=DEV), 1e-5, q, ops.GATE_SILU, H, dv)
-        assert not ops.matrix_state_step_takes(q, state, mode, norm), (H, d, dv, mode)
-    assert not ops.matrix_state_step_takes(q.cpu(), torch.zeros((3, 2, 16, 32)), 0, None)
+    for d, dv in ((8, 16), (30, 16), (132, 16), (16, 512), (128, 129)):
+        assert not ops.matrix_state_step_takes(q, torch.zeros((3, 2, dv, d), device=DEV)), (d, dv)
+    assert not ops.matrix_state_step_takes(q.cpu(), torch.zeros((3, 2, 16, 32)))

@@ -60,6 +60,17 @@ __device__ __forceinline__ void store8(bf16_t* p, const float* v) {
   *reinterpret_cast<uint4*>(p) = o;
 }
 
+// The sum of eight squares as the norms' row kernels round it (the second square by itself, the others as they are
+// added), for the kernels that must have their bits.
+__device__ __forceinline__ float sum_of_squares8(const float* v) {
+  float ss = v[1] * v[1];
+  asm volatile("" : "+v"(ss));
+  ss = fmaf(v[0], v[0], ss);
+#pragma unroll
+  for (int e = 2; e < 8; ++e) ss = fmaf(v[e], v[e], ss);
+  return ss;
+}
+
 // Exchanges inside a wave without a trip through LDS: the partner lane ^ 1 or ^ 2 (inside a quad)
 // and the lanes 4 and 8 further in a row of 16 come by data-parallel moves, the partners lane ^ 16
 // and lane ^ 32 by the row and half swaps of gfx950.

@@ -777,8 +777,7 @@ __global__ __launch_bounds__(1024) void add_rmsnorm_row_kernel(
     } else {
       load8(w + j, w8);
     }
-#pragma unroll
-    for (int e = 0; e < 8; ++e) ss += v[e] * v[e];
+    ss = sum_of_squares8(v);
   }
   ss = block_sum_once(ss, red, (D / 8 + WAVE - 1) / WAVE);
   const float scale = 1.0f / sqrtf(ss / (float)D + eps);
@@ -870,8 +869,7 @@ __global__ __launch_bounds__(1024) void embed_rmsnorm_row_kernel(
                 (c % 4) * 128, v);
     }
     store8(resid + (size_t)i * D + j, v);
-#pragma unroll
-    for (int e = 0; e < 8; ++e) ss += v[e] * v[e];
+    ss = sum_of_squares8(v);
   }
   ss = block_sum_once(ss, red, (D / 8 + WAVE - 1) / WAVE);
   const float scale = 1.0f / sqrtf(ss / (float)D + eps);

@@ -28,7 +28,7 @@
 extern "C" {
 #endif
 
-#define KAPPAI_ENGINE_ABI 12         // bumped with every change of the structs below
+#define KAPPAI_ENGINE_ABI 13         // bumped with every change of the structs below
 #define KAPPAI_MAX_GROUPS 8          // paged groups a batch can carry block tables for
 #define KAPPAI_MAX_TABLES 8         // tables and numbers of the parts' own in a step
 // Norm, rotation and store inside the decode attention that keeps a row in one block: up to this many blocks.  us
@@ -56,6 +56,12 @@ typedef struct kappai_kernels {
   int (*sum_partials)(const float*, int, long, float*, hipStream_t);
   int (*gemm_f32)(const float*, const float*, const float*, float*, int, int, int, int, int,
                   hipStream_t);
+  // into the stream; whether rows of this width are normed inside a product, and such a product
+  int (*gemm_f32_add)(const float*, const float*, const float*, float*, int, int, int, int, int,
+                      hipStream_t);
+  int (*gemm_f32_norms)(int, int);
+  int (*gemm_f32_normed)(const float*, const float*, float, const float*, const float*, float*, int, int, int,
+                         int, int, hipStream_t);
   // gate and up in 32 bits with the gate applied: rows, results and K that it takes, and the product
   int (*gemm_f32_gates)(int, int, int);
   int (*gemm_f32_swiglu)(const float*, const float*, const float*, float*, int, int, int, int, int,
@@ -128,12 +134,15 @@ typedef struct kappai_fold {
 } kappai_fold;
 
 // Rows on their way into a product: plain [M, D] with a row stride, 16 row slots in fragment
-// order, or either of the two still to be divided by the rows' root mean square (ss != null).
+// order, or either of the two still to be divided by the rows' root mean square (ss != null); or the
+// residual stream itself, which the product norms with `norm` (KAPPAI_ROWS_OF_STREAM; float32, and only to
+// parts of the framework whose first product takes it: others get rows that are normed).
+enum { KAPPAI_ROWS_OF_STREAM = 2 };
 typedef struct kappai_rows {
   void* data;
   int is_bf16;
   int M, D, ld;
-  int frag;
+  int frag;                        // 0, 1: fragment order, KAPPAI_ROWS_OF_STREAM
   const float* ss;                 // scaled rows: [ss_parts][16] sums of squares
   int ss_parts;
   float eps;

@@ -307,8 +307,24 @@ kappai_carry linear(Step& c, kappai_rows x, const kappai_linear& lin, int out_bf
   }
   if (lin.w_is_f32) {
     // a matrix stored in 32 bits: true 32-bit arithmetic whatever the activations are
+    if (x.frag == KAPPAI_ROWS_OF_STREAM && !out_bf16 && into == nullptr && aligned16(lin.w) &&
+        k.gemm_f32_norms(M, K)) {
+      out.kind = KAPPAI_CARRY_DELTA;
+      out.is_f32 = 1;
+      out.data = c.a->take(region, (size_t)M * N * 4);
+      LAUNCH(c, k.gemm_f32_normed((const float*)x.data, x.norm->w, x.norm->eps, (const float*)lin.w, lin.bias,
+                                  (float*)out.data, M, N, K, N, 0, c.stream));
+      return out;
+    }
+    if (x.frag == KAPPAI_ROWS_OF_STREAM) x = plain_rows(c, x, (float*)x.data);
     if (x.ss != nullptr || x.frag) {
       refuse(c, "rows in kernel order reached a matrix stored in 32 bits");
+      return out;
+    }
+    if (into != nullptr && !x.is_bf16 && !out_bf16 && c.m->kernels->gemm_f32_norms(M, N)) {
+      // a step of few rows: the result joins the stream, which the next product may norm itself
+      LAUNCH(c, k.gemm_f32_add((const float*)x.data, (const float*)lin.w, lin.bias, into->resid, M, N, K,
+                               M > 1 ? x.ld : K, N, c.stream));
       return out;
     }
     const float* xf = x.is_bf16 ? (const float*)cast_to(c, x.data, (size_t)M * K, 1, 0)
@@ -328,6 +344,7 @@ kappai_carry linear(Step& c, kappai_rows x, const kappai_linear& lin, int out_bf
     }
     return out;
   }
+  if (x.frag == KAPPAI_ROWS_OF_STREAM) x = plain_rows(c, x, (float*)x.data);
   const void* xb = x.data;
   int lda = x.ld;
   if (!x.is_bf16) {

@@ -43,6 +43,8 @@ kappai_rows rows_of(void* data, int M, int D, int is_bf16) {
 // The rows that `consumer` reads after the norm: scaled rows made for this norm go through as
 // they are, else the norm's kernel runs, writing fragment order when that suits the number of
 // rows and the consumer.  The first norm of a step looks the embedding up in the same kernel.
+bool norms_the_stream(const kappai_part* consumer);
+
 kappai_rows rms_norm(kappai_step* s, const void* desc, float* resid, kappai_carry carry, int M,
                      const int* rows, int n_rows, const kappai_part* consumer) {
   const kappai_step_api& api = *s->api;
@@ -76,6 +78,15 @@ kappai_rows rms_norm(kappai_step* s, const void* desc, float* resid, kappai_carr
     if (rows == nullptr && carry.scaled.norm == norm && kernel_order) return carry.scaled;
     carry = kappai_carry{};                      // the sum is in the residual already
     return api.rms_norm(s, norm, resid, carry, M, rows, n_rows, 0);
+  }
+  // float32, few rows, the sum in the stream already: the consumer's first product norms them itself
+  if (carry.kind == KAPPAI_CARRY_NOTHING && rows == nullptr && !m.compute_bf16 && norms_the_stream(consumer) &&
+      consumer->first != nullptr && consumer->first->w_is_f32 && consumer->first->k == D &&
+      aligned16(consumer->first->w) && aligned16(norm->w) && m.kernels->gemm_f32_norms(M, D)) {
+    kappai_rows out = rows_of(resid, M, D, 0);
+    out.frag = KAPPAI_ROWS_OF_STREAM;
+    out.norm = norm;
+    return out;
   }
   const bool fragment = kernel_order && n >= m.tuning.fragment_rows_min && fragment_fits(m, n, D) &&
                         (carry.kind != KAPPAI_CARRY_PARTS || carry.parts <= 8);
@@ -180,7 +191,7 @@ kappai_carry attention_mixer(kappai_step* s, const void* desc, kappai_rows x, fl
     qkv.n = H * d;
     if (qkv.w_frag != nullptr && (H * d) % 16) qkv.w_frag = nullptr;
   }
-  if (!api.takes_kernel_order(&qkv, x.D)) x = api.plain_rows(s, x, resid);
+  if (x.frag != KAPPAI_ROWS_OF_STREAM && !api.takes_kernel_order(&qkv, x.D)) x = api.plain_rows(s, x, resid);
   const bool parts = takes_partial_sums(m, b, M);
   kappai_carry proj = api.linear(s, x, &qkv, m.compute_bf16, parts, nullptr, KAPPAI_REGION_BLOCK);
   if (!api.ok(s)) return none;
@@ -332,10 +343,14 @@ kappai_carry swiglu_ffn(kappai_step* s, const void* desc, kappai_rows x, float* 
   }
   // float rows and matrix: the product's own epilogue, with the bits of the two kernels
   if (!L.fused && !x.is_bf16 && !m.compute_bf16 && L.gate_up.w_is_f32 && L.gate_up.w != nullptr &&
-      L.gate_up.k == D && L.gate_up.n == 2 * F && !x.frag && x.ss == nullptr && x.D == D &&
+      L.gate_up.k == D && L.gate_up.n == 2 * F && x.frag != 1 && x.ss == nullptr && x.D == D &&
       k.gemm_f32_gates(M, F, D)) {
     float* act = (float*)api.take(s, KAPPAI_REGION_BLOCK, (size_t)M * F * 4);
-    LAUNCH(s, k.gemm_f32_swiglu((const float*)x.data, (const float*)L.gate_up.w, L.gate_up.bias, act, M, F, D,
+    if (x.frag == KAPPAI_ROWS_OF_STREAM)
+      LAUNCH(s, k.gemm_f32_normed((const float*)x.data, x.norm->w, x.norm->eps, (const float*)L.gate_up.w,
+                                  L.gate_up.bias, act, M, F, D, F, 1, api.stream(s)));
+    else
+      LAUNCH(s, k.gemm_f32_swiglu((const float*)x.data, (const float*)L.gate_up.w, L.gate_up.bias, act, M, F, D,
                                 M > 1 ? x.ld : D, F, api.stream(s)));
     return api.linear(s, rows_of(act, M, F, 0), &L.down, m.compute_bf16, 1, into, region);
   }
@@ -374,6 +389,11 @@ kappai_carry pre_norm_block(kappai_step* s, const void* desc, float* resid, kapp
   const kappai_into into_next = {resid, fold_for(after_norm, after_consumer)};
   return B.feed_forward.run(s, B.feed_forward.desc, x2, resid,
                             (B.feed_forward.flags & KAPPAI_ADDS_RESIDUAL) ? &into_next : nullptr);
+}
+
+bool norms_the_stream(const kappai_part* consumer) {
+  return consumer != nullptr &&
+         (consumer->run == conv_mixer || consumer->run == attention_mixer || consumer->run == swiglu_ffn);
 }
 
 // registered when the library is loaded

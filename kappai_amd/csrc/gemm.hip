@@ -121,6 +121,63 @@ __device__ __forceinline__ void load_chunk_f32(const float* __restrict__ row, in
   for (int j = 0; j < F32_STEPS; ++j) v[j] = load4_f32<LOADS>(row, k + 16 * j, K);
 }
 
+// M rows of the stream, normed, to LDS (F32_ROW_PAD floats between rows): x * 1/sqrt(mean(x^2) + eps) * w with the
+// bits of add_rmsnorm_row_kernel, whose wave of 64 times eight values is a turn here; a wave takes the turns
+// number wave, wave + NW, ..  `behind_loads` is called once a wave's loads are on their way.
+#define F32_ROW_PAD 16
+#define F32_NORM_TURNS 16                  // turns of all rows, at most
+template <int NW, typename F>
+__device__ __forceinline__ void f32_normed_rows(const float* __restrict__ x, const float* __restrict__ w, float eps,
+                                                int M, int D, int ldx, float* __restrict__ rows, F behind_loads) {
+  constexpr int PER = F32_NORM_TURNS / NW;
+  __shared__ __attribute__((aligned(16))) float sums[F32_NORM_TURNS][4];     // (M <= 16)
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE), lane = threadIdx.x % WAVE;
+  const int a_row = (D + 511) / 512, turns = M * a_row;
+  float v[PER][8], w8[PER][8];
+#pragma unroll
+  for (int t = 0; t < PER; ++t) {
+    const int turn = wave + t * NW, m = turn / a_row, j = (turn - m * a_row) * 512 + lane * 8;
+    if (turn >= turns) break;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) v[t][e] = 0.f;
+    if (j < D) {
+      load8(x + (size_t)m * ldx + j, v[t]);
+      load8(w + j, w8[t]);
+    }
+  }
+  ORDER_FENCE();
+  behind_loads();
+  ORDER_FENCE();
+#pragma unroll
+  for (int t = 0; t < PER; ++t) {
+    const int turn = wave + t * NW, m = turn / a_row;
+    if (turn >= turns) break;
+    const float ss = wave_sum(sum_of_squares8(v[t]));
+    if (lane == 0) sums[m][turn - m * a_row] = ss;
+    if (lane > 0 && lane < 4 && turn == m * a_row && lane >= a_row) sums[m][lane] = 0.f;
+  }
+  // (bare barriers: the loads of W stay under way)
+  __builtin_amdgcn_s_waitcnt(0xC07F);
+  __builtin_amdgcn_s_barrier();
+  ORDER_FENCE();
+#pragma unroll
+  for (int t = 0; t < PER; ++t) {
+    const int turn = wave + t * NW, m = turn / a_row, j = (turn - m * a_row) * 512 + lane * 8;
+    if (turn >= turns) break;
+    const float4 s = *reinterpret_cast<const float4*>(sums[m]);
+    const float scale = 1.0f / sqrtf((((s.x + s.y) + s.z) + s.w) / (float)D + eps);
+    if (j < D) {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) w8[t][e] = v[t][e] * scale * w8[t][e];
+      store8(rows + m * (D + F32_ROW_PAD) + j, w8[t]);
+    }
+  }
+  ORDER_FENCE();
+  __builtin_amdgcn_s_waitcnt(0xC07F);
+  __builtin_amdgcn_s_barrier();
+  ORDER_FENCE();
+}
+
 // 1 to 64 rows: bound by the stream of W, in small matrices by what one block has under way.  A
 // block owns COLS rows of W, a wave one or several runs of K, and the waves meet in LDS.  COLS = 16: a
 // wave walks its RUNS / 8 runs one after the other.  COLS = 8 (up to 8 rows; matrices of few rows, so
@@ -133,14 +190,26 @@ __device__ __forceinline__ void load_chunk_f32(const float* __restrict__ row, in
 // GATED: W holds 2 N rows, gate rows and behind them the up rows; a block's 16 columns are the gates of 8
 // results and their up rows, C[m, n] = silu(gate) up, the bits of the product and kappai_swiglu behind it.
 // (Three rows, 4,608 gates: a kernel of 4.4 us less a layer; 825 rows in blocks: 9.3 us less.)
-template <int MT, int COLS, int RUNS, int LOADS, bool GATED = false>
-__global__ __launch_bounds__((COLS == 8 ? RUNS / 2 : 8) * WAVE) void gemm_f32_skinny_kernel(
+//
+// NORM (decode steps of few rows): A is the residual stream and every block norms its rows itself, with the bits of
+// the norm's row kernel (f32_normed_rows), its first W under way meanwhile; add: the product is added to C, which is
+// that stream, so the norm has no sum left to make.  A norm kernel between two products is 4.8 us of a trace;
+// norming inside costs 9216 x 1024 gated of three rows 1.5 of its 11.2 us, 2048 x 1024 and 3072 x 1024 half a us.
+//
+// ONE: no run has more than a chunk (8 runs, K up to 1,024): nothing is under way beside the chunk, and with the
+// registers of three blocks a CU instead of two, 576 blocks of gate/up run at once (13.1 -> 12.7 us).
+template <int MT, int COLS, int RUNS, int LOADS, bool GATED = false, bool NORM = false, bool ONE = false>
+__global__ __launch_bounds__((COLS == 8 ? RUNS / 2 : 8) * WAVE) __attribute__((amdgpu_waves_per_eu(ONE ? 6 : 1)))
+void gemm_f32_skinny_kernel(
     const float* __restrict__ A, const float* __restrict__ W, const float* __restrict__ bias,
-    float* __restrict__ C, int M, int N, int K, int lda, int ldc) {
+    float* __restrict__ C, int M, int N, int K, int lda, int ldc, int add, const float* __restrict__ norm_w,
+    float eps) {
   constexpr bool SIDE = COLS == 8;               // two runs side by side
   constexpr int NW = SIDE ? RUNS / 2 : 8;
+  static_assert(!NORM || (MT == 1 && LOADS == F32_WHOLE), "few rows of whole chunks");
   static_assert(!SIDE || MT == 1, "two runs side by side leave room for 8 rows");
   __shared__ float red[RUNS][MT][SIDE ? 8 : 16][COLS];
+  extern __shared__ __attribute__((aligned(16))) float f32_rows[];      // NORM: M rows
   const int wave = threadIdx.x / WAVE, lane = threadIdx.x % WAVE;
   const int r = lane % 16, q = lane / 16;
   static_assert(!GATED || COLS == 16, "eight gates and their up rows");
@@ -192,6 +261,13 @@ __global__ __launch_bounds__((COLS == 8 ? RUNS / 2 : 8) * WAVE) void gemm_f32_sk
 #pragma unroll
     for (int j = 0; j < F32_STEPS; ++j) av[mt][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
   const auto load_a = [&](int c) {
+    if constexpr (NORM) {
+      const float* row = f32_rows + live * (K + F32_ROW_PAD) + min(c0 + c, chunks - 1) * F32_CHUNK + 4 * q;
+      if (live < M)
+#pragma unroll
+        for (int j = 0; j < F32_STEPS; ++j) av[0][j] = *reinterpret_cast<const f32x4_t*>(row + 16 * j);
+      return;
+    }
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt)
       if (mt * 16 + live < M) load_chunk_f32<LOADS>(a[mt], min(c0 + c, chunks - 1), q, K, av[mt]);
@@ -215,8 +291,23 @@ __global__ __launch_bounds__((COLS == 8 ? RUNS / 2 : 8) * WAVE) void gemm_f32_sk
 #pragma unroll
       for (int mt = 0; mt < MT; ++mt) tot[mt] += acc[mt];
   };
-  if (most > 0) {
+  // (the value that the thread's first result is added to)
+  constexpr int OUT = GATED ? 8 : COLS;
+  float old = 0.f;
+  if (add && threadIdx.x < MT * (SIDE ? 8 : 16) * OUT) {
+    const int m = threadIdx.x / OUT, n = n0 + threadIdx.x % OUT;
+    if (m < M && n < N) old = C[(size_t)m * ldc + n];
+  }
+  if constexpr (NORM) {
+    f32_normed_rows<NW>(A, norm_w, eps, M, K, lda, f32_rows, [&]() { if (most > 0) load_w(0, wv); });
+  } else if (most > 0) {
     load_w(0, wv);
+  }
+  if (ONE && most > 0) {
+    load_a(0);
+    __builtin_amdgcn_sched_barrier(0);
+    multiply(0);
+  } else if (most > 0) {
     int c = 0;
     for (; c + 1 < most; ++c) {
       f32x4_t wn[F32_STEPS];
@@ -244,12 +335,13 @@ __global__ __launch_bounds__((COLS == 8 ? RUNS / 2 : 8) * WAVE) void gemm_f32_sk
     for (int g = 1; g < RUNS; ++g) s += red[g][m / 16][m % 16][col];
     return s + (bias ? bias[row] : 0.f);
   };
-  constexpr int OUT = GATED ? 8 : COLS;
   for (int at = threadIdx.x; at < MT * (SIDE ? 8 : 16) * OUT; at += NW * WAVE) {
     const int m = at / OUT, n = n0 + at % OUT;
     if (m >= M || n >= N) continue;
     const float s = whole(m, at % OUT, n);
-    C[(size_t)m * ldc + n] = GATED ? f32_gate(s, whole(m, at % OUT + 8 * GATED, N + n)) : s;
+    float* to = C + (size_t)m * ldc + n;
+    if (add) *to = (at < NW * WAVE ? old : *to) + s;
+    else *to = GATED ? f32_gate(s, whole(m, at % OUT + 8 * GATED, N + n)) : s;
   }
 }
 
@@ -522,12 +614,13 @@ static void launch_f32_gated(const float* A, const float* W, const float* bias, 
     launch_f32_blocks<LOADS, 4, 2, true>(A, W, bias, C, M, F, K, lda, ldc, stream);
     return;
   }
-  const bool many = f32_runs((K + F32_CHUNK - 1) / F32_CHUNK) == 32;
-#define F32_GATED(MT, RUNS)                                                                          \
-  hipLaunchKernelGGL((gemm_f32_skinny_kernel<MT, 16, RUNS, LOADS, true>), dim3((F + 7) / 8),         \
-                     dim3(8 * WAVE), 0, stream, A, W, bias, C, M, F, K, lda, ldc)
+  const bool many = f32_runs((K + F32_CHUNK - 1) / F32_CHUNK) == 32, one = K <= 8 * F32_CHUNK;
+#define F32_GATED(MT, RUNS, ...)                                                                     \
+  hipLaunchKernelGGL((gemm_f32_skinny_kernel<MT, 16, RUNS, LOADS, true, ##__VA_ARGS__>), dim3((F + 7) / 8), \
+                     dim3(8 * WAVE), 0, stream, A, W, bias, C, M, F, K, lda, ldc, 0, (const float*)nullptr, 0.f)
   if (M <= 16) {
     if (many) F32_GATED(1, 32);
+    else if (LOADS == F32_WHOLE && one) F32_GATED(1, 8, false, LOADS == F32_WHOLE);
     else F32_GATED(1, 8);
   } else if (M <= 32) {
     if (many) F32_GATED(2, 32);
@@ -539,20 +632,22 @@ static void launch_f32_gated(const float* A, const float* W, const float* bias, 
 #undef F32_GATED
 }
 
+// add (up to 64 rows): to what C holds
 template <int LOADS>
 static void launch_f32(const float* A, const float* W, const float* bias, float* C, int M, int N,
-                       int K, int lda, int ldc, hipStream_t stream) {
+                       int K, int lda, int ldc, hipStream_t stream, int add = 0) {
   if (M <= 64) {
-    const bool many = f32_runs((K + F32_CHUNK - 1) / F32_CHUNK) == 32;
-#define F32_SKINNY(MT, COLS, RUNS)                                                                \
-  hipLaunchKernelGGL((gemm_f32_skinny_kernel<MT, COLS, RUNS, LOADS>), dim3((N + COLS - 1) / COLS), \
+    const bool many = f32_runs((K + F32_CHUNK - 1) / F32_CHUNK) == 32, one = K <= 8 * F32_CHUNK;
+#define F32_SKINNY(MT, COLS, RUNS, ...)                                                           \
+  hipLaunchKernelGGL((gemm_f32_skinny_kernel<MT, COLS, RUNS, LOADS, false, ##__VA_ARGS__>), dim3((N + COLS - 1) / COLS), \
                      dim3((COLS == 8 ? RUNS / 2 : 8) * WAVE), 0, stream, A, W, bias, C, M, N, K,   \
-                     lda, ldc)
+                     lda, ldc, add, (const float*)nullptr, 0.f)
     if (M <= 8 && N <= 256 * 8) {
       if (many) F32_SKINNY(1, 8, 32);
       else F32_SKINNY(1, 8, 8);
     } else if (M <= 16) {
       if (many) F32_SKINNY(1, 16, 32);
+      else if (LOADS == F32_WHOLE && one) F32_SKINNY(1, 16, 8, false, LOADS == F32_WHOLE);
       else F32_SKINNY(1, 16, 8);
     } else if (M <= 32) {
       if (many) F32_SKINNY(2, 16, 32);
@@ -579,6 +674,48 @@ extern "C" int kappai_gemm_f32(const float* A, const float* W, const float* bias
   else if (fours && K % F32_CHUNK == 0) launch_f32<F32_WHOLE>(A, W, bias, C, M, N, K, lda, ldc, stream);
   else if (fours) launch_f32<F32_FOURS>(A, W, bias, C, M, N, K, lda, ldc, stream);
   else launch_f32<F32_ELEMENTS>(A, W, bias, C, M, N, K, lda, ldc, stream);
+  KAPPAI_RETURN_LAUNCH_STATUS();
+}
+
+extern "C" int kappai_gemm_f32_gates(int M, int F, int K);
+// The two ends of a decode step's products that save the norm's kernel between them.
+// kappai_gemm_f32_add: C += A W^T (+ bias), up to 64 rows, the bits of the product and a sum behind it.
+extern "C" int kappai_gemm_f32_add(const float* A, const float* W, const float* bias, float* C, int M, int N, int K,
+                                   int lda, int ldc, hipStream_t stream) {
+  if (M <= 0 || N <= 0) return 0;
+  if (M > 64 || K < 4) return (int)hipErrorInvalidValue;
+  const bool fours = K % 4 == 0 && lda % 4 == 0 && (uintptr_t)A % 16 == 0 && (uintptr_t)W % 16 == 0;
+  if (fours && K % F32_CHUNK == 0) launch_f32<F32_WHOLE>(A, W, bias, C, M, N, K, lda, ldc, stream, 1);
+  else if (fours) launch_f32<F32_FOURS>(A, W, bias, C, M, N, K, lda, ldc, stream, 1);
+  else launch_f32<F32_ELEMENTS>(A, W, bias, C, M, N, K, lda, ldc, stream, 1);
+  KAPPAI_RETURN_LAUNCH_STATUS();
+}
+// kappai_gemm_f32_normed: the product, or with `gated` silu(gate) up over 2 N rows of W, of the RMS-normed rows of x
+// [M, K], the bits of the norm's kernel and the product behind it.  For rows that kappai_gemm_f32_norms takes: up to
+// 8 and 16 turns of 512 values (8 rows of 1,024, 4 of 2,048; every block norms all of them), whole chunks of K.
+extern "C" int kappai_gemm_f32_norms(int M, int K) {
+  return M >= 1 && M <= 8 && K >= F32_CHUNK && K <= 16 * F32_CHUNK && K % F32_CHUNK == 0 &&
+         M * ((K + 511) / 512) <= F32_NORM_TURNS;
+}
+extern "C" int kappai_gemm_f32_normed(const float* x, const float* norm_w, float eps, const float* W,
+                                      const float* bias, float* C, int M, int N, int K, int ldc, int gated,
+                                      hipStream_t stream) {
+  if (M <= 0 || N <= 0) return 0;
+  if (!kappai_gemm_f32_norms(M, K) || ((uintptr_t)x | (uintptr_t)W | (uintptr_t)norm_w) % 16 ||
+      (gated && !kappai_gemm_f32_gates(M, N, K)))
+    return (int)hipErrorInvalidValue;
+  const size_t lds = (size_t)M * (K + F32_ROW_PAD) * sizeof(float);       // (up to 33 KB)
+#define F32_NORMED(COLS, GATED, BLOCK, ONE)                                                             \
+  hipLaunchKernelGGL((gemm_f32_skinny_kernel<1, COLS, 8, F32_WHOLE, GATED, true, ONE>),                 \
+                     dim3((N + BLOCK - 1) / BLOCK), dim3((COLS == 8 ? 4 : 8) * WAVE), lds, stream, x, W, \
+                     bias, C, M, N, K, K, ldc, 0, norm_w, eps)
+  const bool one = K <= 8 * F32_CHUNK;
+  if (gated && one) F32_NORMED(16, true, 8, true);
+  else if (gated) F32_NORMED(16, true, 8, false);
+  else if (N <= 256 * 8) F32_NORMED(8, false, 8, false);
+  else if (one) F32_NORMED(16, false, 16, true);
+  else F32_NORMED(16, false, 16, false);
+#undef F32_NORMED
   KAPPAI_RETURN_LAUNCH_STATUS();
 }
 

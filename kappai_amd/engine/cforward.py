@@ -24,7 +24,7 @@ from ..parts.cdesc import (AttentionKernels, CallDesc, CarryDesc, CPlan, Embedde
                            FoldDesc, LinearDesc, NormPartDesc, PartDesc, RowsDesc, address_of,
                            defined_together)
 
-ENGINE_ABI = 12
+ENGINE_ABI = 13
 MAX_GROUPS = 8
 MAX_TABLES = 8         # KAPPAI_MAX_TABLES
 
@@ -35,7 +35,8 @@ def _ptrs(names):
 
 class Kernels(Structure):
     _fields_ = _ptrs(["embed_rows", "embed_rmsnorm", "add_rmsnorm", "swiglu", "cast",
-                      "sum_partials", "gemm_f32", "gemm_f32_gates", "gemm_f32_swiglu", "gemm_bf16",
+                      "sum_partials", "gemm_f32", "gemm_f32_add", "gemm_f32_norms",
+                      "gemm_f32_normed", "gemm_f32_gates", "gemm_f32_swiglu", "gemm_bf16",
                       "gemm_bf16_any", "gemm_bf16_swiglu", "gemm_bf16_shortconv_step", "shortconv", "shortconv_parts",
                       "qk_norm_rope_store", "paged_attention_rows"])
 
@@ -142,6 +143,9 @@ class CForward:
                          ("swiglu", el.kappai_swiglu), ("cast", el.kappai_cast),
                          ("sum_partials", el.kappai_sum_partials),
                          ("gemm_f32", gm.kappai_gemm_f32),
+                         ("gemm_f32_add", gm.kappai_gemm_f32_add),
+                         ("gemm_f32_norms", gm.kappai_gemm_f32_norms),
+                         ("gemm_f32_normed", gm.kappai_gemm_f32_normed),
                          ("gemm_f32_gates", gm.kappai_gemm_f32_gates),
                          ("gemm_f32_swiglu", gm.kappai_gemm_f32_swiglu),
                          ("gemm_bf16", gm.kappai_gemm_bf16),

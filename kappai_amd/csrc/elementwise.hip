@@ -71,14 +71,14 @@ extern "C" int kappai_embed_rows(const int* ids, const void* table, int table_is
 // A norm on what a sublayer returns: y = scale_a * a (+ scale_b * b), n = y / sqrt(mean(y^2) + eps)
 // * w, then resid += n (or resid = n), and the new resid again in the compute dtype for the next
 // sublayer to read.  a may come as `a_parts` float planes [parts][T][D] that are added in order
-// first (a product cut over its input dimension).  Everything in float32; a block a row, the row
+// first (a product cut over its input dimension); a and b in a type each.  Everything in float32; a block a row, the row
 // kept in LDS between the sum of squares and the scaling.  `vec`: D is a multiple of eight and
 // every pointer of 32 bytes, so a thread takes eight values at a time and asks for the planes
 // four at a time (same sums in the same order).
 // ---------------------------------------------------------------------------------------
-template <typename TA, typename TO>
+template <typename TA, typename TB, typename TO>
 __global__ __launch_bounds__(256) void output_norm_add_kernel(
-    const TA* __restrict__ a, int a_parts, size_t a_plane, float scale_a, const TA* __restrict__ b,
+    const TA* __restrict__ a, int a_parts, size_t a_plane, float scale_a, const TB* __restrict__ b,
     float scale_b, const float* __restrict__ w, float eps, float* __restrict__ resid, int add,
     TO* __restrict__ rows, int D, int vec) {
   extern __shared__ __attribute__((aligned(16))) float ys[];
@@ -143,9 +143,9 @@ __global__ __launch_bounds__(256) void output_norm_add_kernel(
 // scaling, and the weights and the stream are asked for with the planes (above they are a second trip to memory).
 // NP: the number of planes, 1 to 4, else 0 and a loop over a_parts.  Eight rows of 1,024,
 // one plane 2.35 -> 1.94 us one after another, four planes 2.69 -> 2.01; 1,800 rows 5.11 -> 4.53.
-template <typename TA, typename TO, int NP>
+template <typename TA, typename TB, typename TO, int NP>
 __global__ __launch_bounds__(256) void output_norm_add_row_kernel(
-    const TA* __restrict__ a, const float* __restrict__ w, float* __restrict__ resid, const TA* __restrict__ b,
+    const TA* __restrict__ a, const float* __restrict__ w, float* __restrict__ resid, const TB* __restrict__ b,
     size_t a_plane, int D, int a_parts, float scale_a, int add, float scale_b, float eps, TO* __restrict__ rows) {
   __shared__ __attribute__((aligned(16))) float red[16];
   const size_t at = (size_t)blockIdx.x * D;
@@ -196,20 +196,20 @@ __global__ __launch_bounds__(256) void output_norm_add_row_kernel(
   if (rows != nullptr) store8(rows + at + e, y);
 }
 
-template <typename TA, typename TO>
+template <typename TA, typename TB, typename TO>
 static void launch_output_norm_add(const void* a, int a_parts, size_t plane, float scale_a, const void* b,
                                    float scale_b, const float* w, float eps, float* resid, int add, void* rows,
                                    int T, int D, int vec, hipStream_t stream) {
   if (!vec || D > 8 * 256) {
-    hipLaunchKernelGGL((output_norm_add_kernel<TA, TO>), dim3(T), dim3(256), (size_t)D * sizeof(float), stream,
-                       (const TA*)a, a_parts, plane, scale_a, (const TA*)b, scale_b, w, eps, resid, add,
+    hipLaunchKernelGGL((output_norm_add_kernel<TA, TB, TO>), dim3(T), dim3(256), (size_t)D * sizeof(float), stream,
+                       (const TA*)a, a_parts, plane, scale_a, (const TB*)b, scale_b, w, eps, resid, add,
                        (TO*)rows, D, vec);
     return;
   }
   const int threads = ((D / 8 + WAVE - 1) / WAVE) * WAVE;
 #define KAPPAI_OUT_NORM_ROW(NP)                                                                          \
-  hipLaunchKernelGGL((output_norm_add_row_kernel<TA, TO, NP>), dim3(T), dim3(threads), 0, stream,        \
-                     (const TA*)a, w, resid, (const TA*)b, plane, D, a_parts, scale_a, add, scale_b, eps, \
+  hipLaunchKernelGGL((output_norm_add_row_kernel<TA, TB, TO, NP>), dim3(T), dim3(threads), 0, stream,        \
+                     (const TA*)a, w, resid, (const TB*)b, plane, D, a_parts, scale_a, add, scale_b, eps, \
                      (TO*)rows)
   constexpr bool planes = sizeof(TA) == 4;
   if (a_parts == 1 || !planes) KAPPAI_OUT_NORM_ROW(1);
@@ -221,7 +221,7 @@ static void launch_output_norm_add(const void* a, int a_parts, size_t plane, flo
 }
 
 extern "C" int kappai_output_norm_add(const void* a, int a_is_bf16, int a_parts, float scale_a,
-                                      const void* b, float scale_b, const float* w, float eps,
+                                      const void* b, int b_is_bf16, float scale_b, const float* w, float eps,
                                       float* resid, int add, void* rows, int rows_is_bf16, int T,
                                       int D, hipStream_t stream) {
   if (T <= 0) return 0;
@@ -230,13 +230,21 @@ extern "C" int kappai_output_norm_add(const void* a, int a_is_bf16, int a_parts,
   const size_t plane = (size_t)T * D;
   const int vec = D % 8 == 0 && ((uintptr_t)a | (uintptr_t)b | (uintptr_t)w | (uintptr_t)resid |
                                  (uintptr_t)rows) % 32 == 0;
-#define KAPPAI_OUT_NORM(TA, TO)                                                                  \
-  launch_output_norm_add<TA, TO>(a, a_parts, plane, scale_a, b, scale_b, w, eps, resid, add, rows, \
-                                 T, D, vec, stream)
+#define KAPPAI_OUT_NORM(TA, TO)                                                                          \
+  do {                                                                                                  \
+    if (b_is_bf16)                                                                                      \
+      launch_output_norm_add<TA, bf16_t, TO>(a, a_parts, plane, scale_a, b, scale_b, w, eps, resid, add, \
+                                             rows, T, D, vec, stream);                                  \
+    else                                                                                                \
+      launch_output_norm_add<TA, float, TO>(a, a_parts, plane, scale_a, b, scale_b, w, eps, resid, add,  \
+                                            rows, T, D, vec, stream);                                   \
+  } while (0)
   if (a_is_bf16) {
-    if (rows_is_bf16) KAPPAI_OUT_NORM(bf16_t, bf16_t); else KAPPAI_OUT_NORM(bf16_t, float);
+    if (rows_is_bf16) KAPPAI_OUT_NORM(bf16_t, bf16_t);
+    else KAPPAI_OUT_NORM(bf16_t, float);
   } else {
-    if (rows_is_bf16) KAPPAI_OUT_NORM(float, bf16_t); else KAPPAI_OUT_NORM(float, float);
+    if (rows_is_bf16) KAPPAI_OUT_NORM(float, bf16_t);
+    else KAPPAI_OUT_NORM(float, float);
   }
 #undef KAPPAI_OUT_NORM
   KAPPAI_RETURN_LAUNCH_STATUS();
@@ -559,48 +567,76 @@ extern "C" int kappai_rms_norm_step(
 
 // ---------------------------------------------------------------------------------------
 // Two sublayers' results side by side, made one update of the stream in float32:
-// out = scale_a * n_a(a) + scale_b * n_b(b), with n(y) = y / sqrt(mean(y^2) + eps) * w when a
-// weight is given and y itself when not.  a, b [T, D] in float32 or bfloat16 (one dtype); a block
-// a row, both rows in LDS between the sums of squares and the scaling.
+// u = scale_a * n_a(a) + scale_b * n_b(b), with n(y) = y / sqrt(mean(y^2) + eps) * w when a
+// weight is given and y itself when not.  a, b [T, D] in float32 or bfloat16, a type each, or float planes
+// [parts][T][D] that are added in order first; a block a row, both rows in LDS between the sums of squares and the
+// scaling.  resid null: u goes to out.  Else resid += u and, with norm_w, what the product behind the next RMS norm
+// reads (up to 16 rows): rows = bf16(resid * norm_w) and ss[row] the sum of resid^2.
+// In a decode step of few rows the sums over planes, the widening of one side, this and the norm behind it were four
+// kernels of 4 us each.
 // ---------------------------------------------------------------------------------------
-template <typename TA>
+template <typename TA, typename TB>
 __global__ __launch_bounds__(256) void pair_norm_sum_kernel(
-    const TA* __restrict__ a, float scale_a, const float* __restrict__ wa,
-    const TA* __restrict__ b, float scale_b, const float* __restrict__ wb, float eps, int D,
-    float* __restrict__ out) {
+    const TA* __restrict__ a, const TB* __restrict__ b, const float* __restrict__ wa, const float* __restrict__ wb,
+    int a_parts, int b_parts, int D, float scale_a, float scale_b, float eps, size_t plane, float* __restrict__ out,
+    float* __restrict__ resid, const float* __restrict__ norm_w, bf16_t* __restrict__ rows, float* __restrict__ ss) {
   extern __shared__ __attribute__((aligned(16))) float ys[];
   __shared__ float red[16];
   const size_t at = (size_t)blockIdx.x * D;
   float sa = 0.f, sb = 0.f;
   for (int e = threadIdx.x; e < D; e += 256) {
-    const float x = to_f32(a[at + e]), y = to_f32(b[at + e]);
+    float x = to_f32(a[at + e]), y = to_f32(b[at + e]);
+    for (int k = 1; k < a_parts; ++k) x += to_f32(a[k * plane + at + e]);
+    for (int k = 1; k < b_parts; ++k) y += to_f32(b[k * plane + at + e]);
     ys[e] = x;
     ys[D + e] = y;
     sa = fmaf(x, x, sa);
     sb = fmaf(y, y, sb);
   }
-  float fa = scale_a, fb = scale_b;
+  float fa = scale_a, fb = scale_b, q = 0.f;
   if (wa != nullptr) fa *= 1.0f / sqrtf(block_sum(sa, red) / (float)D + eps);
   if (wb != nullptr) fb *= 1.0f / sqrtf(block_sum(sb, red) / (float)D + eps);
   for (int e = threadIdx.x; e < D; e += 256) {
     const float x = ys[e] * fa * (wa != nullptr ? wa[e] : 1.f);
     const float y = ys[D + e] * fb * (wb != nullptr ? wb[e] : 1.f);
-    out[at + e] = x + y;
+    if (resid == nullptr) {
+      out[at + e] = x + y;
+    } else {
+      const float r = resid[at + e] + (x + y);
+      resid[at + e] = r;
+      if (norm_w != nullptr) {
+        rows[at + e] = f32_to_bf16(r * norm_w[e]);
+        q = fmaf(r, r, q);
+      }
+    }
+  }
+  if (norm_w != nullptr) {
+    q = block_sum(q, red);
+    if (threadIdx.x == 0) ss[blockIdx.x] = q;
   }
 }
 
-extern "C" int kappai_pair_norm_sum(const void* a, float scale_a, const float* wa, const void* b,
-                                    float scale_b, const float* wb, float eps, int T, int D,
-                                    float* out, int is_bf16, hipStream_t stream) {
+extern "C" int kappai_pair_norm_sum(const void* a, int a_is_bf16, int a_parts, float scale_a, const float* wa,
+                                    const void* b, int b_is_bf16, int b_parts, float scale_b, const float* wb,
+                                    float eps, int T, int D, float* out, float* resid, const float* norm_w,
+                                    void* rows, float* ss, hipStream_t stream) {
   if (T <= 0) return 0;
-  if (D < 1 || D > 7 * 1024) return (int)hipErrorInvalidValue;
-  const size_t lds = 2 * (size_t)D * sizeof(float);
-  if (is_bf16)
-    hipLaunchKernelGGL(pair_norm_sum_kernel<bf16_t>, dim3(T), dim3(256), lds, stream,
-                       (const bf16_t*)a, scale_a, wa, (const bf16_t*)b, scale_b, wb, eps, D, out);
-  else
-    hipLaunchKernelGGL(pair_norm_sum_kernel<float>, dim3(T), dim3(256), lds, stream,
-                       (const float*)a, scale_a, wa, (const float*)b, scale_b, wb, eps, D, out);
+  if (D < 1 || D > 7 * 1024 || a_parts < 1 || b_parts < 1 || (a_is_bf16 && a_parts != 1) ||
+      (b_is_bf16 && b_parts != 1) || (out == nullptr) == (resid == nullptr) ||
+      (norm_w != nullptr && (resid == nullptr || rows == nullptr || ss == nullptr || T > 16)))
+    return (int)hipErrorInvalidValue;
+#define KAPPAI_PAIR(TA, TB)                                                                               \
+  hipLaunchKernelGGL((pair_norm_sum_kernel<TA, TB>), dim3(T), dim3(256), 2 * (size_t)D * sizeof(float), stream, \
+                     (const TA*)a, (const TB*)b, wa, wb, a_parts, b_parts, D, scale_a, scale_b, eps,      \
+                     (size_t)T * D, out, resid, norm_w, (bf16_t*)rows, ss)
+  if (a_is_bf16) {
+    if (b_is_bf16) KAPPAI_PAIR(bf16_t, bf16_t);
+    else KAPPAI_PAIR(bf16_t, float);
+  } else {
+    if (b_is_bf16) KAPPAI_PAIR(float, bf16_t);
+    else KAPPAI_PAIR(float, float);
+  }
+#undef KAPPAI_PAIR
   KAPPAI_RETURN_LAUNCH_STATUS();
 }
 

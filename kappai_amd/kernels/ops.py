@@ -2128,8 +2128,8 @@ def output_norm_add(resid: torch.Tensor, a: torch.Tensor, weight: torch.Tensor, 
                     scale_b: float = 1.0, add: bool = True) -> Optional[torch.Tensor]:
     """``y = scale_a a (+ scale_b b)``; ``resid (+)= y / sqrt(mean(y^2) + eps) * weight`` in
     float32, in place (``add`` False: the residual becomes the normalised rows).  ``a``: [T, D]
-    in float32 or bfloat16, or float32 partial sums [S, T, D], added in order first; ``b`` like
-    ``a`` but always [T, D].  With ``rows_dtype`` the new residual is also returned rounded to that
+    in float32 or bfloat16, or float32 partial sums [S, T, D], added in order first; ``b`` [T, D] in
+    float32 or bfloat16.  With ``rows_dtype`` the new residual is also returned rounded to that
     dtype, for the next sublayer to read."""
     _gpu("resid", resid, F32)
     _gpu("a", a, (F32, BF16))
@@ -2142,14 +2142,14 @@ def output_norm_add(resid: torch.Tensor, a: torch.Tensor, weight: torch.Tensor, 
     _need(tuple(a.shape[-2:]) == (T, D) and weight.shape == (D,),
           lambda: f"output_norm_add: {tuple(a.shape)} into {tuple(resid.shape)}")
     if b is not None:
-        _gpu("b", b, a.dtype)
+        _gpu("b", b, (F32, BF16))
         _need(tuple(b.shape) == (T, D), lambda: f"output_norm_add: b {tuple(b.shape)}")
     rows = None
     if rows_dtype is not None:
         rows = torch.empty((T, D), dtype=rows_dtype, device=resid.device)
     check(library("elementwise").kappai_output_norm_add(
         _ptr(a), _c_int(_is_bf16(a.dtype)), _c_int(parts), _c_float(scale_a), _ptr(b),
-        _c_float(scale_b), _ptr(weight), _c_float(eps), _ptr(resid), _c_int(1 if add else 0),
+        _c_int(_is_bf16(b.dtype) if b is not None else 0), _c_float(scale_b), _ptr(weight), _c_float(eps), _ptr(resid), _c_int(1 if add else 0),
         _ptr(rows), _c_int(_is_bf16(rows_dtype) if rows is not None else 0), _c_int(T), _c_int(D),
         _stream()), "output_norm_add")
     return rows
@@ -2157,25 +2157,42 @@ def output_norm_add(resid: torch.Tensor, a: torch.Tensor, weight: torch.Tensor, 
 
 def pair_norm_sum(a: torch.Tensor, b: torch.Tensor, scale_a: float = 1.0, scale_b: float = 1.0,
                   weight_a: Optional[torch.Tensor] = None,
-                  weight_b: Optional[torch.Tensor] = None, eps: float = 0.0) -> torch.Tensor:
+                  weight_b: Optional[torch.Tensor] = None, eps: float = 0.0,
+                  add_into: Optional[AddInto] = None):
     """``scale_a * n_a(a) + scale_b * n_b(b)`` in float32, ``n(y) = y / sqrt(mean(y^2) + eps) * w``
-    where a weight [D] is given and ``y`` itself where not.  ``a``, ``b`` [T, D] in one dtype
-    (float32 or bfloat16).  Returns float32 [T, D]."""
-    _gpu("a", a, (F32, BF16))
-    _gpu("b", b, a.dtype)
-    _need(a.dim() == 2 and a.shape == b.shape, lambda: f"pair_norm_sum: {tuple(a.shape)} and "
-                                                       f"{tuple(b.shape)}")
-    T, D = a.shape
+    where a weight [D] is given and ``y`` itself where not.  ``a``, ``b``: [T, D] in float32 or
+    bfloat16, or float32 partial sums [S, T, D], added in order first.  Returns float32 [T, D].
+    ``add_into`` (bfloat16 steps): up to 16 rows are added into the stream, and the norm behind it folded in, as a
+    product does it; the result is then ``Added`` or ``ScaledRows``."""
+    T, D = a.shape[-2:]
+    for name, y in (("a", a), ("b", b)):
+        _gpu(name, y, (F32, BF16))
+        _need((y.dim() == 2 or (y.dim() == 3 and y.dtype == F32)) and tuple(y.shape[-2:]) == (T, D),
+              lambda: f"pair_norm_sum: {tuple(a.shape)} and {tuple(b.shape)}")
     for name, w in (("weight_a", weight_a), ("weight_b", weight_b)):
         if w is not None:
             _gpu(name, w, F32)
             _need(w.shape == (D,), lambda: f"pair_norm_sum: {name} {tuple(w.shape)}")
-    out = torch.empty((T, D), dtype=F32, device=a.device)
+    out = resid = nw = rows = ss = None
+    if (add_into is not None and T <= FUSED_MAX_ROWS and add_into.resid.dtype == F32
+            and add_into.resid.is_contiguous() and tuple(add_into.resid.shape) == (T, D)):
+        resid, nw = add_into.resid, add_into.norm_weight
+        _gpu("resid", resid, F32)
+        if nw is not None:
+            _gpu("norm_weight", nw, F32)
+            _need(nw.shape == (D,), lambda: f"pair_norm_sum: norm weight {tuple(nw.shape)}")
+            rows = torch.empty((T, D), dtype=BF16, device=a.device)
+            ss = torch.empty((1, 16), dtype=F32, device=a.device)
+    else:
+        out = torch.empty((T, D), dtype=F32, device=a.device)
     check(library("elementwise").kappai_pair_norm_sum(
-        _ptr(a), _c_float(scale_a), _ptr(weight_a), _ptr(b), _c_float(scale_b), _ptr(weight_b),
-        _c_float(eps), _c_int(T), _c_int(D), _ptr(out), _c_int(_is_bf16(a.dtype)), _stream()),
-        "pair_norm_sum")
-    return out
+        _ptr(a), _c_int(_is_bf16(a.dtype)), _c_int(a.shape[0] if a.dim() == 3 else 1), _c_float(scale_a),
+        _ptr(weight_a), _ptr(b), _c_int(_is_bf16(b.dtype)), _c_int(b.shape[0] if b.dim() == 3 else 1),
+        _c_float(scale_b), _ptr(weight_b), _c_float(eps), _c_int(T), _c_int(D), _ptr(out), _ptr(resid), _ptr(nw),
+        _ptr(rows), _ptr(ss), _stream()), "pair_norm_sum")
+    if resid is None:
+        return out
+    return Added(resid) if nw is None else ScaledRows(rows, T, False, ss, nw, add_into.eps, resid)
 
 
 def stream_enter(resid: torch.Tensor, delta: Optional[torch.Tensor],

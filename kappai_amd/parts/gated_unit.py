@@ -27,6 +27,9 @@ from .mingru import ScanChunks
 
 
 class RealGatedUnit(Mixer):
+    takes_deferred_rows = True     # (its first product does)
+    adds_residual = True
+
     def __init__(self, prefix: str, width: int, inner: int, blocks: int, taps: int,
                  dtype: torch.dtype, rate: float = 8.0, names=None,
                  weight_suffix: str = ".weight", bias_suffix: str = ".bias"):
@@ -87,7 +90,7 @@ class RealGatedUnit(Mixer):
         lam = tensors[self._lam].to(torch.float64)
         self.softplus_lam = torch.nn.functional.softplus(lam).to(torch.float32).contiguous()
 
-    def forward(self, x, batch, cache, shared_cache: bool = False):
+    def forward(self, x, batch, cache, shared_cache: bool = False, into=None):
         if shared_cache:
             raise ValueError("a recurrent state cannot be read by another layer")
         C = self.inner
@@ -105,7 +108,7 @@ class RealGatedUnit(Mixer):
                 y = ops.gated_unit_step(proj, self.conv_taps, self.conv_bias, conv_state,
                                         self.gate_w, self.gate_b, self.softplus_lam, self.rate,
                                         state, batch.seg_pos0, batch.seg_slot)
-            return self.out.forward(y, partial_sums=True)
+            return self.out.forward(y, partial_sums=True, add_into=into)
         with profile.scope("short_conv"):
             u = ops.conv_silu(proj, self.conv_taps, conv_state, batch.row_pos, batch.row_seg,
                               batch.seg_start, batch.seg_pos0, batch.seg_slot,
@@ -123,7 +126,7 @@ class RealGatedUnit(Mixer):
                 chunks=batch.extra.get("scan_chunks") if chunked else None,
                 seg_chunk0=batch.extra.get("scan_seg_chunk0") if chunked else None,
                 gate_part=part)
-        return self.out.forward(y, partial_sums=True)
+        return self.out.forward(y, partial_sums=True, add_into=into)
 
     def weight_bytes(self) -> int:
         return (self.inputs.weight_bytes() + self.out.weight_bytes()

@@ -146,6 +146,8 @@ register_part("mixer", "gated_linear_attention", GatedLinearAttention)
 
 
 class FixedDecayAttention(Mixer):
+    takes_deferred_rows = True     # (its one product of the rows does)
+
     def __init__(self, prefix: str, width: int, num_heads: int, dim: int, vdim: int, decay,
                  norm_eps: float, dtype: torch.dtype, names=None, weight_suffix: str = ".weight"):
         n = {"q": "q", "k": "k", "v": "v", "g": "g", "norm": "norm", "o": "o"}

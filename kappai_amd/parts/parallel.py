@@ -84,20 +84,29 @@ class ParallelMixer(Mixer):
             self.norm_w = tuple(tensors[name].to(torch.float32).contiguous()
                                 for name in self.side_norms)
 
-    def forward(self, x, batch, cache, shared_cache: bool = False):
+    @property
+    def takes_deferred_rows(self) -> bool:
+        return all(getattr(m, "takes_deferred_rows", False) for _, m in self._sides())
+
+    @property
+    def adds_residual(self) -> bool:
+        return self.summed               # (the sum of the two sides is an update of the stream)
+
+    def forward(self, x, batch, cache, shared_cache: bool = False, into=None):
         if shared_cache:
             raise ValueError("a pair of mixers does not read another layer's cache")
-        out = []
-        for side, m in self._sides():
-            y = m.forward(x, batch, self._view(cache, side, m))
-            if isinstance(y, torch.Tensor) and y.dim() == 3:
-                y = ops.sum_partial_sums(y)
-            out.append(y)
-        if out[0].dtype != out[1].dtype:
+        out = [m.forward(x, batch, self._view(cache, side, m)) for side, m in self._sides()]
+        # the kernel that sums the two reads planes and either type itself; elsewhere they are made alike first
+        in_kernel = out[0].is_cuda
+        for i, y in enumerate(out):
+            if y.dim() == 3 and not (in_kernel and (self.summed or i == 0)):
+                out[i] = ops.sum_partial_sums(y)
+        if out[0].dtype != out[1].dtype and not in_kernel:
             out = [y if y.dtype == torch.float32 else ops.cast(y, torch.float32) for y in out]
         if self.summed:
+            how = {} if into is None or x.dtype != torch.bfloat16 or not in_kernel else {"add_into": into}
             return ops.pair_norm_sum(out[0], out[1], self.left_scale, self.right_scale,
-                                     self.norm_w[0], self.norm_w[1], self.norm_eps)
+                                     self.norm_w[0], self.norm_w[1], self.norm_eps, **how)
         return WeightedTerms(out[0], self.left_scale, out[1], self.right_scale)
 
     def weight_bytes(self) -> int:

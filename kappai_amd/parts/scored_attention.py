@@ -70,6 +70,8 @@ def distance_bias_columns(table: torch.Tensor, far: float) -> torch.Tensor:
 
 
 class ScoredAttention(Mixer):
+    takes_deferred_rows = True     # (its one product of the rows does)
+
     def __init__(self, prefix: str, width: int, num_heads: int, num_kv_heads: int, dim: int,
                  vdim: int, scale: float, dtype: torch.dtype, norm_eps: float = 0.0,
                  whole_qk_norm: bool = False, softcap: float = 0.0,

@@ -1,0 +1,53 @@
+"""Two sublayers' results summed by one kernel: sides of either type and as float planes against the sum of the planes,
+the widening and the sum one behind the other (bit for bit), into the stream with the next norm's rows, and a norm on
+two terms of different types."""
+import pytest
+import torch
+
+from test_kernels_gpu import BF16, DEV, F32, close, ops, rand  # noqa: F401
+
+pytestmark = pytest.mark.gpu
+SIDES = {"bf16": (BF16, 1), "f32": (F32, 1), "planes": (F32, 3)}
+
+
+def side(kind, T, D, seed):
+    dtype, parts = SIDES[kind]
+    y = rand((T, D) if parts == 1 else (parts, T, D), dtype, seed).to(DEV)
+    return y, y.float() if parts == 1 else y[0] + y[1] + y[2]
+
+
+@pytest.mark.parametrize("T,D", [(1, 8), (3, 1024), (16, 260), (17, 1024), (40, 2100)])
+@pytest.mark.parametrize("a", list(SIDES))
+@pytest.mark.parametrize("b", list(SIDES))
+@pytest.mark.parametrize("normed", [False, True])
+def test_two_sides(ops, T, D, a, b, normed):  # noqa: F811
+    (ya, fa), (yb, fb) = side(a, T, D, 1), side(b, T, D, 2)
+    wa, wb = (rand((D,), F32, 3).to(DEV), rand((D,), F32, 4).to(DEV)) if normed else (None, None)
+    want = ops.pair_norm_sum(fa, fb, 0.5, 0.75, wa, wb, 1e-5)
+    assert torch.equal(ops.pair_norm_sum(ya, yb, 0.5, 0.75, wa, wb, 1e-5), want)
+    resid, norm_w = rand((T, D), F32, 5).to(DEV), rand((D,), F32, 6).to(DEV)
+    for nw in (None, norm_w):
+        stream = resid.clone()
+        got = ops.pair_norm_sum(ya, yb, 0.5, 0.75, wa, wb, 1e-5, add_into=ops.AddInto(stream, nw, 1e-5))
+        if T > 16:
+            assert torch.equal(got, want) and torch.equal(stream, resid)
+            continue
+        assert torch.equal(stream, resid + want) and got.resid is stream
+        if nw is None:
+            assert type(got) is ops.Added
+        else:
+            assert torch.equal(got.data, (stream * nw).bfloat16())
+            # (D squares, each added once: no more roundings than that)
+            close(got.ss[0, :T], stream.double().pow(2).sum(-1), (D + 1) * 2.0 ** -24, "sum of squares")
+
+
+@pytest.mark.parametrize("T,D", [(2, 1024), (5, 1028), (3, 2056)])
+@pytest.mark.parametrize("a", list(SIDES))
+@pytest.mark.parametrize("b", ["bf16", "f32"])
+def test_a_norm_on_two_terms(ops, T, D, a, b):  # noqa: F811
+    (ya, fa), (yb, fb) = side(a, T, D, 7), side(b, T, D, 8)
+    w, resid = rand((D,), F32, 9).to(DEV), rand((T, D), F32, 10).to(DEV)
+    one, two = resid.clone(), resid.clone()
+    rows = ops.output_norm_add(one, ya, w, 1e-5, rows_dtype=BF16, scale_a=0.5, b=yb, scale_b=0.25)
+    want = ops.output_norm_add(two, fa, w, 1e-5, rows_dtype=BF16, scale_a=0.5, b=fb, scale_b=0.25)
+    assert torch.equal(rows, want) and torch.equal(one, two)

@@ -40,6 +40,16 @@ __device__ __forceinline__ void in_rounds(int n, int tid, L load, U use) {
 }
 struct Two { float a, b; };
 
+// Blocks a row for `items` places of it, where rows are few: the chip is empty, every round of a block is its own
+// trips to memory behind the row's position, and a block a round makes them at once.  Two rows of a decode step,
+// one block a row and so: rotate_widen_store 6.5 and 4.6 us, latent_store 6.0 and 3.9, projection_norm_store 6.0
+// and 4.2.  Beyond FEW_ROWS rows one block a row, whose position and page are then read once (1,900 rows: 10.5 to
+// 12 us each, which blocks of one round would need ten times as many of).
+#define FEW_ROWS 32
+static int few_rows_blocks(int T, int items) {
+  return T > FEW_ROWS || items < 1 ? 1 : (items + AP_THREADS - 1) / AP_THREADS;
+}
+
 // ---------------------------------------------------------------------------------------
 template <typename T>
 __global__ __launch_bounds__(AP_THREADS) void projection_norm_store_kernel(
@@ -55,21 +65,27 @@ __global__ __launch_bounds__(AP_THREADS) void projection_norm_store_kernel(
   const T* row = proj + (size_t)t * stride;
   const int nq = H * d, nk = G * d;
   const auto value = [&](int i) { return to_f32(row[i]); };
+  // one block: everything; several: the last has keys and values, the others a part of the queries each, after
+  // the same sum over all of them
+  const int parts = gridDim.y > 1 && k_pool != nullptr ? gridDim.y - 1 : gridDim.y, part = blockIdx.y;
+  const bool has_q = part < parts, has_kv = k_pool != nullptr && part == (int)gridDim.y - 1;
   float fq = 1.f, fk = 1.f, sq = 0.f, sk = 0.f;
-  if (q_norm_w != nullptr)
+  if (has_q && q_norm_w != nullptr)
     in_rounds(nq, tid, value, [&](int, float v) { sq = fmaf(v, v, sq); });
-  if (k_norm_w != nullptr)
+  if (has_kv && k_norm_w != nullptr)
     in_rounds(nk, tid, [&](int i) { return value(nq + i); }, [&](int, float v) { sk = fmaf(v, v, sk); });
-  if (q_norm_w != nullptr) fq = 1.0f / sqrtf(block_sum(sq, red) / (float)nq + eps);
-  if (k_norm_w != nullptr) fk = 1.0f / sqrtf(block_sum(sk, red) / (float)nk + eps);
+  if (has_q && q_norm_w != nullptr) fq = 1.0f / sqrtf(block_sum(sq, red) / (float)nq + eps);
+  if (has_kv && k_norm_w != nullptr) fk = 1.0f / sqrtf(block_sum(sk, red) / (float)nk + eps);
   if (temp_coef != 0.f) fq *= 1.0f + temp_coef * logf((float)((pos + 1) / temp_every + 1));
-  in_rounds(H * D, tid, [&](int i) {
-    const int at = i / D * d + min(i % D, d - 1);
+  const int share = (H * D + parts - 1) / parts, q0 = part * share;
+  if (has_q) in_rounds(min(share, H * D - q0), tid, [&](int j) {
+    const int i = q0 + j, at = i / D * d + min(i % D, d - 1);
     return Two{value(at), q_norm_w ? q_norm_w[at] : 1.f};
-  }, [&](int i, Two v) {
+  }, [&](int j, Two v) {
+    const int i = q0 + j;
     from_f32(q_out + (size_t)t * H * D + i, i % D < d ? v.a * fq * v.b : 0.f);
   });
-  if (k_pool == nullptr) return;
+  if (!has_kv) return;
   const int slot = pos % ps;
   struct Kv { float k, w, v; };
   in_rounds(G * D, tid, [&](int i) {
@@ -90,13 +106,14 @@ extern "C" int kappai_projection_norm_store(
   if (T <= 0) return 0;
   if (H < 1 || G < 1 || d < 1 || dv < 1 || D < d || D < dv || ps < 1 || temp_every < 1)
     return (int)hipErrorInvalidValue;
+  const dim3 grid(T, few_rows_blocks(T, H * D) + (T <= FEW_ROWS && k_pool ? 1 : 0));
   if (is_bf16)
-    hipLaunchKernelGGL(projection_norm_store_kernel<bf16_t>, dim3(T), dim3(AP_THREADS), 0, stream,
+    hipLaunchKernelGGL(projection_norm_store_kernel<bf16_t>, grid, dim3(AP_THREADS), 0, stream,
                        (const bf16_t*)proj, stride, q_norm_w, k_norm_w, eps, temp_coef, temp_every,
                        (bf16_t*)k_pool, (bf16_t*)v_pool, row_pos, row_seg, block_tables,
                        max_blocks, H, G, d, dv, D, ps, (bf16_t*)q_out);
   else
-    hipLaunchKernelGGL(projection_norm_store_kernel<float>, dim3(T), dim3(AP_THREADS), 0, stream,
+    hipLaunchKernelGGL(projection_norm_store_kernel<float>, grid, dim3(AP_THREADS), 0, stream,
                        (const float*)proj, stride, q_norm_w, k_norm_w, eps, temp_coef, temp_every,
                        (float*)k_pool, (float*)v_pool, row_pos, row_seg, block_tables, max_blocks,
                        H, G, d, dv, D, ps, (float*)q_out);
@@ -106,16 +123,18 @@ extern "C" int kappai_projection_norm_store(
 // ---------------------------------------------------------------------------------------
 // rot_mode 1: pairs (j, j + rot_dims / 2); 2: pairs (2j, 2j + 1).  cos / sin [positions,
 // rot_dims / 2].  Only the first rot_dims of the rot places turn; the rest pass as they are.
-__device__ __forceinline__ float rotated(const float* x, int e, int rot_dims, int rot_mode,
+template <typename X>
+__device__ __forceinline__ float rotated(const X* x, int e, int rot_dims, int rot_mode,
                                          const float* ct, const float* st) {
-  if (e >= rot_dims || rot_mode == 0) return x[e];
+  if (e >= rot_dims || rot_mode == 0) return to_f32(x[e]);
   const int half = rot_dims / 2;
   int j, partner;
   bool first;
   if (rot_mode == 1) { first = e < half; j = first ? e : e - half; partner = first ? e + half : e - half; }
   else { first = (e & 1) == 0; j = e / 2; partner = e ^ 1; }
   const float c = ct[j], s = st[j];
-  return first ? x[e] * c - x[partner] * s : x[e] * c + x[partner] * s;
+  const float a = to_f32(x[e]), b = to_f32(x[partner]);
+  return first ? a * c - b * s : a * c + b * s;
 }
 
 template <typename T>
@@ -134,25 +153,37 @@ __global__ __launch_bounds__(AP_THREADS) void latent_store_kernel(
   const T* qr = q + (size_t)t * q_stride;
   const float* ct = cos_tab + (size_t)pos * (rot_dims / 2);
   const float* st = sin_tab + (size_t)pos * (rot_dims / 2);
+  // one block: everything; several: the last has the latent, the others a part of the queries' places each,
+  // which they turn from memory
+  if (gridDim.y > 1 && blockIdx.y < gridDim.y - (k_pool != nullptr ? 1 : 0)) {
+    for (int i = blockIdx.y * AP_THREADS + tid; i < H * (D - r); i += gridDim.y * AP_THREADS) {
+      const int h = i / (D - r), e = i % (D - r);
+      from_f32(q_out + (size_t)t * H * D + (size_t)h * D + r + e,
+               e < rot ? rotated(qr + h * (d + rot) + d, e, rot_dims, rot_mode, ct, st) : 0.f);
+    }
+    return;
+  }
+  const int heads = gridDim.y > 1 ? 0 : H;           // queries' heads of this block
   float ss = 0.f;
   for (int e = tid; e < r; e += AP_THREADS) { const float v = to_f32(kvr[e]); ss = fmaf(v, v, ss); }
-  for (int i = tid; i < (H + 1) * rot; i += AP_THREADS) {
+  for (int i = tid; i < (heads + 1) * rot; i += AP_THREADS) {
     const int h = i / rot, e = i % rot;
-    sh[i] = h < H ? to_f32(qr[h * (d + rot) + d + e]) : to_f32(kvr[r + e]);
+    sh[i] = h < heads ? to_f32(qr[h * (d + rot) + d + e]) : to_f32(kvr[r + e]);
   }
+  const size_t page =
+      k_pool == nullptr ? 0 : (size_t)block_tables[(size_t)row_seg[t] * max_blocks + pos / ps];
   const float inv = 1.0f / sqrtf(block_sum(ss, red) / (float)r + eps);      // (barrier inside)
-  for (int i = tid; i < H * (D - r); i += AP_THREADS) {
+  for (int i = tid; i < heads * (D - r); i += AP_THREADS) {
     const int h = i / (D - r), e = i % (D - r);
     const float v = e < rot ? rotated(sh + h * rot, e, rot_dims, rot_mode, ct, st) : 0.f;
     from_f32(q_out + (size_t)t * H * D + (size_t)h * D + r + e, v);
   }
   if (k_pool == nullptr) return;
-  const size_t page = (size_t)block_tables[(size_t)row_seg[t] * max_blocks + pos / ps];
   const int slot = pos % ps;
   for (int e = tid; e < D; e += AP_THREADS) {
     float kvv = 0.f, vv = 0.f;
     if (e < r) kvv = vv = to_f32(kvr[e]) * inv * c_norm_w[e];
-    else if (e < r + rot) kvv = rotated(sh + H * rot, e - r, rot_dims, rot_mode, ct, st);
+    else if (e < r + rot) kvv = rotated(sh + heads * rot, e - r, rot_dims, rot_mode, ct, st);
     from_f32(k_pool + (page * ps + slot) * D + e, kvv);
     from_f32(v_pool + (page * D + e) * ps + slot, vv);
   }
@@ -171,14 +202,15 @@ extern "C" int kappai_latent_store(const void* q, int q_stride, const void* kv, 
     return (int)hipErrorInvalidValue;
   const size_t lds = (size_t)(H + 1) * (rot > 0 ? rot : 1) * sizeof(float);
   if (lds > 48 * 1024) return (int)hipErrorInvalidValue;
+  const dim3 grid(T, few_rows_blocks(T, H * (D - r)) + (T <= FEW_ROWS && k_pool && D > r ? 1 : 0));
   if (is_bf16)
-    hipLaunchKernelGGL(latent_store_kernel<bf16_t>, dim3(T), dim3(AP_THREADS), lds, stream,
+    hipLaunchKernelGGL(latent_store_kernel<bf16_t>, grid, dim3(AP_THREADS), lds, stream,
                        (const bf16_t*)q, q_stride, (const bf16_t*)kv, kv_stride, c_norm_w, eps,
                        cos_tab, sin_tab, rot_dims, rot_mode, (bf16_t*)k_pool, (bf16_t*)v_pool,
                        row_pos, row_seg, block_tables, max_blocks, H, d, rot, r, D, ps,
                        (bf16_t*)q_out);
   else
-    hipLaunchKernelGGL(latent_store_kernel<float>, dim3(T), dim3(AP_THREADS), lds, stream,
+    hipLaunchKernelGGL(latent_store_kernel<float>, grid, dim3(AP_THREADS), lds, stream,
                        (const float*)q, q_stride, (const float*)kv, kv_stride, c_norm_w, eps,
                        cos_tab, sin_tab, rot_dims, rot_mode, (float*)k_pool, (float*)v_pool,
                        row_pos, row_seg, block_tables, max_blocks, H, d, rot, r, D, ps,
@@ -439,14 +471,19 @@ __global__ __launch_bounds__(AP_THREADS) void rotate_widen_store_kernel(
     const float y = to_f32(head[partner]), c = ct[j], s = st[j];
     return first ? x * c - y * s : x * c + y * s;
   };
-  for (int i = tid; i < H * D; i += AP_THREADS) {
+  const int first_item = blockIdx.y * AP_THREADS + tid, stride_items = gridDim.y * AP_THREADS;
+  for (int i = first_item; i < H * D; i += stride_items) {
     const int h = i / D, e = i % D;
     from_f32(q_out + (size_t)t * H * D + i, e < d ? turned(row + h * d, e) : 0.f);
   }
   if (k_pool == nullptr) return;
+  // (items in one list, the queries' first: a block behind them has keys and values only)
+  int i = first_item;
+  if (i < H * D) i += (H * D - i + stride_items - 1) / stride_items * stride_items;
+  if (i >= (H + G) * D) return;
   const size_t page = (size_t)block_tables[(size_t)row_seg[t] * max_blocks + pos / ps];
   const int slot = pos % ps;
-  for (int i = tid; i < G * D; i += AP_THREADS) {
+  for (i -= H * D; i < G * D; i += stride_items) {
     const int g = i / D, e = i % D;
     const T* khead = row + nq + g * d;
     float vv = 0.f;
@@ -467,13 +504,14 @@ extern "C" int kappai_rotate_widen_store(
       (values_are_keys && dv != d) || (rot_mode && rot_dims && (!cos_tab || !sin_tab)))
     return (int)hipErrorInvalidValue;
   if (rot_dims == 0) rot_mode = 0;
+  const dim3 grid(T, few_rows_blocks(T, (H + (k_pool ? G : 0)) * D));
   if (is_bf16)
-    hipLaunchKernelGGL(rotate_widen_store_kernel<bf16_t>, dim3(T), dim3(AP_THREADS), 0, stream,
+    hipLaunchKernelGGL(rotate_widen_store_kernel<bf16_t>, grid, dim3(AP_THREADS), 0, stream,
                        (const bf16_t*)proj, stride, cos_tab, sin_tab, rot_dims, rot_mode,
                        values_are_keys, (bf16_t*)k_pool, (bf16_t*)v_pool, row_pos, row_seg,
                        block_tables, max_blocks, H, G, d, dv, D, ps, (bf16_t*)q_out);
   else
-    hipLaunchKernelGGL(rotate_widen_store_kernel<float>, dim3(T), dim3(AP_THREADS), 0, stream,
+    hipLaunchKernelGGL(rotate_widen_store_kernel<float>, grid, dim3(AP_THREADS), 0, stream,
                        (const float*)proj, stride, cos_tab, sin_tab, rot_dims, rot_mode,
                        values_are_keys, (float*)k_pool, (float*)v_pool, row_pos, row_seg,
                        block_tables, max_blocks, H, G, d, dv, D, ps, (float*)q_out);

@@ -51,3 +51,23 @@ def test_a_norm_on_two_terms(ops, T, D, a, b):  # noqa: F811
     rows = ops.output_norm_add(one, ya, w, 1e-5, rows_dtype=BF16, scale_a=0.5, b=yb, scale_b=0.25)
     want = ops.output_norm_add(two, fa, w, 1e-5, rows_dtype=BF16, scale_a=0.5, b=fb, scale_b=0.25)
     assert torch.equal(rows, want) and torch.equal(one, two)
+
+
+@pytest.mark.parametrize("D", [1, 255, 1024, 1025, 2048])
+@pytest.mark.parametrize("a,b", [(F32, BF16), (BF16, F32), (F32, F32)])
+@pytest.mark.parametrize("normed", [False, True])
+def test_two_sides_as_the_kernel_for_any_row(ops, D, a, b, normed):  # noqa: F811
+    """Up to four planes with everything asked for at once, against the same planes and zeros as a fifth."""
+    T, planes = 3, 4
+    x = [rand((planes, T, D) if t == F32 else (T, D), t, 12 + i).to(DEV) for i, t in enumerate((a, b))]
+    more = [torch.cat([y, torch.zeros_like(y[:1])]) if y.dim() == 3 else y for y in x]
+    ws = [rand((D,), F32, 14 + i).to(DEV) if normed else None for i in range(2)]
+    got, want = (ops.pair_norm_sum(*s, 0.5, 0.75, *ws, 1e-5) for s in (x, more))
+    assert torch.equal(got, want)
+    norm_w, resid = rand((D,), F32, 16).to(DEV), rand((T, D), F32, 17).to(DEV)
+    out = []
+    for s in (x, more):
+        stream = resid.clone()
+        y = ops.pair_norm_sum(*s, 0.5, 0.75, *ws, 1e-5, add_into=ops.AddInto(stream, norm_w, 1e-5))
+        out.append((stream, y.data, y.ss[0, :T]))
+    assert all(torch.equal(p, q) for p, q in zip(*out))

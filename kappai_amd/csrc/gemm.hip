@@ -2244,14 +2244,22 @@ void gemm_bf16_skinny_kernel(
 // two halves meet the one fragment of W in two matrix instructions, whose valid halves are added
 // at the end.  Twice as many blocks stream W as with 16 columns a block, and K needs no split
 // over blocks, so the residual sum can be made here, in a fixed order.
-template <int NW, bool FRAG>
+// ROWS8 (up to 8 rows, FRAG): the rows of A of the two halves share a fragment as well, row r of the first half in
+// place r, of the second in place r + 8, so that one instruction makes both halves' sums (the tile's two quarters
+// on its diagonal; the same sums in the same order) from one load of A where there were two.  A load takes its
+// clocks at the CU's door whether its lanes need anything or not, and these blocks have the CU to themselves: one row
+// of 1024 x 4608 7.0 -> 6.5 us.  In the form with 16 waves: with 8, whose waves have two to four steps, there is no
+// line of loads to wait in (1024 x 1024: 23 us more over 256 products).
+template <int NW, bool FRAG, bool ROWS8>
 __global__ __launch_bounds__(NW * WAVE) void gemm_bf16_into_resid_kernel(
     const bf16_t* __restrict__ A, const bf16_t* __restrict__ W, float* __restrict__ resid, int M, int N,
     int K, int lda, int frags, int ldr, const float* __restrict__ norm_w, const float* __restrict__ bias,
     bf16_t* __restrict__ rows, float* __restrict__ ss, int rows_frag, int spare) {
   // frags: the rows' order, and where not FRAG as the second bit that of W; spare: see above
   const int a_frag = FRAG ? frags : frags & 1, w_frag = FRAG ? 1 : frags & 2;
-  __shared__ f32x4_t red[NW][2][WAVE];
+  static_assert(FRAG || !ROWS8, "");
+  constexpr int HI = ROWS8 ? 0 : 1, ACROSS = ROWS8 ? 40 : 8;   // where a lane's columns 8 further are, and whose
+  __shared__ f32x4_t red[NW][1 + HI][WAVE];
   const int tid = threadIdx.x;
   const int lane = tid % WAVE, wave = __builtin_amdgcn_readfirstlane(tid / WAVE);
   const int col = lane % 16, kg = (lane / 16) * 8;
@@ -2310,21 +2318,27 @@ __global__ __launch_bounds__(NW * WAVE) void gemm_bf16_into_resid_kernel(
         ((lane / 16) * 16 + blockIdx.x % 2 * 8 + col % 8) * 16u + (half ? (uint32_t)khalf * 32u : 0u);
     const __amdgpu_buffer_rsrc_t abuf = raw_buffer(A + (size_t)k0 * (a_frag ? 16 : 1), OUT);
     const uint32_t astep = a_frag ? 1024u : 64u, second = (uint32_t)khalf * (a_frag ? 32u : 2u);
-    const uint32_t aoff = col >= M ? OUT : a_frag ? (uint32_t)lane * 16u : (uint32_t)col * lda * 2u + kg * 2u;
+    const uint32_t aoff =
+        ROWS8 ? (col % 8 >= M ? OUT
+                              : (a_frag ? (uint32_t)(lane - half * 8) * 16u : (uint32_t)(col % 8) * lda * 2u + kg * 2u) +
+                                    (half ? second : 0u))
+              : col >= M ? OUT : a_frag ? (uint32_t)lane * 16u : (uint32_t)col * lda * 2u + kg * 2u;
     const auto run = [&](auto count, int from) {
       constexpr int S = decltype(count)::value;
-      u32x4_t wv[S], a0[S], a1[S];
+      u32x4_t wv[S], a0[S], a1[ROWS8 ? 1 : S];
 #pragma unroll
       for (int u = 0; u < S; ++u) {
         wv[u] = __builtin_amdgcn_raw_buffer_load_b128(wbuf, woff, (from + u) * 1024, 0);
         a0[u] = __builtin_amdgcn_raw_buffer_load_b128(abuf, aoff, (from + u) * astep, 0);
-        a1[u] = __builtin_amdgcn_raw_buffer_load_b128(abuf, aoff, (from + u) * astep + second, 0);
+        if constexpr (!ROWS8)
+          a1[u] = __builtin_amdgcn_raw_buffer_load_b128(abuf, aoff, (from + u) * astep + second, 0);
       }
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
       for (int u = 0; u < S; ++u) {
         acc0 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(a0[u]), as_bf16x8(wv[u]), acc0, 0, 0, 0);
-        acc1 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(a1[u]), as_bf16x8(wv[u]), acc1, 0, 0, 0);
+        if constexpr (!ROWS8)
+          acc1 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(a1[u]), as_bf16x8(wv[u]), acc1, 0, 0, 0);
       }
     };
     int s = 0;
@@ -2359,14 +2373,14 @@ __global__ __launch_bounds__(NW * WAVE) void gemm_bf16_into_resid_kernel(
     }
   }
   red[wave][0][lane] = acc0;
-  red[wave][1][lane] = acc1;
+  if constexpr (!ROWS8) red[wave][HI][lane] = acc1;
   __syncthreads();
   if (wave != 0) return;
-  f32x4_t lo = red[0][0][lane], hi = red[0][1][lane ^ 8];
+  f32x4_t lo = red[0][0][lane], hi = red[0][HI][lane ^ ACROSS];
 #pragma unroll 4
   for (int w = 1; w < NW; ++w) {
     lo += red[w][0][lane];
-    hi += red[w][1][lane ^ 8];
+    hi += red[w][HI][lane ^ ACROSS];
   }
   // columns 0-7: the first half's sums of this lane and the second half's of the lane 8 further
   const bool mine = half == 0 && gn < N;
@@ -2407,12 +2421,16 @@ static void launch_into_resid(const bf16_t* A, const bf16_t* W, const float* bia
                       (size_t)K * 32 < 0x7FFFFF00u && ((size_t)(M - 1) * ro.ldr + N) * 4 < 0x7FFFFF00u;
 #define INTO_RESID(NW)                                                                                 \
   do {                                                                                                 \
-    if (pieces)                                                                                        \
-      hipLaunchKernelGGL((gemm_bf16_into_resid_kernel<NW, true>), grid, dim3(NW * WAVE), 0, stream, A, \
-                         W, ro.resid, M, N, K, lda, frags, ro.ldr, ro.norm_w, bias, ro.rows, ro.ss,    \
-                         ro.rows_frag, 0);                                                             \
+    if (pieces && M <= 8)                                                                              \
+      hipLaunchKernelGGL((gemm_bf16_into_resid_kernel<NW, true, NW == 16>), grid, dim3(NW * WAVE), 0,  \
+                         stream, A, W, ro.resid, M, N, K, lda, frags, ro.ldr, ro.norm_w, bias,         \
+                         ro.rows, ro.ss, ro.rows_frag, 0);                                             \
+    else if (pieces)                                                                                   \
+      hipLaunchKernelGGL((gemm_bf16_into_resid_kernel<NW, true, false>), grid, dim3(NW * WAVE), 0,     \
+                         stream, A, W, ro.resid, M, N, K, lda, frags, ro.ldr, ro.norm_w, bias,         \
+                         ro.rows, ro.ss, ro.rows_frag, 0);                                             \
     else                                                                                               \
-      hipLaunchKernelGGL((gemm_bf16_into_resid_kernel<NW, false>), grid, dim3(NW * WAVE), 0, stream,   \
+      hipLaunchKernelGGL((gemm_bf16_into_resid_kernel<NW, false, false>), grid, dim3(NW * WAVE), 0, stream,   \
                          A, W, ro.resid, M, N, K, lda, frags | w_order, ro.ldr, ro.norm_w, bias,       \
                          ro.rows, ro.ss, ro.rows_frag, 0);                                             \
   } while (0)

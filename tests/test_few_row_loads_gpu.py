@@ -209,3 +209,20 @@ def test_rows_of_x_more_than_two_gibibytes_apart():
         for got, want in zip(results(far), results(x)):
             assert torch.equal(got, want)
         del far
+
+
+@pytest.mark.parametrize("K,N", [(64, 32), (1024, 1024), (2304, 48), (4096, 16), (4608, 1024), (10752, 64)])
+def test_into_the_stream_halves_of_k_share_a_fragment_up_to_8_rows(K, N):
+    """Nine rows take two fragments of x for one of W, eight one: the same bits."""
+    g = _gen(K, N, 18)
+    x = _rows(9, K, g)
+    W, _ = _matrix(N, K, g)
+    norm, resid = torch.rand(N, generator=g, device=DEV) + 0.5, torch.randn(9, N, generator=g, device=DEV)
+    out = []
+    for rows in (9, 8, 3, 1):
+        stream = resid[:rows].clone()
+        got = ops.linear(x[:rows], W, add_into=ops.AddInto(stream, norm, 1e-5))
+        out.append((stream, got.ss[:, :rows]))
+    for stream, ss in out[1:]:
+        n = stream.shape[0]
+        assert torch.equal(stream, out[0][0][:n]) and torch.equal(ss, out[0][1][:, :n])

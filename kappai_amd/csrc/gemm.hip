@@ -1557,8 +1557,14 @@ void gemm_bf16_direct_kernel(const bf16_t* __restrict__ A, const bf16_t* __restr
 // buffers), W from memory: gate/up 16384 x 2048 of 417 rows 31.2 us against 36.8, 9216 x 1024 of 575 rows
 // 14.3 against 18.7; 3072 x 1024 of 575 rows 9.7 against 12.1; 2048 x 2048 of 417 rows in four ranges 9.6
 // against 12.2, 2048 x 8192 in four 21.2 against 24.0; 3072 x 2048 of 2048 rows 27.6 against 32.3.
+// Products that leave CUs without a block of 128 x 128 take 64 x 128, 128 x 64 or 64 x 64 (a wave's tile 32 rows or
+// columns, six and five buffers): more CUs take in less each.  128 x 128 and the best of the three, us: 3072 x 1024
+// of 575 rows 9.0 and 7.4 (216 blocks), 3072 x 2048 of 417 rows 15.4 and 11.6 (192), 1024 x 1024 of 575 rows 8.5 and
+// 5.4 (144), 1024 x 4608 of 417 rows in two ranges 15.2 and 8.9 (224).  Of more blocks than CUs they are slower (2048 x
+// 1024 of 1040 rows 9.3 and 10.6), with three buffers and two blocks a CU too (10.7).
 template <typename TO, int EPI, int WTM, int WTN, int NB>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1)))
+__global__ __launch_bounds__(256)
+    __attribute__((amdgpu_waves_per_eu(1, NB * (WTM + WTN) * 8192 <= 80 * 1024 ? 2 : 1)))   // (as LDS has room for)
 void gemm_bf16_staged_kernel(const bf16_t* __restrict__ A, const bf16_t* __restrict__ W,
                              const float* __restrict__ bias, TO* __restrict__ C, int M, int N,
                              int K, int lda, int ldc, int tiles_m, int tiles_n, uint32_t cut) {
@@ -1640,7 +1646,7 @@ void gemm_bf16_staged_kernel(const bf16_t* __restrict__ A, const bf16_t* __restr
   ORDER_FENCE();
 #pragma unroll
   for (int n = 0; n < NREAD; ++n) read(0, 0, 0, n);
-  constexpr int PRE = NPROD > 4 ? 2 : 1;
+  constexpr int PRE = NPROD > 4 ? 2 : NPROD > 1 ? 1 : 0;
   constexpr int LOADS_AT = 3 * NPROD;                       // slots of the first three 16s of K
   int cur = 0, kt = 0;
   do {
@@ -1656,11 +1662,14 @@ void gemm_bf16_staged_kernel(const bf16_t* __restrict__ A, const bf16_t* __restr
           SCHED_FENCE();
         }
         if (s < 3) {
-          if (t < NREAD) read((s + 1) & 1, cur, s + 1, t);
+          constexpr int AT_ONCE = (NREAD + NPROD - 1) / NPROD;
+#pragma unroll
+          for (int q = 0; q < AT_ONCE; ++q)
+            if (t * AT_ONCE + q < NREAD) read((s + 1) & 1, cur, s + 1, t * AT_ONCE + q);
           const int slot = s * NPROD + t;
           // NLOAD loads spread over the slots
-          if ((slot + 1) * NLOAD / LOADS_AT > slot * NLOAD / LOADS_AT)
-            load(into, kt + NB - 1, slot * NLOAD / LOADS_AT);
+#pragma unroll
+          for (int i = slot * NLOAD / LOADS_AT; i < (slot + 1) * NLOAD / LOADS_AT; ++i) load(into, kt + NB - 1, i);
         } else if (t >= PRE) {
           constexpr int PER = (NREAD + NPROD - PRE - 1) / (NPROD - PRE);
 #pragma unroll
@@ -1741,8 +1750,8 @@ static void launch_fragment_block(const bf16_t* A, const bf16_t* Wf, const float
 // blocks of the same kernel (tiles of 64 of K), 5 = the 256x256 kernel with one wave a SIMD, 6 = its
 // 128x128 form (when the sizes fit them, else 3), 8 = the 128x128 form with four LDS buffers, one
 // block a CU, 9 = the one-wave-a-SIMD kernel with blocks of 256 rows x 192 columns, 11 = 192x128, 12 =
-// 256x128 (both only with W in fragment order, else 6).  With W in fragment order 6 and 8 are one kernel, one
-// block a CU with four buffers.
+// 256x128, 13 = 64x128, 14 = 128x64, 15 = 64x64 (11 to 15 only with W in fragment order, else 6).  With W in
+// fragment order 6 and 8 are one kernel, one block a CU with four buffers.
 template <typename TO, int EPI>
 static void launch_tile(const bf16_t* A, const bf16_t* W, const float* bias, TO* C, int M,
                         int n_rows_w, int K, int lda, int ldc, int ksplit, int shape,
@@ -1761,13 +1770,16 @@ static void launch_tile(const bf16_t* A, const bf16_t* W, const float* bias, TO*
       if (shape == 5) KAPPAI_BLOCKS(4, 4, 4);
       else if (shape == 11) KAPPAI_BLOCKS(3, 2, 3);
       else if (shape == 12) KAPPAI_BLOCKS(4, 2, 3);
+      else if (shape == 13) KAPPAI_BLOCKS(1, 2, 6);
+      else if (shape == 14) KAPPAI_BLOCKS(2, 1, 6);
+      else if (shape == 15) KAPPAI_BLOCKS(1, 1, 5);
       else if (shape != 9) KAPPAI_BLOCKS(2, 2, 4);
       else if constexpr (EPI == 0) KAPPAI_BLOCKS(4, 3, 4);
 #undef KAPPAI_BLOCKS
       return;
     }
   }
-  if (shape == 11 || shape == 12) shape = 6;
+  if (shape >= 11 && shape <= 15) shape = 6;
   if (shape == 0) {
     const int big = ((M + 255) / 256) * ((n_rows_w + 127) / 128) * ksplit;
     const int blocks256 = ((M + 255) / 256) * ((n_rows_w + 255) / 256) * ksplit;
@@ -3056,8 +3068,8 @@ static int launch_bf16(const bf16_t* A, const bf16_t* W, const float* bias, TO* 
 // force_kernel: 0 = by M, 1 = tile kernel, 2 = skinny kernel (M <= 64 only), 3..8 = tile kernel
 // with block shape 1..6 (see launch_tile), 9 = shared-rows kernel (17 to 64 rows, K / ksplit a
 // multiple of 512), 10 = block shape 8, 11 = block shape 9, 12 = the kernel for 25 to 128 rows
-// (1 to 128 rows, W in fragment order, K / ksplit a multiple of 256), 13 and 14 = block shapes 11 and
-// 12; for tests and tuning.
+// (1 to 128 rows, W in fragment order, K / ksplit a multiple of 256), 13 to 17 = block shapes 11 to
+// 15; for tests and tuning.
 // ksplit > 1 (float output only): C is [ksplit][M][ldc] partial sums over K ranges.
 // W_frag: null, or W in fragment order (K a multiple of 32, rows a multiple of 16); W may then
 // be null: every kernel reads the fragment order (only kappai_gemm_bf16_any needs rows).

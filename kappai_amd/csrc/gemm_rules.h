@@ -20,22 +20,31 @@
 // form that the model likes best takes 0.6 % more than the fastest of the five in sum; a fifth of the products
 // each are best in the first, fourth and fifth, two fifths in the third.  Over 366 others, measured later on
 // another card: errors of 6 to 10 %, and 0.6 % again.
+// The last three are for products of at most a block a CU (beyond, a larger block is the faster: 2048 x 1024 of
+// 1040 rows 9.3 us in 128 x 128 and 10.7 in 64 x 128) and for ranges of up to 2,048 of K, 1,536 where the sums are
+// float planes (2048 x 8192 of 417 rows 21.8 us with the norm's share in four ranges of 128 x 128, 23.0 in two of
+// 128 x 64).  Fitted to 185 products of 160 to 1,040 rows on a card that is 4 % slower than the model, good to 4 to
+// 8 %.  Over 240 products, ranges among them, the form that the model likes best takes 0.2 % more than the fastest
+// of the six up to 256 x 128; without these three 17 % more.
 struct kappai_block_form {
   int shape, rows, cols;           // (shape: gemm.hip, launch_tile)
   double tile, fill, round, mb, start;
 };
-static const kappai_block_form KAPPAI_BLOCK_FORMS[5] = {
+static const kappai_block_form KAPPAI_BLOCK_FORMS[8] = {
     {5, 256, 256, 0.95, 0.40, 6.0, 0.112, 2.9},  {9, 256, 192, 0.81, 0.30, 5.5, 0.111, 3.0},
     {12, 256, 128, 0.51, 0.25, 1.9, 0.158, 3.2}, {11, 192, 128, 0.42, 0.22, 0.7, 0.198, 3.2},
-    {8, 128, 128, 0.32, 0.18, 0.1, 0.244, 3.1}};
+    {8, 128, 128, 0.32, 0.18, 0.1, 0.244, 3.1},  {13, 64, 128, 0.180, 0.131, 0.0, 0.095, 3.7},
+    {14, 128, 64, 0.196, 0.062, 0.0, 0.151, 3.7}, {15, 64, 64, 0.147, 0.036, 0.0, 0.165, 2.8}};
 // The shape of the blocks for M rows, N rows of W, K in `split` ranges; `time`: what the model says.
 static inline int kappai_block_shape(int M, int N, int K, int split, double result_mb, bool gated,
                                      double* time) {
   int best = 8;
   double best_t = -1.0;
+  const int longest = result_mb > 3e-6 * M * N * split ? 1536 : 2048;
   for (const kappai_block_form& f : KAPPAI_BLOCK_FORMS) {
     if (gated && f.shape == 9) continue;       // (its waves' columns are no whole pairs of 64)
     const double blocks = (double)((M + f.rows - 1) / f.rows) * ((N + f.cols - 1) / f.cols) * split;
+    if (f.rows * f.cols < 128 * 128 && (blocks > 256 || K / split > longest)) continue;
     const double rounds = (double)(((long)blocks + 255) / 256), tiles = (double)K / split / 64.0;
     const double t = tiles * (f.tile * rounds + f.fill * blocks / 256) + f.round * rounds +
                      f.mb * result_mb + f.start;

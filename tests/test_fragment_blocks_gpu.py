@@ -1,5 +1,5 @@
 """The block products over a matrix in fragment order (256 x 256 and 256 x 192 blocks with W's pieces in
-registers, 256 x 128, 192 x 128 and 128 x 128 with both operands in LDS), at sizes that end inside a block
+registers, 256 x 128 down to 64 x 64 with both operands in LDS), at sizes that end inside a block
 and at the shortest runs of K, against the same product over the matrix's rows (bit for bit: every form adds
 16 of K after 16) and against float64."""
 import ctypes
@@ -10,7 +10,7 @@ import torch
 from test_kernels_gpu import BF16, DEV, F32, close, ops, rand  # noqa: F401
 
 pytestmark = pytest.mark.gpu
-FORMS = {"256x256": 7, "256x192": 11, "256x128": 14, "192x128": 13, "128x128": 10}
+FORMS = {"256x256": 7, "256x192": 11, "256x128": 14, "192x128": 13, "128x128": 10, "64x128": 15, "128x64": 16, "64x64": 17}
 ROWS = 8                       # the kernel for rows, 128 x 128 blocks
 
 
@@ -45,9 +45,10 @@ def test_gated_blocks_over_fragment_order(ops, M, F, K, form):  # noqa: F811
 
 
 # the rule's own choices, one product for every form (by its model: 256 x 256, 256 x 192, 256 x 128,
-# 192 x 128, 128 x 128)
+# 192 x 128, 128 x 128; then 64 x 128, 128 x 64, 64 x 64 in as many blocks as CUs and in a row more)
 @pytest.mark.parametrize("M,N,K", [(2048, 16384, 512), (2048, 6144, 640), (512, 16384, 512),
-                                   (575, 9216, 512), (300, 1024, 256)])
+                                   (575, 9216, 512), (300, 1024, 256), (575, 3072, 1024),
+                                   (417, 3072, 2048), (256, 4096, 1024), (257, 4096, 1024)])
 def test_the_rule_takes_every_form(ops, M, N, K):  # noqa: F811
     x, w = rand((M, K), BF16, 87).to(DEV), rand((N, K), BF16, 88).to(DEV)
     assert torch.equal(ops.linear(x, ops.InFragments.of(w)), ops.linear(x, w, force_kernel=ROWS))

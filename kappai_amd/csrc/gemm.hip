@@ -182,9 +182,11 @@ __device__ __forceinline__ void f32_normed_rows(const float* __restrict__ x, con
 // block owns COLS rows of W, a wave one or several runs of K, and the waves meet in LDS.  COLS = 16: a
 // wave walks its RUNS / 8 runs one after the other.  COLS = 8 (up to 8 rows; matrices of few rows, so
 // that twice the blocks stream them): places 0-7 of both operands hold the wave's first run and 8-15
-// its second, and the product's two diagonal quarters are the two runs' sums.  The next chunk's share
+// its second, and the product's two diagonal quarters are the two runs' sums.  COLS = 4 (up to 4 rows and 1,024
+// columns, a block for every CU): four runs and the four squares on the diagonal; three rows in a decode step, with
+// 8 and 4 columns a block: 1024 x 4608 11.0 and 9.0 us, 1024 x 1024 4.9 and 4.1.  The next chunk's share
 // of W is under way while a chunk is multiplied.  Three rows, W from memory: 9216 x 1024 12 us
-// (3.1 TB/s), 1024 x 4608 9 us, 65536 x 1024 51 us (5.3 TB/s); the vector kernel before took 100 to
+// (3.1 TB/s), 65536 x 1024 51 us (5.3 TB/s); the vector kernel before took 100 to
 // 1,500 us, a block a 64 x 64 tile of which three rows were real.
 //
 // GATED: W holds 2 N rows, gate rows and behind them the up rows; a block's 16 columns are the gates of 8
@@ -199,16 +201,16 @@ __device__ __forceinline__ void f32_normed_rows(const float* __restrict__ x, con
 // ONE: no run has more than a chunk (8 runs, K up to 1,024): nothing is under way beside the chunk, and with the
 // registers of three blocks a CU instead of two, 576 blocks of gate/up run at once (13.1 -> 12.7 us).
 template <int MT, int COLS, int RUNS, int LOADS, bool GATED = false, bool NORM = false, bool ONE = false>
-__global__ __launch_bounds__((COLS == 8 ? RUNS / 2 : 8) * WAVE) __attribute__((amdgpu_waves_per_eu(ONE ? 6 : 1)))
+__global__ __launch_bounds__((COLS < 16 ? RUNS * COLS / 16 : 8) * WAVE) __attribute__((amdgpu_waves_per_eu(ONE ? 6 : 1)))
 void gemm_f32_skinny_kernel(
     const float* __restrict__ A, const float* __restrict__ W, const float* __restrict__ bias,
     float* __restrict__ C, int M, int N, int K, int lda, int ldc, int add, const float* __restrict__ norm_w,
     float eps) {
-  constexpr bool SIDE = COLS == 8;               // two runs side by side
-  constexpr int NW = SIDE ? RUNS / 2 : 8;
+  constexpr bool SIDE = COLS < 16;               // two or four runs side by side
+  constexpr int NW = SIDE ? RUNS * COLS / 16 : 8, ROWS = SIDE ? COLS : 16;
   static_assert(!NORM || (MT == 1 && LOADS == F32_WHOLE), "few rows of whole chunks");
-  static_assert(!SIDE || MT == 1, "two runs side by side leave room for 8 rows");
-  __shared__ float red[RUNS][MT][SIDE ? 8 : 16][COLS];
+  static_assert(!SIDE || MT == 1, "runs side by side leave room for as many rows as columns");
+  __shared__ float red[RUNS][MT][ROWS][COLS];
   extern __shared__ __attribute__((aligned(16))) float f32_rows[];      // NORM: M rows
   const int wave = threadIdx.x / WAVE, lane = threadIdx.x % WAVE;
   const int r = lane % 16, q = lane / 16;
@@ -219,7 +221,7 @@ void gemm_f32_skinny_kernel(
   const float* a[MT];
 #pragma unroll
   for (int mt = 0; mt < MT; ++mt)
-    a[mt] = A + (size_t)min(mt * 16 + (SIDE ? r % 8 : r), M - 1) * lda;
+    a[mt] = A + (size_t)min(mt * 16 + r % ROWS, M - 1) * lda;
 
   const int chunks = (K + F32_CHUNK - 1) / F32_CHUNK;
   // this lane's chunks c0 .. c0 + len - 1; the wave takes `most` steps, a chunk each
@@ -228,12 +230,16 @@ void gemm_f32_skinny_kernel(
   int c0 = f32_run_start(run0, RUNS, chunks);
   int len = f32_run_start(run0 + per, RUNS, chunks) - c0, most = len;
   if (SIDE) {
-    const int mid = f32_run_start(run0 + 1, RUNS, chunks), second = c0 + len - mid;
-    len = mid - c0;
-    most = max(len, second);
-    if (r / 8) {
-      c0 = mid;
-      len = second;
+    most = 0;
+#pragma unroll
+    for (int i = 0, from = c0; i < per; ++i) {
+      const int to = f32_run_start(run0 + i + 1, RUNS, chunks);
+      most = max(most, to - from);
+      if (r / COLS == i) {
+        c0 = from;
+        len = to - from;
+      }
+      from = to;
     }
   }
   f32x4_t tot[MT], wv[F32_STEPS], av[MT][F32_STEPS];
@@ -245,7 +251,7 @@ void gemm_f32_skinny_kernel(
     for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
-        red[run][mt][(4 * q + i) % (SIDE ? 8 : 16)][r % COLS] = tot[mt][i];
+        red[run][mt][(4 * q + i) % ROWS][r % COLS] = tot[mt][i];
         tot[mt][i] = 0.f;
       }
     ++run;
@@ -255,7 +261,7 @@ void gemm_f32_skinny_kernel(
     load_chunk_f32<LOADS>(w, min(c0 + c, chunks - 1), q, K, v);
   };
   // (lanes without a row stay out: a masked load costs what its live lanes do)
-  const int live = SIDE ? r % 8 : r;
+  const int live = r % ROWS;
 #pragma unroll
   for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
@@ -286,7 +292,7 @@ void gemm_f32_skinny_kernel(
 #pragma unroll
         for (int mt = 0; mt < MT; ++mt) acc[mt] = mfma_f32(av[mt][j][e], wv[j][e], acc[mt]);
     }
-    // (side by side, a lane's results belong to the run that its column's half holds)
+    // (side by side, a lane's results belong to the run that its column's part holds)
     if (!SIDE || c < len)
 #pragma unroll
       for (int mt = 0; mt < MT; ++mt) tot[mt] += acc[mt];
@@ -294,7 +300,7 @@ void gemm_f32_skinny_kernel(
   // (the value that the thread's first result is added to)
   constexpr int OUT = GATED ? 8 : COLS;
   float old = 0.f;
-  if (add && threadIdx.x < MT * (SIDE ? 8 : 16) * OUT) {
+  if (add && threadIdx.x < MT * ROWS * OUT) {
     const int m = threadIdx.x / OUT, n = n0 + threadIdx.x % OUT;
     if (m < M && n < N) old = C[(size_t)m * ldc + n];
   }
@@ -323,8 +329,8 @@ void gemm_f32_skinny_kernel(
     multiply(c);
   }
   if (SIDE) {
-    run += r / 8;
-    if (r / 8 == q / 2) write_run();
+    run += r / COLS;
+    if (r / COLS == 4 * q / COLS) write_run();
   } else {
     while (run < run0 + per) write_run();
   }
@@ -335,7 +341,7 @@ void gemm_f32_skinny_kernel(
     for (int g = 1; g < RUNS; ++g) s += red[g][m / 16][m % 16][col];
     return s + (bias ? bias[row] : 0.f);
   };
-  for (int at = threadIdx.x; at < MT * (SIDE ? 8 : 16) * OUT; at += NW * WAVE) {
+  for (int at = threadIdx.x; at < MT * ROWS * OUT; at += NW * WAVE) {
     const int m = at / OUT, n = n0 + at % OUT;
     if (m >= M || n >= N) continue;
     const float s = whole(m, at % OUT, n);
@@ -640,9 +646,12 @@ static void launch_f32(const float* A, const float* W, const float* bias, float*
     const bool many = f32_runs((K + F32_CHUNK - 1) / F32_CHUNK) == 32, one = K <= 8 * F32_CHUNK;
 #define F32_SKINNY(MT, COLS, RUNS, ...)                                                           \
   hipLaunchKernelGGL((gemm_f32_skinny_kernel<MT, COLS, RUNS, LOADS, false, ##__VA_ARGS__>), dim3((N + COLS - 1) / COLS), \
-                     dim3((COLS == 8 ? RUNS / 2 : 8) * WAVE), 0, stream, A, W, bias, C, M, N, K,   \
+                     dim3((COLS < 16 ? RUNS * COLS / 16 : 8) * WAVE), 0, stream, A, W, bias, C, M, N, K,   \
                      lda, ldc, add, (const float*)nullptr, 0.f)
-    if (M <= 8 && N <= 256 * 8) {
+    if (M <= 4 && N <= 256 * 4) {
+      if (many) F32_SKINNY(1, 4, 32);
+      else F32_SKINNY(1, 4, 8);
+    } else if (M <= 8 && N <= 256 * 8) {
       if (many) F32_SKINNY(1, 8, 32);
       else F32_SKINNY(1, 8, 8);
     } else if (M <= 16) {

@@ -185,3 +185,13 @@ def test_blocks_over_operands_of_four_gibibytes_give_the_same_bits(ops, M, N, K)
     assert torch.equal(ops.linear(far, w), ops.linear(x, w))
     if ops.linear_swiglu_f32_takes(x, w):
         assert torch.equal(ops.linear_swiglu_f32(far, w), ops.linear_swiglu_f32(x, w))
+
+
+# up to 4 rows and 1,024 columns a block owns four columns and four runs stand side by side; both sides of either
+@pytest.mark.parametrize("N", [3, 1023, 1024, 1025])
+@pytest.mark.parametrize("K", [20, 130, 1024, 2181, 4608, 5000])
+def test_four_columns_a_block(ops, N, K):  # noqa: F811
+    x, w, b = (rand(shape, F32, 65 + i).to(DEV) for i, shape in enumerate([(9, K), (N, K), (N,)]))
+    whole = ops.linear(x, w, b)
+    for M in (1, 2, 3, 4, 5):
+        assert torch.equal(ops.linear(x[:M].contiguous(), w, b), whole[:M]), M

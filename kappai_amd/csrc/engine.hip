@@ -129,13 +129,15 @@ Ranges ranges_over_rows(int M, int N, int K) {
 // ... of a W in fragment order (its rows a multiple of 16: the model in gemm_rules.h).  The order W is kept in
 // decides the speed, not what the sums are rounded to: where the ranges of the kernels over rows leave float
 // sums, one range over fragment order does too.  2100 x 2048 x 8192 with the norm: 80.0 us so, 78.3 in
-// bfloat16, 98.4 in two ranges; 1600 x 1024 x 1024: 17.0, 15.5 and 17.0.
+// bfloat16, 98.4 in two ranges; 1600 x 1024 x 1024: 17.0, 15.5 and 17.0.  Up to 256 rows the kernels behind in_proj
+// and qkv add planes, and float sums come in two ranges or more as they did (160 rows, one and two ranges: 6144 x 2048
+// 12.5 and 12.2 us, 3072 x 2048 9.3 and 8.3, 2048 x 1024 5.2 and 4.5, 3072 x 1024 5.4 and 5.8).
 Ranges ranges_over_fragments(int M, int N, int K) {
   const bool f32 = ranges_over_rows(M, N, K).f32;
   Ranges best{1, f32};
   double best_t = -1.0;
   for (int split = 1; split < 9; ++split) {
-    if (!ranges_fit(K, split)) continue;
+    if (!ranges_fit(K, split) || (split == 1 && f32 && M <= 256 && ranges_fit(K, 2))) continue;
     const double mb = (split > 1 || f32 ? split : 0.5) * M * (double)N * 4e-6;
     double t;
     kappai_block_shape(M, N, K, split, mb, false, &t);

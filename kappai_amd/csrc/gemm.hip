@@ -2775,11 +2775,8 @@ static bool launch_shared_rows(const bf16_t* A, const bf16_t* W, const float* bi
 // pieces of the wave's 32 rows, 256 bytes of each of two groups of 8 of K.  The waves meet in LDS
 // at the end to add their K parts in a fixed order.  K can be cut over blocks as well (float
 // partial sums), which is what fills the chip for the products with few rows of W.
-// Measured at the LFM2-1.2B shapes, W cold, 128 rows: gate/up 23.2 against 26.7 us (the 128 x 128
-// block form), in_proj 13.0 against 14.1, qkv 9.1 against 12.4, out_proj 7.4 against 8.0, down
-// 15.5 against 20.6; 64 rows against the kernel for 17 to 64 rows: gate/up 18.4 against 20.5, qkv
-// 7.0 against 10.7, in_proj 10.0 against 11.0.  A wave that owns 64 rows of W (half the reads of A
-// from L2 and LDS) was slower (29 us for gate/up at 128 rows), and so were 4 x 2 waves.
+// It takes what the block products do not (launch_rows32): K below 1,024 and results that are not laid out in
+// sixteens of bytes.
 //
 // Host side guarantees: W in fragment order, K / gridDim.y a multiple of 256, lda a multiple of
 // 8, M * lda < 2^31.  Rows of A past M repeat the last row, pieces of W past the end the last
@@ -2983,6 +2980,15 @@ static bool launch_rows32(const bf16_t* A, const bf16_t* Wf, const float* bias, 
       n_rows_w % (EPI == 1 ? 32 : 16) || (lda % 8) || (long)M * lda >= (1L << 31) - 2048 ||
       (out_cols % 4) || (ldc % 4) || ((uintptr_t)C % 16) || (EPI == 1 && sizeof(TO) != 2))
     return false;
+  // the block products wherever the shape fits them and K is one that they were measured over, 1,024 to 10,752 (with
+  // a shorter one this kernel is at a dependent kernel's own time as it is).  Us by them and by this kernel: 64 rows of
+  // 16384 x 2048 gated 15.5 and 18.1, 6144 x 2048 in two ranges 8.5 and 9.6, 2048 x 2048 in eight 4.5 and 5.2, 2048 x
+  // 8192 in eight 9.7 and 11.8; 100 rows of 9216 x 1024 gated 8.5 and 10.3, 3072 x 1024 in four 5.3 and 6.2, 1024 x
+  // 4608 in six 5.1 and 8.0; 33 rows of 2048 x 10752 in six 11.4 and 13.8.
+  if (K >= 1024 && block256_fits<TO, EPI>(A, Wf, C, M, n_rows_w, K, lda, ldc, ksplit)) {
+    launch_tile<TO, EPI>(A, nullptr, bias, C, M, n_rows_w, K, lda, ldc, ksplit, 0, stream, Wf);
+    return true;
+  }
   switch ((M + 31) / 32) {
     case 1: launch_rows32_cfg<TO, 1, EPI>(A, Wf, bias, C, M, n_rows_w, K, lda, ldc, ksplit, stream); break;
     case 2: launch_rows32_cfg<TO, 2, EPI>(A, Wf, bias, C, M, n_rows_w, K, lda, ldc, ksplit, stream); break;
@@ -3015,8 +3021,8 @@ static int launch_bf16(const bf16_t* A, const bf16_t* W, const float* bias, TO* 
   // the 128 x 128 blocks than through the decode kernel, which reads the rows once per 32 columns
   const bool wide_head = EPI == 0 && M > 32 && N >= 16384 && force_kernel == 0 && ksplit == 1 &&
                          block256_fits<TO, EPI>(A, W, C, M, N, K, lda, ldc, ksplit);
-  // 25 to 128 rows: 32 x 32 tiles with the rows through LDS, when W is there in fragment order
-  // and the shape fits (else the kernels below)
+  // 25 to 128 rows: the smallest block products, or 32 x 32 tiles with the rows through LDS, when W is there in
+  // fragment order and the shape fits (else the kernels below)
   if constexpr (EPI != 2) {
     if (force_kernel == 12 || (force_kernel == 0 && M > KAPPAI_ROWS32_MIN_ROWS &&
                                M <= KAPPAI_ROWS32_MAX_ROWS &&

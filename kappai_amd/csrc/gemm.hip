@@ -7,7 +7,7 @@
 //                    does not depend on M; a kernel for up to 64 rows and one for more.
 //   gemm_bf16_direct, gemm_bf16_staged  large products over a W in fragment order (K a multiple of
 //                    128 per K range): bf16 inputs, fp32 accumulation on the matrix cores
-//                    (v_mfma_f32_32x32x16_bf16), 256x256 to 128x128 blocks, tiles of 64 of K loaded
+//                    (v_mfma_f32_32x32x16_bf16), 256x256 to 64x64 blocks, tiles of 64 of K loaded
 //                    straight into LDS (in the largest blocks W's straight into registers).
 //   gemm_bf16_block256  the same over a W that lies as rows.
 //   gemm_bf16_tile   any K that is a multiple of 8: 256x128 or 128x128 blocks staged through
@@ -16,8 +16,8 @@
 //                    waves split K and meet in LDS (v_mfma_f32_16x16x32_bf16).
 //   gemm_bf16_shared_rows  17 <= M <= 64 and a W with many rows: as above, but two waves that
 //                    stream different rows of W share the rows of A through LDS.
-//   gemm_bf16_rows32 25 <= M <= 128: the same idea with 32 x 32 tiles (v_mfma_f32_32x32x16_bf16),
-//                    W from its fragment-order copy.
+//   gemm_bf16_rows32 25 <= M <= 128 where the block products do not fit: the same idea with 32 x 32 tiles
+//                    (v_mfma_f32_32x32x16_bf16), W from its fragment-order copy.
 //   gemm_bf16_any    K or a row stride that is no multiple of 8: a plain kernel, so that no
 //                    width is refused.
 #include "common.h"

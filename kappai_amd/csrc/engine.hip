@@ -323,8 +323,9 @@ kappai_carry linear(Step& c, kappai_rows x, const kappai_linear& lin, int out_bf
       refuse(c, "rows in kernel order reached a matrix stored in 32 bits");
       return out;
     }
-    if (into != nullptr && !x.is_bf16 && !out_bf16 && c.m->kernels->gemm_f32_norms(M, N)) {
-      // a step of few rows: the result joins the stream, which the next product may norm itself
+    if (into != nullptr && !x.is_bf16 && !out_bf16 && K >= 4 && k.gemm_f32_norms(M, N)) {
+      // a step of few rows: the result joins the stream, which the next product may norm itself (kappai_gemm_f32_add
+      // takes K from 4 on; a shorter one goes the plain way below)
       LAUNCH(c, k.gemm_f32_add((const float*)x.data, (const float*)lin.w, lin.bias, into->resid, M, N, K,
                                M > 1 ? x.ld : K, N, c.stream));
       return out;

@@ -135,8 +135,9 @@ typedef struct kappai_fold {
 
 // Rows on their way into a product: plain [M, D] with a row stride, 16 row slots in fragment
 // order, or either of the two still to be divided by the rows' root mean square (ss != null); or the
-// residual stream itself, which the product norms with `norm` (KAPPAI_ROWS_OF_STREAM; float32, and only to
-// parts of the framework whose first product takes it: others get rows that are normed).
+// residual stream itself, which the product norms with `norm` (KAPPAI_ROWS_OF_STREAM; float32).  Those last as long as
+// nothing joins the stream, so only "block.pre_norm" hands them out, to the framework's parts whose first product
+// takes them: the runner "norm.rms" gives every other caller rows of their own.
 enum { KAPPAI_ROWS_OF_STREAM = 2 };
 typedef struct kappai_rows {
   void* data;
@@ -200,8 +201,8 @@ typedef struct kappai_step_api {
   void (*fail)(kappai_step*, const char* message);
   // y = x W^T (+ bias).  out_bf16: the dtype of a plain result.  partial_sums: the result may come
   // as float planes over ranges of K (the caller hands it to a norm or a kernel that adds them).
-  // into: the product may add its result into the residual stream (up to 16 bfloat16 rows), and
-  // fold into->norm in; null: never.  region: where a result that outlives the block goes.
+  // into: the product may add its result into the residual stream (up to 16 bfloat16 rows, or up to 8 float32
+  // ones), and fold into->norm in (bfloat16 only); null: never.  region: where a result that outlives the block goes.
   kappai_carry (*linear)(kappai_step*, kappai_rows x, const kappai_linear* lin, int out_bf16,
                          int partial_sums, const kappai_into* into, int region);
   // rows any kernel can read: scaled rows or rows in fragment order are made anew by the norm

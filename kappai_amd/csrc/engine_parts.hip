@@ -43,10 +43,12 @@ kappai_rows rows_of(void* data, int M, int D, int is_bf16) {
 // The rows that `consumer` reads after the norm: scaled rows made for this norm go through as
 // they are, else the norm's kernel runs, writing fragment order when that suits the number of
 // rows and the consumer.  The first norm of a step looks the embedding up in the same kernel.
+// of_stream: the caller hands the rows to `consumer` alone, before anything else joins the stream, so they may be
+// the stream itself.
 bool norms_the_stream(const kappai_part* consumer);
 
-kappai_rows rms_norm(kappai_step* s, const void* desc, float* resid, kappai_carry carry, int M,
-                     const int* rows, int n_rows, const kappai_part* consumer) {
+kappai_rows normed_rows(kappai_step* s, const void* desc, float* resid, kappai_carry carry, int M,
+                        const int* rows, int n_rows, const kappai_part* consumer, bool of_stream) {
   const kappai_step_api& api = *s->api;
   const kappai_fold* norm = static_cast<const kappai_fold*>(desc);
   const kappai_model& m = *api.model(s);
@@ -80,9 +82,10 @@ kappai_rows rms_norm(kappai_step* s, const void* desc, float* resid, kappai_carr
     return api.rms_norm(s, norm, resid, carry, M, rows, n_rows, 0);
   }
   // float32, few rows, the sum in the stream already: the consumer's first product norms them itself
-  if (carry.kind == KAPPAI_CARRY_NOTHING && rows == nullptr && !m.compute_bf16 && norms_the_stream(consumer) &&
-      consumer->first != nullptr && consumer->first->w_is_f32 && consumer->first->k == D &&
-      aligned16(consumer->first->w) && aligned16(norm->w) && m.kernels->gemm_f32_norms(M, D)) {
+  if (of_stream && carry.kind == KAPPAI_CARRY_NOTHING && rows == nullptr && !m.compute_bf16 &&
+      norms_the_stream(consumer) && consumer->first != nullptr && consumer->first->w_is_f32 &&
+      consumer->first->k == D && aligned16(consumer->first->w) && aligned16(norm->w) &&
+      m.kernels->gemm_f32_norms(M, D)) {
     kappai_rows out = rows_of(resid, M, D, 0);
     out.frag = KAPPAI_ROWS_OF_STREAM;
     out.norm = norm;
@@ -91,6 +94,12 @@ kappai_rows rms_norm(kappai_step* s, const void* desc, float* resid, kappai_carr
   const bool fragment = kernel_order && n >= m.tuning.fragment_rows_min && fragment_fits(m, n, D) &&
                         (carry.kind != KAPPAI_CARRY_PARTS || carry.parts <= 8);
   return api.rms_norm(s, norm, resid, carry, M, rows, n_rows, fragment ? 1 : 0);
+}
+
+// The runner: whoever calls it may do with the rows what they like, so they are never the stream itself.
+kappai_rows rms_norm(kappai_step* s, const void* desc, float* resid, kappai_carry carry, int M,
+                     const int* rows, int n_rows, const kappai_part* consumer) {
+  return normed_rows(s, desc, resid, carry, M, rows, n_rows, consumer, false);
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -378,13 +387,17 @@ kappai_carry pre_norm_block(kappai_step* s, const void* desc, float* resid, kapp
   const kappai_pre_norm_block& B = *static_cast<const kappai_pre_norm_block*>(desc);
   const int T = api.batch(s)->n_rows;
   kappai_carry none = {};
-  kappai_rows x = B.mixer_norm.run(s, B.mixer_norm.desc, resid, carry, T, nullptr, 0, &B.mixer);
+  const auto normed = [&](const kappai_norm_part& norm, const kappai_carry& c, const kappai_part& reader) {
+    return norm.run == rms_norm ? normed_rows(s, norm.desc, resid, c, T, nullptr, 0, &reader, true)
+                                : norm.run(s, norm.desc, resid, c, T, nullptr, 0, &reader);
+  };
+  kappai_rows x = normed(B.mixer_norm, carry, B.mixer);
   if (!api.ok(s)) return none;
   const kappai_into into_ffn = {resid, fold_for(&B.ffn_norm, &B.feed_forward)};
   const kappai_carry mixed = B.mixer.run(
       s, B.mixer.desc, x, resid, (B.mixer.flags & KAPPAI_ADDS_RESIDUAL) ? &into_ffn : nullptr);
   if (!api.ok(s)) return none;
-  kappai_rows x2 = B.ffn_norm.run(s, B.ffn_norm.desc, resid, mixed, T, nullptr, 0, &B.feed_forward);
+  kappai_rows x2 = normed(B.ffn_norm, mixed, B.feed_forward);
   if (!api.ok(s)) return none;
   const kappai_into into_next = {resid, fold_for(after_norm, after_consumer)};
   return B.feed_forward.run(s, B.feed_forward.desc, x2, resid,

@@ -151,5 +151,24 @@ extern "C" kappai_carry toy_parallel_block_run(kappai_step* s, const void* desc,
   return d.feed_forward.run(s, d.feed_forward.desc, h, resid, nullptr);
 }
 
+// A block that gives one norm's rows to two parts, each of which may add its result into the stream itself:
+// h = norm(x); x += mixer(h); x += feed_forward(h).  (The description of the block above.)
+extern "C" kappai_carry toy_two_readers_run(kappai_step* s, const void* desc, float* resid,
+                                            kappai_carry carry, const kappai_norm_part* after_norm,
+                                            const kappai_part* after_consumer) {
+  (void)after_norm;
+  (void)after_consumer;
+  const kappai_step_api& api = *s->api;
+  const toy_parallel_block& d = *static_cast<const toy_parallel_block*>(desc);
+  const int M = api.batch(s)->n_rows, D = api.model(s)->width;
+  const kappai_into into = {resid, nullptr};
+  const kappai_rows h = d.norm.run(s, d.norm.desc, resid, carry, M, nullptr, 0, &d.mixer);
+  kappai_carry mixed = d.mixer.run(s, d.mixer.desc, h, resid, &into);
+  mixed = api.plain_carry(s, mixed, resid, M);
+  if (mixed.kind == KAPPAI_CARRY_DELTA && !api.dry(s) && api.ok(s))
+    api.launched(s, toy_add_launch(resid, mixed.data, mixed.is_f32, (long)M * D, api.stream(s)));
+  return d.feed_forward.run(s, d.feed_forward.desc, h, resid, &into);
+}
+
 extern "C" int toy_layer_norm_desc_bytes(void) { return (int)sizeof(toy_layer_norm); }
 extern "C" int toy_parallel_block_desc_bytes(void) { return (int)sizeof(toy_parallel_block); }

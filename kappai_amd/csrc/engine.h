@@ -202,7 +202,8 @@ typedef struct kappai_step_api {
   // y = x W^T (+ bias).  out_bf16: the dtype of a plain result.  partial_sums: the result may come
   // as float planes over ranges of K (the caller hands it to a norm or a kernel that adds them).
   // into: the product may add its result into the residual stream (up to 16 bfloat16 rows, or up to 8 float32
-  // ones), and fold into->norm in (bfloat16 only); null: never.  region: where a result that outlives the block goes.
+  // ones that do not lie in that stream), and fold into->norm in (bfloat16 only); null: never.  region: where a
+  // result that outlives the block goes.
   kappai_carry (*linear)(kappai_step*, kappai_rows x, const kappai_linear* lin, int out_bf16,
                          int partial_sums, const kappai_into* into, int region);
   // rows any kernel can read: scaled rows or rows in fragment order are made anew by the norm

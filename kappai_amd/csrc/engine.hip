@@ -202,6 +202,10 @@ void decode_splits(int kpw, int max_splits, int waves, int rows, int G, int n_ke
 // what every part may ask of the step
 // ---------------------------------------------------------------------------------------------
 bool aligned16(const void* p) { return ((uintptr_t)p % 16) == 0; }
+// Do n floats from a on and m floats from b on have none in common?
+bool apart(const float* a, size_t n, const float* b, size_t m) {
+  return (uintptr_t)(a + n) <= (uintptr_t)b || (uintptr_t)(b + m) <= (uintptr_t)a;
+}
 
 // Can the kernel for 1 to 16 rows of this matrix read rows in fragment order / scale its results?
 int takes_kernel_order(const kappai_linear* lin, int D) {
@@ -323,9 +327,10 @@ kappai_carry linear(Step& c, kappai_rows x, const kappai_linear& lin, int out_bf
       refuse(c, "rows in kernel order reached a matrix stored in 32 bits");
       return out;
     }
-    if (into != nullptr && !x.is_bf16 && !out_bf16 && K >= 4 && k.gemm_f32_norms(M, N)) {
+    if (into != nullptr && !x.is_bf16 && !out_bf16 && K >= 4 && k.gemm_f32_norms(M, N) &&
+        apart((const float*)x.data, (size_t)(M - 1) * x.ld + K, into->resid, (size_t)M * N)) {
       // a step of few rows: the result joins the stream, which the next product may norm itself (kappai_gemm_f32_add
-      // takes K from 4 on; a shorter one goes the plain way below)
+      // takes K from 4 on, and rows that it does not write meanwhile; others go the plain way below)
       LAUNCH(c, k.gemm_f32_add((const float*)x.data, (const float*)lin.w, lin.bias, into->resid, M, N, K,
                                M > 1 ? x.ld : K, N, c.stream));
       return out;

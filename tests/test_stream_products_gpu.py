@@ -121,3 +121,82 @@ def test_rows_that_two_parts_read(tmp_path, rows):
     raw = {"architectures": ["ToyTwoReadersForCausalLM"], "width": 128, "vocab_size": 211}
     write_random_model(tmp_path / "m", config_from_dict(raw), seed=5, std=0.1, norm_jitter=0.1)
     from_both_sides(load_model(tmp_path / "m", "float32", DEV), one_by_one(raw["vocab_size"], rows), tmp_path)
+
+
+def define_stream_map():
+    """An architecture whose feed-forwards read the stream itself (``toy_stream_map_run`` of
+    tests/toy_parts/layer_norm_block.hip)."""
+    from kappai_amd.config import ModelConfig, register_architecture
+    from kappai_amd.models import Model
+    from kappai_amd.parts import (FEED_FORWARDS, FeedForward, Linear, OutputHead, TokenEmbedding, make_part,
+                                  register_part)
+    from kappai_amd.parts.cdesc import RUNNER_PART, LinearDesc
+    if "toy_stream_map" in FEED_FORWARDS:
+        return
+
+    class StreamMap(FeedForward):
+        adds_residual = True           # (for the stream that comes with ``into``)
+
+        def __init__(self, prefix, width):
+            self.map = Linear([prefix + "map"], width, [width])
+
+        def tensor_specs(self):
+            return self.map.tensor_specs()
+
+        def bind(self, tensors):
+            self.map.bind(tensors)
+
+        def weight_bytes(self):
+            return self.map.weight_bytes()
+
+        def forward(self, x, batch, into=None):
+            return self.map.forward(into.resid)
+
+        def c_part(self, plan, view=None, shared_cache=False):
+            lib = toy_block_library()
+            lib.toy_stream_map_run.restype = None         # only its address is used
+            plan.register_runner("feed_forward.toy_stream_map", RUNNER_PART, lib.toy_stream_map_run, LinearDesc)
+            return plan.part("feed_forward.toy_stream_map", plan.linear(self.map), adds_residual=True)
+
+    register_part("feed_forward", "toy_stream_map", StreamMap)
+
+    @dataclass
+    class Config(ModelConfig):
+        width: int = 0
+        vocab_size: int = 0
+        max_position_embeddings: int = 512
+
+        @classmethod
+        def from_dict(cls, raw):
+            return cls(architecture="ToyStreamMapForCausalLM", width=raw["width"], vocab_size=raw["vocab_size"])
+
+        def to_dict(self):
+            return {"architectures": ["ToyStreamMapForCausalLM"], "width": self.width, "vocab_size": self.vocab_size}
+
+    def build(cfg, dtype):
+        how = dict(width=cfg.width, dtype=dtype)
+
+        def norm(name):
+            return make_part("norm", "rmsnorm", name=name, eps=1e-5, **how)
+        layers = [make_part("block", "pre_norm", mixer_norm=norm(f"b{i}.n1"),
+                            mixer=make_part("mixer", "conv", prefix=f"b{i}.c.", kernel_size=3, bias=True, **how),
+                            ffn_norm=norm(f"b{i}.n2"),
+                            feed_forward=make_part("feed_forward", "toy_stream_map", prefix=f"b{i}.", width=cfg.width))
+                  for i in range(2)]
+        emb = TokenEmbedding("emb", cfg.vocab_size, cfg.width)
+        return Model(cfg, dtype, emb, layers, norm("final"), OutputHead("head", cfg.vocab_size, cfg.width, tied_to=emb))
+
+    register_architecture("ToyStreamMapForCausalLM", Config, build)
+
+
+@pytest.mark.parametrize("rows", [1, 3, 8])
+def test_a_product_of_the_stream_into_the_stream(tmp_path, rows):
+    """Rows that lie in the stream which their product would join: the product may not write them while its other
+    blocks still read them, so it goes another way (width 1,024: a block for every CU reads all of them)."""
+    from kappai_amd.config import config_from_dict
+    from kappai_amd.models import load_model
+    from kappai_amd.weights import write_random_model
+    define_stream_map()
+    raw = {"architectures": ["ToyStreamMapForCausalLM"], "width": 1024, "vocab_size": 211}
+    write_random_model(tmp_path / "m", config_from_dict(raw), seed=5, std=0.03, norm_jitter=0.1)
+    from_both_sides(load_model(tmp_path / "m", "float32", DEV), one_by_one(raw["vocab_size"], rows), tmp_path)

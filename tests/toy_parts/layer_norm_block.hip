@@ -170,5 +170,17 @@ extern "C" kappai_carry toy_two_readers_run(kappai_step* s, const void* desc, fl
   return d.feed_forward.run(s, d.feed_forward.desc, h, resid, &into);
 }
 
+// A feed-forward that reads the stream itself, not the rows it is given: x += W x.
+extern "C" kappai_carry toy_stream_map_run(kappai_step* s, const void* desc, kappai_rows x, float* resid,
+                                           const kappai_into* into) {
+  const kappai_step_api& api = *s->api;
+  kappai_rows rows = {};
+  rows.data = resid;
+  rows.M = x.M;
+  rows.D = rows.ld = api.model(s)->width;
+  return api.linear(s, rows, static_cast<const kappai_linear*>(desc), api.model(s)->compute_bf16, 1, into,
+                    api.carry_region(s));
+}
+
 extern "C" int toy_layer_norm_desc_bytes(void) { return (int)sizeof(toy_layer_norm); }
 extern "C" int toy_parallel_block_desc_bytes(void) { return (int)sizeof(toy_parallel_block); }

@@ -123,6 +123,21 @@ class PositionEncoding(Part):
         return None
 
 
+class WithOwn:
+    """A flag that a class announces for the ``method`` it brings itself, set in its body beside that method
+    (``adds_residual = WithOwn("forward")``): True there and where the method is inherited.  A subclass that brings a
+    method of its own and says nothing of the flag has not announced it."""
+
+    def __init__(self, method: str):
+        self.method = method
+
+    def __set_name__(self, owner, name):
+        self.owner = owner
+
+    def __get__(self, part, cls) -> bool:
+        return getattr(cls, self.method) is self.owner.__dict__[self.method]
+
+
 class Mixer(Part):
     """A token mixer.  ``cache_spec`` says what it needs from the cache manager (a PagedSpec,
     FixedState or None); ``forward`` gets the normalised rows [T, width] in the compute

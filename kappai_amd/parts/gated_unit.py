@@ -21,14 +21,14 @@ import torch
 from ..cache.specs import CacheBundle, FixedState
 from ..kernels import ops, profile, tuning
 from ..weights.spec import INIT_NORMAL, INIT_SMALL, MATRIX, VECTOR, TensorSpec
-from .base import Mixer, register_part
+from .base import Mixer, WithOwn, register_part
 from .linear import Linear
 from .mingru import ScanChunks
 
 
 class RealGatedUnit(Mixer):
-    takes_deferred_rows = True     # (its first product does)
-    adds_residual = True
+    takes_deferred_rows = WithOwn("forward")     # (its first product does)
+    adds_residual = WithOwn("forward")
 
     def __init__(self, prefix: str, width: int, inner: int, blocks: int, taps: int,
                  dtype: torch.dtype, rate: float = 8.0, names=None,

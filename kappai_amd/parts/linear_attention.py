@@ -39,7 +39,7 @@ import torch
 from ..cache.specs import CacheBundle, FixedState
 from ..kernels import ops, profile, tuning
 from ..weights.spec import INIT_ONES, INIT_SMALL, VECTOR, TensorSpec
-from .base import Mixer, register_part
+from .base import Mixer, WithOwn, register_part
 from .linear import Linear
 from .mingru import ScanChunks
 
@@ -146,7 +146,7 @@ register_part("mixer", "gated_linear_attention", GatedLinearAttention)
 
 
 class FixedDecayAttention(Mixer):
-    takes_deferred_rows = True     # (its one product of the rows does)
+    takes_deferred_rows = WithOwn("forward")     # (its one product of the rows does)
 
     def __init__(self, prefix: str, width: int, num_heads: int, dim: int, vdim: int, decay,
                  norm_eps: float, dtype: torch.dtype, names=None, weight_suffix: str = ".weight"):

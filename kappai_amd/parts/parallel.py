@@ -19,7 +19,7 @@ from ..cache.manager import BundleView
 from ..cache.specs import CacheBundle
 from ..kernels import ops
 from ..weights.spec import INIT_ONES, VECTOR, TensorSpec
-from .base import Mixer, WeightedTerms, register_part
+from .base import Mixer, WeightedTerms, WithOwn, register_part
 
 
 class ParallelMixer(Mixer):
@@ -34,6 +34,8 @@ class ParallelMixer(Mixer):
         self.summed = bool(summed) or self.side_norms is not None
         self.width, self.norm_eps = int(width), float(norm_eps)
         self.norm_w = (None, None)
+
+    _own_forward = WithOwn("forward")
 
     def _sides(self):
         return (("left", self.left), ("right", self.right))
@@ -86,11 +88,11 @@ class ParallelMixer(Mixer):
 
     @property
     def takes_deferred_rows(self) -> bool:
-        return all(getattr(m, "takes_deferred_rows", False) for _, m in self._sides())
+        return self._own_forward and all(getattr(m, "takes_deferred_rows", False) for _, m in self._sides())
 
     @property
     def adds_residual(self) -> bool:
-        return self.summed               # (the sum of the two sides is an update of the stream)
+        return self._own_forward and self.summed     # (the sum of the two sides is an update of the stream)
 
     def forward(self, x, batch, cache, shared_cache: bool = False, into=None):
         if shared_cache:

@@ -43,7 +43,7 @@ from ..cache.specs import PagedKV
 from ..kernels import ops, profile, tuning
 from ..weights.spec import INIT_ONES, INIT_SMALL, VECTOR, TensorSpec
 from .attention import AttentionTiles
-from .base import Mixer, register_part
+from .base import Mixer, WithOwn, register_part
 from .linear import Linear
 
 
@@ -70,7 +70,7 @@ def distance_bias_columns(table: torch.Tensor, far: float) -> torch.Tensor:
 
 
 class ScoredAttention(Mixer):
-    takes_deferred_rows = True     # (its one product of the rows does)
+    takes_deferred_rows = WithOwn("forward")     # (its one product of the rows does)
 
     def __init__(self, prefix: str, width: int, num_heads: int, num_kv_heads: int, dim: int,
                  vdim: int, scale: float, dtype: torch.dtype, norm_eps: float = 0.0,

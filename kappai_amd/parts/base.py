@@ -190,8 +190,9 @@ class Hidden:
 @dataclass
 class WeightedTerms:
     """What a mixer made of two returns: ``scale_a * a + scale_b * b``, not summed yet (the norm
-    or the sum that follows does it in float32).  ``a`` and ``b``: [T, width] in float32 or the
-    compute dtype; ``a`` may be float32 partial sums [S, T, width]."""
+    or the sum that follows does it in float32).  ``a`` and ``b``: [T, width] in one dtype; for a norm that
+    announces ``takes_terms_as_made`` in float32 or the compute dtype each, and ``a`` also as float32 partial
+    sums [S, T, width]."""
     a: torch.Tensor
     scale_a: float
     b: torch.Tensor

@@ -271,7 +271,10 @@ class OutputNormBlock(Block):
         x = h.rows if narrow else resid
         if x is None:
             x = ops.cast(resid, self.mixer_norm.dtype)
-        mixed = self.mixer.forward(x, batch, cache, shared_cache=shared_cache)
+        as_made = (getattr(self.mixer, "hands_terms_as_made", False)
+                   and getattr(self.mixer_norm, "takes_terms_as_made", False))
+        how = {"terms_as_made": True} if as_made else {}
+        mixed = self.mixer.forward(x, batch, cache, shared_cache=shared_cache, **how)
         rows = self.mixer_norm.norm_output(resid, mixed, rows_dtype=rows_dtype)
         if self.feed_forward is not None:
             out = self.feed_forward.forward(rows if narrow else resid, batch)

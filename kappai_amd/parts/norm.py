@@ -9,7 +9,7 @@ import torch
 
 from ..kernels import ops, profile, tuning
 from ..weights.spec import INIT_ONES, INIT_SMALL, VECTOR, TensorSpec
-from .base import Norm, NormedUpdate, StreamUpdate, WeightedTerms, register_part
+from .base import Norm, NormedUpdate, StreamUpdate, WeightedTerms, WithOwn, register_part
 from .cdesc import FoldDesc
 
 
@@ -17,6 +17,7 @@ class RMSNorm(Norm):
     takes_partial_sums = True      # the kernel adds [S, T, width] partial sums itself, in order
     takes_normed_update = True     # and RMS-norms a pending update on the way into the stream
     takes_expert_terms = True      # and sums what a mixture's chosen experts left
+    takes_terms_as_made = WithOwn("norm_output")   # and the two sides of a mixer, planes and either type
     can_defer = True      # add_norm(..., defer=True) may hand out ops.ScaledRows or
                           # ops.FragmentRows in place of a tensor
 

@@ -36,6 +36,9 @@ class ParallelMixer(Mixer):
         self.norm_w = (None, None)
 
     _own_forward = WithOwn("forward")
+    # ``forward`` takes ``terms_as_made``: ``WeightedTerms`` may then hold its ``a`` as partial sums and its two sides
+    # in a type each, for a norm that reads them so (a kernel less a side)
+    hands_terms_as_made = WithOwn("forward")
 
     def _sides(self):
         return (("left", self.left), ("right", self.right))
@@ -94,12 +97,12 @@ class ParallelMixer(Mixer):
     def adds_residual(self) -> bool:
         return self._own_forward and self.summed     # (the sum of the two sides is an update of the stream)
 
-    def forward(self, x, batch, cache, shared_cache: bool = False, into=None):
+    def forward(self, x, batch, cache, shared_cache: bool = False, into=None, terms_as_made: bool = False):
         if shared_cache:
             raise ValueError("a pair of mixers does not read another layer's cache")
         out = [m.forward(x, batch, self._view(cache, side, m)) for side, m in self._sides()]
-        # the kernel that sums the two reads planes and either type itself; elsewhere they are made alike first
-        in_kernel = out[0].is_cuda
+        # the kernels that sum the two read planes and either type themselves; elsewhere they are made alike first
+        in_kernel = out[0].is_cuda and (self.summed or terms_as_made)
         for i, y in enumerate(out):
             if y.dim() == 3 and not (in_kernel and (self.summed or i == 0)):
                 out[i] = ops.sum_partial_sums(y)

@@ -71,3 +71,38 @@ def test_two_sides_as_the_kernel_for_any_row(ops, D, a, b, normed):  # noqa: F81
         y = ops.pair_norm_sum(*s, 0.5, 0.75, *ws, 1e-5, add_into=ops.AddInto(stream, norm_w, 1e-5))
         out.append((stream, y.data, y.ss[0, :T]))
     assert all(torch.equal(p, q) for p, q in zip(*out))
+
+
+@pytest.mark.parametrize("a,b", [("planes", "bf16"), ("bf16", "planes"), ("f32", "bf16"), ("bf16", "bf16")])
+def test_a_norm_from_outside_gets_terms_of_one_type(ops, a, b):  # noqa: F811
+    """The two sides of a mixer behind which a norm stands that says nothing of planes or types: [T, D] in one type;
+    the framework's own norm gets them as they were made, with the same stream."""
+    from kappai_amd.parts import Hidden, Mixer, RMSNorm
+    from kappai_amd.parts.block import OutputNormBlock
+    from kappai_amd.parts.parallel import ParallelMixer
+    T, D, seen = 3, 256, []
+    (ya, fa), (yb, fb) = side(a, T, D, 21), side(b, T, D, 22)
+
+    class Side(Mixer):
+        def __init__(self, y):
+            self.y = y
+
+        def forward(self, x, batch, cache, shared_cache=False):
+            return self.y.clone()
+
+    class Outside(RMSNorm):
+        def norm_output(self, resid, y, rows_dtype=None, add=True):
+            seen.append((y.a, y.b))
+            return super().norm_output(resid, y, rows_dtype, add)
+
+    streams = []
+    for cls in (RMSNorm, Outside):
+        norm = cls("n", D, 1e-5, BF16)
+        norm.weight = rand((D,), F32, 23).to(DEV)
+        resid = rand((T, D), F32, 24).to(DEV)
+        block = OutputNormBlock(ParallelMixer(Side(ya), Side(yb), 0.5, 0.25), norm)
+        out = block.forward(Hidden(resid, None, resid.bfloat16()), None, None)
+        streams.append((out.resid, out.rows))
+    assert all(torch.equal(x, y) for x, y in zip(*streams))
+    (got_a, got_b), = seen
+    assert got_a.dtype == got_b.dtype and torch.equal(got_a.float(), fa) and torch.equal(got_b.float(), fb)

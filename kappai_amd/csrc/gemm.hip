@@ -2971,10 +2971,10 @@ static void launch_rows32_cfg(const bf16_t* A, const bf16_t* Wf, const float* bi
 }
 
 // Returns false when the shape does not fit (the caller then takes a block kernel).  The output
-// must allow the kernel's stores of four values (8 or 16 bytes).
+// must allow the kernel's stores of four values (8 or 16 bytes).  itself: no block product in its place.
 template <typename TO, int EPI>
 static bool launch_rows32(const bf16_t* A, const bf16_t* Wf, const float* bias, TO* C, int M,
-                          int n_rows_w, int K, int lda, int ldc, int ksplit, hipStream_t stream) {
+                          int n_rows_w, int K, int lda, int ldc, int ksplit, bool itself, hipStream_t stream) {
   const int out_cols = EPI == 1 ? n_rows_w / 2 : n_rows_w;
   if (Wf == nullptr || M < 1 || M > KAPPAI_ROWS32_MAX_ROWS || ksplit < 1 || K % (ksplit * R32_NWK * 64) ||
       n_rows_w % (EPI == 1 ? 32 : 16) || (lda % 8) || (long)M * lda >= (1L << 31) - 2048 ||
@@ -2985,7 +2985,7 @@ static bool launch_rows32(const bf16_t* A, const bf16_t* Wf, const float* bias, 
   // 16384 x 2048 gated 15.5 and 18.1, 6144 x 2048 in two ranges 8.5 and 9.6, 2048 x 2048 in eight 4.5 and 5.2, 2048 x
   // 8192 in eight 9.7 and 11.8; 100 rows of 9216 x 1024 gated 8.5 and 10.3, 3072 x 1024 in four 5.3 and 6.2, 1024 x
   // 4608 in six 5.1 and 8.0; 33 rows of 2048 x 10752 in six 11.4 and 13.8.
-  if (K >= 1024 && block256_fits<TO, EPI>(A, Wf, C, M, n_rows_w, K, lda, ldc, ksplit)) {
+  if (!itself && K >= 1024 && block256_fits<TO, EPI>(A, Wf, C, M, n_rows_w, K, lda, ldc, ksplit)) {
     launch_tile<TO, EPI>(A, nullptr, bias, C, M, n_rows_w, K, lda, ldc, ksplit, 0, stream, Wf);
     return true;
   }
@@ -3024,15 +3024,15 @@ static int launch_bf16(const bf16_t* A, const bf16_t* W, const float* bias, TO* 
   // 25 to 128 rows: the smallest block products, or 32 x 32 tiles with the rows through LDS, when W is there in
   // fragment order and the shape fits (else the kernels below)
   if constexpr (EPI != 2) {
-    if (force_kernel == 12 || (force_kernel == 0 && M > KAPPAI_ROWS32_MIN_ROWS &&
-                               M <= KAPPAI_ROWS32_MAX_ROWS &&
-                               Wf != nullptr && !wide_head)) {
+    const bool forced = force_kernel == 12 || force_kernel == 18;
+    if (forced || (force_kernel == 0 && M > KAPPAI_ROWS32_MIN_ROWS && M <= KAPPAI_ROWS32_MAX_ROWS &&
+                   Wf != nullptr && !wide_head)) {
       if (launch_rows32<TO, EPI>(A, Wf, bias, C, M, EPI == 1 ? 2 * N : N, K, lda, ldc, ksplit,
-                                 stream))
+                                 force_kernel == 18, stream))
         KAPPAI_RETURN_LAUNCH_STATUS();
-      if (force_kernel == 12) return (int)hipErrorInvalidValue;
+      if (forced) return (int)hipErrorInvalidValue;
     }
-  } else if (force_kernel == 12) {
+  } else if (force_kernel == 12 || force_kernel == 18) {
     return (int)hipErrorInvalidValue;
   }
   // 17 to 64 rows and blocks enough to fill half the chip: the rows go through LDS
@@ -3082,9 +3082,9 @@ static int launch_bf16(const bf16_t* A, const bf16_t* W, const float* bias, TO* 
 // K, lda must be multiples of 8 and A, W 16-byte aligned (checked by the caller).
 // force_kernel: 0 = by M, 1 = tile kernel, 2 = skinny kernel (M <= 64 only), 3..8 = tile kernel
 // with block shape 1..6 (see launch_tile), 9 = shared-rows kernel (17 to 64 rows, K / ksplit a
-// multiple of 512), 10 = block shape 8, 11 = block shape 9, 12 = the kernel for 25 to 128 rows
+// multiple of 512), 10 = block shape 8, 11 = block shape 9, 12 = what steps of 25 to 128 rows take
 // (1 to 128 rows, W in fragment order, K / ksplit a multiple of 256), 13 to 17 = block shapes 11 to
-// 15; for tests and tuning.
+// 15, 18 = gemm_bf16_rows32 wherever 12 is taken; for tests and tuning.
 // ksplit > 1 (float output only): C is [ksplit][M][ldc] partial sums over K ranges.
 // W_frag: null, or W in fragment order (K a multiple of 32, rows a multiple of 16); W may then
 // be null: every kernel reads the fragment order (only kappai_gemm_bf16_any needs rows).

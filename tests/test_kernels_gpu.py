@@ -263,14 +263,15 @@ def test_linear_shared_rows_split_k(ops, M, N, K, S):
     close(parts.sum(0), x.double() @ w.double().T + b.double(), 2e-5, "sum of the partial sums")
 
 
-ROWS32 = 12           # force_kernel: 25 to 128 rows (it takes 1 to 128), 32 x 32 tiles, rows via LDS
+ROWS32 = 18           # force_kernel: 32 x 32 tiles, rows via LDS, 1 to 128 rows
+STEP_ROWS = 12        # force_kernel: what steps of 25 to 128 rows take, this kernel or the block products
 
 
 @pytest.mark.parametrize("M", [1, 31, 65, 96, 97, 128])
-@pytest.mark.parametrize("N,K", [(64, 256), (208, 1024), (2048, 2048), (8208, 1536)])
+@pytest.mark.parametrize("N,K", [(64, 256), (208, 512), (112, 768), (208, 1024), (2048, 2048), (8208, 1536)])
 @pytest.mark.parametrize("out_dtype", [F32, BF16])
 def test_linear_rows32(ops, M, N, K, out_dtype):
-    """The kernel for 25 to 128 rows: every row-tile count, matrices that end inside a block's 64
+    """The kernel with 32 x 32 tiles: every row-tile count, matrices that end inside a block's 64
     columns or inside a wave's 32 (208 = 6 tiles and a half), one and several runs of K, a row
     stride, bias; the matrix in fragment order only, and beside its rows."""
     wide = rand((M, K + 8), BF16, 151)
@@ -284,9 +285,11 @@ def test_linear_rows32(ops, M, N, K, out_dtype):
     got = ops.linear(xd, wd, b.to(DEV), out_dtype=out_dtype, force_kernel=ROWS32,
                      weight_frag=ops.fragment_order(wd))
     close(got.float(), want + b.double(), tol, "rows32 with bias")
+    if K < 1024 and M > 24:     # and it is what such a step takes by itself: the same bits
+        assert torch.equal(ops.linear(xd, kept, b.to(DEV), out_dtype=out_dtype), got)
 
 
-@pytest.mark.parametrize("M,F,K", [(65, 48, 256), (100, 1008, 1024), (128, 8192, 2048)])
+@pytest.mark.parametrize("M,F,K", [(65, 48, 256), (33, 112, 512), (97, 208, 768), (100, 1008, 1024), (128, 8192, 2048)])
 def test_linear_swiglu_rows32(ops, M, F, K):
     x, wg, wu = rand((M, K), BF16, 154), rand((F, K), BF16, 155, 0.2), rand((F, K), BF16, 156, 0.2)
     w = ops.InFragments.of(ops.interleave_gate_up(wg.to(DEV), wu.to(DEV)))
@@ -294,45 +297,68 @@ def test_linear_swiglu_rows32(ops, M, F, K):
     want = g / (1 + torch.exp(-g)) * u
     got = ops.linear_swiglu(x.to(DEV), w, force_kernel=ROWS32)
     close(got.float(), want, BF16_ULP, "rows32")
-    if M > 24:          # and it is what such a step takes by itself: the same bits
-        assert torch.equal(ops.linear_swiglu(x.to(DEV), w), got)
+    step = ops.linear_swiglu(x.to(DEV), w, force_kernel=STEP_ROWS)
+    close(step.float(), want, BF16_ULP, "a step's kernel")
+    assert torch.equal(ops.linear_swiglu(x.to(DEV), w), step)
+    if K < 1024:
+        assert torch.equal(step, got)
 
 
 @pytest.mark.parametrize("M,N,K,S", [(128, 2048, 8192, 8), (70, 112, 3072, 3), (99, 2048, 2048, 2),
-                                     (128, 6144, 2048, 1)])
+                                     (128, 6144, 2048, 1), (33, 208, 512, 2), (97, 112, 768, 3), (65, 304, 1024, 2)])
 def test_linear_rows32_split_k(ops, M, N, K, S):
     x, w, b = rand((M, K), BF16, 157), rand((N, K), BF16, 158, 0.05), rand((N,), F32, 159)
     kept = ops.InFragments.of(w.to(DEV))
-    parts = ops.linear(x.to(DEV), kept, b.to(DEV), partial_sums=True, split_k=S,
-                       force_kernel=ROWS32)
     want = x.double() @ w.double().T + b.double()
-    if S == 1:
-        assert parts.shape == (M, N)
-        close(parts.float(), want, BF16_ULP, "one range")
-        return
-    assert parts.shape == (S, M, N) and parts.dtype == F32
-    close(parts.sum(0), want, 2e-5, "sum of the partial sums")
+    for force in (ROWS32, STEP_ROWS):
+        parts = ops.linear(x.to(DEV), kept, b.to(DEV), partial_sums=True, split_k=S, force_kernel=force)
+        if S == 1:
+            assert parts.shape == (M, N)
+            close(parts.float(), want, BF16_ULP, "one range")
+            continue
+        assert parts.shape == (S, M, N) and parts.dtype == F32
+        close(parts.sum(0), want, 2e-5, "sum of the partial sums")
 
 
-def test_linear_rows32_is_what_steps_of_25_to_128_rows_take(ops):
+# (bfloat16 rows of a result that are no multiple of 16 bytes apart: the block products do not store those)
+@pytest.mark.parametrize("M,N,K", [(25, 208, 512), (70, 112, 1024), (128, 96, 2304)])
+def test_rows32_between_columns_of_others(ops, M, N, K):
+    import ctypes
+    x, w = rand((M, K), BF16, 163).to(DEV), rand((N, K), BF16, 164).to(DEV)
+    frag, mark, ldc = ops.fragment_order(w), -123.5, N + 4
+    want = ops.linear(x, ops.InFragments.of(w), force_kernel=ROWS32)
+    i, none = ctypes.c_int, ctypes.c_void_p(0)
+    at = lambda t: ctypes.c_void_p(t.data_ptr())  # noqa: E731
+    for force in (0, STEP_ROWS, ROWS32):
+        out = torch.full((M + 130, ldc), mark, dtype=BF16, device=DEV)
+        assert ops.library("gemm").kappai_gemm_bf16(
+            at(x), none, at(frag), none, at(out), i(M), i(N), i(K), i(K), i(ldc), i(0), i(force), i(1), i(0), none,
+            i(0), ctypes.c_float(0), none, i(0), none, none, i(0), none,
+            ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)) == 0
+        assert torch.equal(out[:M, :N], want)
+        assert (out[:, N:] == mark).all() and (out[M:] == mark).all()
+
+
+def test_what_steps_of_25_to_128_rows_take(ops):
     """Without a kernel asked for, a product of 25 to 128 rows over a matrix in fragment order is
-    this kernel's (bit for bit), with the K ranges that the rule gives it; a matrix kept as rows
+    the same as asked for by that name (bit for bit), with the K ranges that the rule gives it; a matrix kept as rows
     only, or a K that is no multiple of 256, goes to the block kernels as before."""
     x, w = rand((100, 2048), BF16, 160).to(DEV), rand((3072, 2048), BF16, 161, 0.05).to(DEV)
     kept = ops.InFragments.of(w)
-    assert torch.equal(ops.linear(x, kept), ops.linear(x, kept, force_kernel=ROWS32))
+    assert torch.equal(ops.linear(x, kept), ops.linear(x, kept, force_kernel=STEP_ROWS))
     assert ops.split_k_for(100, 3072, 2048) == 4 and ops.split_k_for(100, 6144, 2048) == 2
     assert ops.split_k_for(128, 2048, 8192) == 8 and ops.split_k_for(65, 16384, 2048) == 1
     assert ops.split_k_for(64, 1024, 4608) == 6          # (not only powers of two)
     parts = ops.linear(x, kept, partial_sums=True)
     assert parts.shape == (4, 100, 3072)
-    assert torch.equal(parts, ops.linear(x, kept, partial_sums=True, force_kernel=ROWS32))
+    assert torch.equal(parts, ops.linear(x, kept, partial_sums=True, force_kernel=STEP_ROWS))
     close(ops.linear(x, w).float(), x.double().cpu() @ w.double().cpu().T, BF16_ULP, "rows only")
-    with pytest.raises(RuntimeError):
-        ops.linear(x, w, force_kernel=ROWS32)                 # no fragment order
     x3, w3 = x[:, :1920].contiguous(), ops.InFragments.of(w[:, :1920].contiguous())
-    with pytest.raises(RuntimeError):
-        ops.linear(x3, w3, force_kernel=ROWS32)               # 1920 is no multiple of 256
+    for force in (STEP_ROWS, ROWS32):
+        with pytest.raises(RuntimeError):
+            ops.linear(x, w, force_kernel=force)                 # no fragment order
+        with pytest.raises(RuntimeError):
+            ops.linear(x3, w3, force_kernel=force)               # 1920 is no multiple of 256
     close(ops.linear(x3, w3).float(), x3.double().cpu() @ w[:, :1920].double().cpu().T, BF16_ULP,
           "K = 1920")
 
@@ -449,13 +475,13 @@ def test_products_read_a_matrix_kept_in_fragment_order_only(ops, M, N, K):
     elif M > 16 and K % 512 == 0:
         forces += [SHARED_ROWS]
     if 24 < M <= 128 and K % 256 == 0:
-        # the kernel for 25 to 128 rows exists for the fragment order only: left to itself the
-        # product over the kept matrix is that kernel's, over the rows a block kernel's; the two
+        # what steps of 25 to 128 rows take is for the fragment order only: left to itself the
+        # product over the kept matrix is one kernel's, over the rows another's; the two may
         # add in another order, so they agree to rounding, not bit for bit
         forces.remove(0)
         close(ops.linear(x, kept, b, out_dtype=F32).float(),
               ops.linear(x, w, b, out_dtype=F32).double(), 2e-5, "another kernel for the kept matrix")
-        assert torch.equal(ops.linear(x, kept, b), ops.linear(x, kept, b, force_kernel=ROWS32))
+        assert torch.equal(ops.linear(x, kept, b), ops.linear(x, kept, b, force_kernel=STEP_ROWS))
     for force in forces:
         for bias in (None, b):
             for out_dtype in (BF16, F32):

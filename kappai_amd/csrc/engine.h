@@ -364,6 +364,11 @@ int kappai_split_k_for(int M, int N, int K);
 // Whether such a product hands its sums on in float (always with more than one range).
 int kappai_sums_in_f32(int M, int N, int K);
 
+// The blocks in which such a product runs over a W of n_rows rows in fragment order, in `split` ranges with results of
+// `elem` bytes (more than 24 rows; K a multiple of 128 in every range): shapes as gemm.hip numbers them, 0 for the
+// kernel with 32 x 32 tiles.  What the kernels' own choice is made of (gemm_rules.h), for tests and tuning.
+int kappai_block_shape_of(int M, int n_rows, int K, int split, int elem, int gated);
+
 // The most keys with which the decode attention keeps a row's keys in one block (attn_decode_block) where
 // `few` is what it takes for any number of rows (at head sizes up to 128; beyond, the most it ever takes).
 // waves: of a block, for the query heads a kv head (decode_block_waves).

@@ -150,11 +150,11 @@ Ranges ranges_over_fragments(int M, int N, int K) {
   return best;
 }
 
-// 25 to 128 rows: the kernel with 32 x 32 tiles gives a block 64 columns and takes K ranges that
-// are multiples of 256; as many equal ranges (at most 8: the norm's row kernel adds up to eight
-// planes, more take its general form, 6.5 against 2.6 us for 64 rows of 2,048) that up to 256 blocks stream the matrix
-// (from sweeps at the 1.2B and 350M shapes: in_proj two and four, qkv four, out_proj eight and
-// four, down eight and six; twice as many blocks were 5 to 40 % slower)
+// 25 to 128 rows: ranges of whole runs of 256, as many equal ones (at most 8: the norm's row kernel adds up to eight
+// planes, more take its general form, 6.5 against 2.6 us for 64 rows of 2,048) as give up to 256 blocks of 64 columns.
+// From sweeps at the 1.2B and 350M shapes with the kernel with 32 x 32 tiles (in_proj two and four, qkv four, out_proj
+// eight and four, down eight and six; twice as many were 5 to 40 % slower).  The block products that take most of
+// these rows since (gemm_rules.h) take 64 columns a block as well up to 64 rows; the ranges were kept.
 int split_k_rows32(int N, int K) {
   const long col_blocks = (N + 63) / 64;
   const int runs = K / KAPPAI_ROWS32_RUN;
@@ -661,6 +661,13 @@ extern "C" const char* kappai_forward_error(void) { return g_error; }
 extern "C" int kappai_split_k_for(int M, int N, int K) { return ranges_for(M, N, K).split; }
 
 extern "C" int kappai_sums_in_f32(int M, int N, int K) { return ranges_for(M, N, K).f32 ? 1 : 0; }
+
+extern "C" int kappai_block_shape_of(int M, int n_rows, int K, int split, int elem, int gated) {
+  if (M > KAPPAI_ROWS32_MIN_ROWS && M <= KAPPAI_ROWS32_MAX_ROWS && K % (KAPPAI_ROWS32_RUN * split) == 0 &&
+      kappai_rows32_takes(M, n_rows, K, split))
+    return 0;
+  return kappai_block_shape_for(M, n_rows, K, split, elem, gated != 0);
+}
 
 // One block a (row, kv head) takes a row's keys in at 50 GB/s or so, but needs no second kernel, and with
 // blocks enough for the chip nothing is won by more of them.  But a long row among short ones is then the whole

@@ -16,8 +16,8 @@
 //                    waves split K and meet in LDS (v_mfma_f32_16x16x32_bf16).
 //   gemm_bf16_shared_rows  17 <= M <= 64 and a W with many rows: as above, but two waves that
 //                    stream different rows of W share the rows of A through LDS.
-//   gemm_bf16_rows32 25 <= M <= 128 where the block products do not fit: the same idea with 32 x 32 tiles
-//                    (v_mfma_f32_32x32x16_bf16), W from its fragment-order copy.
+//   gemm_bf16_rows32 25 <= M <= 128 where the block products do not fit or are the slower: the same idea with
+//                    32 x 32 tiles (v_mfma_f32_32x32x16_bf16), W from its fragment-order copy.
 //   gemm_bf16_any    K or a row stride that is no multiple of 8: a plain kernel, so that no
 //                    width is refused.
 #include "common.h"
@@ -1770,9 +1770,7 @@ static void launch_tile(const bf16_t* A, const bf16_t* W, const float* bias, TO*
   if constexpr (EPI != 2) {
     if (Wf != nullptr && fits && (shape == 0 || shape >= 5)) {
       if (shape == 0)
-        shape = kappai_block_shape(M, n_rows_w, K, ksplit,
-                                   (double)M * n_rows_w * ksplit * sizeof(TO) * (EPI == 1 ? 0.5e-6 : 1e-6),
-                                   EPI == 1, nullptr);
+        shape = kappai_block_shape_for(M, n_rows_w, K, ksplit, sizeof(TO), EPI == 1);
 #define KAPPAI_BLOCKS(...)                                                                         \
   launch_fragment_block<TO, EPI, __VA_ARGS__>(A, Wf, bias, C, M, n_rows_w, K, lda, ldc, ksplit, stream)
       if (shape == 9 && EPI != 0) shape = 5;
@@ -2775,8 +2773,8 @@ static bool launch_shared_rows(const bf16_t* A, const bf16_t* W, const float* bi
 // pieces of the wave's 32 rows, 256 bytes of each of two groups of 8 of K.  The waves meet in LDS
 // at the end to add their K parts in a fixed order.  K can be cut over blocks as well (float
 // partial sums), which is what fills the chip for the products with few rows of W.
-// It takes what the block products do not (launch_rows32): K below 1,024 and results that are not laid out in
-// sixteens of bytes.
+// It takes what the block products do not (launch_rows32): what kappai_rows32_takes names, and results that are not
+// laid out in sixteens of bytes.
 //
 // Host side guarantees: W in fragment order, K / gridDim.y a multiple of 256, lda a multiple of
 // 8, M * lda < 2^31.  Rows of A past M repeat the last row, pieces of W past the end the last
@@ -2980,12 +2978,8 @@ static bool launch_rows32(const bf16_t* A, const bf16_t* Wf, const float* bias, 
       n_rows_w % (EPI == 1 ? 32 : 16) || (lda % 8) || (long)M * lda >= (1L << 31) - 2048 ||
       (out_cols % 4) || (ldc % 4) || ((uintptr_t)C % 16) || (EPI == 1 && sizeof(TO) != 2))
     return false;
-  // the block products wherever the shape fits them and K is one that they were measured over, 1,024 to 10,752 (with
-  // a shorter one this kernel is at a dependent kernel's own time as it is).  Us by them and by this kernel: 64 rows of
-  // 16384 x 2048 gated 15.5 and 18.1, 6144 x 2048 in two ranges 8.5 and 9.6, 2048 x 2048 in eight 4.5 and 5.2, 2048 x
-  // 8192 in eight 9.7 and 11.8; 100 rows of 9216 x 1024 gated 8.5 and 10.3, 3072 x 1024 in four 5.3 and 6.2, 1024 x
-  // 4608 in six 5.1 and 8.0; 33 rows of 2048 x 10752 in six 11.4 and 13.8.
-  if (!itself && K >= 1024 && block256_fits<TO, EPI>(A, Wf, C, M, n_rows_w, K, lda, ldc, ksplit)) {
+  if (!itself && !kappai_rows32_takes(M, n_rows_w, K, ksplit) &&
+      block256_fits<TO, EPI>(A, Wf, C, M, n_rows_w, K, lda, ldc, ksplit)) {
     launch_tile<TO, EPI>(A, nullptr, bias, C, M, n_rows_w, K, lda, ldc, ksplit, 0, stream, Wf);
     return true;
   }
@@ -3021,7 +3015,7 @@ static int launch_bf16(const bf16_t* A, const bf16_t* W, const float* bias, TO* 
   // the 128 x 128 blocks than through the decode kernel, which reads the rows once per 32 columns
   const bool wide_head = EPI == 0 && M > 32 && N >= 16384 && force_kernel == 0 && ksplit == 1 &&
                          block256_fits<TO, EPI>(A, W, C, M, N, K, lda, ldc, ksplit);
-  // 25 to 128 rows: the smallest block products, or 32 x 32 tiles with the rows through LDS, when W is there in
+  // 25 to 128 rows: the block products, or 32 x 32 tiles with the rows through LDS, when W is there in
   // fragment order and the shape fits (else the kernels below)
   if constexpr (EPI != 2) {
     const bool forced = force_kernel == 12 || force_kernel == 18;

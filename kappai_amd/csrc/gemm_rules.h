@@ -2,13 +2,21 @@
 #pragma once
 
 // Steps of more than KAPPAI_ROWS32_MIN_ROWS and up to KAPPAI_ROWS32_MAX_ROWS rows over a W in fragment order, K in runs
-// of KAPPAI_ROWS32_RUN: the smallest block products from K = 1,024 on, else the kernel with 32 x 32 tiles and the
-// rows through LDS (gemm_bf16_rows32).  Below, the kernels with 16 x 16 tiles, which give a matrix kept as rows the
+// of KAPPAI_ROWS32_RUN: the block products (the forms below), or the kernel with 32 x 32 tiles and the rows through LDS
+// (gemm_bf16_rows32, where kappai_rows32_takes says so).  Below, the kernels with 16 x 16 tiles, which give a matrix kept as rows the
 // same bits (24 rows of 9216 x 1024 gated 7.8 us by them, 6.3 in blocks; 1024 x 4608 in eight ranges 4.4, in six 4.7).
 #define KAPPAI_ROWS32_MIN_ROWS 24
 #define KAPPAI_ROWS32_MAX_ROWS 128
 // K of a block of that kernel comes in runs of this many
 #define KAPPAI_ROWS32_RUN 256
+// M rows in `split` ranges of K, n_rows rows of W.  A K below 1,024, where that kernel is at a dependent kernel's own
+// time as it is; and of up to 32 rows, of which it wastes none, the very wide products of a short K (65536 x 1024 28.5
+// us, in blocks 29.6 to 32) and the smallest (256 x 1024 in four ranges 3.3 and 3.4, 64 x 1024 4.4 and 4.7; 512 x 1024
+// in four 3.5 both).  Else the blocks, us by that kernel and by them: 64 rows of 16384 x 2048 gated 17.4 and 15.5, of
+// 6144 x 2048 in two ranges 9.9 and 8.7, of 8192 x 4096 gated 24.7 and 20.2, 100 rows of 1024 x 4608 in six 8.0 and 5.1.
+static inline bool kappai_rows32_takes(int M, int n_rows, int K, int split) {
+  return K < 1024 || (M <= 32 && ((K < 2048 && n_rows > 16384) || (long)n_rows * (K / split) < 131072));
+}
 
 // The blocks of a product of more rows whose W lies in fragment order (gemm_bf16_direct, gemm_bf16_staged),
 // and a model of what each takes, in us: a tile of 64 of K costs `tile` in every round of blocks over the
@@ -24,6 +32,12 @@
 // 128 x 64).  Fitted to 185 products of 160 to 1,040 rows on a card that is 4 % slower than the model, good to 4 to
 // 8 %.  Over 240 products, ranges among them, the form that the model likes best takes 0.2 % more than the fastest
 // of the six up to 256 x 128; without these three 17 % more.
+// Up to 128 rows the blocks of 64 rows or columns are the faster at every K (100 rows of 4096 x 4096 gated 17.4 and
+// 32.6 us in 128 x 128), and 64 x 64 of up to 64 rows also in more blocks than CUs, two to a CU (32 rows of 40960 x
+// 2048 gated 34.4 and 41.9).  There W's stream bounds them and the model's times are 15 to 25 % short, but over 657
+// products (25 to 128 rows, 256 to 65,536 columns, K from 1,024 to 16,384, up to eight ranges, float, bfloat16 and
+// gated results) the form that it likes best, with kappai_rows32_takes, takes 0.2 % more than the fastest in sum; with
+// the limits of more rows 19 % more.
 struct kappai_block_form {
   int shape, rows, cols;           // (shape: gemm.hip, launch_tile)
   double tile, fill, round, mb, start;
@@ -38,11 +52,14 @@ static inline int kappai_block_shape(int M, int N, int K, int split, double resu
                                      double* time) {
   int best = 8;
   double best_t = -1.0;
+  const bool few = M <= KAPPAI_ROWS32_MAX_ROWS;
   const int longest = result_mb > 3e-6 * M * N * split ? 1536 : 2048;
   for (const kappai_block_form& f : KAPPAI_BLOCK_FORMS) {
     if (gated && f.shape == 9) continue;       // (its waves' columns are no whole pairs of 64)
     const double blocks = (double)((M + f.rows - 1) / f.rows) * ((N + f.cols - 1) / f.cols) * split;
-    if (f.rows * f.cols < 128 * 128 && (blocks > 256 || K / split > longest)) continue;
+    if (f.rows * f.cols < 128 * 128 && !(few && f.shape == 15 && M <= 64) &&
+        (blocks > 256 || (!few && K / split > longest)))
+      continue;
     const double rounds = (double)(((long)blocks + 255) / 256), tiles = (double)K / split / 64.0;
     const double t = tiles * (f.tile * rounds + f.fill * blocks / 256) + f.round * rounds +
                      f.mb * result_mb + f.start;
@@ -53,6 +70,10 @@ static inline int kappai_block_shape(int M, int N, int K, int split, double resu
   }
   if (time) *time = best_t;
   return best;
+}
+// The same for results of `elem` bytes each, float planes if there are ranges.
+static inline int kappai_block_shape_for(int M, int N, int K, int split, int elem, bool gated) {
+  return kappai_block_shape(M, N, K, split, (double)M * N * split * elem * (gated ? 0.5e-6 : 1e-6), gated, nullptr);
 }
 
 // The same for a W that lies as rows (gemm_bf16_block256).

@@ -7,6 +7,7 @@ import ctypes
 import pytest
 import torch
 
+from test_block_shapes import FEW
 from test_kernels_gpu import BF16, DEV, F32, close, ops, rand  # noqa: F401
 
 pytestmark = pytest.mark.gpu
@@ -52,6 +53,23 @@ def test_gated_blocks_over_fragment_order(ops, M, F, K, form):  # noqa: F811
 def test_the_rule_takes_every_form(ops, M, N, K):  # noqa: F811
     x, w = rand((M, K), BF16, 87).to(DEV), rand((N, K), BF16, 88).to(DEV)
     assert torch.equal(ops.linear(x, ops.InFragments.of(w)), ops.linear(x, w, force_kernel=ROWS))
+
+
+# 25 to 128 rows: blocks where the rule names some, else the kernel with 32 x 32 tiles, which adds in another order
+@pytest.mark.parametrize("sizes", [s for s in FEW if s[0] <= 128])
+def test_what_25_to_128_rows_take(ops, sizes):  # noqa: F811
+    M, n, K, S, elem, gated = sizes
+    x, w = rand((M, K), BF16, 93).to(DEV), ops.InFragments.of(rand((n, K), BF16, 94, 0.05).to(DEV))
+
+    def product(force):
+        if gated:
+            return ops.linear_swiglu(x, w, force_kernel=force)
+        how = dict(partial_sums=True, split_k=S) if S > 1 else dict(out_dtype=F32 if elem == 4 else BF16)
+        return ops.linear(x, w, force_kernel=force, **how)
+    blocks, tiles = product(FORMS["64x64"]), product(18)
+    assert torch.equal(product(0), tiles if FEW[sizes] == "rows32" else blocks)
+    if K // S > 256:                      # (float sums of one run of 256 may agree, and rounded ones do mostly)
+        assert gated or elem == 2 or not torch.equal(tiles, blocks)
 
 
 # blocks that end behind the last row and the last column, and columns between the rows of the result: nothing is

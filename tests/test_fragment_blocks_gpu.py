@@ -7,7 +7,7 @@ import ctypes
 import pytest
 import torch
 
-from test_block_shapes import FEW
+from test_block_shapes import FEW, WHOLE
 from test_kernels_gpu import BF16, DEV, F32, close, ops, rand  # noqa: F401
 
 pytestmark = pytest.mark.gpu
@@ -45,11 +45,8 @@ def test_gated_blocks_over_fragment_order(ops, M, F, K, form):  # noqa: F811
     assert torch.equal(got, ops.linear_swiglu(x, w, force_kernel=ROWS))
 
 
-# the rule's own choices, one product for every form (by its model: 256 x 256, 256 x 192, 256 x 128,
-# 192 x 128, 128 x 128; then 64 x 128, 128 x 64, 64 x 64 in as many blocks as CUs and in a row more)
-@pytest.mark.parametrize("M,N,K", [(2048, 16384, 512), (2048, 6144, 640), (512, 16384, 512),
-                                   (575, 9216, 512), (300, 1024, 256), (575, 3072, 1024),
-                                   (417, 3072, 2048), (256, 4096, 1024), (257, 4096, 1024)])
+# the rule's own choices, one product or more for every form (test_block_shapes.py has which)
+@pytest.mark.parametrize("M,N,K", list(WHOLE))
 def test_the_rule_takes_every_form(ops, M, N, K):  # noqa: F811
     x, w = rand((M, K), BF16, 87).to(DEV), rand((N, K), BF16, 88).to(DEV)
     assert torch.equal(ops.linear(x, ops.InFragments.of(w)), ops.linear(x, w, force_kernel=ROWS))

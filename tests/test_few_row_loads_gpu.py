@@ -226,3 +226,25 @@ def test_into_the_stream_halves_of_k_share_a_fragment_up_to_8_rows(K, N):
     for stream, ss in out[1:]:
         n = stream.shape[0]
         assert torch.equal(stream, out[0][0][:n]) and torch.equal(ss, out[0][1][:, :n])
+
+
+@pytest.mark.parametrize("K,N", [(1024, 64), (4096, 16), (4608, 1024), (10752, 64)])
+def test_into_the_stream_from_rows_in_fragment_order(K, N):
+    """Rows in fragment order ([K / 32][4][16 row slots][8]) give the bits of plain rows, up to 8 rows and beyond, and
+    what lies in the slots of rows that are not there reaches nothing."""
+    g = _gen(K, N, 19)
+    W, _ = _matrix(N, K, g)
+    norm, resid = torch.rand(N, generator=g, device=DEV) + 0.5, torch.randn(16, N, generator=g, device=DEV)
+    every = _rows(16, K, g)
+    for M in (1, 3, 8, 9, 16):
+        x = every[:M].contiguous()
+        slots = torch.full((16, K), float("nan"), dtype=torch.bfloat16, device=DEV)
+        slots[:M] = x
+        data = slots.view(16, K // 32, 4, 8).permute(1, 2, 0, 3).contiguous().view(16, K)
+        one, two = resid[:M].clone(), resid[:M].clone()
+        want = ops.linear(x, W, add_into=ops.AddInto(one, norm, 1e-5))
+        got = ops.linear(ops.FragmentRows(data, M, two), W, add_into=ops.AddInto(two, norm, 1e-5))
+        assert torch.equal(ops.FragmentRows(data, M, two).materialize(), x)
+        assert torch.equal(one, two) and torch.equal(want.ss[:, :M], got.ss[:, :M]) and torch.isfinite(one).all()
+        kept = [(ops.FragmentRows(r.data, M, one).materialize() if r.fragment else r.data) for r in (want, got)]
+        assert torch.equal(*kept)

@@ -64,4 +64,4 @@ def test_latent_store(ops, dtype, H, d, rot, r, D):  # noqa: F811
     dims = min(8, rot)
     alike(around_the_rule(1, D, dtype, lambda at, kp, vp, pos, seg, tables: ops.latent_store(
         q[at], kv[at], H, d, rot, r, D, w, 1e-5, cos if dims else None, sin if dims else None, dims,
-        1 if dims else 0, kp, vp, pos, seg, tables, PS)), r if r < D else 0, D) if r < D else None
+        1 if dims else 0, kp, vp, pos, seg, tables, PS)), r, D)

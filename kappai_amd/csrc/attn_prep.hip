@@ -44,7 +44,9 @@ struct Two { float a, b; };
 // trips to memory behind the row's position, and a block a round makes them at once.  Two rows of a decode step,
 // one block a row and so: rotate_widen_store 6.5 and 4.6 us, latent_store 6.0 and 3.9, projection_norm_store 6.0
 // and 4.2.  Beyond FEW_ROWS rows one block a row, whose position and page are then read once (1,900 rows: 10.5 to
-// 12 us each, which blocks of one round would need ten times as many of).
+// 12 us each, which blocks of one round would need ten times as many of).  The line is on the near side of where the
+// two meet; one after another in a graph, one block a row and so: 32 rows 4.1 and 2.7, 4.2 and 3.2, 4.3 and 3.2 us, 128
+// rows 4.3 and 2.9, 4.4 and 3.5, 4.5 and 3.8, 512 rows 5.5 and 4.8, 5.5 and 5.1, 5.6 and 7.2.
 #define FEW_ROWS 32
 static int few_rows_blocks(int T, int items) {
   return T > FEW_ROWS || items < 1 ? 1 : (items + AP_THREADS - 1) / AP_THREADS;

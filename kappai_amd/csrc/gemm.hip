@@ -198,8 +198,10 @@ __device__ __forceinline__ void f32_normed_rows(const float* __restrict__ x, con
 // that stream, so the norm has no sum left to make.  A norm kernel between two products is 4.8 us of a trace;
 // norming inside costs 9216 x 1024 gated of three rows 1.5 of its 11.2 us, 2048 x 1024 and 3072 x 1024 half a us.
 //
-// ONE: no run has more than a chunk (8 runs, K up to 1,024): nothing is under way beside the chunk, and with the
-// registers of three blocks a CU instead of two, 576 blocks of gate/up run at once (13.1 -> 12.7 us).
+// ONE: no run has more than a chunk (8 runs, K up to 1,024) and no more than 4 rows: nothing is under way beside the
+// chunk, and with the registers of three blocks a CU instead of two, 576 blocks of gate/up run at once (13.1 -> 12.7
+// us).  With more rows to hold it is the slower (a decode step of the 350M shape, 5 to 9 rows 798 to 930 us with it and
+// 788 to 924 without).
 template <int MT, int COLS, int RUNS, int LOADS, bool GATED = false, bool NORM = false, bool ONE = false>
 __global__ __launch_bounds__((COLS < 16 ? RUNS * COLS / 16 : 8) * WAVE) __attribute__((amdgpu_waves_per_eu(ONE ? 6 : 1)))
 void gemm_f32_skinny_kernel(
@@ -613,6 +615,8 @@ static bool f32_large_blocks(int M, int N) {
   return (big + 255) / 256 * 4 * 8 <= (small + 255) / 256 * 9;
 }
 
+static bool f32_one(int M, int K) { return M <= 4 && K <= 8 * F32_CHUNK; }
+
 template <int LOADS>
 static void launch_f32_gated(const float* A, const float* W, const float* bias, float* C, int M, int F, int K,
                              int lda, int ldc, hipStream_t stream) {
@@ -620,7 +624,7 @@ static void launch_f32_gated(const float* A, const float* W, const float* bias, 
     launch_f32_blocks<LOADS, 4, 2, true>(A, W, bias, C, M, F, K, lda, ldc, stream);
     return;
   }
-  const bool many = f32_runs((K + F32_CHUNK - 1) / F32_CHUNK) == 32, one = K <= 8 * F32_CHUNK;
+  const bool many = f32_runs((K + F32_CHUNK - 1) / F32_CHUNK) == 32, one = f32_one(M, K);
 #define F32_GATED(MT, RUNS, ...)                                                                     \
   hipLaunchKernelGGL((gemm_f32_skinny_kernel<MT, 16, RUNS, LOADS, true, ##__VA_ARGS__>), dim3((F + 7) / 8), \
                      dim3(8 * WAVE), 0, stream, A, W, bias, C, M, F, K, lda, ldc, 0, (const float*)nullptr, 0.f)
@@ -643,7 +647,7 @@ template <int LOADS>
 static void launch_f32(const float* A, const float* W, const float* bias, float* C, int M, int N,
                        int K, int lda, int ldc, hipStream_t stream, int add = 0) {
   if (M <= 64) {
-    const bool many = f32_runs((K + F32_CHUNK - 1) / F32_CHUNK) == 32, one = K <= 8 * F32_CHUNK;
+    const bool many = f32_runs((K + F32_CHUNK - 1) / F32_CHUNK) == 32, one = f32_one(M, K);
 #define F32_SKINNY(MT, COLS, RUNS, ...)                                                           \
   hipLaunchKernelGGL((gemm_f32_skinny_kernel<MT, COLS, RUNS, LOADS, false, ##__VA_ARGS__>), dim3((N + COLS - 1) / COLS), \
                      dim3((COLS < 16 ? RUNS * COLS / 16 : 8) * WAVE), 0, stream, A, W, bias, C, M, N, K,   \
@@ -718,7 +722,7 @@ extern "C" int kappai_gemm_f32_normed(const float* x, const float* norm_w, float
   hipLaunchKernelGGL((gemm_f32_skinny_kernel<1, COLS, 8, F32_WHOLE, GATED, true, ONE>),                 \
                      dim3((N + BLOCK - 1) / BLOCK), dim3((COLS == 8 ? 4 : 8) * WAVE), lds, stream, x, W, \
                      bias, C, M, N, K, K, ldc, 0, norm_w, eps)
-  const bool one = K <= 8 * F32_CHUNK;
+  const bool one = f32_one(M, K);
   if (gated && one) F32_NORMED(16, true, 8, true);
   else if (gated) F32_NORMED(16, true, 8, false);
   else if (N <= 256 * 8) F32_NORMED(8, false, 8, false);

@@ -6,6 +6,7 @@ call's partial results still in the array.  That it allocates nothing is checked
 driver's count of free device memory does not move across the call, and the call can be recorded
 into a HIP graph, where an allocation is an error."""
 import ctypes
+import gc
 import math
 
 import numpy as np
@@ -58,7 +59,10 @@ def run_both(lib, case, T, H, G, d, ps, keys_per_split, n_splits):
     torch.cuda.synchronize()
     # the driver's own count of free bytes (torch's allocator counter would not see a hipMalloc
     # inside the library); the array's address was looked up before (init), so nothing is left
-    # that the call may take
+    # that the call may take.  (What other tests left in cycles, graphs among it, is given back now and
+    # not when a collection happens to fall between the two counts.)
+    gc.collect()
+    torch.cuda.synchronize()
     free_before = torch.cuda.mem_get_info(DEV)[0]
     rc = lib.kappai_attn_decode_static(*common(got), *tables)
     assert rc == 0, (rc, lib.kappai_attn_decode_static_error().decode())

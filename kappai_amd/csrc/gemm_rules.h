@@ -3,8 +3,9 @@
 
 // Steps of more than KAPPAI_ROWS32_MIN_ROWS and up to KAPPAI_ROWS32_MAX_ROWS rows over a W in fragment order, K in runs
 // of KAPPAI_ROWS32_RUN: the block products (the forms below), or the kernel with 32 x 32 tiles and the rows through LDS
-// (gemm_bf16_rows32, where kappai_rows32_takes says so).  Below, the kernels with 16 x 16 tiles, which give a matrix kept as rows the
-// same bits (24 rows of 9216 x 1024 gated 7.8 us by them, 6.3 in blocks; 1024 x 4608 in eight ranges 4.4, in six 4.7).
+// (gemm_bf16_rows32, where kappai_rows32_takes says so).  Below, the kernels with 16 x 16 tiles, which give a matrix
+// kept as rows the same bits (24 rows of 9216 x 1024 gated 7.8 us by them, 6.3 in blocks; 1024 x 4608 in eight ranges
+// 4.4, in six 4.7).
 #define KAPPAI_ROWS32_MIN_ROWS 24
 #define KAPPAI_ROWS32_MAX_ROWS 128
 // K of a block of that kernel comes in runs of this many

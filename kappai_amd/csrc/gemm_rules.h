@@ -33,7 +33,7 @@ static inline bool kappai_rows32_takes(int M, int n_rows, int K, int split) {
 // 128 x 64).  Fitted to 185 products of 160 to 1,040 rows on a card that is 4 % slower than the model, good to 4 to
 // 8 %.  Over 240 products, ranges among them, the form that the model likes best takes 0.2 % more than the fastest
 // of the six up to 256 x 128; without these three 17 % more.
-// Up to 128 rows the blocks of 64 rows or columns are the faster at every K (100 rows of 4096 x 4096 gated 17.4 and
+// Up to 128 rows the blocks of 64 rows or columns are the faster at every K (97 rows of 4096 x 4096 gated 17.4 and
 // 32.6 us in 128 x 128), and 64 x 64 of up to 64 rows also in more blocks than CUs, two to a CU (32 rows of 40960 x
 // 2048 gated 34.4 and 41.9).  There W's stream bounds them and the model's times are 15 to 25 % short, but over 657
 // products (25 to 128 rows, 256 to 65,536 columns, K from 1,024 to 16,384, up to eight ranges, float, bfloat16 and
